@@ -206,6 +206,21 @@ def test_gated_act_mul_in_the_few_rows_kernel_is_bit_identical(hip_ctx, rows):
     assert outs[0][0] == outs[1][0] and np.array_equal(outs[0][1], outs[1][1])
 
 
+@pytest.mark.parametrize("rows", [17, 40, 127, 131])
+def test_prompts_of_dozens_of_rows_against_the_oracle(hip_ctx, rows):
+    """Prompts whose linears run in the register-fed kernel (k_gemm_rows.hip; groups of 128): the fused GatedActMul epilogue and the split-K tiles finished by the next Normalization,
+    against the oracle with the bound that test_layer_taps uses for whole passes: outputs of every layer within 2 % of the oracle's, in the 2-norm."""
+    cfg = S.tiny_qwen(group_size=128)
+    bundle = S.build_model(cfg)
+    prompt = S.synthetic_prompt(rows, cfg.vocab_size)
+    om, hm = O.OracleModel(bundle), HipModel(hip_ctx, bundle, MODEL_DEBUG_TAPS)
+    om.prefill(prompt), hm.prefill(prompt)
+    for layer in range(cfg.num_layers):
+        want, got = S.bf16_bits_to_f32(om.layer_output(layer)).reshape(rows, -1), S.bf16_bits_to_f32(hm.read_layer_output(layer)).reshape(rows, -1)
+        assert np.linalg.norm(want - got) <= 0.02 * np.linalg.norm(want), f"layer {layer}"
+    hm.close(), om.close()
+
+
 @pytest.mark.parametrize("heads,groups,context", [(10, 2, 2200), (6, 1, 1300)])
 def test_long_context_decode_and_odd_gqa_factors(hip_ctx, heads, groups, context):
     """A model whose context capacity is >= 4096: attn_dec takes its doubled key splits and serves 5 or 6 query heads of a KV head

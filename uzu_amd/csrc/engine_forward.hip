@@ -120,7 +120,7 @@ void linear(Enc& e, const DLinear& L, const uint16_t* input, uint16_t* output, u
     p.bits = L.bits, p.group_size = L.group, p.ab_scale = 1.0f;
     p.m = batch, p.n = L.n, p.k = L.k;
     offset_tables(e.m, L, input, batch, &p);
-    if (post && !exchange && !L.out_signs && batch >= 128) p.post_norm = &post->p, p.post_norm_done = &post->done;
+    if (post && !exchange && !L.out_signs && batch >= 17) p.post_norm = &post->p, p.post_norm_done = &post->done;
     const char* variant = "matmul";
     e.begin();
     const uzu_status r = k::matmul(e.s, p, e.m->ctx->num_cus, &variant);
@@ -156,7 +156,7 @@ bool linear_gated(Enc& e, const DLinear& L, const uint16_t* input, uint16_t* gat
     p.act_mul = 1, p.act_type = act_type;
     offset_tables(e.m, L, input, batch, &p);
     // the down projection's row sums from this epilogue (64 gated columns per workgroup): no pre-pass launch in front of it
-    const bool file = consumer && gated_out == e.m->gated && consumer->k == L.n / 2 && k::gemm_q_mfma128_supported(p, e.m->ctx->num_cus) && rowsum_wanted(e.m, *consumer, batch, 64, e.m->rs_gated);
+    const bool file = consumer && gated_out == e.m->gated && consumer->k == L.n / 2 && !k::gemm_rows_preferred(p) && k::gemm_q_mfma128_supported(p, e.m->ctx->num_cus) && rowsum_wanted(e.m, *consumer, batch, 64, e.m->rs_gated);
     if (file) p.gated_rowsum_out = e.m->rs_gated.buf;
     const char* variant = "matmul";
     e.begin();
@@ -551,7 +551,7 @@ uzu_status encode_forward(uzu_hip_model* m, hipStream_t s, uint32_t count, bool 
         }
         hidden_normed = false;
         PostNorm mlp_norm; // the pre-MLP normalisation, offered to the mixer's out projection when nothing sits between them
-        const bool offer_mlp = !L.post_mixer.present && rows >= 128 && !L.pre_mlp.scalar_mode;
+        const bool offer_mlp = !L.post_mixer.present && rows >= 17 && !L.pre_mlp.scalar_mode;
         if (offer_mlp) mlp_norm.p = norm_params(e, L.pre_mlp, m->mixed, m->normed, sc_cur, 2, rows, d, L.d.mlp_kind == UZU_MLP_MOE ? nullptr : &L.up);
         if (L.d.mixer_kind == UZU_MIXER_ATTENTION)
             attention_mixer(e, L, h, m->mixed, q, offer_mlp ? &mlp_norm : nullptr, first_done);
@@ -580,7 +580,7 @@ uzu_status encode_forward(uzu_hip_model* m, hipStream_t s, uint32_t count, bool 
         }
         // the next layer's pre-mixer normalisation rides on this layer's down projection (not past the last layer: the output norm takes one row)
         PostNorm next_norm;
-        const bool offer_next = !is_moe && rows >= 128 && !L.post_mlp.present && !L.d.has_ple && l + 1 < layer_count && m->layers[l + 1].pre_mixer.present;
+        const bool offer_next = !is_moe && rows >= 17 && !L.post_mlp.present && !L.d.has_ple && l + 1 < layer_count && m->layers[l + 1].pre_mixer.present;
         if (offer_next) {
             const DLayer& Nx = m->layers[l + 1];
             next_norm.p = norm_params(e, Nx.pre_mixer, hidden, m->normed, sc_cur, 2, rows, d, Nx.d.mixer_kind == UZU_MIXER_ATTENTION ? &Nx.qkv : &Nx.in_proj);

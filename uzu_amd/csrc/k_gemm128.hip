@@ -874,7 +874,7 @@ static int gemm128_form(const MatmulParams& p, int num_cus, uint32_t splits) {
 }
 // host arithmetic only (uzu_hip_prefill_gemm_plan): which kernel / form / split-K a shape gets; UZU_GEMM_FORM / UZU_GEMM_SPLITS apply as at launch
 void gemm_q_mfma128_plan_query(const MatmulParams& p, int num_cus, uint32_t* large_tile, uint32_t* form, uint32_t* splits, uint32_t* workgroups) {
-    *large_tile = gemm_q_mfma128_supported(p, num_cus) ? 1u : 0u;
+    *large_tile = gemm_q_mfma128_supported(p, num_cus) && !gemm_rows_preferred(p) ? 1u : 0u;
     *form = *splits = *workgroups = 0;
     if (!*large_tile) return;
     *splits = gemm128_splits(p, num_cus);
@@ -944,6 +944,11 @@ uzu_status gemm_q_mfma128(hipStream_t s, const MatmulParams& p, int num_cus, voi
     }
 #undef UZU_LAUNCH
     if (st != UZU_OK || splits == 1) return st;
+    return gemm_split_finish(s, p, partials, splits);
+}
+
+// The end of a split-K product: partial tiles [splits][m, n] added in split order, epilogue, D -- and, where the caller asked for it, the Normalization that reads D next.
+uzu_status gemm_split_finish(hipStream_t s, const MatmulParams& p, const float* partials, uint32_t splits) {
     const size_t total = (size_t)p.m * p.n;
     if (p.post_norm && p.post_norm_done) { // the rows go straight into a Normalization: reduction + epilogue + normalisation as one launch
         const NormPartials sp{partials, splits, total, (const uint16_t*)p.bias, (uint16_t*)p.d};

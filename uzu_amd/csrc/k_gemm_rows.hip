@@ -1,0 +1,302 @@
+// k_gemm_rows.hip -- quantised matmul for dozens to hundreds of activation rows: a register-fed matrix-core kernel without operand staging.
+//
+// Where it sits: behind the few-rows kernel (k_gemv_rows.hip, M <= 16) and in front of the large tiles (k_gemm128.hip).  At these sizes a linear of a 1024-wide
+// model is 1 .. 15 GFLOP and 1 .. 4 MB of codes -- a microsecond or two of either -- and what a tile kernel spends is its chain: a k-step of 64 through LDS with
+// two barriers is ~1 us whatever else the CU does, so a 64 x 64 tile over K = 3584 was 35 us on sixteen workgroups.  Here nothing is staged and nothing waits:
+//   * a wave owns 16 MT tokens x 16 NB weight rows of v_mfma_f32_16x16x32_bf16.  Activations go from the L2 into the A operand (lane (r, g): token r, 16 bytes
+//     at k0 + 32 i + 8 g -- an instruction takes whole 64-byte pieces of 16 rows; at k0 + 32 g + 8 i it would touch every piece four times, which is what bounds
+//     the cache in front of a CU).  A lane loads 16 bytes = 32 codes of weight row r at k0 + 32 g; four lane swaps (v_permlane32_swap, v_permlane16_swap) turn
+//     the (lane group, word) square round, so that word i holds the codes of k0 + 32 i + 8 g, and a word converts to the 8 bf16 (16 + q) of MFMA i
+//     (gemm_convert.h: two codes per v_and_or_b32, pair order (0 4) (1 5) (2 6) (3 7), which the activations are permuted to);
+//   * a step contracts over 128 k = one quant group: the group's products and the tokens' sums (the same A against an all-ones B) are folded with the f32 scale
+//     and offset of the lane's own weight row, so no weight is ever rounded and no scalar crosses lanes.  Scales are read two groups at a time;
+//   * the next step's loads are in flight while a step is computed, waves never meet before the end, and K is cut KW ways over the waves of a workgroup
+//     (added through LDS in wave order) and `splits` ways over workgroups (f32 partial tiles, added in split order by the reduction that also applies the next
+//     Normalization): the cuts are chosen so that the chip has a workgroup per CU and a wave's chain is a few steps.
+// What bounds it: below ~100 rows the launch and two or three dependent loads; above, the L2 traffic of unshared operands (~7 TB/s at 0.3 PFLOP/s).
+// Measured, us per launch, 64 x 64 tiles -> here (weights not in cache): 1024 x 3584, M = 37: 38.0 -> 8.5; 1024 x 2048: 23.7 -> 6.9; 7168 x 1024 + GatedActMul:
+// 14.3 + 4.7 -> 8.1; 8224 x 1024: 14.5 -> 10.1; 4096 x 14336: 163 -> 29; a 37-token prompt of Qwen3.5-0.8B 3.97 -> 2.02 ms.
+#include "decode_epilogue.h"
+#include "device_utils.h"
+#include "kernels.h"
+
+namespace uzu {
+namespace k {
+
+namespace {
+typedef __attribute__((ext_vector_type(8))) __bf16 gm_bf16x8;
+typedef __attribute__((ext_vector_type(4))) float gm_f32x4;
+typedef __attribute__((ext_vector_type(4))) uint32_t gm_u32x4;
+
+struct GemmRowsParams {
+    const uint16_t* a; // [m, k] bf16
+    const uint8_t* w;  // [n, k / 2]
+    const uint16_t* scales;
+    const uint16_t* biases;
+    const uint8_t* zp;
+    const uint16_t* out_bias; // [n] or null
+    void* d;                  // [m, n] (ACT: [m, n / 2]) bf16 or f32
+    float* partials;          // [splits][m, n] f32, or null: the whole sum is here
+    uint32_t m, n, k, d_f32, act_type, splits;
+};
+
+// (lane group g, word j) -> (lane group j, word g): register i of lane group g afterwards holds what word g of lane group i was
+__device__ __forceinline__ void turn_words(gm_u32x4& w) {
+    typedef __attribute__((ext_vector_type(2))) uint32_t pair;
+    pair t = __builtin_bit_cast(pair, __builtin_amdgcn_permlane32_swap(w.x, w.z, false, false));
+    w.x = t.x, w.z = t.y;
+    t = __builtin_bit_cast(pair, __builtin_amdgcn_permlane32_swap(w.y, w.w, false, false));
+    w.y = t.x, w.w = t.y;
+    t = __builtin_bit_cast(pair, __builtin_amdgcn_permlane16_swap(w.x, w.y, false, false));
+    w.x = t.x, w.y = t.y;
+    t = __builtin_bit_cast(pair, __builtin_amdgcn_permlane16_swap(w.z, w.w, false, false));
+    w.z = t.x, w.w = t.y;
+}
+
+// KW waves of the workgroup's four share a tile and split its steps; the other 4 / KW side by side.  ACT: n = 2 h weight rows [up | gate]; blocks 0 .. NB/2 - 1
+// of a wave are up rows, the rest the gate rows of the same outputs, and the epilogue is GatedActMul on the rounded pair.
+template <int NB, int MT, int KW, bool ACT, uint32_t KIND> // KIND: uzu_matmul_b_kind (a branch on it in the loop would wait for every load in flight)
+__global__ void __launch_bounds__(256, 2) gemm_rows_kernel(GemmRowsParams p) {
+    constexpr int OB = ACT ? NB / 2 : NB;   // 16-row blocks of outputs per wave
+    constexpr int PITCH = 16 * NB + 4;      // floats per token of a parked tile
+    constexpr int GROUPS = 4 / KW;          // tiles side by side in the workgroup
+    __shared__ __attribute__((aligned(16))) float s_part[4 * 16 * MT * PITCH];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t r = lane & 15, g = lane >> 4, kw = wave % KW, grp_w = wave / KW;
+    const uint32_t out_n = ACT ? p.n / 2 : p.n, half_k = p.k / 2, G = p.k / 128, pairs = G / 2;
+    const uint32_t row0 = (blockIdx.x * GROUPS + grp_w) * (16 * OB), t0 = blockIdx.y * (16 * MT);
+    // this wave's steps, a whole number of pairs (the host keeps KW * splits <= pairs)
+    const uint32_t part = blockIdx.z * KW + kw, parts = p.splits * KW;
+    const uint32_t s_lo = 2 * (pairs * part / parts), s_hi = 2 * (pairs * (part + 1) / parts);
+    // rows and tokens past the end are read from inside the matrices; their sums are never stored
+    uint32_t wrow[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const uint32_t base = row0 + 16 * (ACT && b >= OB ? b - OB : b), side = ACT && b >= OB ? out_n : 0u;
+        wrow[b] = side + min(base + r, out_n - 1);
+    }
+    const uint16_t* xrow[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) xrow[t] = p.a + (size_t)min(t0 + 16 * t + r, p.m - 1) * p.k + 8 * g;
+    struct Step {
+        gm_u32x4 codes[NB], xv[MT][4];
+    };
+    auto load_step = [&](uint32_t s, Step& st) {
+        const uint32_t c = min(s, G - 1); // (past the end: a reload that is never consumed)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) st.codes[b] = *(const gm_u32x4*)(p.w + (size_t)wrow[b] * half_k + 16 * g + (size_t)c * 64);
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) st.xv[t][i] = *(const gm_u32x4*)(xrow[t] + (size_t)c * 128 + 32 * i);
+    };
+    uint32_t sc2[NB], of2[NB] = {}; // scales / offsets of a pair of groups
+    auto load_scales = [&](uint32_t s) {
+        const uint32_t c = min(s, G - 2);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const size_t at = (size_t)wrow[b] * G + c;
+            sc2[b] = *(const uint32_t*)(p.scales + at);
+            if constexpr (KIND == UZU_MATMUL_B_SCALE_BIAS) of2[b] = *(const uint32_t*)(p.biases + at);
+            else if constexpr (KIND == UZU_MATMUL_B_SCALE_ZERO_POINT) of2[b] = p.zp[at / 2];
+        }
+    };
+    uint32_t mask = 0x00780078u, magic = 0x41804180u, ones = 0x3F803F80u;
+    asm("" : "+s"(mask));
+    asm("" : "+v"(magic));
+    asm("" : "+v"(ones));
+    const gm_u32x4 ones4 = {ones, ones, ones, ones};
+    gm_f32x4 acc[NB][MT]; // tokens 4 g + v of tile t, row r of block b
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[b][t] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](Step& st, const float (&sc)[NB], const float (&of)[NB]) {
+        gm_f32x4 dq[NB][MT], dx[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            dx[t] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int b = 0; b < NB; ++b) dq[b][t] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) turn_words(st.codes[b]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            gm_u32x4 xa[MT];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) { // (x0,x1) (x2,x3) (x4,x5) (x6,x7) -> (x0,x4) (x1,x5) (x2,x6) (x3,x7)
+                const gm_u32x4 u = st.xv[t][i];
+                xa[t].x = __builtin_amdgcn_perm(u.z, u.x, 0x05040100u), xa[t].y = __builtin_amdgcn_perm(u.z, u.x, 0x07060302u);
+                xa[t].z = __builtin_amdgcn_perm(u.w, u.y, 0x05040100u), xa[t].w = __builtin_amdgcn_perm(u.w, u.y, 0x07060302u);
+                dx[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, xa[t]), __builtin_bit_cast(gm_bf16x8, ones4), dx[t], 0, 0, 0);
+            }
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const uint32_t w = st.codes[b][i];
+                gm_u32x4 wv;
+                wv.x = ((w << 3) & mask) | magic, wv.y = ((w >> 1) & mask) | magic, wv.z = ((w >> 5) & mask) | magic, wv.w = ((w >> 9) & mask) | magic;
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                    dq[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, xa[t]), __builtin_bit_cast(gm_bf16x8, wv), dq[b][t], 0, 0, 0);
+            }
+        }
+        // group fold: acc += scale dq + (offset - 16 scale) sum_x
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[b][t][v] = fmaf(sc[b], dq[b][t][v], fmaf(of[b], dx[t][v], acc[b][t][v]));
+    };
+    auto offset_of = [&](float sc, float raw) { // raw: the bf16 offset, or the zero point
+        const float of = KIND == UZU_MATMUL_B_SCALE_BIAS ? raw : KIND == UZU_MATMUL_B_SCALE_ZERO_POINT ? -sc * raw : -sc * 8.0f;
+        return fmaf(-kQ4Offset, sc, of);
+    };
+    Step stA, stB;
+    load_step(s_lo, stA);
+    load_scales(s_lo);
+    for (uint32_t s = s_lo; s < s_hi; s += 2) {
+        float sc0[NB], of0[NB], sc1[NB], of1[NB];
+        load_step(s + 1, stB);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            constexpr bool zp = KIND == UZU_MATMUL_B_SCALE_ZERO_POINT;
+            sc0[b] = bits_to_f32(sc2[b] << 16), sc1[b] = bits_to_f32(sc2[b] & 0xFFFF0000u);
+            of0[b] = offset_of(sc0[b], zp ? (float)(of2[b] & 15u) : bits_to_f32(of2[b] << 16));
+            of1[b] = offset_of(sc1[b], zp ? (float)((of2[b] >> 4) & 15u) : bits_to_f32(of2[b] & 0xFFFF0000u));
+        }
+        load_scales(s + 2);
+        __builtin_amdgcn_sched_barrier(0); // (left alone, the scheduler sinks the loads to their uses and waits for each)
+        compute(stA, sc0, of0);
+        __builtin_amdgcn_sched_barrier(0);
+        load_step(s + 2, stA);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(stB, sc1, of1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // the tile to LDS by token, waves' shares added in wave order; consecutive threads take consecutive quads of a token's outputs (n % 4 == 0: a quad is all
+    // inside or all outside)
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) s_part[((size_t)wave * 16 * MT + 16 * t + 4 * g + v) * PITCH + 16 * b + r] = acc[b][t][v];
+    lds_barrier();
+    constexpr int QUADS = 4 * OB; // per token
+    const uint32_t local = tid % (64 * KW);
+    const float* base = s_part + (size_t)grp_w * KW * 16 * MT * PITCH;
+    for (uint32_t i = local; i < 16 * MT * QUADS; i += 64 * KW) {
+        const uint32_t tl = i / QUADS, quad = i % QUADS, token = t0 + tl, n = row0 + 4 * quad;
+        if (token >= p.m || n >= out_n) continue;
+        const float* at = base + (size_t)tl * PITCH + 4 * quad;
+        gm_f32x4 v = *(const gm_f32x4*)at, gate = v;
+        if (ACT) gate = *(const gm_f32x4*)(at + 16 * OB);
+#pragma unroll
+        for (int w = 1; w < KW; ++w) {
+            v += *(const gm_f32x4*)(at + (size_t)w * 16 * MT * PITCH);
+            if (ACT) gate += *(const gm_f32x4*)(at + (size_t)w * 16 * MT * PITCH + 16 * OB);
+        }
+        if (p.partials) {
+            *(gm_f32x4*)(p.partials + ((size_t)blockIdx.z * p.m + token) * p.n + n) = v;
+            continue;
+        }
+        if (p.out_bias) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[j] += bf16_to_f32(p.out_bias[n + j]);
+                if (ACT) gate[j] += bf16_to_f32(p.out_bias[out_n + n + j]);
+            }
+        }
+        if (!ACT && p.d_f32) {
+            *(gm_f32x4*)((float*)p.d + (size_t)token * out_n + n) = v;
+            continue;
+        }
+        uint16_t o[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) // ACT: the rounded pair the unfused kernels would have stored (gated_act_mul/mod.rs:5-12)
+            o[j] = f32_to_bf16(ACT ? round_bf16(round_bf16(v[j]) * act_bf16(p.act_type, round_bf16(gate[j]), kExp2fTab)) : v[j]);
+        u32x2_v q;
+        q.x = (uint32_t)o[0] | ((uint32_t)o[1] << 16), q.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
+        *(u32x2_v*)((uint16_t*)p.d + (size_t)token * out_n + n) = q;
+    }
+}
+
+struct GemmRowsPlan {
+    int nb, kw;
+    uint32_t splits;
+};
+
+// The cuts: 16-row blocks per wave, waves per tile, K splits over workgroups.  A launch wants about a workgroup per CU; narrow problems take two blocks per wave,
+// then all four waves on one tile, then splits (measured at N 1024 .. 8224, K 1024 .. 3584, M 20 .. 1021).
+GemmRowsPlan gemm_rows_plan(const MatmulParams& p, int num_cus) {
+    GemmRowsPlan q{};
+    const uint32_t blocks = ((p.act_mul ? p.n / 2 : p.n) + 15) / 16, token_tiles = (p.m + 31) / 32, pairs = p.k / 256, cus = (uint32_t)num_cus;
+    auto tiles = [&](uint32_t nb) { const uint32_t ob = p.act_mul ? nb / 2 : nb; return ((blocks + ob - 1) / ob) * token_tiles; };
+    const bool long_k = p.k >= 8192; // enough steps to split four-block tiles as well (4096 x 14336, M = 48: 42 -> 33 us)
+    q.nb = tiles(2) <= (long_k ? cus / 2 : cus) ? 2 : 4;
+    const uint32_t t = tiles(q.nb);
+    q.kw = t <= cus + cus / 4 ? 4 : t <= 2 * cus + cus / 2 ? 2 : 1;
+    q.splits = 1;
+    if (!p.act_mul && (q.nb == 2 || long_k))
+        while (q.splits * 2 * t <= cus && q.splits * 4 <= pairs) q.splits *= 2;
+    return q;
+}
+
+template <int NB, int MT, int KW, bool ACT> uzu_status launch_gr(hipStream_t s, const GemmRowsParams& q, uint32_t kind) {
+    const uint32_t out_n = ACT ? q.n / 2 : q.n, per = 16 * (ACT ? NB / 2 : NB) * (4 / KW);
+    const dim3 grid((out_n + per - 1) / per, (q.m + 16 * MT - 1) / (16 * MT), q.splits);
+    switch (kind) {
+    case UZU_MATMUL_B_SCALE_BIAS: return launch_check([&] { hipLaunchKernelGGL((gemm_rows_kernel<NB, MT, KW, ACT, UZU_MATMUL_B_SCALE_BIAS>), grid, dim3(256), 0, s, q); }, "gemm_rows");
+    case UZU_MATMUL_B_SCALE_ZERO_POINT: return launch_check([&] { hipLaunchKernelGGL((gemm_rows_kernel<NB, MT, KW, ACT, UZU_MATMUL_B_SCALE_ZERO_POINT>), grid, dim3(256), 0, s, q); }, "gemm_rows");
+    default: return launch_check([&] { hipLaunchKernelGGL((gemm_rows_kernel<NB, MT, KW, ACT, UZU_MATMUL_B_SCALE_SYMMETRIC>), grid, dim3(256), 0, s, q); }, "gemm_rows");
+    }
+}
+template <int NB, int MT, bool ACT> uzu_status launch_kw(hipStream_t s, const GemmRowsParams& q, uint32_t kind, int kw) {
+    return kw == 1 ? launch_gr<NB, MT, 1, ACT>(s, q, kind) : kw == 2 ? launch_gr<NB, MT, 2, ACT>(s, q, kind) : launch_gr<NB, MT, 4, ACT>(s, q, kind);
+}
+
+bool gemm_rows_supported(const MatmulParams& p) {
+    if (exact_mode() || p.m < 17 || p.m > 65535 || p.bits != 4 || p.b_kind == UZU_MATMUL_B_FULL_PRECISION) return false;
+    if (p.w_dt != UZU_BF16 || p.a_dt != UZU_BF16 || (p.d_dt != UZU_BF16 && p.d_dt != UZU_F32)) return false;
+    if (p.signed_codes || p.ab_scale != 1.0f || p.accumulate || p.has_soft_cap || p.gather) return false;
+    if (p.act_mul ? (p.n % 8 || p.d_dt != UZU_BF16) : p.n % 4) return false; // whole quads of outputs
+    if (p.group_size != 128 || p.k % 256) return false; // scales and offsets are read two groups at a time
+    if (((uintptr_t)p.scales | (uintptr_t)p.biases) & 3) return false;
+    return (((uintptr_t)p.a | (uintptr_t)p.b | (uintptr_t)p.d) & 15) == 0;
+}
+
+} // namespace
+
+// Where this kernel is the faster one.  Below 128 rows the other choice is the 64 x 64 tile (k_gemm.hip), which pays ~0.6 us per 64 k whatever M is and gains from
+// M only when its tiles fill the chip (28672 x 4096: 59 us at M = 37 .. 64 with GatedActMul as a launch of its own behind it, this kernel 58 .. 66 with it); from 128 rows on it is the 128 x 128 tile (k_gemm128.hip), which
+// reads an operand byte ~4 times as often from LDS instead of the L2 and is ahead as soon as there is work for its tiles: at 8224 x 1024 33 us against 33 at M = 256,
+// 41 against 44 at M = 517; at 1024 x 3584 36 us against 23 at M = 517; at 4096 x 14336 75 us against 53 at M = 128, 79 against 101 at M = 256.
+bool gemm_rows_preferred(const MatmulParams& p) {
+    if (!gemm_rows_supported(p) || (p.m >= 128 && (tune_env("gemm_form") || tune_env("gemm_splits")))) return false; // (a pinned form or split-K is the large tile's)
+    const double gflops = 2e-9 * p.m * p.n * p.k;
+    if (p.k >= 8192) return p.m < 128 || gflops <= 16.0;
+    return gflops <= (p.m >= 128 ? 4.5 : p.act_mul ? 16.0 : 9.0);
+}
+
+uzu_status gemm_rows(hipStream_t s, const MatmulParams& p, int num_cus) {
+    GemmRowsPlan plan = gemm_rows_plan(p, num_cus);
+    GemmRowsParams q{};
+    q.a = (const uint16_t*)p.a, q.w = (const uint8_t*)p.b, q.scales = (const uint16_t*)p.scales, q.biases = (const uint16_t*)p.biases, q.zp = p.zero_points;
+    q.out_bias = (const uint16_t*)p.bias, q.d = p.d, q.m = p.m, q.n = p.n, q.k = p.k;
+    q.d_f32 = p.d_dt == UZU_F32, q.act_type = p.act_type, q.splits = plan.splits;
+    const size_t total = (size_t)p.m * p.n;
+    if (plan.splits > 1) {
+        q.partials = (float*)stream_workspace(s, (size_t)plan.splits * total * 4);
+        if (!q.partials) q.splits = 1; // (a stream under capture has no workspace)
+    }
+    uzu_status st;
+    if (p.act_mul) st = plan.nb == 2 ? launch_kw<2, 2, true>(s, q, p.b_kind, plan.kw) : launch_kw<4, 2, true>(s, q, p.b_kind, plan.kw);
+    else st = plan.nb == 2 ? launch_kw<2, 2, false>(s, q, p.b_kind, plan.kw) : launch_kw<4, 2, false>(s, q, p.b_kind, plan.kw);
+    if (st != UZU_OK || q.splits == 1) return st;
+    return gemm_split_finish(s, p, q.partials, q.splits);
+}
+
+} // namespace k
+} // namespace uzu

@@ -363,6 +363,10 @@ uzu_status matmul(hipStream_t s, const MatmulParams& p, int num_cus, const char*
         if (variant) *variant = "gemv_rows_mfma";
         return gemv_rows_mfma(s, p);
     }
+    if (gemm_rows_preferred(p)) { // dozens of rows (k_gemm_rows.hip)
+        if (variant) *variant = "gemm_rows";
+        return gemm_rows(s, p, num_cus);
+    }
     if (gemm_q_mfma_supported(p)) { // prefill-sized M: bf16 matrix cores (k_gemm.hip)
         if (variant) *variant = p.bits == 4 ? "gemm_q_mfma<4>" : "gemm_q_mfma<8>";
         return gemm_q_mfma(s, p, num_cus);
@@ -380,6 +384,7 @@ bool matmul_act_mul_supported(hipStream_t s, const MatmulParams& p, int num_cus)
     q.act_mul = 1;
     if (exact_mode() || q.b_kind == UZU_MATMUL_B_FULL_PRECISION || (uintptr_t)q.b % 16 || (uintptr_t)q.a % 16) return false;
     if (gemv_rows_mfma_supported(q)) return true; // a handful of rows: the few-rows kernel carries the epilogue too (no workspace: fine under capture)
+    if (gemm_rows_preferred(q)) return true; // (no workspace either)
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false; // no workspace during capture
     return gemm_q_mfma_supported(q) && gemm_q_mfma128_supported(q, num_cus);

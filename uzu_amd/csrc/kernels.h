@@ -68,6 +68,10 @@ uzu_status matmul(hipStream_t s, const MatmulParams& p, int num_cus, const char*
 // true when matmul() can run `p` with the fused GatedActMul epilogue (act_mul = 1: D = [m, n/2]); otherwise run the matmul and
 // gated_act_mul separately
 bool matmul_act_mul_supported(hipStream_t s, const MatmulParams& p, int num_cus);
+// k_gemm_rows.hip: M >= 17 activation rows against int4 codes (group % 128 == 0), register-fed: dozens to hundreds of rows
+bool gemm_rows_preferred(const MatmulParams& p);
+uzu_status gemm_rows(hipStream_t s, const MatmulParams& p, int num_cus);
+uzu_status gemm_split_finish(hipStream_t s, const MatmulParams& p, const float* partials, uint32_t splits); // k_gemm128.hip
 // k_gemv_rows.hip: 2 <= M <= 16 activation rows against int4 codes (group % 128 == 0) as ONE pass over the weights on the matrix cores
 bool gemv_rows_mfma_supported(const MatmulParams& p);
 // Normalization (RMS; ShortcutMode Copy / Add; normalization.rs:56-125) of the m <= 16 activation rows as the PROLOGUE of the few-rows kernel
