@@ -56,6 +56,19 @@ def test_linear_matrix_core_form_equals_the_plain_form(hip_ctx, rows, n, k, batc
     assert np.abs(a - want).max() <= 3e-5 * max(1.0, np.abs(want).max()) and np.abs(c - want).max() <= 3e-5 * max(1.0, np.abs(want).max())
 
 
+@pytest.mark.parametrize("rows,n,k,act", [(129, 8200, 1024, 0), (1000, 1025, 1024, 1), (255, 16400, 256, 0), (513, 8192, 256, 0), (2050, 4100, 128, 1), (128, 4100, 2048, 0)])
+def test_linear_prompt_sized_form(hip_ctx, rows, n, k, act):
+    """Prompt-sized products (both operands by LDS DMA): every tile form and buffer count, ragged last tiles in both directions, two k-steps and many, bias, activation and a residual
+    in place; f32 sums of bf16 products, so the bound of the other matrix-core form holds."""
+    rng = np.random.default_rng(rows + n)
+    x, w = rng.standard_normal((rows, k), dtype=np.float32), O.to_bf16(rng.standard_normal((n, k), dtype=np.float32))
+    b, res = O.to_bf16(rng.standard_normal(n)), rng.standard_normal((rows, n), dtype=np.float32)
+    got = linear(hip_ctx, x, w, b, res, act=act, bf16=1, form=1)
+    want = O.to_bf16(x).astype(np.float64) @ w.T.astype(np.float64) + b
+    want = (np.maximum(want, 0) ** 2 if act else want) + res
+    assert np.abs(got - want).max() <= 3e-5 * max(1.0, np.abs(want).max())
+
+
 @pytest.mark.parametrize("rows,start", [(1, 0), (1, 5), (6, 0), (9, 3)])
 def test_dyn_tanh_and_token_shift_with_state(hip_ctx, rows, start):
     rng = np.random.default_rng(rows + start)
@@ -192,3 +205,24 @@ def test_grouped_expert_form_equals_the_per_row_form(hip_ctx, rows, routed, iden
                   C.c_uint32(ff), C.c_uint32(routed), C.c_uint32(identity), C.c_uint32(top), C.c_uint32(mode))
         outs.append(y)
     assert np.isfinite(outs[1]).all() and np.abs(outs[0] - outs[1]).max() < 2e-4 * max(1.0, np.abs(outs[0]).max())
+
+
+@pytest.mark.parametrize("rows,routed,identity,top,ff,d", [(700, 5, 1, 2, 1088, 1024), (1030, 64, 0, 1, 1024, 1024)])
+def test_grouped_expert_form_prompt_sized(hip_ctx, rows, routed, identity, top, ff, d):
+    """... at sizes whose operands go by LDS DMA: the gated product in the first product's epilogue, odd and many buckets (the most that form takes), a hidden width that is no whole
+    tile.  The forms sum in other orders, so a hidden value h can round to the neighbouring bf16: a result then moves by 2^-8 |h| |w| of its down weight, a few of which may meet."""
+    rng = np.random.default_rng(rows)
+    x, wr = f32(rng.standard_normal((rows, d))), O.to_bf16(rng.standard_normal((routed + identity, d)) * 0.5)
+    corr, res = f32(0.1 * rng.standard_normal(routed + identity)), f32(rng.standard_normal((rows, d)))
+    w13 = O.to_bf16(rng.standard_normal((routed, 2 * ff, d), dtype=np.float32) / np.float32(np.sqrt(d)))
+    w2 = O.to_bf16(rng.standard_normal((routed, d, ff), dtype=np.float32) / np.float32(np.sqrt(ff)))
+    b13, b2, outs = O.bf16_bits(w13), O.bf16_bits(w2), []
+    for mode in (1, 2):
+        y, ids, wts = np.empty((rows, d), dtype=np.float32), np.empty((rows, top), dtype=np.int32), np.empty((rows, top), dtype=np.float32)
+        _ffi.call("uzu_hip_s32_moe", hip_ctx._h, ptr(x), ptr(O.bf16_bits(wr)), ptr(corr), ptr(b13), ptr(b2), ptr(res), ptr(y), ptr(ids), ptr(wts), C.c_uint32(rows), C.c_uint32(d),
+                  C.c_uint32(ff), C.c_uint32(routed), C.c_uint32(identity), C.c_uint32(top), C.c_uint32(mode))
+        outs.append(y)
+    up, gate = np.split(O.to_bf16(x[:64]) @ w13[0].T, 2, axis=1)
+    h = np.abs(gate / (1 + np.exp(-gate)) * up).max()
+    assert np.isfinite(outs[1]).all() and np.abs(outs[0] - outs[1]).max() < 2 * 2.0 ** -8 * h * np.abs(w2).max()
+    assert np.linalg.norm(outs[0] - outs[1]) < 1e-4 * np.linalg.norm(outs[0])

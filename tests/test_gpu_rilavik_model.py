@@ -83,6 +83,17 @@ def in_portions(m, toks, cuts):
     return np.concatenate(rows)
 
 
+def test_prompt_sized_experts_read_their_weighted_input(hip_ctx, tmp_path):
+    """A prompt long enough for the experts' LDS-DMA form (the score multiplies gate and up sums in the product's epilogue) against the same prompt in portions that stay in the
+    other forms: the same bf16 operands and f32 sums, so the logits differ by the order of f32 sums and the few operands that rounds over (measured 0)."""
+    cfg = O.config(vocab=64, width=512, layers=[O.gla_layer(2, 32, 32, tau=8.0, rank=8, mlp=O.moe(4, 2, 512))])
+    _, m = make(hip_ctx, tmp_path, cfg, 5, flags=0, ctx_len=2048)
+    toks = prompt(cfg, 1950, 6)
+    whole, parts = in_portions(m, toks, [1950]), in_portions(m, toks, [500, 500, 500, 450])
+    assert np.median(O.logit_error(whole, parts)) < 1e-3 and np.mean(O.logit_error(whole, parts) < 1e-2) > 0.99
+    m.close()
+
+
 @pytest.mark.parametrize("name", ["a", "b"])
 @pytest.mark.parametrize("full", [True, False])
 def test_whole_prompt_every_position_and_every_layer(models, name, full):

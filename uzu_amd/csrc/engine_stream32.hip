@@ -1344,7 +1344,7 @@ uzu_status s32_create(uzu_hip_context* ctx, const uzu_model_desc* desc, uint32_t
 void s32_destroy(uzu_hip_model* m) {
     if (m->s32->side) {
         (void)hipStreamSynchronize(m->s32->side);
-        (void)hipStreamDestroy(m->s32->side);
+        k::stream_workspace_release(m->s32->side), (void)hipStreamDestroy(m->s32->side);
     }
     if (m->s32->side_fork) (void)hipEventDestroy(m->s32->side_fork);
     if (m->s32->side_join) (void)hipEventDestroy(m->s32->side_join);

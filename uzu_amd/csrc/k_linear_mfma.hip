@@ -10,6 +10,8 @@
 // grid.z batches independent products of one shape (the per-head products of the latent attention).
 #include "device_utils.h"
 #include "gemm_convert.h"
+#include "gemm_tile_map.h"
+#include "kernels.h"
 #include "kernels_stream32.h"
 #include "stream32_epilogue.h"
 
@@ -163,6 +165,204 @@ __global__ void __launch_bounds__(256, MB * NB == 4 && KIND != kEpilogueFull ? 3
     }
 }
 
+
+// ---- prompt-sized products: both operands as bf16 rows in memory, fetched straight into LDS
+// The activations are rounded to bf16 once, in front (linear_bf16_rows, or the producing kernel), instead of by every column of tiles: the kernel above spends its
+// k-step on that conversion and on the operands' way through registers (2048 x 7712 x 2048: 158 us, 409 TFLOP/s), with one buffer and two barriers per k-step.
+// Here a workgroup of four waves (2 x 2, a wave 32 MB x 64 outputs) takes its 64-deep k-steps by global_load_lds_dwordx4 (1 KB a wave-instruction, no registers).
+// A staged row is 64 k = 128 bytes = eight 16-byte chunks; chunk c of row r lies in slot c ^ (r & 7) -- the lane picks the chunk it fetches, the DMA stores lane by
+// lane -- so the eight rows that a quarter-wave reads at one k fall on eight different slots.
+// What bounds it is the wait for a k-step's operands, so the forms differ in who covers it (measured, us, conversion included):
+//   * 128-row tiles, ONE buffer, 32 KB: four workgroups per CU cover each other.  Best from two tiles a CU on: 2048 x 16384 x 2048 183 (two buffers 211),
+//     eight buckets of 4096 rows x 4096 x 2048 105 (111), x 2048 59 (67);
+//   * 128-row tiles, two buffers, two workgroups per CU, the next step on its way during a step: 513 x 8192 x 2048 45 (one buffer 52);
+//   * 64-row tiles, two buffers, three workgroups per CU: at most a 128-row tile a CU: 2048 x 2048 x 4096 58 (128-row tiles 64), 1000 x 3856 x 1024 27 (32).
+// Wider tiles (256 x 128), 32-deep steps and a third buffer were all slower.
+constexpr int DN = 128;
+
+// PIECES KB-pieces from base + v[i] (16 bytes a lane) to dst + 1024 i + 16 lane
+template <int PIECES> __device__ __forceinline__ void dma16(const void* base, const uint32_t (&v)[PIECES], uint32_t dst) {
+    uint32_t keep;
+    if constexpr (PIECES == 2)
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                     "global_load_lds_dwordx4 %3, %1\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
+                     "global_load_lds_dwordx4 %4, %1\n\ts_mov_b32 m0, %0"
+                     : "=&s"(keep) : "s"(base), "s"(dst), "v"(v[0]), "v"(v[1]) : "memory", "scc");
+    else {
+        static_assert(PIECES == 4, "two or four pieces");
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                     "global_load_lds_dwordx4 %3, %1\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
+                     "global_load_lds_dwordx4 %4, %1\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
+                     "global_load_lds_dwordx4 %5, %1\n\ts_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
+                     "global_load_lds_dwordx4 %6, %1\n\ts_mov_b32 m0, %0"
+                     : "=&s"(keep) : "s"(base), "s"(dst), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]) : "memory", "scc");
+    }
+}
+
+constexpr int kEpilogueGated = 16; // grouped experts: the weight rows are [up ; gate], the result act(gate, up) as bf16 rows (GatedRows)
+
+template <int MB, int STAGES, bool GROUPED, int KIND>
+__global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, const uint16_t* xb, uint32_t ldxb, GatedRows gr) {
+    constexpr bool GATED = KIND == kEpilogueGated;
+    constexpr int DK = 64, DM = 64 * MB, AP = DM * DK * 2 / 4096, BP = DN * DK * 2 / 4096; // 1 KB pieces per wave: A, B
+    constexpr uint32_t STAGE = (DM + DN) * DK * 2, ROW = DK * 2, CHUNKS = DK / 8, RPP = 1024 / ROW; // row bytes, 16-byte chunks per row, rows per piece
+    extern __shared__ __attribute__((aligned(1024))) uint8_t s_dma[];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1, l32 = lane & 31, half = lane >> 5;
+    uint32_t r_lo = 0, r_hi = p.rows, m_t, n_t, z = 0;
+    if (GROUPED) { // tiles of the buckets back to back: the wave's lanes hold the buckets' tile counts (batch <= 64)
+        const uint32_t lo = lane < p.batch ? p.row_offsets[lane] : 0u, hi = lane < p.batch ? p.row_offsets[lane + 1] : 0u;
+        uint32_t upto = (hi - lo + DM - 1) / DM;
+        for (uint32_t o = 1; o < 64; o <<= 1) {
+            const uint32_t below = __shfl_up(upto, o, 64);
+            if (lane >= o) upto += below;
+        }
+        const unsigned long long behind = __ballot(upto > blockIdx.y);
+        if (!behind) return; // (workgroup-uniform, in front of every barrier)
+        z = (uint32_t)__builtin_ctzll(behind);
+        r_lo = __builtin_amdgcn_readlane(lo, z), r_hi = __builtin_amdgcn_readlane(hi, z);
+        const uint32_t first = z ? __builtin_amdgcn_readlane(upto, z - 1) : 0u;
+        m_t = blockIdx.y - first, n_t = blockIdx.x;
+    } else {
+        if (!gemm_tile_of_block(blockIdx.x, (p.rows + DM - 1) / DM, (p.n + DN - 1) / DN, &m_t, &n_t)) return;
+    }
+    const uint32_t m0 = r_lo + m_t * DM, n0 = n_t * DN;
+    const uint16_t* w = p.w + (size_t)z * p.w_batch;
+
+    // this wave's pieces of a k-step; rows outside are read from inside (never stored)
+    uint32_t va[AP], vb[BP];
+#pragma unroll
+    for (int i = 0; i < AP; ++i) {
+        const uint32_t row = (wave * AP + i) * RPP + lane / CHUNKS, chunk = (lane % CHUNKS) ^ (row & 7);
+        const uint32_t m = m0 + row < r_hi ? m0 + row : r_hi - 1;
+        va[i] = (GROUPED && p.row_map ? p.row_map[m] : m) * ldxb * 2 + chunk * 16;
+    }
+#pragma unroll
+    for (int i = 0; i < BP; ++i) {
+        const uint32_t row = (wave * BP + i) * RPP + lane / CHUNKS, chunk = (lane % CHUNKS) ^ (row & 7);
+        uint32_t n = n0 + row;
+        if (GATED) { // a wave's first 32 columns are up rows, its second 32 the gate rows of the same outputs: the pair meets in one lane
+            const uint32_t ff = p.n / 2, f = n_t * 64 + (row >> 6) * 32 + (row & 31);
+            n = (f < ff ? f : ff - 1) + (row & 32 ? ff : 0);
+        } else if (n >= p.n) n = p.n - 1;
+        vb[i] = n * p.k * 2 + chunk * 16;
+    }
+    const uint32_t lds0 = (uint32_t)(uintptr_t)s_dma;
+    auto fetch = [&](uint32_t kt, uint32_t buf) {
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * STAGE + wave * AP * 1024), dst_b = __builtin_amdgcn_readfirstlane(lds0 + buf * STAGE + DM * ROW + wave * BP * 1024);
+        dma16<AP>(xb + kt * DK, va, dst);
+        dma16<BP>(w + kt * DK, vb, dst_b);
+    };
+
+    f32x16_t acc[MB][2];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (row_map: nothing of the compiler's is in flight from here on)
+    const uint32_t steps = p.k / DK;
+    if (STAGES == 2) fetch(0, 0);
+    const uint32_t a_base = (wm * 32 * MB + l32) * ROW, b_base = DM * ROW + (wn * 64 + l32) * ROW, key = l32 & 7;
+    for (uint32_t kt = 0; kt < steps; ++kt) {
+        if constexpr (STAGES == 1) {
+            if (kt) lds_barrier(); // every wave has read step kt - 1
+            fetch(kt, 0);
+            asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); // step kt is in LDS
+        } else { // step kt is in LDS and every wave has read step kt - 1: the next step may land in its place
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (kt + 1 < steps) fetch(kt + 1, (kt + 1) & 1);
+        }
+        const uint8_t* at = s_dma + (STAGES == 1 ? 0 : (kt & 1)) * STAGE;
+#pragma unroll
+        for (uint32_t s = 0; s < DK / 16; ++s) {
+            const uint32_t slot = ((2 * s + half) ^ key) * 16;
+            u32x4_t af[MB], bf[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) bf[j] = *(const u32x4_t*)(at + b_base + j * 32 * ROW + slot);
+#pragma unroll
+            for (int i = 0; i < MB; ++i) af[i] = *(const u32x4_t*)(at + a_base + i * 32 * ROW + slot);
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, af[i]), __builtin_bit_cast(bf16x8_t, bf[j]), acc[i][j], 0, 0, 0);
+        }
+    }
+
+    if constexpr (GATED) {
+        const uint32_t ff = p.n / 2, f = n_t * 64 + wn * 32 + l32;
+        if (f >= ff) return;
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t row = m0 + (wm * MB + i) * 32 + 4 * half + (r & 3) + 8 * (r >> 2);
+                if (row >= r_hi) continue;
+                const float wt = gr.row_weight ? gr.row_weight[row] : 1.0f;
+                gr.out[(size_t)row * ff + f] = f32_to_bf16(expert_act(wt * acc[i][1][r], wt * acc[i][0][r], gr.act));
+            }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const uint32_t n = n0 + (wn * 2 + j) * 32 + l32;
+        if (n >= p.n) continue;
+        const float bias = p.bias ? bf16_to_f32(p.bias[n]) : 0.0f;
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+            const uint32_t row0 = m0 + (wm * MB + i) * 32 + 4 * half;
+            float res[16]; // (the residual may be y itself: a block's rows are read before any of them is stored)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t row = row0 + (r & 3) + 8 * (r >> 2);
+                res[r] = p.residual && row < r_hi ? p.residual[(size_t)row * p.ldr + n] : 0.0f;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t row = row0 + (r & 3) + 8 * (r >> 2);
+                if (row >= r_hi) continue;
+                const float v = linear_value<KIND>(acc[i][j][r], bias, p, row, z, n);
+                p.y[(size_t)row * p.ldy + n] = p.residual ? v + res[r] : v;
+            }
+        }
+    }
+}
+
+// f32 rows -> bf16 rows, round to nearest even: what the product's operand is
+__global__ void __launch_bounds__(256) linear_bf16_rows_kernel(const float* x, uint32_t ldx, uint16_t* out, uint32_t k, size_t chunks) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; // chunk of 8
+    if (i >= chunks) return;
+    const uint32_t per_row = k / 8;
+    const size_t r = i / per_row;
+    const uint32_t c = (uint32_t)(i - r * per_row) * 8;
+    const f32x4_v a = *(const f32x4_v*)(x + r * ldx + c), b = *(const f32x4_v*)(x + r * ldx + c + 4);
+    u32x4_v o;
+    o.x = pack_bf16(a.x, a.y), o.y = pack_bf16(a.z, a.w), o.z = pack_bf16(b.x, b.y), o.w = pack_bf16(b.z, b.w);
+    *(u32x4_v*)(out + i * 8) = o;
+}
+
+template <int MB, int STAGES, bool GROUPED, int KIND> uzu_status launch_dma_tile(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, uint32_t ldxb, const GatedRows& gr) {
+    const uint32_t m_tiles = (p.rows + 64 * MB - 1) / (64 * MB), n_tiles = (p.n + DN - 1) / DN;
+    const dim3 grid = GROUPED ? dim3(n_tiles, m_tiles + p.batch) : dim3(gemm_grid_x(m_tiles, n_tiles));
+    UZU_REQUIRE(grid.y <= 65535, "linear_dma: grid too large");
+    const size_t lds = (size_t)STAGES * (64 * MB + DN) * 64 * 2;
+    static LdsLimit lim;
+    UZU_REQUIRE(raise_lds_limit(lim, (const void*)linear_dma_kernel<MB, STAGES, GROUPED, KIND>, lds), "linear_dma: %zu bytes of LDS are not available", lds);
+    return launch_check([&] { hipLaunchKernelGGL((linear_dma_kernel<MB, STAGES, GROUPED, KIND>), grid, dim3(256), lds, s, p, xb, ldxb, gr); }, "linear_dma");
+}
+template <bool GROUPED, int KIND> uzu_status launch_dma(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, uint32_t ldxb, const GatedRows& gr = GatedRows()) {
+    const size_t tiles = (size_t)((p.rows + 127) / 128) * ((p.n + DN - 1) / DN);
+    if (tiles >= 512) return launch_dma_tile<2, 1, GROUPED, KIND>(s, p, xb, ldxb, gr);
+    if (tiles > 256) return launch_dma_tile<2, 2, GROUPED, KIND>(s, p, xb, ldxb, gr);
+    return launch_dma_tile<1, 2, GROUPED, KIND>(s, p, xb, ldxb, gr);
+}
+
+// Prompt-sized shapes with whole k-steps.  (A product below a GFLOP or two ends inside the launch and the conversion in front of it: those stay above.)
+bool dma_shape(uint32_t rows, uint32_t n, uint32_t k) { return rows >= 128 && n >= 64 && k % 64 == 0 && 2e-9 * rows * n * k >= 2.0; }
+bool dma_range(uint32_t rows, uint32_t n, uint32_t k) { return (uint64_t)rows * k * 2 < 1ull << 32 && (uint64_t)n * k * 2 < 1ull << 32; } // 32-bit byte offsets
+
 template <int MB, int NB> uzu_status launch(hipStream_t s, const LinearF32Params& p, const char* what) {
     const dim3 grid((p.n + 64 * NB - 1) / (64 * NB), (p.rows + 64 * MB - 1) / (64 * MB), p.batch);
     UZU_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "linear_mfma: grid too large");
@@ -182,9 +382,32 @@ bool linear_mfma_supported(const LinearF32Params& p) {
     return true;
 }
 
+uzu_status linear_bf16_rows(hipStream_t s, const float* x, uint32_t ldx, uint16_t* out, uint32_t rows, uint32_t k) {
+    const size_t chunks = (size_t)rows * (k / 8);
+    UZU_REQUIRE(k % 8 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0, "linear_bf16_rows: alignment");
+    return launch_check([&] { hipLaunchKernelGGL(linear_bf16_rows_kernel, dim3((uint32_t)((chunks + 255) / 256)), dim3(256), 0, s, x, ldx, out, k, chunks); }, "linear_bf16_rows");
+}
+bool linear_dma_grouped_supported(const LinearF32Params& p) {
+    return linear_mfma_supported(p) && p.row_offsets && p.batch <= 64 && !p.residual && epilogue_kind(p) == kEpilogueLean && dma_shape(p.rows, p.n, p.k) && dma_range(p.rows, p.n, p.k);
+}
+uzu_status linear_dma_grouped(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, uint32_t ldxb, const GatedRows* gated) {
+    UZU_REQUIRE(linear_dma_grouped_supported(p) && ((uintptr_t)xb & 15) == 0 && ldxb % 8 == 0 && ldxb >= p.k && (!gated || (gated->out && p.n % 2 == 0 && !p.bias)), "linear_dma_grouped: shape / alignment not covered");
+    return gated ? launch_dma<true, kEpilogueGated>(s, p, xb, ldxb, *gated) : launch_dma<true, kEpilogueLean>(s, p, xb, ldxb);
+}
+
 uzu_status linear_mfma(hipStream_t s, const LinearF32Params& p) {
     UZU_REQUIRE(linear_mfma_supported(p), "linear_mfma: shape / alignment not covered");
     UZU_REQUIRE(p.row_offsets || !p.row_map, "linear_mfma: gathered rows only in the grouped form");
+    if (!p.row_offsets && p.batch == 1 && dma_shape(p.rows, p.n, p.k) && dma_range(p.rows, p.n, p.k)) {
+        if (uint16_t* xb = (uint16_t*)stream_workspace(s, (size_t)p.rows * p.k * 2)) { // (none while the stream is captured)
+            UZU_PROPAGATE(linear_bf16_rows(s, p.x, p.ldx, xb, p.rows, p.k));
+            switch (epilogue_kind(p)) {
+            case kEpilogueLean: return launch_dma<false, kEpilogueLean>(s, p, xb, p.k);
+            case kEpilogueXielu: return launch_dma<false, kEpilogueXielu>(s, p, xb, p.k);
+            default: return launch_dma<false, kEpilogueFull>(s, p, xb, p.k);
+            }
+        }
+    }
     // tile choice: the widest tile that still fills the chip; narrow outputs (the per-head products) take the narrow tiles
     if (p.row_offsets) { // grouped: every product may need the whole row range, the workgroups beyond a bucket leave at once
         const dim3 grid((p.n + 127) / 128, (p.rows + 127) / 128 + 1, p.batch);

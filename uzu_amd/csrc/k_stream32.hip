@@ -4,6 +4,7 @@
 // reads f32 activation rows and bf16 weights; with `bf16_products` the activation operand is rounded to bf16 as it is loaded (what a bf16 activation buffer
 // would have held), otherwise the product is a true f32 product.  Reductions run in a fixed order: a result does not depend on what else is in the pass.
 #include "device_utils.h"
+#include "kernels.h"
 #include "kernels_stream32.h"
 #include "stream32_epilogue.h"
 
@@ -218,11 +219,6 @@ __global__ void __launch_bounds__(256) depth_mix_kernel(const float* slots, size
     out[i] = acc;
 }
 
-__device__ __forceinline__ float expert_act(float gate, float up, const ExpertAct& a) {
-    const float g = fminf(fmaxf(gate, a.gate_min), a.gate_max), u = fminf(fmaxf(up, a.up_min), a.up_max);
-    if (a.gelu) return gelu_tanh_f32(g) * (u + a.up_offset);
-    return g / (1.0f + expf(-(a.alpha * g))) * (u + a.up_offset);
-}
 
 // thread = (row, hidden unit): a one-row decode step still spreads over ff / 256 workgroups
 __global__ void __launch_bounds__(256) gated_act_rows_kernel(const float* y1, float* hidden, uint32_t ff, ExpertAct act) {
@@ -674,17 +670,27 @@ uzu_status moe_experts_grouped(hipStream_t s, const MoeGroupedParams& p) {
     UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(moe_bucket_kernel, dim3(1), dim3(1024), (size_t)p.routed * 4, s, p.ids, slots, p.routed, p.offsets, p.cursor); }, "moe_bucket"));
     UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(moe_scatter_kernel, dim3((slots + 255) / 256), dim3(256), (size_t)p.routed * 4, s, p.ids, slots, p.routed, p.top, p.offsets, p.cursor, p.perm, p.slot_pos, p.weights, p.pos_weight); },
                                "moe_scatter"));
-    LinearF32Params q{};
+    LinearF32Params q{}, r{};
     const uint32_t n1 = p.act.plain ? p.ff : 2 * p.ff;
     q.x = p.x, q.w = p.w13, q.y = p.y1, q.rows = slots, q.n = n1, q.k = p.d, q.ldx = p.d, q.ldy = n1, q.batch = p.routed, q.w_batch = (size_t)n1 * p.d;
     q.bf16_products = 1, q.row_offsets = p.offsets, q.row_map = p.perm;
     if (p.act.plain) q.y = p.hidden, q.act = 1; // no gate: the activation rides in the product's epilogue
-    UZU_PROPAGATE(linear_mfma(s, q));
-    if (!p.act.plain) UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(moe_act_mul_kernel, dim3(slots), dim3(256), 0, s, p.y1, p.hidden, p.offsets, p.routed, p.ff, p.act, p.pos_weight); }, "moe_act_mul"));
-    LinearF32Params r{};
     r.x = p.hidden, r.w = p.w2, r.y = p.y2, r.rows = slots, r.n = p.d, r.k = p.ff, r.ldx = p.ff, r.ldy = p.d, r.batch = p.routed, r.w_batch = (size_t)p.d * p.ff;
     r.bf16_products = 1, r.row_offsets = p.offsets;
-    UZU_PROPAGATE(linear_mfma(s, r));
+    // prompt-sized: the rows as bf16 once, the gated product in the first product's epilogue, its rows as the bf16 operand of the second
+    const size_t xb_bytes = ((size_t)p.rows * p.d * 2 + 255) / 256 * 256;
+    uint16_t* xb = linear_dma_grouped_supported(q) && linear_dma_grouped_supported(r) && !p.act.plain ? (uint16_t*)stream_workspace(s, xb_bytes + (size_t)slots * p.ff * 2) : nullptr;
+    if (xb) {
+        GatedRows gr;
+        gr.out = (uint16_t*)((char*)xb + xb_bytes), gr.row_weight = p.pos_weight, gr.act = p.act;
+        UZU_PROPAGATE(linear_bf16_rows(s, p.x, p.d, xb, p.rows, p.d));
+        UZU_PROPAGATE(linear_dma_grouped(s, q, xb, p.d, &gr));
+        UZU_PROPAGATE(linear_dma_grouped(s, r, gr.out, p.ff));
+    } else {
+        UZU_PROPAGATE(linear_mfma(s, q));
+        if (!p.act.plain) UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(moe_act_mul_kernel, dim3(slots), dim3(256), 0, s, p.y1, p.hidden, p.offsets, p.routed, p.ff, p.act, p.pos_weight); }, "moe_act_mul"));
+        UZU_PROPAGATE(linear_mfma(s, r));
+    }
     return launch_check([&] { hipLaunchKernelGGL(moe_combine_kernel, dim3(p.rows), dim3(256), 0, s, p.y2, p.x, p.ids, p.pos_weight ? nullptr : p.weights, p.slot_pos, p.residual, p.y, p.d, p.routed, p.top); },
                         "moe_combine");
 }

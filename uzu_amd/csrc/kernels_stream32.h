@@ -121,6 +121,12 @@ uzu_status linear_f32(hipStream_t s, const LinearF32Params& p, const char** vari
 // the matrix-core form (k_linear_mfma.hip): bf16 products only; false = shape / mode not covered, nothing launched
 bool linear_mfma_supported(const LinearF32Params& p);
 uzu_status linear_mfma(hipStream_t s, const LinearF32Params& p);
+// f32 rows (pitch ldx) rounded to bf16, rows of k packed; and the grouped product of rows that are bf16 already (X of `p` unused: row r is xb[row_map ? row_map[r] : r];
+// xb has no more rows than p.rows).  gated: W is [up ; gate] and the result act(gate, up) of every row and hidden unit, as bf16 rows (Y unused).
+struct GatedRows;
+uzu_status linear_bf16_rows(hipStream_t s, const float* x, uint32_t ldx, uint16_t* out, uint32_t rows, uint32_t k);
+bool linear_dma_grouped_supported(const LinearF32Params& p);
+uzu_status linear_dma_grouped(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, uint32_t ldxb, const GatedRows* gated = nullptr);
 size_t linear_f32_bytes(const LinearF32Params& p);
 
 // Score routing: per row scores = softmax(router x) over all `outputs` (= routed + identity) in f32, the `top` largest (score + bias) win (ties: lower index),
@@ -151,6 +157,12 @@ uzu_status moe_route_groups(hipStream_t s, const RouteGroupsParams& p);
 struct ExpertAct {
     float alpha = 1.0f, gate_min = -INFINITY, gate_max = INFINITY, up_min = -INFINITY, up_max = INFINITY, up_offset = 0.0f;
     uint32_t gelu = 0, plain = 0;
+};
+// out[r, f] = bf16(act(w_r gate, w_r up)), bf16 rows of ff; row_weight f32 [rows] or null (1)
+struct GatedRows {
+    uint16_t* out = nullptr;
+    const float* row_weight = nullptr;
+    ExpertAct act;
 };
 // The gated product of a dense block: hidden[r, f] = act(gate = y1[r, ff + f], up = y1[r, f])   (y1 f32 [rows][2 ff]: up rows first, as the packed projection yields them)
 uzu_status gated_act_rows(hipStream_t s, const float* y1, float* hidden, uint32_t rows, uint32_t ff, const ExpertAct& act);

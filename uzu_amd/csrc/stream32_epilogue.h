@@ -10,6 +10,12 @@ namespace k {
 
 __device__ __forceinline__ float gelu_tanh_f32(float z) { return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))); }
 
+__device__ __forceinline__ float expert_act(float gate, float up, const ExpertAct& a) {
+    const float g = fminf(fmaxf(gate, a.gate_min), a.gate_max), u = fminf(fmaxf(up, a.up_min), a.up_max);
+    if (a.gelu) return gelu_tanh_f32(g) * (u + a.up_offset);
+    return g / (1.0f + expf(-(a.alpha * g))) * (u + a.up_offset);
+}
+
 // The matrix-core form unrolls its epilogue over 64 sums per thread: one kernel with every branch inlined 64 times does not fit the instruction cache, so it is
 // compiled for what a launch uses.
 enum EpilogueKind {
