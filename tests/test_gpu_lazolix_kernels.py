@@ -56,7 +56,7 @@ def test_linear_matrix_core_form_equals_the_plain_form(hip_ctx, rows, n, k, batc
     assert np.abs(a - want).max() <= 3e-5 * max(1.0, np.abs(want).max()) and np.abs(c - want).max() <= 3e-5 * max(1.0, np.abs(want).max())
 
 
-@pytest.mark.parametrize("rows,n,k,act", [(129, 8200, 1024, 0), (1000, 1025, 1024, 1), (255, 16400, 256, 0), (513, 8192, 256, 0), (2050, 4100, 128, 1), (128, 4100, 2048, 0)])
+@pytest.mark.parametrize("rows,n,k,act", [(129, 8200, 1024, 0), (1000, 1025, 1024, 1), (255, 16400, 256, 0), (513, 8192, 256, 0), (2050, 4100, 128, 1), (128, 4100, 2048, 0), (33, 1024, 1024, 1), (300, 700, 2048, 0)])
 def test_linear_prompt_sized_form(hip_ctx, rows, n, k, act):
     """Prompt-sized products (both operands by LDS DMA): every tile form and buffer count, ragged last tiles in both directions, two k-steps and many, bias, activation and a residual
     in place; f32 sums of bf16 products, so the bound of the other matrix-core form holds."""
@@ -67,6 +67,33 @@ def test_linear_prompt_sized_form(hip_ctx, rows, n, k, act):
     want = O.to_bf16(x).astype(np.float64) @ w.T.astype(np.float64) + b
     want = (np.maximum(want, 0) ** 2 if act else want) + res
     assert np.abs(got - want).max() <= 3e-5 * max(1.0, np.abs(want).max())
+
+
+@pytest.mark.parametrize("rows,n,k,act", [(17, 1500, 1024, 0), (33, 1025, 832, 1), (17, 70, 256, 0), (129, 4101, 64, 0), (300, 1024, 2048, 1), (64, 64, 8192, 0), (1025, 4100, 128, 0), (2050, 4100, 64, 0)])
+def test_linear_f32_from_three_bf16_parts(hip_ctx, rows, n, k, act):
+    """f32 products of many rows (each operand number as three bf16 numbers): against 64 bits, with numbers of mixed sizes; every tile form, the product cut along k, ragged last
+    tiles.  f32 accumulation of 3 k exact products: each addition rounds a partial sum that is at most sum |x w| by 2^-24, and errors of k steps add like sqrt(k) (factor 4 of room)."""
+    rng = np.random.default_rng(rows + n)
+    x = f32(rng.standard_normal((rows, k)) * np.exp2(rng.integers(-12, 13, (rows, k))))
+    w, b, res = O.to_bf16(rng.standard_normal((n, k), dtype=np.float32)), O.to_bf16(rng.standard_normal(n)), rng.standard_normal((rows, n), dtype=np.float32)
+    got = linear(hip_ctx, x, w, b, res, act=act, bf16=0)
+    lin = x.astype(np.float64) @ w.T.astype(np.float64) + b
+    mass = np.abs(x.astype(np.float64)) @ np.abs(w.T.astype(np.float64)) + np.abs(b)
+    bound = 4 * 2.0 ** -24 * np.sqrt(3 * k) * mass
+    if act:
+        bound = 2 * np.maximum(lin, 0) * bound + bound ** 2 + 2.0 ** -23 * lin ** 2
+    want = (np.maximum(lin, 0) ** 2 if act else lin) + res
+    assert (np.abs(got - want) <= bound + 2.0 ** -23 * (np.abs(want) + np.abs(res))).all()
+
+
+def test_linear_f32_parts_keep_infinities_and_nans(hip_ctx):
+    rng = np.random.default_rng(3)
+    x, w = rng.standard_normal((40, 1024), dtype=np.float32), O.to_bf16(np.abs(rng.standard_normal((700, 1024), dtype=np.float32)) + 0.5)
+    x[3, 5], x[7, 900], x[11, 0], x[20, 1] = np.inf, -np.inf, np.nan, 3.4e38
+    w[:, 1] = 1.0
+    got = linear(hip_ctx, x, w, act=0, bf16=0)
+    assert np.isposinf(got[3]).all() and np.isneginf(got[7]).all() and np.isnan(got[11]).all() and np.isfinite(np.delete(got, [3, 7, 11], 0)).all()
+    assert np.abs(got[20] - 3.4e38).max() <= 3.4e38 * 2.0 ** -22
 
 
 @pytest.mark.parametrize("rows,start", [(1, 0), (1, 5), (6, 0), (9, 3)])

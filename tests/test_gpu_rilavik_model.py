@@ -94,6 +94,20 @@ def test_prompt_sized_experts_read_their_weighted_input(hip_ctx, tmp_path):
     m.close()
 
 
+def test_f32_experts_of_a_prompt_from_bf16_parts(hip_ctx, tmp_path):
+    """f32 experts of 32 rows and more (grouped products from three bf16 parts; buckets of one row to many) against the same prompt in portions of under 32 rows, which take the
+    row kernels: both are f32 products with f32 sums, so the logits differ by the order of the sums."""
+    cfg = O.config(vocab=64, width=128, layers=[O.gla_layer(2, 32, 32, tau=8.0, rank=8, mlp=O.moe(16, 3, 192))])
+    W, m = make(hip_ctx, tmp_path, cfg, 5, ctx_len=512)
+    toks = prompt(cfg, 200, 6)
+    whole, parts = in_portions(m, toks, [200]), in_portions(m, toks, [20] * 10)
+    some = in_portions(m, toks, [33, 31, 136])
+    assert rows_ok(O.logit_error(whole, parts), True) and rows_ok(O.logit_error(some, parts), True)
+    want, _ = O.forward(cfg, W, toks)
+    assert rows_ok(O.logit_error(whole, want), True)
+    m.close()
+
+
 @pytest.mark.parametrize("name", ["a", "b"])
 @pytest.mark.parametrize("full", [True, False])
 def test_whole_prompt_every_position_and_every_layer(models, name, full):

@@ -639,7 +639,8 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
                 gp.x = mlp_in, gp.ids = S.moe_ids, gp.weights = S.moe_w, gp.w13 = L.moe.w13, gp.w2 = L.moe.w2, gp.residual = res, gp.y = moe_out, gp.y1 = S.moe_y1, gp.hidden = S.hid;
                 gp.y2 = S.moe_y2, gp.perm = S.moe_perm, gp.slot_pos = S.moe_slot_pos, gp.offsets = S.moe_offsets, gp.cursor = S.moe_cursor;
                 gp.rows = rows, gp.d = d, gp.ff = ff, gp.routed = E, gp.top = top, gp.act = act, gp.pos_weight = on_input ? S.moe_pos_w : nullptr;
-                if (bf && k::moe_experts_grouped_supported(gp)) { // prefill-sized: buckets per expert through the matrix-core linear
+                gp.f32_products = bf ? 0 : 1;
+                if (k::moe_experts_grouped_supported(gp)) { // prefill-sized: buckets per expert through the matrix-core linear
                     RUN("moe_experts_grouped", (size_t)E * (act.plain ? 2 : 3) * ff * d * 2 + (size_t)rows * top * ((act.plain ? 1 : 3) * ff + 2 * d) * 4, k::moe_experts_grouped(s, gp));
                 } else {
                     RUN("moe_experts_gate_up", (size_t)rows * top * (act.plain ? 1 : 2) * ff * d * 2, k::moe_experts_gate_up(s, mlp_in, S.moe_ids, L.moe.w13, S.hid, rows, d, ff, E, top, bf, act, on_input ? S.moe_w : nullptr));
@@ -1262,11 +1263,11 @@ uzu_status s32_create(uzu_hip_context* ctx, const uzu_model_desc* desc, uint32_t
     if (w_dn_cv) TRY(need_f32(m, R * w_dn_cv, &S.dn_cv));
     if (w_dn_k) TRY(need_f32(m, R * w_dn_k, &S.dn_decay));
     if (w_dn_v) TRY(need_f32(m, R * w_dn_v, &S.dn_o));
-    if (w_pos && !S.full_f32) TRY(need_f32(m, R * w_pos, &S.moe_pos_w));
+    if (w_pos) TRY(need_f32(m, R * w_pos, &S.moe_pos_w));
     TRY(need_f32(m, R * w_top, &S.moe_w));
-    if (w_moe && !S.full_f32) { // workspaces of the grouped expert form (bf16 products only)
+    if (w_moe) { // workspaces of the grouped expert form
         void* q = nullptr;
-        TRY(need_f32(m, R * w_moe, &S.moe_y1));
+        if (!S.full_f32) TRY(need_f32(m, R * w_moe, &S.moe_y1));
         TRY(need_f32(m, R * w_top * d, &S.moe_y2));
         TRY(dev_alloc(m, R * w_top * 4, &q)); S.moe_perm = (uint32_t*)q;
         TRY(dev_alloc(m, R * w_top * 4, &q)); S.moe_slot_pos = (uint32_t*)q;

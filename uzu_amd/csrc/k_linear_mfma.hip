@@ -199,10 +199,24 @@ template <int PIECES> __device__ __forceinline__ void dma16(const void* base, co
     }
 }
 
+// f32 products on the same matrix cores: an f32 number is three bf16 numbers, x = hi + mid + lo exactly (8 + 8 + 8 significant bits, each part the truncation of what the
+// parts before it leave), weights are bf16 already, and a product of two bf16 numbers is exact in f32: the sum over 3 k products, the small parts first, is a sum of the
+// f32 products' own bits with f32 accumulation.  Three bf16 products are five times the rate of the f32 matrix instructions.  (Parts below 2^-126 may be flushed;
+// infinities and NaNs stay in hi.)
+__device__ __forceinline__ void split_bf16(float x, uint16_t& hi, uint16_t& mid, uint16_t& lo) {
+    const uint32_t u = f32_to_bits(x);
+    const bool finite = (u & 0x7F800000u) != 0x7F800000u;
+    const float h = bits_to_f32(u & 0xFFFF0000u), r = x - h, m = bits_to_f32(f32_to_bits(r) & 0xFFFF0000u);
+    hi = finite ? (uint16_t)(u >> 16) : f32_to_bf16(x);
+    mid = finite ? (uint16_t)(f32_to_bits(m) >> 16) : (uint16_t)0;
+    lo = finite ? (uint16_t)(f32_to_bits(r - m) >> 16) : (uint16_t)0;
+}
+
 constexpr int kEpilogueGated = 16; // grouped experts: the weight rows are [up ; gate], the result act(gate, up) as bf16 rows (GatedRows)
 
-template <int MB, int STAGES, bool GROUPED, int KIND>
-__global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, const uint16_t* xb, uint32_t ldxb, GatedRows gr) {
+// parts: 1, or 3 for operand rows [lo | mid | hi].  partials (not GROUPED): blockIdx.z takes its share of the k-steps and leaves its sums there, f32 [z][rows][n].
+template <int MB, int STAGES, bool GROUPED, int KIND, uint32_t parts>
+__global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, const uint16_t* xb, uint32_t ldxb, GatedRows gr, float* partials) {
     constexpr bool GATED = KIND == kEpilogueGated;
     constexpr int DK = 64, DM = 64 * MB, AP = DM * DK * 2 / 4096, BP = DN * DK * 2 / 4096; // 1 KB pieces per wave: A, B
     constexpr uint32_t STAGE = (DM + DN) * DK * 2, ROW = DK * 2, CHUNKS = DK / 8, RPP = 1024 / ROW; // row bytes, 16-byte chunks per row, rows per piece
@@ -247,10 +261,13 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
         vb[i] = n * p.k * 2 + chunk * 16;
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)s_dma;
-    auto fetch = [&](uint32_t kt, uint32_t buf) {
+    const uint32_t w_steps = p.k / DK, all = parts * w_steps;
+    const uint32_t t_lo = GROUPED ? 0u : all * blockIdx.z / gridDim.z, steps = (GROUPED ? all : all * (blockIdx.z + 1) / gridDim.z) - t_lo;
+    auto fetch = [&](uint32_t step, uint32_t buf) {
+        const uint32_t kt = t_lo + step, wt = parts == 1 ? kt : kt >= 2 * w_steps ? kt - 2 * w_steps : kt >= w_steps ? kt - w_steps : kt; // (the parts of a row meet the same weights)
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * STAGE + wave * AP * 1024), dst_b = __builtin_amdgcn_readfirstlane(lds0 + buf * STAGE + DM * ROW + wave * BP * 1024);
         dma16<AP>(xb + kt * DK, va, dst);
-        dma16<BP>(w + kt * DK, vb, dst_b);
+        dma16<BP>(w + wt * DK, vb, dst_b);
     };
 
     f32x16_t acc[MB][2];
@@ -262,7 +279,6 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (row_map: nothing of the compiler's is in flight from here on)
-    const uint32_t steps = p.k / DK;
     if (STAGES == 2) fetch(0, 0);
     const uint32_t a_base = (wm * 32 * MB + l32) * ROW, b_base = DM * ROW + (wn * 64 + l32) * ROW, key = l32 & 7;
     for (uint32_t kt = 0; kt < steps; ++kt) {
@@ -301,8 +317,29 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
                 const uint32_t row = m0 + (wm * MB + i) * 32 + 4 * half + (r & 3) + 8 * (r >> 2);
                 if (row >= r_hi) continue;
                 const float wt = gr.row_weight ? gr.row_weight[row] : 1.0f;
-                gr.out[(size_t)row * ff + f] = f32_to_bf16(expert_act(wt * acc[i][1][r], wt * acc[i][0][r], gr.act));
+                const float h = expert_act(wt * acc[i][1][r], wt * acc[i][0][r], gr.act);
+                if (parts == 1) gr.out[(size_t)row * ff + f] = f32_to_bf16(h);
+                else {
+                    uint16_t* o = gr.out + (size_t)row * 3 * ff + f;
+                    split_bf16(h, o[2 * ff], o[ff], o[0]);
+                }
             }
+        return;
+    }
+    if (!GROUPED && partials) {
+        float* out = partials + (size_t)blockIdx.z * p.rows * p.n;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t n = n0 + (wn * 2 + j) * 32 + l32;
+            if (n >= p.n) continue;
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const uint32_t row = m0 + (wm * MB + i) * 32 + 4 * half + (r & 3) + 8 * (r >> 2);
+                    if (row < r_hi) out[(size_t)row * p.n + n] = acc[i][j][r];
+                }
+        }
         return;
     }
 #pragma unroll
@@ -343,25 +380,83 @@ __global__ void __launch_bounds__(256) linear_bf16_rows_kernel(const float* x, u
     *(u32x4_v*)(out + i * 8) = o;
 }
 
-template <int MB, int STAGES, bool GROUPED, int KIND> uzu_status launch_dma_tile(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, uint32_t ldxb, const GatedRows& gr) {
+// ... and the rows [lo | mid | hi] of 3 k
+__global__ void __launch_bounds__(256) linear_split_rows_kernel(const float* x, uint32_t ldx, uint16_t* out, uint32_t k, size_t chunks) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; // chunk of 4
+    if (i >= chunks) return;
+    const uint32_t per_row = k / 4;
+    const size_t r = i / per_row;
+    const uint32_t c = (uint32_t)(i - r * per_row) * 4;
+    const f32x4_v a = *(const f32x4_v*)(x + r * ldx + c);
+    uint16_t h[4], m[4], l[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) split_bf16(a[j], h[j], m[j], l[j]);
+    uint16_t* o = out + r * 3 * k + c;
+    auto put = [](uint16_t* at, const uint16_t (&v)[4]) { *(u32x2_v*)at = u32x2_v{(uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16)}; };
+    put(o, l), put(o + k, m), put(o + 2 * k, h);
+}
+
+// the shares of a product cut along k, added in their order, and the product's end
+__global__ void __launch_bounds__(256) linear_finish_kernel(LinearF32Params p, const float* partials, uint32_t splits) {
+    const size_t total = (size_t)p.rows * p.n, i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= total) return;
+    float sum = partials[i];
+    for (uint32_t z = 1; z < splits; ++z) sum += partials[z * total + i];
+    const uint32_t row = (uint32_t)(i / p.n), n = (uint32_t)(i - (size_t)row * p.n);
+    p.y[(size_t)row * p.ldy + n] = linear_epilogue(sum, p.bias ? bf16_to_f32(p.bias[n]) : 0.0f, p, row, 0, n);
+}
+
+template <int MB, int STAGES, bool GROUPED, int KIND, uint32_t PARTS>
+uzu_status launch_dma_tile(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, const GatedRows& gr, float* partials, uint32_t splits) {
     const uint32_t m_tiles = (p.rows + 64 * MB - 1) / (64 * MB), n_tiles = (p.n + DN - 1) / DN;
-    const dim3 grid = GROUPED ? dim3(n_tiles, m_tiles + p.batch) : dim3(gemm_grid_x(m_tiles, n_tiles));
+    const dim3 grid = GROUPED ? dim3(n_tiles, m_tiles + p.batch) : dim3(gemm_grid_x(m_tiles, n_tiles), 1, splits);
     UZU_REQUIRE(grid.y <= 65535, "linear_dma: grid too large");
     const size_t lds = (size_t)STAGES * (64 * MB + DN) * 64 * 2;
     static LdsLimit lim;
-    UZU_REQUIRE(raise_lds_limit(lim, (const void*)linear_dma_kernel<MB, STAGES, GROUPED, KIND>, lds), "linear_dma: %zu bytes of LDS are not available", lds);
-    return launch_check([&] { hipLaunchKernelGGL((linear_dma_kernel<MB, STAGES, GROUPED, KIND>), grid, dim3(256), lds, s, p, xb, ldxb, gr); }, "linear_dma");
+    UZU_REQUIRE(raise_lds_limit(lim, (const void*)linear_dma_kernel<MB, STAGES, GROUPED, KIND, PARTS>, lds), "linear_dma: %zu bytes of LDS are not available", lds);
+    return launch_check([&] { hipLaunchKernelGGL((linear_dma_kernel<MB, STAGES, GROUPED, KIND, PARTS>), grid, dim3(256), lds, s, p, xb, PARTS * p.k, gr, partials); }, "linear_dma");
 }
-template <bool GROUPED, int KIND> uzu_status launch_dma(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, uint32_t ldxb, const GatedRows& gr = GatedRows()) {
+template <bool GROUPED, int KIND, uint32_t PARTS> uzu_status launch_dma(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, const GatedRows& gr = GatedRows()) {
     const size_t tiles = (size_t)((p.rows + 127) / 128) * ((p.n + DN - 1) / DN);
-    if (tiles >= 512) return launch_dma_tile<2, 1, GROUPED, KIND>(s, p, xb, ldxb, gr);
-    if (tiles > 256) return launch_dma_tile<2, 2, GROUPED, KIND>(s, p, xb, ldxb, gr);
-    return launch_dma_tile<1, 2, GROUPED, KIND>(s, p, xb, ldxb, gr);
+    if (tiles >= 512) return launch_dma_tile<2, 1, GROUPED, KIND, PARTS>(s, p, xb, gr, nullptr, 1);
+    if (tiles > 256) return launch_dma_tile<2, 2, GROUPED, KIND, PARTS>(s, p, xb, gr, nullptr, 1);
+    return launch_dma_tile<1, 2, GROUPED, KIND, PARTS>(s, p, xb, gr, nullptr, 1);
+}
+// Few tiles, many k-steps: the steps are cut over workgroups (two a CU wanted, eight steps each at least) and the shares added by a launch of their own.
+// 300 x 1024 x 2048: f32 products 56 us in one piece and 21.8 us cut (VALU tile: 217 us), bf16 products 26.5 us in the register-staged form and 16.0 us.
+uint32_t dma_splits(const LinearF32Params& p, uint32_t parts) {
+    const uint32_t tiles = ((p.rows + 63) / 64) * ((p.n + DN - 1) / DN), steps = parts * p.k / 64;
+    uint32_t splits = 1;
+    while (splits < 8 && tiles * splits * 2 <= 512 && steps >= 16 * splits) splits *= 2;
+    return splits;
+}
+// the operand rows and, behind them, the shares of a cut product
+size_t dma_workspace(const LinearF32Params& p, uint32_t parts) {
+    const uint32_t splits = dma_splits(p, parts);
+    return ((size_t)p.rows * p.k * 2 * parts + 255) / 256 * 256 + (splits > 1 ? (size_t)splits * p.rows * p.n * 4 : 0);
+}
+template <uint32_t PARTS> uzu_status launch_dma_plain(hipStream_t s, const LinearF32Params& p, uint16_t* ws) {
+    if (const uint32_t splits = dma_splits(p, PARTS); splits > 1) {
+        float* partials = (float*)((char*)ws + ((size_t)p.rows * p.k * 2 * PARTS + 255) / 256 * 256);
+        UZU_PROPAGATE((launch_dma_tile<1, 2, false, kEpilogueLean, PARTS>(s, p, ws, GatedRows(), partials, splits)));
+        const size_t total = (size_t)p.rows * p.n;
+        return launch_check([&] { hipLaunchKernelGGL(linear_finish_kernel, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, s, p, partials, splits); }, "linear_finish");
+    }
+    switch (epilogue_kind(p)) {
+    case kEpilogueLean: return launch_dma<false, kEpilogueLean, PARTS>(s, p, ws);
+    case kEpilogueXielu: return launch_dma<false, kEpilogueXielu, PARTS>(s, p, ws);
+    default: return launch_dma<false, kEpilogueFull, PARTS>(s, p, ws);
+    }
 }
 
-// Prompt-sized shapes with whole k-steps.  (A product below a GFLOP or two ends inside the launch and the conversion in front of it: those stay above.)
-bool dma_shape(uint32_t rows, uint32_t n, uint32_t k) { return rows >= 128 && n >= 64 && k % 64 == 0 && 2e-9 * rows * n * k >= 2.0; }
-bool dma_range(uint32_t rows, uint32_t n, uint32_t k) { return (uint64_t)rows * k * 2 < 1ull << 32 && (uint64_t)n * k * 2 < 1ull << 32; } // 32-bit byte offsets
+// Shapes with whole k-steps.  The form is three short launches (operand rows, tiles, shares), 12 us at the least.  bf16 products (parts 1): the register-staged form takes
+// 9.5 us at k = 512, 15 us at k = 1024, 26 us at k = 2048 whatever the rows, until there are tiles for the whole chip (2 GFLOP).  f32 products (parts 3): the VALU tile takes
+// 0.1 us per k-step of one (55 us at k = 512, 217 us at k = 2048) against 14 to 22 us.
+bool dma_shape(uint32_t rows, uint32_t n, uint32_t k, uint32_t parts) {
+    const double gflops = 2e-9 * rows * n * k;
+    if (n < 64 || k % 64 || (uint64_t)rows * k * parts * 2 >= 1ull << 32 || (uint64_t)n * k * 2 >= 1ull << 32) return false; // (32-bit byte offsets)
+    return rows > 16 && (parts == 1 ? (rows >= 128 && gflops >= 2.0) || k >= 1024 : k >= 256 || gflops >= 0.05);
+}
 
 template <int MB, int NB> uzu_status launch(hipStream_t s, const LinearF32Params& p, const char* what) {
     const dim3 grid((p.n + 64 * NB - 1) / (64 * NB), (p.rows + 64 * MB - 1) / (64 * MB), p.batch);
@@ -387,25 +482,37 @@ uzu_status linear_bf16_rows(hipStream_t s, const float* x, uint32_t ldx, uint16_
     UZU_REQUIRE(k % 8 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0, "linear_bf16_rows: alignment");
     return launch_check([&] { hipLaunchKernelGGL(linear_bf16_rows_kernel, dim3((uint32_t)((chunks + 255) / 256)), dim3(256), 0, s, x, ldx, out, k, chunks); }, "linear_bf16_rows");
 }
-bool linear_dma_grouped_supported(const LinearF32Params& p) {
-    return linear_mfma_supported(p) && p.row_offsets && p.batch <= 64 && !p.residual && epilogue_kind(p) == kEpilogueLean && dma_shape(p.rows, p.n, p.k) && dma_range(p.rows, p.n, p.k);
+uzu_status linear_split_rows(hipStream_t s, const float* x, uint32_t ldx, uint16_t* out, uint32_t rows, uint32_t k) {
+    const size_t chunks = (size_t)rows * (k / 4);
+    UZU_REQUIRE(k % 4 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0, "linear_split_rows: alignment");
+    return launch_check([&] { hipLaunchKernelGGL(linear_split_rows_kernel, dim3((uint32_t)((chunks + 255) / 256)), dim3(256), 0, s, x, ldx, out, k, chunks); }, "linear_split_rows");
 }
-uzu_status linear_dma_grouped(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, uint32_t ldxb, const GatedRows* gated) {
-    UZU_REQUIRE(linear_dma_grouped_supported(p) && ((uintptr_t)xb & 15) == 0 && ldxb % 8 == 0 && ldxb >= p.k && (!gated || (gated->out && p.n % 2 == 0 && !p.bias)), "linear_dma_grouped: shape / alignment not covered");
-    return gated ? launch_dma<true, kEpilogueGated>(s, p, xb, ldxb, *gated) : launch_dma<true, kEpilogueLean>(s, p, xb, ldxb);
+bool linear_dma_grouped_supported(const LinearF32Params& p) {
+    return p.row_offsets && p.batch <= 64 && !p.residual && epilogue_kind(p) == kEpilogueLean && p.w_batch % 8 == 0 && ((uintptr_t)p.w & 15) == 0 &&
+           dma_shape(p.rows, p.n, p.k, p.bf16_products ? 1 : 3);
+}
+uzu_status linear_dma_grouped(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, const GatedRows* gated) {
+    UZU_REQUIRE(linear_dma_grouped_supported(p) && ((uintptr_t)xb & 15) == 0 && (!gated || (gated->out && p.n % 2 == 0 && !p.bias)), "linear_dma_grouped: shape / alignment not covered");
+    if (p.bf16_products) return gated ? launch_dma<true, kEpilogueGated, 1>(s, p, xb, *gated) : launch_dma<true, kEpilogueLean, 1>(s, p, xb);
+    return gated ? launch_dma<true, kEpilogueGated, 3>(s, p, xb, *gated) : launch_dma<true, kEpilogueLean, 3>(s, p, xb);
+}
+// f32 products of enough rows: false = not covered (or no workspace: the stream is captured), nothing launched
+bool linear_split(hipStream_t s, const LinearF32Params& p, uzu_status* st) {
+    if (p.bf16_products || p.row_offsets || p.row_map || p.batch != 1 || p.ldx % 4 || (((uintptr_t)p.x | (uintptr_t)p.w) & 15) || !dma_shape(p.rows, p.n, p.k, 3)) return false;
+    uint16_t* xb = (uint16_t*)stream_workspace(s, dma_workspace(p, 3));
+    if (!xb) return false;
+    *st = linear_split_rows(s, p.x, p.ldx, xb, p.rows, p.k);
+    if (*st == UZU_OK) *st = launch_dma_plain<3>(s, p, xb);
+    return true;
 }
 
 uzu_status linear_mfma(hipStream_t s, const LinearF32Params& p) {
     UZU_REQUIRE(linear_mfma_supported(p), "linear_mfma: shape / alignment not covered");
     UZU_REQUIRE(p.row_offsets || !p.row_map, "linear_mfma: gathered rows only in the grouped form");
-    if (!p.row_offsets && p.batch == 1 && dma_shape(p.rows, p.n, p.k) && dma_range(p.rows, p.n, p.k)) {
-        if (uint16_t* xb = (uint16_t*)stream_workspace(s, (size_t)p.rows * p.k * 2)) { // (none while the stream is captured)
+    if (!p.row_offsets && p.batch == 1 && dma_shape(p.rows, p.n, p.k, 1)) {
+        if (uint16_t* xb = (uint16_t*)stream_workspace(s, dma_workspace(p, 1))) { // (none while the stream is captured)
             UZU_PROPAGATE(linear_bf16_rows(s, p.x, p.ldx, xb, p.rows, p.k));
-            switch (epilogue_kind(p)) {
-            case kEpilogueLean: return launch_dma<false, kEpilogueLean>(s, p, xb, p.k);
-            case kEpilogueXielu: return launch_dma<false, kEpilogueXielu>(s, p, xb, p.k);
-            default: return launch_dma<false, kEpilogueFull>(s, p, xb, p.k);
-            }
+            return launch_dma_plain<1>(s, p, xb);
         }
     }
     // tile choice: the widest tile that still fills the chip; narrow outputs (the per-head products) take the narrow tiles

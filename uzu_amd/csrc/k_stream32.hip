@@ -652,15 +652,26 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(const float* y2, const
 
 } // namespace
 
+// the two products of the grouped form: gate | up on the gathered rows, down on the hidden rows
+static void moe_products(const MoeGroupedParams& p, LinearF32Params& q, LinearF32Params& r) {
+    const uint32_t n1 = p.act.plain ? p.ff : 2 * p.ff, slots = p.rows * p.top;
+    q = LinearF32Params{}, r = LinearF32Params{};
+    q.x = p.x, q.w = p.w13, q.y = p.y1, q.rows = slots, q.n = n1, q.k = p.d, q.ldx = p.d, q.ldy = n1, q.batch = p.routed, q.w_batch = (size_t)n1 * p.d;
+    q.row_offsets = p.offsets, q.row_map = p.perm;
+    if (p.act.plain) q.y = p.hidden, q.act = 1; // no gate: the activation rides in the product's epilogue
+    r.x = p.hidden, r.w = p.w2, r.y = p.y2, r.rows = slots, r.n = p.d, r.k = p.ff, r.ldx = p.ff, r.ldy = p.d, r.batch = p.routed, r.w_batch = (size_t)p.d * p.ff;
+    r.row_offsets = p.offsets;
+    q.bf16_products = r.bf16_products = p.f32_products ? 0 : 1;
+}
+static bool moe_dma_supported(const MoeGroupedParams& p, const LinearF32Params& q, const LinearF32Params& r) {
+    return !p.act.plain && p.d % 8 == 0 && ((uintptr_t)p.x & 15) == 0 && linear_dma_grouped_supported(q) && linear_dma_grouped_supported(r);
+}
 bool moe_experts_grouped_supported(const MoeGroupedParams& p) {
-    if (!p.routed || p.rows < 64 || p.routed > 8192 || !p.y1 || !p.y2 || !p.hidden || !p.perm) return false;
-    LinearF32Params q{};
-    const uint32_t n1 = p.act.plain ? p.ff : 2 * p.ff;
-    q.x = p.x, q.w = p.w13, q.y = p.y1, q.rows = p.rows * p.top, q.n = n1, q.k = p.d, q.ldx = p.d, q.ldy = n1, q.batch = p.routed, q.w_batch = (size_t)n1 * p.d;
-    q.bf16_products = 1, q.row_offsets = p.offsets, q.row_map = p.perm;
-    LinearF32Params r = q;
-    r.x = p.hidden, r.w = p.w2, r.y = p.y2, r.n = p.d, r.k = p.ff, r.ldx = p.ff, r.ldy = p.d, r.w_batch = (size_t)p.d * p.ff, r.row_map = nullptr;
-    return linear_mfma_supported(q) && linear_mfma_supported(r);
+    if (!p.routed || p.routed > 8192 || !p.y2 || !p.perm) return false;
+    LinearF32Params q, r;
+    moe_products(p, q, r);
+    if (p.f32_products) return p.rows >= 32 && moe_dma_supported(p, q, r); // (the VALU tile has no grouped form)
+    return p.rows >= 64 && p.y1 && p.hidden && linear_mfma_supported(q) && linear_mfma_supported(r);
 }
 
 uzu_status moe_experts_grouped(hipStream_t s, const MoeGroupedParams& p) {
@@ -670,23 +681,20 @@ uzu_status moe_experts_grouped(hipStream_t s, const MoeGroupedParams& p) {
     UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(moe_bucket_kernel, dim3(1), dim3(1024), (size_t)p.routed * 4, s, p.ids, slots, p.routed, p.offsets, p.cursor); }, "moe_bucket"));
     UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(moe_scatter_kernel, dim3((slots + 255) / 256), dim3(256), (size_t)p.routed * 4, s, p.ids, slots, p.routed, p.top, p.offsets, p.cursor, p.perm, p.slot_pos, p.weights, p.pos_weight); },
                                "moe_scatter"));
-    LinearF32Params q{}, r{};
-    const uint32_t n1 = p.act.plain ? p.ff : 2 * p.ff;
-    q.x = p.x, q.w = p.w13, q.y = p.y1, q.rows = slots, q.n = n1, q.k = p.d, q.ldx = p.d, q.ldy = n1, q.batch = p.routed, q.w_batch = (size_t)n1 * p.d;
-    q.bf16_products = 1, q.row_offsets = p.offsets, q.row_map = p.perm;
-    if (p.act.plain) q.y = p.hidden, q.act = 1; // no gate: the activation rides in the product's epilogue
-    r.x = p.hidden, r.w = p.w2, r.y = p.y2, r.rows = slots, r.n = p.d, r.k = p.ff, r.ldx = p.ff, r.ldy = p.d, r.batch = p.routed, r.w_batch = (size_t)p.d * p.ff;
-    r.bf16_products = 1, r.row_offsets = p.offsets;
-    // prompt-sized: the rows as bf16 once, the gated product in the first product's epilogue, its rows as the bf16 operand of the second
-    const size_t xb_bytes = ((size_t)p.rows * p.d * 2 + 255) / 256 * 256;
-    uint16_t* xb = linear_dma_grouped_supported(q) && linear_dma_grouped_supported(r) && !p.act.plain ? (uint16_t*)stream_workspace(s, xb_bytes + (size_t)slots * p.ff * 2) : nullptr;
+    LinearF32Params q, r;
+    moe_products(p, q, r);
+    // prompt-sized: operand rows once, the gated product in the first product's epilogue, its rows as the operand of the second
+    const uint32_t parts = p.f32_products ? 3 : 1;
+    const size_t xb_bytes = ((size_t)p.rows * p.d * 2 * parts + 255) / 256 * 256;
+    uint16_t* xb = moe_dma_supported(p, q, r) ? (uint16_t*)stream_workspace(s, xb_bytes + (size_t)slots * p.ff * 2 * parts) : nullptr;
     if (xb) {
         GatedRows gr;
         gr.out = (uint16_t*)((char*)xb + xb_bytes), gr.row_weight = p.pos_weight, gr.act = p.act;
-        UZU_PROPAGATE(linear_bf16_rows(s, p.x, p.d, xb, p.rows, p.d));
-        UZU_PROPAGATE(linear_dma_grouped(s, q, xb, p.d, &gr));
-        UZU_PROPAGATE(linear_dma_grouped(s, r, gr.out, p.ff));
+        UZU_PROPAGATE(p.f32_products ? linear_split_rows(s, p.x, p.d, xb, p.rows, p.d) : linear_bf16_rows(s, p.x, p.d, xb, p.rows, p.d));
+        UZU_PROPAGATE(linear_dma_grouped(s, q, xb, &gr));
+        UZU_PROPAGATE(linear_dma_grouped(s, r, gr.out));
     } else {
+        UZU_REQUIRE(!p.f32_products, "moe_experts_grouped: no workspace for f32 products");
         UZU_PROPAGATE(linear_mfma(s, q));
         if (!p.act.plain) UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(moe_act_mul_kernel, dim3(slots), dim3(256), 0, s, p.y1, p.hidden, p.offsets, p.routed, p.ff, p.act, p.pos_weight); }, "moe_act_mul"));
         UZU_PROPAGATE(linear_mfma(s, r));
@@ -775,6 +783,11 @@ uzu_status linear_f32(hipStream_t s, const LinearF32Params& p, const char** vari
     if (linear_mfma_supported(p)) {
         if (variant) *variant = "linear_mfma";
         return linear_mfma(s, p);
+    }
+    uzu_status split = UZU_OK;
+    if (linear_split(s, p, &split)) {
+        if (variant) *variant = "linear_split";
+        return split;
     }
     if (variant) *variant = "linear_tile";
     const dim3 grid((p.n + TN - 1) / TN, (p.rows + TM - 1) / TM, p.batch);

@@ -121,12 +121,15 @@ uzu_status linear_f32(hipStream_t s, const LinearF32Params& p, const char** vari
 // the matrix-core form (k_linear_mfma.hip): bf16 products only; false = shape / mode not covered, nothing launched
 bool linear_mfma_supported(const LinearF32Params& p);
 uzu_status linear_mfma(hipStream_t s, const LinearF32Params& p);
-// f32 rows (pitch ldx) rounded to bf16, rows of k packed; and the grouped product of rows that are bf16 already (X of `p` unused: row r is xb[row_map ? row_map[r] : r];
-// xb has no more rows than p.rows).  gated: W is [up ; gate] and the result act(gate, up) of every row and hidden unit, as bf16 rows (Y unused).
-struct GatedRows;
+// f32 rows (pitch ldx) as operands of the LDS-DMA form: rounded to bf16, rows of k packed; or each number as three bf16 parts, exactly, rows [lo | mid | hi] of 3 k packed
 uzu_status linear_bf16_rows(hipStream_t s, const float* x, uint32_t ldx, uint16_t* out, uint32_t rows, uint32_t k);
+uzu_status linear_split_rows(hipStream_t s, const float* x, uint32_t ldx, uint16_t* out, uint32_t rows, uint32_t k);
+// the grouped product of such rows (bf16_products: the first kind, else the second; X of `p` unused: row r is xb[row_map ? row_map[r] : r], xb has no more rows than
+// p.rows).  gated: W is [up ; gate] and the result act(gate, up) of every row and hidden unit, as operand rows of the same kind (Y unused).
+struct GatedRows;
 bool linear_dma_grouped_supported(const LinearF32Params& p);
-uzu_status linear_dma_grouped(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, uint32_t ldxb, const GatedRows* gated = nullptr);
+uzu_status linear_dma_grouped(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, const GatedRows* gated = nullptr);
+bool linear_split(hipStream_t s, const LinearF32Params& p, uzu_status* st);
 size_t linear_f32_bytes(const LinearF32Params& p);
 
 // Score routing: per row scores = softmax(router x) over all `outputs` (= routed + identity) in f32, the `top` largest (score + bias) win (ties: lower index),
@@ -158,7 +161,7 @@ struct ExpertAct {
     float alpha = 1.0f, gate_min = -INFINITY, gate_max = INFINITY, up_min = -INFINITY, up_max = INFINITY, up_offset = 0.0f;
     uint32_t gelu = 0, plain = 0;
 };
-// out[r, f] = bf16(act(w_r gate, w_r up)), bf16 rows of ff; row_weight f32 [rows] or null (1)
+// out[r, f] = act(w_r gate, w_r up) as operand rows of width ff; row_weight f32 [rows] or null (1)
 struct GatedRows {
     uint16_t* out = nullptr;
     const float* row_weight = nullptr;
@@ -176,7 +179,7 @@ uzu_status moe_experts_gate_up(hipStream_t s, const float* x, const int32_t* ids
 uzu_status moe_experts_down_combine(hipStream_t s, const float* hidden, const float* x, const int32_t* ids, const float* weights, const uint16_t* w2, const float* residual,
                                     float* y, uint32_t rows, uint32_t d, uint32_t ff, uint32_t routed, uint32_t top, uint32_t bf16_products);
 
-// The same block for prefill-sized row counts with bf16 products: the (row, slot) pairs are bucketed by expert (counts -> offsets -> positions), every expert runs
+// The same block for prefill-sized row counts: the (row, slot) pairs are bucketed by expert (counts -> offsets -> positions), every expert runs
 // its bucket through the matrix-core linear as one grouped launch (gate | up, then down), and the rows are combined in slot order.  Workspaces: y1
 // [rows * top][2 ff], hidden [rows * top][ff], y2 [rows * top][d] f32; perm / slot_pos [rows * top], offsets [routed + 1], cursor [routed] u32.
 // pos_weight (f32 [rows * top] or null): the winners' weights multiply the experts' inputs instead of their results (not with plain experts).
@@ -191,6 +194,7 @@ struct MoeGroupedParams {
     uint32_t *perm, *slot_pos, *offsets, *cursor;
     uint32_t rows, d, ff, routed, top;
     ExpertAct act;
+    uint32_t f32_products = 0; // true f32 products (y1 / hidden unused)
 };
 bool moe_experts_grouped_supported(const MoeGroupedParams& p);
 uzu_status moe_experts_grouped(hipStream_t s, const MoeGroupedParams& p);
