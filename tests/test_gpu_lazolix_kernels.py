@@ -253,3 +253,46 @@ def test_grouped_expert_form_prompt_sized(hip_ctx, rows, routed, identity, top, 
     h = np.abs(gate / (1 + np.exp(-gate)) * up).max()
     assert np.isfinite(outs[1]).all() and np.abs(outs[0] - outs[1]).max() < 2 * 2.0 ** -8 * h * np.abs(w2).max()
     assert np.linalg.norm(outs[0] - outs[1]) < 1e-4 * np.linalg.norm(outs[0])
+
+
+@pytest.mark.parametrize("rows,n,k,batch,act", [(3, 4097, 64, 1, 0), (5, 15, 128, 1, 1), (8, 70, 1024, 1, 0), (16, 4100, 2048, 1, 1), (7, 48, 192, 3, 0), (15, 2048, 4096, 1, 0), (17, 33, 64, 1, 1),
+                                                (31, 1030, 1024, 1, 0), (32, 8191, 320, 1, 0), (9, 2100, 64, 2, 0), (20, 300, 4096, 1, 0), (24, 8200, 1024, 1, 1)])
+def test_linear_of_a_few_rows(hip_ctx, rows, n, k, batch, act):
+    """bf16 products of 3 to 32 rows: ragged rows and outputs, one chunk of the contraction and many (fewer than waves, no multiple of them), the per-head form, bias, activation and
+    residual; f32 sums of bf16 products, the bound of the other matrix-core forms"""
+    rng = np.random.default_rng(rows + n)
+    x, w = f32(rng.standard_normal((rows, k * batch))), O.to_bf16(rng.standard_normal((batch, n, k)))
+    b = O.to_bf16(rng.standard_normal(n)) if batch == 1 else None
+    res = f32(rng.standard_normal((rows, n))) if batch == 1 else None
+    got = linear(hip_ctx, x, w, b, res, batch=batch, act=act, bf16=1)
+    xb = O.to_bf16(x).astype(np.float64)
+    want = np.concatenate([xb[:, z * k:(z + 1) * k] @ w[z].T.astype(np.float64) for z in range(batch)], axis=1)
+    if batch == 1:
+        want = (np.maximum(want + b, 0) ** 2 if act else want + b) + res
+    assert np.abs(got - want).max() <= 3e-5 * max(1.0, np.abs(want).max())
+
+
+@pytest.mark.parametrize("rows,routed,identity,top,ff,d", [(2, 8, 0, 2, 64, 64), (3, 70, 2, 4, 128, 192), (16, 4, 1, 3, 320, 64), (33, 2, 1, 1, 64, 1024), (63, 3, 0, 3, 192, 128), (61, 16, 3, 16, 64, 64)])
+def test_experts_of_a_few_rows(hip_ctx, rows, routed, identity, top, ff, d):
+    """bf16 products of 2 to 63 rows: fewer (row, slot) pairs than experts and more, an expert with more pairs than a tile holds, every pair on one expert, identity experts; against 64 bits
+    with the router's choice.  A hidden value near the middle of two bf16 numbers may round to the other: a result then moves by 2^-8 |h| |w|, a few of which may meet."""
+    rng = np.random.default_rng(rows)
+    x, wr = f32(rng.standard_normal((rows, d))), O.to_bf16(rng.standard_normal((routed + identity, d)) * 0.5)
+    corr, res = f32(0.1 * rng.standard_normal(routed + identity)), f32(rng.standard_normal((rows, d)))
+    w13 = O.to_bf16(rng.standard_normal((routed, 2 * ff, d), dtype=np.float32) / np.float32(np.sqrt(d)))
+    w2 = O.to_bf16(rng.standard_normal((routed, d, ff), dtype=np.float32) / np.float32(np.sqrt(ff)))
+    y, ids, wts = np.empty((rows, d), dtype=np.float32), np.empty((rows, top), dtype=np.int32), np.empty((rows, top), dtype=np.float32)
+    _ffi.call("uzu_hip_s32_moe", hip_ctx._h, ptr(x), ptr(O.bf16_bits(wr)), ptr(corr), ptr(O.bf16_bits(w13)), ptr(O.bf16_bits(w2)), ptr(res), ptr(y), ptr(ids), ptr(wts), C.c_uint32(rows),
+              C.c_uint32(d), C.c_uint32(ff), C.c_uint32(routed), C.c_uint32(identity), C.c_uint32(top), C.c_uint32(1))
+    want, h_max, xb = res.astype(np.float64), 0.0, O.to_bf16(x).astype(np.float64)
+    for r in range(rows):
+        for e, wt in zip(ids[r], wts[r].astype(np.float64)):
+            if e >= routed:
+                want[r] += wt * x[r]
+                continue
+            up, gate = np.split(w13[e].astype(np.float64) @ xb[r], 2)
+            h = gate / (1 + np.exp(-gate)) * up
+            h_max = max(h_max, np.abs(h).max())
+            want[r] += wt * (w2[e].astype(np.float64) @ O.to_bf16(h.astype(np.float32)).astype(np.float64))
+    err = np.abs(y - want)
+    assert err.max() <= 2 * 2.0 ** -8 * h_max * np.abs(w2).max() + 1e-5 and np.linalg.norm(err) < 1e-4 * np.linalg.norm(want)

@@ -471,7 +471,7 @@ template <int MB, int NB> uzu_status launch(hipStream_t s, const LinearF32Params
 } // namespace
 
 bool linear_mfma_supported(const LinearF32Params& p) {
-    if (!p.bf16_products || (p.rows < 32 && !p.row_offsets) || p.k % 8 || p.ldx % 4 || p.x_batch % 4 || p.w_batch % 8) return false;
+    if (!p.bf16_products || (p.rows <= 16 && !p.row_offsets) || p.k % 8 || p.ldx % 4 || p.x_batch % 4 || p.w_batch % 8) return false;
     if ((uintptr_t)p.x % 16 || (uintptr_t)p.w % 16) return false;
     if (p.row_offsets && ((uint64_t)p.rows * p.ldx >= 1ull << 32 || (uint64_t)p.n * p.k >= 1ull << 32)) return false; // (grouped: element offsets inside a product are 32-bit)
     return true;

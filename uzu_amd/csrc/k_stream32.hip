@@ -770,6 +770,10 @@ uzu_status linear_f32(hipStream_t s, const LinearF32Params& p, const char** vari
         if (variant) *variant = "linear_mfma_grouped";
         return linear_mfma(s, p);
     }
+    if (linear_few_supported(p)) {
+        if (variant) *variant = "linear_few";
+        return linear_few(s, p);
+    }
     if (p.rows <= 16) {
         const uint32_t vec = (p.k % 8 == 0 && p.ldx % 4 == 0 && p.x_batch % 4 == 0 && p.w_batch % 8 == 0 && (uintptr_t)p.x % 16 == 0 && (uintptr_t)p.w % 16 == 0) ? 1u : 0u;
         if (variant) *variant = "linear_rows";
@@ -824,9 +828,12 @@ uzu_status moe_route_groups(hipStream_t s, const RouteGroupsParams& p) {
     return launch_check([&] { hipLaunchKernelGGL(moe_route_groups_kernel<1>, dim3(p.rows), dim3(threads), ((staged ? (size_t)p.d : 0) + per_row) * 4, s, p, staged); }, "moe_route_groups");
 }
 
+constexpr uint32_t kExpertsFewMinRows = 2; // one row: a wave per hidden unit reads the same weights and needs no second launch (6.8 + 4.2 us at 1024)
 uzu_status moe_experts_gate_up(hipStream_t s, const float* x, const int32_t* ids, const uint16_t* w13, float* hidden, uint32_t rows, uint32_t d, uint32_t ff, uint32_t routed,
                                uint32_t top, uint32_t bf16_products, const ExpertAct& act, const float* in_weights) {
     if (!rows || !routed) return UZU_OK;
+    if (bf16_products && rows >= kExpertsFewMinRows && experts_few_supported(x, hidden, w13, w13, rows, d, ff, routed, top, act))
+        return experts_few_gate_up(s, x, ids, w13, hidden, rows, d, ff, routed, top, act, in_weights);
     UZU_UNSUPPORTED((size_t)d * 4 > 48 * 1024, "moe_experts_gate_up: model_dim %u does not fit the workgroup's LDS row", d);
     // few (row, slot) pairs (decode): the hidden units of a pair are spread over more workgroups, so that the expert's rows stream through many CUs
     const uint32_t want = (1024 + rows * top - 1) / (rows * top), most = (ff + 3) / 4;
@@ -838,6 +845,10 @@ uzu_status moe_experts_gate_up(hipStream_t s, const float* x, const int32_t* ids
 uzu_status moe_experts_down_combine(hipStream_t s, const float* hidden, const float* x, const int32_t* ids, const float* weights, const uint16_t* w2, const float* residual,
                                     float* y, uint32_t rows, uint32_t d, uint32_t ff, uint32_t routed, uint32_t top, uint32_t bf16_products) {
     if (!rows) return UZU_OK;
+    if (bf16_products && rows >= kExpertsFewMinRows && experts_few_supported(x, hidden, w2, w2, rows, d, ff, routed, top, ExpertAct())) {
+        if (float* y2 = (float*)stream_workspace(s, (size_t)rows * top * d * 4)) // (none while the stream is captured)
+            return experts_few_down(s, hidden, x, ids, weights, w2, residual, y2, y, rows, d, ff, routed, top);
+    }
     if (rows <= 16)
         return launch_check([&] { hipLaunchKernelGGL(moe_experts_down_rows_kernel, dim3(rows, (d + 3) / 4), dim3(256), 0, s, hidden, x, ids, weights, w2, residual, y, d, ff, routed, top, bf16_products); },
                             "moe_experts_down_rows");

@@ -130,6 +130,9 @@ struct GatedRows;
 bool linear_dma_grouped_supported(const LinearF32Params& p);
 uzu_status linear_dma_grouped(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, const GatedRows* gated = nullptr);
 bool linear_split(hipStream_t s, const LinearF32Params& p, uzu_status* st);
+// 3 to 32 rows (k_few_rows.hip; bf16 products, k in whole chunks of 64); false where another form is the faster one, too
+bool linear_few_supported(const LinearF32Params& p);
+uzu_status linear_few(hipStream_t s, const LinearF32Params& p);
 size_t linear_f32_bytes(const LinearF32Params& p);
 
 // Score routing: per row scores = softmax(router x) over all `outputs` (= routed + identity) in f32, the `top` largest (score + bias) win (ties: lower index),
@@ -178,6 +181,15 @@ uzu_status moe_experts_gate_up(hipStream_t s, const float* x, const int32_t* ids
 // (weights null: 1)
 uzu_status moe_experts_down_combine(hipStream_t s, const float* hidden, const float* x, const int32_t* ids, const float* weights, const uint16_t* w2, const float* residual,
                                     float* y, uint32_t rows, uint32_t d, uint32_t ff, uint32_t routed, uint32_t top, uint32_t bf16_products);
+
+// Both for a few rows with bf16 products (k_few_rows.hip): an expert's weights are read once for all its rows.  experts_few_supported: up to kFewRowsMaxSlots (row, slot) pairs.
+// y2: workspace, f32 [rows * top][d].
+constexpr uint32_t kFewRowsMaxSlots = 1024;
+bool experts_few_supported(const float* x, const float* hidden, const uint16_t* w13, const uint16_t* w2, uint32_t rows, uint32_t d, uint32_t ff, uint32_t routed, uint32_t top, const ExpertAct& act);
+uzu_status experts_few_gate_up(hipStream_t s, const float* x, const int32_t* ids, const uint16_t* w13, float* hidden, uint32_t rows, uint32_t d, uint32_t ff, uint32_t routed, uint32_t top,
+                               const ExpertAct& act, const float* in_weights);
+uzu_status experts_few_down(hipStream_t s, const float* hidden, const float* x, const int32_t* ids, const float* weights, const uint16_t* w2, const float* residual, float* y2, float* y, uint32_t rows,
+                            uint32_t d, uint32_t ff, uint32_t routed, uint32_t top);
 
 // The same block for prefill-sized row counts: the (row, slot) pairs are bucketed by expert (counts -> offsets -> positions), every expert runs
 // its bucket through the matrix-core linear as one grouped launch (gate | up, then down), and the rows are combined in slot order.  Workspaces: y1
