@@ -108,6 +108,34 @@ def test_f32_experts_of_a_prompt_from_bf16_parts(hip_ctx, tmp_path):
     m.close()
 
 
+def test_greedy_choices_of_many_sequences(hip_ctx, tmp_path):
+    """A pass that chooses and commits for more sequences than one commit launch holds, some of them with logits wanted too, some still inside their prompt: every sequence's tokens
+    are those it gets alone, and decode continues from the token a batched step left."""
+    cfg = gla()
+    W = O.weights(cfg, 3)
+    O.write_model_dir(str(tmp_path / "m"), cfg, W)
+    m = HipModel(hip_ctx, loader.load_model_dir(str(tmp_path / "m"), max_context_length=96), MODEL_BATCH(40) | MODEL_FULL_F32)
+    prompts = [prompt(cfg, 1 + i % 5, i) for i in range(37)]
+    states = [m.new_state() for _ in prompts]
+    want = [[len(p) - 1] if i % 3 == 0 else [] for i, p in enumerate(prompts)]
+    logits, first = m.step_batch(states, prompts, want, sample=True)
+    _, second = m.step_batch(states, [[int(t)] for t in first], None, sample=True)
+    assert np.array_equal(np.argmax(logits, axis=1), np.asarray(first)[::3])
+    for i, p in enumerate(prompts):
+        m.bind(states[i])
+        assert states[i].context_length == len(p) + 1
+        third = m.decode(1)[0][0]
+        st = m.new_state()
+        m.bind(st)
+        alone = [m.prefill(p), *(int(t) for t in m.decode(2)[0])]
+        assert alone == [first[i], second[i], third], i
+        m.bind(None)
+        st.close()
+    for st in states:
+        st.close()
+    m.close()
+
+
 @pytest.mark.parametrize("name", ["a", "b"])
 @pytest.mark.parametrize("full", [True, False])
 def test_whole_prompt_every_position_and_every_layer(models, name, full):

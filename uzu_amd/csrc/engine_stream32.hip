@@ -63,6 +63,9 @@ struct Stream32 {
     float *hyper = nullptr, *conv_rows = nullptr, *lat_q = nullptr; // copies of the stream [s][max_rows][d]; a normed row + its convolution; queries behind their latent
     float *out_normed = nullptr, *logits = nullptr;
     size_t logit_rows = 0;
+    uint8_t* tables = nullptr; // one block: the tables below up to tables_bytes, then d_row_seq
+    size_t tables_bytes = 0;
+    uint32_t* d_pass_sampled = nullptr; // [max_seqs]: a pass's greedy choices
     k::SeqSpan* d_spans = nullptr;
     uint32_t *d_row_seq = nullptr, *d_out_rows = nullptr;
     void** d_cache_ptrs = nullptr;  // [layers][max_seqs]: latent rows / key rows / the retention state
@@ -140,6 +143,29 @@ __global__ void s32_commit_kernel(uint32_t* ctx_len, uint32_t* tokens, const uin
     if (span) span->start = len + count;
 }
 
+// The same for the sequences of a pass, a thread each; choice: the sequence's row of `choices`, or none
+struct CommitSeqs {
+    static constexpr uint32_t kMost = 32;
+    struct One {
+        uint32_t *ctx_len, *tokens, *out_token, *sampled;
+        uint32_t count;
+        int32_t choice;
+    } seq[kMost];
+    uint32_t n;
+};
+__global__ void __launch_bounds__(64) s32_commit_seqs_kernel(CommitSeqs c, const uint32_t* choices) {
+    if (threadIdx.x >= c.n) return;
+    const CommitSeqs::One q = c.seq[threadIdx.x];
+    const uint32_t len = *q.ctx_len;
+    if (q.choice >= 0) {
+        const uint32_t t = choices[q.choice];
+        *q.out_token = t;
+        q.sampled[len + q.count - 1] = t;
+        q.tokens[0] = t;
+    }
+    *q.ctx_len = len + q.count;
+}
+
 uzu_status need_f32(uzu_hip_model* m, size_t floats, float** out) {
     void* p = nullptr;
     UZU_PROPAGATE(dev_alloc(m, floats * 4, &p)); // scratch: every row a kernel reads was written earlier in the same pass (poison mode hands it out as NaNs)
@@ -208,11 +234,17 @@ uzu_status s32_upload_tables(uzu_hip_model* m, const std::vector<PassSeq>& seqs,
         rows += seqs[i].count;
     }
     UZU_REQUIRE(rows <= S.max_rows, "engine: a pass of %u rows (at most %u)", rows, S.max_rows);
-    std::vector<void*> cache_ptrs((size_t)nl * S.max_seqs, nullptr), cache2_ptrs((size_t)nl * S.max_seqs, nullptr);
-    std::vector<float*> shift_ptrs((size_t)nl * S.max_seqs, nullptr), pair_state((size_t)nl * S.max_seqs, nullptr), pair_conv((size_t)nl * S.max_seqs, nullptr);
-    std::vector<float*> inconv((size_t)nl * S.max_seqs, nullptr);
-    std::vector<uint32_t*> prev_tok(S.max_seqs, nullptr);
-    for (uint32_t i = 0; i < nseq; ++i) prev_tok[i] = seqs[i].st->prev_token;
+    // the block's image on the host: every table at its place (s32_create), the row map last and only as far as this pass has rows
+    std::vector<uint8_t> image(S.tables_bytes + row_seq.size() * 4, 0);
+    auto at_of = [&](const void* device) { return device ? image.data() + ((const uint8_t*)device - S.tables) : nullptr; };
+    void **cache_ptrs = (void**)at_of(S.d_cache_ptrs), **cache2_ptrs = (void**)at_of(S.d_cache2_ptrs);
+    float **shift_ptrs = (float**)at_of(S.d_shift_ptrs), **pair_state = (float**)at_of(S.d_pair_state_ptrs), **pair_conv = (float**)at_of(S.d_pair_conv_ptrs);
+    float** inconv = (float**)at_of(S.d_inconv_ptrs);
+    uint32_t** prev_tok = (uint32_t**)at_of(S.d_prev_tok_ptrs);
+    memcpy(at_of(S.d_spans), spans.data(), spans.size() * sizeof(k::SeqSpan));
+    memcpy(at_of(S.d_row_seq), row_seq.data(), row_seq.size() * 4);
+    if (prev_tok)
+        for (uint32_t i = 0; i < nseq; ++i) prev_tok[i] = seqs[i].st->prev_token;
     for (uint32_t l = 0; l < nl; ++l) {
         const uzu_layer_desc& h = m->layers[l].d;
         const uint32_t src = h.is_kv_sharing ? h.kv_source_layer_index : l;
@@ -224,22 +256,12 @@ uzu_status s32_upload_tables(uzu_hip_model* m, const std::vector<PassSeq>& seqs,
             else if (h.mixer_kind == UZU_MIXER_RETENTION || h.mixer_kind == UZU_MIXER_GATED_LINEAR_ATTENTION) cache_ptrs[at] = own.ret_state;
             else cache_ptrs[at] = own.latent;
             shift_ptrs[at] = seqs[i].st->layers[l].shift_prev;
-            inconv[at] = seqs[i].st->layers[l].in_conv;
-            if (h.pair_mixer || h.qkv_conv) pair_state[at] = seqs[i].st->layers[l].ssm_state, pair_conv[at] = seqs[i].st->layers[l].conv_state;
+            if (inconv) inconv[at] = seqs[i].st->layers[l].in_conv;
+            if (pair_state && (h.pair_mixer || h.qkv_conv)) pair_state[at] = seqs[i].st->layers[l].ssm_state, pair_conv[at] = seqs[i].st->layers[l].conv_state;
         }
     }
-    // (pageable sources: the copies have left the host buffers when the calls return)
-    HIPCHK(hipMemcpyAsync(S.d_spans, spans.data(), spans.size() * sizeof(k::SeqSpan), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(S.d_row_seq, row_seq.data(), row_seq.size() * 4, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(S.d_cache_ptrs, cache_ptrs.data(), cache_ptrs.size() * sizeof(void*), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(S.d_cache2_ptrs, cache2_ptrs.data(), cache2_ptrs.size() * sizeof(void*), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(S.d_shift_ptrs, shift_ptrs.data(), shift_ptrs.size() * sizeof(float*), hipMemcpyHostToDevice, s));
-    if (S.d_pair_state_ptrs) {
-        HIPCHK(hipMemcpyAsync(S.d_pair_state_ptrs, pair_state.data(), pair_state.size() * sizeof(float*), hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemcpyAsync(S.d_pair_conv_ptrs, pair_conv.data(), pair_conv.size() * sizeof(float*), hipMemcpyHostToDevice, s));
-    }
-    if (S.d_inconv_ptrs) HIPCHK(hipMemcpyAsync(S.d_inconv_ptrs, inconv.data(), inconv.size() * sizeof(float*), hipMemcpyHostToDevice, s));
-    if (S.d_prev_tok_ptrs) HIPCHK(hipMemcpyAsync(S.d_prev_tok_ptrs, prev_tok.data(), prev_tok.size() * sizeof(uint32_t*), hipMemcpyHostToDevice, s));
+    // (pageable sources: the copies have left the host buffers when the calls return; a copy is ~10 us of the host's time whatever it moves, so the tables go as one)
+    HIPCHK(hipMemcpyAsync(S.tables, image.data(), image.size(), hipMemcpyHostToDevice, s));
     if (!out_rows.empty()) HIPCHK(hipMemcpyAsync(S.d_out_rows, out_rows.data(), out_rows.size() * 4, hipMemcpyHostToDevice, s));
     return UZU_OK;
 }
@@ -772,6 +794,30 @@ uzu_status sample_commit(uzu_hip_model* m, uzu_hip_state* st, uint32_t logit_row
     return UZU_OK;
 }
 
+// the greedy choice of the sequences `chosen` (indices into the pass, ascending; their logits are consecutive rows from first_row on), every sequence advanced: three launches
+// for a pass, where three per sequence were 10 us of each
+uzu_status choose_commit(uzu_hip_model* m, const std::vector<PassSeq>& pass, const std::vector<uint32_t>& chosen, size_t first_row) {
+    Stream32& S = *m->s32;
+    hipStream_t s = m->ctx->stream;
+    Enc e{m, s};
+    const uint32_t n = (uint32_t)chosen.size(), V = m->d.vocab_size;
+    if (n) RUN("argmax", (size_t)V * 4 * n, k::argmax(s, S.logits + first_row * V, UZU_F32, S.d_pass_sampled, V, n, m->argmax_scratch));
+    if (e.st != UZU_OK) return e.st;
+    size_t b = 0;
+    for (size_t lo = 0; lo < pass.size(); lo += CommitSeqs::kMost) {
+        CommitSeqs c{};
+        for (size_t a = lo; a < pass.size() && c.n < CommitSeqs::kMost; ++a) {
+            uzu_hip_state* st = pass[a].st;
+            const bool mine = b < chosen.size() && chosen[b] == a;
+            c.seq[c.n++] = {st->d_ctx_len, st->d_tokens, st->d_out_token, st->d_sampled, pass[a].count, mine ? (int32_t)b : -1};
+            b += mine;
+        }
+        hipLaunchKernelGGL(s32_commit_seqs_kernel, dim3(1), dim3(64), 0, s, c, S.d_pass_sampled);
+        ++m->launches;
+    }
+    return UZU_OK;
+}
+
 } // namespace
 
 // ---------------------------------------------------------------------------------- construction
@@ -1276,15 +1322,21 @@ uzu_status s32_create(uzu_hip_context* ctx, const uzu_model_desc* desc, uint32_t
     }
     void* p = nullptr;
     TRY(dev_alloc(m, R * w_top * 4, &p)); S.moe_ids = (int32_t*)p;
-    TRY(dev_alloc(m, S.max_seqs * sizeof(k::SeqSpan), &p)); S.d_spans = (k::SeqSpan*)p;
-    TRY(dev_alloc(m, R * 4, &p)); S.d_row_seq = (uint32_t*)p;
     TRY(dev_alloc(m, R * 4, &p)); S.d_out_rows = (uint32_t*)p;
-    TRY(dev_alloc(m, (size_t)nl * S.max_seqs * sizeof(void*), &p)); S.d_cache_ptrs = (void**)p;
-    TRY(dev_alloc(m, (size_t)nl * S.max_seqs * sizeof(void*), &p)); S.d_cache2_ptrs = (void**)p;
-    TRY(dev_alloc(m, (size_t)nl * S.max_seqs * sizeof(float*), &p)); S.d_shift_ptrs = (float**)p;
-    if (any_pair || any_conv) {
-        TRY(dev_alloc(m, (size_t)nl * S.max_seqs * sizeof(float*), &p)); S.d_pair_state_ptrs = (float**)p;
-        TRY(dev_alloc(m, (size_t)nl * S.max_seqs * sizeof(float*), &p)); S.d_pair_conv_ptrs = (float**)p;
+    { // the tables of a pass: one block (s32_upload_tables), every table 16-byte aligned
+        const size_t per_layer = ((size_t)nl * S.max_seqs * sizeof(void*) + 15) & ~(size_t)15, spans = (S.max_seqs * sizeof(k::SeqSpan) + 15) & ~(size_t)15;
+        const bool pair = any_pair || any_conv;
+        const size_t prev = desc->bigram_buckets ? (S.max_seqs * sizeof(uint32_t*) + 15) & ~(size_t)15 : 0;
+        S.tables_bytes = spans + per_layer * (3 + (pair ? 2 : 0) + (any_inconv ? 1 : 0)) + prev;
+        TRY(dev_alloc(m, S.tables_bytes + R * 4, &p)); S.tables = (uint8_t*)p;
+        uint8_t* at = S.tables;
+        auto take = [&](size_t bytes) { uint8_t* here = at; at += bytes; return here; };
+        S.d_spans = (k::SeqSpan*)take(spans);
+        S.d_cache_ptrs = (void**)take(per_layer), S.d_cache2_ptrs = (void**)take(per_layer), S.d_shift_ptrs = (float**)take(per_layer);
+        if (pair) S.d_pair_state_ptrs = (float**)take(per_layer), S.d_pair_conv_ptrs = (float**)take(per_layer);
+        if (any_inconv) S.d_inconv_ptrs = (float**)take(per_layer);
+        if (prev) S.d_prev_tok_ptrs = (uint32_t**)take(prev);
+        S.d_row_seq = (uint32_t*)at;
     }
     if (any_pair) {
         if (hipStreamCreateWithFlags(&S.side, hipStreamNonBlocking) != hipSuccess || hipEventCreateWithFlags(&S.side_fork, hipEventDisableTiming) != hipSuccess ||
@@ -1293,8 +1345,6 @@ uzu_status s32_create(uzu_hip_context* ctx, const uzu_model_desc* desc, uint32_t
             return fail(UZU_ERR_HIP);
         }
     }
-    if (any_inconv) { TRY(dev_alloc(m, (size_t)nl * S.max_seqs * sizeof(float*), &p)); S.d_inconv_ptrs = (float**)p; }
-    if (desc->bigram_buckets) { TRY(dev_alloc(m, S.max_seqs * sizeof(uint32_t*), &p)); S.d_prev_tok_ptrs = (uint32_t**)p; }
     TRY(dev_alloc(m, R * 4, &p)); m->batch_tokens = (uint32_t*)p;
     if (flags & UZU_MODEL_DEBUG_TAPS) TRY(need_f32(m, (size_t)nl * R * d, &S.taps));
     {
@@ -1323,7 +1373,8 @@ uzu_status s32_create(uzu_hip_context* ctx, const uzu_model_desc* desc, uint32_t
         S.lru_ws_bytes = k::lru_piece_ws_bytes(S.max_rows / 32 + S.max_seqs, w_lru);
         TRY(need_f32(m, S.lru_ws_bytes / 4, &S.lru_ws));
     }
-    TRY(dev_alloc(m, k::argmax_scratch_bytes(1), &m->argmax_scratch));
+    TRY(dev_alloc(m, k::argmax_scratch_bytes(S.max_seqs), &m->argmax_scratch));
+    TRY(dev_alloc(m, S.max_seqs * 4, &p)); S.d_pass_sampled = (uint32_t*)p;
     TRY(dev_alloc(m, k::unified_sampling_scratch_bytes(1), &m->sampling_scratch));
     TRY(dev_alloc(m, 8, &p, true)); m->d_seed = (uint64_t*)p;
     TRY(ensure_logits(m, 16));
@@ -1454,20 +1505,22 @@ uzu_status s32_step_batch(uzu_hip_model* m, uzu_hip_state** states, uint32_t nse
         UZU_PROPAGATE(ensure_logits(m, out_rows.size()));
         HIPCHK(hipMemcpyAsync(m->batch_tokens, pass_tok.data(), pass_tok.size() * 4, hipMemcpyHostToDevice, s));
         UZU_PROPAGATE(s32_pass(m, pass, m->batch_tokens, out_rows));
-        for (size_t a = 0; a < pass.size(); ++a) {
-            size_t srow = 0;
-            bool do_sample = false;
-            for (size_t b = 0; b < sample_seq.size(); ++b)
-                if (sample_seq[b] == a) srow = n_want_rows + b, do_sample = true;
-            UZU_PROPAGATE(sample_commit(m, pass[a].st, (uint32_t)srow, pass[a].count, do_sample));
-        }
+        if (m->sampling.on) { // (a seed per sequence)
+            for (size_t a = 0; a < pass.size(); ++a) {
+                const auto at = std::find(sample_seq.begin(), sample_seq.end(), (uint32_t)a);
+                UZU_PROPAGATE(sample_commit(m, pass[a].st, (uint32_t)(n_want_rows + (at - sample_seq.begin())), pass[a].count, at != sample_seq.end()));
+            }
+        } else UZU_PROPAGATE(choose_commit(m, pass, sample_seq, n_want_rows));
         HIPCHK(hipStreamSynchronize(s));
         for (size_t a = 0; a < pass.size(); ++a) state_set_length(m, pass[a].st, pass[a].start + pass[a].count);
         // the wanted rows of a pass are consecutive entries of want_rows (both ascend): one copy
         if (n_want_rows) HIPCHK(hipMemcpy(logits_out + (size_t)out_dst[0] * V, S.logits, n_want_rows * (size_t)V * 4, hipMemcpyDeviceToHost));
-        for (size_t b = 0; b < sample_seq.size(); ++b) {
-            const uint32_t qi = seq_lo + sample_seq[b];
-            HIPCHK(hipMemcpy(sampled_out + qi, states[qi]->d_out_token, 4, hipMemcpyDeviceToHost));
+        if (m->sampling.on) {
+            for (uint32_t a : sample_seq) HIPCHK(hipMemcpy(sampled_out + seq_lo + a, states[seq_lo + a]->d_out_token, 4, hipMemcpyDeviceToHost));
+        } else if (!sample_seq.empty()) {
+            std::vector<uint32_t> choices(sample_seq.size());
+            HIPCHK(hipMemcpy(choices.data(), S.d_pass_sampled, choices.size() * 4, hipMemcpyDeviceToHost));
+            for (size_t b = 0; b < choices.size(); ++b) sampled_out[seq_lo + sample_seq[b]] = choices[b];
         }
         // sequences that are through leave the window; one that is not stays first
         while (seq_lo < nseq && done[seq_lo] == counts[seq_lo]) ++seq_lo;
