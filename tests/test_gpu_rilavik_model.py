@@ -136,6 +136,25 @@ def test_greedy_choices_of_many_sequences(hip_ctx, tmp_path):
     m.close()
 
 
+def test_copied_state_of_many_allocations(hip_ctx, tmp_path):
+    """A state of more allocations than one copy launch takes (small windows, large caches): the copy continues exactly as its source, which the copy's steps leave alone."""
+    layer = O.parallel_layer(O.left_half(**LEFT), O.right_half(**RIGHT), 0.7, 1.2)
+    cfg = O.config(vocab=53, width=40, layers=[layer] * 36)
+    W, m = make(hip_ctx, tmp_path, cfg, 5, ctx_len=3000)
+    a, b = m.new_state(), m.new_state()
+    m.step_batch([a], [prompt(cfg, 21, 1)], None)
+    m.step_batch([b], [prompt(cfg, 30, 2)], None)
+    b.copy_from(a)
+    assert b.context_length == 21
+    toks = prompt(cfg, 5, 3)
+    on_copy, _ = m.step_batch([b], [toks], [list(range(5))])
+    on_source, _ = m.step_batch([a], [toks], [list(range(5))])
+    assert np.array_equal(on_copy, on_source) and np.isfinite(on_copy).all()
+    for st in (a, b):
+        st.close()
+    m.close()
+
+
 @pytest.mark.parametrize("name", ["a", "b"])
 @pytest.mark.parametrize("full", [True, False])
 def test_whole_prompt_every_position_and_every_layer(models, name, full):

@@ -21,6 +21,28 @@ using namespace uzu::eng;
 namespace uzu {
 namespace eng {
 
+// Copies of many allocations (whole 256-byte blocks) in one launch: y = the allocation, its 64 workgroups share it.  A state is 20 to 70 allocations; a copy each was
+// 3 to 6 us whatever it moved.
+struct CopyTable {
+    static constexpr uint32_t kMost = 128; // (3 KB of kernel arguments)
+    struct One {
+        void* dst;
+        const void* src;
+        size_t bytes;
+    } one[kMost];
+};
+__global__ void __launch_bounds__(256) copy_table_kernel(CopyTable t) {
+    uint4* dst = (uint4*)t.one[blockIdx.y].dst;
+    const uint4* src = (const uint4*)t.one[blockIdx.y].src;
+    const size_t n = t.one[blockIdx.y].bytes / 16, step = (size_t)gridDim.x * 256;
+    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    for (; i + 3 * step < n; i += 4 * step) {
+        const uint4 a = src[i], b = src[i + step], c = src[i + 2 * step], d = src[i + 3 * step];
+        dst[i] = a, dst[i + step] = b, dst[i + 2 * step] = c, dst[i + 3 * step] = d;
+    }
+    for (; i < n; i += step) dst[i] = src[i];
+}
+
 uzu_status dev_alloc(uzu_hip_model* m, size_t bytes, void** out, bool zero) {
     void* p = nullptr;
     const size_t alloc = bytes ? (bytes + 255) & ~(size_t)255 : 256;
@@ -791,7 +813,15 @@ uzu_status uzu_hip_state_copy(uzu_hip_state* dst, const uzu_hip_state* src) {
     UZU_REQUIRE(dst->allocations.size() == src->allocations.size() && dst->allocation_bytes == src->allocation_bytes, "state_copy: the states differ in layout");
     (void)hipSetDevice(m->ctx->device);
     hipStream_t s = m->ctx->stream;
-    for (size_t i = 0; i < dst->allocations.size(); ++i) HIPCHK(hipMemcpyAsync(dst->allocations[i], src->allocations[i], dst->allocation_bytes[i], hipMemcpyDeviceToDevice, s));
+    for (size_t lo = 0; lo < dst->allocations.size(); lo += CopyTable::kMost) {
+        CopyTable t{};
+        uint32_t n = 0;
+        for (size_t i = lo; i < dst->allocations.size() && n < CopyTable::kMost; ++i)
+            if (const size_t bytes = dst->allocation_bytes[i]) t.one[n++] = {dst->allocations[i], src->allocations[i], bytes};
+        if (!n) continue;
+        hipLaunchKernelGGL(copy_table_kernel, dim3(64, n), dim3(256), 0, s, t);
+        HIPCHK(hipGetLastError());
+    }
     HIPCHK(hipStreamSynchronize(s));
     const uint32_t len = m->bound == src ? m->context_length : src->context_length;
     dst->context_length = len;
