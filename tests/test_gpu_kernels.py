@@ -144,9 +144,10 @@ def test_matmul_few_rows_on_the_matrix_cores(hip_ctx, n, k, m, method):
 
 
 @pytest.mark.parametrize("method", [0, 1, 2])
-@pytest.mark.parametrize("n,k,m", [(1024, 3584, 37), (8224, 1024, 17), (4, 256, 31), (20, 512, 33), (1028, 1024, 64), (3072, 1024, 127), (2048, 256, 129), (260, 2304, 300)])
+@pytest.mark.parametrize("n,k,m", [(1024, 3584, 37), (8224, 1024, 17), (4, 256, 31), (20, 512, 33), (1028, 1024, 64), (3072, 1024, 127), (2048, 256, 129), (260, 2304, 300), (8200, 256, 9), (8192, 512, 16),
+                                   (131076, 256, 2)])
 def test_matmul_dozens_of_rows(hip_ctx, n, k, m, method):
-    """csrc/k_gemm_rows.hip (M >= 17, int4 g128, register-fed): edges of the 32-token and 32- / 64-row tiles, K of one pair of groups and of an odd number of pairs, shapes whose K is
+    """csrc/k_gemm_rows.hip (M >= 17, and wide matrices of fewer rows; int4 g128, register-fed): edges of the 32-token and 32- / 64-row tiles, K of one pair of groups and of an odd number of pairs, shapes whose K is
     split over waves and over workgroups, both with the Linear bias.  <= 1 bf16 ulp against the CPU kernel, >= 97 % bit-identical (another order of summation, as above)."""
     rng = np.random.default_rng(n + k + m + method)
     q = quant_matrix(rng, n, k, 4, 128, method)

@@ -97,10 +97,10 @@ __global__ void __launch_bounds__(128) dn_tree_prep_kernel(const uint16_t* __res
 
 // ------------------------------------------------------------------------------------------------ prefix + Gram + solve + out
 // One workgroup = (value head hv, 16 value columns c0 .. c0 + 15), 256 threads, all n nodes.  Every output element is computed by one
-// thread walking the reference's loop in the reference's order (see the file header); LDS rows are padded to 129 floats (threads of a
-// wave read the same element index of different rows).
-constexpr uint32_t kPad = 129;
-struct TreeSolveLds {
+// thread walking the reference's loop in the reference's order (see the file header); LDS rows are padded to 132 floats (threads of a
+// wave read the same four elements of different rows, 16 bytes at a time).
+constexpr uint32_t kPad = 132;
+struct alignas(16) TreeSolveLds {
     float q[kDnTreeMaxNodes][kPad];
     float k[kDnTreeMaxNodes][kPad];
     float h0[16][kPad];
@@ -134,12 +134,38 @@ __global__ void __launch_bounds__(256) dn_tree_solve_kernel(const uint16_t* __re
         const uint32_t token = min(blk * kBlock + tid / 16, n - 1); // clamped: never consumed past n
         v_pre[blk] = bf16_to_f32(v_in[(size_t)token * value_dim + hv * D + c0 + tid % 16]);
     }
-    for (uint32_t idx = tid; idx < n * D; idx += 256) {
-        const uint32_t row = idx / D, d = idx % D;
-        L.q[row][d] = bf16_to_f32(q_in[(size_t)row * key_dim + hk * D + d]);
-        L.k[row][d] = bf16_to_f32(k_in[(size_t)row * key_dim + hk * D + d]);
+    if (((uintptr_t)q_in & 15) == 0 && ((uintptr_t)k_in & 15) == 0 && ((uintptr_t)h0 & 15) == 0) {
+        // 16 bytes a lane and every load in front of the first store: element by element, q and k were seven trips to memory one behind the other at 13 nodes (17.4 us, now 13.4, of which ~2 are launch and the rest the chains below)
+        static_assert(kDnTreeMaxNodes * D / 8 == 512, "two pieces of 8 q / k elements a thread");
+        const uint32_t c = tid % 16 * 8;
+        u32x4_v qv[2], kv[2];
+        f32x4_v hv4[2];
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i) {
+            const size_t at = (size_t)min(tid / 16 + 16 * i, n - 1) * key_dim + hk * D + c;
+            qv[i] = *(const u32x4_v*)(q_in + at), kv[i] = *(const u32x4_v*)(k_in + at);
+            hv4[i] = *(const f32x4_v*)(h0 + ((size_t)hv * D + c0) * D + (tid + 256 * i) * 4); // 16 consecutive state rows: 8 KB contiguous
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i) {
+            const uint32_t row = tid / 16 + 16 * i;
+            *(f32x4_v*)&L.h0[(tid + 256 * i) / 32][(tid + 256 * i) % 32 * 4] = hv4[i];
+            if (row >= n) continue;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                *(f32x4_v*)&L.q[row][c + 4 * h] = f32x4_v{bits_to_f32(qv[i][2 * h] << 16), bits_to_f32(qv[i][2 * h] & 0xFFFF0000u), bits_to_f32(qv[i][2 * h + 1] << 16), bits_to_f32(qv[i][2 * h + 1] & 0xFFFF0000u)};
+                *(f32x4_v*)&L.k[row][c + 4 * h] = f32x4_v{bits_to_f32(kv[i][2 * h] << 16), bits_to_f32(kv[i][2 * h] & 0xFFFF0000u), bits_to_f32(kv[i][2 * h + 1] << 16), bits_to_f32(kv[i][2 * h + 1] & 0xFFFF0000u)};
+            }
+        }
+    } else {
+        for (uint32_t idx = tid; idx < n * D; idx += 256) {
+            const uint32_t row = idx / D, d = idx % D;
+            L.q[row][d] = bf16_to_f32(q_in[(size_t)row * key_dim + hk * D + d]);
+            L.k[row][d] = bf16_to_f32(k_in[(size_t)row * key_dim + hk * D + d]);
+        }
+        for (uint32_t idx = tid; idx < 16 * D; idx += 256) L.h0[idx / D][idx % D] = h0[((size_t)hv * D + c0) * D + idx];
     }
-    for (uint32_t idx = tid; idx < 16 * D; idx += 256) L.h0[idx / D][idx % D] = h0[((size_t)hv * D + c0) * D + idx]; // 16 consecutive state rows: 8 KB contiguous
     __syncthreads();
     if (tid < n) { // prefix.rs:20-36: log decays of the ancestors-or-self, in column order
         float sum = 0.0f;
@@ -152,22 +178,29 @@ __global__ void __launch_bounds__(256) dn_tree_solve_kernel(const uint16_t* __re
         const uint32_t row = idx / n, col = idx % n;
         float qkd = 0.0f, a = 0.0f;
         if (row >= L.t_start[col] && row <= L.t_end[col]) {
+            // (both sums in one walk, 16 bytes a read: two chains of additions side by side, a quarter of the LDS instructions)
             float qk = 0.0f, kk = 0.0f;
-            for (uint32_t d = 0; d < D; ++d) qk += L.q[row][d] * L.k[col][d];
+#pragma unroll 4
+            for (uint32_t d = 0; d < D; d += 4) {
+                const f32x4_v a = *(const f32x4_v*)&L.q[row][d], b = *(const f32x4_v*)&L.k[col][d], c = *(const f32x4_v*)&L.k[row][d];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) qk += a[t] * b[t], kk += c[t] * b[t];
+            }
             const float e = expf_glibc(L.prefix[row] - L.prefix[col]);
             qkd = e * scale * qk;
-            if (row != col) {
-                for (uint32_t d = 0; d < D; ++d) kk += L.k[row][d] * L.k[col][d];
-                a = L.beta[row] * e * kk;
-            }
+            if (row != col) a = L.beta[row] * e * kk;
         }
         L.qkd[row][col] = qkd, L.a[row][col] = a;
     }
     for (uint32_t idx = tid; idx < n * 16; idx += 256) { // tree_gram.rs:139-158 (kh0) and the q . h0 term of out.rs:62-73
         const uint32_t token = idx / 16, j = idx % 16;
         float sk = 0.0f, sq = 0.0f;
-        for (uint32_t d = 0; d < D; ++d) sk += L.k[token][d] * L.h0[j][d];
-        for (uint32_t d = 0; d < D; ++d) sq += L.q[token][d] * L.h0[j][d];
+#pragma unroll 4
+        for (uint32_t d = 0; d < D; d += 4) {
+            const f32x4_v h = *(const f32x4_v*)&L.h0[j][d], a = *(const f32x4_v*)&L.k[token][d], b = *(const f32x4_v*)&L.q[token][d];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) sk += a[t] * h[t], sq += b[t] * h[t];
+        }
         L.kh0[token][j] = sk, L.qh0[token][j] = sq;
     }
     __syncthreads();

@@ -1,6 +1,6 @@
 // k_gemm_rows.hip -- quantised matmul for dozens to hundreds of activation rows: a register-fed matrix-core kernel without operand staging.
 //
-// Where it sits: behind the few-rows kernel (k_gemv_rows.hip, M <= 16) and in front of the large tiles (k_gemm128.hip).  At these sizes a linear of a 1024-wide
+// Where it sits: behind the few-rows kernel (k_gemv_rows.hip, M <= 16; wide matrices come here from 2 rows on) and in front of the large tiles (k_gemm128.hip).  At these sizes a linear of a 1024-wide
 // model is 1 .. 15 GFLOP and 1 .. 4 MB of codes -- a microsecond or two of either -- and what a tile kernel spends is its chain: a k-step of 64 through LDS with
 // two barriers is ~1 us whatever else the CU does, so a 64 x 64 tile over K = 3584 was 35 us on sixteen workgroups.  Here nothing is staged and nothing waits:
 //   * a wave owns 16 MT tokens x 16 NB weight rows of v_mfma_f32_16x16x32_bf16.  Activations go from the L2 into the A operand (lane (r, g): token r, 16 bytes
@@ -258,7 +258,7 @@ template <int NB, int MT, bool ACT> uzu_status launch_kw(hipStream_t s, const Ge
 }
 
 bool gemm_rows_supported(const MatmulParams& p) {
-    if (exact_mode() || p.m < 17 || p.m > 65535 || p.bits != 4 || p.b_kind == UZU_MATMUL_B_FULL_PRECISION) return false;
+    if (exact_mode() || p.m < 2 || p.m > 65535 || p.bits != 4 || p.b_kind == UZU_MATMUL_B_FULL_PRECISION) return false;
     if (p.w_dt != UZU_BF16 || p.a_dt != UZU_BF16 || (p.d_dt != UZU_BF16 && p.d_dt != UZU_F32)) return false;
     if (p.signed_codes || p.ab_scale != 1.0f || p.accumulate || p.has_soft_cap || p.gather) return false;
     if (p.act_mul ? (p.n % 8 || p.d_dt != UZU_BF16) : p.n % 4) return false; // whole quads of outputs
@@ -276,6 +276,9 @@ bool gemm_rows_supported(const MatmulParams& p) {
 bool gemm_rows_preferred(const MatmulParams& p) {
     if (!gemm_rows_supported(p) || (p.m >= 128 && (tune_env("gemm_form") || tune_env("gemm_splits")))) return false; // (a pinned form or split-K is the large tile's)
     const double gflops = 2e-9 * p.m * p.n * p.k;
+    // up to 16 rows: the few-rows kernel (k_gemv_rows.hip) is a workgroup per 16 outputs, 1024 x 3584 in 5.6 us against 6.8 here at 5 rows, but takes 248320 x 1024 in
+    // 67 .. 125 us (2 .. 16 rows) against 46 .. 53, 4096 x 14336 in 25 .. 28 against 16 .. 20, 28672 x 4096 in 28 .. 44 against 28 .. 30, 8224 x 1024 in 7.2 against 6.0 (13 rows)
+    if (p.m <= 16) return (uint64_t)p.n * p.k >= (32u << 20) || (p.m > 8 && p.n >= 8192);
     if (p.k >= 8192) return p.m < 128 || gflops <= 16.0;
     return gflops <= (p.m >= 128 ? 4.5 : p.act_mul ? 16.0 : 9.0);
 }

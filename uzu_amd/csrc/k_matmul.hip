@@ -359,13 +359,13 @@ uzu_status matmul(hipStream_t s, const MatmulParams& p, int num_cus, const char*
         if (variant) *variant = p.bits == 4 ? "gemv_dec<4>" : "gemv_dec<8>";
         return gemv_dec(s, q, num_cus, nullptr);
     }
+    if (gemm_rows_preferred(p)) { // dozens of rows, wide matrices of fewer (k_gemm_rows.hip)
+        if (variant) *variant = "gemm_rows";
+        return gemm_rows(s, p, num_cus);
+    }
     if (gemv_rows_mfma_supported(p)) { // a handful of rows (speculative verify passes, prefill tails): one pass over the weights on the matrix cores
         if (variant) *variant = "gemv_rows_mfma";
         return gemv_rows_mfma(s, p);
-    }
-    if (gemm_rows_preferred(p)) { // dozens of rows (k_gemm_rows.hip)
-        if (variant) *variant = "gemm_rows";
-        return gemm_rows(s, p, num_cus);
     }
     if (gemm_q_mfma_supported(p)) { // prefill-sized M: bf16 matrix cores (k_gemm.hip)
         if (variant) *variant = p.bits == 4 ? "gemm_q_mfma<4>" : "gemm_q_mfma<8>";
