@@ -136,6 +136,29 @@ def test_greedy_choices_of_many_sequences(hip_ctx, tmp_path):
     m.close()
 
 
+def test_attention_tiles_of_more_sequences_than_a_wave_has_lanes(hip_ctx, tmp_path):
+    """70 sequences in one pass through the attention's matrix-core form, prompts (tiles of 128 items, keys in two groups) and then a token each (keys over workgroups and waves): every
+    sequence's logits are those it gets in a pass of its own, up to bf16 products that round the other way."""
+    cfg = O.config(vocab=53, width=64, layers=[O.parallel_layer(O.left_half(4, 2, 32, 24, 40, conv=2), O.right_half(2, 8, 8, groups=1, norm_groups=1, conv=2), 0.9, 0.4)])
+    W = O.weights(cfg, 7)
+    O.write_model_dir(str(tmp_path / "m"), cfg, W)
+    m = HipModel(hip_ctx, loader.load_model_dir(str(tmp_path / "m"), max_context_length=256), MODEL_BATCH(70))
+    prompts = [prompt(cfg, 17 + (i * 29) % 90, i) for i in range(70)]
+    states = [m.new_state() for _ in prompts]
+    together, _ = m.step_batch(states, prompts, [[len(p) - 1] for p in prompts])
+    next_together, _ = m.step_batch(states, [[5]] * 70, [[0]] * 70)
+    for i, p in enumerate(prompts):
+        st = m.new_state()
+        alone, _ = m.step_batch([st], [p], [[len(p) - 1]])
+        next_alone, _ = m.step_batch([st], [[5]], [[0]])
+        st.close()
+        for got, want in ((together[i], alone[0]), (next_together[i], next_alone[0])):
+            assert np.abs(got - want).max() <= 2.0 ** -6 * np.abs(want).max(), i
+    for st in states:
+        st.close()
+    m.close()
+
+
 def test_copied_state_of_many_allocations(hip_ctx, tmp_path):
     """A state of more allocations than one copy launch takes (small windows, large caches): the copy continues exactly as its source, which the copy's steps leave alone."""
     layer = O.parallel_layer(O.left_half(**LEFT), O.right_half(**RIGHT), 0.7, 1.2)

@@ -311,7 +311,7 @@ uzu_status uzu_hip_s32_window_attention(uzu_hip_context* ctx, const float* q, co
     k::WindowAttentionParams p{};
     p.q = dq, p.ldq = heads * dim, p.out = dout, p.key_caches = dkp, p.value_caches = dvp, p.cache_bf16 = cache_bf16, p.sinks = dsink, p.spans = spans, p.row_seq = row_seq;
     p.rows = rows, p.heads = heads, p.kv_heads = kv_heads, p.dim = dim, p.vdim = vdim, p.window = window, p.scale = scale, p.soft_cap = soft_cap, p.form = form, p.nseq = 1;
-    p.tiles = heads % kv_heads == 0 ? (rows * (heads / kv_heads) + 127) / 128 : 0;
+    p.tiles = heads % kv_heads == 0 ? (rows * (heads / kv_heads) + 127) / 128 : 0, p.tiles32 = heads % kv_heads == 0 ? (rows * (heads / kv_heads) + 31) / 32 : 0;
     if (form == 3) { // the matrix-core form with its key blocks split over workgroups + the merge launch
         float* ws = nullptr;
         p.form = 2, p.splits = 5;

@@ -160,6 +160,7 @@ template <int T> __global__ void __launch_bounds__(256) conv_rope_append_kernel(
 
 // ---- the simple form: a wave per (row, head).  Keys in blocks of 64 from the row's first visible key: a lane scores one key of the block (the whole dot
 // product, the query staged in LDS), the block's weights go through LDS, then a lane owns value coordinates lane, lane + 64, ... of the running sum.
+// What bounds it: the wait for a lone wave's loads; f32 caches are read 16 bytes and many loads at a time (300 rows of 8 heads, width 128: 82 -> 44 us).
 constexpr uint32_t kMaxVecPerLane = 8; // value widths up to 512
 __global__ void __launch_bounds__(64) window_attention_simple_kernel(WindowAttentionParams p) {
     extern __shared__ float s_mem[]; // [dim] query + [64] weights
@@ -206,7 +207,17 @@ __global__ void __launch_bounds__(64) window_attention_simple_kernel(WindowAtten
                 }
             } else {
                 const float* kr = (const float*)K + base;
-                for (uint32_t c = 0; c < p.dim; ++c) dot = fmaf(s_q[c], kr[c], dot);
+                if ((p.dim & 31) == 0 && (((uintptr_t)kr) & 15) == 0) { // (the same sum, 16 bytes a load and eight of them in flight)
+                    for (uint32_t c = 0; c < p.dim; c += 32) {
+                        f32x4_v kv[8];
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) kv[i] = *(const f32x4_v*)(kr + c + 4 * i);
+#pragma unroll
+                        for (int i = 0; i < 32; ++i) dot = fmaf(s_q[c + i], kv[i >> 2][i & 3], dot);
+                    }
+                } else {
+                    for (uint32_t c = 0; c < p.dim; ++c) dot = fmaf(s_q[c], kr[c], dot);
+                }
             }
             s = dot * hscale;
             if (p.soft_cap != 0.0f) s = p.soft_cap * tanhf(s / p.soft_cap);
@@ -227,7 +238,16 @@ __global__ void __launch_bounds__(64) window_attention_simple_kernel(WindowAtten
             if (c >= p.vdim) break;
             float sum = acc[i] * corr;
             const size_t vb = (size_t)j0 * vpitch + (size_t)g * p.vdim + c;
-            for (uint32_t jj = 0; jj < nk; ++jj) sum = fmaf(s_p[jj], cache_ld(V, p.cache_bf16, vb + (size_t)jj * vpitch), sum);
+            uint32_t jj = 0;
+            if (!p.cache_bf16) // (sixteen loads in flight: one a key and a wait behind it is what a lone wave spends its time on)
+                for (; jj + 16 <= nk; jj += 16) {
+                    float vv[16];
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) vv[u] = ((const float*)V)[vb + (size_t)(jj + u) * vpitch];
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) sum = fmaf(s_p[jj + u], vv[u], sum);
+                }
+            for (; jj < nk; ++jj) sum = fmaf(s_p[jj], cache_ld(V, p.cache_bf16, vb + (size_t)jj * vpitch), sum);
             acc[i] = sum;
         }
     }

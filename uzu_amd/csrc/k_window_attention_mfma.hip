@@ -1,8 +1,8 @@
 // k_window_attention_mfma.hip -- the matrix-core form of the attention over cached keys and values (kernels_stream32.h::window_attention): prompt-sized
 // passes over bf16 caches.
 //
-// Items are (row, query head) pairs of ONE sequence and ONE key / value head: a wave owns 32 of them, a workgroup 128, so with heads / kv_heads = 4 a
-// workgroup's 32 neighbouring rows share every staged block of 32 keys.  Both products are computed transposed with v_mfma_f32_32x32x16_bf16, so that a lane
+// Items are (row, query head) pairs of ONE sequence and ONE key / value head: a wave owns 32 of them, a workgroup of a prompt 128, so with heads / kv_heads = 4 a
+// workgroup's 32 neighbouring rows share every staged stretch of keys.  Both products are computed transposed with v_mfma_f32_32x32x16_bf16, so that a lane
 // owns one item:
 //   S^T = K Q^T     A = the key block [32][dim] from LDS, B = the item's query, rounded to bf16 as hi + lo (two products: the query keeps 16 significant bits);
 //                   the result gives a lane 16 key scores of ITS item, so scale, cap, mask and the running maximum / sum are per-lane work (one exchange
@@ -25,25 +25,41 @@ __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hi, uint3
     hi = (uint32_t)h0 | ((uint32_t)h1 << 16), lo = (uint32_t)l0 | ((uint32_t)l1 << 16);
 }
 
-// SPLIT (few items, many keys: decode steps): grid.z workgroups share an item tile's key blocks (block i goes to workgroup i mod grid.z) and leave unnormalised
-// sums with their running maximum / denominator in p.split_ws; window_attention_merge_kernel combines them.  The sink belongs to split 0.
-template <int NB, bool SPLIT> // dim and vdim padded to RP = 32 NB
-__global__ void __launch_bounds__(256) window_attention_mfma_kernel(WindowAttentionParams p) {
-    constexpr int RP = 32 * NB, KP = RP * 2 + 16, TP = 80, VEC = RP / 8;
+// IW waves of a workgroup own 32 items each, KG groups of such waves share the keys of a staged stretch (32 KG keys: group i takes its 32), so a workgroup is IW KG waves and
+// their unnormalised results meet in LDS at the end, in group order.  Prompts: IW 4, KG 2; a pass's tiles are about a workgroup per CU, and a wave alone on its SIMD waits for
+// itself at every exponential and every staged block (the next block's loads are in flight meanwhile; values are transposed two keys at a time).  2048 rows of 16 heads on 4,
+// width 128, window 1024: 147 us with four waves and no look-ahead, 61 so.  SPLIT (few items, many keys: decode steps): IW 1, KG 4, and grid.z
+// workgroups share an item tile's stretches (stretch i goes to workgroup i mod grid.z) and leave unnormalised sums with their running maximum / denominator in p.split_ws;
+// window_attention_merge_kernel combines them.  Tiles of 32 items then: with tiles of 128 three waves of four had none (8 sequences' step 25.6 us, now 14.0).  The sink belongs to
+// group 0 of split 0.
+template <int NB, int IW, int KG, bool SPLIT> // dim and vdim padded to RP = 32 NB
+__global__ void __launch_bounds__(64 * IW * KG) window_attention_mfma_kernel(WindowAttentionParams p) {
+    constexpr int RP = 32 * NB, KP = RP * 2 + 16, TP = 80, VEC = RP / 8, T = 64 * IW * KG, KEYS = 32 * KG;
+    constexpr int KN = (KEYS * VEC + T - 1) / T, VN = (KEYS / 2 * VEC + T - 1) / T; // 16-byte pieces of the keys / pairs of them of the values per thread
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    uint8_t* s_k = smem;             // [32 keys][KP bytes]
-    uint8_t* s_vt = smem + 32 * KP;  // [RP][TP bytes]: 32 keys + pad
+    uint8_t* s_k = smem;              // [KEYS][KP bytes]
+    uint8_t* s_vt = smem + KEYS * KP; // [KG][RP][TP bytes]: 32 keys + pad
     const uint32_t hg = p.heads / p.kv_heads, g = blockIdx.y;
-    uint32_t wg = blockIdx.x, z = 0;
-    SeqSpan sp{0, 0, 0};
-    for (;; ++z) {
-        if (z >= p.nseq) return;
-        sp = p.spans[z];
-        const uint32_t n = (sp.count * hg + 127) / 128;
-        if (wg < n) break;
-        wg -= n;
+    // the sequence of this tile (tiles of ITEMS items): a lane per sequence, 64 at a time
+    constexpr uint32_t ITEMS = 32 * IW;
+    uint32_t wg = blockIdx.x, z = 0xFFFFFFFFu, before = 0;
+    for (uint32_t z0 = 0; z0 < p.nseq && z == 0xFFFFFFFFu; z0 += 64) {
+        const uint32_t ln = threadIdx.x & 63;
+        uint32_t upto = z0 + ln < p.nseq ? (p.spans[z0 + ln].count * hg + ITEMS - 1) / ITEMS : 0u;
+        for (uint32_t o = 1; o < 64; o <<= 1) {
+            const uint32_t below = __shfl_up(upto, o, 64);
+            if (ln >= o) upto += below;
+        }
+        const unsigned long long behind = __ballot(before + upto > wg);
+        const uint32_t i = behind ? (uint32_t)__builtin_ctzll(behind) : 64u;
+        before += i ? (uint32_t)__builtin_amdgcn_readlane((int)upto, (int)i - 1) : 0u;
+        if (behind) z = z0 + i;
     }
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, half = lane >> 5;
+    if (z == 0xFFFFFFFFu) return;
+    wg -= before;
+    const SeqSpan sp = p.spans[z];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6) % IW, kg = __builtin_amdgcn_readfirstlane(tid >> 6) / IW; // (item block, key group)
     const uint32_t items = sp.count * hg;
     auto row_lo = [&](uint32_t t) { // the first key the row at position t sees: the window's edge or its chunk's start, whichever is later
         uint32_t lo = (p.window && t + 1 > p.window) ? t + 1 - p.window : 0u;
@@ -51,15 +67,15 @@ __global__ void __launch_bounds__(256) window_attention_mfma_kernel(WindowAttent
         return lo;
     };
     // this lane's item
-    const uint32_t it = wg * 128 + wave * 32 + l32;
+    const uint32_t it = wg * ITEMS + wave * 32 + l32;
     const bool valid = it < items;
     const uint32_t gi = valid ? it : items - 1;
     const uint32_t row = gi / hg, head = g * hg + gi % hg;
     const uint32_t t = sp.start + row, lo = row_lo(t);
     // key ranges of the workgroup and of this wave
-    const uint32_t g_last = (wg * 128 + 128 < items ? wg * 128 + 128 : items) - 1;
-    const uint32_t kmin = row_lo(sp.start + wg * 128 / hg), kmax = sp.start + g_last / hg;
-    const uint32_t w_first = wg * 128 + wave * 32;
+    const uint32_t g_last = (wg * ITEMS + ITEMS < items ? wg * ITEMS + ITEMS : items) - 1;
+    const uint32_t kmin = row_lo(sp.start + wg * ITEMS / hg), kmax = sp.start + g_last / hg;
+    const uint32_t w_first = wg * ITEMS + wave * 32;
     const bool wave_on = w_first < items;
     const uint32_t w_last = (w_first + 32 < items ? w_first + 32 : items) - 1;
     const uint32_t wave_lo = wave_on ? row_lo(sp.start + w_first / hg) : 0, wave_hi = wave_on ? sp.start + w_last / hg : 0;
@@ -80,7 +96,7 @@ __global__ void __launch_bounds__(256) window_attention_mfma_kernel(WindowAttent
             qh[s] = fh, ql[s] = fl;
         }
     }
-    const bool with_sink = p.sinks && (!SPLIT || blockIdx.z == 0);
+    const bool with_sink = p.sinks && kg == 0 && (!SPLIT || blockIdx.z == 0);
     float m_run = with_sink ? p.sinks[head] : -1.0e30f;
     float l_run = with_sink ? 1.0f : 0.0f;
     f32x16_t o[NB];
@@ -94,32 +110,56 @@ __global__ void __launch_bounds__(256) window_attention_mfma_kernel(WindowAttent
     const float inv_cap = p.soft_cap != 0.0f ? 1.0f / p.soft_cap : 0.0f;
     const float hscale = p.head_scale ? p.scale * p.head_scale[head] : p.scale;
 
-    const uint32_t kstep = SPLIT ? 32 * gridDim.z : 32;
-    for (uint32_t kb = kmin + (SPLIT ? 32 * blockIdx.z : 0); kb <= kmax; kb += kstep) {
-        __syncthreads(); // the block before has been read
-        for (uint32_t v = tid; v < 32 * VEC; v += 256) {
-            const uint32_t key = v / VEC, e0 = (v % VEC) * 8, kk = kb + key;
-            u32x4_v kv{0u, 0u, 0u, 0u}, vv{0u, 0u, 0u, 0u};
-            if (kk <= kmax) {
-                if (e0 < p.dim) kv = *(const u32x4_v*)(kc + ((size_t)kk * kpitch + (size_t)g * p.dim + e0) * 2);
-                if (e0 < p.vdim) vv = *(const u32x4_v*)(vc + ((size_t)kk * vpitch + (size_t)g * p.vdim + e0) * 2);
-            }
-            *(u32x4_v*)(s_k + key * KP + e0 * 2) = kv;
-            const uint32_t w[4] = {vv.x, vv.y, vv.z, vv.w};
+    u32x4_v kr[KN], vr[VN][2];
+    auto fetch = [&](uint32_t base) { // (keys behind the last: zeros)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                *(uint16_t*)(s_vt + (e0 + 2 * e) * TP + key * 2) = (uint16_t)(w[e] & 0xFFFFu);
-                *(uint16_t*)(s_vt + (e0 + 2 * e + 1) * TP + key * 2) = (uint16_t)(w[e] >> 16);
+        for (int i = 0; i < KN; ++i) {
+            const uint32_t v = tid + i * T, kk = base + v / VEC, e0 = v % VEC * 8;
+            kr[i] = u32x4_v{0u, 0u, 0u, 0u};
+            if (v < KEYS * VEC && kk <= kmax && e0 < p.dim) kr[i] = *(const u32x4_v*)(kc + ((size_t)kk * kpitch + (size_t)g * p.dim + e0) * 2);
+        }
+#pragma unroll
+        for (int i = 0; i < VN; ++i) {
+            const uint32_t v = tid + i * T, e0 = v / 16 % VEC * 8;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const uint32_t kk = base + v / (16 * VEC) * 32 + v % 16 * 2 + j;
+                vr[i][j] = u32x4_v{0u, 0u, 0u, 0u};
+                if (v < KEYS / 2 * VEC && kk <= kmax && e0 < p.vdim) vr[i][j] = *(const u32x4_v*)(vc + ((size_t)kk * vpitch + (size_t)g * p.vdim + e0) * 2);
             }
         }
+    };
+    const uint32_t kstep = SPLIT ? KEYS * gridDim.z : KEYS, kfirst = kmin + (SPLIT ? KEYS * blockIdx.z : 0);
+    if (kfirst <= kmax) fetch(kfirst);
+    for (uint32_t kb0 = kfirst; kb0 <= kmax; kb0 += kstep) {
+        __syncthreads(); // the stretch before has been read
+#pragma unroll
+        for (int i = 0; i < KN; ++i) {
+            const uint32_t v = tid + i * T;
+            if (v < KEYS * VEC) *(u32x4_v*)(s_k + v / VEC * KP + v % VEC * 16) = kr[i];
+        }
+#pragma unroll
+        for (int i = 0; i < VN; ++i) { // two keys' elements side by side: 16 lanes write 64 bytes of a transposed row
+            const uint32_t v = tid + i * T;
+            if (v < KEYS / 2 * VEC) {
+                uint8_t* to = s_vt + (v / (16 * VEC) * RP + v / 16 % VEC * 8) * TP + v % 16 * 4;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    *(uint32_t*)(to + (2 * e) * TP) = (vr[i][0][e] & 0xFFFFu) | (vr[i][1][e] << 16);
+                    *(uint32_t*)(to + (2 * e + 1) * TP) = (vr[i][0][e] >> 16) | (vr[i][1][e] & 0xFFFF0000u);
+                }
+            }
+        }
+        if (kb0 + kstep <= kmax) fetch(kb0 + kstep);
         __syncthreads();
+        const uint32_t kb = kb0 + 32 * kg;
         if (!wave_on || kb > wave_hi || kb + 31 < wave_lo) continue; // (wave-uniform; the barriers above are reached by every wave)
         f32x16_t st;
 #pragma unroll
         for (int r = 0; r < 16; ++r) st[r] = 0.0f;
 #pragma unroll
         for (int s = 0; s < 2 * NB; ++s) {
-            const u32x4_t a = *(const u32x4_t*)(s_k + l32 * KP + (s * 16 + half * 8) * 2);
+            const u32x4_t a = *(const u32x4_t*)(s_k + (32 * kg + l32) * KP + (s * 16 + half * 8) * 2);
             st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, qh[s]), st, 0, 0, 0);
             st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, ql[s]), st, 0, 0, 0);
         }
@@ -161,12 +201,37 @@ __global__ void __launch_bounds__(256) window_attention_mfma_kernel(WindowAttent
             const u32x4_t hi{hw[0], hw[1], hw[2], hw[3]}, lw{lwv[0], lwv[1], lwv[2], lwv[3]};
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                const uint8_t* cr = s_vt + (b * 32 + l32) * TP + (16 * s2 + 4 * half) * 2;
+                const uint8_t* cr = s_vt + (kg * RP + b * 32 + l32) * TP + (16 * s2 + 4 * half) * 2;
                 const u32x2_v c0 = *(const u32x2_v*)cr, c1 = *(const u32x2_v*)(cr + 16);
                 const u32x4_t cf{c0.x, c0.y, c1.x, c1.y};
                 o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, cf), __builtin_bit_cast(bf16x8_t, hi), o[b], 0, 0, 0);
                 o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, cf), __builtin_bit_cast(bf16x8_t, lw), o[b], 0, 0, 0);
             }
+        }
+    }
+    if (KG > 1) { // the groups' results: [group - 1][item block][value][lane], behind them the maxima and sums
+        float* s_o = (float*)smem;
+        constexpr int PER = (16 * NB + 2) * 64;
+        __syncthreads();
+        if (kg) {
+            float* mine = s_o + ((kg - 1) * IW + wave) * PER + lane;
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mine[(b * 16 + r) * 64] = o[b][r];
+            mine[16 * NB * 64] = m_run, mine[(16 * NB + 1) * 64] = l_run;
+        }
+        __syncthreads();
+        if (kg) return;
+#pragma unroll
+        for (int other = 0; other < KG - 1; ++other) {
+            const float* theirs = s_o + (other * IW + wave) * PER + lane;
+            const float m_o = theirs[16 * NB * 64], l_o = theirs[(16 * NB + 1) * 64], m_new = fmaxf(m_run, m_o), a = fast_exp(m_run - m_new), c = fast_exp(m_o - m_new);
+            l_run = l_run * a + l_o * c, m_run = m_new;
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[b][r] = fmaf(theirs[(b * 16 + r) * 64], c, o[b][r] * a);
         }
     }
     if (!valid) return;
@@ -229,7 +294,7 @@ size_t window_attention_split_ws_bytes(uint32_t rows, uint32_t heads, uint32_t s
 // bf16 caches, head widths that are multiples of 8 up to 128 (16-byte rows); prompt-sized passes, or a decode-sized pass with a workspace to split its keys
 // (without one a decode step's few items would walk all their keys in one nearly empty workgroup: the simple form does that better)
 static bool use_split(const WindowAttentionParams& p) {
-    return p.splits > 1 && p.splits <= 64 && p.split_ws && p.split_ws_bytes >= window_attention_split_ws_bytes(p.rows, p.heads, p.splits);
+    return p.splits > 1 && p.splits <= 64 && p.tiles32 && p.split_ws && p.split_ws_bytes >= window_attention_split_ws_bytes(p.rows, p.heads, p.splits);
 }
 
 bool window_attention_mfma_supported(const WindowAttentionParams& p) {
@@ -238,26 +303,25 @@ bool window_attention_mfma_supported(const WindowAttentionParams& p) {
            (split || p.rows >= 16 * p.nseq) && p.kv_heads <= 65535 && ((uintptr_t)p.q & 15) == 0 && ((uintptr_t)p.out & 15) == 0;
 }
 
+template <int NB, int IW, int KG, bool SPLIT> static uzu_status launch(hipStream_t s, const WindowAttentionParams& p) {
+    constexpr size_t stage = (size_t)32 * KG * (32 * NB * 2 + 16) + (size_t)KG * 32 * NB * 80, meet = (size_t)(KG - 1) * IW * (16 * NB + 2) * 256, lds = stage > meet ? stage : meet;
+    static LdsLimit lim;
+    UZU_REQUIRE(raise_lds_limit(lim, (const void*)window_attention_mfma_kernel<NB, IW, KG, SPLIT>, lds), "window_attention_mfma: %zu bytes of LDS are not available", lds);
+    return launch_check([&] { hipLaunchKernelGGL((window_attention_mfma_kernel<NB, IW, KG, SPLIT>), dim3(IW == 1 ? p.tiles32 : p.tiles, p.kv_heads, SPLIT ? p.splits : 1), dim3(64 * IW * KG), lds, s, p); },
+                        SPLIT ? "window_attention_mfma_split" : "window_attention_mfma");
+}
+
 uzu_status window_attention_mfma(hipStream_t s, const WindowAttentionParams& p) {
     UZU_REQUIRE(window_attention_mfma_supported(p), "window_attention: the matrix-core form does not take this shape");
     const uint32_t nb = blocks_of(p);
-    const size_t lds = (size_t)32 * (32 * nb * 2 + 16) + (size_t)32 * nb * 80;
     if (use_split(p)) {
-        const dim3 grid(p.tiles, p.kv_heads, p.splits);
-#define UZU_WA(NB) UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL((window_attention_mfma_kernel<NB, true>), grid, dim3(256), lds, s, p); }, "window_attention_mfma_split"))
-        if (nb == 1) UZU_WA(1);
-        else if (nb == 2) UZU_WA(2);
-        else UZU_WA(4);
-#undef UZU_WA
+        if (nb == 1) UZU_PROPAGATE((launch<1, 1, 4, true>(s, p)));
+        else if (nb == 2) UZU_PROPAGATE((launch<2, 1, 4, true>(s, p)));
+        else UZU_PROPAGATE((launch<4, 1, 4, true>(s, p)));
         return launch_check([&] { hipLaunchKernelGGL(window_attention_merge_kernel, dim3(p.rows * p.heads), dim3(128), 0, s, (const float*)p.split_ws, p.out, p.splits, p.vdim, 32 * nb, p.gate, p.ldgate, p.heads, p.ldo, p.out_scale); },
                             "window_attention_merge");
     }
-    const dim3 grid(p.tiles, p.kv_heads);
-#define UZU_WA(NB) return launch_check([&] { hipLaunchKernelGGL((window_attention_mfma_kernel<NB, false>), grid, dim3(256), lds, s, p); }, "window_attention_mfma")
-    if (nb == 1) UZU_WA(1);
-    if (nb == 2) UZU_WA(2);
-    UZU_WA(4);
-#undef UZU_WA
+    return nb == 1 ? launch<1, 4, 2, false>(s, p) : nb == 2 ? launch<2, 4, 2, false>(s, p) : launch<4, 4, 2, false>(s, p);
 }
 
 } // namespace k
