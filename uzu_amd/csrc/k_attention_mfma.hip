@@ -45,7 +45,7 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
 __device__ __forceinline__ float other_half(float v) { return __shfl_xor(v, 32, 64); }
 } // namespace
 
-// grid: (kv heads, ceil(gqa * query tiles / tpw)); 256 threads.  Workgroups with the longest key ranges are numbered first.
+// grid: (kv heads, ceil(gqa * query tiles / tpw)); 256 KG threads.  Workgroups with the longest key ranges are numbered first.
 // tpw = wave tasks per workgroup (4, 2 or 1): models with few heads (Qwen3.5-0.8B: 8 q heads -> 256 tasks per 1024-token chunk)
 // would fill 64 CUs at four tasks per workgroup; with fewer tasks the idle waves still help staging the K / V tiles.
 // Key split (few-head models: Qwen3.5-0.8B has 2 kv heads -> 64 workgroups of four tasks per 1024-token chunk): gridDim.z workgroups share a
@@ -55,16 +55,24 @@ __device__ __forceinline__ float other_half(float v) { return __shfl_xor(v, 32, 
 // ring of `prefix` slots, key position = (prefix + i - ring_offset) mod prefix, live iff < ring_length) and attention sinks (the running
 // maximum starts at the head's sink logit with a unit of mass: attention_single_pass.rs:70-74) -- evaluated per key on its POSITION; the
 // plain causal instantiation keeps its one comparison per key.
-template <int HD, bool GEN>
-__global__ void __launch_bounds__(256) attention_prefill_mfma_kernel(AttentionParams a, uint16_t* out, uint32_t tpw, float* part_o, float* part_ml) {
+// KG groups of four waves share a stretch of 32 KG keys, a wave takes its group's 32 of them, and the groups' unnormalised results meet in LDS at the end, in group order: the
+// grid is about a workgroup per CU, and a wave alone on its SIMD waits for itself at every exponential (1021 rows of 32 heads of 128: 72 us with one group, 39 with
+// two).  Heads of 256 need the registers of a wave alone.
+template <int HD, bool GEN, int KG = HD <= 128 ? 2 : 1>
+__global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(AttentionParams a, uint16_t* out, uint32_t tpw, float* part_o, float* part_ml) {
     constexpr int KP = HD * 2 + 16;  // K tile row pitch in bytes (conflict-free ds_read_b128)
     constexpr int VP = TK * 2 + 8;   // V^T tile row pitch in bytes: 32 keys + 8 bytes of pad (conflict-free ds_read_b64)
     constexpr int NS = HD / 16;      // k16 steps of the QK^T contraction
     constexpr int NB = HD / 32;      // 32-row blocks of O^T
-    __shared__ __attribute__((aligned(16))) uint8_t s_k[2][TK * KP];
-    __shared__ __attribute__((aligned(16))) uint8_t s_vt[2][HD * VP];
+    constexpr int T = 256 * KG, KEYS = TK * KG, VEC = HD / 8;
+    constexpr int KB = KEYS * KP, VB = KG * HD * VP; // a stretch's keys / values in LDS
+    constexpr int PER = (16 * NB + 2) * 64;          // floats of a wave's result
+    static_assert(KG == 1 || 4 * (KG - 1) * PER * 4 <= 2 * (KB + VB), "the groups' results fit where the keys and values were");
+    __shared__ __attribute__((aligned(16))) uint8_t s_mem[2 * (KB + VB)];
+    auto s_k = [&](int buf) { return s_mem + buf * KB; };
+    auto s_vt = [&](int buf) { return s_mem + 2 * KB + buf * VB; };
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5, l32 = lane & 31;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, kg = __builtin_amdgcn_readfirstlane(tid >> 8), half = lane >> 5, l32 = lane & 31;
     const uint32_t M = a.suffix_length;
     const uint32_t kv_head = blockIdx.x;
     const uint32_t n_tasks = a.gqa_factor * ((M + TQ - 1) / TQ);
@@ -92,54 +100,51 @@ __global__ void __launch_bounds__(256) attention_prefill_mfma_kernel(AttentionPa
         }
     }
 
-    // ---- staging role: thread -> (key of the tile, 64-byte slice of its hd row)
+    // ---- staging role: thread -> 16 bytes of a key's row; 16 bytes of two neighbouring keys' values
     const uint16_t* kbase = (const uint16_t*)a.keys + (size_t)kv_head * a.k_head_stride;
     const uint16_t* vbase = (const uint16_t*)a.values + (size_t)kv_head * a.v_head_stride;
-    constexpr int SLICES = HD / 32;               // 32 hd elements (64 bytes) per slice
-    constexpr int ROUNDS = (TK * SLICES + 255) / 256;
-    u32x4_v kst[ROUNDS][4], vst[ROUNDS][4]; // native vectors + unconditional loads: stay in registers and in flight across lds_barrier()
+    constexpr int KN = KEYS * VEC / T, VN = (KEYS / 2 * VEC + T - 1) / T;
+    u32x4_v kst[KN], vst[VN][2]; // native vectors + unconditional loads: stay in registers and in flight across lds_barrier()
     // keys visible to ANY query of the workgroup: 0 .. prefix + last query of its last live task (tasks are tile-major)
     const uint32_t last_tile = ((task0 + tpw - 1 < n_tasks ? task0 + tpw - 1 : n_tasks - 1) / a.gqa_factor + 1) * TQ;
     const uint32_t wg_last_q = (last_tile < M ? last_tile : M) - 1;
     const uint32_t key_end = prefix + wg_last_q + 1;
-    const uint32_t n_tiles_all = (key_end + TK - 1) / TK;
+    const uint32_t n_tiles_all = (key_end + KEYS - 1) / KEYS; // (tiles of the workgroup: stretches of KEYS)
     const uint32_t per_split = (n_tiles_all + gridDim.z - 1) / gridDim.z;
     const uint32_t t_lo = min(blockIdx.z * per_split, n_tiles_all), n_tiles = min(t_lo + per_split, n_tiles_all); // this workgroup: tiles [t_lo, n_tiles)
     auto load_tile = [&](uint32_t t) {
+        const u32x4_v zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int r = 0; r < ROUNDS; ++r) {
-            const uint32_t idx = tid + 256 * r, key = idx / SLICES, sl = idx % SLICES;
-            const uint32_t i = t * TK + key;
-            const bool live = idx < TK * SLICES && i < key_end;
-            const uint32_t ic = i < key_end ? i : key_end - 1; // clamped row: masked keys get probability 0 anyway, zeroed for hygiene
-            const u32x4_v* ks = (const u32x4_v*)(kbase + (size_t)ic * a.k_seq_stride + (sl % SLICES) * 32);
-            const u32x4_v* vs = (const u32x4_v*)(vbase + (size_t)ic * a.v_seq_stride + (sl % SLICES) * 32);
-            const u32x4_v zero = {0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const u32x4_v kk = ks[j], vv = vs[j];
-                kst[r][j] = live ? kk : zero, vst[r][j] = live ? vv : zero;
-            }
+        for (int r = 0; r < KN; ++r) {
+            const uint32_t v = tid + r * T, i = t * KEYS + v / VEC;
+            const u32x4_v kk = *(const u32x4_v*)(kbase + (size_t)(i < key_end ? i : key_end - 1) * a.k_seq_stride + v % VEC * 8); // clamped row: masked keys get probability 0 anyway, zeroed for hygiene
+            kst[r] = i < key_end ? kk : zero;
         }
+#pragma unroll
+        for (int r = 0; r < VN; ++r)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const uint32_t v = min((uint32_t)(tid + r * T), (uint32_t)(KEYS / 2 * VEC - 1)), i = t * KEYS + v / (16 * VEC) * TK + v % 16 * 2 + j;
+                const u32x4_v vv = *(const u32x4_v*)(vbase + (size_t)(i < key_end ? i : key_end - 1) * a.v_seq_stride + v / 16 % VEC * 8);
+                vst[r][j] = i < key_end ? vv : zero;
+            }
     };
     auto store_tile = [&](int buf) {
 #pragma unroll
-        for (int r = 0; r < ROUNDS; ++r) {
-            const uint32_t idx = tid + 256 * r, key = idx / SLICES, sl = idx % SLICES;
-            if (idx >= TK * SLICES) continue;
-            uint8_t* kd = &s_k[buf][key * KP + sl * 64];
+        for (int r = 0; r < KN; ++r) {
+            const uint32_t v = tid + r * T;
+            *(u32x4_v*)(s_k(buf) + v / VEC * KP + v % VEC * 16) = kst[r];
+        }
+        // V transposed, two keys' elements side by side: 16 lanes write 64 bytes of a row (element by element was 64 two-byte stores a thread, eight to a bank)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) *(u32x4_v*)(kd + 16 * j) = kst[r][j];
-            // V transposed: element (key, hd) -> s_vt[hd][key]
+        for (int r = 0; r < VN; ++r) {
+            const uint32_t v = tid + r * T;
+            if (v >= (uint32_t)(KEYS / 2 * VEC)) continue;
+            uint8_t* to = s_vt(buf) + (v / (16 * VEC) * HD + v / 16 % VEC * 8) * VP + v % 16 * 4;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t w[4] = {vst[r][j][0], vst[r][j][1], vst[r][j][2], vst[r][j][3]};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t hd0 = sl * 32 + j * 8 + 2 * e;
-                    *(uint16_t*)&s_vt[buf][hd0 * VP + key * 2] = (uint16_t)(w[e] & 0xFFFFu);
-                    *(uint16_t*)&s_vt[buf][(hd0 + 1) * VP + key * 2] = (uint16_t)(w[e] >> 16);
-                }
+            for (int e = 0; e < 4; ++e) {
+                *(uint32_t*)(to + (2 * e) * VP) = (vst[r][0][e] & 0xFFFFu) | (vst[r][1][e] << 16);
+                *(uint32_t*)(to + (2 * e + 1) * VP) = (vst[r][0][e] >> 16) | (vst[r][1][e] & 0xFFFF0000u);
             }
         }
     };
@@ -152,7 +157,7 @@ __global__ void __launch_bounds__(256) attention_prefill_mfma_kernel(AttentionPa
     float m_run = -INFINITY, l_run = 0.f; // l_run: this lane's half of the keys only (merged at the end)
     const uint32_t my_last_key = prefix + qi; // causal: keys 0 .. prefix + qi
     if constexpr (GEN) {
-        if (a.sinks && blockIdx.z == 0) { // the sink's unit of mass is counted once: by half 0 of the first key split
+        if (a.sinks && blockIdx.z == 0 && kg == 0) { // the sink's unit of mass is counted once: by half 0 of the first group of the first key split
             m_run = bf16_to_f32(((const uint16_t*)a.sinks)[head]);
             l_run = half == 0 ? 1.0f : 0.0f;
         }
@@ -169,12 +174,13 @@ __global__ void __launch_bounds__(256) attention_prefill_mfma_kernel(AttentionPa
         load_tile(t + 1 < n_tiles ? t + 1 : t); // unconditional: the compiler can count the loads in flight
         // a wave whose queries all end before this tile has nothing to add (causal), but must keep the barriers
         const uint32_t wave_last_key = prefix + (q0 + TQ - 1 < M ? q0 + TQ - 1 : M - 1);
-        if (wave_live && t * TK <= wave_last_key) {
+        const uint32_t kb = t * KEYS + kg * TK; // this group's first key
+        if (wave_live && kb <= wave_last_key) {
             // ---- S^T = K Q^T
             f32x16_t sacc;
 #pragma unroll
             for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
-            const uint8_t* kt = &s_k[buf][l32 * KP + half * 16];
+            const uint8_t* kt = s_k(buf) + (kg * TK + l32) * KP + half * 16;
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
                 const uint4 kv = *(const uint4*)(kt + s * 32);
@@ -186,7 +192,7 @@ __global__ void __launch_bounds__(256) attention_prefill_mfma_kernel(AttentionPa
             float m_loc = -INFINITY;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const uint32_t key = t * TK + (r & 3) + 8 * (r >> 2) + 4 * half;
+                const uint32_t key = kb + (r & 3) + 8 * (r >> 2) + 4 * half;
                 bool vis = q_live && key <= my_last_key;
                 if constexpr (GEN) { // mask.rs:31-60 on positions
                     uint32_t key_position;
@@ -230,7 +236,7 @@ __global__ void __launch_bounds__(256) attention_prefill_mfma_kernel(AttentionPa
 #pragma unroll
                 for (int b = 0; b < NB; ++b) {
                     // A = V^T: lane = (hd row b*32 + l32, half): keys 16 st + 4 half + {0..3} and 16 st + 8 + 4 half + {0..3}
-                    const uint8_t* vr = &s_vt[buf][(b * 32 + l32) * VP + (16 * st + 4 * half) * 2];
+                    const uint8_t* vr = s_vt(buf) + (kg * HD + b * 32 + l32) * VP + (16 * st + 4 * half) * 2;
                     const uint2 v0 = *(const uint2*)vr, v1 = *(const uint2*)(vr + 16);
                     const u32x4_t vfrag = {v0.x, v0.y, v1.x, v1.y};
                     o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vfrag), __builtin_bit_cast(bf16x8_t, ph), o[b], 0, 0, 0);
@@ -240,6 +246,30 @@ __global__ void __launch_bounds__(256) attention_prefill_mfma_kernel(AttentionPa
         }
         if (t + 1 < n_tiles) store_tile(buf ^ 1);
         lds_barrier();
+    }
+    if constexpr (KG > 1) { // (every wave is past the last barrier: the stretches have been read)
+        float* s_o = (float*)s_mem;
+        if (kg) {
+            float* mine = s_o + ((kg - 1) * 4 + wave) * PER + lane;
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mine[(b * 16 + r) * 64] = o[b][r];
+            mine[16 * NB * 64] = m_run, mine[(16 * NB + 1) * 64] = l_run;
+        }
+        __syncthreads();
+        if (kg) return;
+#pragma unroll
+        for (int other = 0; other < KG - 1; ++other) {
+            const float* theirs = s_o + (other * 4 + wave) * PER + lane;
+            const float m_o = theirs[16 * NB * 64], l_o = theirs[(16 * NB + 1) * 64], m_new = fmaxf(m_run, m_o);
+            const float x = m_run == -INFINITY ? 0.f : fast_exp(m_run - m_new), y = m_o == -INFINITY ? 0.f : fast_exp(m_o - m_new); // (a group that saw no key: m = -inf, l = 0)
+            l_run = l_run * x + l_o * y, m_run = m_new;
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[b][r] = fmaf(theirs[(b * 16 + r) * 64], y, o[b][r] * x);
+        }
     }
     // ---- finish: l = both halves' sums (same maximum), out[q][head][hd] = O / l
     const float l_tot = l_run + other_half(l_run);
@@ -376,8 +406,8 @@ uzu_status attention_prefill_mfma(hipStream_t s, const AttentionParams& a, void*
 #define UZU_LAUNCH(H)                                                                                                                                              \
     {                                                                                                                                                              \
         UZU_PROPAGATE(launch_check([&] {                                                                                                                           \
-            if (general) hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, true>), grid, dim3(256), 0, s, a, (uint16_t*)out, tpw, part_o, part_ml);             \
-            else hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, false>), grid, dim3(256), 0, s, a, (uint16_t*)out, tpw, part_o, part_ml);                    \
+            if (general) hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, true>), grid, dim3(H <= 128 ? 512 : 256), 0, s, a, (uint16_t*)out, tpw, part_o, part_ml);             \
+            else hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, false>), grid, dim3(H <= 128 ? 512 : 256), 0, s, a, (uint16_t*)out, tpw, part_o, part_ml);                    \
         }, "attention_prefill_mfma"));                                                                                                                             \
         if (!part) return UZU_OK;                                                                                                                                  \
         if (gate && gate_done) *gate_done = 1;                                                                                                                     \
