@@ -441,6 +441,27 @@ def test_attention_prepare_bit_exact(hip_ctx):
     assert np.array_equal(bv.download(np.uint16, wv.size).reshape(wv.shape), wv)
 
 
+@pytest.mark.parametrize("nq,nkv,hd,rope_dim,batch,has_kv", [(32, 8, 128, 128, 5, 1), (3, 1, 16, 16, 1, 1), (4, 2, 64, 0, 33, 1), (5, 5, 48, 48, 7, 1), (0, 2, 256, 256, 3, 1), (6, 2, 64, 64, 9, 0)])
+def test_attention_prepare_whole_heads_bit_exact(hip_ctx, nq, nkv, hd, rope_dim, batch, has_kv):
+    """Heads rotated as a whole or not at all (16 bytes a load): one pair of pieces a head and many, units that fill no workgroup, without queries, without keys and values; the oracle's bits."""
+    rng = np.random.default_rng(hd + batch)
+    off, cap, heads = 3, 40, nq + 2 * nkv if has_kv else nq
+    qkv = bf16(rng.normal(0, 1, size=(batch, heads * hd)))
+    cos = rng.uniform(-1, 1, size=(batch, max(rope_dim, 1))).astype(np.float32)
+    sin = rng.uniform(-1, 1, size=(batch, max(rope_dim, 1))).astype(np.float32)
+    wq = np.zeros((max(nq, 1), batch, hd), np.uint16)
+    wk = np.full((cap, nkv * hd), 0x1234, np.uint16)
+    wv = wk.copy()
+    O.call("orc_attention_prepare", qkv, wq, wk, wv, cos, sin, nq, nkv, hd, rope_dim, off, batch, has_kv)
+    kern = B.AttentionPrepareKernel.new(hip_ctx, B.BF16, B.F32, has_kv, 1 if rope_dim else 0)
+    bq, bk, bv = hip_ctx.buffer_from(np.zeros_like(wq)), hip_ctx.buffer_from(np.full((cap, nkv * hd), 0x1234, np.uint16)), hip_ctx.buffer_from(np.full((cap, nkv * hd), 0x1234, np.uint16))
+    bqkv, bc, bs = hip_ctx.buffer_from(qkv), hip_ctx.buffer_from(cos), hip_ctx.buffer_from(sin)
+    run(hip_ctx, lambda cb: kern.encode(bqkv, bq, bk if has_kv else None, bv if has_kv else None, bc if rope_dim else None, bs if rope_dim else None, nq, nkv, hd, rope_dim, off, batch, cb))
+    assert np.array_equal(bq.download(np.uint16, wq.size).reshape(wq.shape), wq)
+    assert np.array_equal(bk.download(np.uint16, wk.size).reshape(wk.shape), wk)
+    assert np.array_equal(bv.download(np.uint16, wv.size).reshape(wv.shape), wv)
+
+
 def test_gated_act_mul_reference_kat_and_bit_exact(hip_ctx):
     """(a) the one literal known-answer test of the reference tree (gated_act_mul_test.rs:139-160):
     non-interleaved, IDENTITY, gate [1,2,3,4], value rows with offset 2 / stride 6 -> [10,40,150,240];
