@@ -13,11 +13,25 @@
 // MI355X execution strategy: weights, KV cache and DeltaNet state resident in HBM; the context length,
 // the next input token and the sampled-token history live in device memory, so ONE captured hipGraph is
 // replayed for every decode step and steps are chained without a host round trip.
+#include <algorithm>
+
 #include "engine_types.h"
 #include "uzu_math.h"
 
 using namespace uzu;
 using namespace uzu::eng;
+
+namespace {
+// the control block behind an accepted path: the tokens at their positions, the next input token, the context length
+struct AcceptedTokens {
+    static constexpr uint32_t kMost = 256;
+    uint32_t token[kMost];
+};
+__global__ void __launch_bounds__(64) accept_commit_kernel(uint32_t* ctx_len, uint32_t* next, uint32_t* out_token, uint32_t* sampled, AcceptedTokens t, uint32_t count, uint32_t new_len) {
+    for (uint32_t i = threadIdx.x; i < count; i += 64) sampled[i] = t.token[i];
+    if (threadIdx.x == 0) *next = *out_token = t.token[count - 1], *ctx_len = new_len;
+}
+} // namespace
 
 extern "C" {
 
@@ -460,6 +474,7 @@ uzu_status uzu_hip_model_accept(uzu_hip_model* m, const uint32_t* accepted_indic
     std::vector<uzu_kv_copy> copies;
     for (uint32_t i = 0; i < count; ++i)
         if (accepted_indices[i] != i) copies.push_back({m->context_length + accepted_indices[i], m->context_length + i});
+    std::vector<CopyBlock> conv_states;
     for (size_t l = 0; l < m->layers.size(); ++l) {
         DLayer& L = m->layers[l];
         if (L.d.mixer_kind == UZU_MIXER_ATTENTION && L.d.is_kv_sharing) continue; // TransformerLayerStateType::Shared: nothing of its own to accept (transformer.rs:63-69)
@@ -474,20 +489,28 @@ uzu_status uzu_hip_model_accept(uzu_hip_model* m, const uint32_t* accepted_indic
             if (!copies.empty()) RUN("kv_cache_update", 0, k::kv_cache_update(s, L.keys, L.values, UZU_BF16, copies.data(), (uint32_t)copies.size(), L.d.num_groups * L.d.head_dim));
         } else {
             const auto& T = m->tree.layers[l];
-            HIPCHK(hipMemcpyAsync(L.conv_state, (const char*)T.conv_states + (size_t)accepted_indices[count - 1] * L.conv_state_bytes, L.conv_state_bytes, hipMemcpyDeviceToDevice, s));
+            conv_states.push_back({L.conv_state, (const char*)T.conv_states + (size_t)accepted_indices[count - 1] * L.conv_state_bytes, L.conv_state_bytes});
             RUN("dn_state_advance", L.ssm_state_bytes * 2, k::delta_net_state_advance(s, T.k, T.v, T.log_decay, T.beta, m->tree.d_accepted, L.ssm_state, count, L.d.dn_num_heads,
                                                                                      L.d.dn_num_groups, L.d.dn_head_dim));
         }
     }
     UZU_PROPAGATE(e.st);
+    UZU_PROPAGATE(copy_blocks(s, conv_states));
     // control block: context length, the sampled tokens of the accepted nodes at their positions, the next input token
     std::vector<uint32_t> toks(count);
     for (uint32_t i = 0; i < count; ++i) toks[i] = m->tree.sampled[accepted_indices[i]];
     const uint32_t new_len = m->context_length + count;
-    HIPCHK(hipMemcpyAsync(m->d_sampled + m->context_length, toks.data(), (size_t)count * 4, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(m->d_tokens, &toks[count - 1], 4, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(m->d_out_token, &toks[count - 1], 4, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(m->d_ctx_len, &new_len, 4, hipMemcpyHostToDevice, s));
+    if (count <= AcceptedTokens::kMost) { // (as kernel arguments: one launch where four copies were)
+        AcceptedTokens t{};
+        std::copy(toks.begin(), toks.end(), t.token);
+        hipLaunchKernelGGL(accept_commit_kernel, dim3(1), dim3(64), 0, s, m->d_ctx_len, m->d_tokens, m->d_out_token, m->d_sampled + m->context_length, t, count, new_len);
+        HIPCHK(hipGetLastError());
+    } else {
+        HIPCHK(hipMemcpyAsync(m->d_sampled + m->context_length, toks.data(), (size_t)count * 4, hipMemcpyHostToDevice, s));
+        HIPCHK(hipMemcpyAsync(m->d_tokens, &toks[count - 1], 4, hipMemcpyHostToDevice, s));
+        HIPCHK(hipMemcpyAsync(m->d_out_token, &toks[count - 1], 4, hipMemcpyHostToDevice, s));
+        HIPCHK(hipMemcpyAsync(m->d_ctx_len, &new_len, 4, hipMemcpyHostToDevice, s));
+    }
     HIPCHK(hipStreamSynchronize(s));
     m->context_length = new_len;
     m->hidden_ready = false;

@@ -13,6 +13,8 @@
 // MI355X execution strategy: weights, KV cache and DeltaNet state resident in HBM; the context length,
 // the next input token and the sampled-token history live in device memory, so ONE captured hipGraph is
 // replayed for every decode step and steps are chained without a host round trip.
+#include <algorithm>
+
 #include "engine_types.h"
 
 using namespace uzu;
@@ -21,26 +23,39 @@ using namespace uzu::eng;
 namespace uzu {
 namespace eng {
 
-// Copies of many allocations (whole 256-byte blocks) in one launch: y = the allocation, its 64 workgroups share it.  A state is 20 to 70 allocations; a copy each was
+// Copies (src null: zeros) of many blocks of whole 4-byte words in one launch: y = the block, its 64 workgroups share it.  A state is 20 to 70 allocations; a copy each was
 // 3 to 6 us whatever it moved.
 struct CopyTable {
     static constexpr uint32_t kMost = 128; // (3 KB of kernel arguments)
-    struct One {
-        void* dst;
-        const void* src;
-        size_t bytes;
-    } one[kMost];
+    CopyBlock one[kMost];
 };
 __global__ void __launch_bounds__(256) copy_table_kernel(CopyTable t) {
-    uint4* dst = (uint4*)t.one[blockIdx.y].dst;
-    const uint4* src = (const uint4*)t.one[blockIdx.y].src;
-    const size_t n = t.one[blockIdx.y].bytes / 16, step = (size_t)gridDim.x * 256;
+    const CopyBlock o = t.one[blockIdx.y];
+    if (!o.src || (((uintptr_t)o.dst | (uintptr_t)o.src | o.bytes) & 15)) {
+        for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < o.bytes / 4; i += (size_t)gridDim.x * 256) ((uint32_t*)o.dst)[i] = o.src ? ((const uint32_t*)o.src)[i] : 0u;
+        return;
+    }
+    uint4* dst = (uint4*)o.dst;
+    const uint4* src = (const uint4*)o.src;
+    const size_t n = o.bytes / 16, step = (size_t)gridDim.x * 256;
     size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     for (; i + 3 * step < n; i += 4 * step) {
         const uint4 a = src[i], b = src[i + step], c = src[i + 2 * step], d = src[i + 3 * step];
         dst[i] = a, dst[i + step] = b, dst[i + 2 * step] = c, dst[i + 3 * step] = d;
     }
     for (; i < n; i += step) dst[i] = src[i];
+}
+
+// the entries in launches of as many as fit
+uzu_status copy_blocks(hipStream_t s, const std::vector<CopyBlock>& all) {
+    for (size_t lo = 0; lo < all.size(); lo += CopyTable::kMost) {
+        CopyTable t{};
+        const uint32_t n = (uint32_t)std::min<size_t>(all.size() - lo, CopyTable::kMost);
+        std::copy(all.begin() + lo, all.begin() + lo + n, t.one);
+        hipLaunchKernelGGL(copy_table_kernel, dim3(64, n), dim3(256), 0, s, t);
+        HIPCHK(hipGetLastError());
+    }
+    return UZU_OK;
 }
 
 uzu_status dev_alloc(uzu_hip_model* m, size_t bytes, void** out, bool zero) {
@@ -745,11 +760,12 @@ void uzu_hip_model_destroy(uzu_hip_model* m) {
 uzu_status uzu_hip_model_reset(uzu_hip_model* m) {
     UZU_REQUIRE(m, "model_reset: null model");
     hipStream_t s = m->ctx->stream;
-    HIPCHK(hipMemsetAsync(m->d_ctx_len, 0, 4, s));
+    std::vector<CopyBlock> all{{m->d_ctx_len, nullptr, 4}}; // (one launch: a fill per state was 36 of 2 us for 18 DeltaNet layers)
     for (auto& L : m->layers) {
-        if (L.conv_state) HIPCHK(hipMemsetAsync(L.conv_state, 0, L.conv_state_bytes, s));
-        if (L.ssm_state) HIPCHK(hipMemsetAsync(L.ssm_state, 0, L.ssm_state_bytes, s));
+        if (L.conv_state) all.push_back({L.conv_state, nullptr, L.conv_state_bytes});
+        if (L.ssm_state) all.push_back({L.ssm_state, nullptr, L.ssm_state_bytes});
     }
+    UZU_PROPAGATE(copy_blocks(s, all));
     HIPCHK(hipStreamSynchronize(s));
     m->context_length = 0;
     m->hidden_ready = false;
@@ -813,15 +829,10 @@ uzu_status uzu_hip_state_copy(uzu_hip_state* dst, const uzu_hip_state* src) {
     UZU_REQUIRE(dst->allocations.size() == src->allocations.size() && dst->allocation_bytes == src->allocation_bytes, "state_copy: the states differ in layout");
     (void)hipSetDevice(m->ctx->device);
     hipStream_t s = m->ctx->stream;
-    for (size_t lo = 0; lo < dst->allocations.size(); lo += CopyTable::kMost) {
-        CopyTable t{};
-        uint32_t n = 0;
-        for (size_t i = lo; i < dst->allocations.size() && n < CopyTable::kMost; ++i)
-            if (const size_t bytes = dst->allocation_bytes[i]) t.one[n++] = {dst->allocations[i], src->allocations[i], bytes};
-        if (!n) continue;
-        hipLaunchKernelGGL(copy_table_kernel, dim3(64, n), dim3(256), 0, s, t);
-        HIPCHK(hipGetLastError());
-    }
+    std::vector<CopyBlock> all;
+    for (size_t i = 0; i < dst->allocations.size(); ++i)
+        if (dst->allocation_bytes[i]) all.push_back({dst->allocations[i], src->allocations[i], dst->allocation_bytes[i]});
+    UZU_PROPAGATE(copy_blocks(s, all));
     HIPCHK(hipStreamSynchronize(s));
     const uint32_t len = m->bound == src ? m->context_length : src->context_length;
     dst->context_length = len;

@@ -312,6 +312,12 @@ namespace eng {
 #define HIPCHK(expr) UZU_HIP_TRY(expr)
 
 // ---- engine_build.hip: device memory of a model / a sequence state, weight upload, RoPE tables
+struct CopyBlock {
+    void* dst;
+    const void* src; // null: zeros
+    size_t bytes;    // whole 4-byte words
+};
+uzu_status copy_blocks(hipStream_t s, const std::vector<CopyBlock>& all);
 uzu_status dev_alloc(uzu_hip_model* m, size_t bytes, void** out, bool zero = false);
 void dev_free(uzu_hip_model* m, void* p);
 uzu_status state_alloc(uzu_hip_state* st, size_t bytes, void** out, bool zero_by_contract = true);

@@ -434,16 +434,21 @@ bool delta_net_conv_out_of_place_supported(const uint16_t* in_proj, const float*
 uzu_status delta_net_conv_out_of_place(hipStream_t s, const uint16_t* in_proj, const float* conv_weight, const float* bias, const float* state, uint16_t* conv_out,
                                        uint32_t suffix_len, uint32_t conv_dim, uint32_t in_stride) {
     if (!suffix_len || !conv_dim) return UZU_OK;
-    // tokens per thread: 8 (rows 11 / 8 per output from the cache instead of 19 / 16, twice the threads) -- UZU_CONV_OOP_TB (lab builds) = 16 for the A/B
-    static const int tb = [] {
+    // tokens per thread: 8 (rows 11 / 8 per output from the cache instead of 19 / 16, twice the threads); 4 while the grid does not cover the chip -- a thread's chain of exact
+    // exponentials is the time then (517 rows 11.6 -> 8.6 us) -- UZU_CONV_OOP_TB (lab builds) = 16 / 8 for the A/B
+    static const int forced = [] {
         const char* e = lab_env("UZU_CONV_OOP_TB");
-        return e && atoi(e) == 16 ? 16 : 8;
+        return e ? atoi(e) : 0;
     }();
+    const int tb = forced == 16 || forced == 8 ? forced : suffix_len <= 1024 ? 4 : 8;
     const uint32_t nblocks = (suffix_len + tb - 1) / tb;
     const size_t a4 = (size_t)nblocks * (conv_dim / 4);
     const uint32_t g4 = (uint32_t)((a4 + 255) / 256 > 16384 ? 16384 : (a4 + 255) / 256);
     if (tb == 16)
         return launch_check([&] { hipLaunchKernelGGL(conv_apply4_oop_kernel<16>, dim3(g4), dim3(256), 0, s, in_proj, conv_weight, bias, state, conv_out, suffix_len, conv_dim, in_stride,
+                                                     nblocks); }, "conv_apply4_oop");
+    if (tb == 4)
+        return launch_check([&] { hipLaunchKernelGGL(conv_apply4_oop_kernel<4>, dim3(g4), dim3(256), 0, s, in_proj, conv_weight, bias, state, conv_out, suffix_len, conv_dim, in_stride,
                                                      nblocks); }, "conv_apply4_oop");
     return launch_check([&] { hipLaunchKernelGGL(conv_apply4_oop_kernel<8>, dim3(g4), dim3(256), 0, s, in_proj, conv_weight, bias, state, conv_out, suffix_len, conv_dim, in_stride,
                                                  nblocks); }, "conv_apply4_oop");

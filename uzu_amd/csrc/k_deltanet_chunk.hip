@@ -712,7 +712,7 @@ bool delta_net_prefill_chunked_supported(uint32_t num_v_heads, uint32_t num_k_he
     if (exact_mode()) return false; // reference-order mode: the token-by-token recurrence in the reference's own loop order (k_exact.hip)
     static const uint32_t min_t = [] {
         const char* e = lab_env("UZU_DN_CHUNK_MIN_T");
-        return e ? (uint32_t)atoi(e) : 64u;
+        return e ? (uint32_t)atoi(e) : 16u; // a prompt of 12 tokens is as fast token by token, one of 63 12 % slower (0.8B model: 2.16 against 1.90 ms)
     }();
     return head_k_dim == DKC && num_k_heads && num_v_heads % num_k_heads == 0 && head_v_dim % 16 == 0 && suffix_len >= min_t;
 }
