@@ -670,7 +670,7 @@ bool moe_experts_grouped_supported(const MoeGroupedParams& p) {
     if (!p.routed || p.routed > 8192 || !p.y2 || !p.perm) return false;
     LinearF32Params q, r;
     moe_products(p, q, r);
-    if (p.f32_products) return p.rows >= 32 && moe_dma_supported(p, q, r); // (the VALU tile has no grouped form)
+    if (p.f32_products) return p.rows >= 32 && p.hidden && moe_dma_supported(p, q, r); // (the VALU tile has no grouped form)
     return p.rows >= 64 && p.y1 && p.hidden && linear_mfma_supported(q) && linear_mfma_supported(r);
 }
 
@@ -678,15 +678,19 @@ uzu_status moe_experts_grouped(hipStream_t s, const MoeGroupedParams& p) {
     UZU_REQUIRE(moe_experts_grouped_supported(p), "moe_experts_grouped: shape not covered");
     UZU_REQUIRE(!p.pos_weight || !p.act.plain, "moe_experts_grouped: weights on the inputs of plain experts");
     const uint32_t slots = p.rows * p.top;
-    UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(moe_bucket_kernel, dim3(1), dim3(1024), (size_t)p.routed * 4, s, p.ids, slots, p.routed, p.offsets, p.cursor); }, "moe_bucket"));
-    UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(moe_scatter_kernel, dim3((slots + 255) / 256), dim3(256), (size_t)p.routed * 4, s, p.ids, slots, p.routed, p.top, p.offsets, p.cursor, p.perm, p.slot_pos, p.weights, p.pos_weight); },
-                               "moe_scatter"));
     LinearF32Params q, r;
     moe_products(p, q, r);
     // prompt-sized: operand rows once, the gated product in the first product's epilogue, its rows as the operand of the second
     const uint32_t parts = p.f32_products ? 3 : 1;
     const size_t xb_bytes = ((size_t)p.rows * p.d * 2 * parts + 255) / 256 * 256;
     uint16_t* xb = moe_dma_supported(p, q, r) ? (uint16_t*)stream_workspace(s, xb_bytes + (size_t)slots * p.ff * 2 * parts) : nullptr;
+    if (!xb && p.f32_products) { // (no workspace, for instance while the stream is captured: the per-row form)
+        UZU_PROPAGATE(moe_experts_gate_up(s, p.x, p.ids, p.w13, p.hidden, p.rows, p.d, p.ff, p.routed, p.top, 0, p.act, p.pos_weight ? p.weights : nullptr));
+        return moe_experts_down_combine(s, p.hidden, p.x, p.ids, p.pos_weight ? nullptr : p.weights, p.w2, p.residual, p.y, p.rows, p.d, p.ff, p.routed, p.top, 0);
+    }
+    UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(moe_bucket_kernel, dim3(1), dim3(1024), (size_t)p.routed * 4, s, p.ids, slots, p.routed, p.offsets, p.cursor); }, "moe_bucket"));
+    UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(moe_scatter_kernel, dim3((slots + 255) / 256), dim3(256), (size_t)p.routed * 4, s, p.ids, slots, p.routed, p.top, p.offsets, p.cursor, p.perm, p.slot_pos, p.weights, p.pos_weight); },
+                               "moe_scatter"));
     if (xb) {
         GatedRows gr;
         gr.out = (uint16_t*)((char*)xb + xb_bytes), gr.row_weight = p.pos_weight, gr.act = p.act;
@@ -694,7 +698,6 @@ uzu_status moe_experts_grouped(hipStream_t s, const MoeGroupedParams& p) {
         UZU_PROPAGATE(linear_dma_grouped(s, q, xb, &gr));
         UZU_PROPAGATE(linear_dma_grouped(s, r, gr.out));
     } else {
-        UZU_REQUIRE(!p.f32_products, "moe_experts_grouped: no workspace for f32 products");
         UZU_PROPAGATE(linear_mfma(s, q));
         if (!p.act.plain) UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(moe_act_mul_kernel, dim3(slots), dim3(256), 0, s, p.y1, p.hidden, p.offsets, p.routed, p.ff, p.act, p.pos_weight); }, "moe_act_mul"));
         UZU_PROPAGATE(linear_mfma(s, r));

@@ -206,7 +206,7 @@ struct MoeGroupedParams {
     uint32_t *perm, *slot_pos, *offsets, *cursor;
     uint32_t rows, d, ff, routed, top;
     ExpertAct act;
-    uint32_t f32_products = 0; // true f32 products (y1 / hidden unused)
+    uint32_t f32_products = 0; // true f32 products (y1 unused)
 };
 bool moe_experts_grouped_supported(const MoeGroupedParams& p);
 uzu_status moe_experts_grouped(hipStream_t s, const MoeGroupedParams& p);
