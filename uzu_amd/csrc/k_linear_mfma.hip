@@ -1,4 +1,5 @@
-// k_linear_mfma.hip -- the full-precision linear of the f32-stream designs on the bf16 matrix cores (kernels_stream32.h: linear_f32 with bf16 products).
+// k_linear_mfma.hip -- the full-precision linear of the f32-stream designs on the bf16 matrix cores (kernels_stream32.h: linear_f32).  Two forms: operands staged through
+// registers (below), and operand rows converted once and brought by LDS DMA (linear_dma_kernel: larger products, products cut along k, true f32 products as three bf16 parts).
 //
 //   Y[r, n] = act(sum_k bf16(X[r, k]) * W[n, k] + bias[n]) + residual[r, n]       X f32 rows, W bf16 [n, k], f32 accumulation, f32 out
 //

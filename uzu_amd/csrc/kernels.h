@@ -68,7 +68,7 @@ uzu_status matmul(hipStream_t s, const MatmulParams& p, int num_cus, const char*
 // true when matmul() can run `p` with the fused GatedActMul epilogue (act_mul = 1: D = [m, n/2]); otherwise run the matmul and
 // gated_act_mul separately
 bool matmul_act_mul_supported(hipStream_t s, const MatmulParams& p, int num_cus);
-// k_gemm_rows.hip: M >= 17 activation rows against int4 codes (group % 128 == 0), register-fed: dozens to hundreds of rows
+// k_gemm_rows.hip: 17 to hundreds of activation rows (wide matrices: 2 and more) against int4 codes in groups of 128, register-fed
 bool gemm_rows_preferred(const MatmulParams& p);
 uzu_status gemm_rows(hipStream_t s, const MatmulParams& p, int num_cus);
 uzu_status gemm_split_finish(hipStream_t s, const MatmulParams& p, const float* partials, uint32_t splits); // k_gemm128.hip

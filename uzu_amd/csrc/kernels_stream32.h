@@ -2,7 +2,8 @@
 // are f32; activations travel between kernels as f32 rows; weights are bf16 [n, k] in HBM.  `bf16_products` != 0: a matrix product rounds its activation
 // operand to bf16 (weights are bf16 already) and accumulates in f32 -- the serving precision; 0: every product is a true f32 product.
 //   k_stream32.hip           embedding rows, dynamic-tanh norm + token shift, depth mix, the full-precision linear, score-routed experts
-//   k_linear_mfma.hip        the full-precision linear on the matrix cores (bf16 products, prefill-sized row counts)
+//   k_linear_mfma.hip        the full-precision linear on the matrix cores (bf16 products; true f32 products as three bf16 parts), more than 16 rows
+//   k_few_rows.hip           linears and experts of a few rows with bf16 products, operands straight from memory
 //   k_latent_attention.hip   latent normalisation + cache append, the latent-space attention core (prompt rows and decode rows)
 //   k_window_attention.hip   rotation + key / value cache append, attention over cached keys and values (grouped heads, score cap, window, sinks)
 //   k_retention.hip          retention: the decayed outer-product state (token by token and in chunks), per-head RMS division + gate
