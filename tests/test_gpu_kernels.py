@@ -17,7 +17,7 @@ import os
 import numpy as np
 import pytest
 
-from helpers import MASK_VARIANTS, bf16, f32, mask_case, quant_matrix, ref_attention_inputs, trie_from_parents, ulp_diff_bf16
+from helpers import MASK_VARIANTS, bf16, dequantize, f32, mask_case, quant_matrix, ref_attention_inputs, trie_from_parents, ulp_diff_bf16
 from oracle import oracle as O
 from uzu_amd import _ffi
 from uzu_amd import backend as B
@@ -157,6 +157,27 @@ def test_matmul_dozens_of_rows(hip_ctx, n, k, m, method):
     ulps = ulp_diff_bf16(want, got)
     assert ulps.max() <= 1.0, f"max {ulps.max()} bf16 ulps"
     assert (want == got).mean() >= 0.97
+
+
+@pytest.mark.parametrize("method", [0, 1, 2])
+@pytest.mark.parametrize("n,k,m", [(1024, 1024, 37), (1024, 3584, 17), (8192, 512, 16), (4096, 2048, 127), (1024, 1024, 256)])
+def test_matmul_dozens_of_rows_f32_sums(hip_ctx, n, k, m, method):
+    """The sums of csrc/k_gemm_rows.hip before any rounding to bf16, against 64 bits.  Products of bf16 activations and centred codes are exact in f32; what is left is the rounding of
+    the partial sums, which are no larger than the result: a few of them add like random numbers of 2^-25 each, below one f32 ulp (2^-23) of the result's norm.  Partial sums of
+    uncentred codes are five times as large and miss that bound."""
+    rng = np.random.default_rng(n + k + m + method)
+    q = quant_matrix(rng, n, k, 4, 128, method)
+    if method == 1:  # (zero points around the middle, as a fitted matrix has them)
+        q["zero_points"] = ((q["zero_points"] & 0x11) + 0x77).astype(np.uint8)
+    a = bf16(rng.standard_normal((m, k)))
+    kern = B.MatmulKernel.new(hip_ctx, B.BF16, B.BF16, B.F32)
+    ba, bw, bs, bd = (hip_ctx.buffer_from(z) for z in (a, q["weights"], q["scales"], np.zeros((m, n), np.float32)))
+    bb, bz = (None if q[z] is None else hip_ctx.buffer_from(q[z]) for z in ("biases", "zero_points"))
+    kind = {0: B.B_SCALE_BIAS, 1: B.B_SCALE_ZERO_POINT, 2: B.B_SCALE_SYMMETRIC}[method]
+    run(hip_ctx, lambda cb: kern.encode(cb, a=ba, b=bw, d=bd, m=m, n=n, k=k, b_kind=kind, scales=bs, biases=bb, zero_points=bz, mode=B.QMODE_U4, group_size=128))
+    want = f32(a).astype(np.float64) @ dequantize(q).T
+    got = bd.download(np.float32, m * n).reshape(m, n)
+    assert np.linalg.norm(got - want) <= 2.0 ** -23 * np.linalg.norm(want)
 
 
 def test_gemv_epilogue_and_ragged(hip_ctx):

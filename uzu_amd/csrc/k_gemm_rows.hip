@@ -6,8 +6,10 @@
 //   * a wave owns 16 MT tokens x 16 NB weight rows of v_mfma_f32_16x16x32_bf16.  Activations go from the L2 into the A operand (lane (r, g): token r, 16 bytes
 //     at k0 + 32 i + 8 g -- an instruction takes whole 64-byte pieces of 16 rows; at k0 + 32 g + 8 i it would touch every piece four times, which is what bounds
 //     the cache in front of a CU).  A lane loads 16 bytes = 32 codes of weight row r at k0 + 32 g; four lane swaps (v_permlane32_swap, v_permlane16_swap) turn
-//     the (lane group, word) square round, so that word i holds the codes of k0 + 32 i + 8 g, and a word converts to the 8 bf16 (16 + q) of MFMA i
-//     (gemm_convert.h: two codes per v_and_or_b32, pair order (0 4) (1 5) (2 6) (3 7), which the activations are permuted to);
+//     the (lane group, word) square round, so that word i holds the codes of k0 + 32 i + 8 g, and a word converts to the 8 bf16 (q - 8) / 16 of MFMA i
+//     (gemm_convert.h: dequant4).  The codes are centred for the sums' sake: with (16 + q), two codes per v_and_or_b32, partial sums are five times the result and the
+//     error against 64 bits is 1.8e-7 of it, here 5e-8 at K = 1024 and 8e-8 at K = 4096 (64 x 64 tiles: 7e-8, 1.4e-7).  The time is the same within 1 %: what the
+//     conversion costs more, the activations' permutation to that pair order did;
 //   * a step contracts over 128 k = one quant group: the group's products and the tokens' sums (the same A against an all-ones B) are folded with the f32 scale
 //     and offset of the lane's own weight row, so no weight is ever rounded and no scalar crosses lanes.  Scales are read two groups at a time;
 //   * the next step's loads are in flight while a step is computed, waves never meet before the end, and K is cut KW ways over the waves of a workgroup
@@ -18,6 +20,7 @@
 // 14.3 + 4.7 -> 8.1; 8224 x 1024: 14.5 -> 10.1; 4096 x 14336: 163 -> 29; a 37-token prompt of Qwen3.5-0.8B 3.97 -> 2.02 ms.
 #include "decode_epilogue.h"
 #include "device_utils.h"
+#include "gemm_convert.h"
 #include "kernels.h"
 
 namespace uzu {
@@ -101,9 +104,7 @@ __global__ void __launch_bounds__(256, 2) gemm_rows_kernel(GemmRowsParams p) {
             else if constexpr (KIND == UZU_MATMUL_B_SCALE_ZERO_POINT) of2[b] = p.zp[at / 2];
         }
     };
-    uint32_t mask = 0x00780078u, magic = 0x41804180u, ones = 0x3F803F80u;
-    asm("" : "+s"(mask));
-    asm("" : "+v"(magic));
+    uint32_t ones = 0x3F803F80u;
     asm("" : "+v"(ones));
     const gm_u32x4 ones4 = {ones, ones, ones, ones};
     gm_f32x4 acc[NB][MT]; // tokens 4 g + v of tile t, row r of block b
@@ -123,35 +124,28 @@ __global__ void __launch_bounds__(256, 2) gemm_rows_kernel(GemmRowsParams p) {
         for (int b = 0; b < NB; ++b) turn_words(st.codes[b]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            gm_u32x4 xa[MT];
+            if constexpr (KIND != UZU_MATMUL_B_SCALE_SYMMETRIC) {
 #pragma unroll
-            for (int t = 0; t < MT; ++t) { // (x0,x1) (x2,x3) (x4,x5) (x6,x7) -> (x0,x4) (x1,x5) (x2,x6) (x3,x7)
-                const gm_u32x4 u = st.xv[t][i];
-                xa[t].x = __builtin_amdgcn_perm(u.z, u.x, 0x05040100u), xa[t].y = __builtin_amdgcn_perm(u.z, u.x, 0x07060302u);
-                xa[t].z = __builtin_amdgcn_perm(u.w, u.y, 0x05040100u), xa[t].w = __builtin_amdgcn_perm(u.w, u.y, 0x07060302u);
-                dx[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, xa[t]), __builtin_bit_cast(gm_bf16x8, ones4), dx[t], 0, 0, 0);
+                for (int t = 0; t < MT; ++t) dx[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, st.xv[t][i]), __builtin_bit_cast(gm_bf16x8, ones4), dx[t], 0, 0, 0);
             }
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                const uint32_t w = st.codes[b][i];
-                gm_u32x4 wv;
-                wv.x = ((w << 3) & mask) | magic, wv.y = ((w >> 1) & mask) | magic, wv.z = ((w >> 5) & mask) | magic, wv.w = ((w >> 9) & mask) | magic;
+                const u32x4_t wv = dequant4(st.codes[b][i] ^ 0x88888888u); // (nibbles as two's complement of q - 8)
 #pragma unroll
                 for (int t = 0; t < MT; ++t)
-                    dq[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, xa[t]), __builtin_bit_cast(gm_bf16x8, wv), dq[b][t], 0, 0, 0);
+                    dq[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, st.xv[t][i]), __builtin_bit_cast(gm_bf16x8, wv), dq[b][t], 0, 0, 0);
             }
         }
-        // group fold: acc += scale dq + (offset - 16 scale) sum_x
+        // group fold: acc += 16 scale dq + (offset + 8 scale) sum_x   (dq = sum (q - 8) / 16 x; a symmetric matrix has nothing left to add)
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
             for (int t = 0; t < MT; ++t)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) acc[b][t][v] = fmaf(sc[b], dq[b][t][v], fmaf(of[b], dx[t][v], acc[b][t][v]));
+                for (int v = 0; v < 4; ++v) acc[b][t][v] = fmaf(sc[b], dq[b][t][v], KIND == UZU_MATMUL_B_SCALE_SYMMETRIC ? acc[b][t][v] : fmaf(of[b], dx[t][v], acc[b][t][v]));
     };
     auto offset_of = [&](float sc, float raw) { // raw: the bf16 offset, or the zero point
-        const float of = KIND == UZU_MATMUL_B_SCALE_BIAS ? raw : KIND == UZU_MATMUL_B_SCALE_ZERO_POINT ? -sc * raw : -sc * 8.0f;
-        return fmaf(-kQ4Offset, sc, of);
+        return KIND == UZU_MATMUL_B_SCALE_BIAS ? fmaf(8.0f, sc, raw) : KIND == UZU_MATMUL_B_SCALE_ZERO_POINT ? sc * (8.0f - raw) : 0.0f;
     };
     Step stA, stB;
     load_step(s_lo, stA);
@@ -165,6 +159,7 @@ __global__ void __launch_bounds__(256, 2) gemm_rows_kernel(GemmRowsParams p) {
             sc0[b] = bits_to_f32(sc2[b] << 16), sc1[b] = bits_to_f32(sc2[b] & 0xFFFF0000u);
             of0[b] = offset_of(sc0[b], zp ? (float)(of2[b] & 15u) : bits_to_f32(of2[b] << 16));
             of1[b] = offset_of(sc1[b], zp ? (float)((of2[b] >> 4) & 15u) : bits_to_f32(of2[b] & 0xFFFF0000u));
+            sc0[b] *= 16.0f, sc1[b] *= 16.0f;
         }
         load_scales(s + 2);
         __builtin_amdgcn_sched_barrier(0); // (left alone, the scheduler sinks the loads to their uses and waits for each)
