@@ -272,6 +272,22 @@ def test_linear_of_a_few_rows(hip_ctx, rows, n, k, batch, act):
     assert np.abs(got - want).max() <= 3e-5 * max(1.0, np.abs(want).max())
 
 
+@pytest.mark.parametrize("rows,n,k", [(3, 4112, 1024), (8, 2048, 4096), (16, 520, 2048), (24, 1024, 2048), (12, 300, 1024)])
+def test_linear_of_a_few_rows_sums(hip_ctx, rows, n, k):
+    """How far the f32 sums are from 64 bits, held to the sums a wave per column makes (64 lanes that add every 64th product one by one, then in pairs; products of bf16 numbers are
+    exact): no further, with 5 % for the chance of the inputs."""
+    rng = np.random.default_rng(rows + n + k)
+    x, w = O.to_bf16(rng.standard_normal((rows, k))).astype(np.float32), O.to_bf16(rng.standard_normal((n, k))).astype(np.float32)
+    want = x.astype(np.float64) @ w.T.astype(np.float64)
+    lanes = np.zeros((rows, n, 64), dtype=np.float32)
+    for at in range(0, k, 64):
+        lanes += x[:, None, at:at + 64] * w[None, :, at:at + 64]
+    while lanes.shape[-1] > 1:
+        lanes = lanes[..., ::2] + lanes[..., 1::2]
+    got = linear(hip_ctx, x, w, act=0, bf16=1)
+    assert np.linalg.norm(got - want) <= 1.05 * np.linalg.norm(lanes[..., 0] - want)
+
+
 @pytest.mark.parametrize("rows,routed,identity,top,ff,d", [(2, 8, 0, 2, 64, 64), (3, 70, 2, 4, 128, 192), (16, 4, 1, 3, 320, 64), (33, 2, 1, 1, 64, 1024), (63, 3, 0, 3, 192, 128), (61, 16, 3, 16, 64, 64)])
 def test_experts_of_a_few_rows(hip_ctx, rows, routed, identity, top, ff, d):
     """bf16 products of 2 to 63 rows: fewer (row, slot) pairs than experts and more, an expert with more pairs than a tile holds, every pair on one expert, identity experts; against 64 bits

@@ -3,7 +3,7 @@
 // At these sizes a product is its weights' way from memory: 7712 x 2048 is 32 MB, 6 us of reading, and 8 rows of it 0.25 GFLOP.  A wave per output column on the VALU
 // (k_stream32.hip, linear_rows) reads a weight once per four rows and pays a conversion and four multiply-adds for it: 26 us.  Here
 //   * a workgroup owns 16 NB output columns, its waves share the contraction in chunks of 64 (wave w takes chunks w, w + W, ..: together they read whole rows), and the
-//     waves' f32 sums meet once, in LDS, in wave order;
+//     waves' f32 sums meet once, in LDS, in pairs;
 //   * a chunk is two v_mfma_f32_16x16x32_bf16 per 16 columns and 16 rows: lane (r, g) loads 32 bytes of weight row r at 16 g and the same 16 elements of activation row r
 //     (f32, rounded to bf16 in registers, from the L2) -- the contraction's order inside a chunk is free as long as both operands share it, and a weight row's 128 bytes
 //     are taken whole;
@@ -41,16 +41,22 @@ __device__ __forceinline__ void few_load(FewBatch<NB, MT, U>& b, const uint16_t*
     }
 }
 __device__ __forceinline__ u32x4_t few_pack(const fw_f32x4& a, const fw_f32x4& b) { return u32x4_t{pack_bf16(a[0], a[1]), pack_bf16(a[2], a[3]), pack_bf16(b[0], b[1]), pack_bf16(b[2], b[3])}; }
-// acc[j][i]: lane (m, g), element t = column 16 j + 4 g + t of row 16 i + m
+// acc[j][i]: lane (m, g), element t = column 16 j + 4 g + t of row 16 i + m.  The matrix core's sums fall short of the exact ones by a rounding that is always downwards: a chain of
+// them through the contraction adds up (8 rows of 2048 x 4096: 1.4e-7 of the result's norm against 64 bits; a wave per column 8.4e-8).  So a chunk's two products are summed from
+// zero, one of them negated, and their difference added: what is missing of both goes out.
 template <int NB, int MT> __device__ __forceinline__ void few_chunk(fw_f32x4 (&acc)[NB][MT], const u32x4_t (&w)[NB][2], const fw_f32x4 (&x)[MT][4]) {
+    const fw_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < MT; ++i) {
+        const bf16x8_t b0 = __builtin_bit_cast(bf16x8_t, few_pack(x[i][0], x[i][1])), b1 = __builtin_bit_cast(bf16x8_t, few_pack(-x[i][2], -x[i][3]));
+        fw_f32x4 s0[NB], s1[NB];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const bf16x8_t b = __builtin_bit_cast(bf16x8_t, few_pack(x[i][2 * h], x[i][2 * h + 1]));
+        for (int j = 0; j < NB; ++j) s0[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[j][0]), b0, zero, 0, 0, 0);
 #pragma unroll
-            for (int j = 0; j < NB; ++j) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[j][h]), b, acc[j][i], 0, 0, 0);
-        }
+        for (int j = 0; j < NB; ++j) s1[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[j][1]), b1, zero, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[j][i] += s0[j] - s1[j];
+    }
 }
 template <int NB, int MT, int U>
 __device__ __forceinline__ void few_contract(fw_f32x4 (&acc)[NB][MT], const uint16_t* const (&wp)[NB], const float* const (&xp)[MT], uint32_t chunks, uint32_t wave, uint32_t waves) {
@@ -82,10 +88,10 @@ template <int T> __device__ __forceinline__ void few_put(float* s_sum, const fw_
 #pragma unroll
     for (int t = 0; t < T; ++t) *(fw_f32x4*)(s_sum + ((size_t)(wave * T + t) * 64 + lane) * 4) = acc[t];
 }
-__device__ __forceinline__ float few_sum(const float* s_sum, uint32_t tiles, uint32_t e, uint32_t waves) {
-    float v = s_sum[e];
-    for (uint32_t w = 1; w < waves; ++w) v += s_sum[w * tiles * 256 + e];
-    return v;
+__device__ __forceinline__ float few_sum(const float* s_sum, uint32_t tiles, uint32_t e, uint32_t waves) { // (four waves or eight, in pairs)
+    auto at = [&](uint32_t w) { return s_sum[w * tiles * 256 + e]; };
+    const float v = (at(0) + at(1)) + (at(2) + at(3));
+    return waves == 4 ? v : v + ((at(4) + at(5)) + (at(6) + at(7)));
 }
 
 template <int NB, int MT, int U> __global__ void __launch_bounds__(512) linear_few_kernel(LinearF32Params p) {
