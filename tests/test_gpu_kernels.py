@@ -995,13 +995,14 @@ def test_delta_net_update(hip_ctx):
     assert ulp_diff_bf16(want, got).max() <= 2.0
 
 
-@pytest.mark.parametrize("T", [37, 64, 200, 513, 1000, 2043])
-def test_delta_net_prefill_path(hip_ctx, T):
+@pytest.mark.parametrize("T,Dv", [(2, 128), (5, 128), (15, 128), (37, 24), (16, 128), (31, 128), (32, 128), (33, 128), (37, 128), (64, 128), (200, 128), (513, 128), (1000, 128), (2043, 128)])
+def test_delta_net_prefill_path(hip_ctx, T, Dv):
     """conv_pack -> conv_scan -> prefill_prep -> prefill -> norm_gate against the oracle (GQA-style Hv = 2 Hk).
-    T = 37 runs the one/two-token recurrence, T >= 64 the chunked form (32-token chunks, ragged last chunk), from 16 chunks (T = 513, 1000, 2043) as
+    Below 16 tokens, and where the value width is no multiple of 16, the one/two-token recurrence runs (over one of its 32-token tiles and over two); from 16 on the chunked form
+    (32-token chunks; a lone ragged chunk, whole ones, a last chunk of one token), from 16 chunks (T = 513, 1000, 2043) as
     two concurrent segments + the S_mid fix-up (k_deltanet_chunk.hip: ScanSplit; T = 513: 9 + 8 chunks, the second segment ends on a 1-token chunk)."""
     rng = np.random.default_rng(15)
-    Hv, Hk, Dk, Dv, ks = 4, 2, 128, 128, 4
+    Hv, Hk, Dk, ks = 4, 2, 128, 4
     key_dim, value_dim = Hk * Dk, Hv * Dv
     conv_dim = 2 * key_dim + value_dim
     total = conv_dim + value_dim + 2 * Hv
@@ -1051,6 +1052,46 @@ def test_delta_net_prefill_path(hip_ctx, T):
     # output every element is within 2e-2 absolute or 1 bf16 ulp (|x| >= 4 has an ulp of 0.031), 99 % within 2 ulps
     err, ulps = np.abs(f32(got) - f32(w_out)), ulp_diff_bf16(w_out, got)
     assert ((err <= 2e-2) | (ulps <= 1)).all() and (ulps <= 2).mean() > 0.99
+
+
+def delta_net_inputs(rng, T, Hv, Hk, Dv, pace):
+    """what DeltaNetPrefill reads: unit keys, queries scaled by 1 / sqrt(128), strengths in (0, 1), decays exp(-pace e^n), values among the in-projection rows, a state"""
+    kd, vd = Hk * 128, Hv * Dv
+    unit = lambda: (lambda z: (z / np.linalg.norm(z, axis=-1, keepdims=True)).astype(np.float32))(rng.normal(size=(T, Hk, 128)))
+    return dict(q=(unit() / np.float32(np.sqrt(128.0))).reshape(T, kd), k=unit().reshape(T, kd), beta=(1 / (1 + np.exp(-rng.normal(size=(T, Hv))))).astype(np.float32),
+                decay=np.exp(-pace * np.exp(rng.normal(size=(T, Hv)))).astype(np.float32), rows=bf16(rng.normal(0, 1, size=(T, 2 * kd + 2 * vd + 2 * Hv))),
+                state=rng.normal(0, 0.3, size=(Hv, Dv, 128)).astype(np.float32))
+
+
+def hip_delta_net_prefill(ctx, z, Hv, Hk, Dv):
+    T, kd, vd = len(z["q"]), Hk * 128, Hv * Dv
+    bq, bk, bb, bd, bi, bs = (ctx.buffer_from(np.ascontiguousarray(z[n])) for n in ("q", "k", "beta", "decay", "rows", "state"))
+    bo = ctx.create_buffer(T * vd * 2)
+    kern = B.DeltaNetPrefillKernel.new(ctx, B.BF16, 128)
+    run(ctx, lambda cb: kern.encode(bq, bk, bb, bd, bi, bs, bo, Hv, Hk, Dv, kd, vd, T, (Dv + 15) // 16, cb))
+    return bo.download(np.uint16, T * vd).reshape(T, vd), bs.download(np.float32, z["state"].size).reshape(z["state"].shape)
+
+
+@pytest.mark.parametrize("pace", [1.0, 0.1, 0.01])
+@pytest.mark.parametrize("T", [16, 24, 37, 63, 200])
+def test_delta_net_prefill_state_precision(hip_ctx, T, pace):
+    """How far the carried f32 state is from 64 bits, under fast and slow decays, held to the recurrence itself in f32 (its dot products summed in pairs, as a half wave does):
+    no further, with a tenth for the chance of the inputs."""
+    Hv, Hk, Dv = 4, 2, 128
+    z = delta_net_inputs(np.random.default_rng(T), T, Hv, Hk, Dv, pace)
+    _, got = hip_delta_net_prefill(hip_ctx, z, Hv, Hk, Dv)
+    v = f32(z["rows"])[:, 2 * Hk * 128:2 * Hk * 128 + Hv * Dv].reshape(T, Hv, Dv)
+    states = []
+    for dt in (np.float64, np.float32):
+        S = z["state"].astype(dt)
+        for t in range(T):
+            k = np.repeat(z["k"][t].reshape(Hk, 128), Hv // Hk, 0).astype(dt)
+            a, b = z["decay"][t].astype(dt)[:, None], z["beta"][t].astype(dt)[:, None]
+            d = b * (v[t].astype(dt) - a * (S * k[:, None, :]).sum(axis=-1, dtype=dt))
+            S = a[:, :, None] * S + d[:, :, None] * k[:, None, :]
+        states.append(S)
+    exact, serial = states
+    assert np.linalg.norm(got - exact) <= 1.1 * np.linalg.norm(serial - exact)
 
 
 # ------------------------------------------------------------------------------------------ command buffer

@@ -12,8 +12,7 @@
 // 32 x 32 Gram matrices + one 32 x 32 forward substitution each).  `dn_chunk_scan_mfma_kernel` then walks the chunks with
 // four small dense products per chunk instead of 32 dependent steps; a workgroup owns 16 of a head's Dv columns, so
 // 128 workgroups are busy and every product has hundreds of independent FMAs per thread.
-// Same algebra, different rounding order: results agree with the one-token recurrence to ~1e-6 relative in f32
-// (tools/ prototype in the commit message), far below the bf16 output rounding.  Decays are carried in log space
+// Same algebra, different rounding order: the state is no further from 64 bits than the recurrence's (dn_chunk_scan_mfma_kernel).  Decays are carried in log space
 // (log a clamped at -80) so that products over a chunk cannot underflow into 0 / 0.
 #include <stdlib.h>
 
@@ -71,6 +70,22 @@ size_t delta_net_chunk_workspace_bytes(uint32_t num_v_heads, uint32_t value_dim,
     return ((size_t)((suffix_len + CC - 1) / CC) * num_v_heads * WS_FLOATS + split_floats(num_v_heads, value_dim, suffix_len)) * sizeof(float);
 }
 
+template <int CTRL> __device__ __forceinline__ double dpp_f64(double v) {
+    const uint64_t u = f64_to_bits(v);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xF, 0xF, true), hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xF, 0xF, true);
+    return bits_to_f64((uint64_t)hi << 32 | lo);
+}
+// log a_t, in 64 bits until an exponential of a difference is rounded: f32 prefix sums of fast decays (a = 1/e: -32 at a chunk's end) cost the state 1e-6 of its norm, the
+// recurrence has 6e-8.  Decay 0: clamped, the state is wiped either way.
+// The sum over the tokens up to this one, a token a lane.
+__device__ __forceinline__ double log_prefix(float d, int token) {
+    double l = fmax(log_wide(d), -80.0);
+    // (lane i - 1, - 2, - 4, - 8 of a row of sixteen, or 0; then row 0's total to row 1)
+    l += dpp_f64<0x111>(l), l += dpp_f64<0x112>(l), l += dpp_f64<0x114>(l), l += dpp_f64<0x118>(l);
+    const double before = dpp_f64<0x142>(l);
+    return token >= 16 ? l + before : l;
+}
+
 // grid (chunks, Hv), 256 threads.
 // FUSED (round 6): DeltaNetPrefillPrep (prefill_prep.rs:30-113; k_deltanet.hip::delta_net_prefill_prep_kernel) runs inside this kernel -- the chunk's q / k rows come
 // straight from the conv'd in-projection rows (bf16), are L2-normalised with that kernel's element mapping and reduction order (a wave per token, two elements per
@@ -90,7 +105,8 @@ __global__ void __launch_bounds__(256) dn_chunk_prep_kernel(const float* q_norm,
     float* const sQK = sQ + CC * TP;
     float* const sM = sQ + 2 * CC * TP;
     static_assert(3 * CC * TP <= CC * KP, "the Gram / M matrices fit in the Q rows");
-    __shared__ float s_lg[CC], s_b[CC];
+    __shared__ double s_lg[CC];
+    __shared__ float s_b[CC];
     __shared__ uint64_t s_exp_tab[32];
     const int tid = threadIdx.x;
     const uint32_t groups_per_head = num_v_heads / num_k_heads;
@@ -165,7 +181,7 @@ __global__ void __launch_bounds__(256) dn_chunk_prep_kernel(const float* q_norm,
                 const float log_decay = -expf_glibc_tab(a_log[hv], s_exp_tab) * sp;
                 d = expf_glibc_tab(log_decay, s_exp_tab);
             }
-            s_lg[tid] = fmaxf(logf_glibc(d), -80.0f);
+            s_lg[tid] = log_prefix(d, tid);
             s_b[tid] = b;
         }
     } else {
@@ -183,18 +199,11 @@ __global__ void __launch_bounds__(256) dn_chunk_prep_kernel(const float* q_norm,
     if (tid < CC) {
         const bool live = t0 + tid < suffix_len;
         const float d = live ? decay_buf[(size_t)(t0 + tid) * num_v_heads + hv] : 1.0f;
-        s_lg[tid] = fmaxf(logf_glibc(d), -80.0f); // log a_t (decay 0 => clamped: the state is wiped either way)
+        s_lg[tid] = log_prefix(d, tid);
         s_b[tid] = live ? beta_buf[(size_t)(t0 + tid) * num_v_heads + hv] : 0.0f;
     }
     }
     __syncthreads();
-    if (tid == 0) { // inclusive prefix sum of 32 logs
-        float run = 0.f;
-        for (int t = 0; t < CC; ++t) {
-            run += s_lg[t];
-            s_lg[t] = run;
-        }
-    }
     // Gram matrices: thread -> row i, four columns j0..j0+3
     {
         const int i = tid >> 3, j0 = (tid & 7) * 4;
@@ -218,13 +227,13 @@ __global__ void __launch_bounds__(256) dn_chunk_prep_kernel(const float* q_norm,
     float* w_p = w_t + CC * CC;
     for (int idx = tid; idx < CC * CC; idx += 256) {
         const int i = idx / CC, j = idx % CC;
-        const float ratio = expf_glibc(fminf(s_lg[i] - s_lg[j], 0.0f)); // A_i / A_j for j <= i
+        const float ratio = exp_wide(fmin(s_lg[i] - s_lg[j], 0.0), FUSED ? s_exp_tab : kExp2fTab); // A_i / A_j for j <= i
         sM[i * TP + j] = j < i ? s_b[i] * ratio * sKK[i * TP + j] : 0.0f;
         w_p[idx] = j <= i ? ratio * sQK[i * TP + j] : 0.0f;
     }
     if (tid < CC) {
-        w_t[2 * CC * CC + tid] = expf_glibc(s_lg[tid]);                      // A_t
-        w_t[2 * CC * CC + CC + tid] = expf_glibc(s_lg[CC - 1] - s_lg[tid]);  // A_C / A_t
+        w_t[2 * CC * CC + tid] = exp_wide(s_lg[tid], FUSED ? s_exp_tab : kExp2fTab);                      // A_t
+        w_t[2 * CC * CC + CC + tid] = exp_wide(s_lg[CC - 1] - s_lg[tid], FUSED ? s_exp_tab : kExp2fTab);  // A_C / A_t
     }
     __syncthreads();
     // T = (I + M)^-1 diag(b): column c by forward substitution, one thread per column (M_ij is a broadcast LDS read)
@@ -251,7 +260,10 @@ __global__ void __launch_bounds__(256) dn_chunk_prep_kernel(const float* q_norm,
 //   stage 4  S = A_C S + (D W)^T K   every wave owns two 16-wide dk tiles of the state in its accumulators, 2 x 8 MFMAs
 // MFMA operand layout (16x16x4): A lane l = row l % 16, k-quarter l / 16; B lane l = column l % 16, k-quarter l / 16; C / D four
 // registers = rows 4 (l / 16) + r of column l % 16.  The contraction index of step s in quarter q is (K / 4) q + s for both
-// operands, so a lane's operand values are consecutive in memory.
+// operands, so a lane's operand values are consecutive in memory; in stages 2 and 4, which contract over tokens, it is 4 s + q: the products are added in time
+// order and the late tokens, which weigh most under a decay, come last (T's columns are stored so that a lane's values are consecutive there too).  With that, four
+// chains in stage 1 and the old state added behind the chunk's own products, the state of 16 to 63 tokens is 4e-8 to 1.2e-7 of its norm from 64 bits; the
+// recurrence token by token: 5e-8 to 1.9e-7.
 __global__ void __launch_bounds__(256) dn_chunk_scan_mfma_kernel(const float* q_norm, const float* k_norm, const uint16_t* in_proj, const float* ws, float* state,
                                                                  uint16_t* out, uint32_t num_v_heads, uint32_t num_k_heads, uint32_t head_v_dim, uint32_t key_dim,
                                                                  uint32_t value_dim, uint32_t suffix_len, uint32_t v_row_stride) {
@@ -318,9 +330,10 @@ __global__ void __launch_bounds__(256) dn_chunk_scan_mfma_kernel(const float* q_
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int idx = tid + 256 * r, t = idx / (DKC / 4), c4 = idx % (DKC / 4);
-            *(f32x4_v*)(sK + t * KP + c4 * 4) = st_k[r];
-            *(f32x4_v*)(sQ + t * KP + c4 * 4) = st_q[r];
-            sT[(idx / CC) * TPP + idx % CC] = st_t[r];
+            const int at = ((t & 16) + 4 * (t & 3) + (t >> 2 & 3)) * KP + c4 * 4; // (four tokens in a row lie sixteen banks apart)
+            *(f32x4_v*)(sK + at) = st_k[r];
+            *(f32x4_v*)(sQ + at) = st_q[r];
+            sT[(idx / CC) * TPP + 8 * (idx % 4) + idx % CC / 4] = st_t[r];
             sP[(idx / CC) * TPP + idx % CC] = st_p[r];
         }
         if (tid < CC) sA[tid] = st_a, sW[tid] = st_w;
@@ -342,15 +355,16 @@ __global__ void __launch_bounds__(256) dn_chunk_scan_mfma_kernel(const float* q_
         // ---- stage 1: rows 16 (wave & 1) .. + 16 of K (waves 0, 1) or Q (waves 2, 3) against S^T, contraction over dk = 32 kq + s
         f32x4_v acc1 = {0.f, 0.f, 0.f, 0.f};
         {
-            const float* xr = (wave < 2 ? sK : sQ) + (16 * (wave & 1) + i16) * KP + 32 * kq;
+            const float* xr = (wave < 2 ? sK : sQ) + (16 * (wave & 1) + 4 * (i16 & 3) + (i16 >> 2)) * KP + 32 * kq;
             const float* sr = sS + i16 * KP + 32 * kq;
-            f32x4_v xa[8], sb[8];
+            f32x4_v xa[8], sb[8], part[4] = {acc1, acc1, acc1, acc1}; // (four chains: shorter, and nearer to the exact sum than one)
 #pragma unroll
             for (int q = 0; q < 8; ++q) xa[q] = *(const f32x4_v*)(xr + 4 * q), sb[q] = *(const f32x4_v*)(sr + 4 * q);
 #pragma unroll
             for (int q = 0; q < 8; ++q)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc1 = mfma4(xa[q][e], sb[q][e], acc1);
+                for (int e = 0; e < 4; ++e) part[e] = mfma4(xa[q][e], sb[q][e], part[e]);
+            acc1 = (part[0] + part[1]) + (part[2] + part[3]);
         }
         if (wave < 2) { // R = V - A (K S^T) for tokens v_row + r, value column i16
 #pragma unroll
@@ -363,7 +377,7 @@ __global__ void __launch_bounds__(256) dn_chunk_scan_mfma_kernel(const float* q_
             const f32x4_v ta0 = *(const f32x4_v*)tr, ta1 = *(const f32x4_v*)(tr + 4);
             f32x4_v d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int s2 = 0; s2 < 8; ++s2) d = mfma4(s2 < 4 ? ta0[s2 & 3] : ta1[s2 & 3], sR[(8 * kq + s2) * RPP + i16], d);
+            for (int s2 = 0; s2 < 8; ++s2) d = mfma4(s2 < 4 ? ta0[s2 & 3] : ta1[s2 & 3], sR[(4 * s2 + kq) * RPP + i16], d);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int t = 16 * wave + 4 * kq + r;
@@ -388,19 +402,20 @@ __global__ void __launch_bounds__(256) dn_chunk_scan_mfma_kernel(const float* q_
                 if (t < suffix_len) out[(size_t)t * value_dim + hv * head_v_dim + dv_base + i16] = f32_to_bf16(o[r]);
             }
         }
-        // ---- stage 4 (all waves): S = A_C S + (D W)^T K for dk tiles 2 wave, 2 wave + 1; contraction over tokens 8 kq + s
+        // ---- stage 4 (all waves): S = A_C S + (D W)^T K for dk tiles 2 wave, 2 wave + 1; contraction over tokens 4 s + kq
         {
             const float a_c = sA[CC - 1];
             float dw[8];
 #pragma unroll
-            for (int s2 = 0; s2 < 8; ++s2) dw[s2] = sDw[(8 * kq + s2) * RPP + i16]; // A operand: row = value column i16
+            for (int s2 = 0; s2 < 8; ++s2) dw[s2] = sDw[(4 * s2 + kq) * RPP + i16]; // A operand: row = value column i16
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
+const float* kc = sK + 4 * kq * KP + 32 * wave + 16 * t + i16;
+                f32x4_v u = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int r = 0; r < 4; ++r) creg[t][r] *= a_c;
-                const float* kc = sK + (8 * kq) * KP + 32 * wave + 16 * t + i16;
+                for (int s2 = 0; s2 < 8; ++s2) u = mfma4(dw[s2], kc[(16 * (s2 >> 2) + (s2 & 3)) * KP], u);
 #pragma unroll
-                for (int s2 = 0; s2 < 8; ++s2) creg[t] = mfma4(dw[s2], kc[s2 * KP], creg[t]);
+                for (int r = 0; r < 4; ++r) creg[t][r] = fmaf(creg[t][r], a_c, u[r]);
             }
         }
         lds_barrier(); // all reads of this chunk's LDS operands are done

@@ -80,21 +80,12 @@ static const uint64_t kExp2fTab[32] = {
 
 // `tab`: the 32-entry table -- kExp2fTab, or a copy of it in LDS (decode epilogues: a table read from global memory is
 // a dependent memory round trip on the critical path of a 4 us kernel)
-UZU_HD float expf_glibc_tab(float x, const uint64_t* tab) {
-    const uint32_t ix = f32_to_bits(x);
-    const uint32_t abstop = (ix >> 20) & 0x7ff;
-    if (abstop >= 0x42b) { // |x| >= 88 or NaN/Inf
-        if (ix == 0xff800000u) return 0.0f;                 // exp(-inf)
-        if (abstop >= 0x7f8) return x + x;                  // NaN, +inf
-        if (x > 88.72283172607421875f) return bits_to_f32(0x7f800000u);   // overflow (0x1.62e42ep6)
-        if (x < -103.97207641601562500f) return 0.0f;       // underflow (-0x1.9fe368p6)
-    }
+UZU_HD float exp_core(double xd, const uint64_t* tab) { // e^xd rounded to f32, |xd| within its range
     const double InvLn2N = 0x1.71547652b82fep+0 * 32.0;
     const double Shift = 0x1.8p+52;
     const double C0 = 0x1.c6af84b912394p-5 / 32.0 / 32.0 / 32.0;
     const double C1 = 0x1.ebfce50fac4f3p-3 / 32.0 / 32.0;
     const double C2 = 0x1.62e42ff0c52d6p-1 / 32.0;
-    const double xd = (double)x;
     double z = InvLn2N * xd;
     double kd = z + Shift;
     const uint64_t ki = f64_to_bits(kd);
@@ -109,6 +100,22 @@ UZU_HD float expf_glibc_tab(float x, const uint64_t* tab) {
     y = __builtin_fma(z, r2, y);
     y = y * s;
     return (float)y;
+}
+UZU_HD float expf_glibc_tab(float x, const uint64_t* tab) {
+    const uint32_t ix = f32_to_bits(x);
+    const uint32_t abstop = (ix >> 20) & 0x7ff;
+    if (abstop >= 0x42b) { // |x| >= 88 or NaN/Inf
+        if (ix == 0xff800000u) return 0.0f;                 // exp(-inf)
+        if (abstop >= 0x7f8) return x + x;                  // NaN, +inf
+        if (x > 88.72283172607421875f) return bits_to_f32(0x7f800000u);   // overflow (0x1.62e42ep6)
+        if (x < -103.97207641601562500f) return 0.0f;       // underflow (-0x1.9fe368p6)
+    }
+    return exp_core((double)x, tab);
+}
+// e^x of an exponent held in 64 bits
+UZU_HD float exp_wide(double x, const uint64_t* tab) {
+    if (!(x >= -103.97207641601562500)) return x != x ? (float)x : 0.0f;
+    return x > 88.72283172607421875 ? bits_to_f32(0x7f800000u) : exp_core(x, tab);
 }
 
 UZU_HD float expf_glibc(float x) { return expf_glibc_tab(x, kExp2fTab); }
@@ -130,7 +137,7 @@ static const double kLogfTab[16][2] = {
     {0x1.886e6037841edp-1, 0x1.1058bc8a07ee1p-2},  {0x1.767dcf5534862p-1, 0x1.4043057b6ee09p-2},
 };
 
-UZU_HD float logf_glibc(float x) {
+UZU_HD double log_wide(float x) { // log x before its rounding to f32
     uint32_t ix = f32_to_bits(x);
     if (ix == 0x3f800000u) return 0.0f;
     if (ix - 0x00800000u >= 0x7f800000u - 0x00800000u) {
@@ -155,8 +162,9 @@ UZU_HD float logf_glibc(float x) {
     double y = __builtin_fma(A1, r, A2);
     y = __builtin_fma(A0, r2, y);
     y = __builtin_fma(y, r2, y0 + r);
-    return (float)y;
+    return y;
 }
+UZU_HD float logf_glibc(float x) { return (float)log_wide(x); }
 
 // activation_type.rs:44-65: x / (1 + exp(-alpha*x)) with alpha = 1, evaluated in f32
 UZU_HD float silu_f32(float x) { return x / (1.0f + expf_glibc(-1.0f * x)); }
