@@ -1094,6 +1094,34 @@ def test_delta_net_prefill_state_precision(hip_ctx, T, pace):
     assert np.linalg.norm(got - exact) <= 1.1 * np.linalg.norm(serial - exact)
 
 
+@pytest.mark.parametrize("T", [17, 63, 130])
+@pytest.mark.parametrize("plant", ["value inf", "value nan", "key inf", "query nan", "beta nan", "decay nan", "decay inf", "decay above 1", "decay below 0", "decay 0", "state inf"])
+def test_delta_net_prefill_unusual_numbers(hip_ctx, T, plant):
+    """The chunked form against the token-by-token oracle where a chunk's zeros or logarithms could change the answer: an infinity or a NaN reaches its own token's outputs and later
+    ones (and of a value only its column), never an earlier token; decays that are no exp(-x) with x > 0 multiply the state as they are."""
+    Hv, Hk, Dv, t = 4, 2, 32, T - 6
+    z = delta_net_inputs(np.random.default_rng(T), T, Hv, Hk, Dv, 0.1)
+    name, what = plant.split(" ", 1)
+    x = {"inf": np.inf, "nan": np.nan, "above 1": 1.25, "below 0": -0.5, "0": 0.0}[what]
+    if name == "value":
+        z["rows"][t, 2 * Hk * 128 + 5] = 0x7F80 if what == "inf" else 0x7FC0
+    elif name == "state":
+        z["state"][1, 3, 7] = x
+    else:
+        z[{"key": "k", "query": "q"}.get(name, name)][t, 3 if name in ("key", "query") else 1] = x
+    if what == "above 1":
+        z["decay"][3:9, 2] = x
+    want_state, want = z["state"].copy(), np.zeros((T, Hv * Dv), np.uint16)
+    O.call("orc_delta_net_prefill", z["q"], z["k"], z["beta"], z["decay"], z["rows"], want_state, want, Hv, Hk, 128, Dv, Hk * 128, Hv * Dv, T)
+    got, state = hip_delta_net_prefill(hip_ctx, z, Hv, Hk, Dv)
+    g, w = f32(got), f32(want)
+    assert np.array_equal(np.isfinite(g), np.isfinite(w)) and np.array_equal(np.isfinite(state), np.isfinite(want_state))
+    ok, sok = np.isfinite(w), np.isfinite(want_state)
+    assert np.isfinite(w[:t]).all() or name == "state"
+    assert (np.abs(g - w)[ok] <= 2e-2 * np.maximum(1.0, np.abs(w[ok]))).all()
+    np.testing.assert_allclose(state[sok], want_state[sok], rtol=1e-4, atol=1e-4)
+
+
 # ------------------------------------------------------------------------------------------ command buffer
 def test_command_buffer_typestate_copy_fill_graph(hip_ctx):
     """CommandBuffer states, encode_copy / encode_fill, gpu_execution_time, and graph replay (re-submit)."""

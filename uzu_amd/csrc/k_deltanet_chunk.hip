@@ -13,7 +13,8 @@
 // four small dense products per chunk instead of 32 dependent steps; a workgroup owns 16 of a head's Dv columns, so
 // 128 workgroups are busy and every product has hundreds of independent FMAs per thread.
 // Same algebra, different rounding order: the state is no further from 64 bits than the recurrence's (dn_chunk_scan_mfma_kernel).  Decays are carried in log space
-// (log a clamped at -80) so that products over a chunk cannot underflow into 0 / 0.
+// (log 0 = -104, whose exponential is 0 in f32) so that products over a chunk cannot underflow into 0 / 0.  An infinity or a NaN would reach the whole chunk through the
+// zeros of T and P, where the recurrence hands it on from its token and its value column only: a workgroup of the plain scan that meets one walks its columns again token by token.
 #include <stdlib.h>
 
 #include "device_utils.h"
@@ -28,7 +29,7 @@ constexpr int CC = 32;        // tokens per chunk
 constexpr int DKC = 128;      // head_k_dim
 constexpr int KP = DKC + 4;   // LDS row pitch of K / Q / S rows in floats (conflict-free b128 reads across rows)
 constexpr int TP = CC + 1;    // LDS row pitch of the 32 x 32 matrices
-constexpr int WS_FLOATS = 2 * CC * CC + 2 * CC; // per (chunk, value head): T, P, A, W
+constexpr int WS_FLOATS = 2 * CC * CC + 4 * CC; // per (chunk, value head): T, P, A, W, the decays a, the strengths b
 } // namespace
 
 // Sequence split (round 4).  The chain of n chunk steps is the scan's whole cost (2.5 us per chunk with half of the CUs idle: 159 us per 2043-token pass
@@ -76,10 +77,11 @@ template <int CTRL> __device__ __forceinline__ double dpp_f64(double v) {
     return bits_to_f64((uint64_t)hi << 32 | lo);
 }
 // log a_t, in 64 bits until an exponential of a difference is rounded: f32 prefix sums of fast decays (a = 1/e: -32 at a chunk's end) cost the state 1e-6 of its norm, the
-// recurrence has 6e-8.  Decay 0: clamped, the state is wiped either way.
+// recurrence has 6e-8.  Decay 0: -104, whose exponential rounds to 0; a NaN or the logarithm of a negative decay stays NaN.
 // The sum over the tokens up to this one, a token a lane.
 __device__ __forceinline__ double log_prefix(float d, int token) {
-    double l = fmax(log_wide(d), -80.0);
+    double l = log_wide(d);
+    l = l < -104.0 ? -104.0 : l;
     // (lane i - 1, - 2, - 4, - 8 of a row of sixteen, or 0; then row 0's total to row 1)
     l += dpp_f64<0x111>(l), l += dpp_f64<0x112>(l), l += dpp_f64<0x114>(l), l += dpp_f64<0x118>(l);
     const double before = dpp_f64<0x142>(l);
@@ -112,6 +114,8 @@ __global__ void __launch_bounds__(256) dn_chunk_prep_kernel(const float* q_norm,
     const uint32_t groups_per_head = num_v_heads / num_k_heads;
     const uint32_t chunk = blockIdx.x, hv = blockIdx.y, hk = hv / groups_per_head;
     const uint32_t t0 = chunk * CC;
+    float* const w_t = ws + ((size_t)chunk * num_v_heads + hv) * WS_FLOATS;
+    float* const w_p = w_t + CC * CC;
     if constexpr (FUSED) {
         if (tid < 32) s_exp_tab[tid] = kExp2fTab[tid];
         const uint32_t lane = tid & 63, wave = tid >> 6;
@@ -183,6 +187,7 @@ __global__ void __launch_bounds__(256) dn_chunk_prep_kernel(const float* q_norm,
             }
             s_lg[tid] = log_prefix(d, tid);
             s_b[tid] = b;
+            w_t[2 * CC * CC + 2 * CC + tid] = d, w_t[2 * CC * CC + 3 * CC + tid] = b;
         }
     } else {
     // K, Q rows of the chunk (zero rows past the end: b = 0, a = 1 there, so they change nothing)
@@ -201,6 +206,7 @@ __global__ void __launch_bounds__(256) dn_chunk_prep_kernel(const float* q_norm,
         const float d = live ? decay_buf[(size_t)(t0 + tid) * num_v_heads + hv] : 1.0f;
         s_lg[tid] = log_prefix(d, tid);
         s_b[tid] = live ? beta_buf[(size_t)(t0 + tid) * num_v_heads + hv] : 0.0f;
+        w_t[2 * CC * CC + 2 * CC + tid] = d, w_t[2 * CC * CC + 3 * CC + tid] = s_b[tid];
     }
     }
     __syncthreads();
@@ -223,11 +229,9 @@ __global__ void __launch_bounds__(256) dn_chunk_prep_kernel(const float* q_norm,
         for (int j = 0; j < 4; ++j) sKK[i * TP + j0 + j] = kk[j], sQK[i * TP + j0 + j] = qk[j];
     }
     __syncthreads();
-    float* w_t = ws + ((size_t)chunk * num_v_heads + hv) * WS_FLOATS;
-    float* w_p = w_t + CC * CC;
     for (int idx = tid; idx < CC * CC; idx += 256) {
         const int i = idx / CC, j = idx % CC;
-        const float ratio = exp_wide(fmin(s_lg[i] - s_lg[j], 0.0), FUSED ? s_exp_tab : kExp2fTab); // A_i / A_j for j <= i
+        const float ratio = exp_wide(j <= i ? s_lg[i] - s_lg[j] : 0.0, FUSED ? s_exp_tab : kExp2fTab); // A_i / A_j for j <= i
         sM[i * TP + j] = j < i ? s_b[i] * ratio * sKK[i * TP + j] : 0.0f;
         w_p[idx] = j <= i ? ratio * sQK[i * TP + j] : 0.0f;
     }
@@ -326,6 +330,7 @@ __global__ void __launch_bounds__(256) dn_chunk_scan_mfma_kernel(const float* q_
         }
     };
     float vreg[4] = {0.f, 0.f, 0.f, 0.f};
+    float off_sum = 0.f; // 0, or NaN behind an output or a state value that is no number
     auto publish = [&]() {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -399,7 +404,7 @@ __global__ void __launch_bounds__(256) dn_chunk_scan_mfma_kernel(const float* q_
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const uint32_t t = t0 + tb + 4 * kq + r;
-                if (t < suffix_len) out[(size_t)t * value_dim + hv * head_v_dim + dv_base + i16] = f32_to_bf16(o[r]);
+                if (t < suffix_len) out[(size_t)t * value_dim + hv * head_v_dim + dv_base + i16] = f32_to_bf16(o[r]), off_sum = fmaf(o[r], 0.f, off_sum);
             }
         }
         // ---- stage 4 (all waves): S = A_C S + (D W)^T K for dk tiles 2 wave, 2 wave + 1; contraction over tokens 4 s + kq
@@ -421,6 +426,41 @@ const float* kc = sK + 4 * kq * KP + 32 * wave + 16 * t + i16;
         lds_barrier(); // all reads of this chunk's LDS operands are done
         if (c + 1 < n_chunks) publish();
         lds_barrier();
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) off_sum = fmaf(creg[t][r], 0.f, off_sum);
+    uint32_t* s_off = (uint32_t*)sR; // (read for the last time in front of the last barrier)
+    const bool off = __ballot(!(off_sum == 0.f)) != 0;
+    if (lane == 0) s_off[wave] = off;
+    lds_barrier();
+    if (s_off[0] | s_off[1] | s_off[2] | s_off[3]) { // the recurrence from the state in memory, 16 lanes a value column
+        __syncthreads(); // (every wave's own outputs have been written: those below replace them)
+        const uint32_t col = tid >> 4, part = tid & 15;
+        float* srow = state + ((size_t)hv * head_v_dim + dv_base + col) * DKC + 8 * part;
+        float sv[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sv[e] = srow[e];
+        for (uint32_t t = 0; t < suffix_len; ++t) {
+            const float* w = ws + ((size_t)(t / CC) * num_v_heads + hv) * WS_FLOATS + 2 * CC * CC + 2 * CC + t % CC;
+            const float *kr = k_norm + (size_t)t * key_dim + hk * DKC + 8 * part, *qr = q_norm + (size_t)t * key_dim + hk * DKC + 8 * part;
+            const float a = w[0], b = w[CC], v = bf16_to_f32(in_proj[(size_t)t * total_proj_dim + 2 * key_dim + hv * head_v_dim + dv_base + col]);
+            float sk = 0.f, o = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sk = fmaf(sv[e], kr[e], sk);
+            const float d = b * (v - a * group_sum<16>(sk));
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                sv[e] = a * sv[e] + d * kr[e];
+                o = fmaf(sv[e], qr[e], o);
+            }
+            o = group_sum<16>(o);
+            if (part == 0) out[(size_t)t * value_dim + hv * head_v_dim + dv_base + col] = f32_to_bf16(o);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) srow[e] = sv[e];
+        return;
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t)
