@@ -86,6 +86,21 @@ def test_linear_f32_from_three_bf16_parts(hip_ctx, rows, n, k, act):
     assert (np.abs(got - want) <= bound + 2.0 ** -23 * (np.abs(want) + np.abs(res))).all()
 
 
+@pytest.mark.parametrize("rows,n,k", [(300, 700, 2048), (1025, 4100, 128), (17, 70, 256), (600, 4100, 1024)])
+@pytest.mark.parametrize("power", [-118, -123])
+def test_linear_f32_parts_of_tiny_numbers(hip_ctx, rows, n, k, power):
+    """... numbers whose last bits lie below the smallest bf16 number: the parts carry them all the same, in whole products and in ones cut along k inside a part.  The bound of the test
+    above; the results themselves are normal numbers (weights of 2^20)."""
+    rng = np.random.default_rng(rows + n)
+    x = f32(rng.uniform(1.0, 4.0, (rows, k)) * rng.choice([-1.0, 1.0], (rows, k)) * 2.0 ** power)
+    w = O.to_bf16(rng.standard_normal((n, k)) * 2.0 ** 20)
+    got = linear(hip_ctx, x, w, act=0, bf16=0).astype(np.float64)
+    want = x.astype(np.float64) @ w.T.astype(np.float64)
+    mass = np.abs(x.astype(np.float64)) @ np.abs(w.T.astype(np.float64))
+    assert (np.abs(got - want) <= 4 * 2.0 ** -24 * np.sqrt(3 * k) * mass).all()
+    assert np.linalg.norm((got - want) / 2.0 ** power) <= 2.0 ** -21 * np.linalg.norm(want / 2.0 ** power)
+
+
 def test_linear_f32_parts_keep_infinities_and_nans(hip_ctx):
     rng = np.random.default_rng(3)
     x, w = rng.standard_normal((40, 1024), dtype=np.float32), O.to_bf16(np.abs(rng.standard_normal((700, 1024), dtype=np.float32)) + 0.5)

@@ -202,23 +202,25 @@ template <int PIECES> __device__ __forceinline__ void dma16(const void* base, co
 
 // f32 products on the same matrix cores: an f32 number is three bf16 numbers, x = hi + mid + lo exactly (8 + 8 + 8 significant bits, each part the truncation of what the
 // parts before it leave), weights are bf16 already, and a product of two bf16 numbers is exact in f32: the sum over 3 k products, the small parts first, is a sum of the
-// f32 products' own bits with f32 accumulation.  Three bf16 products are five times the rate of the f32 matrix instructions.  (Parts below 2^-126 may be flushed;
-// infinities and NaNs stay in hi.)
+// f32 products' own bits with f32 accumulation.  Three bf16 products are five times the rate of the f32 matrix instructions.  The small parts are stored 2^7 and 2^14 times
+// as large, no part larger than x, and the running sum is scaled back at a part's end: bf16 ends at 2^-133, and unscaled parts lose bits of every x below 2^-110 (here
+// below 2^-124).  Infinities and NaNs stay in hi.
+constexpr float kPartDown = 1.0f / 128.0f;
 __device__ __forceinline__ void split_bf16(float x, uint16_t& hi, uint16_t& mid, uint16_t& lo) {
     const uint32_t u = f32_to_bits(x);
     const bool finite = (u & 0x7F800000u) != 0x7F800000u;
-    const float h = bits_to_f32(u & 0xFFFF0000u), r = x - h, m = bits_to_f32(f32_to_bits(r) & 0xFFFF0000u);
+    const float h = bits_to_f32(u & 0xFFFF0000u), r = (x - h) * 128.0f, m = bits_to_f32(f32_to_bits(r) & 0xFFFF0000u);
     hi = finite ? (uint16_t)(u >> 16) : f32_to_bf16(x);
     mid = finite ? (uint16_t)(f32_to_bits(m) >> 16) : (uint16_t)0;
-    lo = finite ? (uint16_t)(f32_to_bits(r - m) >> 16) : (uint16_t)0;
+    lo = finite ? (uint16_t)(f32_to_bits((r - m) * 128.0f) >> 16) : (uint16_t)0;
 }
 
 constexpr int kEpilogueGated = 16; // grouped experts: the weight rows are [up ; gate], the result act(gate, up) as bf16 rows (GatedRows)
 
-// parts: 1, or 3 for operand rows [lo | mid | hi].  partials (not GROUPED): blockIdx.z takes its share of the k-steps and leaves its sums there, f32 [z][rows][n].
+// parts: 1, or 3 for operand rows [lo | mid | hi].  partials (MB 1, not GROUPED): blockIdx.z takes its share of the k-steps and leaves its sums there, f32 [z][rows][n].
 template <int MB, int STAGES, bool GROUPED, int KIND, uint32_t parts>
 __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, const uint16_t* xb, uint32_t ldxb, GatedRows gr, float* partials) {
-    constexpr bool GATED = KIND == kEpilogueGated;
+    constexpr bool GATED = KIND == kEpilogueGated, CUT = !GROUPED && MB == 1;
     constexpr int DK = 64, DM = 64 * MB, AP = DM * DK * 2 / 4096, BP = DN * DK * 2 / 4096; // 1 KB pieces per wave: A, B
     constexpr uint32_t STAGE = (DM + DN) * DK * 2, ROW = DK * 2, CHUNKS = DK / 8, RPP = 1024 / ROW; // row bytes, 16-byte chunks per row, rows per piece
     extern __shared__ __attribute__((aligned(1024))) uint8_t s_dma[];
@@ -291,6 +293,12 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
             if (kt + 1 < steps) fetch(kt + 1, (kt + 1) & 1);
         }
+        if constexpr (parts == 3) {
+            if (t_lo + kt == w_steps || t_lo + kt == 2 * w_steps) { // (a part ends: its sums have its scale)
+#pragma unroll
+                for (int i = 0; i < MB; ++i) acc[i][0] *= kPartDown, acc[i][1] *= kPartDown;
+            }
+        }
         const uint8_t* at = s_dma + (STAGES == 1 ? 0 : (kt & 1)) * STAGE;
 #pragma unroll
         for (uint32_t s = 0; s < DK / 16; ++s) {
@@ -308,6 +316,14 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
         }
     }
 
+    if constexpr (parts == 3) {
+        if (CUT && partials) { // a share that ends inside the small parts
+            const uint32_t last = t_lo + steps - 1;
+            const float down = last >= 2 * w_steps ? 1.0f : last >= w_steps ? kPartDown : kPartDown * kPartDown;
+#pragma unroll
+            for (int i = 0; i < MB; ++i) acc[i][0] *= down, acc[i][1] *= down;
+        }
+    }
     if constexpr (GATED) {
         const uint32_t ff = p.n / 2, f = n_t * 64 + wn * 32 + l32;
         if (f >= ff) return;
@@ -327,7 +343,7 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
             }
         return;
     }
-    if (!GROUPED && partials) {
+    if (CUT && partials) {
         float* out = partials + (size_t)blockIdx.z * p.rows * p.n;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
