@@ -121,7 +121,8 @@ uzu_status uzu_hip_model_read_layer_output_f32(uzu_hip_model* m, uint32_t layer,
  *   dyn_tanh: tanh(alpha x) scales + biases, then (shift != NULL) the token shift from prev_inout (state row in, state row out) at position `start`.
  *   latent_norm_append: RMS-normalised latents of positions start.. into cache_inout [(start + rows)][rank].
  *   latent_attention: latent-space attention core over cache [(start + rows)][rank]; form 0 dispatch, 1 simple, 2 tiled.
- *   moe: score routing (softmax over routed + identity outputs, choice by score + selection_bias) + SiLU-gated experts + identity experts + residual. */
+ *   moe: score routing (softmax over routed + identity outputs, choice by score + selection_bias) + SiLU-gated experts + identity experts + residual;
+ *        bf16_products 0 / 1 row by row, 2 / 3 grouped by expert on the matrix cores with bf16 / f32 products. */
 uzu_status uzu_hip_s32_linear(uzu_hip_context* ctx, const float* x, const uint16_t* w, const uint16_t* bias, const float* residual, float* y, uint32_t rows, uint32_t n, uint32_t k,
                               uint32_t batch, uint32_t act, uint32_t bf16_products, uint32_t form);
 uzu_status uzu_hip_s32_dyn_tanh(uzu_hip_context* ctx, const float* x, const float* scales, const float* biases, float alpha, const float* shift, float* prev_inout, uint32_t start,

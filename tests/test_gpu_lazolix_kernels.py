@@ -101,6 +101,47 @@ def test_linear_f32_parts_of_tiny_numbers(hip_ctx, rows, n, k, power):
     assert np.linalg.norm((got - want) / 2.0 ** power) <= 2.0 ** -21 * np.linalg.norm(want / 2.0 ** power)
 
 
+@pytest.mark.parametrize("rows,n,k", [(40, 700, 1024), (2050, 4100, 64), (600, 4100, 128), (1100, 8200, 64)])
+def test_linear_f32_parts_with_weights_that_are_no_numbers(hip_ctx, rows, n, k):
+    """An infinite weight makes an infinity of every non-zero operand, whichever of its parts are zero, and a NaN of zero; a NaN weight NaNs: in products cut along k and in every tile form."""
+    rng = np.random.default_rng(rows)
+    x = O.to_bf16(rng.standard_normal((rows, k), dtype=np.float32) + np.float32(3.0) * rng.choice([-1, 1], (rows, k)).astype(np.float32))  # (one part)
+    x[::2] = f32(x[::2] * np.float32(1.001))  # (three)
+    w = O.to_bf16(rng.standard_normal((n, k), dtype=np.float32))
+    w[3, 5], w[n - 1, k - 1], w[n // 2, 0] = np.inf, -np.inf, np.nan
+    w[7, 1], w[7, 2] = np.inf, np.inf
+    x[5, 5], x[rows - 1, k - 1], x[9, 1] = 0.0, np.inf, -np.inf
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ w.T.astype(np.float64)
+    got = linear(hip_ctx, x, w, act=0, bf16=0)
+    ok = np.isfinite(want)
+    assert np.array_equal(got[~ok], want[~ok].astype(np.float32), equal_nan=True) and np.isfinite(got[ok]).all()
+    assert np.abs(got[ok] - want[ok]).max() <= 3e-5 * np.abs(want[ok]).max()
+
+
+def test_f32_experts_with_weights_that_are_no_numbers(hip_ctx):
+    """... in the grouped products of the experts, the gated one and the one behind it: infinities and NaNs where 64 bits have them."""
+    rng = np.random.default_rng(6)
+    rows, routed, top, ff, d = 50, 4, 2, 256, 320
+    x, wr = O.to_bf16(rng.standard_normal((rows, d))).astype(np.float32), O.to_bf16(rng.standard_normal((routed, d)) * 0.5)
+    w13 = O.to_bf16(rng.standard_normal((routed, 2 * ff, d)) / np.sqrt(d))
+    w2 = O.to_bf16(rng.standard_normal((routed, d, ff)) / np.sqrt(ff))
+    w13[1, 4, 7], w13[2, ff + 9, 3], w2[0, 11, 2] = np.inf, np.inf, -np.inf  # up, gate, down
+    corr, res = np.zeros(routed, np.float32), np.zeros((rows, d), np.float32)
+    y, ids, wts = np.empty((rows, d), dtype=np.float32), np.empty((rows, top), dtype=np.int32), np.empty((rows, top), dtype=np.float32)
+    _ffi.call("uzu_hip_s32_moe", hip_ctx._h, ptr(x), ptr(O.bf16_bits(wr)), ptr(corr), ptr(O.bf16_bits(w13)), ptr(O.bf16_bits(w2)), ptr(res), ptr(y), ptr(ids), ptr(wts), C.c_uint32(rows),
+              C.c_uint32(d), C.c_uint32(ff), C.c_uint32(routed), C.c_uint32(0), C.c_uint32(top), C.c_uint32(3))
+    want = np.zeros((rows, d))
+    with np.errstate(invalid="ignore", over="ignore"):
+        for r in range(rows):
+            for e, wt in zip(ids[r], wts[r].astype(np.float64)):
+                up, gate = np.split(w13[e].astype(np.float64) @ x[r].astype(np.float64), 2)
+                want[r] += wt * (w2[e].astype(np.float64) @ (gate / (1 + np.exp(-gate)) * up))
+    ok = np.isfinite(want)
+    assert (~ok).any() and np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(y[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
+    assert np.abs(y[ok] - want[ok]).max() <= 2e-5 * np.abs(want[ok]).max()
+
+
 def test_linear_f32_parts_keep_infinities_and_nans(hip_ctx):
     rng = np.random.default_rng(3)
     x, w = rng.standard_normal((40, 1024), dtype=np.float32), O.to_bf16(np.abs(rng.standard_normal((700, 1024), dtype=np.float32)) + 0.5)

@@ -226,8 +226,9 @@ uzu_status uzu_hip_s32_moe(uzu_hip_context* ctx, const float* x, const uint16_t*
     UZU_PROPAGATE(S.up((const float*)nullptr, (size_t)rows * top * (ff ? ff : 1), &dh));
     UZU_PROPAGATE(S.up((const int32_t*)nullptr, (size_t)rows * top, &dids));
     UZU_PROPAGATE(k::moe_route_scores(ctx->stream, dx, dr, dsb, dids, dwt, rows, d, routed + identity, top));
-    if (bf16_products == 2) { // bf16 products through the grouped matrix-core form
+    if (bf16_products >= 2) { // the grouped matrix-core form, 2: bf16 products, 3: f32 products
         k::MoeGroupedParams gp{};
+        gp.f32_products = bf16_products == 3;
         uint32_t *perm, *slot_pos, *offsets, *cursor;
         float *y1, *y2;
         UZU_PROPAGATE(S.up((const float*)nullptr, (size_t)rows * top * 2 * ff, &y1));

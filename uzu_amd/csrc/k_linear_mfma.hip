@@ -214,6 +214,32 @@ __device__ __forceinline__ void split_bf16(float x, uint16_t& hi, uint16_t& mid,
     mid = finite ? (uint16_t)(f32_to_bits(m) >> 16) : (uint16_t)0;
     lo = finite ? (uint16_t)(f32_to_bits((r - m) * 128.0f) >> 16) : (uint16_t)0;
 }
+// A part that is zero times an infinite weight is a NaN where the f32 product is an infinity (the parts have x's sign, so nothing else can go wrong): a sum that came out as NaN
+// is made again from the f32 numbers themselves, one after the other.
+__device__ __forceinline__ float split_dot(const uint16_t* xrow, const uint16_t* wrow, uint32_t k) {
+    float sum = 0.0f;
+#pragma unroll 1
+    for (uint32_t c = 0; c < k; ++c)
+        sum = fmaf(bf16_to_f32(xrow[2 * k + c]) + (bf16_to_f32(xrow[k + c]) * kPartDown + bf16_to_f32(xrow[c]) * (kPartDown * kPartDown)), bf16_to_f32(wrow[c]), sum);
+    return sum;
+}
+// acc[r] = the sum of row row0 + (r & 3) + 8 (r >> 2) and weight row wrow
+__device__ __forceinline__ void split_repair(f32x16_t& acc, const uint16_t* xb, uint32_t k, const uint32_t* row_map, uint32_t row0, uint32_t row_end, const uint16_t* wrow) {
+    float all = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) all = fmaxf(all, acc[r] != acc[r] ? 1.0f : 0.0f);
+    if (!__builtin_expect(__ballot(all != 0.0f) != 0, 0)) return;
+    float sums[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sums[r] = acc[r];
+#pragma unroll 1
+    for (uint32_t r = 0; r < 16; ++r) {
+        const uint32_t row = row0 + (r & 3) + 8 * (r >> 2);
+        if (row < row_end && sums[r] != sums[r]) sums[r] = split_dot(xb + (size_t)(row_map ? row_map[row] : row) * 3 * k, wrow, k);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = sums[r];
+}
 
 constexpr int kEpilogueGated = 16; // grouped experts: the weight rows are [up ; gate], the result act(gate, up) as bf16 rows (GatedRows)
 
@@ -284,7 +310,7 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (row_map: nothing of the compiler's is in flight from here on)
     if (STAGES == 2) fetch(0, 0);
     const uint32_t a_base = (wm * 32 * MB + l32) * ROW, b_base = DM * ROW + (wn * 64 + l32) * ROW, key = l32 & 7;
-    for (uint32_t kt = 0; kt < steps; ++kt) {
+    auto step = [&](uint32_t kt) {
         if constexpr (STAGES == 1) {
             if (kt) lds_barrier(); // every wave has read step kt - 1
             fetch(kt, 0);
@@ -292,12 +318,6 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
         } else { // step kt is in LDS and every wave has read step kt - 1: the next step may land in its place
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
             if (kt + 1 < steps) fetch(kt + 1, (kt + 1) & 1);
-        }
-        if constexpr (parts == 3) {
-            if (t_lo + kt == w_steps || t_lo + kt == 2 * w_steps) { // (a part ends: its sums have its scale)
-#pragma unroll
-                for (int i = 0; i < MB; ++i) acc[i][0] *= kPartDown, acc[i][1] *= kPartDown;
-            }
         }
         const uint8_t* at = s_dma + (STAGES == 1 ? 0 : (kt & 1)) * STAGE;
 #pragma unroll
@@ -314,6 +334,27 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
                 for (int j = 0; j < 2; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, af[i]), __builtin_bit_cast(bf16x8_t, bf[j]), acc[i][j], 0, 0, 0);
         }
+    };
+    auto part_end = [&] { // its sums have its scale
+#pragma unroll
+        for (int i = 0; i < MB; ++i) acc[i][0] *= kPartDown, acc[i][1] *= kPartDown;
+    };
+    if constexpr (parts == 1) {
+        for (uint32_t kt = 0; kt < steps; ++kt) step(kt);
+    } else if constexpr (MB == 2) { // (a loop in a loop would need the sums' registers twice)
+        for (uint32_t kt = 0; kt < steps; ++kt) {
+            if (t_lo + kt == w_steps || t_lo + kt == 2 * w_steps) part_end();
+            step(kt);
+        }
+    } else {
+        uint32_t kt = 0;
+#pragma unroll 1
+        for (uint32_t end = w_steps;; end += w_steps) {
+            const uint32_t upto = end <= t_lo ? 0u : end - t_lo < steps ? end - t_lo : steps;
+            for (; kt < upto; ++kt) step(kt);
+            if (kt == steps) break;
+            part_end();
+        }
     }
 
     if constexpr (parts == 3) {
@@ -322,6 +363,15 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
             const float down = last >= 2 * w_steps ? 1.0f : last >= w_steps ? kPartDown : kPartDown * kPartDown;
 #pragma unroll
             for (int i = 0; i < MB; ++i) acc[i][0] *= down, acc[i][1] *= down;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const uint32_t n = GATED ? n_t * 64 + wn * 32 + l32 : n0 + (wn * 2 + j) * 32 + l32, ends = GATED ? p.n / 2 : p.n;
+                if (n >= ends) continue;
+#pragma unroll
+                for (int i = 0; i < MB; ++i)
+                    split_repair(acc[i][j], xb, p.k, GROUPED ? p.row_map : nullptr, m0 + (wm * MB + i) * 32 + 4 * half, r_hi, w + (size_t)(GATED && j ? ends + n : n) * p.k);
+            }
         }
     }
     if constexpr (GATED) {
@@ -414,12 +464,13 @@ __global__ void __launch_bounds__(256) linear_split_rows_kernel(const float* x, 
 }
 
 // the shares of a product cut along k, added in their order, and the product's end
-__global__ void __launch_bounds__(256) linear_finish_kernel(LinearF32Params p, const float* partials, uint32_t splits) {
+template <uint32_t PARTS> __global__ void __launch_bounds__(256) linear_finish_kernel(LinearF32Params p, const uint16_t* xb, const float* partials, uint32_t splits) {
     const size_t total = (size_t)p.rows * p.n, i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= total) return;
     float sum = partials[i];
     for (uint32_t z = 1; z < splits; ++z) sum += partials[z * total + i];
     const uint32_t row = (uint32_t)(i / p.n), n = (uint32_t)(i - (size_t)row * p.n);
+    if (PARTS == 3 && sum != sum) sum = split_dot(xb + (size_t)row * 3 * p.k, p.w + (size_t)n * p.k, p.k);
     p.y[(size_t)row * p.ldy + n] = linear_epilogue(sum, p.bias ? bf16_to_f32(p.bias[n]) : 0.0f, p, row, 0, n);
 }
 
@@ -457,7 +508,7 @@ template <uint32_t PARTS> uzu_status launch_dma_plain(hipStream_t s, const Linea
         float* partials = (float*)((char*)ws + ((size_t)p.rows * p.k * 2 * PARTS + 255) / 256 * 256);
         UZU_PROPAGATE((launch_dma_tile<1, 2, false, kEpilogueLean, PARTS>(s, p, ws, GatedRows(), partials, splits)));
         const size_t total = (size_t)p.rows * p.n;
-        return launch_check([&] { hipLaunchKernelGGL(linear_finish_kernel, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, s, p, partials, splits); }, "linear_finish");
+        return launch_check([&] { hipLaunchKernelGGL(linear_finish_kernel<PARTS>, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, s, p, ws, partials, splits); }, "linear_finish");
     }
     switch (epilogue_kind(p)) {
     case kEpilogueLean: return launch_dma<false, kEpilogueLean, PARTS>(s, p, ws);
