@@ -56,6 +56,20 @@ def test_linear_matrix_core_form_equals_the_plain_form(hip_ctx, rows, n, k, batc
     assert np.abs(a - want).max() <= 3e-5 * max(1.0, np.abs(want).max()) and np.abs(c - want).max() <= 3e-5 * max(1.0, np.abs(want).max())
 
 
+@pytest.mark.parametrize("rows,n,k,bf16", [(257, 128, 320, 0), (257, 128, 320, 1), (64, 70, 1024, 0), (17, 64, 64, 0)])
+def test_linear_without_the_matrix_cores(hip_ctx, rows, n, k, bf16):
+    """Form 2 keeps off the matrix cores at sizes where the dispatch takes them for f32 products as well: its 64 x 64 tiles add f32 product after f32 product in the order of k, which gives
+    the same bits here (a fused multiply-add: the product is exact in 64 bits; the sum's second rounding on the way to f32 can differ once in 2^29)."""
+    rng = np.random.default_rng(rows + k)
+    x, w = f32(rng.standard_normal((rows, k))), O.to_bf16(rng.standard_normal((n, k)))
+    got = linear(hip_ctx, x, w, act=0, bf16=bf16, form=2)
+    xb = O.to_bf16(x) if bf16 else x
+    want = np.zeros((rows, n), dtype=np.float32)
+    for c in range(k):
+        want = (want + np.multiply.outer(xb[:, c].astype(np.float64), w[:, c].astype(np.float64))).astype(np.float32)
+    assert np.mean(got == want) > 1 - 1e-4
+
+
 @pytest.mark.parametrize("rows,n,k,act", [(129, 8200, 1024, 0), (1000, 1025, 1024, 1), (255, 16400, 256, 0), (513, 8192, 256, 0), (2050, 4100, 128, 1), (128, 4100, 2048, 0), (33, 1024, 1024, 1), (300, 700, 2048, 0)])
 def test_linear_prompt_sized_form(hip_ctx, rows, n, k, act):
     """Prompt-sized products (both operands by LDS DMA): every tile form and buffer count, ragged last tiles in both directions, two k-steps and many, bias, activation and a residual

@@ -67,13 +67,13 @@ uzu_status uzu_hip_s32_linear(uzu_hip_context* ctx, const float* x, const uint16
         UZU_PROPAGATE(k::linear_mfma(ctx->stream, p));
     } else if (form == 2) { // without the matrix cores
         k::LinearF32Params q = p;
-        q.bf16_products = 0; // (the dispatcher only offers the matrix cores to bf16 products)
+        q.bf16_products = 0;
         if (bf16_products) { // round the operand here, then true f32 products: the same numbers as bf16 products
             std::vector<float> xr((size_t)rows * kk * batch);
             for (size_t i = 0; i < xr.size(); ++i) xr[i] = round_bf16(x[i]);
             UZU_HIP_TRY(hipMemcpy(dx, xr.data(), xr.size() * 4, hipMemcpyHostToDevice));
         }
-        UZU_PROPAGATE(k::linear_f32(ctx->stream, q));
+        UZU_PROPAGATE(k::linear_valu(ctx->stream, q));
     } else {
         UZU_PROPAGATE(k::linear_f32(ctx->stream, p));
     }

@@ -762,21 +762,18 @@ uzu_status depth_mix(hipStream_t s, const float* slots, size_t slot_stride, cons
 
 size_t linear_f32_bytes(const LinearF32Params& p) { return (size_t)p.batch * ((size_t)p.n * p.k * 2 + (size_t)p.rows * p.k * 4 + (size_t)p.rows * p.n * 4); }
 
-uzu_status linear_f32(hipStream_t s, const LinearF32Params& p, const char** variant) {
-    if (!p.rows || !p.n || !p.batch) return UZU_OK;
+static uzu_status linear_check(const LinearF32Params& p) {
     UZU_REQUIRE(p.x && p.w && p.y && p.k, "linear_f32: null argument");
     UZU_REQUIRE(!p.residual || p.batch == 1, "linear_f32: a residual only with one product per launch");
     UZU_REQUIRE(!p.mul_table || (p.mul_tokens && p.batch == 1 && !p.row_offsets && p.mul_col0 + p.n <= p.mul_ld), "linear_f32: a token multiplier needs the rows' tokens, one product, columns inside the table");
     UZU_REQUIRE(p.ldx >= p.k && p.ldy >= p.n && p.batch <= 65535, "linear_f32: row pitch below the row length");
-    if (p.row_offsets || p.row_map) { // the grouped / gathered form lives in the matrix-core kernel only
-        UZU_UNSUPPORTED(!linear_mfma_supported(p), "linear_f32: grouped / gathered rows need bf16 products and 8-aligned k");
-        if (variant) *variant = "linear_mfma_grouped";
-        return linear_mfma(s, p);
-    }
-    if (linear_few_supported(p)) {
-        if (variant) *variant = "linear_few";
-        return linear_few(s, p);
-    }
+    return UZU_OK;
+}
+
+uzu_status linear_valu(hipStream_t s, const LinearF32Params& p, const char** variant) {
+    if (!p.rows || !p.n || !p.batch) return UZU_OK;
+    UZU_PROPAGATE(linear_check(p));
+    UZU_UNSUPPORTED(p.row_offsets || p.row_map, "linear_valu: no grouped / gathered rows");
     if (p.rows <= 16) {
         const uint32_t vec = (p.k % 8 == 0 && p.ldx % 4 == 0 && p.x_batch % 4 == 0 && p.w_batch % 8 == 0 && (uintptr_t)p.x % 16 == 0 && (uintptr_t)p.w % 16 == 0) ? 1u : 0u;
         if (variant) *variant = "linear_rows";
@@ -787,19 +784,34 @@ uzu_status linear_f32(hipStream_t s, const LinearF32Params& p, const char** vari
         const dim3 grid((p.n + 3) / 4, (p.rows + 3) / 4, p.batch);
         return launch_check([&] { hipLaunchKernelGGL(linear_rows_kernel<4>, grid, dim3(256), 0, s, p, vec); }, "linear_rows");
     }
-    if (linear_mfma_supported(p)) {
-        if (variant) *variant = "linear_mfma";
-        return linear_mfma(s, p);
-    }
-    uzu_status split = UZU_OK;
-    if (linear_split(s, p, &split)) {
-        if (variant) *variant = "linear_split";
-        return split;
-    }
     if (variant) *variant = "linear_tile";
     const dim3 grid((p.n + TN - 1) / TN, (p.rows + TM - 1) / TM, p.batch);
     UZU_REQUIRE(grid.y <= 65535, "linear_f32: too many rows for one launch");
     return launch_check([&] { hipLaunchKernelGGL(linear_tile_kernel, grid, dim3(256), 0, s, p); }, "linear_tile");
+}
+
+uzu_status linear_f32(hipStream_t s, const LinearF32Params& p, const char** variant) {
+    if (!p.rows || !p.n || !p.batch) return UZU_OK;
+    UZU_PROPAGATE(linear_check(p));
+    if (p.row_offsets || p.row_map) { // the grouped / gathered form lives in the matrix-core kernel only
+        UZU_UNSUPPORTED(!linear_mfma_supported(p), "linear_f32: grouped / gathered rows need bf16 products and 8-aligned k");
+        if (variant) *variant = "linear_mfma_grouped";
+        return linear_mfma(s, p);
+    }
+    if (linear_few_supported(p)) {
+        if (variant) *variant = "linear_few";
+        return linear_few(s, p);
+    }
+    if (p.rows > 16 && linear_mfma_supported(p)) {
+        if (variant) *variant = "linear_mfma";
+        return linear_mfma(s, p);
+    }
+    uzu_status split = UZU_OK;
+    if (p.rows > 16 && linear_split(s, p, &split)) {
+        if (variant) *variant = "linear_split";
+        return split;
+    }
+    return linear_valu(s, p, variant);
 }
 
 uzu_status moe_route_scores(hipStream_t s, const float* x, const uint16_t* router, const float* selection_bias, int32_t* ids, float* weights, uint32_t rows, uint32_t d,

@@ -119,6 +119,8 @@ struct LinearF32Params {
     const uint32_t* row_map;
 };
 uzu_status linear_f32(hipStream_t s, const LinearF32Params& p, const char** variant = nullptr);
+// ... without the matrix cores, in f32 arithmetic throughout: a wave per output column up to 16 rows, 64 x 64 tiles that add in the order of k above
+uzu_status linear_valu(hipStream_t s, const LinearF32Params& p, const char** variant = nullptr);
 // the matrix-core form (k_linear_mfma.hip): bf16 products only; false = shape / mode not covered, nothing launched
 bool linear_mfma_supported(const LinearF32Params& p);
 uzu_status linear_mfma(hipStream_t s, const LinearF32Params& p);
