@@ -121,6 +121,21 @@ def test_attention_split_keys_form_on_few_rows(hip_ctx, H, G, dim, vd, window, c
         assert np.isfinite(got).all() and np.abs(got - want).max() < 6e-5 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("H,G,dim,vd,window,cap,T", [(4, 4, 8, 8, 33, 0.0, 40), (8, 2, 32, 16, 64, 0.0, 130), (6, 2, 16, 64, 128, 3.0, 300), (16, 4, 128, 128, 129, 0.0, 140), (4, 1, 64, 24, 500, 0.0, 620),
+                                                     (40, 1, 16, 16, 300, 0.0, 400), (2, 2, 128, 64, 1100, 0.0, 1200), (4, 2, 32, 32, 0, 0.0, 90)])
+def test_attention_of_decode_sized_passes(hip_ctx, H, G, dim, vd, window, cap, T):
+    """The form and the split of the keys that a pass of a few rows takes by itself: one stretch of 32 keys and the first beyond, two stretches a workgroup, stretches of 128, more items than a
+    tile, a window longer than what is cached; from 33 keys on it is not the simple form, whose bits differ (the query is fed as hi + lo bf16)."""
+    rng = np.random.default_rng(H * 100 + T + 3)
+    q, K, V = qkv(rng, T, H, G, dim, vd)
+    mx = {"heads": H, "kv_heads": G, "scale": 1.7 / np.sqrt(dim), "mask": {"size": window}, "softcap": cap}
+    for rows in (1, 3):
+        want = O.attention_core(f32(q)[T - rows:], O.to_bf16(K), O.to_bf16(V), mx, T - rows)
+        got = attention(hip_ctx, q[T - rows:], K, V, mx, T - rows, bf16=1, form=4)
+        assert np.isfinite(got).all() and np.abs(got - want).max() < 6e-5 * np.abs(want).max()
+        assert not np.array_equal(got, attention(hip_ctx, q[T - rows:], K, V, mx, T - rows, bf16=1, form=1))
+
+
 @pytest.mark.parametrize("bf16,form", [(0, 1), (1, 1), (1, 2)])
 @pytest.mark.parametrize("window", [1, 2, 31, 32, 33, 64, 65, 130])
 def test_one_key_stands_out_just_inside_and_just_outside_the_window(hip_ctx, bf16, form, window):

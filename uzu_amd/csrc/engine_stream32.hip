@@ -461,7 +461,7 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
             // decode-sized passes: spread a tile's key blocks over workgroups (a constant of the layer, so that a captured step stays valid as the context grows)
             uint32_t keys = h.sliding_window_size ? h.sliding_window_size : m->d.max_context_length;
             if (h.attention_chunk_size) keys = std::min(keys, h.attention_chunk_size);
-            if (rows <= 4 * S.max_seqs && rows * H <= 4096) ap.splits = std::min<uint32_t>(16, (keys + 127) / 128), ap.split_ws = S.att_ws, ap.split_ws_bytes = S.att_ws_bytes;
+            if (rows <= 4 * S.max_seqs && rows * H <= 4096) k::window_attention_split_keys(ap, keys, m->ctx->num_cus), ap.split_ws = S.att_ws, ap.split_ws_bytes = S.att_ws_bytes;
             RUN("window_attention", (size_t)rows * H * (hd + vd) * 4, k::window_attention(s, ap));
         } else if (h.mixer_kind == UZU_MIXER_GATED_LINEAR_ATTENTION) { // queries | keys | values | gate | decay down
             const uint32_t ldq = L.qkv.n, v_col = 2 * H * hd, g_col = v_col + H * vd, a_col = g_col + H * vd;

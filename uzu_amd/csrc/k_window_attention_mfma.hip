@@ -10,6 +10,8 @@
 //   O^T += V^T P^T  A = the value block transposed [vdim][32] from LDS, B = those 16 weights as hi + lo bf16; rescaling and the final 1 / l are per lane.
 // The k order inside an MFMA only has to agree between A and B: for O^T the lane's keys are taken in the order the S^T result already holds them.
 // Scores, weights and sums are f32; the sink enters as the initial maximum with weight 1 in the denominator.
+#include <algorithm>
+
 #include "device_utils.h"
 #include "gemm_convert.h"
 #include "kernels_stream32.h"
@@ -28,10 +30,10 @@ __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hi, uint3
 // IW waves of a workgroup own 32 items each, KG groups of such waves share the keys of a staged stretch (32 KG keys: group i takes its 32), so a workgroup is IW KG waves and
 // their unnormalised results meet in LDS at the end, in group order.  Prompts: IW 4, KG 2; a pass's tiles are about a workgroup per CU, and a wave alone on its SIMD waits for
 // itself at every exponential and every staged block (the next block's loads are in flight meanwhile; values are transposed two keys at a time).  2048 rows of 16 heads on 4,
-// width 128, window 1024: 147 us with four waves and no look-ahead, 61 so.  SPLIT (few items, many keys: decode steps): IW 1, KG 4, and grid.z
+// width 128, window 1024: 147 us with four waves and no look-ahead, 61 so.  SPLIT (few items, many keys: decode steps): grid.z
 // workgroups share an item tile's stretches (stretch i goes to workgroup i mod grid.z) and leave unnormalised sums with their running maximum / denominator in p.split_ws;
-// window_attention_merge_kernel combines them.  Tiles of 32 items then: with tiles of 128 three waves of four had none (8 sequences' step 25.6 us, now 14.0).  The sink belongs to
-// group 0 of split 0.
+// window_attention_merge_kernel combines them.  Two forms (window_attention_split_keys): IW 4, KG 1, stretches of 32 keys, and IW 1, KG 4, stretches of 128 (with IW 4 three waves
+// of four have no items, but they help staging).  The sink belongs to group 0 of split 0.
 template <int NB, int IW, int KG, bool SPLIT> // dim and vdim padded to RP = 32 NB
 __global__ void __launch_bounds__(64 * IW * KG) window_attention_mfma_kernel(WindowAttentionParams p) {
     constexpr int RP = 32 * NB, KP = RP * 2 + 16, TP = 80, VEC = RP / 8, T = 64 * IW * KG, KEYS = 32 * KG;
@@ -42,7 +44,7 @@ __global__ void __launch_bounds__(64 * IW * KG) window_attention_mfma_kernel(Win
     const uint32_t hg = p.heads / p.kv_heads, g = blockIdx.y;
     // the sequence of this tile (tiles of ITEMS items): a lane per sequence, 64 at a time
     constexpr uint32_t ITEMS = 32 * IW;
-    uint32_t wg = blockIdx.x, z = 0xFFFFFFFFu, before = 0;
+    uint32_t wg = blockIdx.x, z = p.nseq == 1 ? 0u : 0xFFFFFFFFu, before = 0;
     for (uint32_t z0 = 0; z0 < p.nseq && z == 0xFFFFFFFFu; z0 += 64) {
         const uint32_t ln = threadIdx.x & 63;
         uint32_t upto = z0 + ln < p.nseq ? (p.spans[z0 + ln].count * hg + ITEMS - 1) / ITEMS : 0u;
@@ -291,6 +293,16 @@ uint32_t blocks_of(const WindowAttentionParams& p) {
 
 size_t window_attention_split_ws_bytes(uint32_t rows, uint32_t heads, uint32_t splits) { return (size_t)rows * heads * splits * (128 + 4) * 4; }
 
+// A workgroup that has one or two stretches of 32 keys to walk is through before one with a stretch of 128 has staged it and its four waves have met; with more of them the four
+// waves are the faster walkers.  How few it can have is how many workgroups run at once: one a CU.  Heads of 128, 4 key / value heads, us a launch with its merge, stretches of 32 /
+// of 128: one sequence, window 40 9.8 / 14.0, 128 10.5 / 14.4, 512 (16 splits) 10.1 / 15.4 (4), 1024 (16) 12.6 / 14.6 (8); 8 sequences, window 256 (8) 10.5 / 14.8 (2),
+// 512 (8) 13.0 / 15.1 (4), 1024 (8) 18.3 / 14.1 (8); 32 sequences, window 128 (2) 13.3 / 14.5 (2), 256 (2) 18.5 / 14.6 (2).  Up to 32 keys the simple form is as fast.
+void window_attention_split_keys(WindowAttentionParams& p, uint32_t keys, uint32_t num_cus) {
+    const uint32_t blocks = (keys + 31) / 32, at_once = num_cus / std::max(1u, p.tiles * p.kv_heads), splits = std::min(blocks, std::max(2u, std::min(16u, at_once)));
+    if (blocks <= 2 * splits) p.split_items = 128, p.splits = splits;
+    else p.split_items = 32, p.splits = std::min(16u, std::max(2u, (keys + 127) / 128));
+}
+
 // bf16 caches, head widths that are multiples of 8 up to 128 (16-byte rows); prompt-sized passes, or a decode-sized pass with a workspace to split its keys
 // (without one a decode step's few items would walk all their keys in one nearly empty workgroup: the simple form does that better)
 static bool use_split(const WindowAttentionParams& p) {
@@ -315,9 +327,8 @@ uzu_status window_attention_mfma(hipStream_t s, const WindowAttentionParams& p) 
     UZU_REQUIRE(window_attention_mfma_supported(p), "window_attention: the matrix-core form does not take this shape");
     const uint32_t nb = blocks_of(p);
     if (use_split(p)) {
-        if (nb == 1) UZU_PROPAGATE((launch<1, 1, 4, true>(s, p)));
-        else if (nb == 2) UZU_PROPAGATE((launch<2, 1, 4, true>(s, p)));
-        else UZU_PROPAGATE((launch<4, 1, 4, true>(s, p)));
+        if (p.split_items == 128) UZU_PROPAGATE(nb == 1 ? (launch<1, 4, 1, true>(s, p)) : nb == 2 ? (launch<2, 4, 1, true>(s, p)) : (launch<4, 4, 1, true>(s, p)));
+        else UZU_PROPAGATE(nb == 1 ? (launch<1, 1, 4, true>(s, p)) : nb == 2 ? (launch<2, 1, 4, true>(s, p)) : (launch<4, 1, 4, true>(s, p)));
         return launch_check([&] { hipLaunchKernelGGL(window_attention_merge_kernel, dim3(p.rows * p.heads), dim3(128), 0, s, (const float*)p.split_ws, p.out, p.splits, p.vdim, 32 * nb, p.gate, p.ldgate, p.heads, p.ldo, p.out_scale); },
                             "window_attention_merge");
     }

@@ -342,13 +342,15 @@ struct WindowAttentionParams {
     uint32_t form;  // 0: chosen by shape; 1: the simple form (a wave per row and head); 2: the matrix-core form
     uint32_t nseq;  // entries of `spans`
     uint32_t tiles; // sum over the sequences of ceil(count * (heads / kv_heads) / 128): the matrix-core form's item tiles (the caller knows the counts)
-    uint32_t tiles32; // ... of ceil(count * (heads / kv_heads) / 32): its key-split form's
+    uint32_t tiles32; // ... of ceil(count * (heads / kv_heads) / 32): its key-split form's with split_items = 32
     // matrix-core form, few rows over many keys (decode): `splits` > 1 workgroups share the key blocks of an item tile, partial sums go through split_ws
     // (window_attention_split_ws_bytes(rows, heads, splits) bytes) and a merge launch.  0 / null: one workgroup walks all keys of its tile.
-    uint32_t splits;
+    uint32_t splits, split_items; // split_items: items a workgroup takes, 128 (stretches of 32 keys) or 32 (of 128; also 0)
     float* split_ws;
     size_t split_ws_bytes;
 };
+// `splits` and `split_items` of a decode-sized pass whose rows see `keys` keys at the most, from `tiles` and `kv_heads`: at most 16 splits
+void window_attention_split_keys(WindowAttentionParams& p, uint32_t keys, uint32_t num_cus);
 size_t window_attention_split_ws_bytes(uint32_t rows, uint32_t heads, uint32_t splits);
 bool window_attention_mfma_supported(const WindowAttentionParams& p);
 uzu_status window_attention(hipStream_t s, const WindowAttentionParams& p);
