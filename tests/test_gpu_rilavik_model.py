@@ -137,23 +137,36 @@ def test_greedy_choices_of_many_sequences(hip_ctx, tmp_path):
 
 
 def test_attention_tiles_of_more_sequences_than_a_wave_has_lanes(hip_ctx, tmp_path):
-    """70 sequences in one pass through the attention's matrix-core form, prompts (tiles of 128 items, keys in two groups) and then a token each (keys over workgroups and waves): every
-    sequence's logits are those it gets in a pass of its own, up to bf16 products that round the other way."""
-    cfg = O.config(vocab=53, width=64, layers=[O.parallel_layer(O.left_half(4, 2, 32, 24, 40, conv=2), O.right_half(2, 8, 8, groups=1, norm_groups=1, conv=2), 0.9, 0.4)])
+    """70 sequences in one pass through the attention's matrix-core forms: portions of 16 to 28 tokens (at least 16 rows a sequence, under the 2048 rows of a pass: tiles of 128 items) until the
+    longer window is full, then a token each (two layers: tiles of 128 items over stretches of 32 keys for the window of 40, tiles of 32 over stretches of 128 for the one of 200).
+    Every sequence's logits are those it gets in a pass of its own, up to bf16 products that round the other way; three of them are held to 64 bits."""
+    layer = lambda window: O.parallel_layer(O.left_half(4, 2, 32, 24, window, conv=2), O.right_half(2, 8, 8, groups=1, norm_groups=1, conv=2), 0.9, 0.4)
+    cfg = O.config(vocab=53, width=64, layers=[layer(200), layer(40)])
     W = O.weights(cfg, 7)
     O.write_model_dir(str(tmp_path / "m"), cfg, W)
-    m = HipModel(hip_ctx, loader.load_model_dir(str(tmp_path / "m"), max_context_length=256), MODEL_BATCH(70))
-    prompts = [prompt(cfg, 17 + (i * 29) % 90, i) for i in range(70)]
-    states = [m.new_state() for _ in prompts]
-    together, _ = m.step_batch(states, prompts, [[len(p) - 1] for p in prompts])
-    next_together, _ = m.step_batch(states, [[5]] * 70, [[0]] * 70)
-    for i, p in enumerate(prompts):
-        st = m.new_state()
-        alone, _ = m.step_batch([st], [p], [[len(p) - 1]])
-        next_alone, _ = m.step_batch([st], [[5]], [[0]])
+    m = HipModel(hip_ctx, loader.load_model_dir(str(tmp_path / "m"), max_context_length=320), MODEL_BATCH(70))
+    cuts = [[16 + (5 * i + 7 * j) % 13 for j in range(10)] for i in range(70)]
+    prompts = [prompt(cfg, sum(c), i) for i, c in enumerate(cuts)]
+    assert max(sum(c[j] for c in cuts) for j in range(10)) <= 2048 and min(map(len, prompts)) > 200
+    states, at, together = [m.new_state() for _ in prompts], [0] * 70, []
+    for j in range(10):
+        logits, _ = m.step_batch(states, [p[a:a + c[j]] for p, a, c in zip(prompts, at, cuts)], [[c[j] - 1] for c in cuts])
+        at = [a + c[j] for a, c in zip(at, cuts)]
+        together.append(logits)
+    together.append(m.step_batch(states, [[5]] * 70, [[0]] * 70)[0])
+    for i, (p, c) in enumerate(zip(prompts, cuts)):
+        st, a, alone = m.new_state(), 0, []
+        for n in c:
+            alone.append(m.step_batch([st], [p[a:a + n]], [[n - 1]])[0][0])
+            a += n
+        alone.append(m.step_batch([st], [[5]], [[0]])[0][0])
         st.close()
-        for got, want in ((together[i], alone[0]), (next_together[i], next_alone[0])):
-            assert np.abs(got - want).max() <= 2.0 ** -6 * np.abs(want).max(), i
+        for got, want in zip(together, alone):
+            assert np.abs(got[i] - want).max() <= 2.0 ** -6 * np.abs(want).max(), i
+        if i in (0, 64, 69):
+            exact, _ = O.forward(cfg, {k: v.astype(np.float64) for k, v in W.items()}, p + [5])
+            rows = [*(np.cumsum(c) - 1), sum(c)]
+            assert rows_ok(O.logit_error(np.stack([t[i] for t in together]), exact[rows]), False), i
     for st in states:
         st.close()
     m.close()
