@@ -342,6 +342,17 @@ def test_linear_of_a_few_rows(hip_ctx, rows, n, k, batch, act):
     assert np.abs(got - want).max() <= 3e-5 * max(1.0, np.abs(want).max())
 
 
+def test_experts_of_a_few_rows_refuse_a_row_that_fits_no_workgroup(hip_ctx):
+    """A width that one row's step refuses (its input does not fit the workgroup's LDS) is refused for a few rows as well: a model is served at every row count or not at all."""
+    d, ff = 12352, 64
+    x, w = np.ones((2, d), np.float32), np.zeros((1, 2 * ff, d), np.uint16)
+    y, ids, wts = np.empty((2, d), np.float32), np.empty((2, 1), np.int32), np.empty((2, 1), np.float32)
+    for rows in (1, 2):
+        with pytest.raises(_ffi.UzuHipError, match="LDS row"):
+            _ffi.call("uzu_hip_s32_moe", hip_ctx._h, ptr(x), ptr(w), ptr(np.zeros(1, np.float32)), ptr(w), ptr(w), ptr(x), ptr(y), ptr(ids), ptr(wts), C.c_uint32(rows), C.c_uint32(d),
+                      C.c_uint32(ff), C.c_uint32(1), C.c_uint32(0), C.c_uint32(1), C.c_uint32(1))
+
+
 @pytest.mark.parametrize("rows,n,k", [(3, 4112, 1024), (8, 2048, 4096), (16, 520, 2048), (24, 1024, 2048), (12, 300, 1024)])
 def test_linear_of_a_few_rows_sums(hip_ctx, rows, n, k):
     """How far the f32 sums are from 64 bits, held to the sums a wave per column makes (64 lanes that add every 64th product one by one, then in pairs; products of bf16 numbers are

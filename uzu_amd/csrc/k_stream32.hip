@@ -847,9 +847,9 @@ constexpr uint32_t kExpertsFewMinRows = 2; // one row: a wave per hidden unit re
 uzu_status moe_experts_gate_up(hipStream_t s, const float* x, const int32_t* ids, const uint16_t* w13, float* hidden, uint32_t rows, uint32_t d, uint32_t ff, uint32_t routed,
                                uint32_t top, uint32_t bf16_products, const ExpertAct& act, const float* in_weights) {
     if (!rows || !routed) return UZU_OK;
+    UZU_UNSUPPORTED((size_t)d * 4 > 48 * 1024, "moe_experts_gate_up: model_dim %u does not fit the workgroup's LDS row", d);
     if (bf16_products && rows >= kExpertsFewMinRows && experts_few_supported(x, hidden, w13, w13, rows, d, ff, routed, top, act))
         return experts_few_gate_up(s, x, ids, w13, hidden, rows, d, ff, routed, top, act, in_weights);
-    UZU_UNSUPPORTED((size_t)d * 4 > 48 * 1024, "moe_experts_gate_up: model_dim %u does not fit the workgroup's LDS row", d);
     // few (row, slot) pairs (decode): the hidden units of a pair are spread over more workgroups, so that the expert's rows stream through many CUs
     const uint32_t want = (1024 + rows * top - 1) / (rows * top), most = (ff + 3) / 4;
     const uint32_t gy = want < 1 ? 1 : (want > most ? most : want);
