@@ -24,8 +24,7 @@ using namespace uzu::eng;
 namespace {
 // the control block behind an accepted path: the tokens at their positions, the next input token, the context length
 struct AcceptedTokens {
-    static constexpr uint32_t kMost = 256;
-    uint32_t token[kMost];
+    uint32_t token[k::kDnTreeMaxNodes]; // (no path is longer than the largest tree)
 };
 __global__ void __launch_bounds__(64) accept_commit_kernel(uint32_t* ctx_len, uint32_t* next, uint32_t* out_token, uint32_t* sampled, AcceptedTokens t, uint32_t count, uint32_t new_len) {
     for (uint32_t i = threadIdx.x; i < count; i += 64) sampled[i] = t.token[i];
@@ -500,17 +499,10 @@ uzu_status uzu_hip_model_accept(uzu_hip_model* m, const uint32_t* accepted_indic
     std::vector<uint32_t> toks(count);
     for (uint32_t i = 0; i < count; ++i) toks[i] = m->tree.sampled[accepted_indices[i]];
     const uint32_t new_len = m->context_length + count;
-    if (count <= AcceptedTokens::kMost) { // (as kernel arguments: one launch where four copies were)
-        AcceptedTokens t{};
-        std::copy(toks.begin(), toks.end(), t.token);
-        hipLaunchKernelGGL(accept_commit_kernel, dim3(1), dim3(64), 0, s, m->d_ctx_len, m->d_tokens, m->d_out_token, m->d_sampled + m->context_length, t, count, new_len);
-        HIPCHK(hipGetLastError());
-    } else {
-        HIPCHK(hipMemcpyAsync(m->d_sampled + m->context_length, toks.data(), (size_t)count * 4, hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemcpyAsync(m->d_tokens, &toks[count - 1], 4, hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemcpyAsync(m->d_out_token, &toks[count - 1], 4, hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemcpyAsync(m->d_ctx_len, &new_len, 4, hipMemcpyHostToDevice, s));
-    }
+    AcceptedTokens t{}; // (as kernel arguments: one launch where four copies were)
+    std::copy(toks.begin(), toks.end(), t.token);
+    hipLaunchKernelGGL(accept_commit_kernel, dim3(1), dim3(64), 0, s, m->d_ctx_len, m->d_tokens, m->d_out_token, m->d_sampled + m->context_length, t, count, new_len);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s));
     m->context_length = new_len;
     m->hidden_ready = false;

@@ -124,7 +124,7 @@ void linear(Enc& e, const DLinear& L, const uint16_t* input, uint16_t* output, u
     const char* variant = "matmul";
     e.begin();
     const uzu_status r = k::matmul(e.s, p, e.m->ctx->num_cus, &variant);
-    e.run(r, post && post->done ? "gemm_q_mfma128+norm" : variant, k::matmul_algorithmic_bytes(p));
+    e.run(r, post && post->done ? (strcmp(variant, "gemm_rows") ? "gemm_q_mfma128+norm" : "gemm_rows+norm") : variant, k::matmul_algorithmic_bytes(p));
     if (exchange) {
         const size_t count = (size_t)batch * L.n;
         RUN("all_reduce", count * 4, tp::all_reduce_sum_f32(e.m->tp, e.s, e.m->tp_buf, count, output)); // sums rounded to bf16 into `output`
