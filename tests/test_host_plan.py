@@ -131,6 +131,19 @@ def test_prefill_gemm_plan_follows_the_measured_ab(monkeypatch):
     assert gemm_plan(4096, 4096, 4096).form == 2
 
 
+def test_prefill_gemm_plan_leaves_small_products_to_the_register_fed_kernel(monkeypatch):
+    """csrc/k_gemm_rows.hip::gemm_rows_preferred from 128 rows on, both sides of each of its lines: 4.5 GFLOP, large tiles on three CUs of four whatever the work, and for long K how often
+    its workgroups go round against how far the large tiles can cut K."""
+    monkeypatch.delenv("UZU_HIP_TUNE", raising=False)
+    for m, n, k in ((517, 1024, 3584), (256, 8224, 1024), (600, 4096, 512), (256, 8192, 256), (128, 4096, 8192), (512, 2048, 11008), (256, 4096, 9728), (128, 4096, 14336), (256, 2048, 16384),
+                    (288, 3072, 8192)):
+        assert gemm_plan(m, n, k).large_tile == 0, (m, n, k)
+    for m, n, k in ((517, 8224, 1024), (1500, 2048, 1024), (800, 4096, 512), (300, 8192, 256), (160, 4096, 8192), (576, 1024, 8192), (192, 3072, 8192), (288, 4096, 9728), (256, 4096, 14336),
+                    (288, 2048, 16384)):
+        assert gemm_plan(m, n, k).large_tile == 1, (m, n, k)
+    assert gemm_plan(256, 8192, 256, gated=True).large_tile == 0 and gemm_plan(800, 4096, 512, gated=True).large_tile == 1
+
+
 def test_prefill_gemm_plan_bad_arguments():
     lib = _ffi.lib()
     lib.uzu_hip_prefill_gemm_plan.argtypes = [C.c_uint32] * 7 + [C.POINTER(GemmPlan)]

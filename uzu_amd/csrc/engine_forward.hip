@@ -156,7 +156,7 @@ bool linear_gated(Enc& e, const DLinear& L, const uint16_t* input, uint16_t* gat
     p.act_mul = 1, p.act_type = act_type;
     offset_tables(e.m, L, input, batch, &p);
     // the down projection's row sums from this epilogue (64 gated columns per workgroup): no pre-pass launch in front of it
-    const bool file = consumer && gated_out == e.m->gated && consumer->k == L.n / 2 && !k::gemm_rows_preferred(p) && k::gemm_q_mfma128_supported(p, e.m->ctx->num_cus) && rowsum_wanted(e.m, *consumer, batch, 64, e.m->rs_gated);
+    const bool file = consumer && gated_out == e.m->gated && consumer->k == L.n / 2 && !k::gemm_rows_preferred(p, e.m->ctx->num_cus) && k::gemm_q_mfma128_supported(p, e.m->ctx->num_cus) && rowsum_wanted(e.m, *consumer, batch, 64, e.m->rs_gated);
     if (file) p.gated_rowsum_out = e.m->rs_gated.buf;
     const char* variant = "matmul";
     e.begin();

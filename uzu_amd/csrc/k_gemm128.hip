@@ -845,7 +845,7 @@ __global__ void __launch_bounds__(256) gemm_split_reduce_kernel(MatmulParams p, 
 // ---------------------------------------------------------------------------------------------- host side
 bool gemm_q_mfma128_supported(const MatmulParams& p, int num_cus);
 unsigned long long* g_gemm128_dbg = nullptr; // tools/kbench KB_GEMM_DBG: per-workgroup phase timestamps (100 MHz wall clock)
-static uint32_t gemm128_splits(const MatmulParams& p, int num_cus) {
+uint32_t gemm128_splits(const MatmulParams& p, int num_cus) {
     const char* e = tune_env("gemm_splits"); // read per call: tests/test_gpu_kernels.py pins it to cover both paths
     const int force = e ? atoi(e) : 0;
     const uint32_t G = p.k / p.group_size, gs = p.group_size / BK;
@@ -874,7 +874,7 @@ static int gemm128_form(const MatmulParams& p, int num_cus, uint32_t splits) {
 }
 // host arithmetic only (uzu_hip_prefill_gemm_plan): which kernel / form / split-K a shape gets; UZU_GEMM_FORM / UZU_GEMM_SPLITS apply as at launch
 void gemm_q_mfma128_plan_query(const MatmulParams& p, int num_cus, uint32_t* large_tile, uint32_t* form, uint32_t* splits, uint32_t* workgroups) {
-    *large_tile = gemm_q_mfma128_supported(p, num_cus) && !gemm_rows_preferred(p) ? 1u : 0u;
+    *large_tile = gemm_q_mfma128_supported(p, num_cus) && !gemm_rows_preferred(p, num_cus) ? 1u : 0u;
     *form = *splits = *workgroups = 0;
     if (!*large_tile) return;
     *splits = gemm128_splits(p, num_cus);

@@ -17,7 +17,7 @@
 //     Normalization): the cuts are chosen so that the chip has a workgroup per CU and a wave's chain is a few steps.
 // What bounds it: below ~100 rows the launch and two or three dependent loads; above, the L2 traffic of unshared operands (~7 TB/s at 0.3 PFLOP/s).
 // Measured, us per launch, 64 x 64 tiles -> here (weights not in cache): 1024 x 3584, M = 37: 38.0 -> 8.5; 1024 x 2048: 23.7 -> 6.9; 7168 x 1024 + GatedActMul:
-// 14.3 + 4.7 -> 8.1; 8224 x 1024: 14.5 -> 10.1; 4096 x 14336: 163 -> 29; a 37-token prompt of Qwen3.5-0.8B 3.97 -> 2.02 ms.
+// 14.3 + 4.7 -> 8.1; 8224 x 1024: 14.5 -> 10.3; 4096 x 14336: 163 -> 33; a 37-token prompt of Qwen3.5-0.8B 3.84 -> 2.22 ms.
 #include "decode_epilogue.h"
 #include "device_utils.h"
 #include "gemm_convert.h"
@@ -68,7 +68,7 @@ __global__ void __launch_bounds__(256, 2) gemm_rows_kernel(GemmRowsParams p) {
     const uint32_t r = lane & 15, g = lane >> 4, kw = wave % KW, grp_w = wave / KW;
     const uint32_t out_n = ACT ? p.n / 2 : p.n, half_k = p.k / 2, G = p.k / 128, pairs = G / 2;
     const uint32_t row0 = (blockIdx.x * GROUPS + grp_w) * (16 * OB), t0 = blockIdx.y * (16 * MT);
-    // this wave's steps, a whole number of pairs (the host keeps KW * splits <= pairs)
+    // this wave's steps, a whole number of pairs (none where there are more waves than pairs: such a wave adds zeros)
     const uint32_t part = blockIdx.z * KW + kw, parts = p.splits * KW;
     const uint32_t s_lo = 2 * (pairs * part / parts), s_hi = 2 * (pairs * (part + 1) / parts);
     // rows and tokens past the end are read from inside the matrices; their sums are never stored
@@ -267,15 +267,25 @@ bool gemm_rows_supported(const MatmulParams& p) {
 // Where this kernel is the faster one.  Below 128 rows the other choice is the 64 x 64 tile (k_gemm.hip), which pays ~0.6 us per 64 k whatever M is and gains from
 // M only when its tiles fill the chip (28672 x 4096: 59 us at M = 37 .. 64 with GatedActMul as a launch of its own behind it, this kernel 58 .. 66 with it); from 128 rows on it is the 128 x 128 tile (k_gemm128.hip), which
 // reads an operand byte ~4 times as often from LDS instead of the L2 and is ahead as soon as there is work for its tiles: at 8224 x 1024 33 us against 33 at M = 256,
-// 41 against 44 at M = 517; at 1024 x 3584 36 us against 23 at M = 517; at 4096 x 14336 75 us against 53 at M = 128, 79 against 101 at M = 256.
-bool gemm_rows_preferred(const MatmulParams& p) {
+// 41 against 44 at M = 517; at 1024 x 3584 36 us against 23 at M = 517, and where a short K leaves little to share, from a tile on three CUs of four on: 4096 x 512 27 us
+// against 19 at M = 600 (160 tiles), 14.8 against 19.3 at M = 800 (224); 8192 x 256 11.0 against 8.0 at M = 256 (128), 11.7 against 12.4 at M = 300 (192).
+// From K = 8192 on a workgroup a CU here walks K in 4 us per 1024 and as often as the tiles go round; the large tiles take 12 us and 14 us per 1024 of their share of K, where the
+// number of quant groups lets it be cut: 4096 x 8192 46 us against 33 at M = 128 (one round), 48 against 62 at M = 160 (two); 2048 x 11008, which cannot be cut, 150 against
+// 41 at M = 256, 150 against 74 at M = 512, 4096 x 9728 (two shares) 82 against 62 at M = 256, 85 against 117 at M = 288; 4096 x 14336 74 against 53 at M = 128, 77 against 101 at
+// M = 256; 2048 x 16384 77 against 60 at M = 256, 81 against 118 at M = 288.
+bool gemm_rows_preferred(const MatmulParams& p, int num_cus) {
     if (!gemm_rows_supported(p) || (p.m >= 128 && (tune_env("gemm_form") || tune_env("gemm_splits")))) return false; // (a pinned form or split-K is the large tile's)
     const double gflops = 2e-9 * p.m * p.n * p.k;
     // up to 16 rows: the few-rows kernel (k_gemv_rows.hip) is a workgroup per 16 outputs, 1024 x 3584 in 5.6 us against 6.8 here at 5 rows, but takes 248320 x 1024 in
     // 67 .. 125 us (2 .. 16 rows) against 46 .. 53, 4096 x 14336 in 25 .. 28 against 16 .. 20, 28672 x 4096 in 28 .. 44 against 28 .. 30, 8224 x 1024 in 7.2 against 6.0 (13 rows)
     if (p.m <= 16) return (uint64_t)p.n * p.k >= (32u << 20) || (p.m > 8 && p.n >= 8192);
-    if (p.k >= 8192) return p.m < 128 || gflops <= 16.0;
-    return gflops <= (p.m >= 128 ? 4.5 : p.act_mul ? 16.0 : 9.0);
+    if (p.m < 128) return p.k >= 8192 || gflops <= (p.act_mul ? 16.0 : 9.0);
+    const uint32_t cus = (uint32_t)num_cus, large_tiles = ((p.m + 127) / 128) * ((p.n + 127) / 128);
+    if (p.k < 8192) return gflops <= 4.5 && large_tiles < cus * 3 / 4;
+    const uint32_t splits = gemm128_splits(p, num_cus), rounds = (((p.n + 63) / 64) * ((p.m + 31) / 32) + cus - 1) / cus;
+    if (!splits) return true;
+    const uint32_t large_rounds = (large_tiles * splits + cus - 1) / cus;
+    return 4ull * p.k * rounds <= 12 * 1024 + 14ull * (p.k / splits) * large_rounds;
 }
 
 uzu_status gemm_rows(hipStream_t s, const MatmulParams& p, int num_cus) {

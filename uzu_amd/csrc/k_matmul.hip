@@ -359,7 +359,7 @@ uzu_status matmul(hipStream_t s, const MatmulParams& p, int num_cus, const char*
         if (variant) *variant = p.bits == 4 ? "gemv_dec<4>" : "gemv_dec<8>";
         return gemv_dec(s, q, num_cus, nullptr);
     }
-    if (gemm_rows_preferred(p)) { // dozens of rows, wide matrices of fewer (k_gemm_rows.hip)
+    if (gemm_rows_preferred(p, num_cus)) { // dozens of rows, wide matrices of fewer (k_gemm_rows.hip)
         if (variant) *variant = "gemm_rows";
         return gemm_rows(s, p, num_cus);
     }
@@ -384,7 +384,7 @@ bool matmul_act_mul_supported(hipStream_t s, const MatmulParams& p, int num_cus)
     q.act_mul = 1;
     if (exact_mode() || q.b_kind == UZU_MATMUL_B_FULL_PRECISION || (uintptr_t)q.b % 16 || (uintptr_t)q.a % 16) return false;
     if (gemv_rows_mfma_supported(q)) return true; // a handful of rows: the few-rows kernel carries the epilogue too (no workspace: fine under capture)
-    if (gemm_rows_preferred(q)) return true; // (no workspace either)
+    if (gemm_rows_preferred(q, num_cus)) return true; // (no workspace either)
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false; // no workspace during capture
     return gemm_q_mfma_supported(q) && gemm_q_mfma128_supported(q, num_cus);

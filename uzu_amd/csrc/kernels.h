@@ -69,8 +69,9 @@ uzu_status matmul(hipStream_t s, const MatmulParams& p, int num_cus, const char*
 // gated_act_mul separately
 bool matmul_act_mul_supported(hipStream_t s, const MatmulParams& p, int num_cus);
 // k_gemm_rows.hip: 17 to hundreds of activation rows (wide matrices: 2 and more) against int4 codes in groups of 128, register-fed
-bool gemm_rows_preferred(const MatmulParams& p);
+bool gemm_rows_preferred(const MatmulParams& p, int num_cus);
 uzu_status gemm_rows(hipStream_t s, const MatmulParams& p, int num_cus);
+uint32_t gemm128_splits(const MatmulParams& p, int num_cus); // k_gemm128.hip: the cuts of K of a product on the large tiles (0: none that it takes)
 uzu_status gemm_split_finish(hipStream_t s, const MatmulParams& p, const float* partials, uint32_t splits); // k_gemm128.hip
 // k_gemv_rows.hip: 2 <= M <= 16 activation rows against int4 codes (group % 128 == 0) as ONE pass over the weights on the matrix cores
 bool gemv_rows_mfma_supported(const MatmulParams& p);
