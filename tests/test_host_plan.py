@@ -144,6 +144,28 @@ def test_prefill_gemm_plan_leaves_small_products_to_the_register_fed_kernel(monk
     assert gemm_plan(256, 8192, 256, gated=True).large_tile == 0 and gemm_plan(800, 4096, 512, gated=True).large_tile == 1
 
 
+def test_register_fed_kernel_below_128_rows(monkeypatch):
+    """csrc/k_gemm_rows.hip::gemm_rows_preferred up to 127 rows, measured sizes on both sides of each line (CUS compute units): the few-rows kernel up to 16 rows, the 64 x 64 tile from
+    20 on.  A plan without workgroups is another kernel's."""
+    monkeypatch.delenv("UZU_HIP_TUNE", raising=False)
+    def here(m, n, k, gated=False):
+        p = gemm_plan(m, n, k, gated=gated)
+        assert p.large_tile == 0 and (p.splits > 0) == (p.workgroups > 0)
+        return p.workgroups > 0
+    for m, n, k in ((2, 151936, 1024), (2, 8192, 4096), (4, 7168, 5120), (2, 4096, 14336), (2, 5120, 17408), (8, 12288, 4096), (16, 9216, 4096), (9, 8224, 1024), (17, 28672, 4096), (19, 57344, 8192),
+                    (20, 1024, 3584), (64, 14336, 4096), (127, 7168, 5120), (127, 8192, 8192), (64, 14336, 8192), (96, 10240, 8192), (127, 8192, 28672), (96, 8224, 1024), (64, 11008, 2048)):
+        assert here(m, n, k), (m, n, k)
+    for m, n, k in ((2, 9216, 4096), (4, 12288, 4096), (8, 1024, 3584), (5, 8224, 1024), (65, 14336, 4096), (96, 14336, 8192), (48, 28672, 8192), (127, 28672, 8192), (127, 10240, 8192),
+                    (96, 11008, 2048), (64, 28672, 1024)):
+        assert not here(m, n, k), (m, n, k)
+    for m, n, k in ((2, 28672, 4096), (16, 57344, 8192), (32, 34816, 5120), (127, 7168, 1024)):
+        assert here(m, n, k, gated=True), (m, n, k)
+    for m, n, k in ((16, 34816, 5120), (8, 22016, 2048), (4, 37888, 3584), (33, 28672, 4096), (96, 22016, 2048), (127, 57344, 8192), (64, 34816, 5120)):
+        assert not here(m, n, k, gated=True), (m, n, k)
+    # the grid: 8192 x 8192 at 40 rows, 64 outputs x 32 tokens a workgroup
+    assert gemm_plan(40, 8192, 8192).workgroups == 256
+
+
 def test_prefill_gemm_plan_bad_arguments():
     lib = _ffi.lib()
     lib.uzu_hip_prefill_gemm_plan.argtypes = [C.c_uint32] * 7 + [C.POINTER(GemmPlan)]

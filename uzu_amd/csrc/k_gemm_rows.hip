@@ -18,6 +18,8 @@
 // What bounds it: below ~100 rows the launch and two or three dependent loads; above, the L2 traffic of unshared operands (~7 TB/s at 0.3 PFLOP/s).
 // Measured, us per launch, 64 x 64 tiles -> here (weights not in cache): 1024 x 3584, M = 37: 38.0 -> 8.5; 1024 x 2048: 23.7 -> 6.9; 7168 x 1024 + GatedActMul:
 // 14.3 + 4.7 -> 8.1; 8224 x 1024: 14.5 -> 10.3; 4096 x 14336: 163 -> 33; a 37-token prompt of Qwen3.5-0.8B 3.84 -> 2.22 ms.
+#include <algorithm>
+
 #include "decode_epilogue.h"
 #include "device_utils.h"
 #include "gemm_convert.h"
@@ -220,7 +222,7 @@ __global__ void __launch_bounds__(256, 2) gemm_rows_kernel(GemmRowsParams p) {
 
 struct GemmRowsPlan {
     int nb, kw;
-    uint32_t splits;
+    uint32_t splits, workgroups;
 };
 
 // The cuts: 16-row blocks per wave, waves per tile, K splits over workgroups.  A launch wants about a workgroup per CU; narrow problems take two blocks per wave,
@@ -236,6 +238,8 @@ GemmRowsPlan gemm_rows_plan(const MatmulParams& p, int num_cus) {
     q.splits = 1;
     if (!p.act_mul && (q.nb == 2 || long_k))
         while (q.splits * 2 * t <= cus && q.splits * 4 <= pairs) q.splits *= 2;
+    const uint32_t side_by_side = 4 / q.kw, ob = p.act_mul ? q.nb / 2 : q.nb;
+    q.workgroups = ((blocks + ob * side_by_side - 1) / (ob * side_by_side)) * token_tiles * q.splits;
     return q;
 }
 
@@ -264,8 +268,18 @@ bool gemm_rows_supported(const MatmulParams& p) {
 
 } // namespace
 
-// Where this kernel is the faster one.  Below 128 rows the other choice is the 64 x 64 tile (k_gemm.hip), which pays ~0.6 us per 64 k whatever M is and gains from
-// M only when its tiles fill the chip (28672 x 4096: 59 us at M = 37 .. 64 with GatedActMul as a launch of its own behind it, this kernel 58 .. 66 with it); from 128 rows on it is the 128 x 128 tile (k_gemm128.hip), which
+// Where this kernel is the faster one, from measurements of 33 matrices at 2 to 127 rows and of 24 at 128 to 2043.
+//   * Up to 16 rows the other choice is the few-rows kernel (k_gemv_rows.hip), a workgroup per 16 outputs: 1024 x 3584 in 5.6 us against 6.8 here at 5 rows, but 248320 x 1024
+//     in 67 .. 125 us (2 .. 16 rows) against 46 .. 53, 4096 x 14336 in 25 .. 28 against 16 .. 20, 28672 x 4096 in 28 .. 44 against 28 .. 30, 8224 x 1024 in 7.2 against 6.0
+//     (13 rows).  It also is the better one where a round of workgroups here leaves CUs idle: 34816 x 5120 with GatedActMul (272 workgroups) 40 .. 57 against 53 .. 64,
+//     22016 x 2048 with it (172) 12 .. 16 against 15 .. 17, 12288 x 4096 (192) 12.4 against 13.8 at 2 rows; from 8 rows on 15.6 .. 20 against 14.8 .. 15.7.
+//   * Up to 19 rows there is none but the GEMV (28672 x 4096, 17 rows: 171 us against 30).
+//   * Up to 127 rows it is the 64 x 64 tile (k_gemm.hip), with GatedActMul as a launch of its own behind it.  A tile walks 1024 k in 10.5 us while there is one a CU, in 12.3 while
+//     there are two, then in 4 + 5 a tile of a CU's share.  Here a round of workgroups walks 1024 k in 15 us / waves on a tile / splits, and a round that begins with fewer workgroups than
+//     CUs costs 0.7 of a full one (the workgroups share what the CU reads).  14336 x 4096: 45.6 us against 32.9 at 64 rows, 53 against 60 at 96; 22016 x 2048 with GatedActMul
+//     43 against 66 at 96 rows; 57344 x 8192 with it 217 against 220 at 48, 336 against 465 at 127; 8192 x 8192 86 against 60 at 127.  The faster one is taken but for 8 of 182
+//     sizes, by 16 % at the most (18944 x 3584 at 33 rows, 44.6 against 38.6).
+//   * From 128 rows on it is the 128 x 128 tile (k_gemm128.hip), which
 // reads an operand byte ~4 times as often from LDS instead of the L2 and is ahead as soon as there is work for its tiles: at 8224 x 1024 33 us against 33 at M = 256,
 // 41 against 44 at M = 517; at 1024 x 3584 36 us against 23 at M = 517, and where a short K leaves little to share, from a tile on three CUs of four on: 4096 x 512 27 us
 // against 19 at M = 600 (160 tiles), 14.8 against 19.3 at M = 800 (224); 8192 x 256 11.0 against 8.0 at M = 256 (128), 11.7 against 12.4 at M = 300 (192).
@@ -275,17 +289,32 @@ bool gemm_rows_supported(const MatmulParams& p) {
 // M = 256; 2048 x 16384 77 against 60 at M = 256, 81 against 118 at M = 288.
 bool gemm_rows_preferred(const MatmulParams& p, int num_cus) {
     if (!gemm_rows_supported(p) || (p.m >= 128 && (tune_env("gemm_form") || tune_env("gemm_splits")))) return false; // (a pinned form or split-K is the large tile's)
-    const double gflops = 2e-9 * p.m * p.n * p.k;
-    // up to 16 rows: the few-rows kernel (k_gemv_rows.hip) is a workgroup per 16 outputs, 1024 x 3584 in 5.6 us against 6.8 here at 5 rows, but takes 248320 x 1024 in
-    // 67 .. 125 us (2 .. 16 rows) against 46 .. 53, 4096 x 14336 in 25 .. 28 against 16 .. 20, 28672 x 4096 in 28 .. 44 against 28 .. 30, 8224 x 1024 in 7.2 against 6.0 (13 rows)
-    if (p.m <= 16) return (uint64_t)p.n * p.k >= (32u << 20) || (p.m > 8 && p.n >= 8192);
-    if (p.m < 128) return p.k >= 8192 || gflops <= (p.act_mul ? 16.0 : 9.0);
-    const uint32_t cus = (uint32_t)num_cus, large_tiles = ((p.m + 127) / 128) * ((p.n + 127) / 128);
-    if (p.k < 8192) return gflops <= 4.5 && large_tiles < cus * 3 / 4;
+    const uint32_t cus = (uint32_t)num_cus;
+    if (p.m < 128) {
+        const GemmRowsPlan plan = gemm_rows_plan(p, num_cus);
+        const uint32_t full = plan.workgroups / cus, rest = plan.workgroups % cus, filled = rest ? full + 1 : full;
+        if (p.m <= 16) {
+            if ((uint64_t)p.n * p.k < (32u << 20)) return p.m > 8 && p.n >= 8192;
+            return p.k >= 8192 || (p.m > 4 && !p.act_mul) || 4 * plan.workgroups > 3 * filled * cus;
+        }
+        if (p.m < 20) return true;
+        const double k1024 = p.k / 1024.0, tiles_per_cu = (double)((p.m + 63) / 64) * ((p.n + 63) / 64) / cus;
+        const double here = k1024 * 15.0 / (plan.kw * plan.splits) * (plan.nb / 4.0) * (!rest ? full : full ? full + 0.7 : 1.0);
+        const double tile = k1024 * (tiles_per_cu <= 1.0 ? 10.5 : std::max(12.3, 4.0 + 5.0 * tiles_per_cu)) + (p.act_mul ? 2.0 + 1.5e-6 * p.m * p.n : 0.0);
+        return here <= tile;
+    }
+    const uint32_t large_tiles = ((p.m + 127) / 128) * ((p.n + 127) / 128);
+    if (p.k < 8192) return 2e-9 * p.m * p.n * p.k <= 4.5 && large_tiles < cus * 3 / 4;
     const uint32_t splits = gemm128_splits(p, num_cus), rounds = (((p.n + 63) / 64) * ((p.m + 31) / 32) + cus - 1) / cus;
     if (!splits) return true;
     const uint32_t large_rounds = (large_tiles * splits + cus - 1) / cus;
     return 4ull * p.k * rounds <= 12 * 1024 + 14ull * (p.k / splits) * large_rounds;
+}
+
+// host arithmetic only: the cuts of K over workgroups and the grid
+void gemm_rows_plan_query(const MatmulParams& p, int num_cus, uint32_t* splits, uint32_t* workgroups) {
+    const GemmRowsPlan plan = gemm_rows_plan(p, num_cus);
+    *splits = plan.splits, *workgroups = plan.workgroups;
 }
 
 uzu_status gemm_rows(hipStream_t s, const MatmulParams& p, int num_cus) {

@@ -71,6 +71,7 @@ bool matmul_act_mul_supported(hipStream_t s, const MatmulParams& p, int num_cus)
 // k_gemm_rows.hip: 17 to hundreds of activation rows (wide matrices: 2 and more) against int4 codes in groups of 128, register-fed
 bool gemm_rows_preferred(const MatmulParams& p, int num_cus);
 uzu_status gemm_rows(hipStream_t s, const MatmulParams& p, int num_cus);
+void gemm_rows_plan_query(const MatmulParams& p, int num_cus, uint32_t* splits, uint32_t* workgroups);
 uint32_t gemm128_splits(const MatmulParams& p, int num_cus); // k_gemm128.hip: the cuts of K of a product on the large tiles (0: none that it takes)
 uzu_status gemm_split_finish(hipStream_t s, const MatmulParams& p, const float* partials, uint32_t splits); // k_gemm128.hip
 // k_gemv_rows.hip: 2 <= M <= 16 activation rows against int4 codes (group % 128 == 0) as ONE pass over the weights on the matrix cores
