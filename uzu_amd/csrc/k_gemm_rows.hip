@@ -268,7 +268,7 @@ bool gemm_rows_supported(const MatmulParams& p) {
 
 } // namespace
 
-// Where this kernel is the faster one, from measurements of 33 matrices at 2 to 127 rows and of 24 at 128 to 2043.
+// Where this kernel is the faster one, from measurements of 23 matrices at 2 to 16 rows, of 33 at 20 to 127 and of 24 at 128 to 2043.
 //   * Up to 16 rows the other choice is the few-rows kernel (k_gemv_rows.hip), a workgroup per 16 outputs: 1024 x 3584 in 5.6 us against 6.8 here at 5 rows, but 248320 x 1024
 //     in 67 .. 125 us (2 .. 16 rows) against 46 .. 53, 4096 x 14336 in 25 .. 28 against 16 .. 20, 28672 x 4096 in 28 .. 44 against 28 .. 30, 8224 x 1024 in 7.2 against 6.0
 //     (13 rows).  It also is the better one where a round of workgroups here leaves CUs idle: 34816 x 5120 with GatedActMul (272 workgroups) 40 .. 57 against 53 .. 64,
@@ -277,8 +277,8 @@ bool gemm_rows_supported(const MatmulParams& p) {
 //   * Up to 127 rows it is the 64 x 64 tile (k_gemm.hip), with GatedActMul as a launch of its own behind it.  A tile walks 1024 k in 10.5 us while there is one a CU, in 12.3 while
 //     there are two, then in 4 + 5 a tile of a CU's share.  Here a round of workgroups walks 1024 k in 15 us / waves on a tile / splits, and a round that begins with fewer workgroups than
 //     CUs costs 0.7 of a full one (the workgroups share what the CU reads).  14336 x 4096: 45.6 us against 32.9 at 64 rows, 53 against 60 at 96; 22016 x 2048 with GatedActMul
-//     43 against 66 at 96 rows; 57344 x 8192 with it 217 against 220 at 48, 336 against 465 at 127; 8192 x 8192 86 against 60 at 127.  The faster one is taken but for 8 of 182
-//     sizes, by 16 % at the most (18944 x 3584 at 33 rows, 44.6 against 38.6).
+//     43 against 66 at 96 rows; 57344 x 8192 with it 217 against 220 at 48, 336 against 465 at 127; 8192 x 8192 86 against 60 at 127.  The slower one is
+//     taken at 5 of 264 sizes by more than 3 %, the worst 16 % (18944 x 3584 at 33 rows, 44.6 against 38.6).
 //   * From 128 rows on it is the 128 x 128 tile (k_gemm128.hip), which
 // reads an operand byte ~4 times as often from LDS instead of the L2 and is ahead as soon as there is work for its tiles: at 8224 x 1024 33 us against 33 at M = 256,
 // 41 against 44 at M = 517; at 1024 x 3584 36 us against 23 at M = 517, and where a short K leaves little to share, from a tile on three CUs of four on: 4096 x 512 27 us
