@@ -172,6 +172,35 @@ def test_attention_tiles_of_more_sequences_than_a_wave_has_lanes(hip_ctx, tmp_pa
     m.close()
 
 
+def test_sequences_stepped_together_and_alone(hip_ctx, tmp_path):
+    """Eight sequences a step against each of them alone, bf16 products, contractions of 1024 and more: linears, experts and the attention's key split are chosen by a pass's rows, so
+    f32 sums are added in another order.  A sum moves by ~2e-7 of its norm, one operand in ~20 000 of the next product then rounds the other way, and what that moves makes more of
+    them round the other way behind it.  In the end the two can be no further apart than two products whose operands are rounded independently: 1.2e-3 of a product's norm (bf16:
+    2^-9 / sqrt(3) or so of an element, twice), over ten products one behind the other 4e-3, twice that through scores of gain 2: below 1e-2 (measured 2.3e-3).  The same eight in
+    another order are the same bits."""
+    layer = O.parallel_layer(O.left_half(8, 2, 128, 128, 200), O.right_half(16, 64, 128, groups=2, norm_groups=2, conv=4), 0.7, 1.2, mlp=None)
+    cfg = O.config(vocab=512, width=1024, layers=[layer, O.gla_layer(8, 128, 128, tau=8.0, rank=16, mlp=O.moe(8, 2, 1024))])
+    O.write_model_dir(str(tmp_path / "m"), cfg, O.weights(cfg, 3))
+    m = HipModel(hip_ctx, loader.load_model_dir(str(tmp_path / "m"), max_context_length=512), MODEL_BATCH(8))
+    first, alone, together, turned = [], [], [], []
+    for i in range(8):
+        first.append(m.new_state()), alone.append(m.new_state()), together.append(m.new_state()), turned.append(m.new_state())
+        m.step_batch([first[i]], [prompt(cfg, 20 + 37 * i, i)], None)
+        for st in (alone[i], together[i], turned[i]):
+            st.copy_from(first[i])
+    order = [5, 2, 7, 0, 3, 6, 1, 4]
+    for step in range(4):
+        toks = [(11 * i + 3 * step) % cfg["vocab"] for i in range(8)]
+        want = np.concatenate([m.step_batch([st], [[t]], [[0]])[0] for st, t in zip(alone, toks)])
+        got, _ = m.step_batch(together, [[t] for t in toks], [[0]] * 8)
+        again, _ = m.step_batch([turned[i] for i in order], [[toks[i]] for i in order], [[0]] * 8)
+        assert np.array_equal(again, got[order]), step
+        assert O.logit_error(got, want).max() < 1e-2, (step, O.logit_error(got, want))
+    for st in first + alone + together + turned:
+        st.close()
+    m.close()
+
+
 def test_copied_state_of_many_allocations(hip_ctx, tmp_path):
     """A state of more allocations than one copy launch takes (small windows, large caches): the copy continues exactly as its source, which the copy's steps leave alone."""
     layer = O.parallel_layer(O.left_half(**LEFT), O.right_half(**RIGHT), 0.7, 1.2)

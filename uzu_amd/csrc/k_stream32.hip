@@ -2,7 +2,8 @@
 //
 // Everything here keeps f32 where such a design asks for it: the residual rows, the norm, the router and its softmax, every accumulation.  A matrix product
 // reads f32 activation rows and bf16 weights; with `bf16_products` the activation operand is rounded to bf16 as it is loaded (what a bf16 activation buffer
-// would have held), otherwise the product is a true f32 product.  Reductions run in a fixed order: a result does not depend on what else is in the pass.
+// would have held), otherwise the product is a true f32 product.  Reductions run in a fixed order, and the other rows of
+// a pass do not enter a row's result; how many there are does: the forms and the cuts of a contraction are chosen by it, which moves f32 sums by rounding.
 #include "device_utils.h"
 #include "kernels.h"
 #include "kernels_stream32.h"
