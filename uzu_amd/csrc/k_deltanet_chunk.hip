@@ -415,7 +415,7 @@ __global__ void __launch_bounds__(256) dn_chunk_scan_mfma_kernel(const float* q_
             for (int s2 = 0; s2 < 8; ++s2) dw[s2] = sDw[(4 * s2 + kq) * RPP + i16]; // A operand: row = value column i16
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-const float* kc = sK + 4 * kq * KP + 32 * wave + 16 * t + i16;
+                const float* kc = sK + 4 * kq * KP + 32 * wave + 16 * t + i16;
                 f32x4_v u = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int s2 = 0; s2 < 8; ++s2) u = mfma4(dw[s2], kc[(16 * (s2 >> 2) + (s2 & 3)) * KP], u);
