@@ -24,7 +24,10 @@ struct Scratch { // device allocations of one call
         UZU_HIP_TRY(hipMalloc(&p, count * sizeof(T) + 256));
         ptrs.push_back(p);
         if (host) UZU_HIP_TRY(hipMemcpy(p, host, count * sizeof(T), hipMemcpyHostToDevice));
-        else UZU_HIP_TRY(hipMemset(p, 0xFF, count * sizeof(T))); // an output: what the kernel does not write reads as NaN
+        else { // an output: what the kernel does not write reads as NaN.  The fill is behind the null stream, which the context's stream does not wait for
+            UZU_HIP_TRY(hipMemset(p, 0xFF, count * sizeof(T)));
+            UZU_HIP_TRY(hipStreamSynchronize(nullptr));
+        }
         *out = (T*)p;
         return UZU_OK;
     }
