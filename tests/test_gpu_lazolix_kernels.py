@@ -326,7 +326,7 @@ def test_grouped_expert_form_prompt_sized(hip_ctx, rows, routed, identity, top, 
 
 
 @pytest.mark.parametrize("rows,n,k,batch,act", [(3, 4097, 64, 1, 0), (5, 15, 128, 1, 1), (8, 70, 1024, 1, 0), (16, 4100, 2048, 1, 1), (7, 48, 192, 3, 0), (15, 2048, 4096, 1, 0), (17, 33, 64, 1, 1),
-                                                (31, 1030, 1024, 1, 0), (32, 8191, 320, 1, 0), (9, 2100, 64, 2, 0), (20, 300, 4096, 1, 0), (24, 8200, 1024, 1, 1)])
+                                                (31, 1030, 1024, 1, 0), (32, 8191, 320, 1, 0), (9, 2100, 64, 2, 0), (20, 300, 4096, 1, 0), (24, 8200, 1024, 1, 1), (8, 70, 448, 1, 0), (6, 1990, 1024, 1, 0)])
 def test_linear_of_a_few_rows(hip_ctx, rows, n, k, batch, act):
     """bf16 products of 3 to 32 rows: ragged rows and outputs, one chunk of the contraction and many (fewer than waves, no multiple of them), the per-head form, bias, activation and
     residual; f32 sums of bf16 products, the bound of the other matrix-core forms"""
@@ -353,7 +353,7 @@ def test_experts_of_a_few_rows_refuse_a_row_that_fits_no_workgroup(hip_ctx):
                       C.c_uint32(ff), C.c_uint32(1), C.c_uint32(0), C.c_uint32(1), C.c_uint32(1))
 
 
-@pytest.mark.parametrize("rows,n,k", [(3, 4112, 1024), (8, 2048, 4096), (16, 520, 2048), (24, 1024, 2048), (12, 300, 1024)])
+@pytest.mark.parametrize("rows,n,k", [(3, 4112, 1024), (8, 2048, 4096), (16, 520, 2048), (24, 1024, 2048), (12, 300, 1024), (16, 520, 512), (12, 300, 256), (12, 1500, 2048)])
 def test_linear_of_a_few_rows_sums(hip_ctx, rows, n, k):
     """How far the f32 sums are from 64 bits, held to the sums a wave per column makes (64 lanes that add every 64th product one by one, then in pairs; products of bf16 numbers are
     exact): no further, with 5 % for the chance of the inputs."""

@@ -197,12 +197,22 @@ template <int NB, int MT, int U> uzu_status launch_few(hipStream_t s, const Line
 }
 } // namespace
 
-// Where it is the faster form: one or two rows of a wave per column cost no more than their weights' reading (1024 x 1024 2.9 us, 4 here; narrow outputs up to four rows: 3 rows
-// of 2048 x 4096 8.2 us, 8.4 here).  Above 16 rows the LDS-DMA form (k_linear_mfma.hip) is 12 to 16 us at any of these sizes; here 32 rows are 8.1 us of 1024 x 1024, 13.4 of
+// Where it is the faster form.  Up to 16 rows the other one is a wave per column (k_stream32.hip, linear_rows): workgroups of four columns and four rows, 0.25 us + 0.53 us per 1024 k
+// for every one a CU gets, against 1.15 us + 0.09 us a row per 1024 k here, whatever the columns.  So narrow outputs and long contractions stay there: 192 x 4096 6.0 us against 8.8 .. 12.7
+// (5 .. 16 rows), 512 x 2048 4.7 .. 5.7 against 5.6 .. 7.6, 64 x 1024 3.7 against 3.9 .. 4.9; 1024 x 1024 4.0 .. 5.9 against 4.1 .. 5.1, 2048 x 2048 7.7 .. 12.5 against 5.6 .. 7.5.  One or two
+// rows of a wave per column cost no more than their weights' reading (1024 x 1024 2.9 us, 4 here; narrow outputs up to four rows: 3 rows of 2048 x 4096 8.2 us, 8.4 here).
+// Above 16 rows the LDS-DMA form (k_linear_mfma.hip) is 12 to 16 us at any of these sizes; here 32 rows are 8.1 us of 1024 x 1024, 13.4 of
 // 2048 x 2048, 14.1 of 7712 x 2048, 24 of 8208 x 2048 and of 2048 x 4096.
+static bool few_faster(const LinearF32Params& p) {
+    const size_t columns = (size_t)p.n * p.batch;
+    if (p.rows > 16) return p.k <= 2048 && columns < 8192;
+    if (p.rows <= 2 || columns >= 4096) return p.rows > 2;
+    if (p.rows <= 4) return false;
+    const double k1024 = p.k / 1024.0, a_cu = (double)(((columns + 3) / 4 * ((p.rows + 3) / 4) + 255) / 256);
+    return 2.6 + k1024 * (1.15 + 0.088 * p.rows) <= 3.0 + 0.12 * k1024 + a_cu * (0.25 + 0.53 * k1024);
+}
 bool linear_few_supported(const LinearF32Params& p) {
-    if (p.rows <= 16 ? p.rows <= ((size_t)p.n * p.batch >= 4096 ? 2u : 4u) : p.k > 2048 || (size_t)p.n * p.batch >= 8192) return false;
-    return p.bf16_products && p.rows <= 32 && p.k % kChunk == 0 && p.k && !p.row_offsets && !p.row_map && p.ldx % 4 == 0 && p.x_batch % 4 == 0 && p.w_batch % 8 == 0 &&
+    return p.bf16_products && p.rows <= 32 && p.k % kChunk == 0 && p.k && few_faster(p) && !p.row_offsets && !p.row_map && p.ldx % 4 == 0 && p.x_batch % 4 == 0 && p.w_batch % 8 == 0 &&
            (((uintptr_t)p.x | (uintptr_t)p.w) & 15) == 0;
 }
 uzu_status linear_few(hipStream_t s, const LinearF32Params& p) {
