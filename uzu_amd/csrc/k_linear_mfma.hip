@@ -518,11 +518,17 @@ template <uint32_t PARTS> uzu_status launch_dma_plain(hipStream_t s, const Linea
 }
 
 // Shapes with whole k-steps.  The form is three short launches (operand rows, tiles, shares), 12 us at the least.  bf16 products (parts 1): the register-staged form takes
-// 9.5 us at k = 512, 15 us at k = 1024, 26 us at k = 2048 whatever the rows, until there are tiles for the whole chip (2 GFLOP).  f32 products (parts 3): the VALU tile takes
+// 9.5 us at k = 512, 15 us at k = 1024, 26 us at k = 2048 whatever the rows, until there are tiles for the whole chip (2 GFLOP).  Up to 64 rows it takes 64 columns a workgroup where this
+// form's tiles have 128, and is ahead over wide outputs of short contractions unless this form's last round of tiles, four a CU, is full: 49152 x 1024 (384 tiles) 24 us against 30 at 64 rows,
+// 65536 x 1024 (512) 34 against 38, 151936 x 1024 (1187) 90 against 101, but 131072 x 1024 (1024) 83 against 70 and 32768 x 2048 45 against 40.  f32 products (parts 3): the VALU tile takes
 // 0.1 us per k-step of one (55 us at k = 512, 217 us at k = 2048) against 14 to 22 us.
 bool dma_shape(uint32_t rows, uint32_t n, uint32_t k, uint32_t parts) {
     const double gflops = 2e-9 * rows * n * k;
     if (n < 64 || k % 64 || (uint64_t)rows * k * parts * 2 >= 1ull << 32 || (uint64_t)n * k * 2 >= 1ull << 32) return false; // (32-bit byte offsets)
+    if (parts == 1 && rows <= 64 && n >= 32768 && k < 2048) {
+        const uint32_t tiles = (n + DN - 1) / DN, last = tiles % 1024;
+        if (last && last < 920) return false;
+    }
     return rows > 16 && (parts == 1 ? (rows >= 128 && gflops >= 2.0) || k >= 1024 : k >= 256 || gflops >= 0.05);
 }
 
