@@ -369,7 +369,8 @@ def test_linear_of_a_few_rows_sums(hip_ctx, rows, n, k):
     assert np.linalg.norm(got - want) <= 1.05 * np.linalg.norm(lanes[..., 0] - want)
 
 
-@pytest.mark.parametrize("rows,routed,identity,top,ff,d", [(2, 8, 0, 2, 64, 64), (3, 70, 2, 4, 128, 192), (16, 4, 1, 3, 320, 64), (33, 2, 1, 1, 64, 1024), (63, 3, 0, 3, 192, 128), (61, 16, 3, 16, 64, 64)])
+@pytest.mark.parametrize("rows,routed,identity,top,ff,d", [(2, 8, 0, 2, 64, 64), (3, 70, 2, 4, 128, 192), (16, 4, 1, 3, 320, 64), (33, 2, 1, 1, 64, 1024), (63, 3, 0, 3, 192, 128), (61, 16, 3, 16, 64, 64),
+                                                           (2, 8, 0, 2, 1984, 2112), (3, 70, 2, 4, 640, 704), (16, 4, 1, 3, 512, 64)])
 def test_experts_of_a_few_rows(hip_ctx, rows, routed, identity, top, ff, d):
     """bf16 products of 2 to 63 rows: fewer (row, slot) pairs than experts and more, an expert with more pairs than a tile holds, every pair on one expert, identity experts; against 64 bits
     with the router's choice.  A hidden value near the middle of two bf16 numbers may round to the other: a result then moves by 2^-8 |h| |w|, a few of which may meet."""

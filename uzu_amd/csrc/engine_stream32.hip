@@ -662,7 +662,7 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
                 gp.y2 = S.moe_y2, gp.perm = S.moe_perm, gp.slot_pos = S.moe_slot_pos, gp.offsets = S.moe_offsets, gp.cursor = S.moe_cursor;
                 gp.rows = rows, gp.d = d, gp.ff = ff, gp.routed = E, gp.top = top, gp.act = act, gp.pos_weight = on_input ? S.moe_pos_w : nullptr;
                 gp.f32_products = bf ? 0 : 1;
-                if (k::moe_experts_grouped_supported(gp)) { // prefill-sized: buckets per expert through the matrix-core linear
+                if (k::moe_experts_grouped_faster(gp) && k::moe_experts_grouped_supported(gp)) { // prefill-sized: buckets per expert through the matrix-core linear
                     RUN("moe_experts_grouped", (size_t)E * (act.plain ? 2 : 3) * ff * d * 2 + (size_t)rows * top * ((act.plain ? 1 : 3) * ff + 2 * d) * 4, k::moe_experts_grouped(s, gp));
                 } else {
                     RUN("moe_experts_gate_up", (size_t)rows * top * (act.plain ? 1 : 2) * ff * d * 2, k::moe_experts_gate_up(s, mlp_in, S.moe_ids, L.moe.w13, S.hid, rows, d, ff, E, top, bf, act, on_input ? S.moe_w : nullptr));

@@ -675,6 +675,12 @@ bool moe_experts_grouped_supported(const MoeGroupedParams& p) {
     return p.rows >= 64 && p.y1 && p.hidden && linear_mfma_supported(q) && linear_mfma_supported(r);
 }
 
+// f32 products: five launches against the pairs' two, so enough pairs of enough weights, us: 2 of 8 experts 512 x 256 64 rows 40 / 35, 100 rows 43 / 50; 1024 x 1024 32 rows 71 / 88
+bool moe_experts_grouped_faster(const MoeGroupedParams& p) {
+    const double pairs = (double)p.rows * p.top;
+    return !p.f32_products || pairs * pairs * p.d * p.ff >= 3e9;
+}
+
 uzu_status moe_experts_grouped(hipStream_t s, const MoeGroupedParams& p) {
     UZU_REQUIRE(moe_experts_grouped_supported(p), "moe_experts_grouped: shape not covered");
     UZU_REQUIRE(!p.pos_weight || !p.act.plain, "moe_experts_grouped: weights on the inputs of plain experts");
@@ -844,12 +850,19 @@ uzu_status moe_route_groups(hipStream_t s, const RouteGroupsParams& p) {
     return launch_check([&] { hipLaunchKernelGGL(moe_route_groups_kernel<1>, dim3(p.rows), dim3(threads), ((staged ? (size_t)p.d : 0) + per_row) * 4, s, p, staged); }, "moe_route_groups");
 }
 
-constexpr uint32_t kExpertsFewMinRows = 2; // one row: a wave per hidden unit reads the same weights and needs no second launch (6.8 + 4.2 us at 1024)
+// Whether a pass of a few rows runs expert by expert (k_few_rows.hip) or pair by pair: the first reads a weight once for all its pairs but spends a workgroup a tile and a launch more, so
+// it takes enough pairs of enough weights.  Us, pairs apart / by expert: 2 of 8 experts 512 x 256 8 rows 7.9 / 9.8, 12 rows 9.9 / 9.8; 1024 x 1024 3 rows 13.7 / 15.1, 4 rows 16.9 / 15.3;
+// 1024 x 2816 2 rows 21.3 / 22.6, 3 rows 30.7 / 28.2; 2048 x 2048 2 rows 27.2 / 25.3; 256 x 128 16 rows 7.4 / 9.2, 24 rows
+// 11.2 / 9.4; 1 of 4 experts 2048 x 4096 2 rows 25.7 / 23.7.
+static bool experts_few_faster(uint32_t rows, uint32_t top, uint32_t d, uint32_t ff) {
+    const double pairs = (double)rows * top, weights = (double)d * ff;
+    return rows >= 2 && (pairs * pairs * weights >= 6.4e7 || weights >= 8e6);
+}
 uzu_status moe_experts_gate_up(hipStream_t s, const float* x, const int32_t* ids, const uint16_t* w13, float* hidden, uint32_t rows, uint32_t d, uint32_t ff, uint32_t routed,
                                uint32_t top, uint32_t bf16_products, const ExpertAct& act, const float* in_weights) {
     if (!rows || !routed) return UZU_OK;
     UZU_UNSUPPORTED((size_t)d * 4 > 48 * 1024, "moe_experts_gate_up: model_dim %u does not fit the workgroup's LDS row", d);
-    if (bf16_products && rows >= kExpertsFewMinRows && experts_few_supported(x, hidden, w13, w13, rows, d, ff, routed, top, act))
+    if (bf16_products && experts_few_faster(rows, top, d, ff) && experts_few_supported(x, hidden, w13, w13, rows, d, ff, routed, top, act))
         return experts_few_gate_up(s, x, ids, w13, hidden, rows, d, ff, routed, top, act, in_weights);
     // few (row, slot) pairs (decode): the hidden units of a pair are spread over more workgroups, so that the expert's rows stream through many CUs
     const uint32_t want = (1024 + rows * top - 1) / (rows * top), most = (ff + 3) / 4;
@@ -861,7 +874,7 @@ uzu_status moe_experts_gate_up(hipStream_t s, const float* x, const int32_t* ids
 uzu_status moe_experts_down_combine(hipStream_t s, const float* hidden, const float* x, const int32_t* ids, const float* weights, const uint16_t* w2, const float* residual,
                                     float* y, uint32_t rows, uint32_t d, uint32_t ff, uint32_t routed, uint32_t top, uint32_t bf16_products) {
     if (!rows) return UZU_OK;
-    if (bf16_products && rows >= kExpertsFewMinRows && experts_few_supported(x, hidden, w2, w2, rows, d, ff, routed, top, ExpertAct())) {
+    if (bf16_products && experts_few_faster(rows, top, d, ff) && experts_few_supported(x, hidden, w2, w2, rows, d, ff, routed, top, ExpertAct())) {
         if (float* y2 = (float*)stream_workspace(s, (size_t)rows * top * d * 4)) // (none while the stream is captured)
             return experts_few_down(s, hidden, x, ids, weights, w2, residual, y2, y, rows, d, ff, routed, top);
     }

@@ -212,6 +212,7 @@ struct MoeGroupedParams {
     uint32_t f32_products = 0; // true f32 products (y1 unused)
 };
 bool moe_experts_grouped_supported(const MoeGroupedParams& p);
+bool moe_experts_grouped_faster(const MoeGroupedParams& p); // than row by row
 uzu_status moe_experts_grouped(hipStream_t s, const MoeGroupedParams& p);
 
 // RMS norm of the latent rows (x / sqrt(mean(x^2) + eps) * scales) and append to the sequences' caches: row r goes to cache[seq(r)] + (position of r) * rank,
