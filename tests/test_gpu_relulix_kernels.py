@@ -81,6 +81,9 @@ CASES = [  # heads, kv heads, dim, vdim, window, cap, positions, start
     (4, 4, 8, 8, 5, 0.0, 40, 0), (6, 2, 16, 8, 0, 3.0, 150, 0), (3, 1, 24, 40, 33, 0.0, 100, 0), (2, 2, 64, 64, 70, 5.0, 200, 0),
     (8, 2, 32, 16, 64, 0.0, 130, 100), (4, 4, 8, 16, 1, 2.0, 20, 0), (4, 1, 16, 16, 129, 0.0, 300, 290), (2, 1, 128, 128, 200, 30.0, 260, 0),
 ]
+MANY_TILES = [  # more workgroups than CUs, twice as many, short windows: one key group, with and without the look-ahead
+    (64, 8, 64, 64, 100, 0.0, 540, 0), (64, 8, 64, 48, 0, 2.0, 1030, 3), (64, 8, 128, 120, 70, 3.0, 560, 37), (96, 32, 128, 128, 256, 0.0, 400, 0),
+]
 
 
 @pytest.mark.parametrize("H,G,dim,vd,window,cap,T,start", CASES)
@@ -93,7 +96,7 @@ def test_attention_simple_form_true_f32(hip_ctx, H, G, dim, vd, window, cap, T, 
     assert np.abs(got - want).max() < 2e-5 * np.abs(want).max()
 
 
-@pytest.mark.parametrize("H,G,dim,vd,window,cap,T,start", [c for c in CASES if c[2] % 8 == 0 and c[3] % 8 == 0])
+@pytest.mark.parametrize("H,G,dim,vd,window,cap,T,start", [c for c in CASES if c[2] % 8 == 0 and c[3] % 8 == 0] + MANY_TILES)
 def test_attention_matrix_core_form_equals_the_simple_form(hip_ctx, H, G, dim, vd, window, cap, T, start):
     rng = np.random.default_rng(H * 100 + T + 1)
     q, K, V = qkv(rng, T, H, G, dim, vd)

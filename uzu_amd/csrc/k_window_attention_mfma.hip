@@ -28,13 +28,14 @@ __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hi, uint3
 }
 
 // IW waves of a workgroup own 32 items each, KG groups of such waves share the keys of a staged stretch (32 KG keys: group i takes its 32), so a workgroup is IW KG waves and
-// their unnormalised results meet in LDS at the end, in group order.  Prompts: IW 4, KG 2; a pass's tiles are about a workgroup per CU, and a wave alone on its SIMD waits for
+// their unnormalised results meet in LDS at the end, in group order.  Prompts: IW 4, KG 2 (1 where the tiles are many: window_attention_mfma); a pass's tiles are about a workgroup per CU, and a wave alone on its SIMD waits for
 // itself at every exponential and every staged block (the next block's loads are in flight meanwhile; values are transposed two keys at a time).  2048 rows of 16 heads on 4,
 // width 128, window 1024: 147 us with four waves and no look-ahead, 61 so.  SPLIT (few items, many keys: decode steps): grid.z
 // workgroups share an item tile's stretches (stretch i goes to workgroup i mod grid.z) and leave unnormalised sums with their running maximum / denominator in p.split_ws;
 // window_attention_merge_kernel combines them.  Two forms (window_attention_split_keys): IW 4, KG 1, stretches of 32 keys, and IW 1, KG 4, stretches of 128 (with IW 4 three waves
 // of four have no items, but they help staging).  The sink belongs to group 0 of split 0.
-template <int NB, int IW, int KG, bool SPLIT> // dim and vdim padded to RP = 32 NB
+// AHEAD: the next stretch's loads are in flight while one is computed.
+template <int NB, int IW, int KG, bool SPLIT, bool AHEAD> // dim and vdim padded to RP = 32 NB
 __global__ void __launch_bounds__(64 * IW * KG) window_attention_mfma_kernel(WindowAttentionParams p) {
     constexpr int RP = 32 * NB, KP = RP * 2 + 16, TP = 80, VEC = RP / 8, T = 64 * IW * KG, KEYS = 32 * KG;
     constexpr int KN = (KEYS * VEC + T - 1) / T, VN = (KEYS / 2 * VEC + T - 1) / T; // 16-byte pieces of the keys / pairs of them of the values per thread
@@ -132,8 +133,9 @@ __global__ void __launch_bounds__(64 * IW * KG) window_attention_mfma_kernel(Win
         }
     };
     const uint32_t kstep = SPLIT ? KEYS * gridDim.z : KEYS, kfirst = kmin + (SPLIT ? KEYS * blockIdx.z : 0);
-    if (kfirst <= kmax) fetch(kfirst);
+    if (AHEAD && kfirst <= kmax) fetch(kfirst);
     for (uint32_t kb0 = kfirst; kb0 <= kmax; kb0 += kstep) {
+        if (!AHEAD) fetch(kb0);
         __syncthreads(); // the stretch before has been read
 #pragma unroll
         for (int i = 0; i < KN; ++i) {
@@ -152,7 +154,7 @@ __global__ void __launch_bounds__(64 * IW * KG) window_attention_mfma_kernel(Win
                 }
             }
         }
-        if (kb0 + kstep <= kmax) fetch(kb0 + kstep);
+        if (AHEAD && kb0 + kstep <= kmax) fetch(kb0 + kstep);
         __syncthreads();
         const uint32_t kb = kb0 + 32 * kg;
         if (!wave_on || kb > wave_hi || kb + 31 < wave_lo) continue; // (wave-uniform; the barriers above are reached by every wave)
@@ -315,11 +317,11 @@ bool window_attention_mfma_supported(const WindowAttentionParams& p) {
            (split || p.rows >= 16 * p.nseq) && p.kv_heads <= 65535 && ((uintptr_t)p.q & 15) == 0 && ((uintptr_t)p.out & 15) == 0;
 }
 
-template <int NB, int IW, int KG, bool SPLIT> static uzu_status launch(hipStream_t s, const WindowAttentionParams& p) {
+template <int NB, int IW, int KG, bool SPLIT, bool AHEAD = true> static uzu_status launch(hipStream_t s, const WindowAttentionParams& p) {
     constexpr size_t stage = (size_t)32 * KG * (32 * NB * 2 + 16) + (size_t)KG * 32 * NB * 80, meet = (size_t)(KG - 1) * IW * (16 * NB + 2) * 256, lds = stage > meet ? stage : meet;
     static LdsLimit lim;
-    UZU_REQUIRE(raise_lds_limit(lim, (const void*)window_attention_mfma_kernel<NB, IW, KG, SPLIT>, lds), "window_attention_mfma: %zu bytes of LDS are not available", lds);
-    return launch_check([&] { hipLaunchKernelGGL((window_attention_mfma_kernel<NB, IW, KG, SPLIT>), dim3(IW == 1 ? p.tiles32 : p.tiles, p.kv_heads, SPLIT ? p.splits : 1), dim3(64 * IW * KG), lds, s, p); },
+    UZU_REQUIRE(raise_lds_limit(lim, (const void*)window_attention_mfma_kernel<NB, IW, KG, SPLIT, AHEAD>, lds), "window_attention_mfma: %zu bytes of LDS are not available", lds);
+    return launch_check([&] { hipLaunchKernelGGL((window_attention_mfma_kernel<NB, IW, KG, SPLIT, AHEAD>), dim3(IW == 1 ? p.tiles32 : p.tiles, p.kv_heads, SPLIT ? p.splits : 1), dim3(64 * IW * KG), lds, s, p); },
                         SPLIT ? "window_attention_mfma_split" : "window_attention_mfma");
 }
 
@@ -332,6 +334,15 @@ uzu_status window_attention_mfma(hipStream_t s, const WindowAttentionParams& p) 
         return launch_check([&] { hipLaunchKernelGGL(window_attention_merge_kernel, dim3(p.rows * p.heads), dim3(128), 0, s, (const float*)p.split_ws, p.out, p.splits, p.vdim, 32 * nb, p.gate, p.ldgate, p.heads, p.ldo, p.out_scale); },
                             "window_attention_merge");
     }
+    // Prompts with more tiles than CUs: a second tile on the CU covers a wave's waits as the second key group does, and the groups have to meet.  Us, one group and two: heads of 64, 2048
+    // rows of 32 heads on 8 (512 tiles), window 64 / 256 / 512 / none 16.3 / 30.8 / 50.0 / 158 and 21.5 / 35.3 / 53.3 / 157; 1500 rows of 64 on 8 (752), 64 / 512 / none 21.8 / 61.1 / 124 and
+    // 30.2 / 76.2 / 146; fewer tiles, 1500 rows of 32 on 8 (376), 64 / 128 / 256 14.5 / 19.7 / 29.4 and 19.9 / 24.6 / 33.8, longer keys no better than the two groups.  Heads of 128 do not
+    // fit a second tile and its look-ahead (window 512, 512 tiles: 104 and 71.4): without the look-ahead, over short windows, 376 / 512 / 1024 tiles window 64 24.7 / 25.4 / 55.8 and 32.7 /
+    // 33.2 / 72.5, window 256 42.5 / 44.8 / 84.9 and 46.2 / 50.0 / 103.
+    const uint32_t seen = p.window && p.chunk ? std::min(p.window, p.chunk) : std::max(p.window, p.chunk);
+    const uint64_t workgroups = (uint64_t)p.tiles * p.kv_heads;
+    if (nb == 2 && (workgroups >= 512 || (workgroups > 256 && seen && seen <= 256))) return launch<2, 4, 1, false>(s, p);
+    if (nb == 4 && workgroups > 256 && seen && seen <= 256) return launch<4, 4, 1, false, false>(s, p);
     return nb == 1 ? launch<1, 4, 2, false>(s, p) : nb == 2 ? launch<2, 4, 2, false>(s, p) : launch<4, 4, 2, false>(s, p);
 }
 
