@@ -434,8 +434,9 @@ bool delta_net_conv_out_of_place_supported(const uint16_t* in_proj, const float*
 uzu_status delta_net_conv_out_of_place(hipStream_t s, const uint16_t* in_proj, const float* conv_weight, const float* bias, const float* state, uint16_t* conv_out,
                                        uint32_t suffix_len, uint32_t conv_dim, uint32_t in_stride) {
     if (!suffix_len || !conv_dim) return UZU_OK;
-    // tokens per thread: 8 (rows 11 / 8 per output from the cache instead of 19 / 16, twice the threads); 4 while the grid does not cover the chip -- a thread's chain of exact
-    // exponentials is the time then (517 rows 11.6 -> 8.6 us) -- UZU_CONV_OOP_TB (lab builds) = 16 / 8 for the A/B
+    // tokens per thread: 8 (rows 11 / 8 per output from the cache instead of 19 / 16, twice the threads); 4 up to 1024 rows -- a thread's chain of exact exponentials is the time then,
+    // whatever the channels: 64 / 512 / 1024 rows of 1024 7.8 / 8.1 / 8.3 -> 5.1 / 5.3 / 5.5 us, of 6144 8.0 / 10.2 / 13.0 -> 5.4 / 7.9 / 12.0, of 16384 8.2 / 15.7 / 23.4 -> 5.6 / 14.4 / 22.4 --
+    // UZU_CONV_OOP_TB (lab builds) = 16 / 8 for the A/B
     static const int forced = [] {
         const char* e = lab_env("UZU_CONV_OOP_TB");
         return e ? atoi(e) : 0;
