@@ -164,6 +164,8 @@ def test_register_fed_kernel_below_128_rows(monkeypatch):
         assert not here(m, n, k, gated=True), (m, n, k)
     # the grid: 8192 x 8192 at 40 rows, 64 outputs x 32 tokens a workgroup
     assert gemm_plan(40, 8192, 8192).workgroups == 256
+    # shares of K from 2048 on
+    assert [gemm_plan(33, 1024, k).splits for k in (1024, 1792, 2048, 3584)] == [1, 1, 4, 4]
 
 
 def test_prefill_gemm_plan_bad_arguments():

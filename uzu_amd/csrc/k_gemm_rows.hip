@@ -236,7 +236,9 @@ GemmRowsPlan gemm_rows_plan(const MatmulParams& p, int num_cus) {
     const uint32_t t = tiles(q.nb);
     q.kw = t <= cus + cus / 4 ? 4 : t <= 2 * cus + cus / 2 ? 2 : 1;
     q.splits = 1;
-    if (!p.act_mul && (q.nb == 2 || long_k))
+    // shares of K over workgroups from K = 2048 on (below, a share's launch of its own costs more than the steps it takes off: 1024 x 1024 5.7 us whole, 6.2 in two shares, 1024 x 1536 6.7
+    // and 7.0), at the most two pairs for a share's waves together: 1024 x 2048 6.9 in four, 8.5 in two; 1024 x 3072 7.7 and 9.1 in two; 512 x 3584 8.3 and 9.4 in two (33 rows)
+    if (!p.act_mul && (q.nb == 2 || long_k) && pairs >= 8)
         while (q.splits * 2 * t <= cus && q.splits * 4 <= pairs) q.splits *= 2;
     const uint32_t side_by_side = 4 / q.kw, ob = p.act_mul ? q.nb / 2 : q.nb;
     q.workgroups = ((blocks + ob * side_by_side - 1) / (ob * side_by_side)) * token_tiles * q.splits;
