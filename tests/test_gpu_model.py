@@ -208,7 +208,7 @@ def test_gated_act_mul_in_the_few_rows_kernel_is_bit_identical(hip_ctx, rows):
 
 @pytest.mark.parametrize("rows", [17, 40, 127, 131])
 def test_prompts_of_dozens_of_rows_against_the_oracle(hip_ctx, rows):
-    """Prompts whose linears run in the register-fed kernel (k_gemm_rows.hip; groups of 128): the fused GatedActMul epilogue and the split-K tiles finished by the next Normalization,
+    """Prompts whose linears run in the register-fed kernel (k_gemm_rows.hip; groups of 128) with the fused GatedActMul epilogue,
     against the oracle with the bound that test_layer_taps uses for whole passes: outputs of every layer within 2 % of the oracle's, in the 2-norm."""
     cfg = S.tiny_qwen(group_size=128)
     bundle = S.build_model(cfg)

@@ -23,9 +23,9 @@ pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def _leg(tmp_path, name, **env):
+def _leg(tmp_path, name, args=("--prompt", "700"), **env):
     dump = str(tmp_path / f"{name}.npy")
-    out = subprocess.run([sys.executable, os.path.join(ROOT, "tools", "ab_prefill_bits.py"), "--model", "tiny", "--prompt", "700", "--dump", dump],
+    out = subprocess.run([sys.executable, os.path.join(ROOT, "tools", "ab_prefill_bits.py"), "--model", "tiny", *args, "--dump", dump],
                          env=dict(os.environ, **env), capture_output=True, text=True, timeout=300)
     assert out.returncode == 0, out.stderr[-2000:]
     rec = json.loads(out.stdout.strip().splitlines()[-1])
@@ -53,3 +53,13 @@ def test_prefill_switches_bit_identity_and_tolerance(tmp_path):
     a, b = f32(base["logits"]).astype(np.float64), f32(chain["logits"]).astype(np.float64)
     assert np.abs(a - b).max() <= 0.05 * b.std(), (np.abs(a - b).max(), b.std())
     assert chain["first_token"] == base["first_token"]
+
+
+def test_split_products_of_dozens_of_rows_end_in_the_next_normalization(tmp_path):
+    """The same for a prompt whose down projections run in the register-fed kernel with K split (csrc/k_gemm_rows.hip; K of 2048 in groups of 128): the launch that adds the shares and
+    normalises against the two launches it replaces."""
+    args = ("--prompt", "70", "--hidden", "2048", "--group", "128")
+    base = _leg(tmp_path, "rows", args)
+    two = _leg(tmp_path, "rows_two_launches", args, UZU_HIP_TUNE="norm_partials=0")
+    assert two["logits_sha256"] == base["logits_sha256"] and two["tokens"] == base["tokens"]
+    assert two["prefill_launches"] > base["prefill_launches"], (two["prefill_launches"], base["prefill_launches"])
