@@ -270,6 +270,23 @@ def test_gemm_512_thread_forms_are_bit_identical_to_the_256_thread_form(hip_ctx,
     assert (want == got).mean() >= 0.97
 
 
+@pytest.mark.parametrize("method,n,k,m,splits", [(0, 64, 256, 128, 1), (1, 201, 512, 129, 1), (2, 130, 256, 385, 1), (0, 1160, 1024, 257, 2), (1, 385, 1536, 300, 3), (0, 257, 2048, 128, 1)])
+def test_gemm_dma_forms_are_bit_identical_to_the_register_staged_ones(hip_ctx, method, n, k, m, splits, monkeypatch):
+    """int4 in groups of 128: operands by LDS DMA (k_gemm_dma.hip), 128 and 256 columns a workgroup, against the wave-specialised form: two stages of K only, ragged rows and columns,
+    an odd column count, shares of K."""
+    rng = np.random.default_rng(n + k + m)
+    q = quant_matrix(rng, n, k, 4, 128, method)
+    a = activations(rng, m, k)
+    monkeypatch.setenv("UZU_HIP_TUNE", f"gemm_splits={splits},gemm_form=2")
+    base = hip_matmul(hip_ctx, a, q, m)
+    for form in (0, 1):
+        monkeypatch.setenv("UZU_HIP_TUNE", f"gemm_splits={splits},gemm_form={form}")
+        assert np.array_equal(base, hip_matmul(hip_ctx, a, q, m)), form
+    want = oracle_matmul(a, q, m)
+    assert ulp_diff_bf16(want, base).max() <= 1.0
+    assert (want == base).mean() >= 0.97
+
+
 @pytest.mark.parametrize("m", [131, 203, 1023])
 def test_gemm_mfma_row_count_not_a_multiple_of_four(hip_ctx, m):
     """The offset-term tables are padded to whole quads of rows (k_gemm128.hip pre-pass); 1023 is the second chunk of the

@@ -63,3 +63,14 @@ def test_split_products_of_dozens_of_rows_end_in_the_next_normalization(tmp_path
     two = _leg(tmp_path, "rows_two_launches", args, UZU_HIP_TUNE="norm_partials=0")
     assert two["logits_sha256"] == base["logits_sha256"] and two["tokens"] == base["tokens"]
     assert two["prefill_launches"] > base["prefill_launches"], (two["prefill_launches"], base["prefill_launches"])
+
+
+@pytest.mark.parametrize("dim", [1024, 2048, 4096])
+def test_rows_in_pair_order_leave_the_logits_as_they_are(tmp_path, dim):
+    """Normalizations and the gated epilogue write their rows in the order that the DMA form of the int4 products reads (csrc/k_gemm_dma.hip), a thread's 4, 8 or 16 elements at a
+    time; the wave-specialised form takes plain rows.  The MLP is wider than 4096, so both legs sum a row's groups in the same order: the same bits."""
+    args = ("--prompt", "300", "--dim", str(dim), "--hidden", "4352", "--group", "128")
+    plain = _leg(tmp_path, "plain", args, UZU_HIP_TUNE="gemm_form=2")
+    for form in ("0", "1"):
+        pairs = _leg(tmp_path, f"pairs{form}", args, UZU_HIP_TUNE=f"gemm_form={form}")
+        assert pairs["logits_sha256"] == plain["logits_sha256"] and pairs["tokens"] == plain["tokens"], form

@@ -25,6 +25,7 @@ def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--model", default="tiny")
     ap.add_argument("--prompt", type=int, default=700)
+    ap.add_argument("--dim", type=int, default=1024, help="tiny: the model's width")
     ap.add_argument("--hidden", type=int, default=1536, help="tiny: the MLP's width")
     ap.add_argument("--group", type=int, default=64, help="tiny: the quantisation group")
     ap.add_argument("--dump", default="", help="write the logits (bf16 bits, .npy) here")
@@ -33,7 +34,7 @@ def main():
     from uzu_amd.backend import Context
     from uzu_amd.engine import HipModel
     if args.model == "tiny":  # model_dim 1024: the rows kernels / split-K + normalisation launch need rows of 1024 elements
-        cfg = S.tiny_qwen(model_dim=1024, hidden_dim=args.hidden, group_size=args.group, max_context_length=args.prompt + 64, seed=34)
+        cfg = S.tiny_qwen(model_dim=args.dim, hidden_dim=args.hidden, group_size=args.group, max_context_length=args.prompt + 64, seed=34)
     else:
         cfg = S.PRESETS[args.model](max_context_length=args.prompt + 64)
     ctx = Context.new(0)

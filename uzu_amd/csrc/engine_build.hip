@@ -602,6 +602,7 @@ uzu_status uzu_hip_model_create_tp(uzu_hip_context* ctx, const uzu_model_desc* d
     ALLOC(batch_tokens, uint32_t, CB);
     ALLOC(hidden, uint16_t, CB * d);
     ALLOC(normed, uint16_t, CB * d);
+    if (k::normalization_pairs_supported(d) && CB >= 128) ALLOC(normed_pairs, uint16_t, CB * d);
     m->rowsum_floats = (size_t)(d / 32) * (CB + 4); // groups of >= 32 elements
     ALLOC(rowsum, float, m->rowsum_floats);
     {   // row sums filed by the producers of `gated` (parts of 64 columns) and `delta_out` (parts of one value head) -- sized at their allocations below

@@ -71,7 +71,10 @@ static void offset_tables(uzu_hip_model* m, const DLinear& L, const uint16_t* in
         const char* v = lab_env("UZU_GEMM_TABLES");
         return !v || atoi(v) != 0;
     }();
-    if (!enabled || batch < 128) return;
+    if (batch < 128) return;
+    if (input == m->normed && m->normed_pairs_rows == batch && L.k == m->d.model_dim) p->a_pairs = m->normed_pairs;
+    if (input == m->gated && m->gated_pairs_rows == batch) p->a_pairs = input, p->a = nullptr;
+    if (!enabled) return;
     p->pre_coef = L.coef;
     if (input == m->normed && m->rs_rows == batch && m->rs_k == L.k && m->rs_group == L.group) p->pre_rowsum = m->rowsum;
     const uzu_hip_model::FiledRowSums* f = input == m->gated ? &m->rs_gated : input == m->delta_out ? &m->rs_delta : nullptr;
@@ -82,7 +85,7 @@ static void offset_tables(uzu_hip_model* m, const DLinear& L, const uint16_t* in
 }
 // whether the producer of a prefill GEMM's activation rows should file their row sums in parts of `part` columns for `consumer` (the large-tile kernel reads them
 // instead of launching its pre-pass): same conditions as the normalisation's (norm_params), plus a part that divides the quant group a power-of-two times
-bool rowsum_wanted(const uzu_hip_model* m, const DLinear& consumer, uint32_t rows, uint32_t part, const uzu_hip_model::FiledRowSums& f) {
+bool rowsum_wanted(const uzu_hip_model* m, const DLinear& consumer, uint32_t rows, uint32_t part, const uzu_hip_model::FiledRowSums& f, bool pairs) {
     static const bool enabled = [] { // UZU_GEMM_TABLES=0 (lab builds): the GEMM's own pre-pass launch every time
         const char* v = lab_env("UZU_GEMM_TABLES");
         return !v || atoi(v) != 0;
@@ -94,11 +97,23 @@ bool rowsum_wanted(const uzu_hip_model* m, const DLinear& consumer, uint32_t row
     if (!(lab_mask & (&f == &m->rs_gated ? 1 : 2))) return false;
     // Measured (tools/rs_llama.sh, profiles/r6_rowsum_producers.txt): at K = 14336 / 4096 (Llama-3-8B) the pre-pass launch is cheaper than it looks -- it leaves the
     // rows it sums in the Infinity Cache for the GEMM behind it -- and filing the sums elsewhere LOSES 0.2-0.9 % of a pass; at K <= 3584 (the 0.8B's projections) it wins
-    if (consumer.k > 4096) return false;
+    // (rows that leave in pair order have no pre-pass to leave them to)
+    if (consumer.k > 4096 && !pairs) return false;
     if (!enabled || rows < 128 || !consumer.coef || consumer.in_signs || consumer.lora_rank || k::exact_mode() || !f.buf || !part || consumer.group % part || consumer.k % part) return false;
     const uint32_t ratio = consumer.group / part;
     if ((ratio & (ratio - 1)) || ratio > 4) return false;
     return (size_t)(consumer.k / part) * ((rows + 3) & ~3u) <= f.floats;
+}
+
+// whether linear() takes `rows` rows of this matrix to the int4 DMA product, which reads them in pair order
+static bool pairs_wanted(Enc& e, const DLinear& L, uint32_t rows) {
+    if (rows < 128 || L.in_signs || L.lora_rank || L.method == UZU_QUANT_NONE || !L.coef) return false;
+    k::MatmulParams p{};
+    p.b = L.w, p.scales = L.scales, p.biases = L.biases, p.zero_points = L.zp;
+    p.w_dt = p.a_dt = p.d_dt = UZU_BF16;
+    p.b_kind = L.method == UZU_QUANT_SCALE_BIAS ? UZU_MATMUL_B_SCALE_BIAS : L.method == UZU_QUANT_SCALE_ZERO_POINT ? UZU_MATMUL_B_SCALE_ZERO_POINT : UZU_MATMUL_B_SCALE_SYMMETRIC;
+    p.bits = L.bits, p.group_size = L.group, p.ab_scale = 1.0f, p.m = rows, p.n = L.n, p.k = L.k;
+    return k::gemm_pairs_wanted(p, e.m->ctx->num_cus) && k::stream_workspace(e.s, k::gemm_q_mfma128_workspace_bytes(p, e.m->ctx->num_cus)) != nullptr;
 }
 
 void linear(Enc& e, const DLinear& L, const uint16_t* input, uint16_t* output, uint32_t batch, bool row_parallel, PostNorm* post) {
@@ -139,6 +154,7 @@ void linear(Enc& e, const DLinear& L, const uint16_t* input, uint16_t* output, u
 // up projection + GatedActMul in one kernel (the matrix-core GEMM's epilogue pairs the up and gate columns of an output);
 // false = not available for this shape / mode: the caller runs the two kernels
 bool linear_gated(Enc& e, const DLinear& L, const uint16_t* input, uint16_t* gated_out, uint32_t batch, uint32_t act_type, const DLinear* consumer) {
+    e.m->gated_pairs_rows = 0;
     e.m->rs_gated.rows = 0; // whoever writes `gated` next, the filed sums are stale
     static const bool enabled = [] {
         const char* v = lab_env("UZU_GEMM_ACT");
@@ -156,13 +172,16 @@ bool linear_gated(Enc& e, const DLinear& L, const uint16_t* input, uint16_t* gat
     p.act_mul = 1, p.act_type = act_type;
     offset_tables(e.m, L, input, batch, &p);
     // the down projection's row sums from this epilogue (64 gated columns per workgroup): no pre-pass launch in front of it
-    const bool file = consumer && gated_out == e.m->gated && consumer->k == L.n / 2 && !k::gemm_rows_preferred(p, e.m->ctx->num_cus) && k::gemm_q_mfma128_supported(p, e.m->ctx->num_cus) && rowsum_wanted(e.m, *consumer, batch, 64, e.m->rs_gated);
+    const bool large = consumer && gated_out == e.m->gated && consumer->k == L.n / 2 && !k::gemm_rows_preferred(p, e.m->ctx->num_cus) && k::gemm_q_mfma128_supported(p, e.m->ctx->num_cus);
+    p.d_pairs = large && pairs_wanted(e, *consumer, batch) && rowsum_wanted(e.m, *consumer, batch, 64, e.m->rs_gated, true);
+    const bool file = p.d_pairs || (large && rowsum_wanted(e.m, *consumer, batch, 64, e.m->rs_gated));
     if (file) p.gated_rowsum_out = e.m->rs_gated.buf;
     const char* variant = "matmul";
     e.begin();
     const uzu_status r = k::matmul(e.s, p, e.m->ctx->num_cus, &variant);
     e.run(r, "gemm_q_mfma+act", k::matmul_algorithmic_bytes(p));
     if (file) e.m->rs_gated.rows = batch, e.m->rs_gated.k = L.n / 2, e.m->rs_gated.part = 64;
+    if (p.d_pairs) e.m->gated_pairs_rows = batch;
     return true;
 }
 
@@ -212,8 +231,9 @@ k::NormParams norm_params(Enc& e, const DNorm& N, const uint16_t* input, uint16_
     p.subtract_mean = N.subtract_mean, p.full_layer = N.full_layer;
     p.copy_to_shortcut = mode != 0, p.residual_add = mode == 2;
     uzu_hip_model* m = e.m;
+    if (consumer && output == m->normed && m->normed_pairs && consumer->k == dim && dim == m->d.model_dim && pairs_wanted(e, *consumer, rows)) p.pairs_out = m->normed_pairs;
     // (dim <= 2048: see rowsum_wanted -- at Llama-3-8B's 4096 the GEMM's own pre-pass, which warms the cache with the rows, is the faster route by 0.7-0.9 % of a pass)
-    if (consumer && consumer->coef && !consumer->in_signs && !consumer->lora_rank && output == m->normed && rows >= 128 && consumer->k == dim && dim <= 2048 && !k::exact_mode() &&
+    if (consumer && consumer->coef && !consumer->in_signs && !consumer->lora_rank && output == m->normed && rows >= 128 && consumer->k == dim && (dim <= 2048 || p.pairs_out) && !k::exact_mode() &&
         k::normalization_rowsum_supported(dim, consumer->group) && (size_t)(dim / consumer->group) * ((rows + 3) & ~3u) <= m->rowsum_floats)
         p.rowsum_out = m->rowsum, p.rowsum_group = consumer->group;
     return p;
@@ -221,7 +241,8 @@ k::NormParams norm_params(Enc& e, const DNorm& N, const uint16_t* input, uint16_
 // book-keeping of the filed row sums, at the point where the normalisation `p` is ISSUED (its parameters may have been drawn up earlier: PostNorm)
 void norm_issued(uzu_hip_model* m, const k::NormParams& p) {
     if (p.output != m->normed) return;
-    m->rs_rows = 0; // whatever was filed for the old rows is stale
+    m->rs_rows = m->normed_pairs_rows = 0; // whatever was filed for the old rows is stale
+    if (p.pairs_out) m->normed_pairs_rows = p.batch_size;
     if (p.rowsum_out) m->rs_rows = p.batch_size, m->rs_k = p.element_count, m->rs_group = p.rowsum_group;
 }
 void norm(Enc& e, const DNorm& N, const uint16_t* input, uint16_t* output, uint16_t* shortcut, int mode, uint32_t rows, uint32_t dim, const DLinear* consumer) {

@@ -224,6 +224,10 @@ struct uzu_hip_model {
     float* rowsum = nullptr;
     size_t rowsum_floats = 0;
     uint32_t rs_rows = 0, rs_k = 0, rs_group = 0;
+    // rows in the pair order of the int4 DMA products (MatmulParams::a_pairs): a copy of `normed` by its normalisation, `gated` itself by the up projection's epilogue;
+    // valid for that many rows, 0: not written
+    uint16_t* normed_pairs = nullptr;
+    uint32_t normed_pairs_rows = 0, gated_pairs_rows = 0;
     // the same for the two other buffers a prefill GEMM reads: `gated` (filed by the up projection's GatedActMul epilogue in parts of 64 columns) and `delta_out`
     // (filed by the DeltaNet norm-gate in parts of one value head): MatmulParams::pre_rowsum + rowsum_parts_log2 of the down / out projection (round 6)
     struct FiledRowSums {
@@ -390,7 +394,7 @@ struct Seqs {
 };
 void linear(Enc& e, const DLinear& L, const uint16_t* input, uint16_t* output, uint32_t batch, bool row_parallel = false, PostNorm* post = nullptr);
 bool linear_gated(Enc& e, const DLinear& L, const uint16_t* input, uint16_t* gated_out, uint32_t batch, uint32_t act_type, const DLinear* consumer = nullptr);
-bool rowsum_wanted(const uzu_hip_model* m, const DLinear& consumer, uint32_t rows, uint32_t part, const uzu_hip_model::FiledRowSums& f);
+bool rowsum_wanted(const uzu_hip_model* m, const DLinear& consumer, uint32_t rows, uint32_t part, const uzu_hip_model::FiledRowSums& f, bool pairs = false);
 k::NormParams norm_params(Enc& e, const DNorm& N, const uint16_t* input, uint16_t* output, uint16_t* shortcut, int mode, uint32_t rows, uint32_t dim, const DLinear* consumer = nullptr);
 void norm_issued(uzu_hip_model* m, const k::NormParams& p);
 void norm(Enc& e, const DNorm& N, const uint16_t* input, uint16_t* output, uint16_t* shortcut, int mode, uint32_t rows, uint32_t dim, const DLinear* consumer = nullptr);

@@ -4,6 +4,7 @@
 // rounding points exactly (compiled with -ffp-contract=off, glibc-exact expf), so they are BIT-EXACT
 // against the CPU path; kernels with a reduction (norms, argmax is exact) use fixed-order trees.
 #include "device_utils.h"
+#include "gemm_convert.h"
 #include "gemv_core.h"
 #include "kernels.h"
 #include "rht_stripe.h"
@@ -161,6 +162,8 @@ __global__ void __launch_bounds__(256) normalization_rows_kernel(NormParams p, N
     const float rms_inv = 1.0f / sqrtf(variance + p.epsilon);
     uint16_t* out = (uint16_t*)p.output;
     float gsum = 0.f;
+    [[maybe_unused]] u32x2_v before = {0u, 0u};
+    [[maybe_unused]] float ev = 0.f, od = 0.f, eight[(NV + 1) / 2];
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         float r[4];
@@ -180,14 +183,33 @@ __global__ void __launch_bounds__(256) normalization_rows_kernel(NormParams p, N
             if (biases) result = round_bf16(result + biv[4 * j + i]);
             if (p.scale_output) result = round_bf16(result * round_bf16(p.post_layer_scalar));
             r[i] = result;
-            gsum += result;
+            if constexpr (NV < 4 || NV % 2) gsum += result;
+        }
+        if constexpr (NV >= 4 && NV % 2 == 0) { // the order of the product's pre-pass, which sums rows of this width otherwise: eight elements by even and odd, then pairs of eights
+            if (j & 1) eight[j >> 1] = (ev + r[0] + r[2]) + (od + r[1] + r[3]);
+            else ev = r[0] + r[2], od = r[1] + r[3];
         }
         u32x2_v o;
         o.x = (f32_to_bits(r[0]) >> 16) | (f32_to_bits(r[1]) & 0xFFFF0000u);
         o.y = (f32_to_bits(r[2]) >> 16) | (f32_to_bits(r[3]) & 0xFFFF0000u);
         *(u32x2_v*)(out + off + e0 + 4 * j) = o;
+        if constexpr (NV == 1) { // pair order of eight elements: this thread's four and its neighbour's
+            if (p.pairs_out) {
+                const bool odd = threadIdx.x & 1;
+                const uint32_t other = __shfl_xor(odd ? o.x : o.y, 1, 64), lo = odd ? other : o.x, hi = odd ? o.y : other;
+                u32x2_v q;
+                q.x = __builtin_amdgcn_perm(hi, lo, 0x05040100u), q.y = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
+                *(u32x2_v*)(p.pairs_out + off + e0) = q;
+            }
+        } else if constexpr (NV % 2 == 0) {
+            if (j & 1) {
+                if (p.pairs_out) *(u32x4_v*)(p.pairs_out + off + e0 + 4 * (j - 1)) = permute_pairs(u32x4_v{before.x, before.y, o.x, o.y});
+            } else before = o;
+        }
     }
     if (p.rowsum_out) {
+        if constexpr (NV == 4) gsum = eight[0] + eight[1];
+        if constexpr (NV == 8) gsum = (eight[0] + eight[1]) + (eight[2] + eight[3]);
         const uint32_t lanes = p.rowsum_group / E, Mp = (p.batch_size + 3) & ~3u;
         for (uint32_t o = 1; o < lanes; o <<= 1) gsum += __shfl_xor(gsum, (int)o, 64);
         if (threadIdx.x % lanes == 0) p.rowsum_out[(size_t)(e0 / p.rowsum_group) * Mp + blockIdx.x] = gsum;
@@ -204,8 +226,15 @@ bool normalization_rowsum_supported(uint32_t n, uint32_t group) {
     return lanes >= 1 && lanes <= 64 && (lanes & (lanes - 1)) == 0;
 }
 
+bool normalization_pairs_supported(uint32_t n) { return n == 1024 || n == 2048 || n == 4096 || n == 8192; }
+
 uzu_status normalization(hipStream_t s, const NormParams& p) {
     if (p.batch_size == 0) return UZU_OK;
+    if (p.pairs_out && (exact_mode() || !normalization_pairs_supported(p.element_count) || p.io_dt != UZU_BF16 || p.batch_size < 2 || (uintptr_t)p.pairs_out % 16 ||
+                        (((uintptr_t)p.input | (uintptr_t)p.output | (uintptr_t)p.shortcut) & 7))) {
+        set_error("normalization: rows of %u elements are not available in pair order", p.element_count);
+        return UZU_ERR_UNSUPPORTED;
+    }
     if (p.rowsum_out && (exact_mode() || !normalization_rowsum_supported(p.element_count, p.rowsum_group))) {
         set_error("normalization: rowsum_out is not available for %u elements in groups of %u (or in reference-order mode)", p.element_count, p.rowsum_group);
         return UZU_ERR_UNSUPPORTED;

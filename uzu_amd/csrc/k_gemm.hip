@@ -318,6 +318,10 @@ uzu_status gemm_q_mfma(hipStream_t s, const MatmulParams& p, int num_cus) {
     if ((force != 64 || p.act_mul) && gemm_q_mfma128_supported(p, num_cus)) {
         if (void* ws = stream_workspace(s, gemm_q_mfma128_workspace_bytes(p, num_cus))) return gemm_q_mfma128(s, p, num_cus, ws);
     }
+    if (!p.a) {
+        set_error("matmul: rows in pair order and no workspace for the form that reads them");
+        return UZU_ERR_UNSUPPORTED;
+    }
     if (p.act_mul) {
         set_error("matmul: the fused GatedActMul epilogue is not available for this shape (callers ask matmul_act_mul_supported first)");
         return UZU_ERR_UNSUPPORTED;

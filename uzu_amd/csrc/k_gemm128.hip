@@ -13,6 +13,7 @@
 //     MFMAs and no per-group offset work in the main loop.
 //   * Every global load is unconditional (rows / columns / steps clamped into range) and prefetched into a register
 //     ring; the loop is unrolled by the ring depth so that all indices are static (vmcnt waits stay counted).
+//   * int4 in groups of 128 takes the first two of the three forms (gemm128_form) with its operands by LDS DMA instead: k_gemm_dma.hip.
 //   * Tiles are numbered in 8 x 8 super-tiles per XCD (tile_map) so that the ~64 workgroups an XCD runs at a time share
 //     their activation and weight panels in its L2; few-tile shapes split K over gridDim.y with f32 partial tiles and
 //     a fixed-order reduction.  bf16 results leave through LDS as 16-byte row segments.
@@ -21,6 +22,7 @@
 #include <type_traits>
 
 #include "device_utils.h"
+#include "gemm128_epilogue.h"
 #include "gemm_convert.h"
 #include "gemm_tile_map.h"
 #include "kernels.h"
@@ -59,7 +61,7 @@ constexpr bool kPairs = UZU_GEMM_PAIR_DEQUANT != 0;
 // Blocks [0, rowsum_blocks): rowsum[g][m] = sum of A[m, k in group g] (f32), row stride Mp = M rounded up to 4 (pad rows are
 // zero); the remaining blocks: coef[g][n].  Row sums: one wave per row; lane l owns the 8-element chunks l, l + 64, ...;
 // the lanes of a group (group_size / 8, a power of two <= 64) are reduced with xor shuffles in a fixed order.
-__global__ void __launch_bounds__(256) gemm_prepass_kernel(MatmulParams p, float* rowsum, float* coef, uint32_t rowsum_blocks) {
+__global__ void __launch_bounds__(256) gemm_prepass_kernel(MatmulParams p, float* rowsum, float* coef, uint16_t* pairs, uint32_t rowsum_blocks) {
     const uint32_t M = p.m, K = p.k, N = p.n, group_size = p.group_size, G = K / group_size;
     if (blockIdx.x >= rowsum_blocks) {
         // coef[g][n] (f32, the layout the epilogue's f32 MFMA operand wants: lanes = consecutive columns):
@@ -98,6 +100,7 @@ __global__ void __launch_bounds__(256) gemm_prepass_kernel(MatmulParams p, float
         float s = 0.f;
         if (chunk < K / 8) {
             const u32x4_v v = *(const u32x4_v*)(row + (size_t)chunk * 8);
+            if (pairs) *(u32x4_v*)(pairs + (size_t)m * K + (size_t)chunk * 8) = permute_pairs(v);
             const uint32_t w[4] = {v.x, v.y, v.z, v.w};
             float s0 = 0.f, s1 = 0.f;
 #pragma unroll
@@ -681,140 +684,8 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
     }
     ts[2] = wall_clock64();
 
-    // ---- offset term: acc_t[m, n] += sum_g rowsum[g][m] * coef[g][n] over this split's groups, on the matrix cores in
-    // f32 (v_mfma_f32_32x32x2_f32: products and sums exact to f32): lane (c, h) supplies row / column c of group 2 i + h,
-    // every load is one coalesced dword per lane.
-    if (p.b_kind != UZU_MATMUL_B_SCALE_SYMMETRIC || (kPairs && BITS == 4)) {
-        const uint32_t Mp = (M + 3) & ~3u;
-        uint32_t arow[2];
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb) arow[mb] = min(m0 + wm * 64 + mb * 32 + c, Mp - 1);
-        // (a producer may have filed 2^PL partial sums per group, rows [g << PL, (g + 1) << PL) of `rowsum`: added here in part order -- more loads in flight per
-        // iteration, the same number of iterations and MFMAs; walking the parts as extra iterations cost the long-K down projections more than the pre-pass saved)
-        const uint32_t PL = p.rowsum_parts_log2, g_end = g_lo + Gz;
-#pragma unroll 4
-        for (uint32_t g2 = g_lo; g2 < g_end; g2 += 2) {
-            const uint32_t g = min(g2 + h, g_end - 1);
-            const bool live = g2 + h < g_end;
-            float av[2], bv[2];
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb) {
-                const float* rp = rowsum + (size_t)(g << PL) * Mp + arow[mb];
-                av[mb] = rp[0];
-                if (PL >= 1) av[mb] += rp[Mp]; // (wave-uniform; PL <= 2: host-checked)
-                if (PL >= 2) av[mb] += rp[2 * (size_t)Mp], av[mb] += rp[3 * (size_t)Mp];
-            }
-#pragma unroll
-            for (int nb = 0; nb < 2; ++nb) bv[nb] = live ? coef[(size_t)g * N + ncol[nb]] : 0.f;
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb) acc_t[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[mb], bv[nb], acc_t[mb][nb], 0, 0, 0);
-        }
-    }
-
-    // ---- epilogue (kernel.rs:281-292): lane holds column n, rows (r & 3) + 8 (r >> 2) + 4 h of each block
-    uint16_t* d = (uint16_t*)p.d;
-    float* d32 = (float*)p.d;
-    const bool out_f32 = p.d_dt == UZU_F32;
-    const bool via_lds = !partials && !out_f32 && !p.accumulate && !p.has_soft_cap && (gated ? H : N) % 8 == 0 && (uintptr_t)p.d % 16 == 0; // gated: host-checked
-    if (via_lds) {
-        // Common case, branch-free: bf16(ab_scale * acc + bias) goes to a wave-private LDS tile (64 rows x 64 columns,
-        // 144-byte pitch; the activation buffers are free after the last barrier) and leaves as 16-byte row segments,
-        // 8 lanes per 128-byte row -- instead of 64 two-byte stores per lane.
-        uint16_t* s_d = (uint16_t*)s_ep + wave * (64 * 72);
-        const float ab = p.ab_scale;
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-            const float bias = p.bias ? bf16_to_f32(((const uint16_t*)p.bias)[ncol[nb]]) : 0.0f;
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                for (int r = 0; r < 16; r += 2) { // rows r and r + 1 are consecutive
-                    const uint32_t lr = mb * 32 + (r & 3) + 8 * (r >> 2) + 4 * h;
-                    const uint32_t pk = pack_bf16(__fadd_rn(__fmul_rn(ab, acc_t[mb][nb][r]), bias), __fadd_rn(__fmul_rn(ab, acc_t[mb][nb][r + 1]), bias)); // two roundings, as the reference
-                    s_d[lr * 72 + nb * 32 + c] = (uint16_t)pk;
-                    s_d[(lr + 1) * 72 + nb * 32 + c] = (uint16_t)(pk >> 16);
-                }
-        }
-        const int seg = lane & 7, rsub = lane >> 3;
-        if (gated) {
-            // the up tile (wave wm * 2) and the gate tile (wave wm * 2 + 1) hold the same (row, column) positions:
-            // out = bf16(up * act(gate)), both operands already rounded to bf16 as the separate kernels would see them; each of the
-            // pair's waves combines 32 of the 64 rows; the exp table of SiLU / softplus sits in LDS (a table read from memory per
-            // element is a dependent round trip with two waves to hide it)
-            if (tid < 32) s_exp_tab[tid] = kExp2fTab[tid];
-            __syncthreads();
-            const uint16_t* s_u = (const uint16_t*)s_ep + (wm * 2) * (64 * 72);
-            const uint16_t* s_g = s_u + 64 * 72;
-#pragma unroll
-            for (int pass = 0; pass < 4; ++pass) {
-                const uint32_t lr = wn * 32 + pass * 8 + rsub, m = m0 + wm * 64 + lr, n = n_t * 64 + seg * 8;
-                const u32x4_v uv = *(const u32x4_v*)(s_u + lr * 72 + seg * 8), gv = *(const u32x4_v*)(s_g + lr * 72 + seg * 8);
-                u32x4_v ov;
-                float part = 0.f; // the row's sum over this lane's 8 ROUNDED outputs (columns past H count as zero)
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    const float u0 = bits_to_f32(uv[w] << 16), u1 = bits_to_f32(uv[w] & 0xFFFF0000u);
-                    const float g0 = bits_to_f32(gv[w] << 16), g1 = bits_to_f32(gv[w] & 0xFFFF0000u);
-                    ov[w] = pack_bf16(u0 * activate_bf16_tab(p.act_type, g0, s_exp_tab), u1 * activate_bf16_tab(p.act_type, g1, s_exp_tab));
-                    part += bits_to_f32(ov[w] << 16);
-                    part += bits_to_f32(ov[w] & 0xFFFF0000u);
-                }
-                if (m < Mst && n < H) *(u32x4_v*)(d + (size_t)m * H + n) = ov;
-                if (p.gated_rowsum_out) { // the 8 lanes of a row segment group are neighbours: three butterfly steps, lane seg 0 files the 64-column sum
-                    if (n >= H) part = 0.f;
-                    part += __shfl_xor(part, 1);
-                    part += __shfl_xor(part, 2);
-                    part += __shfl_xor(part, 4);
-                    const uint32_t Mp = (M + 3) & ~3u;
-                    if (seg == 0 && live && m < Mp) p.gated_rowsum_out[(size_t)n_t * Mp + m] = m < M ? part : 0.f;
-                }
-            }
-        } else {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // wave-private region: no workgroup barrier needed
-#pragma unroll
-            for (int pass = 0; pass < 8; ++pass) {
-                const uint32_t lr = pass * 8 + rsub, m = m0 + wm * 64 + lr, n = n0 + wn * 64 + seg * 8;
-                const u32x4_v v = *(const u32x4_v*)(s_d + lr * 72 + seg * 8);
-                if (m < Mst && n < N) *(u32x4_v*)(d + (size_t)m * N + n) = v;
-            }
-        }
-    } else if (partials) { // split-K: raw f32 partial tile (32 lanes = one 128-byte row segment per store)
-        float* pz = partials + (size_t)z * M * N;
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-            const uint32_t n = n0 + wn * 64 + nb * 32 + c;
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const uint32_t m = m0 + wm * 64 + mb * 32 + (r & 3) + 8 * (r >> 2) + 4 * h;
-                    if (m < Mst && n < N) pz[(size_t)m * N + n] = acc_t[mb][nb][r];
-                }
-        }
-    } else {
-#pragma unroll 1
-        for (int nb = 0; nb < 2; ++nb) {
-            const uint32_t n = n0 + wn * 64 + nb * 32 + c;
-            const float bias = (p.bias && n < N) ? bf16_to_f32(((const uint16_t*)p.bias)[n]) : 0.0f;
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const uint32_t m = m0 + wm * 64 + mb * 32 + (r & 3) + 8 * (r >> 2) + 4 * h;
-                    if (m >= Mst || n >= N) continue;
-                    const size_t idx = (size_t)m * N + n;
-                    const float acc = nb ? acc_t[mb][1][r] : acc_t[mb][0][r];
-                    float value = p.ab_scale * acc;
-                    if (p.accumulate) value += out_f32 ? d32[idx] : bf16_to_f32(d[idx]);
-                    if (p.bias) value += bias;
-                    if (p.has_soft_cap) value = p.soft_cap * tanhf(value / p.soft_cap);
-                    if (out_f32) d32[idx] = value;
-                    else d[idx] = f32_to_bf16(value);
-                }
-        }
-    }
+    const GemmTile t{m0 + wm * 64, n0 + wn * 64, n_t * 64, n_t, {ncol[0], ncol[1]}, (uint32_t)wave, (uint32_t)wn, M, Mst, N, H, g_lo, g_lo + Gz, z, gated, live};
+    gemm_tile_finish<(kPairs && BITS == 4)>(p, t, rowsum, coef, partials, acc_t, s_ep, s_exp_tab);
     if (PP && !half) lds_barrier(); // the partner half's last phase barrier (it runs one phase behind)
     if (dbg && tid == 0 && live) {
         ts[3] = wall_clock64();
@@ -890,6 +761,10 @@ bool gemm_q_mfma128_supported(const MatmulParams& p, int num_cus) {
     if ((uint64_t)p.m * p.k >= (1ull << 32) || (uint64_t)p.n * p.k * p.bits / 8 >= (1ull << 32)) return false; // 32-bit element offsets
     return gemm128_splits(p, num_cus) != 0;
 }
+bool gemm_pairs_wanted(const MatmulParams& p, int num_cus) {
+    if (exact_mode() || p.m < 128 || gemm_rows_preferred(p, num_cus) || !gemm_q_mfma_supported(p) || !gemm_q_mfma128_supported(p, num_cus)) return false;
+    return gemm_q4_dma_supported(p) && gemm128_form(p, num_cus, gemm128_splits(p, num_cus)) < 2;
+}
 bool gemm_coef_table_supported(const MatmulParams& p) {
     if (p.b_kind == UZU_MATMUL_B_FULL_PRECISION || !(p.bits == 4 || p.bits == 8)) return false;
     if (p.group_size != 64 && p.group_size != 128 && p.group_size != 256) return false;
@@ -898,13 +773,14 @@ bool gemm_coef_table_supported(const MatmulParams& p) {
 }
 uzu_status gemm_coef_table(hipStream_t s, const MatmulParams& p, float* coef) {
     const uint32_t G = p.k / p.group_size;
-    return launch_check([&] { hipLaunchKernelGGL(gemm_prepass_kernel, dim3((p.n * G + 255) / 256), dim3(256), 0, s, p, (float*)nullptr, coef, 0u); }, "gemm_coef_table");
+    return launch_check([&] { hipLaunchKernelGGL(gemm_prepass_kernel, dim3((p.n * G + 255) / 256), dim3(256), 0, s, p, (float*)nullptr, coef, (uint16_t*)nullptr, 0u); }, "gemm_coef_table");
 }
 size_t gemm_q_mfma128_workspace_bytes(const MatmulParams& p, int num_cus) {
     const uint32_t G = p.k / p.group_size;
     const uint32_t splits = gemm128_splits(p, num_cus);
     size_t bytes = ((size_t)((p.m + 3) & ~3u) * G * 4 + 255) / 256 * 256 + ((size_t)p.n * G * 4 + 255) / 256 * 256;
-    if (splits > 1) bytes += (size_t)splits * p.m * p.n * 4;
+    if (splits > 1) bytes += ((size_t)splits * p.m * p.n * 4 + 255) / 256 * 256;
+    if (gemm_q4_dma_supported(p) && !p.a_pairs) bytes += (size_t)p.m * p.k * 2;
     return bytes;
 }
 uzu_status gemm_q_mfma128(hipStream_t s, const MatmulParams& p, int num_cus, void* workspace) {
@@ -915,18 +791,29 @@ uzu_status gemm_q_mfma128(hipStream_t s, const MatmulParams& p, int num_cus, voi
     float* coef = (float*)((uint8_t*)workspace + rowsum_bytes);
     float* partials = splits > 1 ? (float*)((uint8_t*)workspace + rowsum_bytes + coef_bytes) : nullptr;
     uzu_status st = UZU_OK;
+    const int form = gemm128_form(p, num_cus, splits);
+    const bool dma = form < 2 && gemm_q4_dma_supported(p);
+    if (!dma && !p.a) {
+        set_error("gemm_q_mfma128: rows in pair order, but not the form that reads them");
+        return UZU_ERR_UNSUPPORTED;
+    }
+    uint16_t* pairs = dma && !p.a_pairs ? (uint16_t*)((uint8_t*)workspace + rowsum_bytes + coef_bytes + (splits > 1 ? ((size_t)splits * p.m * p.n * 4 + 255) / 256 * 256 : 0)) : nullptr;
     if (p.b_kind != UZU_MATMUL_B_SCALE_SYMMETRIC || (kPairs && p.bits == 4)) {
         // the caller may bring either table (engine: coefficients tabulated at load, row sums written by the normalisation that produced A)
-        const uint32_t rowsum_blocks = p.pre_rowsum ? 0u : (((p.m + 3) & ~3u) + 3) / 4, coef_blocks = p.pre_coef ? 0u : (p.n * G + 255) / 256;
+        const uint32_t rowsum_blocks = p.pre_rowsum && !pairs ? 0u : (((p.m + 3) & ~3u) + 3) / 4, coef_blocks = p.pre_coef ? 0u : (p.n * G + 255) / 256;
         if (rowsum_blocks + coef_blocks) {
-            st = launch_check([&] { hipLaunchKernelGGL(gemm_prepass_kernel, dim3(rowsum_blocks + coef_blocks), dim3(256), 0, s, p, rowsum, coef, rowsum_blocks); }, "gemm_prepass");
+            st = launch_check([&] { hipLaunchKernelGGL(gemm_prepass_kernel, dim3(rowsum_blocks + coef_blocks), dim3(256), 0, s, p, rowsum, coef, pairs, rowsum_blocks); }, "gemm_prepass");
             if (st != UZU_OK) return st;
         }
     }
     const float* rowsum_in = p.pre_rowsum ? p.pre_rowsum : rowsum;
     const float* coef_in = p.pre_coef ? p.pre_coef : coef;
     const uint32_t m_tiles = (p.m + BM - 1) / BM, n_tiles = p.act_mul ? (p.n / 2 + 63) / 64 : (p.n + BN - 1) / BN;
-    const int form = gemm128_form(p, num_cus, splits);
+    if (dma) {
+        st = gemm_q4_dma(s, p, p.a_pairs ? p.a_pairs : pairs, rowsum_in, coef_in, partials, splits, form == 1);
+        if (st != UZU_OK || splits == 1) return st;
+        return gemm_split_finish(s, p, partials, splits);
+    }
     const dim3 grid(form == 1 ? gemm_grid_x(m_tiles, (n_tiles + 1) / 2) : gemm_grid_x(m_tiles, n_tiles), splits), block(form ? 512 : 256);
 #define UZU_LAUNCH(B, GSV)                                                                                                                                            \
     st = form == 2 ? launch_check([&] { hipLaunchKernelGGL((gemm_q_mfma128_kernel<B, GSV, 2>), grid, block, 0, s, p, rowsum_in, coef_in, partials, g_gemm128_dbg); }, "gemm_q_mfma128ws") \

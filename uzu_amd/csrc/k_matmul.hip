@@ -337,6 +337,10 @@ uzu_status matmul(hipStream_t s, const MatmulParams& p, int num_cus, const char*
         set_error("matmul: group size must be non-zero");
         return UZU_ERR_UNSUPPORTED;
     }
+    if (!p.a && !(quant && p.a_pairs && gemm_pairs_wanted(p, num_cus))) {
+        set_error("matmul: no activation rows in the order that this product reads");
+        return UZU_ERR_UNSUPPORTED;
+    }
     const uint32_t wpc = quant ? 32 : 1; // a lane step covers 32 K elements (gemv_core.h)
     const bool aligned = ((uintptr_t)p.b % 16 == 0) && ((uintptr_t)p.a % 16 == 0);
     const bool fast = quant && !exact_mode() && aligned && p.k % wpc == 0 && p.group_size % wpc == 0 &&

@@ -52,6 +52,10 @@ struct MatmulParams {
     // act_mul: the epilogue also files the f32 sums of the 64 gated columns it writes per row, [n / 2 / 64][Mp] (Mp = m rounded up to 4, pad rows zero) --
     // pre_rowsum (parts of 64 columns) of the GEMM that reads D next, which then needs no pre-pass launch.  The large-tile kernel only; null = not filed.
     float* gated_rowsum_out;
+    // The int4 DMA form (k_gemm_dma.hip) multiplies rows in pair order: every eight consecutive k as 0 4 1 5 2 6 3 7 (gemm_convert.h).  a_pairs: A's rows in that order, where their
+    // producer wrote them so; null: the product's pre-pass makes the copy.  a null beside it: no other form of the rows exists (only where gemm_pairs_wanted said so).
+    const uint16_t* a_pairs;
+    uint32_t d_pairs; // act_mul on the large tile: D leaves in pair order
     // The Normalization that reads D next (engine prefill: out-projection -> pre-MLP norm, down-projection -> the next layer's pre-mixer norm; its
     // `input` is D).  A split-K GEMM then finishes with ONE launch that adds the partial tiles, applies the epilogue, stores D and normalises the rows
     // (normalization_from_partials) and sets *post_norm_done; every other kernel choice ignores it and the caller runs the normalisation itself.
@@ -96,6 +100,9 @@ bool gemm_q_mfma128_supported(const MatmulParams& p, int num_cus);
 size_t gemm_q_mfma128_workspace_bytes(const MatmulParams& p, int num_cus);
 uzu_status gemm_q_mfma128(hipStream_t s, const MatmulParams& p, int num_cus, void* workspace);
 void gemm_q_mfma128_plan_query(const MatmulParams& p, int num_cus, uint32_t* large_tile, uint32_t* form, uint32_t* splits, uint32_t* workgroups);
+bool gemm_pairs_wanted(const MatmulParams& p, int num_cus);   // matmul() takes `p` to the DMA form: a producer of A may write its rows in pair order
+bool gemm_q4_dma_supported(const MatmulParams& p);           // k_gemm_dma.hip
+uzu_status gemm_q4_dma(hipStream_t s, const MatmulParams& p, const uint16_t* pairs, const float* rowsum, const float* coef, float* partials, uint32_t splits, bool wide);
 extern unsigned long long* g_gemm128_dbg; // profiling aid (tools/kbench KB_GEMM_DBG)
 size_t matmul_algorithmic_bytes(const MatmulParams& p); // codes + scales + correction + A + D, SURVEY.md §8d
 
@@ -114,7 +121,9 @@ struct NormParams {
     // rounded up to 4 (pad rows zeroed) -- MatmulParams::pre_rowsum of the GEMM that consumes the rows (see normalization_rowsum_supported)
     float* rowsum_out;
     uint32_t rowsum_group;
+    uint16_t* pairs_out; // optional: the output rows once more, in pair order (MatmulParams::a_pairs); normalization_pairs_supported
 };
+bool normalization_pairs_supported(uint32_t element_count);
 uzu_status normalization(hipStream_t s, const NormParams& p);
 bool normalization_rowsum_supported(uint32_t element_count, uint32_t group);
 // rows that are still split-K partial tiles [splits][total] f32 of the GEMM producing them (`d` = that GEMM's bf16 output, `bias` its bf16 epilogue bias or null)

@@ -190,4 +190,10 @@ UZU_HD float activate_bf16_tab(uint32_t act, float x, const uint64_t* tab) {
     default: return activate_bf16(act, x);
     }
 }
+// activate_bf16_tab(0, x) from a quotient y known to within 16 f32 ulps: only a y within 32 ulps of a bf16 tie (one in a thousand) or an |x| beyond 80 needs the exact one
+UZU_HD float silu_bf16_near(float x, float y, const uint64_t* tab) {
+    const uint32_t over = (f32_to_bits(y) + 0x8020u) & 0xFFFFu; // 0x20 at a tie
+    if (__builtin_expect(!(x > -80.0f && x < 80.0f) || over <= 0x40u, 0)) return activate_bf16_tab(0, x, tab);
+    return round_bf16(y);
+}
 } // namespace uzu
