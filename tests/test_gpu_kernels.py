@@ -1111,6 +1111,19 @@ def test_delta_net_prefill_state_precision(hip_ctx, T, pace):
     assert np.linalg.norm(got - exact) <= 1.1 * np.linalg.norm(serial - exact)
 
 
+@pytest.mark.parametrize("T,Hv,Hk,Dv", [(33, 2, 1, 144), (64, 3, 3, 272), (736, 4, 4, 128), (737, 4, 2, 128), (800, 2, 2, 128)])
+def test_delta_net_prefill_wide_values_and_the_split(hip_ctx, T, Hv, Hk, Dv):
+    """The chunk preparation's substitution over more than 128 value columns (two and three passes, the last one ragged), and both sides of the count of chunks from which the scan runs
+    as two segments (23 and 24; ends on a chunk of one token and on a whole one)."""
+    z = delta_net_inputs(np.random.default_rng(T + Dv), T, Hv, Hk, Dv, 0.1)
+    want_state, want = z["state"].copy(), np.zeros((T, Hv * Dv), np.uint16)
+    O.call("orc_delta_net_prefill", z["q"], z["k"], z["beta"], z["decay"], z["rows"], want_state, want, Hv, Hk, 128, Dv, Hk * 128, Hv * Dv, T)
+    got, state = hip_delta_net_prefill(hip_ctx, z, Hv, Hk, Dv)
+    err, ulps = np.abs(f32(got) - f32(want)), ulp_diff_bf16(want, got)
+    assert ((err <= 2e-2) | (ulps <= 1)).all() and (ulps <= 2).mean() > 0.99  # (the bounds of test_delta_net_prefill_path)
+    np.testing.assert_allclose(state, want_state, rtol=1e-4, atol=1e-4)
+
+
 @pytest.mark.parametrize("T", [17, 63, 130])
 @pytest.mark.parametrize("plant", ["value inf", "value nan", "key inf", "query nan", "beta nan", "decay nan", "decay inf", "decay above 1", "decay below 0", "decay 0", "state inf"])
 def test_delta_net_prefill_unusual_numbers(hip_ctx, T, plant):

@@ -689,7 +689,7 @@ uzu_status delta_net_prefill(hipStream_t s, const float* q_norm, const float* k_
     }
     const uint32_t rows = num_v_heads * head_v_dim;
     if (!rows || !suffix_len) return UZU_OK;
-    if (delta_net_prefill_chunked_supported(num_v_heads, num_k_heads, head_k_dim, head_v_dim, suffix_len)) {
+    if (delta_net_prefill_chunked_supported(num_v_heads, num_k_heads, head_k_dim, head_v_dim, suffix_len) && rows <= value_dim) {
         // 16 tokens and more: chunked form; scratch = the stream's workspace block (not while the stream is being captured)
         if (void* ws = stream_workspace(s, delta_net_chunk_workspace_bytes(num_v_heads, value_dim, suffix_len)))
             return delta_net_prefill_chunked(s, q_norm, k_norm, beta, decay, in_proj, state, out, (float*)ws, num_v_heads, num_k_heads, head_v_dim, key_dim,

@@ -5,17 +5,18 @@
 // is sequential in t, and with only Hv * Dv = 2048 independent rows a row-per-half-wave scan
 // (k_deltanet.hip::delta_net_prefill_kernel) runs one wave per SIMD at ~650 cycles per token: latency, not work.
 // Over a chunk of C = 32 tokens starting at S_0 the same recurrence has a closed form (A_t = prod_{i<=t} a_i):
-//     D = T (V - diag(A) K S_0^T)            T = (I + diag(b) L)^-1 diag(b),  L_ij = (A_i / A_j) k_i.k_j   (j < i)
-//     O = diag(A) Q S_0^T + P D              P_ti = (A_t / A_i) q_t.k_i                                   (i <= t)
+//     (I + M) D = diag(b) (V - diag(A) K S_0^T),   M_ij = b_i (A_i / A_j) k_i.k_j   (j < i)
+//     D = U - G S_0^T         (I + M) [U, G] = diag(b) [V, diag(A) K]
+//     O = diag(A) Q S_0^T + P D                    P_ti = (A_t / A_i) q_t.k_i       (i <= t)
 //     S_C = A_C S_0 + D^T diag(A_C / A_i) K
-// T and P do not involve the state: `dn_chunk_prep_kernel` builds them for all chunks and heads in parallel (two
-// 32 x 32 Gram matrices + one 32 x 32 forward substitution each).  `dn_chunk_scan_mfma_kernel` then walks the chunks with
-// four small dense products per chunk instead of 32 dependent steps; a workgroup owns 16 of a head's Dv columns, so
-// 128 workgroups are busy and every product has hundreds of independent FMAs per thread.
-// Same algebra, different rounding order: the state is no further from 64 bits than the recurrence's (dn_chunk_scan_mfma_kernel).  Decays are carried in log space
+// U, G and P do not involve the state: `dn_chunk_prep_kernel` makes them for all chunks and heads in parallel (two 32 x 32 Gram matrices and one forward substitution with
+// Dv + 128 right-hand sides each).  `dn_chunk_scan_kernel` then walks the chunks with two dependent products per chunk, G S^T and D^T K, and the outputs beside them.
+// Same algebra, different rounding order: the state is no further from 64 bits than the recurrence's (dn_chunk_scan_kernel).  Decays are carried in log space
 // (log 0 = -104, whose exponential is 0 in f32) so that products over a chunk cannot underflow into 0 / 0.  An infinity or a NaN would reach the whole chunk through the
-// zeros of T and P, where the recurrence hands it on from its token and its value column only: a workgroup of the plain scan that meets one walks its columns again token by token.
+// zeros of G and P, where the recurrence hands it on from its token and its value column only: a workgroup of the plain scan that meets one walks its columns again token by token.
 #include <stdlib.h>
+
+#include <type_traits>
 
 #include "device_utils.h"
 #include "internal.h"
@@ -28,20 +29,19 @@ namespace {
 constexpr int CC = 32;        // tokens per chunk
 constexpr int DKC = 128;      // head_k_dim
 constexpr int KP = DKC + 4;   // LDS row pitch of K / Q / S rows in floats (conflict-free b128 reads across rows)
-constexpr int TP = CC + 1;    // LDS row pitch of the 32 x 32 matrices
-constexpr int WS_FLOATS = 2 * CC * CC + 4 * CC; // per (chunk, value head): T, P, A, W, the decays a, the strengths b
+constexpr int TP = CC + 4;    // LDS row pitch of the 32 x 32 matrices (16-byte rows)
+// per (chunk, value head): -G [32][128], P [32][32], A, W = A_C / A, the decays a, the strengths b; behind all of them U [32][Dv] per (chunk, value head)
+constexpr int WS_P = CC * DKC, WS_A = WS_P + CC * CC, WS_W = WS_A + CC, WS_DECAY = WS_W + CC, WS_FLOATS = WS_DECAY + 2 * CC;
 } // namespace
 
-// Sequence split (round 4).  The chain of n chunk steps is the scan's whole cost (2.5 us per chunk with half of the CUs idle: 159 us per 2043-token pass
-// of the 0.8B model), and the recurrence is AFFINE in the state, row by row -- S_t[i,:] = S_{t-1}[i,:] a_t (I - b_t k_t k_t^T) + b_t v_t[i] k_t^T -- with the
+// Sequence split.  The chain of n chunk steps is the scan's whole cost (1.46 us per chunk with half of the CUs idle), and the recurrence is AFFINE in the state, row by
+// row -- S_t[i,:] = S_{t-1}[i,:] a_t (I - b_t k_t k_t^T) + b_t v_t[i] k_t^T -- with the
 // same linear part for every row.  So the chunks [mid, n) do not have to wait for the chunks [0, mid): they run at the same time from a ZERO state with the
 // real values (Z_t, outputs Z_t q_t) and, as Dk more "value columns" per head, from the IDENTITY with zero values (H_t, outputs u_t = H_t q_t); then
 //     S_t = S_mid H_t + Z_t        o_t = Z_t q_t + S_mid u_t        (S_mid = the state after chunk mid - 1)
 // and `dn_chunk_fixup_kernel` adds the S_mid terms (one [tokens, Dk] x [Dk, Dv] product per head on the f32 matrix cores) before the outputs are rounded.
-// Twice the scan work for segment 1, on the CUs the single chain leaves idle.  Placement decides what that buys: as three 4-wave workgroups per tile
-// (first form, 384 workgroups) the pairs that happen to share a CU share its matrix pipes and run 3.6 us per chunk -- 116 us for 32 + 32 chunks.  Here a
-// segment-1 workgroup is EIGHT waves: group 0 the real tile, group 1 the homogeneous tile of the same head (same K / Q / T / P operands, staged once, each
-// group fetching half of them), one workgroup per CU, and segment 0 -- alone on its CUs at 2.5 us per chunk -- takes the larger share of the chunks.
+// Twice the scan work for segment 1, on the CUs the single chain leaves idle.  Placement decides what that buys: a segment-1 workgroup is EIGHT waves, group 0 the real tile,
+// group 1 the homogeneous tile of the same head, one workgroup per CU, 2.8 us a chunk; segment 0 -- alone on its CUs at 1.46 us per chunk -- takes the larger share of the chunks.
 struct ScanSplit {
     uint32_t mid_chunk; // 0: one segment (the plain scan)
     float* mid_state;   // [Hv][Dv][Dk]  final state of segment 0
@@ -51,13 +51,14 @@ struct ScanSplit {
     float* u;           // [T - 32 mid][Hv Dk] f32: H_t q_t
 };
 static uint32_t split_mid_chunk(uint32_t n_chunks, uint32_t head_v_dim) {
-    static const uint32_t min_chunks = [] { // UZU_DN_SPLIT: chunks from which the scan is split (0 = never; A/B runs).  Below ~12 chunks the fix-up launch costs more than the shorter chain saves
+    static const uint32_t min_chunks = [] { // chunks from which the scan is split (0 = never; A/B runs): the fix-up launch is 8 us + 0.12 a chunk, the shorter chain saves 0.5 a chunk
+        // (17 chunks of the 0.8B model: one chain 28.6 us, split 22 + 9.9)
         const char* e = tune_env("dn_split");
-        return e ? (uint32_t)atoi(e) : 16u;
+        return e ? (uint32_t)atoi(e) : 24u;
     }();
-    static const uint32_t pct = [] { // UZU_DN_SPLIT_PCT: segment 0's share of the chunks (its workgroups run ~2.5 us per chunk, segment 1's double groups ~3.4)
+    static const uint32_t pct = [] { // UZU_DN_SPLIT_PCT: segment 0's share of the chunks (its workgroups run 1.46 us per chunk, segment 1's double groups 2.8)
         const char* e = lab_env("UZU_DN_SPLIT_PCT");
-        const int v = e ? atoi(e) : 58;
+        const int v = e ? atoi(e) : 66;
         return (uint32_t)(v < 10 ? 10 : v > 90 ? 90 : v);
     }();
     if (!min_chunks || n_chunks < min_chunks || head_v_dim != (uint32_t)DKC) return 0u; // (a segment-1 workgroup pairs value tile i with homogeneous tile i: Dv = Dk)
@@ -68,7 +69,7 @@ static size_t split_floats(uint32_t num_v_heads, uint32_t value_dim, uint32_t su
     return (size_t)2 * value_dim * DKC + (size_t)num_v_heads * DKC * DKC + (size_t)suffix_len * value_dim + (size_t)suffix_len * num_v_heads * DKC;
 }
 size_t delta_net_chunk_workspace_bytes(uint32_t num_v_heads, uint32_t value_dim, uint32_t suffix_len) {
-    return ((size_t)((suffix_len + CC - 1) / CC) * num_v_heads * WS_FLOATS + split_floats(num_v_heads, value_dim, suffix_len)) * sizeof(float);
+    return ((size_t)((suffix_len + CC - 1) / CC) * ((size_t)num_v_heads * WS_FLOATS + (size_t)CC * value_dim) + split_floats(num_v_heads, value_dim, suffix_len)) * sizeof(float);
 }
 
 template <int CTRL> __device__ __forceinline__ double dpp_f64(double v) {
@@ -89,198 +90,300 @@ __device__ __forceinline__ double log_prefix(float d, int token) {
 }
 
 // grid (chunks, Hv), 256 threads.
-// FUSED (round 6): DeltaNetPrefillPrep (prefill_prep.rs:30-113; k_deltanet.hip::delta_net_prefill_prep_kernel) runs inside this kernel -- the chunk's q / k rows come
+// FUSED: DeltaNetPrefillPrep (prefill_prep.rs:30-113; k_deltanet.hip::delta_net_prefill_prep_kernel) runs inside this kernel -- the chunk's q / k rows come
 // straight from the conv'd in-projection rows (bf16), are L2-normalised with that kernel's element mapping and reduction order (a wave per token, two elements per
 // lane, wave_sum: the same bits), land in LDS for the Gram matrices AND in q_norm / k_norm for the scan (written by the first value head of a key head); beta and the
-// decay of the chunk's tokens are computed where they are used.  One launch and one 33 MB read of the f32 rows less per DeltaNet layer (9.85 -> 9.57 ms per 2043-token
-// pass of the 0.8B).  Also convolving the q / k channels here (the conv kernel then rewriting the v channels only) was built, bit-identical, and bought nothing
-// (9.66-9.73 vs 9.60-9.72 ms, profiles/r6_prep_fused_ab.txt): the window loads and 4 SiLUs per token cost this kernel what the conv kernel saved; not kept.
+// decay of the chunk's tokens are computed where they are used.  Also convolving the q / k channels here (the conv kernel then rewriting the v channels only) was built,
+// bit-identical, and bought nothing (9.66-9.73 vs 9.60-9.72 ms, profiles/r6_prep_fused_ab.txt): the window loads and 4 SiLUs per token cost this kernel what the conv kernel
+// saved; not kept.
+// What it costs is the chain of its phases, so each takes all waves or runs beside another: wave 0 the decays (three exponentials and a logarithm of a token in 64 bits) while
+// the others normalise the rows, a wave's reciprocal roots all at once; the Gram tiles at and below the diagonal on the f32 matrix cores, two a wave in waves 0 and 1, one in waves 2 and 3, which make the decay
+// ratios besides; the forward substitution with a thread per right-hand side, row by row as soon as the row above is known (right-looking: the sums of a row in the same order,
+// the FMAs of different rows independent).  Sixteen heads of a 37-token prompt: 17.1 us (one thread a column of T, a
+// sum after the other) -> 11.3, of 2043 tokens 28.6 -> 28.8 (and U and G besides).
 template <bool FUSED>
-__global__ void __launch_bounds__(256) dn_chunk_prep_kernel(const float* q_norm, const float* k_norm, const float* beta_buf, const float* decay_buf,
-                                                            float* ws, uint32_t num_v_heads, uint32_t num_k_heads, uint32_t key_dim, uint32_t suffix_len,
+__global__ void __launch_bounds__(256, 3) dn_chunk_prep_kernel(const float* q_norm, const float* k_norm, const float* beta_buf, const float* decay_buf,
+                                                            float* ws, float* u_out, uint32_t num_v_heads, uint32_t num_k_heads, uint32_t head_v_dim, uint32_t key_dim, uint32_t suffix_len,
                                                             const uint16_t* in_proj, const float* a_log, const float* dt_bias, float* q_norm_out, float* k_norm_out,
                                                             uint32_t value_dim, const uint16_t* conv_rows, float* conv_state) {
-    __shared__ __attribute__((aligned(16))) float sK[CC * KP], sQ[CC * KP];
-    // the three 32 x 32 matrices live in the Q rows once the Gram products have read them (a barrier in between): 34 KB of LDS per workgroup instead of 47 -- four
-    // workgroups per CU, the whole grid of a 2048-token pass (1024 workgroups) resident at once
-    float* const sKK = sQ;
-    float* const sQK = sQ + CC * TP;
-    float* const sM = sQ + 2 * CC * TP;
-    static_assert(3 * CC * TP <= CC * KP, "the Gram / M matrices fit in the Q rows");
+    __shared__ __attribute__((aligned(16))) float sK[CC * KP], sQ[CC * KP], sV[CC * KP];
+    // M (by columns) and the decay ratios: in the Q rows once the Gram products have read them (a barrier in between): four workgroups per CU
+    float* const sMt = sQ;
+    float* const sRat = sQ + CC * TP;
+    static_assert(2 * CC * TP <= CC * KP, "the matrices fit in the Q rows");
     __shared__ double s_lg[CC];
-    __shared__ float s_b[CC];
+    __shared__ float s_b[CC], s_ba[CC];
     __shared__ uint64_t s_exp_tab[32];
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i16 = lane & 15, kq = lane >> 4;
     const uint32_t groups_per_head = num_v_heads / num_k_heads;
     const uint32_t chunk = blockIdx.x, hv = blockIdx.y, hk = hv / groups_per_head;
     const uint32_t t0 = chunk * CC;
-    float* const w_t = ws + ((size_t)chunk * num_v_heads + hv) * WS_FLOATS;
-    float* const w_p = w_t + CC * CC;
+    const uint32_t conv_dim = 2 * key_dim + value_dim;
+    const size_t total_proj_dim = (size_t)conv_dim + value_dim + 2 * num_v_heads;
+    float* const w_g = ws + ((size_t)chunk * num_v_heads + hv) * WS_FLOATS;
+    float* const w_u = u_out + ((size_t)chunk * num_v_heads + hv) * CC * head_v_dim;
+    const uint32_t live_rows = min(suffix_len - t0, (uint32_t)CC);
+    auto row_of = [&](uint32_t i) { return min(i, live_rows - 1); }; // of the chunk; past the end: the last one
+    // the next pass's carried conv state, the last three raw rows (T >= 3: delta_net_prefill_chunked_supported) -- the out-of-place conv kernel only reads the state; the first
+    // chunk's workgroups share the channels, the first two of a thread are read here and written at the end
+    auto next_state = [&](uint32_t c, float (&nx)[3]) {
+#pragma unroll
+        for (int tap = 0; tap < 3; ++tap) nx[tap] = bf16_to_f32(in_proj[(size_t)(suffix_len - 3 + tap) * total_proj_dim + c]);
+    };
+    const bool carries = FUSED && conv_state && chunk == 0;
+    const uint32_t c0 = hv * 256 + tid, c_step = num_v_heads * 256;
+    float nx[2][3] = {};
+    if (carries) {
+        if (c0 < conv_dim) next_state(c0, nx[0]);
+        if (c0 + c_step < conv_dim) next_state(c0 + c_step, nx[1]);
+    }
+    // the chunk's values, 128 columns at a time: f32 rows in LDS
+    const uint32_t v_stride = conv_rows ? conv_dim : (uint32_t)total_proj_dim;
+    const uint16_t* v_base = (conv_rows ? conv_rows : in_proj) + (size_t)t0 * v_stride + 2 * key_dim + hv * head_v_dim;
+    uint32_t vraw[8];
+    auto load_values = [&](uint32_t column) {
+        const uint16_t* v = v_base + min(column + 2 * lane, head_v_dim - 2);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) vraw[r] = *(const uint32_t*)(v + row_of(wave + 4 * r) * v_stride);
+    };
+    auto put_values = [&]() {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) *(float2*)(sV + (wave + 4 * r) * KP + 2 * lane) = make_float2(bits_to_f32(vraw[r] << 16), bits_to_f32(vraw[r] & 0xFFFF0000u));
+    };
+    load_values(0);
     if constexpr (FUSED) {
-        if (tid < 32) s_exp_tab[tid] = kExp2fTab[tid];
-        const uint32_t lane = tid & 63, wave = tid >> 6;
-        const uint32_t conv_dim = 2 * key_dim + value_dim;
-        const size_t total_proj_dim = (size_t)conv_dim + value_dim + 2 * num_v_heads;
-        const bool writer = hv % groups_per_head == 0; // one value head per key head files the rows for the scan
-        constexpr int TW = CC / 4; // this wave's 8 tokens: every load requested before the first reduction
-        const uint32_t tl0 = wave * TW;
-        uint32_t qw[TW], kw[TW];
-#pragma unroll
-        for (int i = 0; i < TW; ++i) {
-            const uint32_t t = min(t0 + tl0 + i, suffix_len - 1);
+        if (wave) { // the rows: waves 1 .. 3, 11, 11 and 10 tokens
+            const bool writer = hv % groups_per_head == 0; // one value head per key head files the rows for the scan
+            constexpr int TW = 11; // every load requested before the first reduction
+            uint32_t qw[TW], kw[TW];
+            const int tl0 = (wave - 1) * TW, count = wave == 3 ? CC - 2 * TW : TW;
             // (conv_rows: the conv'd channels were written out of place -- k_deltanet.hip::conv_apply4_oop_kernel -- and the in-projection rows are still raw)
-            const uint16_t* row = (conv_rows ? conv_rows + (size_t)t * conv_dim : in_proj + (size_t)t * total_proj_dim) + hk * DKC + lane * 2;
-            qw[i] = *(const uint32_t*)row;
-            kw[i] = *(const uint32_t*)(row + key_dim);
-        }
+            const uint32_t stride = conv_rows ? conv_dim : (uint32_t)total_proj_dim;
+            const uint16_t* rows = (conv_rows ? conv_rows : in_proj) + (size_t)t0 * stride + hk * DKC;
 #pragma unroll
-        for (int i = 0; i < TW; ++i) {
-            const uint32_t tl = tl0 + i, t = t0 + tl;
-            const float qv[2] = {bits_to_f32(qw[i] << 16), bits_to_f32(qw[i] & 0xFFFF0000u)}, kv[2] = {bits_to_f32(kw[i] << 16), bits_to_f32(kw[i] & 0xFFFF0000u)};
-            float q_sq = 0.f, k_sq = 0.f;
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                q_sq += qv[e] * qv[e];
-                k_sq += kv[e] * kv[e];
+            for (int i = 0; i < TW; ++i) {
+                const uint16_t* row = rows + row_of(tl0 + i) * stride;
+                qw[i] = *(const uint32_t*)(row + lane * 2);
+                kw[i] = *(const uint32_t*)(row + key_dim + lane * 2);
             }
-            q_sq = wave_sum(q_sq);
-            k_sq = wave_sum(k_sq);
-            const float q_inv = 1.0f / sqrtf(q_sq + 1e-6f);
-            const float q_scale = 1.0f / sqrtf((float)DKC);
-            const float k_inv = 1.0f / sqrtf(k_sq + 1e-6f);
-            const bool live = t < suffix_len;
-            float2 qn = make_float2(0.f, 0.f), kn = qn; // zero rows past the end: b = 0, a = 1 there, so they change nothing
-            if (live) qn = make_float2(qv[0] * q_inv * q_scale, qv[1] * q_inv * q_scale), kn = make_float2(kv[0] * k_inv, kv[1] * k_inv);
-            *(float2*)(sQ + tl * KP + lane * 2) = qn;
-            *(float2*)(sK + tl * KP + lane * 2) = kn;
-            if (live && writer) {
-                *(float2*)(q_norm_out + (size_t)t * key_dim + hk * DKC + lane * 2) = qn;
-                *(float2*)(k_norm_out + (size_t)t * key_dim + hk * DKC + lane * 2) = kn;
-            }
-        }
-        if (conv_state && chunk == 0) { // the next pass's carried conv state X[T - 3 + tap] (X = [state | raw rows]) -- the out-of-place conv kernel only reads the state;
-            // the first chunk's workgroups share the channels; a channel's three values are read before any is written (one thread)
-            for (uint32_t c = hv * 256 + tid; c < conv_dim; c += num_v_heads * 256) {
-                float nx[3];
+            float sq = 0.f; // lane i: the square sum of token i's query, lane 16 + i: of its key
 #pragma unroll
-                for (int tap = 0; tap < 3; ++tap) {
-                    const int i = (int)suffix_len - 3 + tap;
-                    nx[tap] = i < 0 ? conv_state[(size_t)c * 3 + 3 + i] : bf16_to_f32(in_proj[(size_t)i * total_proj_dim + c]);
+            for (int i = 0; i < TW; ++i) {
+                const float qv[2] = {bits_to_f32(qw[i] << 16), bits_to_f32(qw[i] & 0xFFFF0000u)}, kv[2] = {bits_to_f32(kw[i] << 16), bits_to_f32(kw[i] & 0xFFFF0000u)};
+                float q_sq = 0.f, k_sq = 0.f;
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    q_sq += qv[e] * qv[e];
+                    k_sq += kv[e] * kv[e];
                 }
+                q_sq = wave_sum(q_sq);
+                k_sq = wave_sum(k_sq);
+                sq = lane == i ? q_sq : lane == 16 + i ? k_sq : sq;
+            }
+            const float inv = 1.0f / sqrtf(sq + 1e-6f);
+            const float q_scale = 1.0f / sqrtf((float)DKC);
 #pragma unroll
-                for (int tap = 0; tap < 3; ++tap) conv_state[(size_t)c * 3 + tap] = nx[tap];
+            for (int i = 0; i < TW; ++i) {
+                const uint32_t tl = tl0 + i;
+                const float q_inv = bits_to_f32(__builtin_amdgcn_readlane(f32_to_bits(inv), i)), k_inv = bits_to_f32(__builtin_amdgcn_readlane(f32_to_bits(inv), 16 + i));
+                float2 qn = make_float2(0.f, 0.f), kn = qn; // zero rows past the end: b = 0, a = 1 there, so they change nothing
+                const bool live = tl < live_rows;
+                if (live) {
+                    qn = make_float2(bits_to_f32(qw[i] << 16) * q_inv * q_scale, bits_to_f32(qw[i] & 0xFFFF0000u) * q_inv * q_scale);
+                    kn = make_float2(bits_to_f32(kw[i] << 16) * k_inv, bits_to_f32(kw[i] & 0xFFFF0000u) * k_inv);
+                }
+                if (i < count) {
+                    *(float2*)(sQ + tl * KP + lane * 2) = qn;
+                    *(float2*)(sK + tl * KP + lane * 2) = kn;
+                    if (live && writer) {
+                        *(float2*)(q_norm_out + (size_t)(t0 + tl) * key_dim + hk * DKC + lane * 2) = qn;
+                        *(float2*)(k_norm_out + (size_t)(t0 + tl) * key_dim + hk * DKC + lane * 2) = kn;
+                    }
+                }
             }
-        }
-        __syncthreads(); // (the exp table)
-        if (tid < CC) {
-            const bool live = t0 + tid < suffix_len;
-            float d = 1.0f, b = 0.0f;
-            if (live) {
-                const uint16_t* row = in_proj + (size_t)(t0 + tid) * total_proj_dim + conv_dim + value_dim;
-                const float beta_raw = bf16_to_f32(row[hv]);
-                b = 1.0f / (1.0f + expf_glibc_tab(-beta_raw, s_exp_tab));
-                const float a_raw = bf16_to_f32(row[num_v_heads + hv]);
-                const float sp_in = a_raw + dt_bias[hv];
-                const float sp = sp_in > 20.0f ? sp_in : logf_glibc(1.0f + expf_glibc_tab(sp_in, s_exp_tab));
-                const float log_decay = -expf_glibc_tab(a_log[hv], s_exp_tab) * sp;
-                d = expf_glibc_tab(log_decay, s_exp_tab);
-            }
-            s_lg[tid] = log_prefix(d, tid);
-            s_b[tid] = b;
-            w_t[2 * CC * CC + 2 * CC + tid] = d, w_t[2 * CC * CC + 3 * CC + tid] = b;
         }
     } else {
-    // K, Q rows of the chunk (zero rows past the end: b = 0, a = 1 there, so they change nothing)
-    for (int idx = tid; idx < CC * (DKC / 4); idx += 256) {
-        const int t = idx / (DKC / 4), c4 = idx % (DKC / 4);
-        float4 kv = make_float4(0.f, 0.f, 0.f, 0.f), qv = kv;
-        if (t0 + t < suffix_len) {
-            kv = *(const float4*)(k_norm + (size_t)(t0 + t) * key_dim + hk * DKC + c4 * 4);
-            qv = *(const float4*)(q_norm + (size_t)(t0 + t) * key_dim + hk * DKC + c4 * 4);
-        }
-        *(float4*)(sK + t * KP + c4 * 4) = kv;
-        *(float4*)(sQ + t * KP + c4 * 4) = qv;
-    }
-    if (tid < CC) {
-        const bool live = t0 + tid < suffix_len;
-        const float d = live ? decay_buf[(size_t)(t0 + tid) * num_v_heads + hv] : 1.0f;
-        s_lg[tid] = log_prefix(d, tid);
-        s_b[tid] = live ? beta_buf[(size_t)(t0 + tid) * num_v_heads + hv] : 0.0f;
-        w_t[2 * CC * CC + 2 * CC + tid] = d, w_t[2 * CC * CC + 3 * CC + tid] = s_b[tid];
-    }
-    }
-    __syncthreads();
-    // Gram matrices: thread -> row i, four columns j0..j0+3
-    {
-        const int i = tid >> 3, j0 = (tid & 7) * 4;
-        float kk[4] = {0.f, 0.f, 0.f, 0.f}, qk[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-        for (int d4 = 0; d4 < DKC; d4 += 4) {
-            const float4 ki = *(const float4*)(sK + i * KP + d4), qi = *(const float4*)(sQ + i * KP + d4);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float4 kj = *(const float4*)(sK + (j0 + j) * KP + d4);
-                kk[j] = fmaf(ki.x, kj.x, kk[j]), kk[j] = fmaf(ki.y, kj.y, kk[j]), kk[j] = fmaf(ki.z, kj.z, kk[j]), kk[j] = fmaf(ki.w, kj.w, kk[j]);
-                qk[j] = fmaf(qi.x, kj.x, qk[j]), qk[j] = fmaf(qi.y, kj.y, qk[j]), qk[j] = fmaf(qi.z, kj.z, qk[j]), qk[j] = fmaf(qi.w, kj.w, qk[j]);
+        // K, Q rows of the chunk (zero rows past the end: b = 0, a = 1 there, so they change nothing)
+        for (int idx = tid; idx < CC * (DKC / 4); idx += 256) {
+            const int t = idx / (DKC / 4), c4 = idx % (DKC / 4);
+            float4 kv = make_float4(0.f, 0.f, 0.f, 0.f), qv = kv;
+            if (t0 + t < suffix_len) {
+                kv = *(const float4*)(k_norm + (size_t)(t0 + t) * key_dim + hk * DKC + c4 * 4);
+                qv = *(const float4*)(q_norm + (size_t)(t0 + t) * key_dim + hk * DKC + c4 * 4);
             }
+            *(float4*)(sK + t * KP + c4 * 4) = kv;
+            *(float4*)(sQ + t * KP + c4 * 4) = qv;
         }
-        __syncthreads(); // every thread has read its K / Q rows: the Q rows become the matrices
+    }
+    if (wave == 0) { // decays and strengths, a token a lane
+        const uint32_t tok = t0 + row_of(lane);
+        float raw_b, raw_a;
+        if constexpr (FUSED) {
+            const uint16_t* row = in_proj + (size_t)tok * total_proj_dim + conv_dim + value_dim;
+            raw_b = bf16_to_f32(row[hv]), raw_a = bf16_to_f32(row[num_v_heads + hv]);
+        } else raw_b = beta_buf[(size_t)tok * num_v_heads + hv], raw_a = decay_buf[(size_t)tok * num_v_heads + hv];
+        if (lane < 32) s_exp_tab[lane] = kExp2fTab[lane];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (this wave reads it now, the others behind the barrier)
+        if (lane < CC) {
+            float d = 1.0f, b = 0.0f;
+            if ((uint32_t)lane < live_rows) {
+                if constexpr (FUSED) {
+                    b = 1.0f / (1.0f + expf_glibc_tab(-raw_b, s_exp_tab));
+                    const float sp_in = raw_a + dt_bias[hv];
+                    const float sp = sp_in > 20.0f ? sp_in : logf_glibc(1.0f + expf_glibc_tab(sp_in, s_exp_tab));
+                    const float log_decay = -expf_glibc_tab(a_log[hv], s_exp_tab) * sp;
+                    d = expf_glibc_tab(log_decay, s_exp_tab);
+                } else d = raw_a, b = raw_b;
+            }
+            const double lg = log_prefix(d, lane);
+            const float a_t = exp_wide(lg, s_exp_tab);
+            s_lg[lane] = lg, s_b[lane] = b, s_ba[lane] = -b * a_t;
+            w_g[WS_DECAY + lane] = d, w_g[WS_DECAY + CC + lane] = b;
+            w_g[WS_A + lane] = a_t;
+        }
+    }
+    put_values();
+    __syncthreads();
+    // Gram tiles (rows 16 x .., columns 16 y ..; D: rows 4 kq + r, column i16): waves 0, 1: K K^T (0, 0) and (1, 0) | (1, 1), Q K^T (0, 0); waves 2, 3: Q K^T (1, 0) | (1, 1)
+    typedef __attribute__((ext_vector_type(4))) float acc_t;
+    auto gram = [&](const float* rows, int x, int y) {
+        const float *xr = rows + (16 * x + i16) * KP + 4 * kq, *yr = sK + (16 * y + i16) * KP + 4 * kq;
+        acc_t part[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sKK[i * TP + j0 + j] = kk[j], sQK[i * TP + j0 + j] = qk[j];
+        for (int g = 0; g < DKC / 16; ++g) { // contraction index of step e in quarter kq: 16 g + 4 kq + e
+            const f32x4_v a = *(const f32x4_v*)(xr + 16 * g), b = *(const f32x4_v*)(yr + 16 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], part[e & 1], 0, 0, 0);
+        }
+        return part[0] + part[1];
+    };
+    acc_t tile0, tile1 = {0.f, 0.f, 0.f, 0.f};
+    if (wave == 0) tile0 = gram(sK, 0, 0), tile1 = gram(sK, 1, 0);
+    else if (wave == 1) tile0 = gram(sK, 1, 1), tile1 = gram(sQ, 0, 0);
+    else tile0 = gram(sQ, 1, wave - 2);
+    float ratio[5];
+    if (wave >= 2) { // A_i / A_j for j <= i: 528 of them, row r and row 31 - r together 33
+#pragma unroll
+        for (int n = 0; n < 5; ++n) {
+            const int p = min(tid - DKC + 128 * n, 527), r = p / 33, q = p % 33, i = q <= r ? r : 31 - r, j = q <= r ? q : q - r - 1;
+            ratio[n] = exp_wide(s_lg[i] - s_lg[j], s_exp_tab);
+        }
+    }
+    __syncthreads(); // every wave has read its K / Q rows: the Q rows become the matrices
+    if (wave >= 2) {
+#pragma unroll
+        for (int n = 0; n < 5; ++n) {
+            const int p = min(tid - DKC + 128 * n, 527), r = p / 33, q = p % 33, i = q <= r ? r : 31 - r, j = q <= r ? q : q - r - 1;
+            sRat[i * TP + j] = ratio[n];
+        }
     }
     __syncthreads();
-    for (int idx = tid; idx < CC * CC; idx += 256) {
-        const int i = idx / CC, j = idx % CC;
-        const float ratio = exp_wide(j <= i ? s_lg[i] - s_lg[j] : 0.0, FUSED ? s_exp_tab : kExp2fTab); // A_i / A_j for j <= i
-        sM[i * TP + j] = j < i ? s_b[i] * ratio * sKK[i * TP + j] : 0.0f;
-        w_p[idx] = j <= i ? ratio * sQK[i * TP + j] : 0.0f;
+    auto put_m = [&](const acc_t& kk, int x, int y) { // M_ij = b_i A_i / A_j k_i.k_j below the diagonal, by columns
+        const int j = 16 * y + i16, i0 = 16 * x + 4 * kq;
+        f32x4_v m;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) m[r] = j < i0 + r ? s_b[i0 + r] * sRat[(i0 + r) * TP + j] * kk[r] : 0.0f;
+        *(f32x4_v*)(sMt + j * TP + i0) = m;
+    };
+    auto put_p = [&](const acc_t& qk, int x, int y) {
+        const int j = 16 * y + i16, i0 = 16 * x + 4 * kq;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) w_g[WS_P + (i0 + r) * CC + j] = j <= i0 + r ? sRat[(i0 + r) * TP + j] * qk[r] : 0.0f;
+    };
+    if (tid < CC) { // behind a column of M: its row's coefficients of the right-hand sides
+        w_g[WS_W + tid] = exp_wide(s_lg[CC - 1] - s_lg[tid], s_exp_tab); // A_C / A_t
+        *(float2*)(sMt + tid * TP + CC) = make_float2(s_b[tid], s_ba[tid]);
     }
-    if (tid < CC) {
-        w_t[2 * CC * CC + tid] = exp_wide(s_lg[tid], FUSED ? s_exp_tab : kExp2fTab);                      // A_t
-        w_t[2 * CC * CC + CC + tid] = exp_wide(s_lg[CC - 1] - s_lg[tid], FUSED ? s_exp_tab : kExp2fTab);  // A_C / A_t
+    if (wave == 0) put_m(tile0, 0, 0), put_m(tile1, 1, 0);
+    else if (wave == 1) put_m(tile0, 1, 1), put_p(tile1, 0, 0);
+    else {
+        put_p(tile0, 1, wave - 2);
+        if (wave == 2) { // P above the diagonal
+#pragma unroll
+            for (int r = 0; r < 4; ++r) w_g[WS_P + (4 * kq + r) * CC + 16 + i16] = 0.0f;
+        }
     }
     __syncthreads();
-    // T = (I + M)^-1 diag(b): column c by forward substitution, one thread per column (M_ij is a broadcast LDS read)
-    if (tid < CC) {
-        float x[CC];
+    // (I + M) X = diag(b) [-diag(A) K, V]: column c of 128 + Dv in a thread.  A row's sum over the rows above it is gathered first, its own term joins it in one rounding: started
+    // from that term, which is the larger one, the sum would be rounded at its size 31 times (a state of fast decays 1.6 times as far from 64 bits)
+    const bool key = tid < DKC; // (a whole wave's columns)
+    for (uint32_t v0 = 0; v0 < head_v_dim; v0 += DKC) {
+        const uint32_t c = key ? tid : v0 + tid - DKC;
+        if (v0) { // values wider than 128
+            __syncthreads();
+            load_values(v0);
+            put_values();
+            __syncthreads();
+        }
+        if (key ? v0 != 0 : c >= head_v_dim) continue;
+        const float* val = key ? sK + tid : sV + tid - DKC;
+        float x[CC] = {};
+        f32x4_v m[2][8]; // column j of M, the next one on its way
+        float2 coef[2];
+        float rhs[2];
+        auto column = [&](int j) {
+            coef[j & 1] = *(const float2*)(sMt + j * TP + CC);
+            rhs[j & 1] = val[j * KP];
 #pragma unroll
-        for (int i = 0; i < CC; ++i) {
-            float acc = i == tid ? s_b[i] : 0.0f;
+            for (int q = (j + 1) / 4; q < 8; ++q) m[j & 1][q] = *(const f32x4_v*)(sMt + j * TP + 4 * q);
+        };
+        column(0);
 #pragma unroll
-            for (int j = 0; j < i; ++j) acc = fmaf(-sM[i * TP + j], x[j], acc);
-            x[i] = acc;
-            w_t[i * CC + tid] = acc;
+        for (int j = 0; j < CC; ++j) {
+            if (j + 1 < CC) column(j + 1);
+            x[j] = fmaf(key ? coef[j & 1].y : coef[j & 1].x, rhs[j & 1], -x[j]);
+#pragma unroll
+            for (int i = j + 1; i < CC; ++i) x[i] = fmaf(m[j & 1][i / 4][i % 4], x[j], x[i]);
+            __builtin_amdgcn_sched_barrier(0); // (all columns at once would not fit the registers)
+        }
+        float* dst = key ? w_g + c : w_u + c;
+        const uint32_t stride = key ? (uint32_t)DKC : head_v_dim;
+#pragma unroll
+        for (int i = 0; i < CC; ++i) dst[(size_t)i * stride] = x[i];
+    }
+    if (carries) {
+#pragma unroll
+        for (int tap = 0; tap < 3; ++tap) {
+            if (c0 < conv_dim) conv_state[(size_t)c0 * 3 + tap] = nx[0][tap];
+            if (c0 + c_step < conv_dim) conv_state[(size_t)(c0 + c_step) * 3 + tap] = nx[1][tap];
+        }
+        for (uint32_t c = c0 + 2 * c_step; c < conv_dim; c += c_step) {
+            next_state(c, nx[0]);
+#pragma unroll
+            for (int tap = 0; tap < 3; ++tap) conv_state[(size_t)c * 3 + tap] = nx[0][tap];
         }
     }
 }
 
-// Matrix-core scan.  (The VALU scans of rounds 1-2 read two LDS operands per four FMAs: 780 KB of LDS reads per chunk and workgroup,
-// 158 us per 1024 tokens at the 0.8B shape; removed in round 4, git history has them.)  The four products of a chunk run on v_mfma_f32_16x16x4_f32 -- f32
-// operands, exact f32 products, f32 accumulation: the arithmetic of the VALU scan in another summation order -- with operands
-// fetched once per chunk into registers.  A workgroup owns 16 value columns of a head (grid (Dv / 16, Hv), 4 waves):
-//   stage 1  [K; Q] S^T     wave w = one 16-token tile of K (w = 0, 1) or Q (w = 2, 3): 16 x 16 x 128, 32 MFMAs
-//   stage 2  D = T R        waves 0, 1: one 16-token tile each, 8 MFMAs; D and D diag(W) parked in LDS
-//   stage 3  O = A Q S^T + P D   waves 2, 3: their stage-1 accumulator is the C operand, 8 MFMAs
-//   stage 4  S = A_C S + (D W)^T K   every wave owns two 16-wide dk tiles of the state in its accumulators, 2 x 8 MFMAs
+// The scan, v_mfma_f32_16x16x4_f32 throughout -- f32 operands, exact f32 products, f32 accumulation.  Four waves own 16 value columns of a head:
+//   stage 1  waves 0, 1: D = U - G S^T for 16 tokens each, 32 MFMAs; waves 2, 3: Q S^T
+//   stage 2  S = A_C S + (D W)^T K   every wave owns 32 dk of the state in its accumulators, 2 x 8 MFMAs
+//   stage 3  O = A Q S^T + P D   waves 2, 3: 8 MFMAs, behind their part of the new state
+// The chunk chain is the cost, so nothing else is on it: every operand but the state and D goes from memory straight into the registers that the MFMAs read, one chunk ahead
+// (G, U, P as the preparation wrote them, Q and K as rows); only S and D pass through LDS, with a barrier each.  (K, Q, T and P staged in LDS, T as a third dependent product,
+// four barriers: 2.75 us a chunk; this form 1.46, a segment-1 workgroup of two tiles 2.8.)
 // MFMA operand layout (16x16x4): A lane l = row l % 16, k-quarter l / 16; B lane l = column l % 16, k-quarter l / 16; C / D four
-// registers = rows 4 (l / 16) + r of column l % 16.  The contraction index of step s in quarter q is (K / 4) q + s for both
-// operands, so a lane's operand values are consecutive in memory; in stages 2 and 4, which contract over tokens, it is 4 s + q: the products are added in time
-// order and the late tokens, which weigh most under a decay, come last (T's columns are stored so that a lane's values are consecutive there too).  With that, four
-// chains in stage 1 and the old state added behind the chunk's own products, the state of 16 to 63 tokens is 4e-8 to 1.2e-7 of its norm from 64 bits; the
-// recurrence token by token: 5e-8 to 1.9e-7.
-__global__ void __launch_bounds__(256) dn_chunk_scan_mfma_kernel(const float* q_norm, const float* k_norm, const uint16_t* in_proj, const float* ws, float* state,
-                                                                 uint16_t* out, uint32_t num_v_heads, uint32_t num_k_heads, uint32_t head_v_dim, uint32_t key_dim,
-                                                                 uint32_t value_dim, uint32_t suffix_len, uint32_t v_row_stride) {
-    constexpr int DVT = 16, TPP = 36, RPP = 18; // value columns per workgroup; LDS pitches of T / P (16-byte rows) and R / D (conflict-free column walks)
-    __shared__ __attribute__((aligned(16))) float sK[CC * KP], sQ[CC * KP], sS[DVT * KP];
-    __shared__ __attribute__((aligned(16))) float sT[CC * TPP], sP[CC * TPP];
-    __shared__ float sR[CC * RPP], sD[CC * RPP], sDw[CC * RPP];
-    __shared__ float sA[CC], sW[CC];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i16 = lane & 15, kq = lane >> 4;
-    // XCD-aware (head, value tile) <- workgroup: consecutive workgroup ids go round the 8 XCDs, and the Dv / 16 workgroups of a head all walk
-    // the head's K / Q rows: with the plain (x = tile, y = head) numbering every one of them sits on another XCD and the rows are fetched
-    // 8 times (r2_pmc_fetch_size.csv: 186 MB against ~28 MB).  Here XCD x takes the pairs [x * total / 8, (x + 1) * total / 8): a head's tiles
-    // share one L2.
+// registers = rows 4 (l / 16) + r of column l % 16.  Contraction index of step (g, e) in quarter q: stage 1 dk = 16 g + 4 q + e, stage 3 token 8 q + s (a lane's values
+// lie together in memory); stage 2 token 4 s + q: the products are added in time order and the late tokens, which weigh most under a decay, come last.  With that, four
+// chains in stage 1 and the old state added behind the chunk's own products, the state of 16 to 200 tokens is 0.4 to 1.0 times as far from 64 bits as the recurrence token by token.
+//
+// DUAL (ScanSplit): grid (2 Dv / 16, Hv), 512 threads = two such groups of four waves;
+//   workgroups [0, Dv / 16) of a head: segment 0, chunks [0, mid): group 0 = the value tile from the carried state; group 1 leaves;
+//   the others:                        segment 1, chunks [mid, n): group 0 = the value tile from a zero state, group 1 = the homogeneous tile (identity, U = 0).
+template <bool DUAL>
+__global__ void __launch_bounds__(DUAL ? 512 : 256) dn_chunk_scan_kernel(const float* q_norm, const float* k_norm, const uint16_t* in_proj, const float* ws, const float* u_ws, const float* state_in,
+                                                                         float* state, uint16_t* out, uint32_t num_v_heads, uint32_t num_k_heads, uint32_t head_v_dim, uint32_t key_dim,
+                                                                         uint32_t value_dim, uint32_t suffix_len, ScanSplit sp, uint32_t v_row_stride) {
+    constexpr int DVT = 16, DP = CC + 4; // value columns of a tile; LDS pitch of D's columns
+    __shared__ __attribute__((aligned(16))) float smem[DUAL ? 2 : 1][DVT * KP + 2 * DVT * DP];
+    __shared__ uint32_t s_off[4];
+    const int tid = threadIdx.x, grp = DUAL ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0, ltid = tid & 255, lane = ltid & 63, wave = __builtin_amdgcn_readfirstlane(ltid >> 6), i16 = lane & 15, kq = lane >> 4;
+    float* const sS = smem[grp];           // [DVT][KP]: the state's rows (value columns)
+    float* const sD = sS + DVT * KP;       // [DVT][DP]: D by value columns, tokens in order
+    float* const sDw = sD + DVT * DP;      // D W, token 4 s + q at 8 q + s
+    // XCD-aware (head, value tile) <- workgroup: consecutive workgroup ids go round the 8 XCDs, and the workgroups of a head all walk
+    // the head's K / Q / G rows: with the plain (x = tile, y = head) numbering every one of them sits on another XCD and the rows are fetched
+    // 8 times.  Here XCD x takes the pairs [x * total / 8, (x + 1) * total / 8): a head's tiles share one L2.
     uint32_t hv = blockIdx.y, tile = blockIdx.x;
     {
         const uint32_t nx = gridDim.x, total = nx * gridDim.y, lin = blockIdx.x + nx * blockIdx.y;
@@ -289,161 +392,191 @@ __global__ void __launch_bounds__(256) dn_chunk_scan_mfma_kernel(const float* q_
             hv = pair / nx, tile = pair % nx;
         }
     }
+    const uint32_t tiles_v = head_v_dim / DVT;
+    const bool seg1 = DUAL && tile >= tiles_v, homog = seg1 && grp == 1;
+    if (DUAL && !seg1 && grp == 1) return; // (whole waves, in front of every barrier)
+    if (seg1) tile -= tiles_v;
     const uint32_t dv_base = tile * DVT, hk = hv / (num_v_heads / num_k_heads);
-    const uint32_t conv_dim = 2 * key_dim + value_dim;
-    // (v_row_stride != 0: `in_proj` is the out-of-place conv buffer, rows of conv_dim channels in the same q | k | v order)
-    const size_t total_proj_dim = v_row_stride ? (size_t)v_row_stride : (size_t)conv_dim + value_dim + 2 * num_v_heads;
     const uint32_t n_chunks = (suffix_len + CC - 1) / CC;
+    const uint32_t c_begin = seg1 ? sp.mid_chunk : 0u, c_end = DUAL && !seg1 ? sp.mid_chunk : n_chunks;
 
-    // state: wave w owns dk tiles 2 w, 2 w + 1 in accumulator layout: creg[tile][r] = S[dv = 4 kq + r][dk = 16 (2 w + tile) + i16]
+    // the state: wave w owns dk 32 w .. in accumulator layout, creg[t][r] = S[dv = 4 kq + r][dk = 32 w + 2 i16 + t]
     f32x4_v creg[2];
-    float* sbase = state + ((size_t)hv * head_v_dim + dv_base + 4 * kq) * DKC + 32 * wave + i16;
+    const size_t s_at = ((size_t)hv * head_v_dim + dv_base + 4 * kq) * DKC + 32 * wave + 2 * i16;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) creg[t][r] = sbase[(size_t)r * DKC + 16 * t];
-
-    // ---- operand staging: registers <- memory (chunk c + 1) while chunk c is computed, LDS <- registers at the chunk boundary
-    f32x4_v st_k[4], st_q[4];
-    float st_t[4], st_p[4], st_a = 0.f, st_w = 0.f, st_v[4];
-    const int v_row = 16 * (wave & 1) + 4 * kq; // stage-1 accumulator rows of waves 0, 1 (tokens of the chunk)
-    auto fetch = [&](uint32_t c) {
-        const uint32_t t0 = c * CC;
-        const float* w_t = ws + ((size_t)c * num_v_heads + hv) * WS_FLOATS;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int idx = tid + 256 * r, t = idx / (DKC / 4), c4 = idx % (DKC / 4);
-            const bool live = t0 + t < suffix_len;
-            const size_t tok = live ? t0 + t : suffix_len - 1; // clamped + zeroed: unconditional loads stay countable
-            const f32x4_v zero = {0.f, 0.f, 0.f, 0.f};
-            const f32x4_v kv = *(const f32x4_v*)(k_norm + tok * key_dim + hk * DKC + c4 * 4);
-            const f32x4_v qv = *(const f32x4_v*)(q_norm + tok * key_dim + hk * DKC + c4 * 4);
-            st_k[r] = live ? kv : zero, st_q[r] = live ? qv : zero;
-            st_t[r] = w_t[idx], st_p[r] = w_t[CC * CC + idx];
+    for (int r = 0; r < 4; ++r) {
+        float2 v = make_float2(0.f, 0.f);
+        if (!seg1) v = *(const float2*)(state_in + s_at + (size_t)r * DKC);
+        else if (homog) {
+            const uint32_t one = dv_base + 4 * kq + r, dk = 32 * wave + 2 * i16;
+            v = make_float2(one == dk ? 1.f : 0.f, one == dk + 1 ? 1.f : 0.f);
         }
-        st_a = w_t[2 * CC * CC + (tid & (CC - 1))], st_w = w_t[2 * CC * CC + CC + (tid & (CC - 1))];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const bool live = t0 + v_row + r < suffix_len;
-            const float vv = bf16_to_f32(in_proj[(size_t)(live ? t0 + v_row + r : suffix_len - 1) * total_proj_dim + 2 * key_dim + hv * head_v_dim + dv_base + i16]);
-            st_v[r] = live ? vv : 0.f;
-        }
-    };
-    float vreg[4] = {0.f, 0.f, 0.f, 0.f};
-    float off_sum = 0.f; // 0, or NaN behind an output or a state value that is no number
+        creg[0][r] = v.x, creg[1][r] = v.y;
+    }
     auto publish = [&]() {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int idx = tid + 256 * r, t = idx / (DKC / 4), c4 = idx % (DKC / 4);
-            const int at = ((t & 16) + 4 * (t & 3) + (t >> 2 & 3)) * KP + c4 * 4; // (four tokens in a row lie sixteen banks apart)
-            *(f32x4_v*)(sK + at) = st_k[r];
-            *(f32x4_v*)(sQ + at) = st_q[r];
-            sT[(idx / CC) * TPP + 8 * (idx % 4) + idx % CC / 4] = st_t[r];
-            sP[(idx / CC) * TPP + idx % CC] = st_p[r];
-        }
-        if (tid < CC) sA[tid] = st_a, sW[tid] = st_w;
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sS[(4 * kq + r) * KP + 32 * wave + 16 * t + i16] = creg[t][r];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) vreg[r] = st_v[r];
+        for (int r = 0; r < 4; ++r) *(float2*)(sS + (4 * kq + r) * KP + 32 * wave + 2 * i16) = make_float2(creg[0][r], creg[1][r]);
     };
-    auto mfma4 = [](float a, float b, f32x4_v c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); };
 
-    fetch(0);
-    publish();
-    __syncthreads();
-    for (uint32_t c = 0; c < n_chunks; ++c) {
-        const uint32_t t0 = c * CC;
-        fetch(c + 1 < n_chunks ? c + 1 : c); // unconditional (the last chunk refetches itself)
-        // ---- stage 1: rows 16 (wave & 1) .. + 16 of K (waves 0, 1) or Q (waves 2, 3) against S^T, contraction over dk = 32 kq + s
-        f32x4_v acc1 = {0.f, 0.f, 0.f, 0.f};
-        {
-            const float* xr = (wave < 2 ? sK : sQ) + (16 * (wave & 1) + 4 * (i16 & 3) + (i16 >> 2)) * KP + 32 * kq;
-            const float* sr = sS + i16 * KP + 32 * kq;
-            f32x4_v xa[8], sb[8], part[4] = {acc1, acc1, acc1, acc1}; // (four chains: shorter, and nearer to the exact sum than one)
+    auto mfma4 = [](float a, float b, f32x4_v c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); };
+    float off_sum = 0.f; // 0, or NaN behind an output or a state value that is no number
+    const int tb = 16 * (wave & 1);
+    const uint32_t u_keep = homog ? 0u : 0xFFFFFFFFu;
+    // segment 0's outputs (and the plain scan's) are final; segment 1's go to f32 rows that the fix-up finishes
+    uint16_t* const out16 = out + (size_t)hv * head_v_dim + dv_base + i16;
+    const size_t o_stride = homog ? (size_t)num_v_heads * DKC : (size_t)value_dim;
+    float* const o32 = !DUAL ? nullptr : homog ? sp.u + (size_t)hv * DKC + dv_base + i16 - (size_t)sp.mid_chunk * CC * o_stride : sp.o32 + (size_t)hv * head_v_dim + dv_base + i16;
+
+    // The chain, once for the waves of each role: a role's or a lane's condition around loads or stores of the loop makes the compiler wait, at the join, for the chunk's stores and the
+    // next chunk's operands with them (3.2 us a chunk).  Only the last chunk can be ragged.
+    auto walk = [&](auto front_c, auto seg1_c) {
+        constexpr bool FRONT = decltype(front_c)::value, SEG1 = decltype(seg1_c)::value; // stage 1: D or Q S^T
+        struct Operands {
+            f32x4_v x[8], p[2], aw;
+            float u[4], a_c;
+            float2 k[8];
+        };
+        // one chunk's operands, piece by piece.  WHOLE: the chunk has all its tokens (uniform bases, the lane's offset); else rows past the end are the last one (G and U are zero there,
+        // outputs are not stored)
+        const uint32_t x_lane = FRONT ? (uint32_t)((tb + i16) * DKC + 4 * kq) : (uint32_t)(tb + i16) * key_dim + 4 * kq, k_lane = (uint32_t)kq * key_dim + 32 * wave + 2 * i16;
+        auto block = [&](uint32_t c) { return ws + ((size_t)c * num_v_heads + hv) * WS_FLOATS; };
+        auto fetch_x = [&](uint32_t c, Operands& o, int g, auto whole) {
+            if constexpr (FRONT) o.x[g] = *(const f32x4_v*)(block(c) + x_lane + 16 * g);
+            else if constexpr (decltype(whole)::value) o.x[g] = *(const f32x4_v*)(q_norm + (size_t)c * CC * key_dim + hk * DKC + x_lane + 16 * g);
+            else o.x[g] = *(const f32x4_v*)(q_norm + (size_t)min(c * CC + tb + i16, suffix_len - 1) * key_dim + hk * DKC + 4 * kq + 16 * g);
+        };
+        auto fetch_k = [&](uint32_t c, Operands& o, int s2, auto whole) {
+            if constexpr (decltype(whole)::value) o.k[s2] = *(const float2*)(k_norm + (size_t)(c * CC + 4 * s2) * key_dim + hk * DKC + k_lane);
+            else o.k[s2] = *(const float2*)(k_norm + (size_t)min(c * CC + 4 * s2 + kq, suffix_len - 1) * key_dim + hk * DKC + 32 * wave + 2 * i16);
+        };
+        auto fetch_rest = [&](uint32_t c, Operands& o) {
+            const float* w = block(c);
+            if constexpr (FRONT) {
+                const float* ur = u_ws + ((size_t)c * num_v_heads + hv) * CC * head_v_dim + (uint32_t)((tb + 4 * kq) * head_v_dim + dv_base + i16);
 #pragma unroll
-            for (int q = 0; q < 8; ++q) xa[q] = *(const f32x4_v*)(xr + 4 * q), sb[q] = *(const f32x4_v*)(sr + 4 * q);
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) part[e] = mfma4(xa[q][e], sb[q][e], part[e]);
-            acc1 = (part[0] + part[1]) + (part[2] + part[3]);
-        }
-        if (wave < 2) { // R = V - A (K S^T) for tokens v_row + r, value column i16
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sR[(v_row + r) * RPP + i16] = vreg[r] - sA[v_row + r] * acc1[r];
-        }
-        lds_barrier();
-        // ---- stage 2 (waves 0, 1): D = T R for tokens 16 wave + 4 kq + r; contraction over i = 8 kq + s
-        if (wave < 2) {
-            const float* tr = sT + (16 * wave + i16) * TPP + 8 * kq;
-            const f32x4_v ta0 = *(const f32x4_v*)tr, ta1 = *(const f32x4_v*)(tr + 4);
-            f32x4_v d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int s2 = 0; s2 < 8; ++s2) d = mfma4(s2 < 4 ? ta0[s2 & 3] : ta1[s2 & 3], sR[(4 * s2 + kq) * RPP + i16], d);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int t = 16 * wave + 4 * kq + r;
-                sD[t * RPP + i16] = d[r];
-                sDw[t * RPP + i16] = d[r] * sW[t];
+                for (int r = 0; r < 4; ++r) o.u[r] = ur[r * head_v_dim];
+            } else {
+                const float* pr = w + WS_P + (uint32_t)((tb + i16) * CC + 8 * kq);
+                o.p[0] = *(const f32x4_v*)pr, o.p[1] = *(const f32x4_v*)(pr + 4);
             }
-        }
-        lds_barrier();
-        // ---- stage 3 (waves 2, 3): O = A (Q S^T) + P D for tokens 16 (wave - 2) + 4 kq + r
-        if (wave >= 2) {
-            const int tb = 16 * (wave - 2);
-            const float* pr = sP + (tb + i16) * TPP + 8 * kq;
-            const f32x4_v pa0 = *(const f32x4_v*)pr, pa1 = *(const f32x4_v*)(pr + 4);
-            f32x4_v o;
+            o.aw = *(const f32x4_v*)(w + (FRONT ? WS_W : WS_A) + (uint32_t)(tb + 4 * kq));
+            o.a_c = w[WS_A + CC - 1];
+        };
+        auto step_barrier = [&]() { // (waves 2, 3 write nothing in front of the first one: their MFMAs would be moved behind it, after those that they are to run beside)
+            __builtin_amdgcn_sched_barrier(0);
+            lds_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // The next chunk's operands are requested one by one between the MFMAs: 24 requests in a row keep a wave from its first MFMA until the L1 has served them (2.2 us a chunk
+        // instead of 1.46)
+        auto step = [&](uint32_t c, const Operands& o, Operands& next, bool ragged, auto whole) {
+            const uint32_t n = c + 1 < c_end ? c + 1 : c; // unconditional (the last chunk refetches itself)
+            // ---- stage 1
+            f32x4_v part[4] = {}; // (four chains: shorter, and nearer to the exact sum than one)
+            const float* sr = sS + i16 * KP + 4 * kq;
+            f32x4_v sb[8];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o[r] = sA[tb + 4 * kq + r] * acc1[r];
+            for (int g = 0; g < 8; ++g) sb[g] = *(const f32x4_v*)(sr + 16 * g);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int s2 = 0; s2 < 8; ++s2) o = mfma4(s2 < 4 ? pa0[s2 & 3] : pa1[s2 & 3], sD[(8 * kq + s2) * RPP + i16], o);
+            for (int g = 0; g < 8; ++g) {
+                fetch_x(n, next, g, whole);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t t = t0 + tb + 4 * kq + r;
-                if (t < suffix_len) out[(size_t)t * value_dim + hv * head_v_dim + dv_base + i16] = f32_to_bf16(o[r]), off_sum = fmaf(o[r], 0.f, off_sum);
+                for (int e = 0; e < 4; ++e) part[e] = mfma4(o.x[g][e], sb[g][e], part[e]);
+                __builtin_amdgcn_sched_barrier(0);
             }
-        }
-        // ---- stage 4 (all waves): S = A_C S + (D W)^T K for dk tiles 2 wave, 2 wave + 1; contraction over tokens 4 s + kq
-        {
-            const float a_c = sA[CC - 1];
-            float dw[8];
+            f32x4_v acc = (part[0] + part[1]) + (part[2] + part[3]);
+            if constexpr (FRONT) {
 #pragma unroll
-            for (int s2 = 0; s2 < 8; ++s2) dw[s2] = sDw[(4 * s2 + kq) * RPP + i16]; // A operand: row = value column i16
+                for (int r = 0; r < 4; ++r) acc[r] += bits_to_f32(f32_to_bits(o.u[r]) & u_keep); // (last: U is the larger term, and in front of the chain it would be rounded eight times)
+                *(f32x4_v*)(sD + i16 * DP + tb + 4 * kq) = acc;
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const float* kc = sK + 4 * kq * KP + 32 * wave + 16 * t + i16;
-                f32x4_v u = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int s2 = 0; s2 < 8; ++s2) u = mfma4(dw[s2], kc[(16 * (s2 >> 2) + (s2 & 3)) * KP], u);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) creg[t][r] = fmaf(creg[t][r], a_c, u[r]);
+                for (int r = 0; r < 4; ++r) sDw[i16 * DP + 8 * r + tb / 4 + kq] = acc[r] * o.aw[r];
             }
-        }
-        lds_barrier(); // all reads of this chunk's LDS operands are done
-        if (c + 1 < n_chunks) publish();
+            step_barrier();
+            // ---- stage 2
+            const f32x4_v d0 = *(const f32x4_v*)(sDw + i16 * DP + 8 * kq), d1 = *(const f32x4_v*)(sDw + i16 * DP + 8 * kq + 4); // A operand: row = value column i16
+            f32x4_v u[2] = {};
+#pragma unroll
+            for (int s2 = 0; s2 < 8; ++s2) {
+                const float d = s2 < 4 ? d0[s2 & 3] : d1[s2 & 3];
+                fetch_k(n, next, s2, whole);
+                u[0] = mfma4(d, o.k[s2].x, u[0]), u[1] = mfma4(d, o.k[s2].y, u[1]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) creg[t][r] = fmaf(creg[t][r], o.a_c, u[t][r]);
+            publish(); // (every wave has read the old state: the barrier above)
+            __builtin_amdgcn_sched_barrier(0);
+            fetch_rest(n, next);
+            // ---- stage 3
+            if constexpr (!FRONT) {
+                const f32x4_v e0 = *(const f32x4_v*)(sD + i16 * DP + 8 * kq), e1 = *(const f32x4_v*)(sD + i16 * DP + 8 * kq + 4);
+                f32x4_v y = o.aw * acc;
+#pragma unroll
+                for (int s2 = 0; s2 < 8; ++s2) y = mfma4(o.p[s2 >> 2][s2 & 3], s2 < 4 ? e0[s2 & 3] : e1[s2 & 3], y);
+                const uint32_t t = c * CC + tb + 4 * kq;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (ragged && t + r >= suffix_len) continue;
+                    if constexpr (SEG1) o32[(size_t)(t + r) * o_stride] = y[r];
+                    else out16[(size_t)(t + r) * value_dim] = f32_to_bf16(y[r]), off_sum = fmaf(y[r], 0.f, off_sum);
+                }
+            }
+            step_barrier();
+        };
+        typedef std::integral_constant<bool, true> yes;
+        typedef std::integral_constant<bool, false> no;
+        Operands even, odd;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) fetch_x(c_begin, even, g, no());
+#pragma unroll
+        for (int s2 = 0; s2 < 8; ++s2) fetch_k(c_begin, even, s2, no());
+        fetch_rest(c_begin, even);
+        publish();
         lds_barrier();
+        const uint32_t full = min(c_end, suffix_len / CC); // chunks [c_begin, full) have all their tokens
+        uint32_t c = c_begin;
+        for (; c + 2 < full; c += 2) step(c, even, odd, false, yes()), step(c + 1, odd, even, false, yes());
+        for (; c < c_end; ++c) { // at most three
+            step(c, even, odd, c >= full, no());
+            even = odd;
+        }
+    };
+    typedef std::integral_constant<bool, true> yes;
+    typedef std::integral_constant<bool, false> no;
+    if (DUAL && seg1) {
+        if (wave < 2) walk(yes(), std::integral_constant<bool, DUAL>());
+        else walk(no(), std::integral_constant<bool, DUAL>());
+    } else if (wave < 2) walk(yes(), no());
+    else walk(no(), no());
+    if constexpr (DUAL) {
+        float* sfin = homog ? sp.h_end + ((size_t)hv * DKC + dv_base + 4 * kq) * DKC + 32 * wave + 2 * i16 : (seg1 ? sp.z_end : sp.mid_state) + s_at;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) *(float2*)(sfin + (size_t)r * DKC) = make_float2(creg[0][r], creg[1][r]);
+        return;
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) off_sum = fmaf(creg[t][r], 0.f, off_sum);
-    uint32_t* s_off = (uint32_t*)sR; // (read for the last time in front of the last barrier)
     const bool off = __ballot(!(off_sum == 0.f)) != 0;
     if (lane == 0) s_off[wave] = off;
     lds_barrier();
     if (s_off[0] | s_off[1] | s_off[2] | s_off[3]) { // the recurrence from the state in memory, 16 lanes a value column
         __syncthreads(); // (every wave's own outputs have been written: those below replace them)
+        const uint32_t conv_dim = 2 * key_dim + value_dim;
+        // (v_row_stride != 0: `in_proj` is the out-of-place conv buffer, rows of conv_dim channels in the same q | k | v order)
+        const size_t total_proj_dim = v_row_stride ? (size_t)v_row_stride : (size_t)conv_dim + value_dim + 2 * num_v_heads;
         const uint32_t col = tid >> 4, part = tid & 15;
         float* srow = state + ((size_t)hv * head_v_dim + dv_base + col) * DKC + 8 * part;
         float sv[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) sv[e] = srow[e];
         for (uint32_t t = 0; t < suffix_len; ++t) {
-            const float* w = ws + ((size_t)(t / CC) * num_v_heads + hv) * WS_FLOATS + 2 * CC * CC + 2 * CC + t % CC;
+            const float* w = ws + ((size_t)(t / CC) * num_v_heads + hv) * WS_FLOATS + WS_DECAY + t % CC;
             const float *kr = k_norm + (size_t)t * key_dim + hk * DKC + 8 * part, *qr = q_norm + (size_t)t * key_dim + hk * DKC + 8 * part;
             const float a = w[0], b = w[CC], v = bf16_to_f32(in_proj[(size_t)t * total_proj_dim + 2 * key_dim + hv * head_v_dim + dv_base + col]);
             float sk = 0.f, o = 0.f;
@@ -463,209 +596,8 @@ __global__ void __launch_bounds__(256) dn_chunk_scan_mfma_kernel(const float* q_
         return;
     }
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sbase[(size_t)r * DKC + 16 * t] = creg[t][r];
+    for (int r = 0; r < 4; ++r) *(float2*)(state + s_at + (size_t)r * DKC) = make_float2(creg[0][r], creg[1][r]);
 }
-
-// The split scan (ScanSplit).  grid (2 Dv / 16, Hv), 512 threads = two groups of the plain kernel's four waves; the stage code is the plain kernel's.
-//   workgroups [0, Dv / 16) of a head: segment 0, chunks [0, mid): group 0 = the value tile from the carried state, group 1 only stages operands;
-//   the others:                        segment 1, chunks [mid, n): group 0 = the value tile from a zero state, group 1 = the homogeneous tile (identity, v = 0).
-// Shared LDS operands K, Q, T, P, A, W: group 0's threads fetch and publish K and T, group 1's Q and P (pointer selects, no branch: a role-dependent branch
-// around global loads or stores makes the compiler wait for every outstanding load at the join -- the next chunk's operands fetched ahead: 2.5 -> 3.8 us per
-// chunk in the first form).  Every output goes to an f32 row of its role's buffer AND, rounded, to the output row, through one store path.
-__global__ void __launch_bounds__(512) dn_chunk_scan_dual_kernel(const float* q_norm, const float* k_norm, const uint16_t* in_proj, const float* ws, const float* state,
-                                                                 uint16_t* out, uint32_t num_v_heads, uint32_t num_k_heads, uint32_t head_v_dim, uint32_t key_dim, uint32_t value_dim,
-                                                                 uint32_t suffix_len, ScanSplit sp, uint32_t v_row_stride) {
-    constexpr int DVT = 16, TPP = 36, RPP = 18;
-    extern __shared__ __attribute__((aligned(16))) float dual_smem[];
-    float* sK = dual_smem;                 // [CC][KP]
-    float* sQ = sK + CC * KP;              // [CC][KP]
-    float* sT = sQ + CC * KP;              // [CC][TPP]
-    float* sP = sT + CC * TPP;             // [CC][TPP]
-    float* sA = sP + CC * TPP;             // [CC]
-    float* sW = sA + CC;                   // [CC]
-    float* grp_base = sW + CC;             // per group: sS [DVT][KP], sR / sD / sDw [CC][RPP]
-    constexpr int GRP_FLOATS = DVT * KP + 3 * CC * RPP;
-    const int tid = threadIdx.x, grp = tid >> 8, ltid = tid & 255, lane = ltid & 63, wave = ltid >> 6, i16 = lane & 15, kq = lane >> 4;
-    float* sS = grp_base + grp * GRP_FLOATS;
-    float* sR = sS + DVT * KP;
-    float* sD = sR + CC * RPP;
-    float* sDw = sD + CC * RPP;
-    uint32_t hv = blockIdx.y, tile = blockIdx.x;
-    { // XCD-aware numbering as in the plain kernel: a head's workgroups share one L2
-        const uint32_t nx = gridDim.x, total = nx * gridDim.y, lin = blockIdx.x + nx * blockIdx.y;
-        if (total % 8 == 0) {
-            const uint32_t pair = (lin % 8) * (total / 8) + lin / 8;
-            hv = pair / nx, tile = pair % nx;
-        }
-    }
-    const uint32_t tiles_v = head_v_dim / DVT;
-    const bool seg1 = tile >= tiles_v;
-    if (seg1) tile -= tiles_v;
-    const bool active = seg1 || grp == 0;   // group 1 of a segment-0 workgroup only stages operands
-    const bool homog = seg1 && grp == 1;
-    const uint32_t dv_base = tile * DVT, hk = hv / (num_v_heads / num_k_heads);
-    const uint32_t conv_dim = 2 * key_dim + value_dim;
-    // (v_row_stride != 0: `in_proj` is the out-of-place conv buffer, rows of conv_dim channels in the same q | k | v order)
-    const size_t total_proj_dim = v_row_stride ? (size_t)v_row_stride : (size_t)conv_dim + value_dim + 2 * num_v_heads;
-    const uint32_t n_chunks = (suffix_len + CC - 1) / CC;
-    const uint32_t c_begin = seg1 ? sp.mid_chunk : 0u, c_end = seg1 ? n_chunks : sp.mid_chunk;
-    // f32 output row of token t = o32[t * o_stride] (real tiles: the shared [T][Hv Dv] buffer; homogeneous tile: u, whose row 0 is token 32 mid)
-    const size_t o_stride = homog ? (size_t)num_v_heads * DKC : (size_t)value_dim;
-    float* o32 = homog ? sp.u + (size_t)hv * DKC + dv_base + i16 - (size_t)sp.mid_chunk * CC * o_stride : sp.o32 + (size_t)hv * head_v_dim + dv_base + i16;
-    // ... and, rounded, to the bf16 output row as well: final for segment 0 (its outputs need nothing more), overwritten by the fix-up for segment 1 (whose two
-    // groups write the same cells: Dv = Dk) -- one store path for every role, and the fix-up has no conversion pass over segment 0
-    uint16_t* out16 = out + (size_t)hv * head_v_dim + dv_base + i16;
-    const uint32_t store_end = active ? suffix_len : 0u;
-    const uint32_t v_keep = (active && !homog) ? 0xFFFFFFFFu : 0u; // the homogeneous rows have zero values
-
-    // state in accumulator layout (plain kernel): creg[t][r] = S[dv = 4 kq + r][dk = 16 (2 wave + t) + i16]
-    f32x4_v creg[2];
-    {
-        const float* sinit = state + ((size_t)hv * head_v_dim + dv_base + 4 * kq) * DKC + 32 * wave + i16;
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                creg[t][r] = (!seg1 && grp == 0) ? sinit[(size_t)r * DKC + 16 * t] : (homog && dv_base + 4 * kq + r == (uint32_t)(32 * wave + 16 * t + i16)) ? 1.0f : 0.0f;
-    }
-
-    // ---- operand staging: this group's half of the shared operands (K + T | Q + P), A / W, its value rows
-    const float* kq_src = grp ? q_norm : k_norm;
-    float* kq_dst = grp ? sQ : sK;
-    float* tp_dst = grp ? sP : sT;
-    const uint32_t tp_off = grp ? CC * CC : 0;
-    f32x4_v st_kq[4];
-    float st_tp[4], st_a = 0.f, st_w = 0.f, st_v[4];
-    const int v_row = 16 * (wave & 1) + 4 * kq;
-    auto fetch = [&](uint32_t c) {
-        const uint32_t t0 = c * CC;
-        const float* w_t = ws + ((size_t)c * num_v_heads + hv) * WS_FLOATS;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int idx = ltid + 256 * r, t = idx / (DKC / 4), c4 = idx % (DKC / 4);
-            const bool live = t0 + t < suffix_len;
-            const size_t tok = live ? t0 + t : suffix_len - 1; // clamped + zeroed: unconditional loads stay countable
-            const f32x4_v zero = {0.f, 0.f, 0.f, 0.f};
-            const f32x4_v xv = *(const f32x4_v*)(kq_src + tok * key_dim + hk * DKC + c4 * 4);
-            st_kq[r] = live ? xv : zero;
-            st_tp[r] = w_t[tp_off + idx];
-        }
-        st_a = w_t[2 * CC * CC + (ltid & (CC - 1))], st_w = w_t[2 * CC * CC + CC + (ltid & (CC - 1))];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const bool live = t0 + v_row + r < suffix_len;
-            const float vv = bf16_to_f32(in_proj[(size_t)(live ? t0 + v_row + r : suffix_len - 1) * total_proj_dim + 2 * key_dim + hv * head_v_dim + dv_base + i16]);
-            st_v[r] = live ? vv : 0.f;
-        }
-    };
-    float vreg[4] = {0.f, 0.f, 0.f, 0.f};
-    auto publish = [&]() {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int idx = ltid + 256 * r, t = idx / (DKC / 4), c4 = idx % (DKC / 4);
-            *(f32x4_v*)(kq_dst + t * KP + c4 * 4) = st_kq[r];
-            tp_dst[(idx / CC) * TPP + idx % CC] = st_tp[r];
-        }
-        if (tid < CC) sA[tid] = st_a, sW[tid] = st_w;
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sS[(4 * kq + r) * KP + 32 * wave + 16 * t + i16] = creg[t][r];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) vreg[r] = bits_to_f32(f32_to_bits(st_v[r]) & v_keep); // (masked here, not at the load: a role condition in `fetch` puts the loads behind branches)
-    };
-    auto mfma4 = [](float a, float b, f32x4_v c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); };
-
-    fetch(c_begin);
-    publish();
-    __syncthreads();
-    for (uint32_t c = c_begin; c < c_end; ++c) {
-        const uint32_t t0 = c * CC;
-        fetch(c + 1 < c_end ? c + 1 : c); // unconditional (the last chunk refetches itself)
-        // ---- stage 1: rows 16 (wave & 1) .. + 16 of K (waves 0, 1) or Q (waves 2, 3) against S^T
-        f32x4_v acc1 = {0.f, 0.f, 0.f, 0.f};
-        if (active) {
-            const float* xr = (wave < 2 ? sK : sQ) + (16 * (wave & 1) + i16) * KP + 32 * kq;
-            const float* sr = sS + i16 * KP + 32 * kq;
-            f32x4_v xa[8], sb[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) xa[q] = *(const f32x4_v*)(xr + 4 * q), sb[q] = *(const f32x4_v*)(sr + 4 * q);
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc1 = mfma4(xa[q][e], sb[q][e], acc1);
-            if (wave < 2) { // R = V - A (K S^T)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) sR[(v_row + r) * RPP + i16] = vreg[r] - sA[v_row + r] * acc1[r];
-            }
-        }
-        lds_barrier();
-        // ---- stage 2 (waves 0, 1): D = T R
-        if (active && wave < 2) {
-            const float* tr = sT + (16 * wave + i16) * TPP + 8 * kq;
-            const f32x4_v ta0 = *(const f32x4_v*)tr, ta1 = *(const f32x4_v*)(tr + 4);
-            f32x4_v d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int s2 = 0; s2 < 8; ++s2) d = mfma4(s2 < 4 ? ta0[s2 & 3] : ta1[s2 & 3], sR[(8 * kq + s2) * RPP + i16], d);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int t = 16 * wave + 4 * kq + r;
-                sD[t * RPP + i16] = d[r];
-                sDw[t * RPP + i16] = d[r] * sW[t];
-            }
-        }
-        lds_barrier();
-        // ---- stage 3 (waves 2, 3): O = A (Q S^T) + P D
-        if (active && wave >= 2) {
-            const int tb = 16 * (wave - 2);
-            const float* pr = sP + (tb + i16) * TPP + 8 * kq;
-            const f32x4_v pa0 = *(const f32x4_v*)pr, pa1 = *(const f32x4_v*)(pr + 4);
-            f32x4_v o;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o[r] = sA[tb + 4 * kq + r] * acc1[r];
-#pragma unroll
-            for (int s2 = 0; s2 < 8; ++s2) o = mfma4(s2 < 4 ? pa0[s2 & 3] : pa1[s2 & 3], sD[(8 * kq + s2) * RPP + i16], o);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t t = t0 + tb + 4 * kq + r;
-                if (t < store_end) {
-                    o32[(size_t)t * o_stride] = o[r];
-                    out16[(size_t)t * value_dim] = f32_to_bf16(o[r]);
-                }
-            }
-        }
-        // ---- stage 4: S = A_C S + (D W)^T K
-        if (active) {
-            const float a_c = sA[CC - 1];
-            float dw[8];
-#pragma unroll
-            for (int s2 = 0; s2 < 8; ++s2) dw[s2] = sDw[(8 * kq + s2) * RPP + i16];
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) creg[t][r] *= a_c;
-                const float* kc = sK + (8 * kq) * KP + 32 * wave + 16 * t + i16;
-#pragma unroll
-                for (int s2 = 0; s2 < 8; ++s2) creg[t] = mfma4(dw[s2], kc[s2 * KP], creg[t]);
-            }
-        }
-        lds_barrier();
-        if (c + 1 < c_end) publish();
-        lds_barrier();
-    }
-    if (active) {
-        float* sfin = homog  ? sp.h_end + ((size_t)hv * DKC + dv_base + 4 * kq) * DKC + 32 * wave + i16
-                      : seg1 ? sp.z_end + ((size_t)hv * head_v_dim + dv_base + 4 * kq) * DKC + 32 * wave + i16
-                             : sp.mid_state + ((size_t)hv * head_v_dim + dv_base + 4 * kq) * DKC + 32 * wave + i16;
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sfin[(size_t)r * DKC + 16 * t] = creg[t][r];
-    }
-}
-constexpr size_t kDualLdsBytes = (size_t)(2 * CC * KP + 2 * CC * 36 + 2 * CC + 2 * (16 * KP + 3 * CC * 18)) * sizeof(float);
 
 // The S_mid terms of a split scan (see ScanSplit).  grid (tok_blocks + Dk / 16, Hv), 4 waves;
 // v_mfma_f32_16x16x4_f32 with the operand layout of the scan (lane l: row / column l % 16, contraction indices 32 (l / 16) + s over 32 steps: a lane's
@@ -784,31 +716,30 @@ static uzu_status prefill_chunked(hipStream_t s, float* q_norm, float* k_norm, c
     const uint32_t n_chunks = (suffix_len + CC - 1) / CC;
     const uint16_t* v_rows = prep && prep->conv_rows ? prep->conv_rows : in_proj; // where the scans read the conv'd v channels
     const uint32_t v_stride = prep && prep->conv_rows ? 2 * key_dim + value_dim : 0u;
+    float* const u_ws = workspace + (size_t)n_chunks * num_v_heads * WS_FLOATS; // U
     if (prep)
         UZU_PROPAGATE(launch_check([&] {
             hipLaunchKernelGGL(dn_chunk_prep_kernel<true>, dim3(n_chunks, num_v_heads), dim3(256), 0, s, (const float*)nullptr, (const float*)nullptr, (const float*)nullptr,
-                               (const float*)nullptr, workspace, num_v_heads, num_k_heads, key_dim, suffix_len, in_proj, prep->a_log, prep->dt_bias, q_norm, k_norm, value_dim, prep->conv_rows,
-                               prep->conv_state);
+                               (const float*)nullptr, workspace, u_ws, num_v_heads, num_k_heads, head_v_dim, key_dim, suffix_len, in_proj, prep->a_log, prep->dt_bias, q_norm, k_norm, value_dim,
+                               prep->conv_rows, prep->conv_state);
         }, "delta_net_chunk_prep_fused"));
     else
         UZU_PROPAGATE(launch_check([&] {
-            hipLaunchKernelGGL(dn_chunk_prep_kernel<false>, dim3(n_chunks, num_v_heads), dim3(256), 0, s, (const float*)q_norm, (const float*)k_norm, beta, decay, workspace,
-                               num_v_heads, num_k_heads, key_dim, suffix_len, (const uint16_t*)nullptr, (const float*)nullptr, (const float*)nullptr, (float*)nullptr,
+            hipLaunchKernelGGL(dn_chunk_prep_kernel<false>, dim3(n_chunks, num_v_heads), dim3(256), 0, s, (const float*)q_norm, (const float*)k_norm, beta, decay, workspace, u_ws,
+                               num_v_heads, num_k_heads, head_v_dim, key_dim, suffix_len, in_proj, (const float*)nullptr, (const float*)nullptr, (float*)nullptr,
                                (float*)nullptr, value_dim, (const uint16_t*)nullptr, (float*)nullptr);
         }, "delta_net_chunk_prep"));
     ScanSplit sp{};
     sp.mid_chunk = value_dim == num_v_heads * head_v_dim ? split_mid_chunk(n_chunks, head_v_dim) : 0u;
-    static LdsLimit dual_lds;
     static LdsLimit fix_lds;
-    if (sp.mid_chunk && !(raise_lds_limit(dual_lds, (const void*)dn_chunk_scan_dual_kernel, kDualLdsBytes) && raise_lds_limit(fix_lds, (const void*)dn_chunk_fixup_kernel, kFixLdsBytes)))
-        sp.mid_chunk = 0; // (74 KB / 68 KB of LDS per workgroup)
+    if (sp.mid_chunk && !raise_lds_limit(fix_lds, (const void*)dn_chunk_fixup_kernel, kFixLdsBytes)) sp.mid_chunk = 0; // (68 KB of LDS per workgroup)
     if (!sp.mid_chunk)
         return launch_check([&] {
-            hipLaunchKernelGGL(dn_chunk_scan_mfma_kernel, dim3(head_v_dim / 16, num_v_heads), dim3(256), 0, s, q_norm, k_norm, v_rows, workspace, state, out,
-                               num_v_heads, num_k_heads, head_v_dim, key_dim, value_dim, suffix_len, v_stride);
+            hipLaunchKernelGGL(dn_chunk_scan_kernel<false>, dim3(head_v_dim / 16, num_v_heads), dim3(256), 0, s, q_norm, k_norm, v_rows, (const float*)workspace, (const float*)u_ws,
+                               (const float*)state, state, out, num_v_heads, num_k_heads, head_v_dim, key_dim, value_dim, suffix_len, sp, v_stride);
         }, "delta_net_chunk_scan");
-    { // the split's pieces live behind the T / P matrices (delta_net_chunk_workspace_bytes)
-        float* w = workspace + (size_t)n_chunks * num_v_heads * WS_FLOATS;
+    { // the split's pieces live behind U (delta_net_chunk_workspace_bytes)
+        float* w = u_ws + (size_t)n_chunks * CC * value_dim;
         sp.mid_state = w, w += (size_t)value_dim * DKC;
         sp.z_end = w, w += (size_t)value_dim * DKC;
         sp.h_end = w, w += (size_t)num_v_heads * DKC * DKC;
@@ -816,8 +747,8 @@ static uzu_status prefill_chunked(hipStream_t s, float* q_norm, float* k_norm, c
         sp.u = w;
     }
     UZU_PROPAGATE(launch_check([&] {
-        hipLaunchKernelGGL(dn_chunk_scan_dual_kernel, dim3(2 * (head_v_dim / 16), num_v_heads), dim3(512), kDualLdsBytes, s, q_norm, k_norm, v_rows, workspace,
-                           (const float*)state, out, num_v_heads, num_k_heads, head_v_dim, key_dim, value_dim, suffix_len, sp, v_stride);
+        hipLaunchKernelGGL(dn_chunk_scan_kernel<true>, dim3(2 * (head_v_dim / 16), num_v_heads), dim3(512), 0, s, q_norm, k_norm, v_rows, (const float*)workspace, (const float*)u_ws,
+                           (const float*)state, state, out, num_v_heads, num_k_heads, head_v_dim, key_dim, value_dim, suffix_len, sp, v_stride);
     }, "delta_net_chunk_scan_dual"));
     const uint32_t t_mid = sp.mid_chunk * CC, t2 = suffix_len - t_mid;
     return launch_check([&] {
