@@ -100,6 +100,24 @@ def test_linear_f32_from_three_bf16_parts(hip_ctx, rows, n, k, act):
     assert (np.abs(got - want) <= bound + 2.0 ** -23 * (np.abs(want) + np.abs(res))).all()
 
 
+@pytest.mark.parametrize("bf16", [0, 1])
+@pytest.mark.parametrize("rows,n,k,act", [(65, 129, 1024, 0), (129, 385, 4096, 1), (20, 64, 1152, 0), (513, 2049, 512, 0), (1030, 3900, 128, 1), (2048, 2048, 320, 0), (700, 1030, 1088, 0)])
+def test_linear_on_eight_waves_a_tile(hip_ctx, rows, n, k, act, bf16):
+    """At most a 128 x 128 tile a CU (csrc/k_linear_mfma.hip: eight_wave_splits): whole and cut into two to eight shares with uneven counts of k-steps, fewer steps than buffers, ragged last
+    tiles, all 256 tiles.  Against 64 bits, with the bound of the products above (bf16 products: k of them)."""
+    rng = np.random.default_rng(rows + n + k)
+    x = rng.standard_normal((rows, k), dtype=np.float32)
+    w, b, res = O.to_bf16(rng.standard_normal((n, k), dtype=np.float32)), O.to_bf16(rng.standard_normal(n)), rng.standard_normal((rows, n), dtype=np.float32)
+    got = linear(hip_ctx, x, w, b, res, act=act, bf16=bf16)
+    xr = O.to_bf16(x).astype(np.float64) if bf16 else x.astype(np.float64)
+    lin = xr @ w.T.astype(np.float64) + b
+    bound = 4 * 2.0 ** -24 * np.sqrt((1 if bf16 else 3) * k) * (np.abs(xr) @ np.abs(w.T.astype(np.float64)) + np.abs(b))
+    if act:
+        bound = 2 * np.maximum(lin, 0) * bound + bound ** 2 + 2.0 ** -23 * lin ** 2
+    want = (np.maximum(lin, 0) ** 2 if act else lin) + res
+    assert (np.abs(got - want) <= bound + 2.0 ** -23 * (np.abs(want) + np.abs(res))).all()
+
+
 @pytest.mark.parametrize("rows,n,k", [(300, 700, 2048), (1025, 4100, 128), (17, 70, 256), (600, 4100, 1024)])
 @pytest.mark.parametrize("power", [-118, -123])
 def test_linear_f32_parts_of_tiny_numbers(hip_ctx, rows, n, k, power):

@@ -35,3 +35,12 @@ def test_silu_from_a_quick_quotient_is_the_exact_one():
         subprocess.run(["g++", "-O2", "-ffp-contract=off", "-o", exe, os.path.join(ROOT, "tests", "host", "silu_near_check.cpp"), "-lm"], check=True)
         out = subprocess.check_output([exe]).decode()
     assert out.strip().endswith(" 0 bad") and int(out.split()[0]) == 65536 * 33, out
+
+
+def test_tile_order_visits_every_tile_once_and_balances_the_xcds():
+    """uzu_amd/csrc/gemm_tile_order.h (workgroup id -> output tile of the large-tile products): exhaustive host check over 48 x 160 tile counts."""
+    with tempfile.TemporaryDirectory() as td:
+        exe = os.path.join(td, "tile_order_check")
+        subprocess.run(["g++", "-O2", "-std=c++17", "-o", exe, os.path.join(ROOT, "tests", "host", "tile_order_check.cpp")], check=True)
+        out = subprocess.check_output([exe]).decode()
+    assert out.strip().endswith(" 0 bad"), out

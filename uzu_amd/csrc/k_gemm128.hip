@@ -14,7 +14,7 @@
 //   * Every global load is unconditional (rows / columns / steps clamped into range) and prefetched into a register
 //     ring; the loop is unrolled by the ring depth so that all indices are static (vmcnt waits stay counted).
 //   * int4 in groups of 128 takes the first two of the three forms (gemm128_form) with its operands by LDS DMA instead: k_gemm_dma.hip.
-//   * Tiles are numbered in 8 x 8 super-tiles per XCD (tile_map) so that the ~64 workgroups an XCD runs at a time share
+//   * Tiles are numbered in blocks of 8 x 8 per XCD (gemm_tile_order.h) so that the ~64 workgroups an XCD runs at a time share
 //     their activation and weight panels in its L2; few-tile shapes split K over gridDim.y with f32 partial tiles and
 //     a fixed-order reduction.  bf16 results leave through LDS as 16-byte row segments.
 #include <stdlib.h>
@@ -24,7 +24,7 @@
 #include "device_utils.h"
 #include "gemm128_epilogue.h"
 #include "gemm_convert.h"
-#include "gemm_tile_map.h"
+#include "gemm_tile_order.h"
 #include "kernels.h"
 #include "uzu_math.h"
 
@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(256) gemm_prepass_kernel(MatmulParams p, float
 }
 
 // ---------------------------------------------------------------------------------------------- main kernel
-// grid (8 S ceil(Q / 8), splits), see tile_map().  GS = k-steps per quant group (1, 2, 4 <=> group 64, 128, 256).
+// grid (tiles, splits), see gemm_tile_order.h.  GS = k-steps per quant group (1, 2, 4 <=> group 64, 128, 256).
 //
 // PP ("ping-pong", round 5): ONE 512-thread workgroup per CU works on a 128 x 256 tile: two halves of four waves, each half the 128 x 128
 // tile of the 256-thread form (same k order, same fold -> bit-identical results) over ONE activation tile in LDS that all eight waves
@@ -162,12 +162,12 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
     bool live;
     if (PP) { // the tile map runs over PAIRS of column tiles; half h takes column tile 2 pair + h of the same row block
         uint32_t pr;
-        if (!gemm_tile_of_block(blockIdx.x, m_tiles, (n_tiles + 1) / 2, &m_t, &pr)) return;
+        if (!tile_of_block(blockIdx.x, m_tiles, (n_tiles + 1) / 2, &m_t, &pr)) return;
         n_t = 2 * pr + half;
         live = n_t < n_tiles;
         if (!live) n_t = n_tiles - 1; // odd tile count: the idle half walks its neighbour's tile for the barriers' sake and stores nothing
     } else {
-        live = gemm_tile_of_block(blockIdx.x, m_tiles, n_tiles, &m_t, &n_t);
+        live = tile_of_block(blockIdx.x, m_tiles, n_tiles, &m_t, &n_t);
         if (!live) return;
     }
     const uint32_t vblock = PP ? blockIdx.x * 2 + half : blockIdx.x;
@@ -814,7 +814,7 @@ uzu_status gemm_q_mfma128(hipStream_t s, const MatmulParams& p, int num_cus, voi
         if (st != UZU_OK || splits == 1) return st;
         return gemm_split_finish(s, p, partials, splits);
     }
-    const dim3 grid(form == 1 ? gemm_grid_x(m_tiles, (n_tiles + 1) / 2) : gemm_grid_x(m_tiles, n_tiles), splits), block(form ? 512 : 256);
+    const dim3 grid(form == 1 ? tile_order_grid(m_tiles, (n_tiles + 1) / 2) : tile_order_grid(m_tiles, n_tiles), splits), block(form ? 512 : 256);
 #define UZU_LAUNCH(B, GSV)                                                                                                                                            \
     st = form == 2 ? launch_check([&] { hipLaunchKernelGGL((gemm_q_mfma128_kernel<B, GSV, 2>), grid, block, 0, s, p, rowsum_in, coef_in, partials, g_gemm128_dbg); }, "gemm_q_mfma128ws") \
        : form == 1 ? launch_check([&] { hipLaunchKernelGGL((gemm_q_mfma128_kernel<B, GSV, 1>), grid, block, 0, s, p, rowsum_in, coef_in, partials, g_gemm128_dbg); }, "gemm_q_mfma128pp") \

@@ -12,7 +12,7 @@
 #include "device_utils.h"
 #include "gemm128_epilogue.h"
 #include "gemm_convert.h"
-#include "gemm_tile_map.h"
+#include "gemm_tile_order.h"
 #include "kernels.h"
 #include "uzu_math.h"
 
@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(64 * NW, 2) gemm_q4_dma_kernel(MatmulParams p,
     const bool gated = p.act_mul != 0;
     const uint32_t H = N / 2, m_tiles = (M + DM - 1) / DM, n_tiles = gated ? (H + 32 * NWN - 1) / (32 * NWN) : (N + 64 * NWN - 1) / (64 * NWN);
     uint32_t m_t, n_t;
-    if (!gemm_tile_of_block(blockIdx.x, m_tiles, n_tiles, &m_t, &n_t)) return;
+    if (!tile_of_block(blockIdx.x, m_tiles, n_tiles, &m_t, &n_t)) return;
     const uint32_t m0 = m_t * DM, n0 = n_t * 64 * NWN;
     const uint32_t z = blockIdx.y, Gz = G / gridDim.y, g_lo = z * Gz;
     const uint32_t flip = p.signed_codes ? 0x88888888u : 0u; // the unsigned code u of bf16(16 + u)
@@ -206,7 +206,7 @@ bool gemm_q4_dma_supported(const MatmulParams& p) {
 }
 uint32_t gemm_q4_dma_blocks(uint32_t m, uint32_t n, bool gated, bool wide) {
     const uint32_t m_tiles = (m + DM - 1) / DM, cols = wide ? 256 : 128, n_tiles = gated ? (n / 2 + cols / 2 - 1) / (cols / 2) : (n + cols - 1) / cols;
-    return gemm_grid_x(m_tiles, n_tiles);
+    return tile_order_grid(m_tiles, n_tiles);
 }
 uzu_status gemm_q4_dma(hipStream_t s, const MatmulParams& p, const uint16_t* pairs, const float* rowsum, const float* coef, float* partials, uint32_t splits, bool wide) {
     const dim3 grid(gemm_q4_dma_blocks(p.m, p.n, p.act_mul != 0, wide), splits);

@@ -9,9 +9,11 @@
 // The next k-step's global loads are issued before the MFMAs of the current one and stored behind them (one LDS buffer, two barriers per k-step).
 // An MFMA lane holds column n = lane % 32 of a block and rows (i & 3) + 8 (i >> 2) + 4 (lane / 32): a row's 32 columns leave as one 128-byte segment.
 // grid.z batches independent products of one shape (the per-head products of the latent attention).
+#include <algorithm>
+
 #include "device_utils.h"
 #include "gemm_convert.h"
-#include "gemm_tile_map.h"
+#include "gemm_tile_order.h"
 #include "kernels.h"
 #include "kernels_stream32.h"
 #include "stream32_epilogue.h"
@@ -170,15 +172,16 @@ __global__ void __launch_bounds__(256, MB * NB == 4 && KIND != kEpilogueFull ? 3
 // ---- prompt-sized products: both operands as bf16 rows in memory, fetched straight into LDS
 // The activations are rounded to bf16 once, in front (linear_bf16_rows, or the producing kernel), instead of by every column of tiles: the kernel above spends its
 // k-step on that conversion and on the operands' way through registers (2048 x 7712 x 2048: 158 us, 409 TFLOP/s), with one buffer and two barriers per k-step.
-// Here a workgroup of four waves (2 x 2, a wave 32 MB x 64 outputs) takes its 64-deep k-steps by global_load_lds_dwordx4 (1 KB a wave-instruction, no registers).
-// A staged row is 64 k = 128 bytes = eight 16-byte chunks; chunk c of row r lies in slot c ^ (r & 7) -- the lane picks the chunk it fetches, the DMA stores lane by
-// lane -- so the eight rows that a quarter-wave reads at one k fall on eight different slots.
+// Here a workgroup of WM x WN waves, a wave 32 MB x 64 outputs, takes its 64-deep k-steps by global_load_lds_dwordx4 (1 KB a wave-instruction, no registers).
+// A staged row is 64 k = 128 bytes = eight 16-byte chunks; chunk c of row r lies in slot c ^ (r / 2 & 7) -- the lane picks the chunk it fetches, the DMA stores lane by
+// lane -- so the sixteen rows that a quarter-wave reads at one k fall on the sixteen different 16-byte slots of two rows.
 // What bounds it is the wait for a k-step's operands, so the forms differ in who covers it (measured, us, conversion included):
 //   * 128-row tiles, ONE buffer, 32 KB: four workgroups per CU cover each other.  Best from two tiles a CU on: 2048 x 16384 x 2048 183 (two buffers 211),
 //     eight buckets of 4096 rows x 4096 x 2048 105 (111), x 2048 59 (67);
 //   * 128-row tiles, two buffers, two workgroups per CU, the next step on its way during a step: 513 x 8192 x 2048 45 (one buffer 52);
-//   * 64-row tiles, two buffers, three workgroups per CU: at most a 128-row tile a CU: 2048 x 2048 x 4096 58 (128-row tiles 64), 1000 x 3856 x 1024 27 (32).
-// Wider tiles (256 x 128), 32-deep steps and a third buffer were all slower.
+//   * up to a 128-row tile a CU: eight waves on it (eight_wave_splits), or 64-row tiles of four waves, two buffers, three workgroups per CU.
+// 256 columns or rows a workgroup, eight waves of 64 x 64 or 128 x 64, were slower from two tiles a CU on, too (2048 x 7712 x 2048 97, 94 and 81 us against 82; eight buckets of 512 rows
+// x 4096 x 2048 122 .. 136 against 108), as were 32-deep steps.
 constexpr int DN = 128;
 
 // PIECES KB-pieces from base + v[i] (16 bytes a lane) to dst + 1024 i + 16 lane
@@ -244,13 +247,14 @@ __device__ __forceinline__ void split_repair(f32x16_t& acc, const uint16_t* xb, 
 constexpr int kEpilogueGated = 16; // grouped experts: the weight rows are [up ; gate], the result act(gate, up) as bf16 rows (GatedRows)
 
 // parts: 1, or 3 for operand rows [lo | mid | hi].  partials (MB 1, not GROUPED): blockIdx.z takes its share of the k-steps and leaves its sums there, f32 [z][rows][n].
-template <int MB, int STAGES, bool GROUPED, int KIND, uint32_t parts>
-__global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, const uint16_t* xb, uint32_t ldxb, GatedRows gr, float* partials) {
+// WM x WN waves, a wave 32 MB x 64 outputs
+template <int WM, int WN, int MB, int STAGES, bool GROUPED, int KIND, uint32_t parts>
+__global__ void __launch_bounds__(64 * WM * WN, WM * WN == 4 ? 4 : 2) linear_dma_kernel(LinearF32Params p, const uint16_t* xb, uint32_t ldxb, GatedRows gr, float* partials) {
     constexpr bool GATED = KIND == kEpilogueGated, CUT = !GROUPED && MB == 1;
-    constexpr int DK = 64, DM = 64 * MB, AP = DM * DK * 2 / 4096, BP = DN * DK * 2 / 4096; // 1 KB pieces per wave: A, B
+    constexpr int DK = 64, DM = 32 * WM * MB, DN = 64 * WN, AP = DM * DK * 2 / 1024 / (WM * WN), BP = DN * DK * 2 / 1024 / (WM * WN); // 1 KB pieces per wave: A, B
     constexpr uint32_t STAGE = (DM + DN) * DK * 2, ROW = DK * 2, CHUNKS = DK / 8, RPP = 1024 / ROW; // row bytes, 16-byte chunks per row, rows per piece
     extern __shared__ __attribute__((aligned(1024))) uint8_t s_dma[];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1, l32 = lane & 31, half = lane >> 5;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave / WN, wn = wave % WN, l32 = lane & 31, half = lane >> 5;
     uint32_t r_lo = 0, r_hi = p.rows, m_t, n_t, z = 0;
     if (GROUPED) { // tiles of the buckets back to back: the wave's lanes hold the buckets' tile counts (batch <= 64)
         const uint32_t lo = lane < p.batch ? p.row_offsets[lane] : 0u, hi = lane < p.batch ? p.row_offsets[lane + 1] : 0u;
@@ -266,7 +270,7 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
         const uint32_t first = z ? __builtin_amdgcn_readlane(upto, z - 1) : 0u;
         m_t = blockIdx.y - first, n_t = blockIdx.x;
     } else {
-        if (!gemm_tile_of_block(blockIdx.x, (p.rows + DM - 1) / DM, (p.n + DN - 1) / DN, &m_t, &n_t)) return;
+        if (!tile_of_block(blockIdx.x, (p.rows + DM - 1) / DM, (p.n + DN - 1) / DN, &m_t, &n_t)) return;
     }
     const uint32_t m0 = r_lo + m_t * DM, n0 = n_t * DN;
     const uint16_t* w = p.w + (size_t)z * p.w_batch;
@@ -275,16 +279,16 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
     uint32_t va[AP], vb[BP];
 #pragma unroll
     for (int i = 0; i < AP; ++i) {
-        const uint32_t row = (wave * AP + i) * RPP + lane / CHUNKS, chunk = (lane % CHUNKS) ^ (row & 7);
+        const uint32_t row = (wave * AP + i) * RPP + lane / CHUNKS, chunk = (lane % CHUNKS) ^ (row >> 1 & 7);
         const uint32_t m = m0 + row < r_hi ? m0 + row : r_hi - 1;
         va[i] = (GROUPED && p.row_map ? p.row_map[m] : m) * ldxb * 2 + chunk * 16;
     }
 #pragma unroll
     for (int i = 0; i < BP; ++i) {
-        const uint32_t row = (wave * BP + i) * RPP + lane / CHUNKS, chunk = (lane % CHUNKS) ^ (row & 7);
+        const uint32_t row = (wave * BP + i) * RPP + lane / CHUNKS, chunk = (lane % CHUNKS) ^ (row >> 1 & 7);
         uint32_t n = n0 + row;
         if (GATED) { // a wave's first 32 columns are up rows, its second 32 the gate rows of the same outputs: the pair meets in one lane
-            const uint32_t ff = p.n / 2, f = n_t * 64 + (row >> 6) * 32 + (row & 31);
+            const uint32_t ff = p.n / 2, f = n_t * (DN / 2) + (row >> 6) * 32 + (row & 31);
             n = (f < ff ? f : ff - 1) + (row & 32 ? ff : 0);
         } else if (n >= p.n) n = p.n - 1;
         vb[i] = n * p.k * 2 + chunk * 16;
@@ -308,18 +312,26 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (row_map: nothing of the compiler's is in flight from here on)
-    if (STAGES == 2) fetch(0, 0);
-    const uint32_t a_base = (wm * 32 * MB + l32) * ROW, b_base = DM * ROW + (wn * 64 + l32) * ROW, key = l32 & 7;
+    constexpr int OPS = AP + BP; // wave-instructions of a stage
+    if constexpr (STAGES > 1) {
+#pragma unroll
+        for (uint32_t i = 0; i + 1 < STAGES; ++i)
+            if (i < steps) fetch(i, i);
+    }
+    uint32_t buf = 0;
+    const uint32_t a_base = (wm * 32 * MB + l32) * ROW, b_base = DM * ROW + (wn * 64 + l32) * ROW, key = l32 >> 1 & 7;
     auto step = [&](uint32_t kt) {
         if constexpr (STAGES == 1) {
             if (kt) lds_barrier(); // every wave has read step kt - 1
             fetch(kt, 0);
             asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); // step kt is in LDS
-        } else { // step kt is in LDS and every wave has read step kt - 1: the next step may land in its place
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (kt + 1 < steps) fetch(kt + 1, (kt + 1) & 1);
+        } else { // step kt is in LDS and every wave has read step kt - 1: step kt + STAGES - 1 may land in its place
+            if (STAGES > 2 && kt + STAGES - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((STAGES - 2) * OPS) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (kt + STAGES - 1 < steps) fetch(kt + STAGES - 1, buf == 0 ? STAGES - 1 : buf - 1);
         }
-        const uint8_t* at = s_dma + (STAGES == 1 ? 0 : (kt & 1)) * STAGE;
+        const uint8_t* at = s_dma + buf * STAGE;
+        if (STAGES > 1) buf = buf + 1 == STAGES ? 0 : buf + 1;
 #pragma unroll
         for (uint32_t s = 0; s < DK / 16; ++s) {
             const uint32_t slot = ((2 * s + half) ^ key) * 16;
@@ -341,7 +353,7 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
     };
     if constexpr (parts == 1) {
         for (uint32_t kt = 0; kt < steps; ++kt) step(kt);
-    } else if constexpr (MB == 2) { // (a loop in a loop would need the sums' registers twice)
+    } else if constexpr (MB >= 2) { // (a loop in a loop would need the sums' registers twice)
         for (uint32_t kt = 0; kt < steps; ++kt) {
             if (t_lo + kt == w_steps || t_lo + kt == 2 * w_steps) part_end();
             step(kt);
@@ -366,7 +378,7 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
         } else {
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const uint32_t n = GATED ? n_t * 64 + wn * 32 + l32 : n0 + (wn * 2 + j) * 32 + l32, ends = GATED ? p.n / 2 : p.n;
+                const uint32_t n = GATED ? n_t * (DN / 2) + wn * 32 + l32 : n0 + (wn * 2 + j) * 32 + l32, ends = GATED ? p.n / 2 : p.n;
                 if (n >= ends) continue;
 #pragma unroll
                 for (int i = 0; i < MB; ++i)
@@ -375,7 +387,7 @@ __global__ void __launch_bounds__(256, 4) linear_dma_kernel(LinearF32Params p, c
         }
     }
     if constexpr (GATED) {
-        const uint32_t ff = p.n / 2, f = n_t * 64 + wn * 32 + l32;
+        const uint32_t ff = p.n / 2, f = n_t * (DN / 2) + wn * 32 + l32;
         if (f >= ff) return;
 #pragma unroll
         for (int i = 0; i < MB; ++i)
@@ -474,21 +486,22 @@ template <uint32_t PARTS> __global__ void __launch_bounds__(256) linear_finish_k
     p.y[(size_t)row * p.ldy + n] = linear_epilogue(sum, p.bias ? bf16_to_f32(p.bias[n]) : 0.0f, p, row, 0, n);
 }
 
-template <int MB, int STAGES, bool GROUPED, int KIND, uint32_t PARTS>
+template <int WM, int WN, int MB, int STAGES, bool GROUPED, int KIND, uint32_t PARTS>
 uzu_status launch_dma_tile(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, const GatedRows& gr, float* partials, uint32_t splits) {
-    const uint32_t m_tiles = (p.rows + 64 * MB - 1) / (64 * MB), n_tiles = (p.n + DN - 1) / DN;
-    const dim3 grid = GROUPED ? dim3(n_tiles, m_tiles + p.batch) : dim3(gemm_grid_x(m_tiles, n_tiles), 1, splits);
+    constexpr uint32_t DM = 32 * WM * MB, TN = 64 * WN;
+    const uint32_t m_tiles = (p.rows + DM - 1) / DM, n_tiles = (p.n + TN - 1) / TN;
+    const dim3 grid = GROUPED ? dim3(n_tiles, m_tiles + p.batch) : dim3(tile_order_grid(m_tiles, n_tiles), 1, splits);
     UZU_REQUIRE(grid.y <= 65535, "linear_dma: grid too large");
-    const size_t lds = (size_t)STAGES * (64 * MB + DN) * 64 * 2;
+    const size_t lds = (size_t)STAGES * (DM + TN) * 64 * 2;
     static LdsLimit lim;
-    UZU_REQUIRE(raise_lds_limit(lim, (const void*)linear_dma_kernel<MB, STAGES, GROUPED, KIND, PARTS>, lds), "linear_dma: %zu bytes of LDS are not available", lds);
-    return launch_check([&] { hipLaunchKernelGGL((linear_dma_kernel<MB, STAGES, GROUPED, KIND, PARTS>), grid, dim3(256), lds, s, p, xb, PARTS * p.k, gr, partials); }, "linear_dma");
+    UZU_REQUIRE(raise_lds_limit(lim, (const void*)linear_dma_kernel<WM, WN, MB, STAGES, GROUPED, KIND, PARTS>, lds), "linear_dma: %zu bytes of LDS are not available", lds);
+    return launch_check([&] { hipLaunchKernelGGL((linear_dma_kernel<WM, WN, MB, STAGES, GROUPED, KIND, PARTS>), grid, dim3(64 * WM * WN), lds, s, p, xb, PARTS * p.k, gr, partials); }, "linear_dma");
 }
 template <bool GROUPED, int KIND, uint32_t PARTS> uzu_status launch_dma(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, const GatedRows& gr = GatedRows()) {
     const size_t tiles = (size_t)((p.rows + 127) / 128) * ((p.n + DN - 1) / DN);
-    if (tiles >= 512) return launch_dma_tile<2, 1, GROUPED, KIND, PARTS>(s, p, xb, gr, nullptr, 1);
-    if (tiles > 256) return launch_dma_tile<2, 2, GROUPED, KIND, PARTS>(s, p, xb, gr, nullptr, 1);
-    return launch_dma_tile<1, 2, GROUPED, KIND, PARTS>(s, p, xb, gr, nullptr, 1);
+    if (tiles >= 512) return launch_dma_tile<2, 2, 2, 1, GROUPED, KIND, PARTS>(s, p, xb, gr, nullptr, 1);
+    if (tiles > 256) return launch_dma_tile<2, 2, 2, 2, GROUPED, KIND, PARTS>(s, p, xb, gr, nullptr, 1);
+    return launch_dma_tile<2, 2, 1, 2, GROUPED, KIND, PARTS>(s, p, xb, gr, nullptr, 1);
 }
 // Few tiles, many k-steps: the steps are cut over workgroups (two a CU wanted, eight steps each at least) and the shares added by a launch of their own.
 // 300 x 1024 x 2048: f32 products 56 us in one piece and 21.8 us cut (VALU tile: 217 us), bf16 products 26.5 us in the register-staged form and 16.0 us.
@@ -498,17 +511,39 @@ uint32_t dma_splits(const LinearF32Params& p, uint32_t parts) {
     while (splits < 8 && tiles * splits * 2 <= 512 && steps >= 16 * splits) splits *= 2;
     return splits;
 }
+// Up to a 128 x 128 tile a CU: eight waves on it (32 x 64 outputs each) over four buffers of one k-step, and K cut until there is about a workgroup a CU, eight steps each at least;
+// 0: not this form.  Against the 64-row tiles, us: 2048 x 2048 x 4096 70 -> 53, 1000 x 2048 x 4096 46 -> 36 (two shares), 517 x 2048 x 4096 38.5 -> 27.9 (three), 300 x 7712 x 2048
+// 37 -> 29; f32 products 517 x 2048 x 4096 74 -> 50, 300 x 2048 x 4096 44 -> 36.  Those stay ahead where half of these tiles' rows would be empty and there are many of them
+// (64 x 7712 x 2048 18.8 against 20.2), where the steps allow no more than half of the chip (1000 x 1024 x 1024 18 against 20) and where they cut an f32 product that this form cannot
+// (400 x 4112 x 1024 29 against 37).
+uint32_t eight_wave_splits(const LinearF32Params& p, uint32_t parts) {
+    const uint32_t tiles = ((p.rows + 127) / 128) * ((p.n + 127) / 128), steps = parts * p.k / 64;
+    if (tiles > 256 || (p.rows <= 64 && tiles > 48)) return 0;
+    uint32_t splits = std::min(8u, 256 / tiles);
+    while (splits > 1 && steps < 8 * splits) --splits;
+    if (tiles >= 64 && tiles * splits <= 128) return 0;
+    return parts == 3 && splits == 1 && dma_splits(p, parts) > 1 ? 0 : splits;
+}
 // the operand rows and, behind them, the shares of a cut product
 size_t dma_workspace(const LinearF32Params& p, uint32_t parts) {
-    const uint32_t splits = dma_splits(p, parts);
+    const uint32_t splits = std::max(dma_splits(p, parts), eight_wave_splits(p, parts));
     return ((size_t)p.rows * p.k * 2 * parts + 255) / 256 * 256 + (splits > 1 ? (size_t)splits * p.rows * p.n * 4 : 0);
 }
 template <uint32_t PARTS> uzu_status launch_dma_plain(hipStream_t s, const LinearF32Params& p, uint16_t* ws) {
-    if (const uint32_t splits = dma_splits(p, PARTS); splits > 1) {
-        float* partials = (float*)((char*)ws + ((size_t)p.rows * p.k * 2 * PARTS + 255) / 256 * 256);
-        UZU_PROPAGATE((launch_dma_tile<1, 2, false, kEpilogueLean, PARTS>(s, p, ws, GatedRows(), partials, splits)));
+    float* partials = (float*)((char*)ws + ((size_t)p.rows * p.k * 2 * PARTS + 255) / 256 * 256);
+    const uint32_t eight = eight_wave_splits(p, PARTS);
+    if (const uint32_t splits = eight ? eight : dma_splits(p, PARTS); splits > 1) {
+        if (eight) UZU_PROPAGATE((launch_dma_tile<4, 2, 1, 4, false, kEpilogueLean, PARTS>(s, p, ws, GatedRows(), partials, splits)));
+        else UZU_PROPAGATE((launch_dma_tile<2, 2, 1, 2, false, kEpilogueLean, PARTS>(s, p, ws, GatedRows(), partials, splits)));
         const size_t total = (size_t)p.rows * p.n;
         return launch_check([&] { hipLaunchKernelGGL(linear_finish_kernel<PARTS>, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, s, p, ws, partials, splits); }, "linear_finish");
+    }
+    if (eight) {
+        switch (epilogue_kind(p)) {
+        case kEpilogueLean: return launch_dma_tile<4, 2, 1, 4, false, kEpilogueLean, PARTS>(s, p, ws, GatedRows(), nullptr, 1);
+        case kEpilogueXielu: return launch_dma_tile<4, 2, 1, 4, false, kEpilogueXielu, PARTS>(s, p, ws, GatedRows(), nullptr, 1);
+        default: return launch_dma_tile<4, 2, 1, 4, false, kEpilogueFull, PARTS>(s, p, ws, GatedRows(), nullptr, 1);
+        }
     }
     switch (epilogue_kind(p)) {
     case kEpilogueLean: return launch_dma<false, kEpilogueLean, PARTS>(s, p, ws);
