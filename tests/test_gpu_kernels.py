@@ -180,6 +180,36 @@ def test_matmul_dozens_of_rows_f32_sums(hip_ctx, n, k, m, method):
     assert np.linalg.norm(got - want) <= 2.0 ** -23 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("method", [0, 1, 2])
+@pytest.mark.parametrize("n,k,m,d_f32", [(5120, 256, 512, False), (3076, 768, 449, False), (8200, 768, 129, True), (1028, 3584, 300, False), (1028, 2304, 577, True)])
+def test_matmul_hundreds_of_rows_staged(hip_ctx, n, k, m, d_f32, method):
+    """csrc/k_gemm_rows.hip, the staged kernel: two groups of K and many, whole and ragged tiles of 64 tokens x 128 weight rows, K in equal and in unequal shares, each output type.  f32: the
+    bound of the sums above; bf16: <= 1 ulp against the CPU kernel, >= 97 % bit-identical, with the Linear bias."""
+    from test_host_plan import gemm_plan
+    plan = gemm_plan(m, n, k)
+    assert plan.large_tile == 0 and plan.workgroups == -(-m // 64) * -(-n // 128) * plan.splits  # (the staged kernel's grid)
+    rng = np.random.default_rng(n + k + m + method)
+    q = quant_matrix(rng, n, k, 4, 128, method)
+    if not d_f32:
+        a, bias = activations(rng, m, k), bf16(rng.uniform(-0.5, 0.5, size=(n,)))
+        want, got = oracle_matmul(a, q, m, bias=bias), hip_matmul(hip_ctx, a, q, m, bias=bias)
+        ulps = ulp_diff_bf16(want, got)
+        assert ulps.max() <= 1.0, f"max {ulps.max()} bf16 ulps"
+        assert (want == got).mean() >= 0.97
+        return
+    if method == 1:
+        q["zero_points"] = ((q["zero_points"] & 0x11) + 0x77).astype(np.uint8)
+    a = bf16(rng.standard_normal((m, k)))
+    kern = B.MatmulKernel.new(hip_ctx, B.BF16, B.BF16, B.F32)
+    ba, bw, bs, bd = (hip_ctx.buffer_from(z) for z in (a, q["weights"], q["scales"], np.zeros((m, n), np.float32)))
+    bb, bz = (None if q[z] is None else hip_ctx.buffer_from(q[z]) for z in ("biases", "zero_points"))
+    kind = {0: B.B_SCALE_BIAS, 1: B.B_SCALE_ZERO_POINT, 2: B.B_SCALE_SYMMETRIC}[method]
+    run(hip_ctx, lambda cb: kern.encode(cb, a=ba, b=bw, d=bd, m=m, n=n, k=k, b_kind=kind, scales=bs, biases=bb, zero_points=bz, mode=B.QMODE_U4, group_size=128))
+    want = f32(a).astype(np.float64) @ dequantize(q).T
+    got = bd.download(np.float32, m * n).reshape(m, n)
+    assert np.linalg.norm(got - want) <= 2.0 ** -23 * np.linalg.norm(want)
+
+
 def test_gemv_epilogue_and_ragged(hip_ctx):
     """ab_scale + accumulate + bias + soft-cap epilogue, N not a multiple of the tile, signed codes, gather."""
     rng = np.random.default_rng(5)

@@ -19,10 +19,12 @@
 // Measured, us per launch, 64 x 64 tiles -> here (weights not in cache): 1024 x 3584, M = 37: 38.0 -> 8.5; 1024 x 2048: 23.7 -> 6.9; 7168 x 1024 + GatedActMul:
 // 14.3 + 4.7 -> 8.1; 8224 x 1024: 14.5 -> 10.3; 4096 x 14336: 163 -> 33; a 37-token prompt of Qwen3.5-0.8B 3.84 -> 2.22 ms.
 #include <algorithm>
+#include <type_traits>
 
 #include "decode_epilogue.h"
 #include "device_utils.h"
 #include "gemm_convert.h"
+#include "gemm_tile_order.h"
 #include "kernels.h"
 
 namespace uzu {
@@ -56,6 +58,21 @@ __device__ __forceinline__ void turn_words(gm_u32x4& w) {
     w.x = t.x, w.y = t.y;
     t = __builtin_bit_cast(pair, __builtin_amdgcn_permlane16_swap(w.z, w.w, false, false));
     w.z = t.x, w.w = t.y;
+}
+
+// four consecutive outputs of a token, the whole sums: + bias, f32 or bf16
+__device__ __forceinline__ void store_quad(const GemmRowsParams& p, uint32_t token, uint32_t n, gm_f32x4 v) {
+    if (p.out_bias) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += bf16_to_f32(p.out_bias[n + j]);
+    }
+    if (p.d_f32) {
+        *(gm_f32x4*)((float*)p.d + (size_t)token * p.n + n) = v;
+        return;
+    }
+    u32x2_v q;
+    q.x = (uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16), q.y = (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16);
+    *(u32x2_v*)((uint16_t*)p.d + (size_t)token * p.n + n) = q;
 }
 
 // KW waves of the workgroup's four share a tile and split its steps; the other 4 / KW side by side.  ACT: n = 2 h weight rows [up | gate]; blocks 0 .. NB/2 - 1
@@ -199,30 +216,216 @@ __global__ void __launch_bounds__(256, 2) gemm_rows_kernel(GemmRowsParams p) {
             *(gm_f32x4*)(p.partials + ((size_t)blockIdx.z * p.m + token) * p.n + n) = v;
             continue;
         }
-        if (p.out_bias) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                v[j] += bf16_to_f32(p.out_bias[n + j]);
-                if (ACT) gate[j] += bf16_to_f32(p.out_bias[out_n + n + j]);
-            }
-        }
-        if (!ACT && p.d_f32) {
-            *(gm_f32x4*)((float*)p.d + (size_t)token * out_n + n) = v;
+        if (!ACT) {
+            store_quad(p, token, n, v);
             continue;
         }
         uint16_t o[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) // ACT: the rounded pair the unfused kernels would have stored (gated_act_mul/mod.rs:5-12)
-            o[j] = f32_to_bf16(ACT ? round_bf16(round_bf16(v[j]) * act_bf16(p.act_type, round_bf16(gate[j]), kExp2fTab)) : v[j]);
+        for (int j = 0; j < 4; ++j) { // the rounded pair the unfused kernels would have stored (gated_act_mul/mod.rs:5-12)
+            if (p.out_bias) v[j] += bf16_to_f32(p.out_bias[n + j]), gate[j] += bf16_to_f32(p.out_bias[out_n + n + j]);
+            o[j] = f32_to_bf16(round_bf16(round_bf16(v[j]) * act_bf16(p.act_type, round_bf16(gate[j]), kExp2fTab)));
+        }
         u32x2_v q;
         q.x = (uint32_t)o[0] | ((uint32_t)o[1] << 16), q.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
         *(u32x2_v*)((uint16_t*)p.d + (size_t)token * out_n + n) = q;
     }
 }
 
+// ---- hundreds of rows: the same arithmetic, 64 tokens x 128 weight rows a workgroup, operands staged by LDS DMA.
+// Four register-fed waves on a tile of 32 x 64 read every operand for themselves, 344 KB a workgroup and 3584 k, and the L2 bounds them (4.7 TB/s).  Here rows, codes, scales and
+// offsets of a quant group (26 KB) come by global_load_lds into a ring of three stages, two on their way, and one barrier a group; a wave converts 32 weight rows for all 64 tokens (the A
+// operands from LDS), so a code is converted once a workgroup.  What bounds it: vector instructions (240 a wave and group: 112 of the conversion, 64 of the fold) and MFMAs (36) hardly
+// overlap, 0.66 us a group with two workgroups a CU, 1.0 with one.  Tried: a wave's activation sums for itself (48 MFMAs) or all tiles' (here: one's, the others' from LDS) and slots
+// keyed to the row alone (3 of 7 LDS cycles conflicts): 2 to 3 % each; partials by non-temporal stores: 2 us off here, 1 to 4 us more in whoever reads them.
+constexpr int ST = 64, SN = 128; // tokens, weight rows of a staged tile
+struct StagedShape {
+    static constexpr uint32_t A_BYTES = ST * 256, W_BYTES = SN * 64, S_BYTES = 4 * 256, O_BYTES = 4 * 256, STAGE = A_BYTES + W_BYTES + S_BYTES + O_BYTES, STAGES = 3;
+    static constexpr int PITCH = SN + 4; // floats per token of the parked tile
+};
+static_assert(ST * StagedShape::PITCH * 4 <= StagedShape::STAGE * StagedShape::STAGES, "the parked tile takes the stages' place");
+
+template <uint32_t KIND>
+__global__ void __launch_bounds__(256, 2) gemm_rows_staged_kernel(GemmRowsParams p) {
+    using S = StagedShape;
+    constexpr int OPS = KIND == UZU_MATMUL_B_SCALE_SYMMETRIC ? 7 : 8; // wave-instructions of a stage
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[S::STAGE * S::STAGES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t r = lane & 15, g = lane >> 4, G = p.k / 128;
+    uint32_t m_t, n_t;
+    if (!tile_of_block(blockIdx.x, (p.m + ST - 1) / ST, (p.n + SN - 1) / SN, &m_t, &n_t)) return;
+    const uint32_t t0 = m_t * ST, row0 = n_t * SN;
+    const uint32_t g_lo = G * blockIdx.y / p.splits, T = G * (blockIdx.y + 1) / p.splits - g_lo;
+    // where this lane's pieces come from (rows and tokens past the end: from inside the matrices, never stored).  The 16-byte chunk x of a staged row lies in slot x ^ key(row): the 16 rows
+    // that a quarter-wave reads fall on different banks, 256 bytes wide together
+    auto a_key = [](uint32_t row) { return row >> 2 | (row & 3) << 2; };
+    auto w_key = [](uint32_t row) { return (0u - (row >> 2)) & 3u; };
+    uint32_t va[4], vw[2], vs;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t row = wave * 16 + i * 4 + lane / 16;
+        va[i] = min(row, p.m - 1 - t0) * p.k * 2 + ((lane & 15) ^ a_key(row & 15)) * 16;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t row = wave * 32 + i * 16 + lane / 4;
+        vw[i] = min(row0 + row, p.n - 1) * (p.k / 2) + ((lane & 3) ^ w_key(row & 15)) * 16;
+    }
+    vs = min(row0 + wave * 32 + (lane & 31), p.n - 1) * G; // (two lanes bring the same)
+    const uint8_t* a_base = (const uint8_t*)(p.a + (size_t)t0 * p.k);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+    auto dma16 = [&](const void* base, uint32_t v, uint32_t dst) {
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %0" : : "s"(base), "s"(dst), "v"(v) : "memory", "m0");
+    };
+    auto fetch = [&](uint32_t t, uint32_t buf) {
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * S::STAGE), grp = g_lo + t;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dma16(a_base + (size_t)grp * 256, va[i], dst + (wave * 4 + i) * 1024);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) dma16(p.w + (size_t)grp * 64, vw[i], dst + S::A_BYTES + (wave * 2 + i) * 1024);
+        const uint32_t at = (vs + grp) & ~1u, s_dst = dst + S::A_BYTES + S::W_BYTES + wave * 256; // (G is even: the aligned pair of groups)
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, %0" : : "s"(p.scales), "s"(s_dst), "v"(at * 2) : "memory", "m0");
+        if constexpr (KIND == UZU_MATMUL_B_SCALE_BIAS) asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, %0" : : "s"(p.biases), "s"(s_dst + S::S_BYTES), "v"(at * 2) : "memory", "m0");
+        else if constexpr (KIND == UZU_MATMUL_B_SCALE_ZERO_POINT)
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_ubyte %2, %0" : : "s"(p.zp), "s"(s_dst + S::S_BYTES), "v"(at / 2) : "memory", "m0");
+    };
+    // wave w alone sums the activations of token tile w (against an all-ones B) and hands the sums to the others through LDS
+    __shared__ __attribute__((aligned(16))) float s_sum[2][ST];
+    constexpr bool SUMS = KIND != UZU_MATMUL_B_SCALE_SYMMETRIC;
+    const uint32_t w_at = S::A_BYTES + (wave * 32 + r) * 64 + (g ^ w_key(r)) * 16, s_at = S::A_BYTES + S::W_BYTES + wave * 256 + r * 4;
+    uint32_t a_at[4]; // MFMA i contracts k = 32 g + 8 i .. of the group in lane group g: word i of the lane's codes as they lie
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a_at[i] = r * 256 + ((4 * g + i) ^ a_key(r)) * 16;
+    gm_u32x4 af[4][4], raw[2], wv[2][2];
+    uint32_t sraw[2], oraw[2] = {0u, 0u};
+    auto rows = [&](const uint8_t* st, int i) {
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) af[i][tt] = *(const gm_u32x4*)(st + a_at[i] + tt * 4096);
+    };
+    gm_u32x4 own[4]; // the wave's own tile
+    auto own_rows = [&](const uint8_t* st) {
+        if constexpr (SUMS)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) own[i] = *(const gm_u32x4*)(st + a_at[i] + wave * 4096);
+    };
+    auto codes = [&](const uint8_t* st) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            raw[b] = *(const gm_u32x4*)(st + w_at + b * 1024);
+            sraw[b] = *(const uint32_t*)(st + s_at + b * 64);
+            if constexpr (SUMS) oraw[b] = *(const uint32_t*)(st + s_at + S::S_BYTES + b * 64);
+        }
+    };
+    auto convert = [&](int i) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) wv[i & 1][b] = dequant4(raw[b][i] ^ 0x88888888u);
+    };
+    uint32_t ones = 0x3F803F80u;
+    asm("" : "+v"(ones));
+    const gm_u32x4 ones4 = {ones, ones, ones, ones};
+    gm_f32x4 acc[2][4], dq[2][4], sums[4]; // dq: a group's products
+    float sc[2] = {0.f, 0.f}, of[2] = {0.f, 0.f};
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt) acc[0][tt] = acc[1][tt] = dq[0][tt] = dq[1][tt] = sums[tt] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+    auto read_sums = [&](uint32_t which) {
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) sums[tt] = *(const gm_f32x4*)(s_sum[which] + 16 * tt + 4 * g);
+    };
+    auto fold = [&](int b, int tt) { // acc += 16 scale dq + (offset + 8 scale) sum_x
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[b][tt][v] = fmaf(sc[b], dq[b][tt][v], SUMS ? fmaf(of[b], sums[tt][v], acc[b][tt][v]) : acc[b][tt][v]);
+    };
+
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the counts below are the DMA's alone
+    fetch(0, 0);
+    if (T > 1) fetch(1, 1);
+    uint32_t buf = 0;
+    // stage t has landed and every wave has read stage t - 1, whose place stage t + 2 takes
+    auto enter = [&](uint32_t t) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + 1 < T) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(OPS) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (t + 2 < T) fetch(t + 2, buf == 0 ? 2 : buf - 1);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // MFMAs with the vector instructions between them (left alone, the scheduler puts a step's conversions in front of its MFMAs, and the wave's matrix core waits)
+    auto interleave = [&](auto mfmas, auto valu) {
+#pragma unroll
+        for (int i = 0; i < decltype(mfmas)::value; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, decltype(valu)::value, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    enter(0);
+    codes(smem), rows(smem, 0), rows(smem, 1), own_rows(smem), convert(0);
+    for (uint32_t t = 0; t < T; ++t) {
+        const uint8_t* st = smem + buf * S::STAGE;
+        const gm_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        const bool hi = (g_lo + t) & 1;
+        float nsc[2], nof[2] = {0.f, 0.f};
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const float s = bits_to_f32(hi ? sraw[b] & 0xFFFF0000u : sraw[b] << 16);
+            if constexpr (KIND == UZU_MATMUL_B_SCALE_BIAS) nof[b] = fmaf(8.0f, s, bits_to_f32(hi ? oraw[b] & 0xFFFF0000u : oraw[b] << 16));
+            else if constexpr (KIND == UZU_MATMUL_B_SCALE_ZERO_POINT) nof[b] = s * (8.0f - (float)((oraw[b] >> (hi ? 4 : 0)) & 15u));
+            nsc[b] = s * 16.0f;
+        }
+        gm_f32x4 dx = zero;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (i < 2) rows(st, i + 2);
+            if (i < 3) convert(i + 1);
+            if (i == 1 && SUMS && r == 0) *(gm_f32x4*)(s_sum[t & 1] + 16 * wave + 4 * g) = dx;
+            if (i == 2) { // stage t's operands are in registers
+                buf = buf == 2 ? 0 : buf + 1;
+                enter(t + 1);
+                if constexpr (SUMS) read_sums(t & 1);
+                codes(smem + buf * S::STAGE), rows(smem + buf * S::STAGE, 0);
+            }
+            if (i == 3) rows(smem + buf * S::STAGE, 1);
+            if (SUMS && i == 0)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) dx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, own[j]), __builtin_bit_cast(gm_bf16x8, ones4), dx, 0, 0, 0);
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    if (i == 0) fold(b, tt); // the group before
+                    dq[b][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gm_bf16x8, af[i][tt]), __builtin_bit_cast(gm_bf16x8, wv[i & 1][b]), i ? dq[b][tt] : zero, 0, 0, 0);
+                }
+            if (i == 3) own_rows(smem + buf * S::STAGE), convert(0);
+            if (i == 0) interleave(std::integral_constant<int, SUMS ? 12 : 8>(), std::integral_constant<int, 8>());
+            else interleave(std::integral_constant<int, 8>(), std::integral_constant<int, 4>());
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b) sc[b] = nsc[b], of[b] = nof[b];
+    }
+    lds_barrier(); // (the reads beyond the last stage) the stages are free
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt) fold(0, tt), fold(1, tt);
+    float* s_tile = (float*)smem;
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) s_tile[(16 * tt + 4 * g + v) * S::PITCH + wave * 32 + 16 * b + r] = acc[b][tt][v];
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < ST * SN / 4 / 256; ++i) {
+        const uint32_t at = i * 256 + tid, token = t0 + at / (SN / 4), n = row0 + at % (SN / 4) * 4;
+        if (token >= p.m || n >= p.n) continue;
+        gm_f32x4 v = *(const gm_f32x4*)(s_tile + at / (SN / 4) * S::PITCH + at % (SN / 4) * 4);
+        if (p.partials) *(gm_f32x4*)(p.partials + ((size_t)blockIdx.y * p.m + token) * p.n + n) = v;
+        else store_quad(p, token, n, v);
+    }
+}
+
 struct GemmRowsPlan {
     int nb, kw;
     uint32_t splits, workgroups;
+    bool staged;
 };
 
 // The cuts: 16-row blocks per wave, waves per tile, K splits over workgroups.  A launch wants about a workgroup per CU; narrow problems take two blocks per wave,
@@ -242,6 +445,22 @@ GemmRowsPlan gemm_rows_plan(const MatmulParams& p, int num_cus) {
         while (q.splits * 2 * t <= cus && q.splits * 4 <= pairs) q.splits *= 2;
     const uint32_t side_by_side = 4 / q.kw, ob = p.act_mul ? q.nb / 2 : q.nb;
     q.workgroups = ((blocks + ob * side_by_side - 1) / (ob * side_by_side)) * token_tiles * q.splits;
+    if (p.m < 128 || p.act_mul || (uint64_t)p.n * p.k / 2 >= (1ull << 32) || (uint64_t)ST * p.k * 2 >= (1ull << 32)) return q; // (the staged kernel's 32-bit offsets)
+    // From 128 rows on the staged kernel may be the faster one; both in us, fitted to 68 sizes of 128 to 640 rows (the worst choice among them costs 1.3 us).  Register-fed: 4 + 15 per 1024 k over the waves
+    // and shares that walk it, a begun round 0.9 of a full one.  Staged: 4.5 + 1.0 a group of its share while there is at most one workgroup a CU, 6 + 1.43 for two, and in proportion
+    // beyond.  Shares cost what writing the partial tiles takes, and a launch to add them unless the Normalization behind does.
+    // us, register-fed -> staged: 517 x 1024 x 2048 18.1 -> 13.0 (three shares), x 3584 23.2 -> 16.0; 517 x 2048 x 1024 16.4 -> 12.4, x 3072 18.0 -> 12.7, x 4096 27.3 -> 16.9; 256 x 8224 x 1024
+    // 32.5 -> 16.8; 256 x 4096 x 8192 62.6 -> 37.6 + 5; the other way round 128 x 1024 x 1024 5.8 and 8.3, 256 x 1024 x 2048 8.8 and 10.8, 384 x 1024 x 1024 7.7 and 9.4.
+    const bool norm = p.post_norm && p.post_norm_done;
+    auto shares = [&](uint32_t splits) { const double mb = 4e-6 * p.m * p.n * splits; return splits == 1 ? 0.0 : mb / 3 + (norm ? mb / 8 : 2.5 + mb / 4); };
+    const uint32_t full = q.workgroups / cus, rest = q.workgroups % cus;
+    double best = 4.0 + p.k / 1024.0 * 15.0 / (q.kw * q.splits) * (q.nb / 4.0) * (!rest ? full : full ? full + 0.9 : 1.0) + shares(q.splits);
+    const uint32_t staged = ((p.m + ST - 1) / ST) * ((p.n + SN - 1) / SN), groups = p.k / 128;
+    for (uint32_t splits = 1; splits <= 16 && 2 * splits <= groups; ++splits) {
+        const uint32_t each = (groups + splits - 1) / splits, per_cu = (staged * splits + cus - 1) / cus;
+        const double us = (per_cu == 1 ? 4.5 + each : 6.0 + 0.715 * each * per_cu) + shares(splits);
+        if (us < best) best = us, q.staged = true, q.splits = splits, q.workgroups = staged * splits;
+    }
     return q;
 }
 
@@ -252,6 +471,14 @@ template <int NB, int MT, int KW, bool ACT> uzu_status launch_gr(hipStream_t s, 
     case UZU_MATMUL_B_SCALE_BIAS: return launch_check([&] { hipLaunchKernelGGL((gemm_rows_kernel<NB, MT, KW, ACT, UZU_MATMUL_B_SCALE_BIAS>), grid, dim3(256), 0, s, q); }, "gemm_rows");
     case UZU_MATMUL_B_SCALE_ZERO_POINT: return launch_check([&] { hipLaunchKernelGGL((gemm_rows_kernel<NB, MT, KW, ACT, UZU_MATMUL_B_SCALE_ZERO_POINT>), grid, dim3(256), 0, s, q); }, "gemm_rows");
     default: return launch_check([&] { hipLaunchKernelGGL((gemm_rows_kernel<NB, MT, KW, ACT, UZU_MATMUL_B_SCALE_SYMMETRIC>), grid, dim3(256), 0, s, q); }, "gemm_rows");
+    }
+}
+uzu_status launch_staged(hipStream_t s, const GemmRowsParams& q, uint32_t kind) {
+    const dim3 grid(tile_order_grid((q.m + ST - 1) / ST, (q.n + SN - 1) / SN), q.splits);
+    switch (kind) {
+    case UZU_MATMUL_B_SCALE_BIAS: return launch_check([&] { hipLaunchKernelGGL(gemm_rows_staged_kernel<UZU_MATMUL_B_SCALE_BIAS>, grid, dim3(256), 0, s, q); }, "gemm_rows_staged");
+    case UZU_MATMUL_B_SCALE_ZERO_POINT: return launch_check([&] { hipLaunchKernelGGL(gemm_rows_staged_kernel<UZU_MATMUL_B_SCALE_ZERO_POINT>, grid, dim3(256), 0, s, q); }, "gemm_rows_staged");
+    default: return launch_check([&] { hipLaunchKernelGGL(gemm_rows_staged_kernel<UZU_MATMUL_B_SCALE_SYMMETRIC>, grid, dim3(256), 0, s, q); }, "gemm_rows_staged");
     }
 }
 template <int NB, int MT, bool ACT> uzu_status launch_kw(hipStream_t s, const GemmRowsParams& q, uint32_t kind, int kw) {
@@ -328,10 +555,11 @@ uzu_status gemm_rows(hipStream_t s, const MatmulParams& p, int num_cus) {
     const size_t total = (size_t)p.m * p.n;
     if (plan.splits > 1) {
         q.partials = (float*)stream_workspace(s, (size_t)plan.splits * total * 4);
-        if (!q.partials) q.splits = 1; // (a stream under capture has no workspace)
+        if (!q.partials) q.splits = 1, plan.staged = false; // (a stream under capture has no workspace)
     }
     uzu_status st;
-    if (p.act_mul) st = plan.nb == 2 ? launch_kw<2, 2, true>(s, q, p.b_kind, plan.kw) : launch_kw<4, 2, true>(s, q, p.b_kind, plan.kw);
+    if (plan.staged) st = launch_staged(s, q, p.b_kind);
+    else if (p.act_mul) st = plan.nb == 2 ? launch_kw<2, 2, true>(s, q, p.b_kind, plan.kw) : launch_kw<4, 2, true>(s, q, p.b_kind, plan.kw);
     else st = plan.nb == 2 ? launch_kw<2, 2, false>(s, q, p.b_kind, plan.kw) : launch_kw<4, 2, false>(s, q, p.b_kind, plan.kw);
     if (st != UZU_OK || q.splits == 1) return st;
     return gemm_split_finish(s, p, q.partials, q.splits);
