@@ -428,6 +428,9 @@ struct GemmRowsPlan {
     bool staged;
 };
 
+uint32_t staged_tiles(const MatmulParams& p) { return ((p.m + ST - 1) / ST) * ((p.n + SN - 1) / SN); }
+bool staged_fits(const MatmulParams& p) { return p.m >= 128 && !p.act_mul && (uint64_t)p.n * p.k / 2 < (1ull << 32) && (uint64_t)ST * p.k * 2 < (1ull << 32); } // (32-bit offsets)
+
 // The cuts: 16-row blocks per wave, waves per tile, K splits over workgroups.  A launch wants about a workgroup per CU; narrow problems take two blocks per wave,
 // then all four waves on one tile, then splits (measured at N 1024 .. 8224, K 1024 .. 3584, M 20 .. 1021).
 GemmRowsPlan gemm_rows_plan(const MatmulParams& p, int num_cus) {
@@ -445,7 +448,7 @@ GemmRowsPlan gemm_rows_plan(const MatmulParams& p, int num_cus) {
         while (q.splits * 2 * t <= cus && q.splits * 4 <= pairs) q.splits *= 2;
     const uint32_t side_by_side = 4 / q.kw, ob = p.act_mul ? q.nb / 2 : q.nb;
     q.workgroups = ((blocks + ob * side_by_side - 1) / (ob * side_by_side)) * token_tiles * q.splits;
-    if (p.m < 128 || p.act_mul || (uint64_t)p.n * p.k / 2 >= (1ull << 32) || (uint64_t)ST * p.k * 2 >= (1ull << 32)) return q; // (the staged kernel's 32-bit offsets)
+    if (!staged_fits(p)) return q;
     // From 128 rows on the staged kernel may be the faster one; both in us, fitted to 68 sizes of 128 to 640 rows (the worst choice among them costs 1.3 us).  Register-fed: 4 + 15 per 1024 k over the waves
     // and shares that walk it, a begun round 0.9 of a full one.  Staged: 4.5 + 1.0 a group of its share while there is at most one workgroup a CU, 6 + 1.43 for two, and in proportion
     // beyond.  Shares cost what writing the partial tiles takes, and a launch to add them unless the Normalization behind does.
@@ -455,7 +458,7 @@ GemmRowsPlan gemm_rows_plan(const MatmulParams& p, int num_cus) {
     auto shares = [&](uint32_t splits) { const double mb = 4e-6 * p.m * p.n * splits; return splits == 1 ? 0.0 : mb / 3 + (norm ? mb / 8 : 2.5 + mb / 4); };
     const uint32_t full = q.workgroups / cus, rest = q.workgroups % cus;
     double best = 4.0 + p.k / 1024.0 * 15.0 / (q.kw * q.splits) * (q.nb / 4.0) * (!rest ? full : full ? full + 0.9 : 1.0) + shares(q.splits);
-    const uint32_t staged = ((p.m + ST - 1) / ST) * ((p.n + SN - 1) / SN), groups = p.k / 128;
+    const uint32_t staged = staged_tiles(p), groups = p.k / 128;
     for (uint32_t splits = 1; splits <= 16 && 2 * splits <= groups; ++splits) {
         const uint32_t each = (groups + splits - 1) / splits, per_cu = (staged * splits + cus - 1) / cus;
         const double us = (per_cu == 1 ? 4.5 + each : 6.0 + 0.715 * each * per_cu) + shares(splits);
@@ -508,10 +511,10 @@ bool gemm_rows_supported(const MatmulParams& p) {
 //     CUs costs 0.7 of a full one (the workgroups share what the CU reads).  14336 x 4096: 45.6 us against 32.9 at 64 rows, 53 against 60 at 96; 22016 x 2048 with GatedActMul
 //     43 against 66 at 96 rows; 57344 x 8192 with it 217 against 220 at 48, 336 against 465 at 127; 8192 x 8192 86 against 60 at 127.  The slower one is
 //     taken at 5 of 264 sizes by more than 3 %, the worst 16 % (18944 x 3584 at 33 rows, 44.6 against 38.6).
-//   * From 128 rows on it is the 128 x 128 tile (k_gemm128.hip), which
-// reads an operand byte ~4 times as often from LDS instead of the L2 and is ahead as soon as there is work for its tiles: at 8224 x 1024 33 us against 33 at M = 256,
-// 41 against 44 at M = 517; at 1024 x 3584 36 us against 23 at M = 517, and where a short K leaves little to share, from a tile on three CUs of four on: 4096 x 512 27 us
-// against 19 at M = 600 (160 tiles), 14.8 against 19.3 at M = 800 (224); 8192 x 256 11.0 against 8.0 at M = 256 (128), 11.7 against 12.4 at M = 300 (192).
+//   * From 128 rows on it is the 128 x 128 tile (k_gemm128.hip).  The staged kernel is ahead while its tiles leave a CU free, at every K below 8192 (us, all launches of a product, large tile
+// against here): 1021 x 1024 x 2048 26.1 and 20.2, x 3584 38.6 and 28.3, x 7168 48.4 and 36.1; 448 x 4096 x 2048 35.4 and 21.5, x 4096 46.0 and 37.5; 300 x 6144 x 2048 40.0 and 21.6,
+// x 7168 89.0 and 58.6; 1021 x 1920 x 1024 27.3 and 13.8; 1900 x 1024 x 1536 28.3 and 17.5.  Beyond, and where GatedActMul is in it, by the work: at 517 x 8224 x 1024 the large tile takes 24.6, the
+// staged one 26.7; 1024 rows of 4096 x 512 14.8 and 19.3 (register-fed), 300 x 8192 x 256 11.7 and 12.4.
 // From K = 8192 on a workgroup a CU here walks K in 4 us per 1024 and as often as the tiles go round; the large tiles take 12 us and 14 us per 1024 of their share of K, where the
 // number of quant groups lets it be cut: 4096 x 8192 46 us against 33 at M = 128 (one round), 48 against 62 at M = 160 (two); 2048 x 11008, which cannot be cut, 150 against
 // 41 at M = 256, 150 against 74 at M = 512, 4096 x 9728 (two shares) 82 against 62 at M = 256, 85 against 117 at M = 288; 4096 x 14336 74 against 53 at M = 128, 77 against 101 at
@@ -533,7 +536,7 @@ bool gemm_rows_preferred(const MatmulParams& p, int num_cus) {
         return here <= tile;
     }
     const uint32_t large_tiles = ((p.m + 127) / 128) * ((p.n + 127) / 128);
-    if (p.k < 8192) return 2e-9 * p.m * p.n * p.k <= 4.5 && large_tiles < cus * 3 / 4;
+    if (p.k < 8192) return (staged_fits(p) && staged_tiles(p) < cus) || (2e-9 * p.m * p.n * p.k <= 4.5 && large_tiles < cus * 3 / 4);
     const uint32_t splits = gemm128_splits(p, num_cus), rounds = (((p.n + 63) / 64) * ((p.m + 31) / 32) + cus - 1) / cus;
     if (!splits) return true;
     const uint32_t large_rounds = (large_tiles * splits + cus - 1) / cus;
