@@ -659,6 +659,7 @@ uzu_status uzu_hip_model_create_tp(uzu_hip_context* ctx, const uzu_model_desc* d
         ALLOC(decay, float, C * max_hv);
     }
     ALLOC(shortcut_b, uint16_t, C * d);
+    ALLOC(few_partials, float, k::kFewPartials);
     if (desc->has_ple) {
         const size_t total = (size_t)desc->num_layers * desc->ple_dim;
         ALLOC(ple_inputs, uint16_t, CB * total);

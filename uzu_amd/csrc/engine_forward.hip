@@ -135,11 +135,11 @@ void linear(Enc& e, const DLinear& L, const uint16_t* input, uint16_t* output, u
     p.bits = L.bits, p.group_size = L.group, p.ab_scale = 1.0f;
     p.m = batch, p.n = L.n, p.k = L.k;
     offset_tables(e.m, L, input, batch, &p);
-    if (post && !exchange && !L.out_signs && batch >= 17) p.post_norm = &post->p, p.post_norm_done = &post->done;
+    if (post && !exchange && !L.out_signs) p.post_norm = &post->p, p.post_norm_done = &post->done, p.few_partials = e.m->few_partials;
     const char* variant = "matmul";
     e.begin();
     const uzu_status r = k::matmul(e.s, p, e.m->ctx->num_cus, &variant);
-    e.run(r, post && post->done ? (strcmp(variant, "gemm_rows") ? "gemm_q_mfma128+norm" : "gemm_rows+norm") : variant, k::matmul_algorithmic_bytes(p));
+    e.run(r, post && post->done ? (!strcmp(variant, "gemm_rows") ? "gemm_rows+norm" : !strcmp(variant, "gemv_rows_mfma") ? "gemv_rows_mfma+norm" : "gemm_q_mfma128+norm") : variant, k::matmul_algorithmic_bytes(p));
     if (exchange) {
         const size_t count = (size_t)batch * L.n;
         RUN("all_reduce", count * 4, tp::all_reduce_sum_f32(e.m->tp, e.s, e.m->tp_buf, count, output)); // sums rounded to bf16 into `output`
@@ -215,7 +215,7 @@ bool linear_normed(Enc& e, const DNorm& N, int mode, const DLinear& L, const uin
     rn.scales = N.scales, rn.eps = N.eps, rn.offset = N.offset, rn.full_layer = N.full_layer, rn.residual_add = mode == 2;
     rn.shortcut_in = mode == 2 ? sc_in : nullptr, rn.shortcut_out = sc_out, rn.normed_out = normed_out;
     e.begin();
-    e.run(k::gemv_rows_mfma(e.s, p, &rn), gated ? "gemv_rows[norm+up+act]" : "gemv_rows[norm+linear]", k::matmul_algorithmic_bytes(p));
+    e.run(k::gemv_rows_mfma(e.s, p, e.m->ctx->num_cus, &rn), gated ? "gemv_rows[norm+up+act]" : "gemv_rows[norm+linear]", k::matmul_algorithmic_bytes(p));
     return true;
 }
 
@@ -572,7 +572,7 @@ uzu_status encode_forward(uzu_hip_model* m, hipStream_t s, uint32_t count, bool 
         }
         hidden_normed = false;
         PostNorm mlp_norm; // the pre-MLP normalisation, offered to the mixer's out projection when nothing sits between them
-        const bool offer_mlp = !L.post_mixer.present && rows >= 17 && !L.pre_mlp.scalar_mode;
+        const bool offer_mlp = !L.post_mixer.present && rows >= 4 && !L.pre_mlp.scalar_mode;
         if (offer_mlp) mlp_norm.p = norm_params(e, L.pre_mlp, m->mixed, m->normed, sc_cur, 2, rows, d, L.d.mlp_kind == UZU_MLP_MOE ? nullptr : &L.up);
         if (L.d.mixer_kind == UZU_MIXER_ATTENTION)
             attention_mixer(e, L, h, m->mixed, q, offer_mlp ? &mlp_norm : nullptr, first_done);
@@ -601,7 +601,9 @@ uzu_status encode_forward(uzu_hip_model* m, hipStream_t s, uint32_t count, bool 
         }
         // the next layer's pre-mixer normalisation rides on this layer's down projection (not past the last layer: the output norm takes one row)
         PostNorm next_norm;
-        const bool offer_next = !is_moe && rows >= 17 && !L.post_mlp.present && !L.d.has_ple && l + 1 < layer_count && m->layers[l + 1].pre_mixer.present;
+        // (nor from a layer whose residual rows are filed below: the normalisation adds `hidden` to them)
+        const bool filed = std::find(m->feature_layers.begin(), m->feature_layers.end(), l) != m->feature_layers.end();
+        const bool offer_next = !is_moe && !filed && rows >= 4 && !L.post_mlp.present && !L.d.has_ple && l + 1 < layer_count && m->layers[l + 1].pre_mixer.present;
         if (offer_next) {
             const DLayer& Nx = m->layers[l + 1];
             next_norm.p = norm_params(e, Nx.pre_mixer, hidden, m->normed, sc_cur, 2, rows, d, Nx.d.mixer_kind == UZU_MIXER_ATTENTION ? &Nx.qkv : &Nx.in_proj);

@@ -218,6 +218,7 @@ struct uzu_hip_model {
     // fused decode path
     bool fusable = false;
     uint16_t* shortcut_b = nullptr; // ping-pong partner of `shortcut`
+    float* few_partials = nullptr;  // MatmulParams::few_partials
     uint16_t* rht_scratch = nullptr; // [rows][widest RHT input]: InputRht works on a copy of the rows
     // group row sums of `normed`, written by the normalisation that produced it (MatmulParams::pre_rowsum of the GEMMs that read it):
     // valid for (rs_rows rows, rs_k elements, groups of rs_group) until `normed` is written again

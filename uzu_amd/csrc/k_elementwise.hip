@@ -279,7 +279,7 @@ bool normalization_from_partials_supported(const NormParams& p, const NormPartia
         const char* e = tune_env("norm_partials");
         return !e || atoi(e) != 0;
     }();
-    if (!on || exact_mode() || p.io_dt != UZU_BF16 || p.batch_size < 16 || p.element_count % 1024 || (p.affine_dt != UZU_F32 && p.affine_dt != UZU_BF16)) return false;
+    if (!on || exact_mode() || p.io_dt != UZU_BF16 || p.batch_size < 2 || p.element_count % 1024 || (p.affine_dt != UZU_F32 && p.affine_dt != UZU_BF16)) return false;
     const uint32_t nv = p.element_count / 1024;
     if (nv != 1 && nv != 2 && nv != 4 && nv != 5 && nv != 8) return false;
     if (!sp.partials || sp.splits < 2 || !sp.d || sp.total != (size_t)p.batch_size * p.element_count) return false;

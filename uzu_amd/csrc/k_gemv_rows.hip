@@ -16,9 +16,12 @@
 //     a 16-lane row with DPP row_share;
 //   * sum_k x of the group (the offset term, and the 16 of the code trick) comes from the matrix core as well: the same B against an
 //     all-ones A -- no vector work;
-//   * the workgroup's waves split K (steps w, w + NW, ...) and add their tiles through LDS in wave order.
+//   * the workgroup's waves split K (steps w, w + NW, ...) and add their tiles through LDS in wave order; workgroups may share K as well (f32 partial tiles, added in
+//     share order by the Normalization behind).
 // Per 1 KiB of codes: 32 conversions + ~24 fold / broadcast VALU + 8 MFMAs for ALL 16 rows -- the M = 1 GEMV's instruction budget.
 // Results are tolerance-class against the scalar reference like every reduction kernel (f32 accumulation in another order).
+#include <algorithm>
+
 #include "decode_epilogue.h"
 #include "device_utils.h"
 #include "kernels.h"
@@ -46,6 +49,7 @@ struct RowsParams {
     void* d;                  // [m, n] bf16 or f32
     uint32_t m, n, k, group_size, kind, d_f32;
     uint32_t act_type; // ACT instances: n = 2 h weight rows [up | gate]; d = [m, h] = up * act(gate) (GatedActMul, gated_act_mul.rs:36-70)
+    float* partials;   // [gridDim.y][m, n] f32, or null: the whole sum is here
     RowsNorm norm;     // NORM instances: `a` holds the raw rows
 };
 
@@ -100,7 +104,8 @@ __global__ void __launch_bounds__(64 * NW) gemv_rows_mfma_kernel(RowsParams p) {
     };
     (void)wp;
     Step stA, stB;
-    load_step(wave, stA); // in flight while the activations are staged
+    const uint32_t s_lo = steps * blockIdx.y / gridDim.y, s_hi = steps * (blockIdx.y + 1) / gridDim.y; // this workgroup's share of K
+    load_step(s_lo + wave, stA); // in flight while the activations are staged
     // ---- stage the activation rows: 16-byte chunks (8 consecutive k) in the conversion's k order; rows >= m are zero
     if constexpr (NORM) {
         // Normalization prologue (normalization.rs:56-125 with AccumT = f32, no mean / biases): normalization_kernel's arithmetic per row -- thread t of
@@ -231,11 +236,11 @@ __global__ void __launch_bounds__(64 * NW) gemv_rows_mfma_kernel(RowsParams p) {
             acc[b].w = fmaf(s3, dq[b].w, fmaf(o3, dx.x, acc[b].w));
         }
     };
-    for (uint32_t s = wave; s < steps; s += 2 * NW) {
+    for (uint32_t s = s_lo + wave; s < s_hi; s += 2 * NW) {
         load_step(s + NW, stB);
         compute(s, stA);
         load_step(s + 2 * NW, stA);
-        if (s + NW < steps) compute(s + NW, stB);
+        if (s + NW < s_hi) compute(s + NW, stB);
     }
     // ---- add the waves' tiles in wave order, bias, store: thread t = (row t / 16, token t % 16)
 #pragma unroll
@@ -254,6 +259,10 @@ __global__ void __launch_bounds__(64 * NW) gemv_rows_mfma_kernel(RowsParams p) {
             for (int w = 1; w < NW; ++w) v[b] += s_part[((size_t)w * NB + b) * 256 + tid];
         }
         if (j < p.m && row0 + row < out_n) {
+            if (p.partials) {
+                p.partials[((size_t)blockIdx.y * p.m + j) * out_n + row0 + row] = v[0];
+                return;
+            }
             float value = 1.0f * v[0]; // MatmulKernel epilogue with ab_scale = 1 (kernel.rs:281-292)
             if (p.out_bias) value += bf16_to_f32(p.out_bias[row0 + row]);
             if constexpr (ACT) {
@@ -289,16 +298,16 @@ bool gemv_rows_norm_supported(const MatmulParams& p) {
     return gemv_rows_mfma_supported(p) && p.k % 1024 == 0 && (size_t)16 * (p.k * 2 + 16) + 8 * 256 * 4 <= 150 * 1024;
 }
 
-template <int NW, bool ACT, bool NORM> static uzu_status launch_rows(hipStream_t s, const RowsParams& q, uint32_t blocks, size_t lds) {
+template <int NW, bool ACT, bool NORM> static uzu_status launch_rows(hipStream_t s, const RowsParams& q, uint32_t blocks, size_t lds, uint32_t splits = 1) {
     static LdsLimit lim;
     if (!raise_lds_limit(lim, (const void*)gemv_rows_mfma_kernel<NW, ACT, NORM>, lds)) {
         set_error("gemv_rows: %zu bytes of LDS are not available", lds);
         return UZU_ERR_UNSUPPORTED;
     }
-    return launch_check([&] { hipLaunchKernelGGL((gemv_rows_mfma_kernel<NW, ACT, NORM>), dim3(blocks), dim3(64 * NW), lds, s, q); }, "gemv_rows_mfma");
+    return launch_check([&] { hipLaunchKernelGGL((gemv_rows_mfma_kernel<NW, ACT, NORM>), dim3(blocks, splits), dim3(64 * NW), lds, s, q); }, "gemv_rows_mfma");
 }
 
-uzu_status gemv_rows_mfma(hipStream_t s, const MatmulParams& p, const RowsNorm* norm) {
+uzu_status gemv_rows_mfma(hipStream_t s, const MatmulParams& p, int num_cus, const RowsNorm* norm) {
     RowsParams q{};
     q.a = (const uint16_t*)p.a, q.w = (const uint8_t*)p.b, q.scales = (const uint16_t*)p.scales, q.biases = (const uint16_t*)p.biases, q.zp = p.zero_points;
     q.out_bias = (const uint16_t*)p.bias, q.d = p.d, q.m = p.m, q.n = p.n, q.k = p.k, q.group_size = p.group_size, q.kind = p.b_kind, q.d_f32 = p.d_dt == UZU_F32;
@@ -314,6 +323,17 @@ uzu_status gemv_rows_mfma(hipStream_t s, const MatmulParams& p, const RowsNorm* 
     const uint32_t blocks = ((act ? p.n / 2 : p.n) + 15) / 16, steps = p.k / 128;
     // eight waves split K where the row blocks alone leave most of the chip idle and there are steps to share
     const bool wide = !act && blocks < 256 && steps >= 16;
+    // ... or shares of K over workgroups of four, where a Normalization behind adds them: a workgroup reads the rows' whole share of K through its CU's cache, which bounds it.  The chip filled
+    // once, four steps a share or more.  13 rows, us, eight waves -> shares: 1024 x 2048 5.5 -> 3.9 (four), 1024 x 3584 7.5 -> 4.6 (four); 2048 x 4096 (16 rows) 8.9 -> 6.7 (two).
+    if (wide && !norm && p.few_partials) {
+        uint32_t splits = 1;
+        while (splits * 2 * blocks <= std::min((uint32_t)num_cus, 256u) && splits * 8 <= steps) splits *= 2;
+        if (splits > 1 && gemm_split_joins_norm(p, p.few_partials, splits)) {
+            q.partials = p.few_partials;
+            const uzu_status st = launch_rows<4, false, false>(s, q, blocks, (size_t)4 * 256 * 4, splits);
+            return st == UZU_OK ? gemm_split_finish(s, p, q.partials, splits) : st;
+        }
+    }
     const int nw = wide ? 8 : 4;
     const size_t lds = (norm ? (size_t)16 * (p.k * 2 + 16) : 0) + (size_t)nw * (act ? 2 : 1) * 256 * 4; // the staged rows only where the prologue writes them
     if (norm) return act ? launch_rows<4, true, true>(s, q, blocks, lds) : wide ? launch_rows<8, false, true>(s, q, blocks, lds) : launch_rows<4, false, true>(s, q, blocks, lds);

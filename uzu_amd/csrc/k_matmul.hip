@@ -369,7 +369,7 @@ uzu_status matmul(hipStream_t s, const MatmulParams& p, int num_cus, const char*
     }
     if (gemv_rows_mfma_supported(p)) { // a handful of rows (speculative verify passes, prefill tails): one pass over the weights on the matrix cores
         if (variant) *variant = "gemv_rows_mfma";
-        return gemv_rows_mfma(s, p);
+        return gemv_rows_mfma(s, p, num_cus);
     }
     if (gemm_q_mfma_supported(p)) { // prefill-sized M: bf16 matrix cores (k_gemm.hip)
         if (variant) *variant = p.bits == 4 ? "gemm_q_mfma<4>" : "gemm_q_mfma<8>";

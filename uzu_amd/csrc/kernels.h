@@ -61,6 +61,7 @@ struct MatmulParams {
     // (normalization_from_partials) and sets *post_norm_done; every other kernel choice ignores it and the caller runs the normalisation itself.
     const NormParams* post_norm;
     uint32_t* post_norm_done;
+    float* few_partials; // optional: kFewPartials floats for the few-rows kernel's shares of K (k_gemv_rows.hip), also while the stream is captured
 };
 bool gemm_coef_table_supported(const MatmulParams& p);                          // the large-tile kernel's quantisation family
 uzu_status gemm_coef_table(hipStream_t s, const MatmulParams& p, float* coef); // coef[g][n]; p needs b / scales / biases / zero_points, n, k, bits, group_size, b_kind
@@ -77,9 +78,11 @@ bool gemm_rows_preferred(const MatmulParams& p, int num_cus);
 uzu_status gemm_rows(hipStream_t s, const MatmulParams& p, int num_cus);
 void gemm_rows_plan_query(const MatmulParams& p, int num_cus, uint32_t* splits, uint32_t* workgroups);
 uint32_t gemm128_splits(const MatmulParams& p, int num_cus); // k_gemm128.hip: the cuts of K of a product on the large tiles (0: none that it takes)
+bool gemm_split_joins_norm(const MatmulParams& p, const float* partials, uint32_t splits); // k_gemm128.hip: whether gemm_split_finish leaves the sums to p.post_norm
 uzu_status gemm_split_finish(hipStream_t s, const MatmulParams& p, const float* partials, uint32_t splits); // k_gemm128.hip
 // k_gemv_rows.hip: 2 <= M <= 16 activation rows against int4 codes (group % 128 == 0) as ONE pass over the weights on the matrix cores
 bool gemv_rows_mfma_supported(const MatmulParams& p);
+constexpr size_t kFewPartials = 16 * 4096; // 16 rows x (splits x n), which is 16 columns for each of at most 256 workgroups
 // Normalization (RMS; ShortcutMode Copy / Add; normalization.rs:56-125) of the m <= 16 activation rows as the PROLOGUE of the few-rows kernel
 // (speculative verify passes, prefill tails: round 5): every workgroup normalises the rows while it stages them, with the element mapping and
 // reduction order of normalization_kernel (bit-identical rows); workgroup 0 also writes the residual rows and, if asked, the normalised rows.
@@ -92,7 +95,7 @@ struct RowsNorm {
     uint16_t* normed_out;        // bf16 [m, k] or null: the normalised rows (for a second linear that reads the same rows)
 };
 bool gemv_rows_norm_supported(const MatmulParams& p);
-uzu_status gemv_rows_mfma(hipStream_t s, const MatmulParams& p, const RowsNorm* norm = nullptr);
+uzu_status gemv_rows_mfma(hipStream_t s, const MatmulParams& p, int num_cus, const RowsNorm* norm = nullptr);
 bool gemm_q_mfma_supported(const MatmulParams& p);   // k_gemm.hip: M >= 20, bf16 activations, int4/int8 codes, group % 64 == 0
 uzu_status gemm_q_mfma(hipStream_t s, const MatmulParams& p, int num_cus);
 // k_gemm128.hip: 128 x 128 tiles, M >= 128, group 64 / 128 / 256; `workspace` holds the activation row-sum pieces (+ split-K partials)
