@@ -581,6 +581,39 @@ def test_llama3_8b_full_depth_matches_oracle_fixture(hip_ctx, name):
 ROBUST_PROMPT_MULTIPLIERS = {"tiny-qwen": (21, 13, 37), "tiny-llama": (149, 373, 223)}
 
 
+@pytest.mark.parametrize("nseq,count,gate", [(3, 250, False), (9, 70, False), (3, 250, True)])
+def test_batched_prefill_with_the_sequences_attention_in_one_launch(hip_ctx, nseq, count, gate):
+    """Sequences of a batched pass whose attention goes out in one launch (csrc/k_attention_mfma.hip: AttentionSeqs): behind contexts of different lengths, a ragged last query tile, more
+    sequences than a launch takes, with and without the output gate; the next step's logits against each sequence alone (the projections see other row counts: tolerance-class)."""
+    cfg = S.tiny_llama(num_heads=32, num_groups=8, max_context_length=400, has_gate=gate, seed=45)
+    hm = HipModel(hip_ctx, S.build_model(cfg), MODEL_BATCH(nseq))
+    base = S.synthetic_prompt(count, cfg.vocab_size).astype(np.int64)
+    prompts = np.stack([(base * (2 * i + 3) + 11 * i) % cfg.vocab_size for i in range(nseq)]).astype(np.uint32)
+    contexts = [prompts[(i + 1) % nseq][: 5 + 13 * (i % 4)] for i in range(nseq)]
+    alone = []
+    for i in range(nseq):
+        hm.reset()
+        hm.prefill(contexts[i])
+        hm.prefill(prompts[i])
+        alone.append(hm.read_logits())
+    states = [hm.new_state() for _ in range(nseq)]
+    for i in range(nseq):
+        hm.bind(states[i])
+        hm.prefill(contexts[i])
+    first = hm.prefill_batch(states, prompts)
+    for i in range(nseq):
+        a = f32(alone[i]).astype(np.float64).ravel()
+        assert a.max() - a[int(first[i])] <= 0.1 * a.std()  # the token that the pass sampled is the best of the logits alone, or tied with it
+        hm.bind(states[i])
+        hm.decode(1)
+        batched = hm.read_logits()
+        hm.reset()
+        hm.prefill(contexts[i])
+        hm.prefill(prompts[i])
+        hm.prefill(np.array([first[i]], np.uint32))
+        assert logits_close(hm.read_logits(), batched).all()
+
+
 @pytest.mark.parametrize("preset", ["tiny-qwen", "tiny-llama"])
 def test_sequence_states_are_independent_and_batched_prefill_matches_single(hip_ctx, preset):
     """LanguageModelState split from the model (state.rs:9-16): three sequences with different prompts share one set of

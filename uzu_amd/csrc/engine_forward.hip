@@ -287,7 +287,15 @@ uzu_status ensure_partials(uzu_hip_model* m, uint32_t rows, uint32_t head_dim) {
 // streamed once for all sequences), attention / KV append / DeltaNet run per sequence on its own state.  The reference
 // has no cross-sequence batching: per sequence the arithmetic is that of the single-sequence pass.
 
-void attention_core(Enc& e, DLayer& L, uint32_t batch, size_t row0, bool fuse_norms);
+// the sequences of a batched prefill whose attention goes out in one launch (k_attention_mfma.hip)
+struct JoinedAttention {
+    uint32_t sequences;
+    k::AttentionParams a{};
+    k::AttentionSeqs seqs{};
+    size_t row0[k::AttentionSeqs::kMost];
+};
+void attention_joined(Enc& e, DLayer& L, uint32_t batch, JoinedAttention& j);
+void attention_core(Enc& e, DLayer& L, uint32_t batch, size_t row0, bool fuse_norms, JoinedAttention* join = nullptr);
 
 static bool attention_fusions_enabled() {
     const char* e = tune_env("attn_fused");
@@ -316,9 +324,11 @@ void attention_mixer(Enc& e, DLayer& L, const uint16_t* hidden, uint16_t* out, c
     if (q.n == 0) {
         attention_core(e, L, q.count, 0, fuse_norms);
     } else {
+        JoinedAttention join{q.n};
         for (uint32_t i = 0; i < q.n; ++i) {
             bind_state(m, q.st[i]);
-            attention_core(e, L, q.count, (size_t)i * q.count, fuse_norms);
+            attention_core(e, L, q.count, (size_t)i * q.count, fuse_norms, &join);
+            if (join.seqs.n == k::AttentionSeqs::kMost || i + 1 == q.n) attention_joined(e, L, q.count, join);
         }
     }
     // (SigmoidGate: attention_core applies it per sequence -- inside the key-split merge of a prefill pass where there is one)
@@ -326,7 +336,17 @@ void attention_mixer(Enc& e, DLayer& L, const uint16_t* hidden, uint16_t* out, c
 }
 
 // AttentionPrepare + attention of `batch` rows of the bound sequence, which start at row `row0` of qkv / queries / attn_out
-void attention_core(Enc& e, DLayer& L, uint32_t batch, size_t row0, bool fuse_norms) {
+void attention_joined(Enc& e, DLayer& L, uint32_t batch, JoinedAttention& j) {
+    uzu_hip_model* m = e.m;
+    if (!j.seqs.n) return;
+    const uint32_t hd = L.d.head_dim, nq = L.d.num_heads;
+    RUN("attention_prefill_mfma", 0, k::attention_prefill_mfma_seqs(e.s, j.a, j.seqs));
+    if (L.d.has_gate)
+        for (uint32_t i = 0; i < j.seqs.n; ++i)
+            RUN("sigmoid_gate", 0, k::sigmoid_gate(e.s, m->gate + j.row0[i] * nq * hd, m->attn_out + j.row0[i] * nq * hd, UZU_BF16, batch * nq * hd));
+    j.seqs.n = 0;
+}
+void attention_core(Enc& e, DLayer& L, uint32_t batch, size_t row0, bool fuse_norms, JoinedAttention* join) {
     uzu_hip_model* m = e.m;
     const bool has_kv = !L.d.is_kv_sharing; // prepare_queries (mode.rs:234-259): no KV rows are written; the source layer wrote this pass's already
     const uint32_t hd = L.d.head_dim, nq = L.d.num_heads, nkv = L.d.num_groups, total_heads = nq + (has_kv ? 2 * nkv : 0);
@@ -364,6 +384,12 @@ void attention_core(Enc& e, DLayer& L, uint32_t batch, size_t row0, bool fuse_no
     const size_t kv_bytes = (size_t)2 * (physical_prefix + batch) * nkv * hd * 2; // K and V rows read once
     const bool two_pass = (m->regime_override >= 0 && !W) ? m->regime_override == 1 : physical_prefix + batch > 1024; // core/mod.rs:89-92
     bool gated = false;
+    if (join && k::attention_prefill_mfma_joins(a, join->sequences)) { // (attention_joined: the launch and the gate, behind the last sequence's rows)
+        const uint32_t i = join->seqs.n++;
+        join->a = a, join->row0[i] = row0;
+        join->seqs.queries[i] = a.queries, join->seqs.keys[i] = a.keys, join->seqs.values[i] = a.values, join->seqs.dyn[i] = a.dyn, join->seqs.out[i] = attn_out;
+        return;
+    }
     if (k::attention_prefill_mfma_supported(a)) { // prefill chunk: flash-attention tiles on the matrix cores, any context length
         uint32_t gate_done = 0; // SigmoidGate inside the key-split merge launch when the pass has one (bit-identical to the separate launch)
         RUN("attention_prefill_mfma", kv_bytes, k::attention_prefill_mfma(e.s, a, attn_out, L.d.has_gate && attention_fusions_enabled() ? m->gate + row0 * nq * hd : nullptr, &gate_done));

@@ -22,6 +22,9 @@
 //     the summation order.
 #include <stdlib.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "device_utils.h"
 #include "kernels.h"
 
@@ -58,8 +61,10 @@ __device__ __forceinline__ float other_half(float v) { return __shfl_xor(v, 32, 
 // KG groups of four waves share a stretch of 32 KG keys, a wave takes its group's 32 of them, and the groups' unnormalised results meet in LDS at the end, in group order: the
 // grid is about a workgroup per CU, and a wave alone on its SIMD waits for itself at every exponential (1021 rows of 32 heads of 128: 72 us with one group, 39 with
 // two).  Heads of 256 need the registers of a wave alone.
-template <int HD, bool GEN, int KG = HD <= 128 ? 2 : 1>
-__global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(AttentionParams a, uint16_t* out, uint32_t tpw, float* part_o, float* part_ml) {
+// SEQS: several sequences, each with its own rows and cache, gridDim.x = kv heads x sequences and no key splits: the workgroups with the longest key ranges of all of them come first, and the
+// short ones fill what a sequence by itself leaves idle (four of 1021 rows, 32 heads of 128: 4 x 39 us -> 99).
+template <int HD, bool GEN, bool SEQS = false, int KG = HD <= 128 ? 2 : 1>
+__global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(AttentionParams a, uint16_t* out, uint32_t tpw, float* part_o, float* part_ml, std::conditional_t<SEQS, AttentionSeqs, uint32_t> seqs) {
     constexpr int KP = HD * 2 + 16;  // K tile row pitch in bytes (conflict-free ds_read_b128)
     constexpr int VP = TK * 2 + 8;   // V^T tile row pitch in bytes: 32 keys + 8 bytes of pad (conflict-free ds_read_b64)
     constexpr int NS = HD / 16;      // k16 steps of the QK^T contraction
@@ -74,7 +79,12 @@ __global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(Attent
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, kg = __builtin_amdgcn_readfirstlane(tid >> 8), half = lane >> 5, l32 = lane & 31;
     const uint32_t M = a.suffix_length;
-    const uint32_t kv_head = blockIdx.x;
+    uint32_t kv_head = blockIdx.x;
+    if constexpr (SEQS) {
+        const uint32_t kv_heads = a.num_heads / a.gqa_factor, seq = kv_head / kv_heads;
+        kv_head -= seq * kv_heads;
+        a.queries = seqs.queries[seq], a.keys = seqs.keys[seq], a.values = seqs.values[seq], a.dyn = seqs.dyn[seq], out = (uint16_t*)seqs.out[seq];
+    }
     const uint32_t n_tasks = a.gqa_factor * ((M + TQ - 1) / TQ);
     const uint32_t task0 = (gridDim.y - 1 - blockIdx.y) * tpw; // heaviest (last query tiles) first
     const uint32_t task = task0 + wave;
@@ -406,14 +416,34 @@ uzu_status attention_prefill_mfma(hipStream_t s, const AttentionParams& a, void*
 #define UZU_LAUNCH(H)                                                                                                                                              \
     {                                                                                                                                                              \
         UZU_PROPAGATE(launch_check([&] {                                                                                                                           \
-            if (general) hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, true>), grid, dim3(H <= 128 ? 512 : 256), 0, s, a, (uint16_t*)out, tpw, part_o, part_ml);             \
-            else hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, false>), grid, dim3(H <= 128 ? 512 : 256), 0, s, a, (uint16_t*)out, tpw, part_o, part_ml);                    \
+            if (general) hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, true>), grid, dim3(H <= 128 ? 512 : 256), 0, s, a, (uint16_t*)out, tpw, part_o, part_ml, 0u);             \
+            else hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, false>), grid, dim3(H <= 128 ? 512 : 256), 0, s, a, (uint16_t*)out, tpw, part_o, part_ml, 0u);                    \
         }, "attention_prefill_mfma"));                                                                                                                             \
         if (!part) return UZU_OK;                                                                                                                                  \
         if (gate && gate_done) *gate_done = 1;                                                                                                                     \
         return launch_check([&] { hipLaunchKernelGGL(attention_prefill_merge_kernel<H>, dim3((uint32_t)((rows + 3) / 4)), dim3(256), 0, s, part_o, part_ml, (uint16_t*)out, (uint32_t)rows, splits, gate_done ? (const uint16_t*)gate : nullptr); }, \
                             "attention_prefill_merge");                                                                                                            \
     }
+    switch (a.head_dim) {
+    case 64: UZU_LAUNCH(64);
+    case 128: UZU_LAUNCH(128);
+    default: UZU_LAUNCH(256);
+    }
+#undef UZU_LAUNCH
+}
+
+// Where the sequences' workgroups of four tasks together cover three CUs of four, as one sequence's have to for a launch without key splits; windows, rings and sinks stay one by one.
+bool attention_prefill_mfma_joins(const AttentionParams& a, uint32_t sequences) {
+    if (sequences < 2 || a.sinks || a.is_sliding_window || a.is_kv_cache_ring || !attention_prefill_mfma_supported(a)) return false;
+    const uint32_t n_tasks = a.gqa_factor * ((a.suffix_length + TQ - 1) / TQ);
+    return std::min(sequences, AttentionSeqs::kMost) * (a.num_heads / a.gqa_factor) * ((n_tasks + 3) / 4) >= 192;
+}
+uzu_status attention_prefill_mfma_seqs(hipStream_t s, const AttentionParams& a, const AttentionSeqs& q) {
+    const uint32_t n_tasks = a.gqa_factor * ((a.suffix_length + TQ - 1) / TQ);
+    const dim3 grid(a.num_heads / a.gqa_factor * q.n, (n_tasks + 3) / 4);
+#define UZU_LAUNCH(H)                                                                                                                                              \
+    return launch_check([&] { hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, false, true>), grid, dim3(H <= 128 ? 512 : 256), 0, s, a, (uint16_t*)nullptr, 4u, (float*)nullptr, (float*)nullptr, q); }, \
+                        "attention_prefill_mfma_seqs")
     switch (a.head_dim) {
     case 64: UZU_LAUNCH(64);
     case 128: UZU_LAUNCH(128);

@@ -213,6 +213,18 @@ uzu_status attention_single_pass(hipStream_t s, const AttentionParams& p, void* 
 bool attention_prefill_mfma_supported(const AttentionParams& p); // k_attention_mfma.hip: causal bf16 prefill tiles on the matrix cores
 // gate / gate_done (optional): when the pass ends in the key-split merge, SigmoidGate of `gate` (bf16, the layout of `out`) is applied there and *gate_done = 1
 // (bit-identical to the separate launch); otherwise the caller runs sigmoid_gate itself
+// the same attention of several sequences in one launch (equal suffix lengths; `p` is any one of them): kMost at a time
+struct AttentionSeqs {
+    static constexpr uint32_t kMost = 8;
+    const void* queries[kMost];
+    const void* keys[kMost];
+    const void* values[kMost];
+    const uint32_t* dyn[kMost];
+    void* out[kMost];
+    uint32_t n;
+};
+bool attention_prefill_mfma_joins(const AttentionParams& p, uint32_t sequences); // whether a sequence of such a batch is to go into an AttentionSeqs launch
+uzu_status attention_prefill_mfma_seqs(hipStream_t s, const AttentionParams& p, const AttentionSeqs& q);
 uzu_status attention_prefill_mfma(hipStream_t s, const AttentionParams& p, void* out, const void* gate = nullptr, uint32_t* gate_done = nullptr);
 uzu_status attention_two_pass1(hipStream_t s, const AttentionParams& p, float* partials, float* sums, float* maxs);
 uzu_status attention_two_pass2(hipStream_t s, const float* partials, const float* sums, const float* maxs, void* out,
