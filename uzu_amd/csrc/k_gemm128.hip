@@ -155,9 +155,8 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
     const bool gated = p.act_mul != 0;
     const uint32_t H = N / 2;
     const uint32_t m_tiles = (M + BM - 1) / BM, n_tiles = gated ? (H + 63) / 64 : (N + BN - 1) / BN;
-    // Workgroups are dealt to the 8 XCDs round-robin and an XCD runs ~64 of them at a time, so tile numbering decides
-    // what each 4 MB L2 sees: XCD x works through super-tiles x, x + 8, ... of TM x TN tiles (8 x 8 when the matrix is
-    // large enough) -- the 64 resident workgroups then share 8 activation row blocks and 8 weight column blocks.
+    // Workgroups are dealt to the 8 XCDs round-robin and an XCD runs ~64 of them at a time, so tile numbering decides what each 4 MB L2 sees: every XCD has an equal share of the
+    // tiles, about 8 x 8 of them at a time (gemm_tile_order.h).
     uint32_t m_t, n_t;
     bool live;
     if (PP) { // the tile map runs over PAIRS of column tiles; half h takes column tile 2 pair + h of the same row block
@@ -751,7 +750,7 @@ void gemm_q_mfma128_plan_query(const MatmulParams& p, int num_cus, uint32_t* lar
     *splits = gemm128_splits(p, num_cus);
     *form = (uint32_t)gemm128_form(p, num_cus, *splits);
     const uint32_t m_tiles = (p.m + BM - 1) / BM, n_tiles = p.act_mul ? (p.n / 2 + 63) / 64 : (p.n + BN - 1) / BN;
-    *workgroups = (*form == 1 ? m_tiles * ((n_tiles + 1) / 2) : m_tiles * n_tiles) * *splits; // tiles with work (the launch grid pads them to whole super-tiles)
+    *workgroups = (*form == 1 ? m_tiles * ((n_tiles + 1) / 2) : m_tiles * n_tiles) * *splits; // tiles with work (the launch grid pads them to a multiple of the XCDs)
 }
 bool gemm_q_mfma128_supported(const MatmulParams& p, int num_cus) {
     if (p.m < 128 || p.n < 64) return false;

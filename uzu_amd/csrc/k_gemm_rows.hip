@@ -1,4 +1,4 @@
-// k_gemm_rows.hip -- quantised matmul for dozens to hundreds of activation rows: a register-fed matrix-core kernel without operand staging.
+// k_gemm_rows.hip -- quantised matmul for dozens to hundreds of activation rows: a register-fed matrix-core kernel without operand staging, and for hundreds of rows its staged sibling (below).
 //
 // Where it sits: behind the few-rows kernel (k_gemv_rows.hip, M <= 16; wide matrices come here from 2 rows on) and in front of the large tiles (k_gemm128.hip).  At these sizes a linear of a 1024-wide
 // model is 1 .. 15 GFLOP and 1 .. 4 MB of codes -- a microsecond or two of either -- and what a tile kernel spends is its chain: a k-step of 64 through LDS with
@@ -15,7 +15,7 @@
 //   * the next step's loads are in flight while a step is computed, waves never meet before the end, and K is cut KW ways over the waves of a workgroup
 //     (added through LDS in wave order) and `splits` ways over workgroups (f32 partial tiles, added in split order by the reduction that also applies the next
 //     Normalization): the cuts are chosen so that the chip has a workgroup per CU and a wave's chain is a few steps.
-// What bounds it: below ~100 rows the launch and two or three dependent loads; above, the L2 traffic of unshared operands (~7 TB/s at 0.3 PFLOP/s).
+// What bounds it: below ~100 rows the launch and two or three dependent loads; above, the L2 traffic of unshared operands (~7 TB/s at 0.3 PFLOP/s), which the staged kernel shares.
 // Measured, us per launch, 64 x 64 tiles -> here (weights not in cache): 1024 x 3584, M = 37: 38.0 -> 8.5; 1024 x 2048: 23.7 -> 6.9; 7168 x 1024 + GatedActMul:
 // 14.3 + 4.7 -> 8.1; 8224 x 1024: 14.5 -> 10.3; 4096 x 14336: 163 -> 33; a 37-token prompt of Qwen3.5-0.8B 3.84 -> 2.22 ms.
 #include <algorithm>

@@ -73,7 +73,7 @@ uzu_status matmul(hipStream_t s, const MatmulParams& p, int num_cus, const char*
 // true when matmul() can run `p` with the fused GatedActMul epilogue (act_mul = 1: D = [m, n/2]); otherwise run the matmul and
 // gated_act_mul separately
 bool matmul_act_mul_supported(hipStream_t s, const MatmulParams& p, int num_cus);
-// k_gemm_rows.hip: 17 to hundreds of activation rows (wide matrices: 2 and more) against int4 codes in groups of 128, register-fed
+// k_gemm_rows.hip: 17 to hundreds of activation rows (wide matrices: 2 and more) against int4 codes in groups of 128, register-fed or (from 128 rows on) staged in tiles of 64 x 128
 bool gemm_rows_preferred(const MatmulParams& p, int num_cus);
 uzu_status gemm_rows(hipStream_t s, const MatmulParams& p, int num_cus);
 void gemm_rows_plan_query(const MatmulParams& p, int num_cus, uint32_t* splits, uint32_t* workgroups);
