@@ -433,7 +433,7 @@ bool staged_fits(const MatmulParams& p) { return p.m >= 128 && !p.act_mul && (ui
 
 // The cuts: 16-row blocks per wave, waves per tile, K splits over workgroups.  A launch wants about a workgroup per CU; narrow problems take two blocks per wave,
 // then all four waves on one tile, then splits (measured at N 1024 .. 8224, K 1024 .. 3584, M 20 .. 1021).
-GemmRowsPlan gemm_rows_plan(const MatmulParams& p, int num_cus) {
+GemmRowsPlan gemm_rows_plan(const MatmulParams& p, int num_cus, bool shares_fit = true) { // (no shares of K over workgroups where there is no room for their sums)
     GemmRowsPlan q{};
     const uint32_t blocks = ((p.act_mul ? p.n / 2 : p.n) + 15) / 16, token_tiles = (p.m + 31) / 32, pairs = p.k / 256, cus = (uint32_t)num_cus;
     auto tiles = [&](uint32_t nb) { const uint32_t ob = p.act_mul ? nb / 2 : nb; return ((blocks + ob - 1) / ob) * token_tiles; };
@@ -444,7 +444,7 @@ GemmRowsPlan gemm_rows_plan(const MatmulParams& p, int num_cus) {
     q.splits = 1;
     // shares of K over workgroups from K = 2048 on (below, a share's launch of its own costs more than the steps it takes off: 1024 x 1024 5.7 us whole, 6.2 in two shares, 1024 x 1536 6.7
     // and 7.0), at the most two pairs for a share's waves together: 1024 x 2048 6.9 in four, 8.5 in two; 1024 x 3072 7.7 and 9.1 in two; 512 x 3584 8.3 and 9.4 in two (33 rows)
-    if (!p.act_mul && (q.nb == 2 || long_k) && pairs >= 8)
+    if (shares_fit && !p.act_mul && (q.nb == 2 || long_k) && pairs >= 8)
         while (q.splits * 2 * t <= cus && q.splits * 4 <= pairs) q.splits *= 2;
     const uint32_t side_by_side = 4 / q.kw, ob = p.act_mul ? q.nb / 2 : q.nb;
     q.workgroups = ((blocks + ob * side_by_side - 1) / (ob * side_by_side)) * token_tiles * q.splits;
@@ -459,7 +459,7 @@ GemmRowsPlan gemm_rows_plan(const MatmulParams& p, int num_cus) {
     const uint32_t full = q.workgroups / cus, rest = q.workgroups % cus;
     double best = 4.0 + p.k / 1024.0 * 15.0 / (q.kw * q.splits) * (q.nb / 4.0) * (!rest ? full : full ? full + 0.9 : 1.0) + shares(q.splits);
     const uint32_t staged = staged_tiles(p), groups = p.k / 128;
-    for (uint32_t splits = 1; splits <= 16 && 2 * splits <= groups; ++splits) {
+    for (uint32_t splits = 1; splits <= (shares_fit ? 16u : 1u) && 2 * splits <= groups; ++splits) {
         const uint32_t each = (groups + splits - 1) / splits, per_cu = (staged * splits + cus - 1) / cus;
         const double us = (per_cu == 1 ? 4.5 + each : 6.0 + 0.715 * each * per_cu) + shares(splits);
         if (us < best) best = us, q.staged = true, q.splits = splits, q.workgroups = staged * splits;
@@ -558,7 +558,7 @@ uzu_status gemm_rows(hipStream_t s, const MatmulParams& p, int num_cus) {
     const size_t total = (size_t)p.m * p.n;
     if (plan.splits > 1) {
         q.partials = (float*)stream_workspace(s, (size_t)plan.splits * total * 4);
-        if (!q.partials) q.splits = 1, plan.staged = false; // (a stream under capture has no workspace)
+        if (!q.partials) plan = gemm_rows_plan(p, num_cus, false), q.splits = 1; // (a stream under capture has no workspace)
     }
     uzu_status st;
     if (plan.staged) st = launch_staged(s, q, p.b_kind);
