@@ -90,6 +90,23 @@ def test_exact_mode_features_draft_and_trie_are_bit_identical(hip_ctx, preset):
         _set_exact(False)
 
 
+@pytest.mark.parametrize("rows", [13, 40])
+def test_filed_rows_of_a_layer_whose_projection_is_cut_along_k(hip_ctx, rows):
+    """A width at which the next layer's Normalization would ride on the down projection's shares of K and add its rows to the residual ones: not from a layer that files residual + output
+    (engine_forward.hip), which would count the output twice.  The bound of the test below."""
+    cfg = S.tiny_qwen(model_dim=1024, hidden_dim=2048, group_size=128, seed=34)
+    bundle = S.build_model(cfg)
+    om, hm = O.OracleModel(bundle), HipModel(hip_ctx, bundle)
+    om.capture_features(True)
+    hm.set_feature_layers([0, 1, 2])
+    prompt = _prompt(cfg, rows)
+    om.prefill(prompt), hm.prefill(prompt)
+    for l, a in enumerate(hm.hidden_features()):
+        b = om.hidden_feature(l)
+        assert np.abs(f32(a).astype(np.float64) - f32(b)).max() <= 2.0 ** -5 * np.abs(f32(b)).max(), l
+    hm.close()
+
+
 @pytest.mark.parametrize("preset", list(PRESETS))
 def test_production_kernels_within_tolerance(hip_ctx, preset):
     cfg = PRESETS[preset]()
