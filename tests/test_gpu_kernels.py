@@ -1154,12 +1154,13 @@ def test_delta_net_prefill_wide_values_and_the_split(hip_ctx, T, Hv, Hk, Dv):
     np.testing.assert_allclose(state, want_state, rtol=1e-4, atol=1e-4)
 
 
-@pytest.mark.parametrize("T", [17, 63, 130])
+@pytest.mark.parametrize("T,Dv,t", [(17, 32, 11), (63, 32, 57), (130, 32, 124), (790, 128, 200), (790, 128, 784)])
 @pytest.mark.parametrize("plant", ["value inf", "value nan", "key inf", "query nan", "beta nan", "decay nan", "decay inf", "decay above 1", "decay below 0", "decay 0", "state inf"])
-def test_delta_net_prefill_unusual_numbers(hip_ctx, T, plant):
+def test_delta_net_prefill_unusual_numbers(hip_ctx, T, Dv, t, plant):
     """The chunked form against the token-by-token oracle where a chunk's zeros or logarithms could change the answer: an infinity or a NaN reaches its own token's outputs and later
-    ones (and of a value only its column), never an earlier token; decays that are no exp(-x) with x > 0 multiply the state as they are."""
-    Hv, Hk, Dv, t = 4, 2, 32, T - 6
+    ones (and of a value only its column), never an earlier token; decays that are no exp(-x) with x > 0 multiply the state as they are.  In one segment (up to 736 tokens) and in either
+    of two (tokens 0 .. 543 and the rest of 790)."""
+    Hv, Hk = 4, 2
     z = delta_net_inputs(np.random.default_rng(T), T, Hv, Hk, Dv, 0.1)
     name, what = plant.split(" ", 1)
     x = {"inf": np.inf, "nan": np.nan, "above 1": 1.25, "below 0": -0.5, "0": 0.0}[what]

@@ -13,7 +13,8 @@
 // Dv + 128 right-hand sides each).  `dn_chunk_scan_kernel` then walks the chunks with two dependent products per chunk, G S^T and D^T K, and the outputs beside them.
 // Same algebra, different rounding order: the state is no further from 64 bits than the recurrence's (dn_chunk_scan_kernel).  Decays are carried in log space
 // (log 0 = -104, whose exponential is 0 in f32) so that products over a chunk cannot underflow into 0 / 0.  An infinity or a NaN would reach the whole chunk through the
-// zeros of G and P, where the recurrence hands it on from its token and its value column only: a workgroup of the plain scan that meets one walks its columns again token by token.
+// zeros of G and P, where the recurrence hands it on from its token and its value column only: the columns of a scan workgroup that meets one are walked again token by token
+// (dn_recurrence_tile), by the same workgroup in the plain scan and by the fix-up in the split one.
 #include <stdlib.h>
 
 #include <type_traits>
@@ -32,6 +33,7 @@ constexpr int KP = DKC + 4;   // LDS row pitch of K / Q / S rows in floats (conf
 constexpr int TP = CC + 4;    // LDS row pitch of the 32 x 32 matrices (16-byte rows)
 // per (chunk, value head): -G [32][128], P [32][32], A, W = A_C / A, the decays a, the strengths b; behind all of them U [32][Dv] per (chunk, value head)
 constexpr int WS_P = CC * DKC, WS_A = WS_P + CC * CC, WS_W = WS_A + CC, WS_DECAY = WS_W + CC, WS_FLOATS = WS_DECAY + 2 * CC;
+constexpr int SPLIT_OFF = 3 * (DKC / 16) * 4; // ScanSplit::off of a head
 } // namespace
 
 // Sequence split.  The chain of n chunk steps is the scan's whole cost (1.46 us per chunk with half of the CUs idle), and the recurrence is AFFINE in the state, row by
@@ -49,6 +51,7 @@ struct ScanSplit {
     float* h_end;       // [Hv][Dk][Dk]  final homogeneous rows of segment 1 (started from the identity)
     float* o32;         // [T][Hv Dv] f32: the real tiles' own outputs (rows of segment 1: Z_t q_t; segment 0's rows are not read again)
     float* u;           // [T - 32 mid][Hv Dk] f32: H_t q_t
+    uint32_t* off;      // [Hv][segment 0, segment 1, homogeneous][8 tiles][4 waves]: not 0 where a wave ends on a state value that is no number, or too large for the fix-up's products
 };
 static uint32_t split_mid_chunk(uint32_t n_chunks, uint32_t head_v_dim) {
     static const uint32_t min_chunks = [] { // chunks from which the scan is split (0 = never; A/B runs): the fix-up launch is 8 us + 0.12 a chunk, the shorter chain saves 0.5 a chunk
@@ -66,7 +69,7 @@ static uint32_t split_mid_chunk(uint32_t n_chunks, uint32_t head_v_dim) {
     return mid < 1 ? 1u : mid > n_chunks - 1 ? n_chunks - 1 : mid;
 }
 static size_t split_floats(uint32_t num_v_heads, uint32_t value_dim, uint32_t suffix_len) {
-    return (size_t)2 * value_dim * DKC + (size_t)num_v_heads * DKC * DKC + (size_t)suffix_len * value_dim + (size_t)suffix_len * num_v_heads * DKC;
+    return (size_t)2 * value_dim * DKC + (size_t)num_v_heads * DKC * DKC + (size_t)suffix_len * value_dim + (size_t)suffix_len * num_v_heads * DKC + (size_t)num_v_heads * SPLIT_OFF;
 }
 size_t delta_net_chunk_workspace_bytes(uint32_t num_v_heads, uint32_t value_dim, uint32_t suffix_len) {
     return ((size_t)((suffix_len + CC - 1) / CC) * ((size_t)num_v_heads * WS_FLOATS + (size_t)CC * value_dim) + split_floats(num_v_heads, value_dim, suffix_len)) * sizeof(float);
@@ -355,6 +358,36 @@ __global__ void __launch_bounds__(256, 3) dn_chunk_prep_kernel(const float* q_no
     }
 }
 
+// The recurrence token by token from the state in memory: value columns [dv_base, dv_base + 16) of head hv, 256 threads, 16 lanes a column.
+// (v_row_stride != 0: `in_proj` is the out-of-place conv buffer, rows of conv_dim channels in the same q | k | v order)
+__device__ __forceinline__ void dn_recurrence_tile(const float* q_norm, const float* k_norm, const uint16_t* in_proj, const float* ws, float* state, uint16_t* out, uint32_t hv, uint32_t dv_base,
+                                                uint32_t num_v_heads, uint32_t num_k_heads, uint32_t head_v_dim, uint32_t key_dim, uint32_t value_dim, uint32_t suffix_len, uint32_t v_row_stride) {
+    const size_t v_stride = v_row_stride ? (size_t)v_row_stride : (size_t)2 * key_dim + 2 * value_dim + 2 * num_v_heads;
+    const uint32_t hk = hv / (num_v_heads / num_k_heads), col = threadIdx.x >> 4, part = threadIdx.x & 15;
+    float* srow = state + ((size_t)hv * head_v_dim + dv_base + col) * DKC + 8 * part;
+    float sv[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sv[e] = srow[e];
+    for (uint32_t t = 0; t < suffix_len; ++t) {
+        const float* w = ws + ((size_t)(t / CC) * num_v_heads + hv) * WS_FLOATS + WS_DECAY + t % CC;
+        const float *kr = k_norm + (size_t)t * key_dim + hk * DKC + 8 * part, *qr = q_norm + (size_t)t * key_dim + hk * DKC + 8 * part;
+        const float a = w[0], b = w[CC], v = bf16_to_f32(in_proj[(size_t)t * v_stride + 2 * key_dim + hv * head_v_dim + dv_base + col]);
+        float sk = 0.f, o = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sk = fmaf(sv[e], kr[e], sk);
+        const float d = b * (v - a * group_sum<16>(sk));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            sv[e] = a * sv[e] + d * kr[e];
+            o = fmaf(sv[e], qr[e], o);
+        }
+        o = group_sum<16>(o);
+        if (part == 0) out[(size_t)t * value_dim + hv * head_v_dim + dv_base + col] = f32_to_bf16(o);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) srow[e] = sv[e];
+}
+
 // The scan, v_mfma_f32_16x16x4_f32 throughout -- f32 operands, exact f32 products, f32 accumulation.  Four waves own 16 value columns of a head:
 //   stage 1  waves 0, 1: D = U - G S^T for 16 tokens each, 32 MFMAs; waves 2, 3: Q S^T
 //   stage 2  S = A_C S + (D W)^T K   every wave owns 32 dk of the state in its accumulators, 2 x 8 MFMAs
@@ -419,7 +452,7 @@ __global__ void __launch_bounds__(DUAL ? 512 : 256) dn_chunk_scan_kernel(const f
     };
 
     auto mfma4 = [](float a, float b, f32x4_v c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); };
-    float off_sum = 0.f; // 0, or NaN behind an output or a state value that is no number
+    float off_sum = 0.f; // plain scan: 0, or NaN behind an output or a state value that is no number
     const int tb = 16 * (wave & 1);
     const uint32_t u_keep = homog ? 0u : 0xFFFFFFFFu;
     // segment 0's outputs (and the plain scan's) are final; segment 1's go to f32 rows that the fix-up finishes
@@ -522,7 +555,8 @@ __global__ void __launch_bounds__(DUAL ? 512 : 256) dn_chunk_scan_kernel(const f
                 for (int r = 0; r < 4; ++r) {
                     if (ragged && t + r >= suffix_len) continue;
                     if constexpr (SEG1) o32[(size_t)(t + r) * o_stride] = y[r];
-                    else out16[(size_t)(t + r) * value_dim] = f32_to_bf16(y[r]), off_sum = fmaf(y[r], 0.f, off_sum);
+                    else out16[(size_t)(t + r) * value_dim] = f32_to_bf16(y[r]);
+                    if constexpr (!DUAL) off_sum = fmaf(y[r], 0.f, off_sum);
                 }
             }
             step_barrier();
@@ -553,9 +587,16 @@ __global__ void __launch_bounds__(DUAL ? 512 : 256) dn_chunk_scan_kernel(const f
     } else if (wave < 2) walk(yes(), no());
     else walk(no(), no());
     if constexpr (DUAL) {
+        // (whatever of a chunk is no number, but for a query, which its own outputs alone see, makes a row of D none, and D stays in the state: 0 times it is none either)
+        uint32_t peak = 0; // the largest magnitude's bits; a NaN's are larger than any
         float* sfin = homog ? sp.h_end + ((size_t)hv * DKC + dv_base + 4 * kq) * DKC + 32 * wave + 2 * i16 : (seg1 ? sp.z_end : sp.mid_state) + s_at;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) *(float2*)(sfin + (size_t)r * DKC) = make_float2(creg[0][r], creg[1][r]);
+        for (int r = 0; r < 4; ++r) {
+            *(float2*)(sfin + (size_t)r * DKC) = make_float2(creg[0][r], creg[1][r]);
+            peak = max(peak, max(f32_to_bits(creg[0][r]) & 0x7FFFFFFFu, f32_to_bits(creg[1][r]) & 0x7FFFFFFFu));
+        }
+        const bool off = __ballot(peak > f32_to_bits(0x1p60f)) != 0; // (128 products of two numbers up to that are a number)
+        if (lane == 0) sp.off[((hv * 3 + (homog ? 2 : seg1 ? 1 : 0)) * (DKC / 16) + dv_base / 16) * 4 + wave] = off;
         return;
     }
 #pragma unroll
@@ -565,34 +606,9 @@ __global__ void __launch_bounds__(DUAL ? 512 : 256) dn_chunk_scan_kernel(const f
     const bool off = __ballot(!(off_sum == 0.f)) != 0;
     if (lane == 0) s_off[wave] = off;
     lds_barrier();
-    if (s_off[0] | s_off[1] | s_off[2] | s_off[3]) { // the recurrence from the state in memory, 16 lanes a value column
+    if (s_off[0] | s_off[1] | s_off[2] | s_off[3]) {
         __syncthreads(); // (every wave's own outputs have been written: those below replace them)
-        const uint32_t conv_dim = 2 * key_dim + value_dim;
-        // (v_row_stride != 0: `in_proj` is the out-of-place conv buffer, rows of conv_dim channels in the same q | k | v order)
-        const size_t total_proj_dim = v_row_stride ? (size_t)v_row_stride : (size_t)conv_dim + value_dim + 2 * num_v_heads;
-        const uint32_t col = tid >> 4, part = tid & 15;
-        float* srow = state + ((size_t)hv * head_v_dim + dv_base + col) * DKC + 8 * part;
-        float sv[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sv[e] = srow[e];
-        for (uint32_t t = 0; t < suffix_len; ++t) {
-            const float* w = ws + ((size_t)(t / CC) * num_v_heads + hv) * WS_FLOATS + WS_DECAY + t % CC;
-            const float *kr = k_norm + (size_t)t * key_dim + hk * DKC + 8 * part, *qr = q_norm + (size_t)t * key_dim + hk * DKC + 8 * part;
-            const float a = w[0], b = w[CC], v = bf16_to_f32(in_proj[(size_t)t * total_proj_dim + 2 * key_dim + hv * head_v_dim + dv_base + col]);
-            float sk = 0.f, o = 0.f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) sk = fmaf(sv[e], kr[e], sk);
-            const float d = b * (v - a * group_sum<16>(sk));
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                sv[e] = a * sv[e] + d * kr[e];
-                o = fmaf(sv[e], qr[e], o);
-            }
-            o = group_sum<16>(o);
-            if (part == 0) out[(size_t)t * value_dim + hv * head_v_dim + dv_base + col] = f32_to_bf16(o);
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) srow[e] = sv[e];
+        dn_recurrence_tile(q_norm, k_norm, in_proj, ws, state, out, hv, dv_base, num_v_heads, num_k_heads, head_v_dim, key_dim, value_dim, suffix_len, v_row_stride);
         return;
     }
 #pragma unroll
@@ -607,14 +623,22 @@ __global__ void __launch_bounds__(DUAL ? 512 : 256) dn_chunk_scan_kernel(const f
 //   the last Dk / 16 blocks: 16 state columns:         S[dv, dk] = z_end[dv, dk] + sum_j S_mid[dv, j] h_end[j, dk]       A = S_mid rows, B = h_end columns
 constexpr int FIX_TOK = 64;
 constexpr size_t kFixLdsBytes = (size_t)DKC * KP * sizeof(float); // S_mid of one head, rows 4 banks apart
-__global__ void __launch_bounds__(256) dn_chunk_fixup_kernel(ScanSplit sp, float* state, uint16_t* out, uint32_t num_v_heads, uint32_t head_v_dim, uint32_t value_dim,
-                                                             uint32_t suffix_len) {
+// Value tiles that ScanSplit::off names are left alone, and block i of the last ones walks tile i token by token instead: the state in memory is still the one before the pass there.
+__global__ void __launch_bounds__(256) dn_chunk_fixup_kernel(ScanSplit sp, float* state, uint16_t* out, uint32_t num_v_heads, uint32_t head_v_dim, uint32_t value_dim, uint32_t suffix_len,
+                                                             const float* q_norm, const float* k_norm, const uint16_t* in_proj, const float* ws, uint32_t num_k_heads, uint32_t key_dim,
+                                                             uint32_t v_row_stride) {
     constexpr uint32_t DV_TILES = DKC / 16;
     extern __shared__ __attribute__((aligned(16))) float fix_smem[]; // [Dv][KP]: S_mid of the head (token blocks)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i16 = lane & 15, kq = lane >> 4;
     const uint32_t hv = blockIdx.y, t_mid = sp.mid_chunk * CC, T2 = suffix_len - t_mid;
     const uint32_t tok_blocks = (T2 + FIX_TOK - 1) / FIX_TOK;
     const float* smid = sp.mid_state + (size_t)hv * head_v_dim * DKC;
+    uint4 off4 = make_uint4(0, 0, 0, 0);
+    if (lane < 3 * (int)DV_TILES) off4 = *(const uint4*)(sp.off + (size_t)hv * SPLIT_OFF + 4 * lane);
+    auto off_tiles = [&]() -> uint32_t { // (a homogeneous tile serves every value tile)
+        const uint64_t b = __ballot((off4.x | off4.y | off4.z | off4.w) != 0);
+        return b >> (2 * DV_TILES) ? (1u << DV_TILES) - 1 : (uint32_t)(b | b >> DV_TILES) & ((1u << DV_TILES) - 1);
+    };
     auto mfma4 = [](float a, float b, f32x4_v c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); };
     // the token blocks come first in the grid: they are the long ones (one global round trip + 256 matrix instructions per wave)
     if (blockIdx.x < tok_blocks) {
@@ -643,6 +667,7 @@ __global__ void __launch_bounds__(256) dn_chunk_fixup_kernel(ScanSplit sp, float
             const uint32_t e = (tid + 256 * r) * 4; // element of the [Dv][Dk] state
             *(f32x4_v*)(fix_smem + (e / DKC) * KP + e % DKC) = sm[r];
         }
+        const uint32_t skip = off_tiles();
         lds_barrier();
 #pragma unroll
         for (uint32_t vt = 0; vt < DV_TILES; ++vt) {
@@ -657,7 +682,7 @@ __global__ void __launch_bounds__(256) dn_chunk_fixup_kernel(ScanSplit sp, float
 #pragma unroll
             for (int r = 0; r < 4; ++r) { // rows = tokens 4 kq + r of the tile, column = dv
                 const uint32_t t = tok + 4 * kq + r;
-                if (t < T2) out[(size_t)(t_mid + t) * value_dim + (size_t)hv * head_v_dim + vt * 16 + i16] = f32_to_bf16(prev[vt][r] + acc[r]);
+                if (t < T2 && !(skip >> vt & 1)) out[(size_t)(t_mid + t) * value_dim + (size_t)hv * head_v_dim + vt * 16 + i16] = f32_to_bf16(prev[vt][r] + acc[r]);
             }
         }
     } else {
@@ -680,6 +705,7 @@ __global__ void __launch_bounds__(256) dn_chunk_fixup_kernel(ScanSplit sp, float
             for (int r = 0; r < 4; ++r) zv[h][r] = sp.z_end[((size_t)hv * head_v_dim + vt * 16 + 4 * kq + r) * DKC + dk0 + i16];
         }
         __builtin_amdgcn_sched_barrier(0); // (the scheduler would sink the loads back to their uses)
+        const uint32_t skip = off_tiles();
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const uint32_t vt = wave + 4 * h;
@@ -690,8 +716,10 @@ __global__ void __launch_bounds__(256) dn_chunk_fixup_kernel(ScanSplit sp, float
                 for (int e = 0; e < 4; ++e) acc = mfma4(sa[h][q][e], hb[4 * q + e], acc);
 #pragma unroll
             for (int r = 0; r < 4; ++r) // rows dv = 16 vt + 4 kq + r, column dk
-                state[((size_t)hv * head_v_dim + vt * 16 + 4 * kq + r) * DKC + dk0 + i16] = zv[h][r] + acc[r];
+                if (!(skip >> vt & 1)) state[((size_t)hv * head_v_dim + vt * 16 + 4 * kq + r) * DKC + dk0 + i16] = zv[h][r] + acc[r];
         }
+        const uint32_t tile = blockIdx.x - tok_blocks;
+        if (skip >> tile & 1) dn_recurrence_tile(q_norm, k_norm, in_proj, ws, state, out, hv, tile * 16, num_v_heads, num_k_heads, head_v_dim, key_dim, value_dim, suffix_len, v_row_stride);
     }
 }
 
@@ -744,7 +772,8 @@ static uzu_status prefill_chunked(hipStream_t s, float* q_norm, float* k_norm, c
         sp.z_end = w, w += (size_t)value_dim * DKC;
         sp.h_end = w, w += (size_t)num_v_heads * DKC * DKC;
         sp.o32 = w, w += (size_t)suffix_len * value_dim;
-        sp.u = w;
+        sp.u = w, w += (size_t)suffix_len * num_v_heads * DKC;
+        sp.off = (uint32_t*)w;
     }
     UZU_PROPAGATE(launch_check([&] {
         hipLaunchKernelGGL(dn_chunk_scan_kernel<true>, dim3(2 * (head_v_dim / 16), num_v_heads), dim3(512), 0, s, q_norm, k_norm, v_rows, (const float*)workspace, (const float*)u_ws,
@@ -753,7 +782,7 @@ static uzu_status prefill_chunked(hipStream_t s, float* q_norm, float* k_norm, c
     const uint32_t t_mid = sp.mid_chunk * CC, t2 = suffix_len - t_mid;
     return launch_check([&] {
         hipLaunchKernelGGL(dn_chunk_fixup_kernel, dim3((t2 + FIX_TOK - 1) / FIX_TOK + DKC / 16, num_v_heads), dim3(256), kFixLdsBytes, s, sp, state, out,
-                           num_v_heads, head_v_dim, value_dim, suffix_len);
+                           num_v_heads, head_v_dim, value_dim, suffix_len, (const float*)q_norm, (const float*)k_norm, v_rows, (const float*)workspace, num_k_heads, key_dim, v_stride);
     }, "delta_net_chunk_fixup");
 }
 
