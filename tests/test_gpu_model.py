@@ -581,11 +581,11 @@ def test_llama3_8b_full_depth_matches_oracle_fixture(hip_ctx, name):
 ROBUST_PROMPT_MULTIPLIERS = {"tiny-qwen": (21, 13, 37), "tiny-llama": (149, 373, 223)}
 
 
-@pytest.mark.parametrize("nseq,count,gate", [(3, 250, False), (9, 70, False), (3, 250, True)])
-def test_batched_prefill_with_the_sequences_attention_in_one_launch(hip_ctx, nseq, count, gate):
+@pytest.mark.parametrize("nseq,count,gate,head_dim", [(3, 250, False, 64), (9, 70, False, 64), (3, 250, True, 64), (9, 200, False, 64), (9, 130, True, 64), (3, 250, False, 128), (3, 250, True, 256)])
+def test_batched_prefill_with_the_sequences_attention_in_one_launch(hip_ctx, nseq, count, gate, head_dim):
     """Sequences of a batched pass whose attention goes out in one launch (csrc/k_attention_mfma.hip: AttentionSeqs): behind contexts of different lengths, a ragged last query tile, more
-    sequences than a launch takes, with and without the output gate; the next step's logits against each sequence alone (the projections see other row counts: tolerance-class)."""
-    cfg = S.tiny_llama(num_heads=32, num_groups=8, max_context_length=400, has_gate=gate, seed=45)
+    sequences than a launch takes, with and without the output gate, each head width; the next step's logits against each sequence alone (the projections see other row counts: tolerance-class)."""
+    cfg = S.tiny_llama(num_heads=32, num_groups=8, head_dim=head_dim, max_context_length=400, has_gate=gate, seed=45)
     hm = HipModel(hip_ctx, S.build_model(cfg), MODEL_BATCH(nseq))
     base = S.synthetic_prompt(count, cfg.vocab_size).astype(np.int64)
     prompts = np.stack([(base * (2 * i + 3) + 11 * i) % cfg.vocab_size for i in range(nseq)]).astype(np.uint32)
@@ -612,6 +612,25 @@ def test_batched_prefill_with_the_sequences_attention_in_one_launch(hip_ctx, nse
         hm.prefill(prompts[i])
         hm.prefill(np.array([first[i]], np.uint32))
         assert logits_close(hm.read_logits(), batched).all()
+
+
+def test_attention_of_sequences_is_joined_where_they_cover_the_chip(hip_ctx):
+    """Sequences of 70 rows, 24 workgroups each: eight cover three CUs of four and go out as one launch, nine as two; six and seven do not and go out one by one (engine_forward.hip:
+    attention_mixer).  Counted in the pass's launches: what a sequence of its own adds is linear in their number."""
+    cfg = S.tiny_llama(num_heads=32, num_groups=8, max_context_length=80, seed=45)
+    hm = HipModel(hip_ctx, S.build_model(cfg), MODEL_BATCH(9))
+    base = S.synthetic_prompt(70, cfg.vocab_size).astype(np.int64)
+    states, launches = [hm.new_state() for _ in range(9)], {}
+    for n in (6, 7, 8, 9):
+        for s in states:
+            s.reset()
+        hm.prefill_batch(states[:n], np.stack([(base * (2 * i + 3)) % cfg.vocab_size for i in range(n)]).astype(np.uint32))
+        launches[n] = hm.decode_launch_count
+    for s in states:
+        s.close()
+    hm.close()
+    alone = launches[7] - launches[6]
+    assert launches[8] == launches[7] + alone - 7 * cfg.num_layers and launches[9] == launches[7] + 2 * alone - 7 * cfg.num_layers, launches
 
 
 @pytest.mark.parametrize("preset", ["tiny-qwen", "tiny-llama"])

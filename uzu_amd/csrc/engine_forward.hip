@@ -289,7 +289,7 @@ uzu_status ensure_partials(uzu_hip_model* m, uint32_t rows, uint32_t head_dim) {
 
 // the sequences of a batched prefill whose attention goes out in one launch (k_attention_mfma.hip)
 struct JoinedAttention {
-    uint32_t sequences;
+    uint32_t sequences; // of a full launch
     k::AttentionParams a{};
     k::AttentionSeqs seqs{};
     size_t row0[k::AttentionSeqs::kMost];
@@ -324,18 +324,23 @@ void attention_mixer(Enc& e, DLayer& L, const uint16_t* hidden, uint16_t* out, c
     if (q.n == 0) {
         attention_core(e, L, q.count, 0, fuse_norms);
     } else {
-        JoinedAttention join{q.n};
-        for (uint32_t i = 0; i < q.n; ++i) {
-            bind_state(m, q.st[i]);
-            attention_core(e, L, q.count, (size_t)i * q.count, fuse_norms, &join);
-            if (join.seqs.n == k::AttentionSeqs::kMost || i + 1 == q.n) attention_joined(e, L, q.count, join);
+        // Launches of at most kMost sequences, as equal as they come: eight and one left over take as long as eight and a launch with an eighth of the chip.  9 sequences of 250 rows, 32
+        // heads on 8, us of attention a layer, eight and one joined / the ninth by itself with its keys split / five and four: heads of 128 40.8, 44.1, 37.8; of 256 75.3, 70.7, 65.7.
+        const uint32_t launches = (q.n + k::AttentionSeqs::kMost - 1) / k::AttentionSeqs::kMost;
+        for (uint32_t g = 0; g < launches; ++g) {
+            const uint32_t first = q.n * g / launches, end = q.n * (g + 1) / launches;
+            JoinedAttention join{std::min(q.n, k::AttentionSeqs::kMost)};
+            for (uint32_t i = first; i < end; ++i) {
+                bind_state(m, q.st[i]);
+                attention_core(e, L, q.count, (size_t)i * q.count, fuse_norms, &join);
+            }
+            attention_joined(e, L, q.count, join);
         }
     }
     // (SigmoidGate: attention_core applies it per sequence -- inside the key-split merge of a prefill pass where there is one)
     linear(e, L.out, m->attn_out, out, rows, true, post);
 }
 
-// AttentionPrepare + attention of `batch` rows of the bound sequence, which start at row `row0` of qkv / queries / attn_out
 void attention_joined(Enc& e, DLayer& L, uint32_t batch, JoinedAttention& j) {
     uzu_hip_model* m = e.m;
     if (!j.seqs.n) return;
@@ -346,6 +351,7 @@ void attention_joined(Enc& e, DLayer& L, uint32_t batch, JoinedAttention& j) {
             RUN("sigmoid_gate", 0, k::sigmoid_gate(e.s, m->gate + j.row0[i] * nq * hd, m->attn_out + j.row0[i] * nq * hd, UZU_BF16, batch * nq * hd));
     j.seqs.n = 0;
 }
+// AttentionPrepare + attention of `batch` rows of the bound sequence, which start at row `row0` of qkv / queries / attn_out
 void attention_core(Enc& e, DLayer& L, uint32_t batch, size_t row0, bool fuse_norms, JoinedAttention* join) {
     uzu_hip_model* m = e.m;
     const bool has_kv = !L.d.is_kv_sharing; // prepare_queries (mode.rs:234-259): no KV rows are written; the source layer wrote this pass's already
