@@ -101,7 +101,7 @@ def test_linear_f32_from_three_bf16_parts(hip_ctx, rows, n, k, act):
 
 
 @pytest.mark.parametrize("bf16", [0, 1])
-@pytest.mark.parametrize("rows,n,k,act", [(65, 129, 1024, 0), (129, 385, 4096, 1), (20, 64, 1152, 0), (513, 2049, 512, 0), (1030, 3900, 128, 1), (2048, 2048, 320, 0), (700, 1030, 1088, 0)])
+@pytest.mark.parametrize("rows,n,k,act", [(65, 129, 1024, 0), (129, 385, 4096, 1), (20, 64, 1152, 0), (513, 2049, 512, 0), (1030, 3900, 128, 1), (2048, 2048, 320, 0), (700, 1030, 1088, 0), (700, 765, 4096, 1)])
 def test_linear_on_eight_waves_a_tile(hip_ctx, rows, n, k, act, bf16):
     """At most a 128 x 128 tile a CU (csrc/k_linear_mfma.hip: eight_wave_splits): whole and cut into two to eight shares with uneven counts of k-steps, fewer steps than buffers, ragged last
     tiles, all 256 tiles.  Against 64 bits, with the bound of the products above (bf16 products: k of them)."""
