@@ -33,5 +33,21 @@ UZU_ORDER_HD inline bool tile_of_block(uint32_t block, uint32_t m_tiles, uint32_
     return true;
 }
 
+// Two variations for products whose weights are small beside the rows (linear_tile_order, k_linear_mfma.hip), with the same shares per XCD:
+// row by row, where a row of tiles is short; and a last column that is mostly padding behind the whole tiles, so that what goes beyond a full round of workgroups is its cheap tiles.
+enum TileOrder { kTileBlocks, kTileRows, kTileLastColumnBehind };
+UZU_ORDER_HD inline bool tile_of_block(uint32_t block, uint32_t m_tiles, uint32_t n_tiles, TileOrder order, uint32_t* m_t, uint32_t* n_t) {
+    if (order == kTileBlocks || (order == kTileLastColumnBehind && n_tiles == 1)) return tile_of_block(block, m_tiles, n_tiles, m_t, n_t);
+    const uint32_t whole = m_tiles * (order == kTileRows ? n_tiles : n_tiles - 1), more = whole % 8, xcd = block & 7, slot = block >> 3, share = whole / 8 + (xcd < more ? 1u : 0u);
+    if (order == kTileRows) {
+        const uint32_t t = xcd * (whole / 8) + (xcd < more ? xcd : more) + slot;
+        *m_t = t / n_tiles, *n_t = t % n_tiles;
+        return slot < share;
+    }
+    if (slot < share) return tile_of_block(block, m_tiles, n_tiles - 1, m_t, n_t);
+    *m_t = (slot - share) * 8 + ((xcd - more) & 7u), *n_t = n_tiles - 1;
+    return *m_t < m_tiles;
+}
+
 } // namespace k
 } // namespace uzu
