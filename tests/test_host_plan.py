@@ -168,6 +168,16 @@ def test_register_fed_kernel_below_128_rows(monkeypatch):
     assert [gemm_plan(33, 1024, k).splits for k in (1024, 1792, 2048, 3584)] == [1, 1, 4, 4]
 
 
+def test_staged_products_take_shares_that_fit_an_xcds_cus(monkeypatch):
+    """csrc/k_gemm_rows.hip: tiles are dealt to eight XCDs of 32 CUs share by share, so a share counts an eighth of its tiles rounded up: 36 tiles in seven shares or 42 in six are more than a
+    workgroup a CU on some."""
+    monkeypatch.delenv("UZU_HIP_TUNE", raising=False)
+    for m, n, k in ((400, 768, 3584), (517, 512, 3584), (400, 768, 4096), (517, 512, 7168), (300, 1024, 3584)):
+        p = gemm_plan(m, n, k)
+        tiles = -(-m // 64) * -(-n // 128)
+        assert p.large_tile == 0 and p.workgroups == tiles * p.splits and p.splits > 4 and -(-tiles // 8) * p.splits <= CUS // 8, (m, n, k, p.splits)
+
+
 def test_prefill_gemm_plan_bad_arguments():
     lib = _ffi.lib()
     lib.uzu_hip_prefill_gemm_plan.argtypes = [C.c_uint32] * 7 + [C.POINTER(GemmPlan)]

@@ -458,9 +458,10 @@ GemmRowsPlan gemm_rows_plan(const MatmulParams& p, int num_cus, bool shares_fit 
     auto shares = [&](uint32_t splits) { const double mb = 4e-6 * p.m * p.n * splits; return splits == 1 ? 0.0 : mb / 3 + (norm ? mb / 8 : 2.5 + mb / 4); };
     const uint32_t full = q.workgroups / cus, rest = q.workgroups % cus;
     double best = 4.0 + p.k / 1024.0 * 15.0 / (q.kw * q.splits) * (q.nb / 4.0) * (!rest ? full : full ? full + 0.9 : 1.0) + shares(q.splits);
-    const uint32_t staged = staged_tiles(p), groups = p.k / 128;
+    // (an XCD has an eighth of a share's tiles, rounded up: 400 x 768 x 3584 in six shares of 42 tiles, 36 workgroups on some XCDs' 32 CUs, 17.9 us, in five 15.4)
+    const uint32_t staged = staged_tiles(p), groups = p.k / 128, xcd_cus = std::max(cus / 8, 1u);
     for (uint32_t splits = 1; splits <= (shares_fit ? 16u : 1u) && 2 * splits <= groups; ++splits) {
-        const uint32_t each = (groups + splits - 1) / splits, per_cu = (staged * splits + cus - 1) / cus;
+        const uint32_t each = (groups + splits - 1) / splits, per_cu = ((staged + 7) / 8 * splits + xcd_cus - 1) / xcd_cus;
         const double us = (per_cu == 1 ? 4.5 + each : 6.0 + 0.715 * each * per_cu) + shares(splits);
         if (us < best) best = us, q.staged = true, q.splits = splits, q.workgroups = staged * splits;
     }
