@@ -317,6 +317,23 @@ def test_gemm_dma_forms_are_bit_identical_to_the_register_staged_ones(hip_ctx, m
     assert (want == base).mean() >= 0.97
 
 
+@pytest.mark.parametrize("n,k,m,misaligned", [(3072, 256, 1021, False), (6152, 256, 641, False), (8200, 256, 520, True), (6144, 3072, 1500, True)])
+def test_gemm_register_staged_form_is_bit_identical_to_the_dma_one(hip_ctx, n, k, m, misaligned, monkeypatch):
+    """int4 in groups of 128 whose tiles leave no CU two of them, or whose scales lie off a 4-byte boundary (also where eight waves would take a tile): the register-staged four-wave
+    kernel (k_gemm128.hip: takes_dma) against the DMA form, ragged rows and columns."""
+    rng = np.random.default_rng(n + k + m)
+    q, a = quant_matrix(rng, n, k, 4, 128, 2), activations(rng, m, k)
+    monkeypatch.setenv("UZU_HIP_TUNE", "gemm_form=0")
+    base = hip_matmul(hip_ctx, a, q, m)
+    monkeypatch.delenv("UZU_HIP_TUNE")
+    kern = B.MatmulKernel.new(hip_ctx, B.BF16, B.BF16, B.BF16)
+    ba, bw, bd = (hip_ctx.buffer_from(z) for z in (a, q["weights"], np.zeros((m, n), np.uint16)))
+    scales = np.concatenate([np.zeros(1, np.uint16), q["scales"].ravel()]) if misaligned else q["scales"]
+    bs = hip_ctx.buffer_from(scales)
+    run(hip_ctx, lambda cb: kern.encode(cb, a=ba, b=bw, d=bd, m=m, n=n, k=k, b_kind=B.B_SCALE_SYMMETRIC, scales=(bs, 2) if misaligned else bs, mode=B.QMODE_U4, group_size=128))
+    assert np.array_equal(bd.download(np.uint16, m * n).reshape(m, n), base)
+
+
 @pytest.mark.parametrize("m", [131, 203, 1023])
 def test_gemm_mfma_row_count_not_a_multiple_of_four(hip_ctx, m):
     """The offset-term tables are padded to whole quads of rows (k_gemm128.hip pre-pass); 1023 is the second chunk of the

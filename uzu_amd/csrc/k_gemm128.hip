@@ -13,7 +13,7 @@
 //     MFMAs and no per-group offset work in the main loop.
 //   * Every global load is unconditional (rows / columns / steps clamped into range) and prefetched into a register
 //     ring; the loop is unrolled by the ring depth so that all indices are static (vmcnt waits stay counted).
-//   * int4 in groups of 128 takes the first two of the three forms (gemm128_form) with its operands by LDS DMA instead: k_gemm_dma.hip.
+//   * int4 in groups of 128 has two forms with its operands by LDS DMA besides (takes_dma): k_gemm_dma.hip.
 //   * Tiles are numbered in blocks of 8 x 8 per XCD (gemm_tile_order.h) so that the ~64 workgroups an XCD runs at a time share
 //     their activation and weight panels in its L2; few-tile shapes split K over gridDim.y with f32 partial tiles and
 //     a fixed-order reduction.  bf16 results leave through LDS as 16-byte row segments.
@@ -730,7 +730,8 @@ uint32_t gemm128_splits(const MatmulParams& p, int num_cus) {
     return best;
 }
 // Which form runs (0 = 256-thread, 1 = ping-pong, 2 = wave-specialised).  UZU_GEMM_FORM forces one (read per call: A/B runs and the bit-identity
-// test flip it); otherwise the plan, from same-box A/B runs of all three (tools/kbench KB_GEMM_AB, profiles/r5_gemm_pp_ab.txt):
+// test flip it); otherwise the plan, from same-box A/B runs of all three (tools/kbench KB_GEMM_AB, profiles/r5_gemm_pp_ab.txt).  int4 in groups of 128 by LDS DMA (takes_dma) has four waves a
+// tile for 0 and eight for 1, and the same line: 4096 rows of 14336 x 4096 540 and 522 us, 4096 x 14336 617 and 537, 6144 x 4096 252 and 255, 2048 of 8224 x 1024 64 and 73.
 //   * ping-pong (x1.05-1.16): long reductions (>= 48 k-steps: its one workgroup per CU has no second workgroup whose main loop would cover its
 //     prologue / epilogue), at least one 128 x 256 tile per CU, no split-K, no gated epilogue;
 //   * wave-specialised (x1.02-1.05): the few-tile split-K shapes (N = 1024 projections of the 0.8B model);
@@ -741,6 +742,15 @@ static int gemm128_form(const MatmulParams& p, int num_cus, uint32_t splits) {
     if (splits > 1) return 2;
     const uint32_t m_tiles = (p.m + BM - 1) / BM, n_tiles = (p.n + BN - 1) / BN;
     return (p.k / BK >= 48 && m_tiles * ((n_tiles + 1) / 2) >= (uint32_t)num_cus) ? 1 : 0;
+}
+// Whether int4 in groups of 128 comes by LDS DMA (k_gemm_dma.hip).  Always where its producer has left the rows in pair order; else the pre-pass copies them, which pays where a CU has
+// several tiles to cover it and the product is long or wide enough.  Copy included, us, register-staged and DMA: 1021 x 4096 x 1024 (256 tiles) 20.9 and 23.2, x 7168 96.8 and 101.1,
+// 2043 x 2048 x 1024 20.9 and 25.0, 400 x 6144 x 2048 32.0 and 33.9; 2043 x 4096 x 1024 (512) 29.2 and 31.1, 2043 x 3072 x 512 19.6 and 20.4; the other way round 300 x 12288 x 512 (288)
+// 18.4 and 16.9, 1021 x 6144 x 4096 84.7 and 77.1, 1500 x 6144 x 3584 148.7 and 129.7.  (251 sizes of 256 to 2043 rows: the slower one by 2 to 4 % at eight of them.)
+static bool takes_dma(const MatmulParams& p, int num_cus, int form) {
+    if (form > 1 || !gemm_q4_dma_supported(p)) return false;
+    if (p.a_pairs || tune_env("gemm_form")) return true;
+    return ((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN) > (uint32_t)num_cus && (p.k >= 2048 || p.n >= 8192);
 }
 // host arithmetic only (uzu_hip_prefill_gemm_plan): which kernel / form / split-K a shape gets; UZU_GEMM_FORM / UZU_GEMM_SPLITS apply as at launch
 void gemm_q_mfma128_plan_query(const MatmulParams& p, int num_cus, uint32_t* large_tile, uint32_t* form, uint32_t* splits, uint32_t* workgroups) {
@@ -779,7 +789,7 @@ size_t gemm_q_mfma128_workspace_bytes(const MatmulParams& p, int num_cus) {
     const uint32_t splits = gemm128_splits(p, num_cus);
     size_t bytes = ((size_t)((p.m + 3) & ~3u) * G * 4 + 255) / 256 * 256 + ((size_t)p.n * G * 4 + 255) / 256 * 256;
     if (splits > 1) bytes += ((size_t)splits * p.m * p.n * 4 + 255) / 256 * 256;
-    if (gemm_q4_dma_supported(p) && !p.a_pairs) bytes += (size_t)p.m * p.k * 2;
+    if (!p.a_pairs && takes_dma(p, num_cus, gemm128_form(p, num_cus, splits))) bytes += (size_t)p.m * p.k * 2;
     return bytes;
 }
 uzu_status gemm_q_mfma128(hipStream_t s, const MatmulParams& p, int num_cus, void* workspace) {
@@ -790,8 +800,8 @@ uzu_status gemm_q_mfma128(hipStream_t s, const MatmulParams& p, int num_cus, voi
     float* coef = (float*)((uint8_t*)workspace + rowsum_bytes);
     float* partials = splits > 1 ? (float*)((uint8_t*)workspace + rowsum_bytes + coef_bytes) : nullptr;
     uzu_status st = UZU_OK;
-    const int form = gemm128_form(p, num_cus, splits);
-    const bool dma = form < 2 && gemm_q4_dma_supported(p);
+    int form = gemm128_form(p, num_cus, splits);
+    const bool dma = takes_dma(p, num_cus, form);
     if (!dma && !p.a) {
         set_error("gemm_q_mfma128: rows in pair order, but not the form that reads them");
         return UZU_ERR_UNSUPPORTED;
@@ -813,10 +823,11 @@ uzu_status gemm_q_mfma128(hipStream_t s, const MatmulParams& p, int num_cus, voi
         if (st != UZU_OK || splits == 1) return st;
         return gemm_split_finish(s, p, partials, splits);
     }
+    if (form == 1 && p.bits == 4 && p.group_size == 128) form = 0; // (only operands out of the DMA's alignment come here)
     const dim3 grid(form == 1 ? tile_order_grid(m_tiles, (n_tiles + 1) / 2) : tile_order_grid(m_tiles, n_tiles), splits), block(form ? 512 : 256);
 #define UZU_LAUNCH(B, GSV)                                                                                                                                            \
     st = form == 2 ? launch_check([&] { hipLaunchKernelGGL((gemm_q_mfma128_kernel<B, GSV, 2>), grid, block, 0, s, p, rowsum_in, coef_in, partials, g_gemm128_dbg); }, "gemm_q_mfma128ws") \
-       : form == 1 ? launch_check([&] { hipLaunchKernelGGL((gemm_q_mfma128_kernel<B, GSV, 1>), grid, block, 0, s, p, rowsum_in, coef_in, partials, g_gemm128_dbg); }, "gemm_q_mfma128pp") \
+       : form == 1 ? launch_check([&] { hipLaunchKernelGGL((gemm_q_mfma128_kernel<B, GSV, (B) == 4 && (GSV) == 2 ? 0 : 1>), grid, block, 0, s, p, rowsum_in, coef_in, partials, g_gemm128_dbg); }, "gemm_q_mfma128pp") \
                    : launch_check([&] { hipLaunchKernelGGL((gemm_q_mfma128_kernel<B, GSV, 0>), grid, block, 0, s, p, rowsum_in, coef_in, partials, g_gemm128_dbg); }, "gemm_q_mfma128")
     const uint32_t gs = p.group_size / BK;
     if (p.bits == 4) {
