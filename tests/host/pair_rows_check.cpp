@@ -1,0 +1,32 @@
+// Products whose rows exist in pair order only (MatmulParams::a null) are refused on the host where a kernel would read plain rows: without the rows' sums, without pair rows, or for a
+// product that another form takes.  Nothing is launched: run without a GPU, a launch fails with another status.
+#include <stdio.h>
+
+#include "../../uzu_amd/csrc/kernels.h"
+
+using namespace uzu::k;
+
+int main() {
+    static uint8_t memory[64] __attribute__((aligned(64))); // never read: the addresses only
+    MatmulParams p{};
+    p.b = memory, p.scales = memory, p.biases = memory, p.d = memory, p.pre_coef = (const float*)memory;
+    p.w_dt = p.a_dt = p.d_dt = UZU_BF16, p.b_kind = UZU_MATMUL_B_SCALE_BIAS, p.bits = 4, p.group_size = 128, p.ab_scale = 1.0f;
+    p.m = 512, p.n = 8192, p.k = 2048;
+    int bad = 0;
+    auto refused = [&](const char* what, const MatmulParams& q) {
+        const uzu_status direct = gemm_q_mfma128(nullptr, q, 256, memory), dispatched = matmul(nullptr, q, 256, nullptr);
+        printf("%s: %d %d\n", what, (int)direct, (int)dispatched);
+        bad += direct != UZU_ERR_UNSUPPORTED || dispatched != UZU_ERR_UNSUPPORTED;
+    };
+    refused("no rows", p);
+    p.a_pairs = (const uint16_t*)memory;
+    refused("pair rows without their sums", p);
+    p.pre_rowsum = (const float*)memory;
+    MatmulParams other = p;
+    other.group_size = 64; // the register-staged forms
+    refused("another form", other);
+    other = p, other.a_pairs = nullptr;
+    refused("sums without rows", other);
+    printf("%d bad\n", bad);
+    return bad;
+}

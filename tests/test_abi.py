@@ -73,6 +73,18 @@ def test_desc_struct_layout_matches_c():
     assert sizes == [ctypes.sizeof(D.LinearDesc), ctypes.sizeof(D.NormDesc), ctypes.sizeof(D.RopeDesc), ctypes.sizeof(D.LayerDesc), ctypes.sizeof(D.ModelDesc)]
 
 
+def test_rows_in_pair_order_are_refused_where_a_kernel_would_read_plain_ones(tmp_path):
+    """tests/host/pair_rows_check.cpp: the host's checks in front of the int4 products (csrc/k_matmul.hip, k_gemm128.hip), against the library itself, no device visible."""
+    import subprocess
+    from uzu_amd import _ffi
+    _ffi.build()
+    exe, libdir = str(tmp_path / "pair_rows_check"), os.path.dirname(_ffi.LIB_PATH)
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(ROOT, "tests", "host", "pair_rows_check.cpp"),
+                    "-L", libdir, "-luzu_hip", f"-Wl,-rpath,{libdir}", "-o", exe], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=120, env=dict(os.environ, HIP_VISIBLE_DEVICES=""))
+    assert out.returncode == 0 and out.stdout.endswith("\n0 bad\n"), out.stdout + out.stderr
+
+
 def _build_abi_smoke(tmp_path):
     """tests/host/abi_smoke.c: plain C99 against include/uzu_hip.h + libuzu_hip.so -- the header as an FFI generator sees it."""
     import subprocess

@@ -73,7 +73,8 @@ static void offset_tables(uzu_hip_model* m, const DLinear& L, const uint16_t* in
     }();
     if (batch < 128) return;
     if (input == m->normed && m->normed_pairs_rows == batch && L.k == m->d.model_dim) p->a_pairs = m->normed_pairs;
-    if (input == m->gated && m->gated_pairs_rows == batch) p->a_pairs = input, p->a = nullptr;
+    // (rows in pair order only; matmul() refuses them without the sums filed below, and to a matrix of another K)
+    if (input == m->gated && m->gated_pairs_rows == batch) p->a_pairs = L.k == m->rs_gated.k ? input : nullptr, p->a = nullptr;
     if (!enabled) return;
     p->pre_coef = L.coef;
     if (input == m->normed && m->rs_rows == batch && m->rs_k == L.k && m->rs_group == L.group) p->pre_rowsum = m->rowsum;

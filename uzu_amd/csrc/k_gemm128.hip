@@ -802,8 +802,8 @@ uzu_status gemm_q_mfma128(hipStream_t s, const MatmulParams& p, int num_cus, voi
     uzu_status st = UZU_OK;
     int form = gemm128_form(p, num_cus, splits);
     const bool dma = takes_dma(p, num_cus, form);
-    if (!dma && !p.a) {
-        set_error("gemm_q_mfma128: rows in pair order, but not the form that reads them");
+    if (!p.a && !(dma && p.a_pairs && p.pre_rowsum)) { // (the pre-pass would read plain rows)
+        set_error("gemm_q_mfma128: no plain rows, and not rows in pair order with their sums for the form that reads them");
         return UZU_ERR_UNSUPPORTED;
     }
     uint16_t* pairs = dma && !p.a_pairs ? (uint16_t*)((uint8_t*)workspace + rowsum_bytes + coef_bytes + (splits > 1 ? ((size_t)splits * p.m * p.n * 4 + 255) / 256 * 256 : 0)) : nullptr;

@@ -337,7 +337,7 @@ uzu_status matmul(hipStream_t s, const MatmulParams& p, int num_cus, const char*
         set_error("matmul: group size must be non-zero");
         return UZU_ERR_UNSUPPORTED;
     }
-    if (!p.a && !(quant && p.a_pairs && gemm_pairs_wanted(p, num_cus))) {
+    if (!p.a && !(quant && p.a_pairs && p.pre_rowsum && gemm_pairs_wanted(p, num_cus))) {
         set_error("matmul: no activation rows in the order that this product reads");
         return UZU_ERR_UNSUPPORTED;
     }

@@ -53,7 +53,8 @@ struct MatmulParams {
     // pre_rowsum (parts of 64 columns) of the GEMM that reads D next, which then needs no pre-pass launch.  The large-tile kernel only; null = not filed.
     float* gated_rowsum_out;
     // The int4 DMA form (k_gemm_dma.hip) multiplies rows in pair order: every eight consecutive k as 0 4 1 5 2 6 3 7 (gemm_convert.h).  a_pairs: A's rows in that order, where their
-    // producer wrote them so; null: the product's pre-pass makes the copy.  a null beside it: no other form of the rows exists (only where gemm_pairs_wanted said so).
+    // producer wrote them so; null: the product's pre-pass makes the copy.  a null beside it: no other form of the rows exists (only where gemm_pairs_wanted said so, and
+    // with pre_rowsum).
     const uint16_t* a_pairs;
     uint32_t d_pairs; // act_mul on the large tile: D leaves in pair order
     // The Normalization that reads D next (engine prefill: out-projection -> pre-MLP norm, down-projection -> the next layer's pre-mixer norm; its
