@@ -1,5 +1,5 @@
 // Products whose rows exist in pair order only (MatmulParams::a null) are refused on the host where a kernel would read plain rows: without the rows' sums, without pair rows, or for a
-// product that another form takes.  Nothing is launched: run without a GPU, a launch fails with another status.
+// product that another form takes.  And a Normalization is refused pair rows where the kernel that writes them is not the one that would run.  Nothing is launched: run without a GPU, a launch fails with another status.
 #include <stdio.h>
 
 #include "../../uzu_amd/csrc/kernels.h"
@@ -27,6 +27,24 @@ int main() {
     refused("another form", other);
     other = p, other.a_pairs = nullptr;
     refused("sums without rows", other);
+    NormParams n{};
+    n.input = n.output = memory, n.scales = memory, n.pairs_out = (uint16_t*)memory, n.io_dt = UZU_BF16, n.affine_dt = UZU_F32, n.batch_size = 128, n.element_count = 1024, n.epsilon = 1e-5f;
+    auto norm_refused = [&](const char* what, const NormParams& q) {
+        const uzu_status status = normalization(nullptr, q);
+        printf("%s: %d\n", what, (int)status);
+        bad += status != UZU_ERR_UNSUPPORTED;
+    };
+    for (uint32_t width : {512u, 1000u, 5120u, 3072u}) {
+        NormParams q = n;
+        q.element_count = width;
+        norm_refused("another width", q);
+    }
+    NormParams q = n;
+    q.batch_size = 1, norm_refused("one row", q);
+    q = n, q.io_dt = UZU_F32, norm_refused("f32 rows", q);
+    q = n, q.affine_dt = 77, norm_refused("another scale type", q);
+    q = n, q.input = memory + 4, norm_refused("input off 8 bytes", q);
+    q = n, q.pairs_out = (uint16_t*)(memory + 8), norm_refused("pair rows off 16 bytes", q);
     printf("%d bad\n", bad);
     return bad;
 }

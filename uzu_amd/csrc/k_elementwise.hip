@@ -230,8 +230,9 @@ bool normalization_pairs_supported(uint32_t n) { return n == 1024 || n == 2048 |
 
 uzu_status normalization(hipStream_t s, const NormParams& p) {
     if (p.batch_size == 0) return UZU_OK;
-    if (p.pairs_out && (exact_mode() || !normalization_pairs_supported(p.element_count) || p.io_dt != UZU_BF16 || p.batch_size < 2 || (uintptr_t)p.pairs_out % 16 ||
-                        (((uintptr_t)p.input | (uintptr_t)p.output | (uintptr_t)p.shortcut) & 7))) {
+    const bool rows_kernel = !exact_mode() && p.io_dt == UZU_BF16 && p.batch_size >= 2 && p.element_count % 1024 == 0 && (p.affine_dt == UZU_F32 || p.affine_dt == UZU_BF16) &&
+                             (((uintptr_t)p.input | (uintptr_t)p.output | (uintptr_t)p.shortcut) & 7) == 0;
+    if (p.pairs_out && (!rows_kernel || !normalization_pairs_supported(p.element_count) || (uintptr_t)p.pairs_out % 16)) { // (no other kernel writes them)
         set_error("normalization: rows of %u elements are not available in pair order", p.element_count);
         return UZU_ERR_UNSUPPORTED;
     }
@@ -240,12 +241,7 @@ uzu_status normalization(hipStream_t s, const NormParams& p) {
         return UZU_ERR_UNSUPPORTED;
     }
     if (exact_mode()) return normalization_exact(s, p);
-    static const bool fast_rows = [] { // UZU_NORM_ROWS=0: the general kernel everywhere (A/B runs)
-        const char* e = lab_env("UZU_NORM_ROWS");
-        return !e || atoi(e) != 0;
-    }();
-    if (fast_rows && p.io_dt == UZU_BF16 && p.batch_size >= 2 && p.element_count % 1024 == 0 && (p.affine_dt == UZU_F32 || p.affine_dt == UZU_BF16) &&
-        (((uintptr_t)p.input | (uintptr_t)p.output | (uintptr_t)p.shortcut) & 7) == 0) {
+    if (rows_kernel) {
         const uint32_t nv = p.element_count / 1024;
         const NormPartials none{};
 #define UZU_ROWS(NVV)                                                                                                                            \
