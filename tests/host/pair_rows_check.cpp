@@ -27,6 +27,13 @@ int main() {
     refused("another form", other);
     other = p, other.a_pairs = nullptr;
     refused("sums without rows", other);
+    MatmulParams copied = p; // 512 rows of 8192 x 2048, 256 tiles; 1024 rows, 512 tiles: their copy's room only where the rows are not brought
+    copied.m = 1024, copied.a = memory, copied.a_pairs = nullptr;
+    MatmulParams brought = copied;
+    brought.a_pairs = (const uint16_t*)memory;
+    bad += gemm_q_mfma128_workspace_bytes(copied, 256) != gemm_q_mfma128_workspace_bytes(brought, 256) + (size_t)1024 * 2048 * 2;
+    copied.m = brought.m = 512;
+    bad += gemm_q_mfma128_workspace_bytes(copied, 256) != gemm_q_mfma128_workspace_bytes(brought, 256);
     NormParams n{};
     n.input = n.output = memory, n.scales = memory, n.pairs_out = (uint16_t*)memory, n.io_dt = UZU_BF16, n.affine_dt = UZU_F32, n.batch_size = 128, n.element_count = 1024, n.epsilon = 1e-5f;
     auto norm_refused = [&](const char* what, const NormParams& q) {

@@ -114,6 +114,7 @@ static bool pairs_wanted(Enc& e, const DLinear& L, uint32_t rows) {
     p.w_dt = p.a_dt = p.d_dt = UZU_BF16;
     p.b_kind = L.method == UZU_QUANT_SCALE_BIAS ? UZU_MATMUL_B_SCALE_BIAS : L.method == UZU_QUANT_SCALE_ZERO_POINT ? UZU_MATMUL_B_SCALE_ZERO_POINT : UZU_MATMUL_B_SCALE_SYMMETRIC;
     p.bits = L.bits, p.group_size = L.group, p.ab_scale = 1.0f, p.m = rows, p.n = L.n, p.k = L.k;
+    p.a_pairs = e.m->normed; // (whichever they are: the workspace needs no room for the pre-pass's copy)
     return k::gemm_pairs_wanted(p, e.m->ctx->num_cus) && k::stream_workspace(e.s, k::gemm_q_mfma128_workspace_bytes(p, e.m->ctx->num_cus)) != nullptr;
 }
 
