@@ -2,8 +2,7 @@
 # GPU box (gpurun): same-box A/B of the prefill switches of one library build.
 #   UZU_GEMM_ACT=0|1       GatedActMul as its own kernel | in the up projection's GEMM epilogue (shipping)
 #   UZU_ATTN_TPW=4|2|1|0   wave tasks per workgroup of the flash-attention prefill kernel (0 = chosen by grid size, shipping)
-# The GEMM loop variants (pair-form conversion, pipelined k16 steps) are compile-time: build k_gemm128.hip with
-# -DUZU_GEMM_PAIR_DEQUANT=0 / -DUZU_GEMM_PIPE=0 into a second library directory and compare with
+# The GEMM loop variants are compile-time: build k_gemm128.hip with -DUZU_GEMM_PIPE=0 into a second library directory and compare with
 #   LD_LIBRARY_PATH=uzu_amd/<dir> KB_GEMM=1 tools/kbench        (profiles/r2_gemm128_pmc.txt holds the round-2 run)
 ROOT=${GRAFT_REPO_ROOT:-$(cd "$(dirname "$0")/.." && pwd)}
 cd $ROOT

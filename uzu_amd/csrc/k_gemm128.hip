@@ -31,14 +31,9 @@
 namespace uzu {
 namespace k {
 
-
-#ifndef UZU_GEMM_PAIR_DEQUANT
-#define UZU_GEMM_PAIR_DEQUANT 1 // int4: bf16(16 + u) pairs (gemm_convert.h::dequant4_pairs); 0 = centred (u - 8) / 16 per code (A/B builds)
-#endif
 namespace {
 constexpr int BK = 64, BM = 128, BN = 128;
 constexpr int A_PITCH = 144;
-constexpr bool kPairs = UZU_GEMM_PAIR_DEQUANT != 0;
 #ifndef UZU_GEMM_PP_DB
 #define UZU_GEMM_PP_DB 4 // ping-pong form: weight ring depth
 #endif
@@ -70,7 +65,7 @@ __global__ void __launch_bounds__(256) gemm_prepass_kernel(MatmulParams p, float
         if (idx >= N * G) return;
         const uint32_t n = idx / G, g = idx % G; // consecutive threads read consecutive scales
         // `mid` = what the main loop subtracted from the unsigned code: 2^(bits-1) (centred codes) or -16 (int4 pair form: 16 + u)
-        const float mid = (kPairs && p.bits == 4) ? -16.0f : (float)(1u << (p.bits - 1));
+        const float mid = p.bits == 4 ? -16.0f : (float)(1u << (p.bits - 1));
         const float scale = bf16_to_f32(((const uint16_t*)p.scales)[(size_t)n * G + g]);
         float c;
         if (p.b_kind == UZU_MATMUL_B_SCALE_ZERO_POINT) {
@@ -181,7 +176,7 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
     const uint32_t kt_lo = g_lo * GS, KTz = Gz * GS; // KTz % U == 0 (host-checked)
     const uint32_t row_bytes = K * BITS / 8;
     // codes as the conversion wants them: two's complement of u - mid (centred form) or the unsigned u (int4 pair form)
-    const uint32_t flip = (kPairs && BITS == 4) ? (p.signed_codes ? 0x88888888u : 0u) : p.signed_codes ? 0u : (BITS == 4 ? 0x88888888u : 0x80808080u);
+    const uint32_t flip = BITS == 4 ? (p.signed_codes ? 0x88888888u : 0u) : (p.signed_codes ? 0u : 0x80808080u);
 
     // ---- activation staging role: 8 lanes fetch one row's 128 bytes (one cache line per row per instruction), four
     // passes of 32 rows.  (One thread per (row, 64-byte half) costs 45 L1 accesses per wave instruction -- rocprofv3
@@ -204,7 +199,7 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
         uint8_t* dst = &s_a[kt & 1][rpass * A_PITCH + chunk * 16];
 #pragma unroll
         for (int j = 0; j < NR; ++j) {
-            u32x4_v v = (kPairs && BITS == 4) ? permute_pairs(st[j]) : st[j];
+            u32x4_v v = BITS == 4 ? permute_pairs(st[j]) : st[j];
 #ifdef UZU_GEMM_LAB_SWAP // LAB: the wave-specialised form with two k slots of every operand exchanged -- is the MFMA's sum independent of the slot order?
             if (WS) { const uint32_t t = v.x; v.x = v.w, v.w = t; }
 #endif
@@ -262,7 +257,7 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
 #ifdef UZU_GEMM_LAB_NOCONV // LAB (wrong results): one and-or per fragment instead of nine instructions -- the loop without its conversion work (finite operands: arbitrary bit patterns cost clock)
                 { const uint32_t one = (raw[nb][0][s] & 0x00010001u) | 0x3f803f80u; bf[nb] = u32x4_t{one, one, one, one}; } // bf16 1.0 / 1.0078: finite, benign
 #else
-                if (BITS == 4) bf[nb] = kPairs ? dequant4_pairs(raw[nb][0][s] ^ flip) : dequant4(raw[nb][0][s] ^ flip);
+                if (BITS == 4) bf[nb] = dequant4_pairs(raw[nb][0][s] ^ flip);
                 else bf[nb] = dequant8(raw[nb][s >> 1][(s & 1) * 2] ^ flip, raw[nb][s >> 1][(s & 1) * 2 + 1] ^ flip);
 #endif
             }
@@ -321,7 +316,7 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
     auto fold = [&](bool hazard_wait = true) { // acc_t += scale * acc_g at a group boundary
         f32x2_t sc[2];
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) sc[nb].x = sc[nb].y = ((BITS == 4 && !kPairs) ? 16.0f : 1.0f) * bits_to_f32(sc_cur[nb] << 16);
+        for (int nb = 0; nb < 2; ++nb) sc[nb].x = sc[nb].y = bits_to_f32(sc_cur[nb] << 16);
         // In place on acc_t through inline asm: left to itself the register allocator writes the result over acc_g and
         // permutes the 16-register accumulator tuples around the loop (60-180 VGPRs of spills at the 256 budget).  The
         // hazard recogniser cannot see an MFMA -> VALU read through inline asm, so the wait for the last MFMA of the
@@ -380,7 +375,7 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
                     u32x4_t f;
-                    if (BITS == 4) f = kPairs ? dequant4_pairs(raw[0][s] ^ flip) : dequant4(raw[0][s] ^ flip);
+                    if (BITS == 4) f = dequant4_pairs(raw[0][s] ^ flip);
                     else f = dequant8(raw[s >> 1][(s & 1) * 2] ^ flip, raw[s >> 1][(s & 1) * 2 + 1] ^ flip);
 #ifdef UZU_GEMM_LAB_SWAP
                     { const uint32_t t = f.x; f.x = f.w, f.w = t; }
@@ -500,7 +495,7 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 u32x4_t f;
-                if (BITS == 4) f = kPairs ? dequant4_pairs(raw[0][s] ^ flip) : dequant4(raw[0][s] ^ flip);
+                if (BITS == 4) f = dequant4_pairs(raw[0][s] ^ flip);
                 else f = dequant8(raw[s >> 1][(s & 1) * 2] ^ flip, raw[s >> 1][(s & 1) * 2 + 1] ^ flip);
                 *(u32x4_t*)(s_bw + s * 1024) = f;
             }
@@ -684,7 +679,7 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
     ts[2] = wall_clock64();
 
     const GemmTile t{m0 + wm * 64, n0 + wn * 64, n_t * 64, n_t, {ncol[0], ncol[1]}, (uint32_t)wave, (uint32_t)wn, M, Mst, N, H, g_lo, g_lo + Gz, z, gated, live};
-    gemm_tile_finish<(kPairs && BITS == 4)>(p, t, rowsum, coef, partials, acc_t, s_ep, s_exp_tab);
+    gemm_tile_finish<BITS == 4>(p, t, rowsum, coef, partials, acc_t, s_ep, s_exp_tab);
     if (PP && !half) lds_barrier(); // the partner half's last phase barrier (it runs one phase behind)
     if (dbg && tid == 0 && live) {
         ts[3] = wall_clock64();
@@ -778,7 +773,7 @@ bool gemm_coef_table_supported(const MatmulParams& p) {
     if (p.b_kind == UZU_MATMUL_B_FULL_PRECISION || !(p.bits == 4 || p.bits == 8)) return false;
     if (p.group_size != 64 && p.group_size != 128 && p.group_size != 256) return false;
     if (p.k % p.group_size) return false;
-    return p.b_kind != UZU_MATMUL_B_SCALE_SYMMETRIC || (kPairs && p.bits == 4);
+    return p.b_kind != UZU_MATMUL_B_SCALE_SYMMETRIC || p.bits == 4;
 }
 uzu_status gemm_coef_table(hipStream_t s, const MatmulParams& p, float* coef) {
     const uint32_t G = p.k / p.group_size;
@@ -807,7 +802,7 @@ uzu_status gemm_q_mfma128(hipStream_t s, const MatmulParams& p, int num_cus, voi
         return UZU_ERR_UNSUPPORTED;
     }
     uint16_t* pairs = dma && !p.a_pairs ? (uint16_t*)((uint8_t*)workspace + rowsum_bytes + coef_bytes + (splits > 1 ? ((size_t)splits * p.m * p.n * 4 + 255) / 256 * 256 : 0)) : nullptr;
-    if (p.b_kind != UZU_MATMUL_B_SCALE_SYMMETRIC || (kPairs && p.bits == 4)) {
+    if (p.b_kind != UZU_MATMUL_B_SCALE_SYMMETRIC || p.bits == 4) {
         // the caller may bring either table (engine: coefficients tabulated at load, row sums written by the normalisation that produced A)
         const uint32_t rowsum_blocks = p.pre_rowsum && !pairs ? 0u : (((p.m + 3) & ~3u) + 3) / 4, coef_blocks = p.pre_coef ? 0u : (p.n * G + 255) / 256;
         if (rowsum_blocks + coef_blocks) {
