@@ -40,9 +40,6 @@ constexpr int A_PITCH = 144;
 #ifndef UZU_GEMM_PP_DA
 #define UZU_GEMM_PP_DA 2 // ping-pong form: activation register stages
 #endif
-#ifndef UZU_GEMM_FOLD_PK
-#define UZU_GEMM_FOLD_PK 0 // group fold with v_pk_fma_f32 (1) or pairs of v_fma_f32 (0)
-#endif
 #ifndef UZU_GEMM_PP_MSCHED
 #define UZU_GEMM_PP_MSCHED 2 // ping-pong form, MFMA phase: 0 = operands | 16 MFMAs | staging; 1 = staging interleaved with the MFMAs; 2 = staging first
 #endif
@@ -200,9 +197,6 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
 #pragma unroll
         for (int j = 0; j < NR; ++j) {
             u32x4_v v = BITS == 4 ? permute_pairs(st[j]) : st[j];
-#ifdef UZU_GEMM_LAB_SWAP // LAB: the wave-specialised form with two k slots of every operand exchanged -- is the MFMA's sum independent of the slot order?
-            if (WS) { const uint32_t t = v.x; v.x = v.w, v.w = t; }
-#endif
             *(u32x4_v*)(dst + j * RSTEP * A_PITCH) = v;
         }
     };
@@ -254,12 +248,8 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
             for (int mb = 0; mb < 2; ++mb) af[mb] = *(const u32x4_t*)(ab + mb * 32 * A_PITCH + s * 16);
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
-#ifdef UZU_GEMM_LAB_NOCONV // LAB (wrong results): one and-or per fragment instead of nine instructions -- the loop without its conversion work (finite operands: arbitrary bit patterns cost clock)
-                { const uint32_t one = (raw[nb][0][s] & 0x00010001u) | 0x3f803f80u; bf[nb] = u32x4_t{one, one, one, one}; } // bf16 1.0 / 1.0078: finite, benign
-#else
                 if (BITS == 4) bf[nb] = dequant4_pairs(raw[nb][0][s] ^ flip);
                 else bf[nb] = dequant8(raw[nb][s >> 1][(s & 1) * 2] ^ flip, raw[nb][s >> 1][(s & 1) * 2 + 1] ^ flip);
-#endif
             }
         };
 #if UZU_GEMM_PIPE
@@ -328,25 +318,10 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-#ifdef UZU_GEMM_LAB_NOFOLD // LAB (wrong results): two of a block's sixteen registers folded -- the MFMAs stay live, 7/8 of the fold's FMAs are gone
-                for (int r = 0; r < 2; r += 2) {
-#else
                 for (int r = 0; r < 16; r += 2) {
-#endif
-#if UZU_GEMM_FOLD_PK == 1
-                    f32x2_t t = {acc_t[mb][nb][r], acc_t[mb][nb][r + 1]};
-                    const f32x2_t g = {acc_g[mb][nb][r], acc_g[mb][nb][r + 1]};
-                    asm volatile("v_pk_fma_f32 %0, %1, %2, %0" : "+v"(t) : "v"(sc[nb]), "v"(g));
-                    acc_t[mb][nb][r] = t.x, acc_t[mb][nb][r + 1] = t.y;
-#else
                     float t0 = acc_t[mb][nb][r], t1 = acc_t[mb][nb][r + 1];
-#if UZU_GEMM_FOLD_PK == 2
-                    asm volatile("v_fmac_f32_e32 %0, %2, %3\n\tv_fmac_f32_e32 %1, %2, %4" : "+v"(t0), "+v"(t1) : "v"(sc[nb].x), "v"(acc_g[mb][nb][r]), "v"(acc_g[mb][nb][r + 1]));
-#else
                     asm volatile("v_fma_f32 %0, %2, %3, %0\n\tv_fma_f32 %1, %2, %4, %1" : "+v"(t0), "+v"(t1) : "v"(sc[nb].x), "v"(acc_g[mb][nb][r]), "v"(acc_g[mb][nb][r + 1]));
-#endif
                     acc_t[mb][nb][r] = t0, acc_t[mb][nb][r + 1] = t1;
-#endif
                 }
         __builtin_amdgcn_sched_barrier(0); // the next group's first MFMA must not be hoisted above the fold (it would need a second acc_g)
         UZU_FOLD_MARK(7)
@@ -377,9 +352,6 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
                     u32x4_t f;
                     if (BITS == 4) f = dequant4_pairs(raw[0][s] ^ flip);
                     else f = dequant8(raw[s >> 1][(s & 1) * 2] ^ flip, raw[s >> 1][(s & 1) * 2 + 1] ^ flip);
-#ifdef UZU_GEMM_LAB_SWAP
-                    { const uint32_t t = f.x; f.x = f.w, f.w = t; }
-#endif
                     *(u32x4_t*)(dst + s * 1024) = f;
                 }
             };
@@ -658,21 +630,16 @@ __global__ void __launch_bounds__(MODE ? 512 : 256, MODE ? 1 : 2) gemm_q_mfma128
     #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const uint32_t kt = kt0 + u;
-                // (UZU_GEMM_LAB_*: ablation builds for tools/kbench -- wrong results, one ingredient of the k-step removed at a time)
                 load_w(kt + DB - 1, ring[(u + DB - 1) % DB]);
                 mfma_codes(kt, ring[u % DB], u % GS == 0);
-#ifndef UZU_GEMM_LAB_NOSTAGE
                 stage_a(kt + 1, a_st[(u + 1) % DA]); // tile kt + 1 (requested DA k-steps ago) -> the other LDS buffer
                 load_a(kt + 1 + DA, a_st[(u + 1) % DA]);
-#endif
                 if ((u + 1) % GS == 0) {
                     fold();
                     sc_cur[0] = sc_nxt[0], sc_cur[1] = sc_nxt[1];
                     load_scale((kt + 1) / GS + 1, sc_nxt);
                 }
-#ifndef UZU_GEMM_LAB_NOBAR
                 lds_barrier();
-#endif
             }
         }
     }
