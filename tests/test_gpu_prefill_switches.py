@@ -88,3 +88,23 @@ def test_rows_in_pair_order_leave_the_logits_as_they_are(tmp_path, dim):
     for form in ("0", "1"):
         pairs = _leg(tmp_path, f"pairs{form}", args, UZU_HIP_TUNE=f"gemm_form={form}")
         assert pairs["logits_sha256"] == plain["logits_sha256"] and pairs["tokens"] == plain["tokens"], form
+
+
+def test_producers_write_the_rows_in_pair_order(tmp_path):
+    """The same bits come from the copy that a product's pre-pass makes of plain rows: that the producers wrote them shows in the first pass's memory, the workspace without the copy of the
+    down projection's 1021 x 16384 rows (33 MB; 38 and 70 MiB seen)."""
+    args = ("--prompt", "1021", "--hidden", "16384", "--group", "128")
+    pairs = _leg(tmp_path, "pairs", args, UZU_HIP_TUNE="gemm_form=0")
+    assert pairs["first_pass_bytes"] < 55 << 20, pairs["first_pass_bytes"]
+
+
+@pytest.mark.parametrize("prompt,dim,hidden", [(520, 4096, 4352), (449, 4096, 4096)])
+def test_gated_rows_in_pair_order_reach_the_form_that_reads_them(tmp_path, prompt, dim, hidden):
+    """Down projections just above the staged kernel's count of tiles (csrc/k_gemm_rows.hip), with their choice of kernel unpinned: gated rows exist in pair order only, and a product that
+    did not take them would fail the pass.  Other products of the pass sum in other orders than those of plain rows on one form, and a flipped rounding of the residual rows moves logits by
+    up to 0.14 sigma here, so each is held against the reference-order pass: as close as plain rows (RMS; a quarter for the flips, as above)."""
+    args = ("--prompt", str(prompt), "--dim", str(dim), "--hidden", str(hidden), "--group", "128")
+    legs = _leg(tmp_path, "exact", args, UZU_HIP_EXACT="1"), _leg(tmp_path, "auto", args), _leg(tmp_path, "plain", args, UZU_HIP_TUNE="gemm_form=2")
+    exact, a, b = (f32(r["logits"]).astype(np.float64) for r in legs)
+    rms = lambda d: np.sqrt((d ** 2).mean())
+    assert rms(a - exact) <= 1.25 * rms(b - exact), (rms(a - exact), rms(b - exact), exact.std())

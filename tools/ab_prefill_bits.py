@@ -30,6 +30,7 @@ def main():
     ap.add_argument("--group", type=int, default=64, help="tiny: the quantisation group")
     ap.add_argument("--dump", default="", help="write the logits (bf16 bits, .npy) here")
     args = ap.parse_args()
+    import torch
     from uzu_amd import synthetic as S
     from uzu_amd.backend import Context
     from uzu_amd.engine import HipModel
@@ -40,7 +41,9 @@ def main():
     ctx = Context.new(0)
     hm = HipModel(ctx, S.build_model(cfg))
     prompt = S.synthetic_prompt(args.prompt, cfg.vocab_size)
+    free = torch.cuda.mem_get_info()[0]
     hm.prefill(prompt)  # warm-up pass (workspace allocation, code objects)
+    first_pass_bytes = free - torch.cuda.mem_get_info()[0]
     hm.reset()
     ctx.synchronize()
     t0 = time.perf_counter()
@@ -54,7 +57,7 @@ def main():
         np.save(args.dump, logits)
     f = (logits.astype(np.uint32) << 16).view(np.float32)
     print(json.dumps({"model": cfg.name, "prompt": args.prompt, "switches": os.environ.get("UZU_HIP_TUNE", ""),
-                      "prefill_launches": launches, "prefill_ms": round(dt * 1e3, 3), "prompt_tokens_per_s": round(args.prompt / dt, 1), "first_token": int(first),
+                      "prefill_launches": launches, "prefill_ms": round(dt * 1e3, 3), "prompt_tokens_per_s": round(args.prompt / dt, 1), "first_token": int(first), "first_pass_bytes": int(first_pass_bytes),
                       "tokens": [int(t) for t in toks], "logits_sha256": hashlib.sha256(logits.tobytes()).hexdigest()[:16],
                       "logits_rms": float(np.sqrt(np.mean(f.astype(np.float64) ** 2)))}))
     hm.close()
