@@ -85,6 +85,19 @@ def test_rows_in_pair_order_are_refused_where_a_kernel_would_read_plain_ones(tmp
     assert out.returncode == 0 and out.stdout.endswith("\n0 bad\n"), out.stdout + out.stderr
 
 
+@pytest.mark.gpu
+def test_gated_epilogue_has_the_exact_silu_for_every_gate(tmp_path):
+    """tests/host/gated_silu_check.cpp: the quick quotient of csrc/gemm128_epilogue.h on the device, through the library's product, on each of its forms."""
+    import subprocess
+    from uzu_amd import _ffi
+    _ffi.lib()
+    exe, libdir = str(tmp_path / "gated_silu_check"), os.path.dirname(_ffi.LIB_PATH)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(ROOT, "tests", "host", "gated_silu_check.cpp"),
+                    "-L", libdir, "-luzu_hip", "-L/opt/rocm/lib", "-lamdhip64", f"-Wl,-rpath,{libdir}", "-o", exe], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0 and out.stdout.endswith("\n0 bad\n"), out.stdout + out.stderr
+
+
 def _build_abi_smoke(tmp_path):
     """tests/host/abi_smoke.c: plain C99 against include/uzu_hip.h + libuzu_hip.so -- the header as an FFI generator sees it."""
     import subprocess
