@@ -37,15 +37,17 @@ UZU_ORDER_HD inline bool tile_of_block(uint32_t block, uint32_t m_tiles, uint32_
 // row by row, where a row of tiles is short; and a last column that is mostly padding behind the whole tiles, so that what goes beyond a full round of workgroups is its cheap tiles.
 enum TileOrder { kTileBlocks, kTileRows, kTileLastColumnBehind };
 UZU_ORDER_HD inline bool tile_of_block(uint32_t block, uint32_t m_tiles, uint32_t n_tiles, TileOrder order, uint32_t* m_t, uint32_t* n_t) {
-    if (order == kTileBlocks || (order == kTileLastColumnBehind && n_tiles == 1)) return tile_of_block(block, m_tiles, n_tiles, m_t, n_t);
-    const uint32_t whole = m_tiles * (order == kTileRows ? n_tiles : n_tiles - 1), more = whole % 8, xcd = block & 7, slot = block >> 3, share = whole / 8 + (xcd < more ? 1u : 0u);
+    const uint32_t xcd = block & 7, slot = block >> 3;
     if (order == kTileRows) {
-        const uint32_t t = xcd * (whole / 8) + (xcd < more ? xcd : more) + slot;
-        *m_t = t / n_tiles, *n_t = t % n_tiles;
-        return slot < share;
+        const uint32_t total = m_tiles * n_tiles, share = total / 8, more = total % 8, t = xcd * share + (xcd < more ? xcd : more) + slot;
+        *m_t = t / n_tiles, *n_t = t - *m_t * n_tiles;
+        return slot < share + (xcd < more ? 1u : 0u);
     }
-    if (slot < share) return tile_of_block(block, m_tiles, n_tiles - 1, m_t, n_t);
-    *m_t = (slot - share) * 8 + ((xcd - more) & 7u), *n_t = n_tiles - 1;
+    const uint32_t behind = order == kTileLastColumnBehind && n_tiles > 1 ? 1 : 0;
+    if (tile_of_block(block, m_tiles, n_tiles - behind, m_t, n_t)) return true;
+    if (!behind) return false;
+    const uint32_t whole = m_tiles * (n_tiles - 1), more = whole % 8;
+    *m_t = (slot - whole / 8 - (xcd < more ? 1u : 0u)) * 8 + ((xcd - more) & 7u), *n_t = n_tiles - 1;
     return *m_t < m_tiles;
 }
 

@@ -247,18 +247,19 @@ __device__ __forceinline__ void split_repair(f32x16_t& acc, const uint16_t* xb, 
 constexpr int kEpilogueGated = 16; // grouped experts: the weight rows are [up ; gate], the result act(gate, up) as bf16 rows (GatedRows)
 
 // bf16 products row by row up to 1024 columns and 2048 k: the weights fit an L2, and the rows are read by one XCD (us: 1280 x 1024 x 1024 20.5 -> 19.1, 517 x 1024 x 2048 19.8 -> 18.0,
-// 768 x 1024 x 1536 19.9 -> 18.0; at 4096 k 517 rows 21.6 -> 22.6, f32 products of 517 x 1024 x 1024 20.9 -> 22.8).  A last column of at most 32 behind the others while the weights are at most 48 x 1024 columns' k: 900 x 4112 x 1024 (264 tiles) 28.6 -> 27.3,
+// 768 x 1024 x 1536 19.9 -> 18.0; at 4096 k 517 rows 21.6 -> 22.6, f32 products of 517 x 1024 x 1024 20.9 -> 22.8).
+// Where there is more than a 128 x 128 tile a CU, a last column of at most 32 behind the others while the weights are at most 48 x 1024 columns' k: 900 x 4112 x 1024 (264 tiles) 28.6 -> 27.3,
 // 4000 x 4112 x 512 (1056) 47.4 -> 43.3, 2048 x 8208 x 512 (1040) 45.5 -> 41.6; of more weights 2048 x 8208 x 2048 110 -> 116, 4000 x 4112 x 2048 110 -> 115.
-__device__ __forceinline__ TileOrder linear_tile_order(uint32_t n, uint32_t k, uint32_t parts) {
-    const uint32_t columns = (n + DN - 1) / DN, last = n % DN;
-    if (columns <= 8) return parts == 1 && k <= 2048 ? kTileRows : kTileBlocks;
-    return last && last <= 32 && columns * k <= 48 * 1024 ? kTileLastColumnBehind : kTileBlocks;
+static TileOrder linear_tile_order(const LinearF32Params& p, uint32_t parts) {
+    const uint32_t columns = (p.n + DN - 1) / DN, last = p.n % DN;
+    if (columns <= 8) return parts == 1 && p.k <= 2048 ? kTileRows : kTileBlocks;
+    return (p.rows + 127) / 128 * columns > 256 && last && last <= 32 && (uint64_t)columns * p.k <= 48 * 1024 ? kTileLastColumnBehind : kTileBlocks;
 }
 
 // parts: 1, or 3 for operand rows [lo | mid | hi].  partials (MB 1, not GROUPED): blockIdx.z takes its share of the k-steps and leaves its sums there, f32 [z][rows][n].
 // WM x WN waves, a wave 32 MB x 64 outputs
 template <int WM, int WN, int MB, int STAGES, bool GROUPED, int KIND, uint32_t parts>
-__global__ void __launch_bounds__(64 * WM * WN, WM * WN == 4 ? 4 : 2) linear_dma_kernel(LinearF32Params p, const uint16_t* xb, uint32_t ldxb, GatedRows gr, float* partials) {
+__global__ void __launch_bounds__(64 * WM * WN, WM * WN == 4 ? 4 : 2) linear_dma_kernel(LinearF32Params p, const uint16_t* xb, uint32_t ldxb, GatedRows gr, float* partials, TileOrder order) {
     constexpr bool GATED = KIND == kEpilogueGated, CUT = !GROUPED && MB == 1;
     constexpr int DK = 64, DM = 32 * WM * MB, DN = 64 * WN, AP = DM * DK * 2 / 1024 / (WM * WN), BP = DN * DK * 2 / 1024 / (WM * WN); // 1 KB pieces per wave: A, B
     constexpr uint32_t STAGE = (DM + DN) * DK * 2, ROW = DK * 2, CHUNKS = DK / 8, RPP = 1024 / ROW; // row bytes, 16-byte chunks per row, rows per piece
@@ -279,7 +280,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WM * WN == 4 ? 4 : 2) linear_dma
         const uint32_t first = z ? __builtin_amdgcn_readlane(upto, z - 1) : 0u;
         m_t = blockIdx.y - first, n_t = blockIdx.x;
     } else {
-        if (!tile_of_block(blockIdx.x, (p.rows + DM - 1) / DM, (p.n + DN - 1) / DN, linear_tile_order(p.n, p.k, parts), &m_t, &n_t)) return;
+        if (!tile_of_block(blockIdx.x, (p.rows + DM - 1) / DM, (p.n + DN - 1) / DN, order, &m_t, &n_t)) return;
     }
     const uint32_t m0 = r_lo + m_t * DM, n0 = n_t * DN;
     const uint16_t* w = p.w + (size_t)z * p.w_batch;
@@ -504,7 +505,7 @@ uzu_status launch_dma_tile(hipStream_t s, const LinearF32Params& p, const uint16
     const size_t lds = (size_t)STAGES * (DM + TN) * 64 * 2;
     static LdsLimit lim;
     UZU_REQUIRE(raise_lds_limit(lim, (const void*)linear_dma_kernel<WM, WN, MB, STAGES, GROUPED, KIND, PARTS>, lds), "linear_dma: %zu bytes of LDS are not available", lds);
-    return launch_check([&] { hipLaunchKernelGGL((linear_dma_kernel<WM, WN, MB, STAGES, GROUPED, KIND, PARTS>), grid, dim3(64 * WM * WN), lds, s, p, xb, PARTS * p.k, gr, partials); }, "linear_dma");
+    return launch_check([&] { hipLaunchKernelGGL((linear_dma_kernel<WM, WN, MB, STAGES, GROUPED, KIND, PARTS>), grid, dim3(64 * WM * WN), lds, s, p, xb, PARTS * p.k, gr, partials, linear_tile_order(p, PARTS)); }, "linear_dma");
 }
 template <bool GROUPED, int KIND, uint32_t PARTS> uzu_status launch_dma(hipStream_t s, const LinearF32Params& p, const uint16_t* xb, const GatedRows& gr = GatedRows()) {
     const size_t tiles = (size_t)((p.rows + 127) / 128) * ((p.n + DN - 1) / DN);
