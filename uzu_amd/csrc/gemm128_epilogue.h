@@ -11,7 +11,7 @@ namespace uzu {
 namespace k {
 
 // activate_bf16_tab of a gate that holds a bf16 number: SiLU by the hardware's exp2 and reciprocal.  -x times log2 e's leading 15 bits is exact, the rest of the constant joins
-// as a factor: the quotient is within 8 f32 ulps, and silu_bf16_near has the 64-bit exponential decide where that could change the
+// as a factor (its square, dropped, is 0.6 ulp at 80; the exponential, the reciprocal and three roundings 1 or 1/2 each): the quotient is within 8 f32 ulps, and silu_bf16_near has the 64-bit exponential decide where that could change the
 // bf16 rounding.  4096 x 28672 x 4096: 1145 -> 1081 us.
 __device__ __forceinline__ float gate_act(uint32_t act, float x, const uint64_t* tab) {
     if (act != 0) return activate_bf16_tab(act, x, tab);

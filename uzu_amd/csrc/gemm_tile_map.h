@@ -1,4 +1,5 @@
-// gemm_tile_map.h -- workgroup id -> output tile of the large-tile prefill GEMM (k_gemm128.hip).
+// gemm_tile_map.h -- workgroup id -> output tile of the W8A8 GEMM (k_activation_transform.hip): super-tiles dealt to the XCDs whole, which leaves some with more tiles than others where there are
+// few (gemm_tile_order.h: equal shares; the other large-tile products).
 // Plain C++ so that tests/test_host_math.py can compile it for the host and check that every tile is visited exactly once.
 #pragma once
 #include <stdint.h>

@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(256, 3) dn_chunk_prep_kernel(const float* q_no
                                                             const uint16_t* in_proj, const float* a_log, const float* dt_bias, float* q_norm_out, float* k_norm_out,
                                                             uint32_t value_dim, const uint16_t* conv_rows, float* conv_state) {
     __shared__ __attribute__((aligned(16))) float sK[CC * KP], sQ[CC * KP], sV[CC * KP];
-    // M (by columns) and the decay ratios: in the Q rows once the Gram products have read them (a barrier in between): four workgroups per CU
+    // M (by columns) and the decay ratios: in the Q rows once the Gram products have read them (a barrier in between): 51 KB, three workgroups per CU
     float* const sMt = sQ;
     float* const sRat = sQ + CC * TP;
     static_assert(2 * CC * TP <= CC * KP, "the matrices fit in the Q rows");
@@ -791,7 +791,6 @@ uzu_status delta_net_prefill_chunked(hipStream_t s, const float* q_norm, const f
                                      uint32_t key_dim, uint32_t value_dim, uint32_t suffix_len) {
     return prefill_chunked(s, (float*)q_norm, (float*)k_norm, beta, decay, in_proj, state, out, workspace, num_v_heads, num_k_heads, head_v_dim, key_dim, value_dim, suffix_len, nullptr);
 }
-// UZU_HIP_TUNE=prep_fused=0: DeltaNetPrefillPrep as its own launch in front (tests/test_gpu_prefill_switches.py holds the fused kernel to it, bit for bit)
 // UZU_HIP_TUNE=prep_fused=0: DeltaNetPrefillPrep as its own launch in front (tests/test_gpu_prefill_switches.py holds the fused kernel to it, bit for bit)
 bool delta_net_prefill_prep_fused_enabled() {
     const char* e = tune_env("prep_fused");

@@ -4,13 +4,13 @@
 //   * Four waves as 2 x 2, each wave 64 x 64 = 2 x 2 blocks of v_mfma_f32_32x32x16_bf16.  The k order inside a k-step
 //     is free as long as A and B agree: lanes 0..31 take k = 8s..8s+7, lanes 32..63 take k = 32+8s..32+8s+7 at MFMA
 //     s of a 64-wide k-step, so the B operand of a lane is one 16-byte vector of its column's packed codes: global ->
-//     VGPR -> exact centred bf16 codes (v_cvt_off_f32_i4 / sext byte converts, as in k_gemm.hip) -> MFMA.  Only the
+//     VGPR -> exact bf16 codes (int4: 16 + u in pairs, gemm_convert.h; int8: sext byte converts) -> MFMA.  Only the
 //     activations are staged through LDS (double buffered, 144-byte pitch), one LDS-only barrier per k-step.
 //   * A quant group accumulates into acc_g (first MFMA of the group takes C = 0); at the group boundary
-//     acc_t += scale[n,g] * acc_g on the VALU (packed f32 FMAs).
+//     acc_t += scale[n,g] * acc_g on the VALU.
 //   * The offset term  sum_g coef[n,g] * rowsum_g(A)[m]  is added once, in the epilogue: a pre-pass writes the group
-//     row sums of A (f32, [group][row]), and every lane runs G packed FMAs per pair of its 64 outputs -- no row-sum
-//     MFMAs and no per-group offset work in the main loop.
+//     row sums of A (f32, [group][row]) unless A's producer has filed them, and f32 MFMAs contract them with the
+//     coefficients -- no per-group offset work in the main loop.
 //   * Every global load is unconditional (rows / columns / steps clamped into range) and prefetched into a register
 //     ring; the loop is unrolled by the ring depth so that all indices are static (vmcnt waits stay counted).
 //   * int4 in groups of 128 has two forms with its operands by LDS DMA besides (takes_dma): k_gemm_dma.hip.

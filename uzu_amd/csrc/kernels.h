@@ -77,6 +77,7 @@ bool matmul_act_mul_supported(hipStream_t s, const MatmulParams& p, int num_cus)
 // k_gemm_rows.hip: 17 to hundreds of activation rows (wide matrices: 2 and more) against int4 codes in groups of 128, register-fed or (from 128 rows on) staged in tiles of 64 x 128
 bool gemm_rows_preferred(const MatmulParams& p, int num_cus);
 uzu_status gemm_rows(hipStream_t s, const MatmulParams& p, int num_cus);
+// (of a product without a Normalization behind: one that adds the shares makes them cheaper, and K may be cut further, which is another order of the f32 sums)
 void gemm_rows_plan_query(const MatmulParams& p, int num_cus, uint32_t* splits, uint32_t* workgroups);
 uint32_t gemm128_splits(const MatmulParams& p, int num_cus); // k_gemm128.hip: the cuts of K of a product on the large tiles (0: none that it takes)
 bool gemm_split_joins_norm(const MatmulParams& p, const float* partials, uint32_t splits); // k_gemm128.hip: whether gemm_split_finish leaves the sums to p.post_norm
@@ -212,8 +213,6 @@ __host__ __device__ inline void attention_resolve_dyn(AttentionParams& a) {
 }
 uzu_status attention_single_pass(hipStream_t s, const AttentionParams& p, void* out);
 bool attention_prefill_mfma_supported(const AttentionParams& p); // k_attention_mfma.hip: causal bf16 prefill tiles on the matrix cores
-// gate / gate_done (optional): when the pass ends in the key-split merge, SigmoidGate of `gate` (bf16, the layout of `out`) is applied there and *gate_done = 1
-// (bit-identical to the separate launch); otherwise the caller runs sigmoid_gate itself
 // the same attention of several sequences in one launch (equal suffix lengths; `p` is any one of them): kMost at a time
 struct AttentionSeqs {
     static constexpr uint32_t kMost = 8;
@@ -224,8 +223,10 @@ struct AttentionSeqs {
     void* out[kMost];
     uint32_t n;
 };
-bool attention_prefill_mfma_joins(const AttentionParams& p, uint32_t sequences); // whether a sequence of such a batch is to go into an AttentionSeqs launch
+bool attention_prefill_mfma_joins(const AttentionParams& p, uint32_t sequences); // whether a sequence goes into an AttentionSeqs launch, of which a full one has that many
 uzu_status attention_prefill_mfma_seqs(hipStream_t s, const AttentionParams& p, const AttentionSeqs& q);
+// gate / gate_done (optional): when the pass ends in the key-split merge, SigmoidGate of `gate` (bf16, the layout of `out`) is applied there and *gate_done = 1
+// (bit-identical to the separate launch); otherwise the caller runs sigmoid_gate itself
 uzu_status attention_prefill_mfma(hipStream_t s, const AttentionParams& p, void* out, const void* gate = nullptr, uint32_t* gate_done = nullptr);
 uzu_status attention_two_pass1(hipStream_t s, const AttentionParams& p, float* partials, float* sums, float* maxs);
 uzu_status attention_two_pass2(hipStream_t s, const float* partials, const float* sums, const float* maxs, void* out,
