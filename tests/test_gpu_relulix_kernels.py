@@ -139,6 +139,35 @@ def test_attention_of_decode_sized_passes(hip_ctx, H, G, dim, vd, window, cap, T
         assert not np.array_equal(got, attention(hip_ctx, q[T - rows:], K, V, mx, T - rows, bf16=1, form=1))
 
 
+@pytest.mark.parametrize("sinks", ["unit", None])
+@pytest.mark.parametrize("H,G,dim,vd,window,cap,T", [(1, 1, 128, 128, 1, 0.0, 5), (3, 1, 24, 40, 33, 0.0, 100), (8, 2, 128, 128, 64, 0.0, 70), (8, 2, 128, 128, 65, 5.0, 70), (8, 2, 128, 120, 1024, 0.0, 1400),
+                                                     (5, 1, 64, 64, 0, 0.0, 1), (5, 1, 64, 48, 257, 0.0, 258), (2, 2, 32, 8, 300, 0.0, 299), (12, 2, 8, 32, 1000, 2.0, 700), (16, 4, 128, 128, 0, 0.0, 2100)])
+def test_attention_step_form(hip_ctx, H, G, dim, vd, window, cap, T, sinks):
+    """One row per sequence: one share and many, a share's turns of 32 / 64 / 128 keys at their edges, shares without a key, query heads in blocks of one, two and four with a rest, widths that are
+    padded.  The products are exact and added in f32, so it is as close to the oracle as the simple form."""
+    rng = np.random.default_rng(H * 100 + T + 4)
+    q, K, V = qkv(rng, T, H, G, dim, vd)
+    mx = {"heads": H, "kv_heads": G, "scale": 1.7 / np.sqrt(dim), "mask": {"size": window}, "softcap": cap}
+    Kb, Vb = O.to_bf16(K), O.to_bf16(V)
+    if sinks is None:
+        want = np.stack([simple_softmax(f32(q)[-1, a], Kb, Vb, mx, a // (H // G)) for a in range(H)])[None]
+    else:
+        want = O.attention_core(f32(q)[T - 1:], Kb, Vb, mx, T - 1)
+    got = attention(hip_ctx, q[T - 1:], K, V, mx, T - 1, sinks=sinks, bf16=1, form=4)
+    assert np.isfinite(got).all() and np.abs(got - want).max() < 2e-5 * np.abs(want).max()
+
+
+def simple_softmax(q, K, V, mx, g):
+    """one query over the keys of its window, no sink"""
+    window = int(mx["mask"]["size"])
+    lo = max(0, len(K) - window) if window else 0
+    s = (K[lo:, g] @ q) * np.float32(mx["scale"])
+    if mx["softcap"]:
+        s = mx["softcap"] * np.tanh(s / mx["softcap"])
+    e = np.exp(s - s.max())
+    return (e / e.sum()) @ V[lo:, g]
+
+
 @pytest.mark.parametrize("bf16,form", [(0, 1), (1, 1), (1, 2)])
 @pytest.mark.parametrize("window", [1, 2, 31, 32, 33, 64, 65, 130])
 def test_one_key_stands_out_just_inside_and_just_outside_the_window(hip_ctx, bf16, form, window):

@@ -320,7 +320,7 @@ uzu_status uzu_hip_s32_window_attention(uzu_hip_context* ctx, const float* q, co
     if (form >= 3) { // the matrix-core form with its key blocks split over workgroups + the merge launch
         float* ws = nullptr;
         if (form == 3) p.form = 2, p.splits = 5;
-        else p.form = 0, k::window_attention_split_keys(p, window ? std::min(window, start + rows) : start + rows, ctx->num_cus);
+        else p.form = 0, p.one_row = rows == 1, k::window_attention_split_keys(p, window ? std::min(window, start + rows) : start + rows, ctx->num_cus);
         p.split_ws_bytes = k::window_attention_split_ws_bytes(rows, heads, p.splits);
         UZU_PROPAGATE(S.up((const float*)nullptr, p.split_ws_bytes / 4, &ws));
         p.split_ws = ws;

@@ -403,6 +403,25 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
         }
         bool conv_rides = false;
         const uint32_t ldj = (X.joint.n + 3) / 4 * 4, ldo_joint = X.joint_out.k; // row pitches of the joint projection and of its halves' results
+        // the state-space mixer beside attention: x | B | C stand behind q | k | v in the convolved rows, z | dt behind all of them in the projected ones
+        const uint32_t state_inner = h.dn_num_heads * h.dn_value_head_dim, z_col = X.conv_channels;
+        bool state_beside = false; // its recurrence and norm ran in the attention's launches
+        auto state_params = [&]() {
+            const uint32_t Gs = h.dn_num_groups, N = h.dn_head_dim, x_col = X.conv_act_from;
+            k::DecayedStateParams dp{};
+            dp.rows_in = S.dn_cv, dp.ld = X.conv_channels, dp.q_col = x_col + state_inner + Gs * N, dp.k_col = x_col + state_inner, dp.v_col = x_col, dp.decay = S.q + z_col + state_inner;
+            dp.lddecay = ldj, dp.per_head = 1, dp.a_log = L.a_log, dp.dt_bias = L.dt_bias, dp.skip = X.ssd_skip, dp.q_scale = 1.0f, dp.out = S.dn_o;
+            dp.states = S.d_pair_state_ptrs + (size_t)l * S.max_seqs, dp.spans = S.d_spans, dp.nseq = nseq, dp.rows = rows, dp.heads = h.dn_num_heads, dp.groups = Gs, dp.dim = N;
+            dp.vdim = h.dn_value_head_dim, dp.chunk_ws = S.lin_ws, dp.chunk_ws_bytes = S.lin_ws_bytes;
+            for (uint32_t i = 0; i < nseq; ++i) dp.chunks += (counts[i] + 63) / 64;
+            return dp;
+        };
+        auto gated_norm_params = [&]() {
+            k::GatedNormParams np{};
+            np.y = S.dn_o, np.ldy = state_inner, np.gate = S.q + z_col, np.ldgate = ldj, np.weight = X.ssd_norm, np.out = S.attn + H * vd, np.ldo = ldo_joint, np.eps = h.dn_norm_epsilon;
+            np.out_scale = h.pair_scale_second != 0.0f ? h.pair_scale_second : 1.0e-37f, np.rows = rows, np.width = state_inner, np.parts = h.ssd_norm_groups ? h.ssd_norm_groups : 1;
+            return np;
+        };
         if (joint) {
             k::LinearF32Params jp = lin(S, X.joint, mix_in, S.q, rows);
             jp.ldy = ldj;
@@ -461,8 +480,18 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
             // decode-sized passes: spread a tile's key blocks over workgroups (a constant of the layer, so that a captured step stays valid as the context grows)
             uint32_t keys = h.sliding_window_size ? h.sliding_window_size : m->d.max_context_length;
             if (h.attention_chunk_size) keys = std::min(keys, h.attention_chunk_size);
-            if (rows <= 4 * S.max_seqs && rows * H <= 4096) k::window_attention_split_keys(ap, keys, m->ctx->num_cus), ap.split_ws = S.att_ws, ap.split_ws_bytes = S.att_ws_bytes;
-            RUN("window_attention", (size_t)rows * H * (hd + vd) * 4, k::window_attention(s, ap));
+            ap.one_row = max_count == 1;
+            if (rows <= 4 * S.max_seqs && rows * H <= 4096) ap.split_ws = S.att_ws, ap.split_ws_bytes = S.att_ws_bytes, k::window_attention_split_keys(ap, keys, m->ctx->num_cus);
+            state_beside = joint && k::window_attention_step_supported(ap) && k::window_attention_step_beside(state_params());
+            if (state_beside) { // a decode step: the other half's recurrence beside the shares of the keys, its norm beside their merge
+                const k::DecayedStateParams dp = state_params();
+                const k::GatedNormParams np = gated_norm_params();
+                RUN("window_attention+decayed_state", (size_t)rows * H * (hd + vd) * 4 + (size_t)nseq * dp.heads * dp.dim * dp.vdim * 8, k::window_attention_step(s, ap, &dp));
+                if (ap.splits > 1) RUN("window_attention_merge+gated_norm", (size_t)rows * (np.width * 12 + H * vd * 4 * (ap.splits + 1)), k::window_attention_merge(s, ap, &np));
+                else RUN("gated_norm_rows", (size_t)rows * np.width * 12, k::gated_norm_rows(s, np));
+            } else {
+                RUN("window_attention", (size_t)rows * H * (hd + vd) * 4, k::window_attention(s, ap));
+            }
         } else if (h.mixer_kind == UZU_MIXER_GATED_LINEAR_ATTENTION) { // queries | keys | values | gate | decay down
             const uint32_t ldq = L.qkv.n, v_col = 2 * H * hd, g_col = v_col + H * vd, a_col = g_col + H * vd;
             {   // the decay's second factor: what enters the recurrence is never rounded, a true f32 product in both precisions
@@ -561,19 +590,13 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
             if (hipEventRecord(S.side_join, S.side) != hipSuccess && e.st == UZU_OK) set_error("engine: recording the side stream's join failed"), e.st = UZU_ERR_HIP;
             s = main_stream, e.s = main_stream;
         }
-        if (joint) { // the state-space mixer beside attention: x | B | C stand behind q | k | v in the convolved rows, z | dt behind all of them in the projected ones
-            const uint32_t Hs = h.dn_num_heads, Gs = h.dn_num_groups, N = h.dn_head_dim, pv = h.dn_value_head_dim, inner = Hs * pv, x_col = X.conv_act_from;
-            const uint32_t z_col = X.conv_channels, dt_col = z_col + inner;
-            k::DecayedStateParams dp{};
-            dp.rows_in = S.dn_cv, dp.ld = X.conv_channels, dp.q_col = x_col + inner + Gs * N, dp.k_col = x_col + inner, dp.v_col = x_col, dp.decay = S.q + dt_col, dp.lddecay = ldj, dp.per_head = 1;
-            dp.a_log = L.a_log, dp.dt_bias = L.dt_bias, dp.skip = X.ssd_skip, dp.q_scale = 1.0f, dp.out = S.dn_o, dp.states = S.d_pair_state_ptrs + (size_t)l * S.max_seqs, dp.spans = S.d_spans;
-            dp.nseq = nseq, dp.rows = rows, dp.heads = Hs, dp.groups = Gs, dp.dim = N, dp.vdim = pv, dp.chunk_ws = S.lin_ws, dp.chunk_ws_bytes = S.lin_ws_bytes;
-            for (uint32_t i = 0; i < nseq; ++i) dp.chunks += (counts[i] + 63) / 64;
-            RUN("decayed_state", (size_t)rows * (2 * inner + 2 * Gs * N) * 4 + (size_t)nseq * Hs * N * pv * 8, k::decayed_state(s, dp));
-            k::GatedNormParams np{};
-            np.y = S.dn_o, np.ldy = inner, np.gate = S.q + z_col, np.ldgate = ldj, np.weight = X.ssd_norm, np.out = S.attn + H * vd, np.ldo = ldo_joint, np.eps = h.dn_norm_epsilon;
-            np.out_scale = h.pair_scale_second != 0.0f ? h.pair_scale_second : 1.0e-37f, np.rows = rows, np.width = inner, np.parts = h.ssd_norm_groups ? h.ssd_norm_groups : 1;
-            RUN("gated_norm_rows", (size_t)rows * inner * 12, k::gated_norm_rows(s, np));
+        if (joint) {
+            if (!state_beside) {
+                const k::DecayedStateParams dp = state_params();
+                RUN("decayed_state", (size_t)rows * (2 * dp.heads * dp.vdim + 2 * dp.groups * dp.dim) * 4 + (size_t)nseq * dp.heads * dp.dim * dp.vdim * 8, k::decayed_state(s, dp));
+                const k::GatedNormParams np = gated_norm_params();
+                RUN("gated_norm_rows", (size_t)rows * np.width * 12, k::gated_norm_rows(s, np));
+            }
             if (forked && hipStreamWaitEvent(main_stream, S.side_join, 0) != hipSuccess && e.st == UZU_OK) set_error("engine: waiting for the side stream failed"), e.st = UZU_ERR_HIP;
             run_linear(e, lin(S, X.joint_out, S.attn, S.tmp, rows)); // both halves' out projections, summed
             add_normed(S.tmp, cur, slot, L.post_mixer, X.ls1, pre_mlp_fused ? &L.pre_mlp : (h.no_mlp && !h.has_ple) ? next_pre : nullptr);

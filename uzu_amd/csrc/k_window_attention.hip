@@ -308,6 +308,10 @@ uzu_status window_attention(hipStream_t s, const WindowAttentionParams& params) 
     UZU_REQUIRE(p.heads && p.kv_heads && p.heads % p.kv_heads == 0 && p.dim && p.vdim, "window_attention: %u query heads on %u key / value heads", p.heads, p.kv_heads);
     UZU_UNSUPPORTED(p.vdim > 64 * kMaxVecPerLane || p.dim > 8192, "window_attention: value width %u (at most %u)", p.vdim, 64 * kMaxVecPerLane);
     UZU_REQUIRE(!p.dist_bias || p.dist_rows, "window_attention: a distance bias without its rows");
+    if (p.form == 0 && window_attention_step_supported(p)) {
+        UZU_PROPAGATE(window_attention_step(s, p, nullptr));
+        return p.splits > 1 ? window_attention_merge(s, p, nullptr) : UZU_OK;
+    }
     if (p.form == 2 || (p.form == 0 && window_attention_mfma_supported(p))) {
         UZU_UNSUPPORTED(!window_attention_mfma_supported(p), "window_attention: the matrix-core form does not take this shape");
         return window_attention_mfma(s, p);

@@ -349,12 +349,22 @@ struct WindowAttentionParams {
     uint32_t splits, split_items; // split_items: items a workgroup takes, 128 (stretches of 32 keys) or 32 (of 128; also 0)
     float* split_ws;
     size_t split_ws_bytes;
+    uint32_t one_row; // every sequence of the pass brings exactly one row (row r is sequence r's): the step form, with `splits` >= 1 shares of a row's keys
 };
-// `splits` and `split_items` of a decode-sized pass whose rows see `keys` keys at the most, from `tiles` and `kv_heads`: at most 16 splits
+// `splits` and `split_items` of a decode-sized pass whose rows see `keys` keys at the most, from `rows`, `tiles` and `kv_heads`: at most 16 splits, of the step form at most 32
 void window_attention_split_keys(WindowAttentionParams& p, uint32_t keys, uint32_t num_cus);
 size_t window_attention_split_ws_bytes(uint32_t rows, uint32_t heads, uint32_t splits);
 bool window_attention_mfma_supported(const WindowAttentionParams& p);
 uzu_status window_attention(hipStream_t s, const WindowAttentionParams& p);
+// The step form's two launches (k_window_attention_step.hip) with work of a mixer beside attention in further workgroups: the recurrence of one row per sequence with the shares of the keys,
+// a norm of rows of its own with the merge of the shares (only with `splits` > 1).  ldo and out_scale are set.
+struct DecayedStateParams;
+struct GatedNormParams;
+bool window_attention_step_supported(const WindowAttentionParams& p);
+bool window_attention_step_beside(const DecayedStateParams& d);
+uint32_t window_attention_step_splits(const WindowAttentionParams& p, uint32_t keys, uint32_t num_cus);
+uzu_status window_attention_step(hipStream_t s, const WindowAttentionParams& p, const DecayedStateParams* beside);
+uzu_status window_attention_merge(hipStream_t s, const WindowAttentionParams& p, const GatedNormParams* beside);
 
 // Hyper-connections.  The residual stream is `streams` = s copies x_a of every row (copy a at src + a * src_stride, rows of width d).  Per row, in this order:
 //   join (y != null):  x_b <- sum_a mix[a, b] x_a + mult * out[b] * y       all from the old ones; stored at dst + b * dst_stride (dst may be src; null: not stored)
