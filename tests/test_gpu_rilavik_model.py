@@ -108,6 +108,25 @@ def test_f32_experts_of_a_prompt_from_bf16_parts(hip_ctx, tmp_path):
     m.close()
 
 
+@pytest.mark.parametrize("width,experts,top,ff", [(8, 1, 1, 8), (520, 9, 8, 13), (1024, 64, 2, 40), (2056, 3, 3, 16), (4096, 8, 2, 24), (4104, 8, 2, 24)])
+def test_decode_steps_that_join_norm_and_route_in_one_launch(hip_ctx, tmp_path, width, experts, top, ff):
+    """A row joins the stream, is normed and routed in front of its experts: one round of four coordinates a thread and two with a rest, outputs below, at and above a workgroup's waves, as many
+    winners as are kept, and a width that the launch does not take; one sequence alone (the experts' first products in the same launch) and three together."""
+    cfg = gla(heads=1, dim=8, vdim=8, mlp=O.moe(experts, top, ff), width=width)
+    W, m = make(hip_ctx, tmp_path, cfg, experts + width, ctx_len=32)
+    toks = [prompt(cfg, 6, seed) for seed in (1, 2)]
+    for t in toks:
+        want, _ = O.forward(cfg, W, t)
+        assert rows_ok(O.logit_error(in_portions(m, t, [1] * 6), want), True)
+    states = [m.new_state() for _ in toks]
+    got = [m.step_batch(states, [[t[i]] for t in toks], [[0], [0]])[0] for i in range(6)]
+    for s, t in enumerate(toks):
+        assert rows_ok(O.logit_error(np.stack([g[s] for g in got]), O.forward(cfg, W, t)[0]), True)
+    for st in states:
+        st.close()
+    m.close()
+
+
 def test_greedy_choices_of_many_sequences(hip_ctx, tmp_path):
     """A pass that chooses and commits for more sequences than one commit launch holds, some of them with logits wanted too, some still inside their prompt: every sequence's tokens
     are those it gets alone, and decode continues from the token a batched step left."""

@@ -359,6 +359,29 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
         const bool pre_mlp_fused = !h.no_mlp && !h.parallel_block && L.post_mixer.present && L.post_mixer.groups <= 1 && L.pre_mlp.present && h.pre_mlp_norm.kind == UZU_NORM_STATISTICS &&
                                    L.pre_mlp.groups <= 1;
         if (next_pre && ((L.post_mixer.present && L.post_mixer.groups > 1) || (L.post_mlp.present && L.post_mlp.groups > 1) || (h.has_ple && L.ple_norm.groups > 1))) next_pre = nullptr;
+        // a decode step's experts: the launch that joins the mixer's result to the stream and norms it also routes the row (and, one row, runs the winners' first products)
+        const bool route_rides = pre_mlp_fused && rows <= 64 && !hs && h.mlp_kind == UZU_MLP_MOE && h.moe.routing == UZU_MOE_ROUTE_SIGMOID_GROUPS && !X.in_conv_mlp;
+        auto route_params = [&](const float* x) {
+            const uzu_moe_desc& M = h.moe;
+            k::RouteGroupsParams rp{};
+            rp.x = x, rp.router = L.moe.router_weights, rp.selection_bias = X.selection_bias, rp.ids = S.moe_ids, rp.weights = S.moe_w, rp.rows = rows, rp.d = d, rp.outputs = M.num_routed_experts;
+            rp.top = M.num_active_experts, rp.groups = M.router_groups ? M.router_groups : 1, rp.keep = M.router_groups_keep ? M.router_groups_keep : rp.groups, rp.bf16_products = bf;
+            rp.scale = M.router_scale != 0.0f ? M.router_scale : 1.0f, rp.raw = M.router_raw;
+            return rp;
+        };
+        k::NormAddParams join_add{};
+        bool join_waits = false; // the mixer's result joins in the router's launch
+        auto join_mixer = [&](float* slot) { // the mixer's result in S.tmp joins the stream behind its own norm (and the layer scale)
+            const DNorm* next = pre_mlp_fused ? &L.pre_mlp : (h.no_mlp && !h.has_ple) ? next_pre : nullptr;
+            if (route_rides) {
+                join_add.y = S.tmp, join_add.residual = cur, join_add.out = slot, join_add.scales = L.post_mixer.scales, join_add.layer_scale = X.ls1, join_add.offset = L.post_mixer.offset;
+                join_add.eps = L.post_mixer.eps, join_add.next = S.normed, join_add.next_scales = next->scales, join_add.next_offset = next->offset, join_add.next_eps = next->eps;
+                join_add.rows = rows, join_add.d = d;
+                join_waits = k::norm_route_supported(join_add, route_params(S.normed));
+            }
+            if (!join_waits) add_normed(S.tmp, cur, slot, L.post_mixer, X.ls1, next);
+            normed_ready = h.no_mlp && !h.has_ple && next_pre;
+        };
         const bool have_normed = normed_ready;
         normed_ready = false;
         const float* mix_in = S.normed; // the rows the mixer reads
@@ -599,8 +622,7 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
             }
             if (forked && hipStreamWaitEvent(main_stream, S.side_join, 0) != hipSuccess && e.st == UZU_OK) set_error("engine: waiting for the side stream failed"), e.st = UZU_ERR_HIP;
             run_linear(e, lin(S, X.joint_out, S.attn, S.tmp, rows)); // both halves' out projections, summed
-            add_normed(S.tmp, cur, slot, L.post_mixer, X.ls1, pre_mlp_fused ? &L.pre_mlp : (h.no_mlp && !h.has_ple) ? next_pre : nullptr);
-            normed_ready = h.no_mlp && !h.has_ple && next_pre;
+            join_mixer(slot);
         } else if (h.pair_mixer) { // the second mixer beside the first: a delta rule with a decay per head and key channel, reading the same rows
             const uint32_t Hd = h.dn_num_heads, Gd = h.dn_num_groups, dk = h.dn_head_dim, dv = h.dn_value_head_dim, taps = h.dn_kernel_size, ldi = L.in_proj.n;
             const uint32_t conv_dim = 2 * Gd * dk + Hd * dv, b_col = conv_dim, a_col = b_col + Hd, g_col = a_col + h.dn_decay_rank;
@@ -645,8 +667,7 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
             add_normed(S.tmp, cur, slot, L.post_mixer, X.ls1, nullptr);
         } else if (L.post_mixer.present) { // the mixer's result joins the stream behind its own norm (and the layer scale)
             run_linear(e, lin(S, L.out, S.attn, S.tmp, rows));
-            add_normed(S.tmp, cur, slot, L.post_mixer, X.ls1, pre_mlp_fused ? &L.pre_mlp : (h.no_mlp && !h.has_ple) ? next_pre : nullptr);
-            normed_ready = h.no_mlp && !h.has_ple && next_pre;
+            join_mixer(slot);
         } else { // X_(l+1) = input + out projection
             k::LinearF32Params p = lin(S, L.out, S.attn, slot, rows);
             if (!hs) p.residual = cur, p.ldr = d;
@@ -668,12 +689,15 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
                 const float* res = hs || L.post_mlp.present ? nullptr : slot;
                 float* moe_out = L.post_mlp.present ? S.tmp : slot;
                 const bool on_input = M.weight_on_input != 0;
-                if (M.routing == UZU_MOE_ROUTE_SIGMOID_GROUPS) {
-                    k::RouteGroupsParams rp{};
-                    rp.x = mlp_in, rp.router = L.moe.router_weights, rp.selection_bias = X.selection_bias, rp.ids = S.moe_ids, rp.weights = S.moe_w, rp.rows = rows, rp.d = d, rp.outputs = E;
-                    rp.top = top, rp.groups = M.router_groups ? M.router_groups : 1, rp.keep = M.router_groups_keep ? M.router_groups_keep : rp.groups, rp.bf16_products = bf;
-                    rp.scale = M.router_scale != 0.0f ? M.router_scale : 1.0f, rp.raw = M.router_raw;
-                    RUN("moe_route_groups", (size_t)E * d * 2, k::moe_route_groups(s, rp));
+                bool gate_up_done = false;
+                if (join_waits) {
+                    const k::RouteGroupsParams rp = route_params(mlp_in);
+                    gate_up_done = k::norm_route_gate_up_supported(join_add, rp, L.moe.w13, ff, act);
+                    if (gate_up_done)
+                        RUN("norm_add+route+gate_up", (size_t)d * 24 + (size_t)E * d * 2 + (size_t)top * 2 * ff * d * 2, k::norm_route_gate_up(s, join_add, rp, L.moe.w13, S.hid, ff, act, on_input));
+                    else RUN("norm_add+route", (size_t)rows * d * 16 + (size_t)E * d * 2, k::norm_route_rows(s, join_add, rp));
+                } else if (M.routing == UZU_MOE_ROUTE_SIGMOID_GROUPS) {
+                    RUN("moe_route_groups", (size_t)E * d * 2, k::moe_route_groups(s, route_params(mlp_in)));
                 } else if (M.routing == UZU_MOE_ROUTE_SCORES) {
                     RUN("moe_route_scores", (size_t)(E + M.num_identity_experts) * d * 2,
                         k::moe_route_scores(s, mlp_in, L.moe.router_weights, X.selection_bias, S.moe_ids, S.moe_w, rows, d, E + M.num_identity_experts, top));
@@ -685,10 +709,10 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
                 gp.y2 = S.moe_y2, gp.perm = S.moe_perm, gp.slot_pos = S.moe_slot_pos, gp.offsets = S.moe_offsets, gp.cursor = S.moe_cursor;
                 gp.rows = rows, gp.d = d, gp.ff = ff, gp.routed = E, gp.top = top, gp.act = act, gp.pos_weight = on_input ? S.moe_pos_w : nullptr;
                 gp.f32_products = bf ? 0 : 1;
-                if (k::moe_experts_grouped_faster(gp) && k::moe_experts_grouped_supported(gp)) { // prefill-sized: buckets per expert through the matrix-core linear
+                if (!gate_up_done && k::moe_experts_grouped_faster(gp) && k::moe_experts_grouped_supported(gp)) { // prefill-sized: buckets per expert through the matrix-core linear
                     RUN("moe_experts_grouped", (size_t)E * (act.plain ? 2 : 3) * ff * d * 2 + (size_t)rows * top * ((act.plain ? 1 : 3) * ff + 2 * d) * 4, k::moe_experts_grouped(s, gp));
                 } else {
-                    RUN("moe_experts_gate_up", (size_t)rows * top * (act.plain ? 1 : 2) * ff * d * 2, k::moe_experts_gate_up(s, mlp_in, S.moe_ids, L.moe.w13, S.hid, rows, d, ff, E, top, bf, act, on_input ? S.moe_w : nullptr));
+                    if (!gate_up_done) RUN("moe_experts_gate_up", (size_t)rows * top * (act.plain ? 1 : 2) * ff * d * 2, k::moe_experts_gate_up(s, mlp_in, S.moe_ids, L.moe.w13, S.hid, rows, d, ff, E, top, bf, act, on_input ? S.moe_w : nullptr));
                     RUN("moe_experts_down_combine", (size_t)rows * top * ff * d * 2,
                         k::moe_experts_down_combine(s, S.hid, mlp_in, S.moe_ids, on_input ? nullptr : S.moe_w, L.moe.w2, res, moe_out, rows, d, ff, E, top, bf));
                 }

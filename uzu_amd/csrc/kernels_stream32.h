@@ -176,6 +176,24 @@ struct GatedRows {
 // The gated product of a dense block: hidden[r, f] = act(gate = y1[r, ff + f], up = y1[r, f])   (y1 f32 [rows][2 ff]: up rows first, as the packed projection yields them)
 uzu_status gated_act_rows(hipStream_t s, const float* y1, float* hidden, uint32_t rows, uint32_t ff, const ExpertAct& act);
 
+// rms_norm_add_rows with its `next`, as a part of other launches: out[r] = residual[r] + rms(y[r]) * (scales + offset) * layer_scale, next[r] = rms(out[r]) * (next_scales + next_offset)
+struct NormAddParams {
+    const float *y, *residual;
+    float* out;
+    const float *scales, *layer_scale; // layer_scale: f32 [d] or null
+    float offset, eps;
+    float* next;
+    const float* next_scales;
+    float next_offset, next_eps;
+    uint32_t rows, d;
+};
+bool norm_add_step_supported(const NormAddParams& n); // rows of up to 4096, a multiple of 8
+// ... and moe_route_groups of next (one group of outputs, up to 64 of them, up to 8 winners) in one launch; p.x is not read
+bool norm_route_supported(const NormAddParams& n, const RouteGroupsParams& p);
+uzu_status norm_route_rows(hipStream_t s, const NormAddParams& n, const RouteGroupsParams& p);
+// ... and, one row, moe_experts_gate_up of the winners as well (weight_on_input: the winners' weights multiply their products).  n.out apart from n.residual and n.y.
+bool norm_route_gate_up_supported(const NormAddParams& n, const RouteGroupsParams& p, const uint16_t* w13, uint32_t ff, const ExpertAct& act);
+uzu_status norm_route_gate_up(hipStream_t s, const NormAddParams& n, const RouteGroupsParams& p, const uint16_t* w13, float* hidden, uint32_t ff, const ExpertAct& act, uint32_t weight_on_input);
 // hidden[r * top + j, f] = act(gate_e x_r, up_e x_r) for e = ids[r, j] < routed; w13 bf16 [routed][2 ff][d], rows [0, ff) of an expert = up, [ff, 2 ff) = gate
 // in_weights (f32 [rows, top] or null): the expert reads in_weights[r, j] * x_r instead (both products are multiplied by it in front of the activation)
 uzu_status moe_experts_gate_up(hipStream_t s, const float* x, const int32_t* ids, const uint16_t* w13, float* hidden, uint32_t rows, uint32_t d, uint32_t ff, uint32_t routed,
