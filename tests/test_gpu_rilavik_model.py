@@ -127,6 +127,32 @@ def test_decode_steps_that_join_norm_and_route_in_one_launch(hip_ctx, tmp_path, 
     m.close()
 
 
+@pytest.mark.parametrize("width,vocab,layers", [(40, 53, 1), (1032, 530, 1), (64, 4099, 2), (2056, 97, 2), (4104, 61, 1), (36, 4099, 2)])
+def test_chained_greedy_steps(hip_ctx, tmp_path, width, vocab, layers):
+    """Decode steps that turn into one another on the device: the end of a layer and the projection (or the read-out) behind it in one launch, the choice among its workgroups' largest logits, the next
+    embedding row and norm -- and widths that those launches do not take.  A second half of the vocabulary repeats the first half's read-out rows, so every choice is a tie between two workgroups or
+    columns; a step from outside (another state, the same scratch) stands between two calls."""
+    pair = O.parallel_layer(O.left_half(2, 1, 8, 8, 9, conv=3), O.right_half(2, 8, 8, groups=1, norm_groups=1, conv=4), 0.7, 1.2, mlp=O.moe(3, 2, 16))
+    cfg = O.config(vocab=vocab, width=width, layers=[O.gla_layer(1, 8, 8, mlp=O.moe(3, 2, 16)), pair][-layers:])
+    W = O.weights(cfg, width)
+    W["head"] = O.to_bf16(W["head"] * 3.0)  # wider margins between the logits
+    half = (vocab + 1) // 2
+    W["head"][half:] = W["head"][:vocab - half]
+    O.write_model_dir(str(tmp_path / "m"), cfg, W)
+    m = HipModel(hip_ctx, loader.load_model_dir(str(tmp_path / "m"), max_context_length=64), MODEL_BATCH(2) | MODEL_FULL_F32)
+    p = prompt(cfg, 7, 3)
+    want = O.greedy(cfg, {k: v.astype(np.float64) for k, v in W.items()}, p, 9)
+    other = m.new_state()
+    got = [m.prefill(np.asarray(p, dtype=np.uint32))]
+    for steps in (1, 5, 2):
+        got += [int(t) for t in m.decode(steps)[0]]
+        assert int(np.argmax(m.read_logits_f32())) == got[-1] < half
+        m.step_batch([other], [[1, 2]], None, sample=True)
+    assert got == want and m.context_length == len(p) + 8
+    other.close()
+    m.close()
+
+
 def test_greedy_choices_of_many_sequences(hip_ctx, tmp_path):
     """A pass that chooses and commits for more sequences than one commit launch holds, some of them with logits wanted too, some still inside their prompt: every sequence's tokens
     are those it gets alone, and decode continues from the token a batched step left."""

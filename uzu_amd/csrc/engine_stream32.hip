@@ -66,6 +66,8 @@ struct Stream32 {
     uint8_t* tables = nullptr; // one block: the tables below up to tables_bytes, then d_row_seq
     size_t tables_bytes = 0;
     uint32_t* d_pass_sampled = nullptr; // [max_seqs]: a pass's greedy choices
+    float* turn_value = nullptr;        // [kNormLinearParts]: the largest logits of the read-out's workgroups in a decode step that chains
+    uint32_t* turn_index = nullptr;     // ... and their tokens
     k::SeqSpan* d_spans = nullptr;
     uint32_t *d_row_seq = nullptr, *d_out_rows = nullptr;
     void** d_cache_ptrs = nullptr;  // [layers][max_seqs]: latent rows / key rows / the retention state
@@ -266,10 +268,24 @@ uzu_status s32_upload_tables(uzu_hip_model* m, const std::vector<PassSeq>& seqs,
     return UZU_OK;
 }
 
+// What turns one greedy decode step into the next (k::step_turn) for the sequence `st` (or none: the parts that do not depend on it)
+k::StepTurnParams s32_turn_params(const uzu_hip_model* m, const uzu_hip_state* st = nullptr) {
+    const Stream32& S = *m->s32;
+    const uzu_layer_desc& h = m->layers[0].d;
+    const DNorm& N = m->layers[0].pre_mixer;
+    k::StepTurnParams p{};
+    if (st) p.part_value = S.turn_value, p.part_index = S.turn_index, p.ctx_len = st->d_ctx_len, p.tokens = st->d_tokens, p.out_token = st->d_out_token, p.sampled = st->d_sampled, p.span = S.d_spans;
+    p.table = (const uint16_t*)m->embedding.w, p.vocab = m->d.vocab_size, p.d = m->d.model_dim, p.scale = m->d.input_scale, p.out = S.slots;
+    if (N.present && h.pre_mixer_norm.kind == UZU_NORM_STATISTICS && N.groups <= 1 && !S.layers[0].reentry_a.w) p.normed = S.normed, p.scales = N.scales, p.offset = N.offset, p.eps = N.eps;
+    return p;
+}
+
 // The launches of one pass (tables uploaded before): rows = sum of the sequences' counts (<= max_rows), token ids on the device, row-major in sequence order;
 // n_out rows (S.d_out_rows) get logits in S.logits [n_out][vocab] f32.  Nothing here depends on the sequences' positions -- the kernels read them from the
 // device-side spans -- so a one-token step can be captured once and replayed.  Does not move the sequences' context lengths.
-uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, const uint32_t* d_tokens, uint32_t n_out) {
+// in_order: row i of the wanted logits is row i of the pass, all of them.  turn (decode steps that chain, s32_turn_params): the rows' embedding and the first norm are there already, and the
+// read-out leaves its parts' largest logits in S.turn_value / turn_index, *turn of them.
+uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, const uint32_t* d_tokens, uint32_t n_out, bool in_order = false, uint32_t* turn = nullptr) {
     Stream32& S = *m->s32;
     hipStream_t s = m->ctx->stream; // (the stream the next launch goes to: a pair's first mixer switches it to S.side and back)
     const hipStream_t main_stream = s;
@@ -283,7 +299,8 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
     const uint32_t bf = S.full_f32 ? 0u : 1u;
     uint32_t max_count = 0;
     for (uint32_t c : counts) max_count = std::max(max_count, c);
-    if (S.pair_table) { // + the hashed (previous token, token) row; two launches: the rows, then the sequences' new previous tokens
+    if (turn) {
+    } else if (S.pair_table) { // + the hashed (previous token, token) row; two launches: the rows, then the sequences' new previous tokens
         k::EmbedPairParams ep{};
         ep.tokens = d_tokens, ep.table = (const uint16_t*)m->embedding.w, ep.pair_table = S.pair_table, ep.out = S.slots, ep.rows = rows, ep.vocab = m->d.vocab_size, ep.d = d;
         ep.scale = m->d.input_scale, ep.buckets = m->d.bigram_buckets, ep.mul_prev = m->d.bigram_mul_prev, ep.mul_cur = m->d.bigram_mul_cur, ep.spans = S.d_spans;
@@ -337,7 +354,29 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
         copies |= join != nullptr;
         return fused ? S.normed : conv_input(l, S.normed, conv_w, taps, which);
     };
-    bool normed_ready = false; // S.normed already holds this run's pre-mixer norm (left by the run before)
+    bool normed_ready = turn != nullptr && s32_turn_params(m).normed != nullptr; // S.normed already holds this run's pre-mixer norm (left by the run before)
+    // One row: the end of a layer and the projection that reads its norm are one launch.  Then the new row goes to S.xin: other workgroups may still read the old one.
+    k::NormAddParams ahead{};
+    bool add_waits = false;
+    bool any_depth = false;
+    for (const Stream32::Layer& X : S.layers) any_depth |= X.depth_weights != nullptr;
+    auto run_first_linear = [&](const k::LinearF32Params& p) {
+        if (!add_waits) return run_linear(e, p);
+        add_waits = false;
+        RUN("norm_add+linear", (size_t)p.n * p.k * 2 + (size_t)d * 24, k::norm_linear(s, ahead, p));
+    };
+    auto first_linear = [&](uint32_t l, const float* x) { // the projection that reads layer l's normed rows
+        const Stream32::Layer& X = S.layers[l];
+        k::LinearF32Params p = lin(S, X.joint.w ? X.joint : m->layers[l].qkv, x, S.q, rows);
+        if (X.joint.w) p.ldy = (X.joint.n + 3) / 4 * 4;
+        return p;
+    };
+    auto head_linear = [&](const float* x) {
+        k::LinearF32Params head = lin(S, m->d.tied_embeddings ? m->embedding : m->output_embedding, x, S.logits, n_out);
+        if (m->d.logit_scale != 1.0f) head.y_scale = m->d.logit_scale; // (0 = a description that never set it)
+        head.soft_cap = m->d.logit_soft_cap;
+        return head;
+    };
     for (uint32_t l = 0; l < nl; ++l) {
         DLayer& L = m->layers[l];
         const Stream32::Layer& X = S.layers[l];
@@ -356,6 +395,8 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
         if (l + 1 < nl && !X.depth_weights && !S.layers[l + 1].reentry_a.w && m->layers[l + 1].pre_mixer.present && m->layers[l + 1].d.pre_mixer_norm.kind == UZU_NORM_STATISTICS &&
             m->layers[l + 1].pre_mixer.groups <= 1)
             next_pre = &m->layers[l + 1].pre_mixer;
+        // (the last layer: the read-out's norm, where the read-out takes all rows in order)
+        const DNorm* out_norm = l + 1 == nl && n_out == rows && in_order && !hs && !X.depth_weights && m->d.output_norm.kind == UZU_NORM_STATISTICS && m->output_norm.groups <= 1 && L.post_mlp.groups <= 1 ? &m->output_norm : nullptr;
         const bool pre_mlp_fused = !h.no_mlp && !h.parallel_block && L.post_mixer.present && L.post_mixer.groups <= 1 && L.pre_mlp.present && h.pre_mlp_norm.kind == UZU_NORM_STATISTICS &&
                                    L.pre_mlp.groups <= 1;
         if (next_pre && ((L.post_mixer.present && L.post_mixer.groups > 1) || (L.post_mlp.present && L.post_mlp.groups > 1) || (h.has_ple && L.ple_norm.groups > 1))) next_pre = nullptr;
@@ -381,6 +422,16 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
             }
             if (!join_waits) add_normed(S.tmp, cur, slot, L.post_mixer, X.ls1, next);
             normed_ready = h.no_mlp && !h.has_ple && next_pre;
+        };
+        auto join_mlp = [&]() { // the MLP's result in S.tmp joins, with the norm of what reads the layer's rows: the next layer's projection, or the read-out
+            const DNorm* next = h.has_ple ? nullptr : l + 1 < nl ? next_pre : out_norm;
+            normed_ready = next != nullptr;
+            if (next && rows == 1 && !hs && !any_depth && !S.taps && L.post_mlp.groups <= 1 && (l + 1 == nl || !S.layers[l + 1].in_conv_mixer)) {
+                ahead.y = S.tmp, ahead.residual = slot, ahead.out = S.xin, ahead.scales = L.post_mlp.scales, ahead.layer_scale = X.ls2, ahead.offset = L.post_mlp.offset, ahead.eps = L.post_mlp.eps;
+                ahead.next = S.normed, ahead.next_scales = next->scales, ahead.next_offset = next->offset, ahead.next_eps = next->eps, ahead.rows = rows, ahead.d = d;
+                add_waits = k::norm_linear_supported(ahead, l + 1 < nl ? first_linear(l + 1, S.normed) : head_linear(S.normed));
+            }
+            if (!add_waits) add_normed(S.tmp, slot, slot, L.post_mlp, X.ls2, next);
         };
         const bool have_normed = normed_ready;
         normed_ready = false;
@@ -446,9 +497,7 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
             return np;
         };
         if (joint) {
-            k::LinearF32Params jp = lin(S, X.joint, mix_in, S.q, rows);
-            jp.ldy = ldj;
-            run_linear(e, jp);
+            run_first_linear(first_linear(l, mix_in));
             mixer_conv(ldj);
             conv_rides = rows < 256 && k::conv_rope_append_supported(rp, conv);
             if (!conv_rides) run_mixer_conv();
@@ -463,7 +512,7 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
                 forked = true, s = S.side, e.s = S.side;
         }
         if (!joint) {
-            run_linear(e, lin(S, L.qkv, mix_in, S.q, rows)); // the packed projection of the mixer (queries first)
+            run_first_linear(first_linear(l, mix_in)); // the packed projection of the mixer (queries first)
             if (X.conv_w) {
                 mixer_conv(L.qkv.n);
                 conv_rides = rows < 256 && k::conv_rope_append_supported(rp, conv);
@@ -716,10 +765,7 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
                     RUN("moe_experts_down_combine", (size_t)rows * top * ff * d * 2,
                         k::moe_experts_down_combine(s, S.hid, mlp_in, S.moe_ids, on_input ? nullptr : S.moe_w, L.moe.w2, res, moe_out, rows, d, ff, E, top, bf));
                 }
-                if (L.post_mlp.present) {
-                    add_normed(S.tmp, slot, slot, L.post_mlp, X.ls2, h.has_ple ? nullptr : next_pre);
-                    normed_ready = !h.has_ple && next_pre;
-                }
+                if (L.post_mlp.present) join_mlp();
             } else {
                 if (h.mlp_plain) {
                     k::LinearF32Params up = lin(S, L.up, mlp_in, S.hid, rows);
@@ -733,8 +779,7 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
                 }
                 if (L.post_mlp.present) {
                     run_linear(e, lin(S, L.down, S.hid, S.tmp, rows));
-                    add_normed(S.tmp, slot, slot, L.post_mlp, X.ls2, h.has_ple ? nullptr : next_pre);
-                    normed_ready = !h.has_ple && next_pre;
+                    join_mlp();
                 } else {
                     k::LinearF32Params down = lin(S, L.down, S.hid, slot, rows);
                     if (!hs) down.residual = slot, down.ldr = d;
@@ -756,7 +801,7 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
             RUN("depth_mix", (size_t)rows * d * 4 * (l + 3), k::depth_mix(s, S.slots, slot_stride, X.depth_weights, h.num_depth_weights, S.xin, rows, d));
             cur = S.xin;
         } else {
-            cur = slot;
+            cur = add_waits ? S.xin : slot;
         }
         if (S.taps && !hs) HIPCHK(hipMemcpyAsync(S.taps + (size_t)l * slot_stride, cur, (size_t)rows * d * 4, hipMemcpyDeviceToDevice, s));
     }
@@ -773,11 +818,10 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
             const DNorm& N = m->output_norm;
             hp.h = S.out_normed, hp.scales = N.scales, hp.offset = N.offset, hp.eps = N.eps, hp.row_index = S.d_out_rows, hp.rows = n_out;
             RUN("hyper_step", (size_t)n_out * d * 4 * (hs + 2), k::hyper_step(s, hp));
-        } else run_norm(e, m->output_norm, m->d.output_norm.kind, S.alpha_out, cur, S.out_normed, n_out, d, S.d_out_rows);
-        k::LinearF32Params head = lin(S, m->d.tied_embeddings ? m->embedding : m->output_embedding, S.out_normed, S.logits, n_out);
-        if (m->d.logit_scale != 1.0f) head.y_scale = m->d.logit_scale; // (0 = a description that never set it)
-        head.soft_cap = m->d.logit_soft_cap;
-        run_linear(e, head);
+        } else if (!normed_ready) run_norm(e, m->output_norm, m->d.output_norm.kind, S.alpha_out, cur, S.out_normed, n_out, d, S.d_out_rows);
+        const k::LinearF32Params head = head_linear(normed_ready ? S.normed : S.out_normed);
+        if (add_waits) RUN("norm_add+readout", (size_t)head.n * head.k * 2, k::norm_linear(s, ahead, head, turn ? S.turn_value : nullptr, turn ? S.turn_index : nullptr, turn));
+        else run_linear(e, head);
         S.last_logit_rows = n_out;
     }
     if (e.st != UZU_OK) return e.st;
@@ -793,7 +837,9 @@ uzu_status s32_pass(uzu_hip_model* m, const std::vector<PassSeq>& seqs, const ui
     UZU_PROPAGATE(s32_upload_tables(m, seqs, out_rows));
     std::vector<uint32_t> counts;
     for (const PassSeq& q : seqs) counts.push_back(q.count);
-    return s32_encode(m, counts, d_tokens, (uint32_t)out_rows.size());
+    bool in_order = true;
+    for (size_t i = 0; i < out_rows.size(); ++i) in_order &= out_rows[i] == i;
+    return s32_encode(m, counts, d_tokens, (uint32_t)out_rows.size(), in_order);
 }
 
 uzu_status ensure_logits(uzu_hip_model* m, size_t rows) {
@@ -1334,6 +1380,12 @@ uzu_status s32_create(uzu_hip_context* ctx, const uzu_model_desc* desc, uint32_t
     if (any_normed_conv) TRY(need_f32(m, R * d, &S.conv_rows));
     if (w_latq) TRY(need_f32(m, R * w_latq, &S.lat_q));
     TRY(need_f32(m, R * d, &S.xin));
+    TRY(need_f32(m, k::kNormLinearParts, &S.turn_value));
+    {
+        float* q = nullptr;
+        TRY(need_f32(m, k::kNormLinearParts, &q));
+        S.turn_index = (uint32_t*)q;
+    }
     TRY(need_f32(m, R * d, &S.normed));
     TRY(need_f32(m, R * d, &S.out_normed));
     TRY(need_f32(m, R * w_q, &S.q));
@@ -1584,6 +1636,22 @@ uzu_status s32_prefill(uzu_hip_model* m, const uint32_t* token_ids, uint32_t cou
     return UZU_OK;
 }
 
+// Whether a decode step's last launch can choose its token: greedy, the last layer's end and the read-out one launch (what s32_encode asks for in join_mlp), the embedding a plain row
+bool s32_chains(const uzu_hip_model* m) {
+    const Stream32& S = *m->s32;
+    const uint32_t last = m->d.num_layers - 1;
+    const uzu_layer_desc& h = m->layers[last].d;
+    if (m->sampling.on || S.pair_table || m->d.hyper_streams || S.taps || h.no_mlp || h.has_ple || m->d.output_norm.kind != UZU_NORM_STATISTICS || m->output_norm.groups > 1) return false;
+    for (const Stream32::Layer& X : S.layers)
+        if (X.depth_weights) return false;
+    if (!m->layers[last].post_mlp.present || m->layers[last].post_mlp.groups > 1) return false;
+    const DLinear& head = m->d.tied_embeddings ? m->embedding : m->output_embedding;
+    k::NormAddParams n{};
+    n.y = S.tmp, n.residual = S.slots, n.out = S.xin, n.scales = m->layers[last].post_mlp.scales, n.layer_scale = S.layers[last].ls2, n.next = S.normed, n.next_scales = m->output_norm.scales, n.rows = 1;
+    n.d = m->d.model_dim;
+    return k::norm_linear_supported(n, lin(S, head, S.normed, S.logits, 1));
+}
+
 // `steps` chained decode steps of the bound sequence: the input token of a step is the one the step before left in the control block
 uzu_status s32_decode_enqueue(uzu_hip_model* m, uint32_t steps) {
     uzu_hip_state* st = m->bound;
@@ -1599,11 +1667,26 @@ uzu_status s32_decode_enqueue(uzu_hip_model* m, uint32_t steps) {
         if (m->graph_single) (void)hipGraphExecDestroy(m->graph_single);
         m->graph_single = nullptr, m->graph_epoch = m->sampling_epoch;
     }
+    // Greedy steps chain on the device: the read-out's launch leaves its parts' largest logits, one small launch chooses, moves the control block on and leaves the next step's embedding row
+    // and first norm.
+    const k::StepTurnParams first_row = s32_turn_params(m, st);
+    const bool chain = s32_chains(m) && k::step_turn_supported(first_row);
+    auto step = [&]() -> uzu_status {
+        if (!chain) {
+            UZU_PROPAGATE(s32_encode(m, one, st->d_tokens, 1, true));
+            return sample_commit(m, st, 0, 1, true, S.d_spans);
+        }
+        k::StepTurnParams turn = first_row;
+        UZU_PROPAGATE(s32_encode(m, one, st->d_tokens, 1, true, &turn.parts));
+        UZU_REQUIRE(turn.parts, "model_decode: the read-out left no choice");
+        UZU_PROPAGATE(k::step_turn(s, turn));
+        ++m->launches;
+        return UZU_OK;
+    };
     if (graph && !m->graph_single) { // one decode step of THIS state (its token / cache / control-block pointers) as a hipGraph
         HIPCHK(hipStreamSynchronize(s));
         HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        uzu_status r = s32_encode(m, one, st->d_tokens, 1);
-        if (r == UZU_OK) r = sample_commit(m, st, 0, 1, true, S.d_spans);
+        const uzu_status r = step();
         hipGraph_t g = nullptr;
         const hipError_t ce = hipStreamEndCapture(s, &g);
         if (r != UZU_OK || ce != hipSuccess) {
@@ -1614,13 +1697,10 @@ uzu_status s32_decode_enqueue(uzu_hip_model* m, uint32_t steps) {
         HIPCHK(hipGraphInstantiate(&m->graph_single, g, nullptr, nullptr, 0));
         HIPCHK(hipGraphDestroy(g));
     }
+    if (chain) UZU_PROPAGATE(k::step_turn(s, first_row));
     for (uint32_t i = 0; i < steps; ++i) {
-        if (graph) {
-            HIPCHK(hipGraphLaunch(m->graph_single, s));
-        } else {
-            UZU_PROPAGATE(s32_encode(m, one, st->d_tokens, 1));
-            UZU_PROPAGATE(sample_commit(m, st, 0, 1, true, S.d_spans));
-        }
+        if (graph) HIPCHK(hipGraphLaunch(m->graph_single, s));
+        else UZU_PROPAGATE(step());
         state_set_length(m, st, m->context_length + 1);
     }
     return UZU_OK;

@@ -1,7 +1,8 @@
 // k_step32.hip -- launches of an f32-stream design's decode step that do the work of several (kernels_stream32.h): a pass of a few rows is a chain of launches of 3 to 7 us whose bodies
 // are memory round trips, so what only one row's workgroup would do is done in front of (or by every workgroup of) the launch that reads it.
 // Us, width 1024, 2 of 8 experts of 1024: rms_norm_add_rows 3.1 + moe_route_groups 5.0 + moe_experts_gate_up 6.8 -> norm_route_gate_up 7.4 (256 workgroups that each read 36 KB of the
-// same numbers from the L2, 8 KB of experts' rows a wave); 8 rows of 2048: 4.3 + 7.0 -> norm_route_rows 5.5.
+// same numbers from the L2, 8 KB of experts' rows a wave); 8 rows of 2048: 4.3 + 7.0 -> norm_route_rows 5.5.  rms_norm_add_rows 3.1 + a projection onto 4112 columns 4.7 -> norm_linear 6.9;
+// ... + rms_norm_rows 2.8 + the read-out onto 32768 15.6 + argmax_pass1 4.7 -> 14.9; argmax_pass2 4.3 + commit 2.9 + embed_rows 3.8 + rms_norm_rows 2.8 -> step_turn 4.2.
 #include <algorithm>
 
 #include "device_utils.h"
@@ -17,6 +18,24 @@ constexpr uint32_t kStepThreads = 512, kStepWaves = kStepThreads / 64, kStepUnro
 constexpr uint32_t kStepMaxOutputs = 64, kStepMaxTop = 8;
 
 __device__ __forceinline__ float step_operand(float v, uint32_t bf16_products) { return bf16_products ? round_bf16(v) : v; }
+
+// the order of arg-max candidates (k_elementwise.hip): the larger value, of equal ones the lower index; a NaN never wins
+__device__ __forceinline__ void step_amax(float& bv, uint32_t& bi, float v, uint32_t i) {
+    if (v > bv || (v == bv && i < bi)) bv = v, bi = i;
+}
+// over the workgroup; the result in thread 0
+__device__ __forceinline__ void step_amax_block(float& bv, uint32_t& bi, float* s_v, uint32_t* s_i) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const float ov = __shfl_xor(bv, off, 64);
+        const uint32_t oi = __shfl_xor(bi, off, 64);
+        step_amax(bv, bi, ov, oi);
+    }
+    if ((threadIdx.x & 63) == 0) s_v[threadIdx.x >> 6] = bv, s_i[threadIdx.x >> 6] = bi;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (uint32_t w = 1; w < kStepWaves; ++w) step_amax(bv, bi, s_v[w], s_i[w]);
+}
 
 // A row's stream: new = residual + rms(y) * (scales + offset) * layer_scale, its norm for the sublayer that follows left in s_x (rounded if it enters bf16 products).  `write`: the
 // row and its norm go to memory as well.  Everything is loaded before the first sum is known.
@@ -178,7 +197,138 @@ __global__ void __launch_bounds__(kStepThreads) norm_route_gate_up_kernel(NormAd
     }
 }
 
+// One row: every workgroup norms it for itself, then a wave per output column and turn, the next column's weights on their way; J: pieces of 512 of a row.  AMAX: a workgroup's largest value
+// and its column as well (the read-out).
+template <int J, bool AMAX>
+__global__ void __launch_bounds__(kStepThreads) norm_linear_kernel(NormAddParams n, LinearF32Params p, float* part_value, uint32_t* part_index) {
+    extern __shared__ __attribute__((aligned(16))) float s_x[]; // [k]
+    __shared__ float s_red[16];
+    __shared__ uint32_t s_i[kStepWaves];
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = gridDim.x * kStepWaves, k = p.k;
+    u32x4_v w[J], next[J];
+    auto load = [&](uint32_t col, u32x4_v (&to)[J]) {
+        const uint16_t* row = p.w + (size_t)min(col, p.n - 1) * k;
+#pragma unroll
+        for (int j = 0; j < J; ++j) to[j] = *(const u32x4_v*)(row + min(j * 512 + lane * 8, k - 8)); // (pieces past the row's end meet zeros)
+    };
+    uint32_t col = blockIdx.x * kStepWaves + wave;
+    load(col, w);
+    step_norm_add(n, 0, s_x, s_red, p.bf16_products, blockIdx.x == 0);
+    __syncthreads();
+    float x[J][8];
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[j][e] = j * 512 + lane * 8 < k ? s_x[j * 512 + lane * 8 + e] : 0.0f;
+    float bv = -INFINITY;
+    uint32_t bi = 0xFFFFFFFFu;
+    for (; col < p.n; col += waves) {
+        load(col + waves, next);
+        float acc = 0.0f;
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                acc = fmaf(x[j][2 * i], bits_to_f32(w[j][i] << 16), acc);
+                acc = fmaf(x[j][2 * i + 1], bits_to_f32(w[j][i] & 0xFFFF0000u), acc);
+            }
+        acc = wave_sum(acc);
+        const float v = linear_epilogue(acc, p.bias ? bf16_to_f32(p.bias[col]) : 0.0f, p, 0, 0, col);
+        if (lane == 0) p.y[col] = v;
+        if (AMAX) step_amax(bv, bi, col == 0 && !(v == v) ? INFINITY : v, col); // (a NaN in front is never replaced)
+#pragma unroll
+        for (int j = 0; j < J; ++j) w[j] = next[j];
+    }
+    if (!AMAX) return;
+    step_amax_block(bv, bi, s_red, s_i);
+    if (threadIdx.x == 0) part_value[blockIdx.x] = bv, part_index[blockIdx.x] = bi;
+}
+
+// What stands between the read-out of a decode step and the first projection of the next one: the choice among the parts' largest logits, the sequence's control block moved on, the chosen token's
+// embedding row and its norm.
+__global__ void __launch_bounds__(kStepThreads) step_turn_kernel(StepTurnParams p) {
+    __shared__ float s_red[16];
+    __shared__ uint32_t s_i[kStepWaves + 1];
+    const uint32_t tid = threadIdx.x;
+    float sv[kStepUnroll][4];
+#pragma unroll
+    for (uint32_t u = 0; u < kStepUnroll; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sv[u][e] = (p.normed && (tid + u * kStepThreads) * 4 < p.d) ? p.scales[(tid + u * kStepThreads) * 4 + e] : 0.0f;
+    if (p.parts) {
+        const uint32_t len = *p.ctx_len;
+        float bv = -INFINITY;
+        uint32_t bi = 0xFFFFFFFFu;
+        for (uint32_t i = tid; i < p.parts; i += kStepThreads) step_amax(bv, bi, p.part_value[i], p.part_index[i]);
+        step_amax_block(bv, bi, s_red, s_i);
+        if (tid == 0) {
+            if (bi == 0xFFFFFFFFu) bi = 0;
+            s_i[kStepWaves] = bi;
+            *p.out_token = bi, p.sampled[len] = bi, p.tokens[0] = bi, *p.ctx_len = len + 1, p.span->start = len + 1;
+        }
+    } else if (tid == 0) s_i[kStepWaves] = p.tokens[0]; // (in front of the first step)
+    __syncthreads();
+    uint32_t t = s_i[kStepWaves];
+    if (t >= p.vocab) t = 0;
+    f32x4_v x[kStepUnroll];
+    float acc = 0.0f;
+#pragma unroll
+    for (uint32_t u = 0; u < kStepUnroll; ++u) {
+        const uint32_t i = (tid + u * kStepThreads) * 4;
+        x[u] = f32x4_v{0.0f, 0.0f, 0.0f, 0.0f};
+        if (i >= p.d) continue;
+        const u32x2_v b = *(const u32x2_v*)(p.table + (size_t)t * p.d + i);
+        x[u] = f32x4_v{bits_to_f32(b.x << 16), bits_to_f32(b.x & 0xFFFF0000u), bits_to_f32(b.y << 16), bits_to_f32(b.y & 0xFFFF0000u)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[u][e] *= p.scale, acc = fmaf(x[u][e], x[u][e], acc);
+        *(f32x4_v*)(p.out + i) = x[u];
+    }
+    if (!p.normed) return;
+    const float inv = 1.0f / sqrtf(block_sum(acc, s_red) / (float)p.d + p.eps);
+#pragma unroll
+    for (uint32_t u = 0; u < kStepUnroll; ++u) {
+        const uint32_t i = (tid + u * kStepThreads) * 4;
+        if (i >= p.d) continue;
+        f32x4_v o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = x[u][e] * inv * (sv[u][e] + p.offset);
+        *(f32x4_v*)(p.normed + i) = o;
+    }
+}
+
+// as many columns a wave as 512 workgroups need, and no more workgroups than those columns take (each reads the row and its weights for itself)
+uint32_t norm_linear_blocks(uint32_t n) {
+    const uint32_t each = (n + kStepWaves * kNormLinearParts - 1) / (kStepWaves * kNormLinearParts) * kStepWaves;
+    return (n + each - 1) / each;
+}
+
 } // namespace
+
+bool norm_linear_supported(const NormAddParams& n, const LinearF32Params& p) {
+    return n.rows == 1 && p.rows == 1 && p.batch == 1 && norm_add_step_supported(n) && n.out != n.residual && n.out != n.y && p.k == n.d && p.n && p.y && p.w && ((uintptr_t)p.w & 15) == 0 && !p.residual &&
+           !p.gate && !p.mul_table && !p.row_offsets && !p.row_map;
+}
+uzu_status norm_linear(hipStream_t s, const NormAddParams& n, const LinearF32Params& p, float* part_value, uint32_t* part_index, uint32_t* parts) {
+    UZU_REQUIRE(norm_linear_supported(n, p) && (!part_value) == (!part_index), "norm_linear: one row of %u (a multiple of 8, up to %u)", n.d, kStepMaxWidth);
+    const dim3 grid(norm_linear_blocks(p.n));
+    if (parts) *parts = grid.x;
+#define UZU_NL(J)                                                                                                                                                                \
+    return launch_check([&] {                                                                                                                                                    \
+        if (part_value) hipLaunchKernelGGL((norm_linear_kernel<J, true>), grid, dim3(kStepThreads), (size_t)n.d * 4, s, n, p, part_value, part_index);                           \
+        else hipLaunchKernelGGL((norm_linear_kernel<J, false>), grid, dim3(kStepThreads), (size_t)n.d * 4, s, n, p, part_value, part_index);                                     \
+    }, "norm_linear")
+    if (n.d <= 1024) UZU_NL(2);
+    if (n.d <= 2048) UZU_NL(4);
+    UZU_NL(8);
+#undef UZU_NL
+}
+bool step_turn_supported(const StepTurnParams& p) {
+    return p.d >= 8 && p.d % 8 == 0 && p.d <= kStepMaxWidth && p.table && p.out && p.tokens && (((uintptr_t)p.table | (uintptr_t)p.out | (uintptr_t)p.normed) & 15) == 0 && (!p.normed || p.scales);
+}
+uzu_status step_turn(hipStream_t s, const StepTurnParams& p) {
+    UZU_REQUIRE(step_turn_supported(p) && (!p.parts || (p.part_value && p.part_index && p.ctx_len && p.out_token && p.sampled && p.span)), "step_turn: rows of %u", p.d);
+    return launch_check([&] { hipLaunchKernelGGL(step_turn_kernel, dim3(1), dim3(kStepThreads), 0, s, p); }, "step_turn");
+}
 
 bool norm_add_step_supported(const NormAddParams& n) {
     return n.d >= 8 && n.d % 8 == 0 && n.d <= kStepMaxWidth && n.y && n.residual && n.out && n.scales && n.next && n.next_scales &&

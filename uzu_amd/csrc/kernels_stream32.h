@@ -194,6 +194,29 @@ uzu_status norm_route_rows(hipStream_t s, const NormAddParams& n, const RouteGro
 // ... and, one row, moe_experts_gate_up of the winners as well (weight_on_input: the winners' weights multiply their products).  n.out apart from n.residual and n.y.
 bool norm_route_gate_up_supported(const NormAddParams& n, const RouteGroupsParams& p, const uint16_t* w13, uint32_t ff, const ExpertAct& act);
 uzu_status norm_route_gate_up(hipStream_t s, const NormAddParams& n, const RouteGroupsParams& p, const uint16_t* w13, float* hidden, uint32_t ff, const ExpertAct& act, uint32_t weight_on_input);
+// ... and, one row, a linear of next (p.x is not read; no residual, gate or table); with part_value / part_index the largest result of each of up to kNormLinearParts workgroups and its
+// column, *parts of them.  n.out apart from n.residual and n.y.
+constexpr uint32_t kNormLinearParts = 512;
+bool norm_linear_supported(const NormAddParams& n, const LinearF32Params& p);
+uzu_status norm_linear(hipStream_t s, const NormAddParams& n, const LinearF32Params& p, float* part_value = nullptr, uint32_t* part_index = nullptr, uint32_t* parts = nullptr);
+// Between two decode steps of one sequence: the greedy choice among such parts (of equal values the lowest index), *out_token, sampled[*ctx_len], tokens[0], *ctx_len + 1 and the span behind it;
+// then out = scale * the token's embedding row and, with `normed`, its RMS norm * (scales + offset).  parts 0: only the latter two, for tokens[0].
+struct StepTurnParams {
+    const float* part_value;
+    const uint32_t* part_index;
+    uint32_t parts;
+    uint32_t *ctx_len, *tokens, *out_token, *sampled;
+    SeqSpan* span;
+    const uint16_t* table;
+    uint32_t vocab, d;
+    float scale;
+    float* out;
+    float* normed;
+    const float* scales;
+    float offset, eps;
+};
+bool step_turn_supported(const StepTurnParams& p);
+uzu_status step_turn(hipStream_t s, const StepTurnParams& p);
 // hidden[r * top + j, f] = act(gate_e x_r, up_e x_r) for e = ids[r, j] < routed; w13 bf16 [routed][2 ff][d], rows [0, ff) of an expert = up, [ff, 2 ff) = gate
 // in_weights (f32 [rows, top] or null): the expert reads in_weights[r, j] * x_r instead (both products are multiplied by it in front of the activation)
 uzu_status moe_experts_gate_up(hipStream_t s, const float* x, const int32_t* ids, const uint16_t* w13, float* hidden, uint32_t rows, uint32_t d, uint32_t ff, uint32_t routed,
