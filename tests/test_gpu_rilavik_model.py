@@ -703,6 +703,24 @@ def test_decode_graph_replays_equal_plain_launches(hip_ctx, tmp_path, full):
         m.close()
 
 
+@pytest.mark.parametrize("name", ["a", "b"])
+@pytest.mark.parametrize("held", [1, 7, 33])
+def test_a_copy_into_a_state_that_held_a_longer_sequence(models, name, held):
+    """What a copy brings of a cache ends with the source's context: behind it the state still holds its own longer sequence, which nothing may read."""
+    cfg, W, ms = models[name]
+    m = ms[True]
+    toks, longer = prompt(cfg, held + 9, 16), prompt(cfg, 90, 17)
+    a, b = m.new_state(), m.new_state()
+    m.step_batch([b], [longer], [[]])
+    m.step_batch([a], [toks[:held]], [[]])
+    b.copy_from(a)
+    assert b.context_length == held
+    rows = [m.step_batch([b], [[t]], [[0]])[0][0] for t in toks[held:held + 3]]
+    rows += list(m.step_batch([b], [toks[held + 3:]], [list(range(6))])[0])
+    assert O.logit_error(np.stack(rows), O.forward(cfg, W, toks)[0][held:]).max() < TOL[True]
+    a.close(), b.close()
+
+
 def test_copied_states_go_their_own_ways(models):
     cfg, W, ms = models["a"]
     m = ms[True]

@@ -1518,12 +1518,12 @@ uzu_status s32_state_layer(uzu_hip_model* m, uzu_hip_state* st, uint32_t l) {
         st->layers[l].conv_state = (float*)p;
     } else if (!h.is_kv_sharing) { // rows are written before they are read (the append precedes the core in every pass)
         if (h.mixer_kind == UZU_MIXER_ATTENTION) {
-            UZU_PROPAGATE(state_alloc(st, (size_t)m->max_positions * h.num_groups * h.head_dim * elem, &p, false));
+            UZU_PROPAGATE(state_alloc(st, (size_t)m->max_positions * h.num_groups * h.head_dim * elem, &p, false, h.num_groups * h.head_dim * elem));
             st->layers[l].cache_k = p;
-            UZU_PROPAGATE(state_alloc(st, (size_t)m->max_positions * h.num_groups * h.value_head_dim * elem, &p, false));
+            UZU_PROPAGATE(state_alloc(st, (size_t)m->max_positions * h.num_groups * h.value_head_dim * elem, &p, false, h.num_groups * h.value_head_dim * elem));
             st->layers[l].cache_v = p;
         } else {
-            UZU_PROPAGATE(state_alloc(st, (size_t)m->max_positions * (h.latent_rank + h.latent_rope_dim) * elem, &p, false));
+            UZU_PROPAGATE(state_alloc(st, (size_t)m->max_positions * (h.latent_rank + h.latent_rope_dim) * elem, &p, false, (h.latent_rank + h.latent_rope_dim) * elem));
             st->layers[l].latent = p;
         }
     }

@@ -137,6 +137,7 @@ struct uzu_hip_state {
     uint32_t graph_epoch = 0; // sampling_epoch of the model when the graphs were captured (they bake the sampling kernels in)
     std::vector<void*> allocations;
     std::vector<size_t> allocation_bytes; // parallel to `allocations` (uzu_hip_state_copy)
+    std::vector<size_t> allocation_row_bytes; // ... of a position, where the rows behind the context are undefined; 0: the whole block counts
     size_t bytes = 0;
 };
 
@@ -325,7 +326,7 @@ struct CopyBlock {
 uzu_status copy_blocks(hipStream_t s, const std::vector<CopyBlock>& all);
 uzu_status dev_alloc(uzu_hip_model* m, size_t bytes, void** out, bool zero = false);
 void dev_free(uzu_hip_model* m, void* p);
-uzu_status state_alloc(uzu_hip_state* st, size_t bytes, void** out, bool zero_by_contract = true);
+uzu_status state_alloc(uzu_hip_state* st, size_t bytes, void** out, bool zero_by_contract = true, size_t row_bytes = 0);
 void state_release(uzu_hip_state* st);
 void state_free(uzu_hip_state* st);
 uzu_status state_build(uzu_hip_model* m, uzu_hip_state** out);
