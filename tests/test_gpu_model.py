@@ -315,6 +315,28 @@ def test_fused_decode_matches_unfused(hip_ctx):
                 assert logits_close(a, b).all()
 
 
+@pytest.mark.parametrize("hidden,vocab,attention", [(4096, 4099, False), (6144, 4099, True), (4096, 65601, False)])
+def test_large_int8_matrices_of_a_decode_step_match_unfused(hip_ctx, hidden, vocab, attention):
+    """Matrices from 8 MB on go through the weight stream (k_decode_large.hip): gated rows behind the Normalization, plain rows of two and three steps, a read-out with its arg-max whose rows do not
+    divide by the waves (and one long enough for three items a wave), qkv beside a gate.  Its arithmetic is the one-kernel-per-reference-kernel path's: bit-identical logits without attention."""
+    kinds = [D.MIXER_DELTA_NET, D.MIXER_ATTENTION] if attention else [D.MIXER_DELTA_NET]
+    extra = dict(num_heads=16, num_groups=4, head_dim=128) if attention else {}
+    bundle = S.build_model(S.tiny_qwen(model_dim=2048, hidden_dim=hidden, vocab_size=vocab, bits=8, layer_kinds=kinds, group_size=128, **extra))
+    prompt = S.synthetic_prompt(21, vocab)
+    outs = []
+    for flags in (0, MODEL_NO_FUSION):
+        hm = HipModel(hip_ctx, bundle, flags)
+        toks, logits = [hm.prefill(prompt)], []
+        for _ in range(4):
+            toks.append(int(hm.decode(1)[0][0]))
+            logits.append(hm.read_logits())
+        outs.append((toks, logits))
+        hm.close()
+    assert outs[0][0] == outs[1][0]
+    for a, b in zip(outs[0][1], outs[1][1]):
+        assert logits_close(a, b).all() if attention else np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("preset,kw,exact", [
     ("tiny-qwen", {"rht": True, "model_dim": 1024, "layer_kinds": [D.MIXER_DELTA_NET] * 3}, True),   # DeltaNet only: every kernel of the two paths rounds at the same points
     ("tiny-qwen", {"rht": True, "model_dim": 1024}, False),                                      # + a gated attention layer (gate behind its OWN input transform: a launch of its own)

@@ -1156,6 +1156,7 @@ uzu_status gemv_dec(hipStream_t s, const DecGemvParams& p_in, int num_cus, uint3
         const uzu_status st = gemv_stream(s, p_in, num_cus, grid_out);
         if (st != UZU_ERR_UNSUPPORTED) return st;
     }
+    if (gemv_large_wanted(p)) return gemv_large(s, p, num_cus, grid_out); // (k_decode_large.hip)
     int lpr_log2, R;
     bool wide = false;
     const uint32_t want = gemv_dec_plan(p, num_cus, &lpr_log2, &R, &wide);
@@ -1167,7 +1168,7 @@ uzu_status gemv_dec(hipStream_t s, const DecGemvParams& p_in, int num_cus, uint3
     return launch_gemv_dec_cpl<8, false>(s, p, want, lpr_log2, R, num_cus, grid_out, wide);
 }
 
-// The launch plan gemv_dec takes for a shape, without launching (host arithmetic only: callable without a GPU).  `wide_waves` is the
+// The launch plan of gemv_dec's own kernels for a shape, without launching (host arithmetic only: callable without a GPU); large int8 matrices go to k_decode_large.hip instead.  `wide_waves` is the
 // launcher's workgroup width (launch_gemv_dec_c: 16 waves, 12 on the 4-step register path, 4 otherwise); `wg_batches` / `workgroups`
 // are the spread of a partial round (0 / 0 when the grid is the persistent one, whose size depends on the instance's occupancy).
 void gemv_dec_plan_query(const DecGemvParams& p, int num_cus, DecGemvPlan* out) {
