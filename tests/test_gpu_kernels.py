@@ -17,7 +17,7 @@ import os
 import numpy as np
 import pytest
 
-from helpers import MASK_VARIANTS, bf16, dequantize, f32, mask_case, quant_matrix, ref_attention_inputs, trie_from_parents, ulp_diff_bf16
+from helpers import MASK_VARIANTS, attention_float64, bf16, dequantize, f32, mask_case, quant_matrix, ref_attention_inputs, trie_from_parents, ulp_diff_bf16
 from oracle import oracle as O
 from uzu_amd import _ffi
 from uzu_amd import backend as B
@@ -966,6 +966,33 @@ def test_attention_trie_mask(hip_ctx, tree, window, heads, kv_heads, hd, prefix)
     finally:
         set_exact(0)
     assert np.array_equal(bo.download(np.uint16, want.size).reshape(want.shape), want)
+
+
+@pytest.mark.parametrize("n,heads,kv_heads,hd,prefix", [(1, 4, 4, 64, 0), (2, 8, 2, 128, 1), (13, 8, 2, 256, 1023), (16, 16, 4, 64, 31), (17, 14, 2, 64, 96), (31, 6, 3, 256, 32), (32, 8, 1, 128, 2100)])
+def test_attention_of_a_tree_on_the_matrix_cores(hip_ctx, n, heads, kv_heads, hd, prefix):
+    """The tree form (k_tree_attention.hip) at its edges against float64: a column tile that is full, one over and nearly empty, groups of columns (heads a kv head x nodes
+    past 64), a first tile of keys that is the tree's own, shares with none, one and several tiles, rows behind the last key that hold NaN.
+    The bound: the bf16 rounding of the result, and the f32 sums of the scores (hd terms) and of the rows (a key a term), carried to the result by at most max |v|."""
+    rng = np.random.default_rng(n * hd + prefix)
+    parents, path = [-1], [0]
+    for i in range(1, n):  # depth-first: deeper, or back up a few nodes first
+        while len(path) > 1 and rng.random() < 0.45:
+            path.pop()
+        parents.append(path[-1])
+        path.append(i)
+    seq = prefix + n
+    trie = trie_from_parents(parents)
+    q, k, v, _ = attention_case(rng, heads, kv_heads, hd, seq, n, seq + 40)
+    k[seq:], v[seq:] = 0x7FC0, 0x7FC0
+    scale = 1.0 / np.sqrt(hd)
+    want = attention_float64(q, k, v, heads, kv_heads, hd, seq, n, hd, kv_heads * hd, scale, 1, None, None, None, parents)
+    bq, bk, bv, bt, bo = hip_ctx.buffer_from(q), hip_ctx.buffer_from(k), hip_ctx.buffer_from(v), hip_ctx.buffer_from(trie), hip_ctx.create_buffer(n * heads * hd * 2)
+    kern = B.AttentionSinglePassKernel.new(hip_ctx, B.BF16, hd, 0, 0, 1, 1, 0)
+    run(hip_ctx, lambda cb: kern.encode(bq, bk, bv, bo, heads // kv_heads, seq, hd, kv_heads * hd, hd, kv_heads * hd, None, scale, bt, None, None, heads, n, cb))
+    got = f32(bo.download(np.uint16, n * heads * hd)).reshape(n, heads, hd).astype(np.float64)
+    score = scale * np.abs(f32(q)).sum(-1).max() * np.abs(f32(k[:seq])).max()
+    bound = 2.0 ** -8 * np.abs(want) + 2.0 ** -24 * (hd * score / np.sqrt(hd) + seq ** 0.5) * np.abs(f32(v[:seq])).max()
+    assert np.isfinite(got).all() and (np.abs(got - want) <= bound).all(), np.max(np.abs(got - want) - bound)
 
 
 def test_trie_verify_then_compaction_equals_linear_decode(hip_ctx):

@@ -16,6 +16,7 @@
 #include <algorithm>
 
 #include "engine_types.h"
+#include "tree_pass.h"
 #include "uzu_math.h"
 
 using namespace uzu;
@@ -399,15 +400,16 @@ uzu_status uzu_hip_model_verify_tree_seeded(uzu_hip_model* m, const uint32_t* to
     m->tree.host_seeds = seeds != nullptr && m->sampling.on;
     if (m->tree.host_seeds) HIPCHK(hipMemcpyAsync(m->tree.d_seeds, seeds, (size_t)tree_size * 8, hipMemcpyHostToDevice, s));
     {
-        uint32_t max_heads = 0, max_hd = 0;
-        bool two_pass = false;
+        // the largest of the layers' partial results, at any context: of the tree form (columns of all shares), or of the two-pass form behind 1024 keys (32 blocks a row)
+        size_t rows = 0;
+        uint32_t max_hd = 0;
         for (auto& L : m->layers)
             if (L.d.mixer_kind == UZU_MIXER_ATTENTION) {
-                max_heads = max_heads > L.d.num_heads ? max_heads : L.d.num_heads;
+                const size_t columns = L.d.num_groups ? k::attention_tree_columns(L.d.num_heads, L.d.num_heads / L.d.num_groups, tree_size) : 0;
+                rows = std::max({rows, (size_t)tree_size * L.d.num_heads, (columns + 31) / 32});
                 max_hd = max_hd > L.d.head_dim ? max_hd : L.d.head_dim;
-                two_pass = two_pass || m->context_length + tree_size > 1024;
             }
-        if (max_heads && two_pass) UZU_PROPAGATE(ensure_partials(m, tree_size * max_heads, max_hd));
+        if (rows) UZU_PROPAGATE(ensure_partials(m, (uint32_t)rows, max_hd));
     }
     const bool two_pass_regime = m->context_length + tree_size > 1024;
     HIPCHK(hipEventRecord(m->ev0, s));
