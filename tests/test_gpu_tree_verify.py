@@ -9,7 +9,7 @@ import pytest
 from helpers import bf16, f32, ulp_diff_bf16
 from oracle import oracle as O
 from test_gpu_kernels import run
-from test_oracle_tree_verify import linear_stream, logit_error_sigma, random_tree
+from test_oracle_tree_verify import linear_stream, logit_error_sigma, path_of, random_tree
 from uzu_amd import _ffi
 from uzu_amd import backend as B
 from uzu_amd import synthetic as S
@@ -265,6 +265,38 @@ def test_engine_verify_and_accept_on_ring_kv_states(hip_ctx):
         assert int(t) == tok
     hm.close()
     om.close()
+
+
+@pytest.mark.parametrize("n,groups,kernel", [(1, 2, 4), (2, 4, 3), (13, 1, 4), (16, 4, 2), (17, 2, 4), (31, 4, 4), (32, 2, 3)])
+def test_engine_tree_passes_of_every_size_are_bit_identical_in_reference_order_mode(hip_ctx, n, groups, kernel):
+    """The DeltaNet layers' pass over a tree in one launch (dn_tree_step): tree sizes around a block of 16 nodes, the smallest and the largest, key heads of one, two and four value
+    heads (who files the keys), two to four taps; every node's logits, and after an accepted path (keys, values, decays and conv states that the launch filed) a decode step's."""
+    rng = np.random.default_rng(n)
+    cfg = S.tiny_qwen(dn_num_groups=groups, dn_kernel_size=kernel)
+    bundle = S.build_model(cfg)
+    prompt = ((S.synthetic_prompt(37, cfg.vocab_size).astype(np.int64) * 81 + 891) % cfg.vocab_size).astype(np.uint32)
+    nodes, parents = random_tree(n, rng)
+    om = O.OracleModel(bundle)
+    _set_exact(True)
+    try:
+        hm = HipModel(hip_ctx, bundle)
+        tok = om.prefill(prompt)
+        assert hm.prefill(prompt) == tok
+        tokens = np.concatenate([[tok], rng.integers(0, cfg.vocab_size, n - 1)]).astype(np.uint32)
+        o_sampled, o_logits = om.verify_tree(tokens, nodes, True)
+        h_sampled = hm.verify_tree(tokens, nodes)
+        h_logits = hm.read_tree_logits()
+        assert np.array_equal(h_logits, o_logits), f"{(h_logits != o_logits).sum()} of {o_logits.size} tree logits differ"
+        path = path_of(parents, n - 1)
+        om.accept(path)
+        hm.accept(path)
+        _, lg = om.forward([int(o_sampled[path[-1]])], True)
+        hm.decode(1)
+        assert np.array_equal(hm.read_logits(), lg)
+        hm.close()
+    finally:
+        _set_exact(False)
+        om.close()
 
 
 def test_engine_tree_pass_with_stochastic_sampling_uses_each_nodes_own_seed(hip_ctx):

@@ -419,7 +419,7 @@ void attention_core(Enc& e, DLayer& L, uint32_t batch, size_t row0, bool fuse_no
 
 void delta_net_core(Enc& e, DLayer& L, uint32_t batch, size_t row0, uint32_t file_rows = 0);
 
-// DeltaNet::encode_tree_verify (delta_net.rs:334-437): conv tree scan + tree prep (one launch), the tree-verify composite, norm-gate;
+// DeltaNet::encode_tree_verify (delta_net.rs:334-437): conv tree scan, tree prep and the tree-verify composite (one launch, or prep and composite), norm-gate;
 // the layer's DeltaNetSuffixStatus::Tree stays in m->tree.layers[layer] for uzu_hip_model_accept
 void delta_net_tree_core(Enc& e, DLayer& L, uint32_t layer, uint32_t n) {
     uzu_hip_model* m = e.m;
@@ -427,9 +427,14 @@ void delta_net_tree_core(Enc& e, DLayer& L, uint32_t layer, uint32_t n) {
     const uint32_t key_dim = Hk * Dk, value_dim = Hv * Dv, conv_dim = 2 * key_dim + value_dim;
     const uint32_t total_proj_dim = conv_dim + value_dim + 2 * Hv, ks = L.d.dn_kernel_size;
     uzu_hip_model::TreeLayer& T = m->tree.layers[layer];
-    RUN("dn_tree_prep", 0, k::delta_net_tree_prep(e.s, m->in_proj, L.conv_w, L.conv_b, L.conv_state, m->tree.d_parents, nullptr, T.conv_states, L.a_log, L.dt_bias, m->tree.q,
-                                                   T.k, T.v, T.beta, T.log_decay, n, ks, Hk, Hv, Dk, Dv, true, true));
-    RUN("dn_tree_verify", (size_t)Hv * Dv * Dk * 4, k::delta_net_tree_verify(e.s, m->tree.q, T.k, T.v, m->tree.d_trie, T.log_decay, T.beta, L.ssm_state, m->delta_out, n, Hk, Hv, Dk, Dv));
+    if (k::delta_net_tree_step_supported(m->in_proj, L.ssm_state, n, ks, Hk, Hv, Dk, Dv)) {
+        RUN("dn_tree_step", (size_t)Hv * Dv * Dk * 4, k::delta_net_tree_step(e.s, m->in_proj, L.conv_w, L.conv_b, L.conv_state, m->tree.d_parents, m->tree.d_trie, L.a_log, L.dt_bias, L.ssm_state,
+                                                                           T.conv_states, T.k, T.v, T.beta, T.log_decay, m->delta_out, n, ks, Hk, Hv));
+    } else {
+        RUN("dn_tree_prep", 0, k::delta_net_tree_prep(e.s, m->in_proj, L.conv_w, L.conv_b, L.conv_state, m->tree.d_parents, nullptr, T.conv_states, L.a_log, L.dt_bias, m->tree.q,
+                                                       T.k, T.v, T.beta, T.log_decay, n, ks, Hk, Hv, Dk, Dv, true, true));
+        RUN("dn_tree_verify", (size_t)Hv * Dv * Dk * 4, k::delta_net_tree_verify(e.s, m->tree.q, T.k, T.v, m->tree.d_trie, T.log_decay, T.beta, L.ssm_state, m->delta_out, n, Hk, Hv, Dk, Dv));
+    }
     // the norm-gate reads z from the rows' pass-through section: ConvTreeScan copies those channels unchanged, so the in-proj rows serve
     RUN("delta_net_norm_gate", 0, k::delta_net_norm_gate(e.s, m->delta_out, m->in_proj, L.dn_norm, Hv, Dv, value_dim, conv_dim, total_proj_dim, L.d.dn_norm_epsilon, n));
 }

@@ -15,7 +15,7 @@
 // sequential delta-rule steps in reference order would be one thread per row (~100 us); the production form gives a row to a half-wave
 // (tolerance-class like the decode update), the reference-order form exists for uzu_hip_set_exact(1).
 #include "device_utils.h"
-#include "kernels.h"
+#include "tree_pass.h"
 
 namespace uzu {
 namespace k {
@@ -250,6 +250,259 @@ __global__ void __launch_bounds__(256) dn_tree_solve_kernel(const uint16_t* __re
     }
 }
 
+// ------------------------------------------------------------------------------------------------ the pass in one launch
+// Conv scan, preparation, prefix, Gram, solve and out of a verify pass: dn_tree_prep_kernel and dn_tree_solve_kernel in one launch, every value by the same operations in the
+// same order, so bit-identical to the two (and to the CPU kernels).  What they cost was trips to memory and idle lanes, not work: the preparation walked the parents by
+// dependent loads, its rows went out and came back, and 256 threads took the 128-long sums of one after the other (20.5 us a layer at 13 nodes, now 11.4).
+// One workgroup = (value head hv, 16 value columns), 1024 threads, all n nodes.  It convolves its head's q and k channels for itself, eight workgroups of a head the same:
+// 13 x 256 channels are 2.8 us of a compute unit, the launch and the trips that they replace 6.8.  Tile t of a head files the nodes t, t + 8, ... for the acceptance that follows.
+constexpr uint32_t kTreeStepMaxKernel = 4; // taps: the history of a channel in registers, a node's source rows in a byte each
+struct alignas(16) TreeStepLds {
+    float q[kDnTreeMaxNodes][kPad];
+    float k[kDnTreeMaxNodes][kPad];
+    float h0[16][kPad];
+    uint16_t x[kDnTreeMaxNodes][272]; // the rows' q, k and the tile's v channels in front of the convolution
+    float a[kDnTreeMaxNodes][kDnTreeMaxNodes + 4]; // (rows of 16 bytes' multiples)
+    float qkd[kDnTreeMaxNodes][kDnTreeMaxNodes + 4];
+    float a_inv[kDnTreeMaxNodes / kBlock][kBlock][kBlock + 4];
+    float v[kDnTreeMaxNodes][17], kh0[kDnTreeMaxNodes][17], qh0[kDnTreeMaxNodes][17], u[kDnTreeMaxNodes][17];
+    float acc[kBlock][17];
+    float prefix[kDnTreeMaxNodes], e_prefix[kDnTreeMaxNodes], beta[kDnTreeMaxNodes], inv[2][kDnTreeMaxNodes];
+    uint64_t exp_tab[32];
+    uint32_t rows[kDnTreeMaxNodes]; // a node's source rows, newest tap first, a signed byte each: a node, or -1, -2, -3 into the sequence's history
+    uint32_t t_start[kDnTreeMaxNodes], t_end[kDnTreeMaxNodes];
+};
+template <uint32_t KS>
+__global__ void __launch_bounds__(1024) dn_tree_step_kernel(const uint16_t* __restrict__ in_proj, const float* __restrict__ conv_w, const float* __restrict__ conv_b,
+                                                            const float* __restrict__ base_state, const int32_t* __restrict__ parents, const uint32_t* __restrict__ trie,
+                                                            const float* __restrict__ a_log, const float* __restrict__ dt_bias, const float* __restrict__ h0,
+                                                            float* __restrict__ suffix_state, uint16_t* __restrict__ k_out, uint16_t* __restrict__ v_out,
+                                                            float* __restrict__ beta_out, float* __restrict__ log_decay_out, uint16_t* __restrict__ o, uint32_t n, uint32_t Hk,
+                                                            uint32_t Hv) {
+    constexpr uint32_t D = 128, T = 1024, tiles = D / 16, history = KS - 1, kGroups = 3;
+    __shared__ TreeStepLds L;
+    const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, hv = blockIdx.x / tiles, t = blockIdx.x % tiles, c0 = t * 16, hk = hv / (Hv / Hk);
+    const uint32_t key_dim = Hk * D, value_dim = Hv * D, conv_dim = 2 * key_dim + value_dim, total = conv_dim + value_dim + 2 * Hv;
+    const bool files_k = hv % (Hv / Hk) == 0; // (value heads that share a key head: the first of them files it)
+    // ---- every operand is requested before the first is used
+    // rows: 16 bytes a thread, 16 pieces of q and 16 of k a node, and two of v
+    const uint32_t x_node = min(tid / 32, n - 1), x_piece = tid % 32, xv_node = min(tid / 2, n - 1);
+    const u32x4_v x = *(const u32x4_v*)(in_proj + (size_t)x_node * total + (x_piece < 16 ? 0 : key_dim) + hk * D + x_piece % 16 * 8);
+    u32x4_v xv = {0u, 0u, 0u, 0u};
+    if (wave == 0) xv = *(const u32x4_v*)(in_proj + (size_t)xv_node * total + 2 * key_dim + hv * D + c0 + tid % 2 * 8);
+    f32x4_v state = {0.f, 0.f, 0.f, 0.f};
+    if (wave < 8) state = *(const f32x4_v*)(h0 + ((size_t)hv * D + c0) * D + tid * 4);
+    // the convolution's roles: waves 0 .. 11 a q or k channel a thread, three groups of nodes; 12 .. 14 a value channel, twelve nodes at a time; the last one the nodes' scalars
+    const uint32_t c = tid % 256, channel = wave < 12 ? (c < D ? 0 : key_dim) + hk * D + c % D : 2 * key_dim + hv * D + c0 + tid % 16;
+    float w[KS], past[history];
+#pragma unroll
+    for (uint32_t i = 0; i < KS; ++i) w[i] = conv_w[(size_t)channel * KS + i];
+#pragma unroll
+    for (uint32_t i = 0; i < history; ++i) past[i] = base_state[(size_t)channel * history + i];
+    const float bias = conv_b ? conv_b[channel] : 0.0f;
+    float beta_raw = 0.f, a_raw = 0.f, bias_dt = 0.f, log_a = 0.f;
+    uint32_t start = 1, end = 0;
+    if (wave == 15 && lane < n) {
+        beta_raw = bf16_to_f32(in_proj[(size_t)lane * total + conv_dim + value_dim + hv]);
+        a_raw = bf16_to_f32(in_proj[(size_t)lane * total + conv_dim + value_dim + Hv + hv]);
+        bias_dt = dt_bias[hv], log_a = a_log[hv];
+        start = trie[3 * lane], end = trie[3 * lane + 1];
+        L.t_start[lane] = start, L.t_end[lane] = end;
+    }
+    if (wave == 14 && lane < n) { // conv_scan.rs:43-65: the node, its ancestors, then the history backwards
+        int32_t row = (int32_t)lane;
+        uint32_t packed = 0;
+#pragma unroll
+        for (uint32_t h = 0; h < KS; ++h) {
+            packed |= ((uint32_t)row & 255u) << (8 * h);
+            if (h + 1 < KS) row = row >= 0 ? parents[row] : row - 1;
+        }
+        L.rows[lane] = packed;
+    }
+    if (tid < 32) L.exp_tab[tid] = kExp2fTab[tid];
+    for (uint32_t i = tid; i < kDnTreeMaxNodes * (kDnTreeMaxNodes + 4); i += T) (&L.a[0][0])[i] = 0.0f, (&L.qkd[0][0])[i] = 0.0f;
+    if (tid / 32 < n) *(u32x4_v*)&L.x[tid / 32][x_piece * 8] = x;
+    if (tid < 2 * n) *(u32x4_v*)&L.x[tid / 2][256 + tid % 2 * 8] = xv;
+    if (wave < 8) *(f32x4_v*)&L.h0[tid / 32][tid % 32 * 4] = state;
+    __syncthreads();
+    auto convolve = [&](uint32_t node, uint32_t packed, uint32_t at, bool files) { // taps newest first
+        float acc = bias;
+#pragma unroll
+        for (uint32_t h = 0; h < KS; ++h) {
+            const int32_t row = (int32_t)(packed << (24 - 8 * h)) >> 24;
+            float sample = bf16_to_f32(L.x[max(row, 0)][at]);
+#pragma unroll
+            for (uint32_t i = 0; i < history; ++i) sample = row == (int32_t)i - (int32_t)history ? past[i] : sample;
+            acc += sample * w[KS - 1 - h];
+            if (files && h < history) suffix_state[((size_t)node * conv_dim + channel) * history + (history - 1 - h)] = sample;
+        }
+        return f32_to_bf16(silu_f32_tab(acc, L.exp_tab));
+    };
+    if (wave < 4 * kGroups) {
+        for (uint32_t node = wave / 4; node < n; node += kGroups) {
+            const float xb = bf16_to_f32(convolve(node, __builtin_amdgcn_readfirstlane(L.rows[node]), c, files_k && node % tiles == t));
+            if (c < D) L.q[node][c] = xb;
+            else L.k[node][c - D] = xb;
+        }
+    } else if (wave < 15) {
+        for (uint32_t node = (tid - 256 * kGroups) / 16; node < n; node += 12) {
+            const uint16_t bits = convolve(node, L.rows[node], 256 + tid % 16, true);
+            L.v[node][tid % 16] = bf16_to_f32(bits);
+            v_out[(size_t)node * value_dim + hv * D + c0 + tid % 16] = bits;
+        }
+    } else {
+        const float beta = 1.0f / (1.0f + expf_glibc_tab(-beta_raw, L.exp_tab));
+        const float sp_in = a_raw + bias_dt;
+        const float sp = sp_in > 20.0f ? sp_in : logf_glibc(1.0f + expf_glibc_tab(sp_in, L.exp_tab));
+        const float decay = -expf_glibc_tab(log_a, L.exp_tab) * sp;
+        float sum = 0.0f; // prefix.rs:20-36: log decays of the ancestors-or-self, in column order
+        for (uint32_t col = 0; col < n; ++col) {
+            const uint32_t first = __builtin_amdgcn_readlane(start, col), last = __builtin_amdgcn_readlane(end, col);
+            const float with = sum + bits_to_f32(__builtin_amdgcn_readlane(f32_to_bits(decay), col));
+            sum = lane >= first && lane <= last ? with : sum;
+        }
+        if (lane < n) {
+            L.beta[lane] = beta, L.prefix[lane] = sum, L.e_prefix[lane] = expf_glibc_tab(sum, L.exp_tab);
+            if (t == 0) beta_out[(size_t)lane * Hv + hv] = beta, log_decay_out[(size_t)lane * Hv + hv] = decay;
+        }
+    }
+    __syncthreads();
+    // a sum of 128 products in their order: the reads of the next 16 are on their way while the adders work (waited for two by two: 4400 cycles a round of sums, now 3200)
+    auto dot = [&](const float* left, const float* right) {
+        f32x4_v l[2][4], r[2][4];
+        float sum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) l[0][i] = *(const f32x4_v*)(left + 4 * i), r[0][i] = *(const f32x4_v*)(right + 4 * i);
+#pragma unroll
+        for (uint32_t d = 0; d < D; d += 16) {
+            const int now = d / 16 % 2;
+            if (d + 16 < D) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) l[now ^ 1][i] = *(const f32x4_v*)(left + d + 16 + 4 * i), r[now ^ 1][i] = *(const f32x4_v*)(right + d + 16 + 4 * i);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum += l[now][i][e] * r[now][i][e];
+            asm volatile("" : "+v"(sum)); // (here, not behind all the reads)
+        }
+        return sum;
+    };
+    if (tid < 2 * n) { // the reference's sums of squares: sequential from 0 (prefill_prep.rs:57-62, 72-77)
+        const float* row = tid < n ? L.q[tid] : L.k[tid - n];
+        L.inv[tid < n ? 0 : 1][tid < n ? tid : tid - n] = 1.0f / sqrtf(dot(row, row) + 1e-6f);
+    }
+    __syncthreads();
+    for (uint32_t node = tid / 256; node < n; node += T / 256) {
+        if (c < D) {
+            const float q_scale = 1.0f / sqrtf((float)D);
+            L.q[node][c] = bf16_to_f32(f32_to_bf16(L.q[node][c] * L.inv[0][node] * q_scale));
+        } else {
+            const uint16_t bits = f32_to_bf16(L.k[node][c - D] * L.inv[1][node]);
+            L.k[node][c - D] = bf16_to_f32(bits);
+            if (files_k && node % tiles == t) k_out[(size_t)node * key_dim + hk * D + c - D] = bits;
+        }
+    }
+    __syncthreads();
+    // ---- the 128-long sums, one a thread: q . k and k . k of the pairs row >= col (tree_gram.rs:44-96; an ancestor comes first), k . h0 and q . h0 (tree_gram.rs:139-158,
+    // out.rs:62-73)
+    const uint32_t pairs = n * (n + 1) / 2;
+    for (uint32_t i = tid; i < 2 * pairs + 32 * n; i += T) {
+        uint32_t row, col;
+        const float *left, *right;
+        const bool pair = i < 2 * pairs;
+        const uint32_t which = pair ? (i < pairs ? 0u : 1u) : (i - 2 * pairs < 16 * n ? 0u : 1u); // 0: q with k, k with h0; 1: k with k, q with h0
+        if (pair) {
+            const uint32_t p = which ? i - pairs : i;
+            row = (uint32_t)((sqrtf((float)(8 * p + 1)) - 1.0f) * 0.5f);
+            if (row * (row + 1) / 2 > p) --row;
+            else if ((row + 1) * (row + 2) / 2 <= p) ++row;
+            col = p - row * (row + 1) / 2;
+            left = which ? L.k[row] : L.q[row], right = L.k[col];
+        } else {
+            const uint32_t p = i - 2 * pairs - which * 16 * n;
+            row = p / 16, col = p % 16;
+            left = which ? L.q[row] : L.k[row], right = L.h0[col];
+        }
+        const float sum = dot(left, right);
+        if (!pair) {
+            (which ? L.qh0 : L.kh0)[row][col] = sum;
+        } else if (row >= L.t_start[col] && row <= L.t_end[col]) {
+            const float e = expf_glibc_tab(L.prefix[row] - L.prefix[col], L.exp_tab);
+            if (!which) L.qkd[row][col] = e * 1.0f * sum; // (the composite's scale: q carries its own)
+            else if (row != col) L.a[row][col] = L.beta[row] * e * sum;
+        }
+    }
+    __syncthreads();
+    const uint32_t nb = (n + kBlock - 1) / kBlock;
+    const uint32_t lt = (tid & 255) / 16, j = tid % 16; // (token of the block, value column)
+    if (wave == 0) { // tree_gram.rs:98-128: (I + A_diag)^-1 by forward substitution; a thread owns one column of one block (rows past the last node: of zeros)
+        const uint32_t blk = lane / kBlock % (kDnTreeMaxNodes / kBlock), col = lane % kBlock;
+        float inv[kBlock];
+        f32x4_v a[2][kBlock / 4]; // a row and the one behind it
+        auto read = [&](uint32_t row) {
+#pragma unroll
+            for (uint32_t i = 0; 4 * i < row; ++i) a[row % 2][i] = *(const f32x4_v*)&L.a[blk * kBlock + row][blk * kBlock + 4 * i];
+        };
+#pragma unroll
+        for (uint32_t row = 0; row < kBlock; ++row) {
+            if (row + 1 < kBlock) read(row + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            float sum = 0.0f;
+#pragma unroll
+            for (uint32_t prev = 0; prev < row; ++prev) {
+                const float with = sum + a[row % 2][prev / 4][prev % 4] * inv[prev];
+                sum = prev >= col ? with : sum;
+            }
+            inv[row] = row > col ? -sum : row == col ? 1.0f : 0.0f;
+            asm volatile("" : "+v"(inv[row]));
+        }
+        if (lane < kDnTreeMaxNodes) {
+#pragma unroll
+            for (uint32_t row = 0; row < kBlock; ++row) L.a_inv[blk][row][col] = inv[row];
+        }
+    } else if (tid >= 256 && tid < 512 && lt < n) { // tree_update_solve.rs:58-127, the first block's right-hand side meanwhile
+        L.acc[lt][j] = L.beta[lt] * (L.v[lt][j] - L.e_prefix[lt] * L.kh0[lt][j]);
+    }
+    __syncthreads();
+    for (uint32_t blk = 0; blk < nb; ++blk) {
+        const uint32_t token = blk * kBlock + lt;
+        if (blk) {
+            if (tid < 256 && token < n) {
+                float acc = L.beta[token] * (L.v[token][j] - L.e_prefix[token] * L.kh0[token][j]);
+#pragma unroll
+                for (uint32_t prev = 0; prev < kBlock; ++prev) acc -= L.a[token][prev] * L.u[prev][j]; // (kDnTreeMaxNodes / kBlock == 2: one block in front)
+                L.acc[lt][j] = acc;
+            }
+            __syncthreads();
+        }
+        if (tid < 256 && token < n) {
+            float sum = 0.0f;
+#pragma unroll
+            for (uint32_t lp = 0; lp < kBlock; ++lp) {
+                const float with = sum + L.a_inv[blk][lt][lp] * L.acc[lp][j];
+                sum = blk * kBlock + lp < n ? with : sum;
+            }
+            L.u[token][j] = sum;
+        }
+        __syncthreads();
+    }
+    static_assert(kDnTreeMaxNodes / kBlock == 2, "the second block has one block in front of it");
+    if (tid / 16 < n) { // out.rs:55-84
+        const uint32_t row = tid / 16;
+        float acc = 0.0f;
+        acc += L.e_prefix[row] * 1.0f * L.qh0[row][j];
+        for (uint32_t col0 = 0; col0 < n; col0 += 8)
+#pragma unroll
+            for (uint32_t col = col0; col < col0 + 8; ++col) {
+                const float with = acc + L.qkd[row][col] * L.u[col][j];
+                acc = col < n ? with : acc;
+            }
+        o[(size_t)row * value_dim + hv * D + c0 + j] = f32_to_bf16(acc);
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ state advance
 // state_advance.rs:25-58.  Production: a state row (hv, dv) lives in the registers of a half-wave (4 consecutive dk per lane) across the
 // accepted path; per accepted node: decay, k . row (butterfly over the 32 lanes), delta, rank-one update.
@@ -335,6 +588,20 @@ uzu_status delta_net_tree_verify(hipStream_t s, const uint16_t* q, const uint16_
     UZU_PROPAGATE(check_dims("delta_net_tree_verify", n, Hk, Hv, Dk, Dv));
     return launch_check([&] { hipLaunchKernelGGL(dn_tree_solve_kernel, dim3(Hv * (Dv / 16)), dim3(256), 0, s, q, k, v, trie, log_decay, beta, h0, out, 1.0f, n, Hk, Hv); },
                         "dn_tree_solve");
+}
+
+bool delta_net_tree_step_supported(const uint16_t* in_proj, const float* h0, uint32_t n, uint32_t kernel_size, uint32_t Hk, uint32_t Hv, uint32_t Dk, uint32_t Dv) {
+    return n && n <= kDnTreeMaxNodes && kernel_size >= 2 && kernel_size <= kTreeStepMaxKernel && Dk == 128 && Dv == 128 && Hk && Hv && Hv % Hk == 0 && Hv % 4 == 0 /* rows of 16 bytes' multiples */ &&
+           (((uintptr_t)in_proj | (uintptr_t)h0) & 15) == 0;
+}
+uzu_status delta_net_tree_step(hipStream_t s, const uint16_t* in_proj, const float* conv_w, const float* conv_b, const float* base_state, const int32_t* parents, const uint32_t* trie,
+                               const float* a_log, const float* dt_bias, const float* h0, float* suffix_state, uint16_t* k_out, uint16_t* v_out, float* beta_out, float* log_decay_out,
+                               uint16_t* out, uint32_t n, uint32_t kernel_size, uint32_t Hk, uint32_t Hv) {
+    return launch_check([&] {
+        const auto step = kernel_size == 4 ? dn_tree_step_kernel<4> : kernel_size == 3 ? dn_tree_step_kernel<3> : dn_tree_step_kernel<2>;
+        hipLaunchKernelGGL(step, dim3(Hv * 8), dim3(1024), 0, s, in_proj, conv_w, conv_b, base_state, parents, trie, a_log, dt_bias, h0, suffix_state, k_out, v_out, beta_out, log_decay_out, out,
+                           n, Hk, Hv);
+    }, "dn_tree_step");
 }
 
 uzu_status delta_net_state_advance(hipStream_t s, const uint16_t* k_norm, const uint16_t* v, const float* log_decay, const float* beta, const uint32_t* accepted_indices,
