@@ -12,6 +12,7 @@ from test_gpu_kernels import run
 from test_oracle_tree_verify import linear_stream, logit_error_sigma, path_of, random_tree
 from uzu_amd import _ffi
 from uzu_amd import backend as B
+from uzu_amd import desc as D
 from uzu_amd import synthetic as S
 from uzu_amd.engine import MODEL_BATCH, HipModel
 from uzu_amd.trie import TrieNode
@@ -293,6 +294,36 @@ def test_engine_tree_passes_of_every_size_are_bit_identical_in_reference_order_m
         _, lg = om.forward([int(o_sampled[path[-1]])], True)
         hm.decode(1)
         assert np.array_equal(hm.read_logits(), lg)
+        hm.close()
+    finally:
+        _set_exact(False)
+        om.close()
+
+
+def test_engine_accept_advances_the_states_of_more_layers_than_one_table_holds(hip_ctx):
+    """65 DeltaNet layers: a table of 64 states and one of a single one (dn_states_advance).  Everything but the acceptance in reference order, so that what differs from the oracle is
+    the advanced states' f32 sums (1e-5 of a state, test_state_advance): the logits behind the accepted path within the 0.25 sigma that the tests above give whole production passes."""
+    cfg = S.tiny_qwen(layer_kinds=[D.MIXER_DELTA_NET] * 65 + [D.MIXER_ATTENTION], vocab_size=512)
+    bundle = S.build_model(cfg)
+    row_mult = S.readout_row_multipliers(cfg)
+    prompt = S.synthetic_prompt(21, cfg.vocab_size)
+    om = O.OracleModel(bundle)
+    _set_exact(True)
+    try:
+        hm = HipModel(hip_ctx, bundle)
+        tok = om.prefill(prompt)
+        assert hm.prefill(prompt) == tok
+        nodes, _ = random_tree(4, np.random.default_rng(1), branch=0.0)  # a chain
+        tokens = np.array([tok, 3, 141, 59], np.uint32)
+        o_sampled = om.verify_tree(tokens, nodes)
+        assert np.array_equal(hm.verify_tree(tokens, nodes), o_sampled)
+        om.accept([0, 1, 2, 3])
+        _set_exact(False)
+        hm.accept([0, 1, 2, 3])
+        _set_exact(True)
+        _, want = om.forward([int(o_sampled[3])], True)
+        hm.decode(1)
+        assert logit_error_sigma(want, hm.read_logits(), row_mult) <= 0.25
         hm.close()
     finally:
         _set_exact(False)

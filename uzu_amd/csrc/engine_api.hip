@@ -472,11 +472,20 @@ uzu_status uzu_hip_model_accept(uzu_hip_model* m, const uint32_t* accepted_indic
     }
     hipStream_t s = m->ctx->stream;
     Enc e{m, s};
-    HIPCHK(hipMemcpyAsync(m->tree.d_accepted, accepted_indices, (size_t)count * 4, hipMemcpyHostToDevice, s));
     std::vector<uzu_kv_copy> copies;
     for (uint32_t i = 0; i < count; ++i)
         if (accepted_indices[i] != i) copies.push_back({m->context_length + accepted_indices[i], m->context_length + i});
     std::vector<CopyBlock> conv_states;
+    k::TreeStates states{};
+    states.accepted_len = count;
+    std::copy(accepted_indices, accepted_indices + count, states.accepted);
+    uint32_t n_states = 0;
+    size_t state_bytes = 0;
+    bool indices_copied = false;
+    const auto advance = [&] {
+        if (n_states) RUN("dn_states_advance", state_bytes, k::delta_net_states_advance(s, states, n_states));
+        n_states = 0, state_bytes = 0;
+    };
     for (size_t l = 0; l < m->layers.size(); ++l) {
         DLayer& L = m->layers[l];
         if (L.d.mixer_kind == UZU_MIXER_ATTENTION && L.d.is_kv_sharing) continue; // TransformerLayerStateType::Shared: nothing of its own to accept (transformer.rs:63-69)
@@ -492,10 +501,19 @@ uzu_status uzu_hip_model_accept(uzu_hip_model* m, const uint32_t* accepted_indic
         } else {
             const auto& T = m->tree.layers[l];
             conv_states.push_back({L.conv_state, (const char*)T.conv_states + (size_t)accepted_indices[count - 1] * L.conv_state_bytes, L.conv_state_bytes});
-            RUN("dn_state_advance", L.ssm_state_bytes * 2, k::delta_net_state_advance(s, T.k, T.v, T.log_decay, T.beta, m->tree.d_accepted, L.ssm_state, count, L.d.dn_num_heads,
-                                                                                     L.d.dn_num_groups, L.d.dn_head_dim));
+            if (k::exact_mode() || L.d.dn_head_dim != 128) {
+                if (!indices_copied) HIPCHK(hipMemcpyAsync(m->tree.d_accepted, accepted_indices, (size_t)count * 4, hipMemcpyHostToDevice, s));
+                indices_copied = true;
+                RUN("dn_state_advance", L.ssm_state_bytes * 2, k::delta_net_state_advance(s, T.k, T.v, T.log_decay, T.beta, m->tree.d_accepted, L.ssm_state, count, L.d.dn_num_heads,
+                                                                                         L.d.dn_num_groups, L.d.dn_head_dim));
+            } else { // the layers' states together, a table of them a launch
+                states.layer[n_states++] = {T.k, T.v, T.log_decay, T.beta, L.ssm_state, L.d.dn_num_heads, L.d.dn_num_groups};
+                state_bytes += L.ssm_state_bytes * 2;
+                if (n_states == k::kTreeStateLayers) advance();
+            }
         }
     }
+    advance();
     UZU_PROPAGATE(e.st);
     UZU_PROPAGATE(copy_blocks(s, conv_states));
     // control block: context length, the sampled tokens of the accepted nodes at their positions, the next input token

@@ -506,9 +506,8 @@ __global__ void __launch_bounds__(1024) dn_tree_step_kernel(const uint16_t* __re
 // ------------------------------------------------------------------------------------------------ state advance
 // state_advance.rs:25-58.  Production: a state row (hv, dv) lives in the registers of a half-wave (4 consecutive dk per lane) across the
 // accepted path; per accepted node: decay, k . row (butterfly over the 32 lanes), delta, rank-one update.
-__global__ void __launch_bounds__(256) dn_state_advance_kernel(const uint16_t* __restrict__ k_norm, const uint16_t* __restrict__ v, const float* __restrict__ log_decay,
-                                                               const float* __restrict__ beta, const uint32_t* __restrict__ accepted, float* __restrict__ state,
-                                                               uint32_t accepted_len, uint32_t Hv, uint32_t Hk) {
+__device__ __forceinline__ void state_advance(const uint16_t* __restrict__ k_norm, const uint16_t* __restrict__ v, const float* __restrict__ log_decay, const float* __restrict__ beta,
+                                              const uint32_t* accepted, float* __restrict__ state, uint32_t accepted_len, uint32_t Hv, uint32_t Hk) {
     constexpr uint32_t D = 128;
     const uint32_t row = blockIdx.x * 8 + threadIdx.x / 32, sub = threadIdx.x % 32; // 8 state rows per workgroup
     const uint32_t hv = row / D, dv = row % D, hk = hv / (Hv / Hk);
@@ -529,6 +528,18 @@ __global__ void __launch_bounds__(256) dn_state_advance_kernel(const uint16_t* _
         st.x += k0 * delta, st.y += k1 * delta, st.z += k2 * delta, st.w += k3 * delta;
     }
     *(f32x4_v*)srow = st;
+}
+__global__ void __launch_bounds__(256) dn_state_advance_kernel(const uint16_t* __restrict__ k_norm, const uint16_t* __restrict__ v, const float* __restrict__ log_decay,
+                                                               const float* __restrict__ beta, const uint32_t* __restrict__ accepted, float* __restrict__ state,
+                                                               uint32_t accepted_len, uint32_t Hv, uint32_t Hk) {
+    state_advance(k_norm, v, log_decay, beta, accepted, state, accepted_len, Hv, Hk);
+}
+// The layers' states in one launch, grid.y = layers: a megabyte of state a layer is less than a launch (18 layers of 16 heads: 66 us in 18 launches, now 13; the indices come as
+// arguments, which saves their copy)
+__global__ void __launch_bounds__(256) dn_states_advance_kernel(TreeStates t) {
+    const TreeState& L = t.layer[blockIdx.y];
+    if (blockIdx.x * 8 >= L.Hv * 128) return; // (layers of fewer heads)
+    state_advance(L.k, L.v, L.log_decay, L.beta, t.accepted, L.state, t.accepted_len, L.Hv, L.Hk);
 }
 // reference order: one thread per state row, everything sequential (uzu_hip_set_exact)
 __global__ void __launch_bounds__(64) dn_state_advance_exact_kernel(const uint16_t* k_norm, const uint16_t* v, const float* log_decay, const float* beta, const uint32_t* accepted,
@@ -615,6 +626,16 @@ uzu_status delta_net_state_advance(hipStream_t s, const uint16_t* k_norm, const 
     return launch_check([&] {
         hipLaunchKernelGGL(dn_state_advance_kernel, dim3(Hv * Dk / 8), dim3(256), 0, s, k_norm, v, log_decay, beta, accepted_indices, state, accepted_len, Hv, Hk);
     }, "dn_state_advance");
+}
+
+uzu_status delta_net_states_advance(hipStream_t s, const TreeStates& t, uint32_t layers) {
+    uint32_t heads = 0;
+    for (uint32_t l = 0; l < layers; ++l) {
+        UZU_PROPAGATE(check_dims("state_advance", 0, t.layer[l].Hk, t.layer[l].Hv, 128, 128));
+        heads = heads > t.layer[l].Hv ? heads : t.layer[l].Hv;
+    }
+    if (!layers || !t.accepted_len) return UZU_OK;
+    return launch_check([&] { hipLaunchKernelGGL(dn_states_advance_kernel, dim3(heads * 16, layers), dim3(256), 0, s, t); }, "dn_states_advance");
 }
 
 } // namespace k

@@ -23,5 +23,19 @@ uzu_status delta_net_tree_step(hipStream_t s, const uint16_t* in_proj, const flo
                                const float* a_log, const float* dt_bias, const float* h0, float* suffix_state, uint16_t* k_out, uint16_t* v_out, float* beta_out, float* log_decay_out,
                                uint16_t* out, uint32_t n, uint32_t kernel_size, uint32_t Hk, uint32_t Hv);
 
+// StateAdvance of several layers along one accepted path (head_dim 128), in one launch; passed by value
+struct TreeState {
+    const uint16_t *k, *v;
+    const float *log_decay, *beta;
+    float* state;
+    uint32_t Hv, Hk;
+};
+constexpr uint32_t kTreeStateLayers = 64; // (3.2 KB of kernel arguments)
+struct TreeStates {
+    TreeState layer[kTreeStateLayers];
+    uint32_t accepted[kDnTreeMaxNodes], accepted_len;
+};
+uzu_status delta_net_states_advance(hipStream_t s, const TreeStates& t, uint32_t layers);
+
 } // namespace k
 } // namespace uzu
