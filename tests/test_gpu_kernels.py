@@ -1145,6 +1145,28 @@ def test_delta_net_prefill_path(hip_ctx, T, Dv):
     assert ((err <= 2e-2) | (ulps <= 1)).all() and (ulps <= 2).mean() > 0.99
 
 
+@pytest.mark.parametrize("T,Hv", [(1, 4), (5, 4), (37, 12), (32, 16), (9, 2)])
+def test_delta_net_norm_gate_of_every_gate(hip_ctx, T, Hv):
+    """The norm-gate by sixteen lanes a head (and by a wave a head: two heads, rows of odd multiples of 8 bytes), the last workgroup nearly empty and full.  Rows of +-1, whose sum of
+    squares is the same in every order, and 32 x 16 heads of 128 gates are all bf16 numbers: bit-identical to the oracle's 64-bit exponential, quick quotients and all."""
+    rng = np.random.default_rng(T * Hv)
+    value_dim = Hv * 128
+    conv_dim = 2 * 256 + value_dim
+    total = conv_dim + value_dim + 2 * Hv
+    out = bf16(rng.choice([-1.0, 1.0], size=(T, value_dim)))
+    rows = bf16(rng.normal(size=(T, total)))
+    z = np.arange(65536, dtype=np.uint32).astype(np.uint16)
+    rows[:, conv_dim:conv_dim + value_dim] = rng.permutation(z)[:T * value_dim].reshape(T, value_dim)
+    w = rng.normal(size=128).astype(np.float32)
+    want = out.copy()
+    O.call("orc_delta_net_norm_gate", want, rows, w, Hv, 128, value_dim, conv_dim, total, 1e-6, T)
+    k = B.DeltaNetNormGateKernel.new(hip_ctx, B.BF16)
+    bo, bi, bw = hip_ctx.buffer_from(out), hip_ctx.buffer_from(rows), hip_ctx.buffer_from(w)
+    run(hip_ctx, lambda cb: k.encode(bo, bi, bw, Hv, 128, value_dim, conv_dim, total, 1e-6, T, cb))
+    got = bo.download(np.uint16, out.size).reshape(out.shape)
+    assert ((got == want) | (np.isnan(f32(got)) & np.isnan(f32(want)))).all()
+
+
 def delta_net_inputs(rng, T, Hv, Hk, Dv, pace):
     """what DeltaNetPrefill reads: unit keys, queries scaled by 1 / sqrt(128), strengths in (0, 1), decays exp(-pace e^n), values among the in-projection rows, a state"""
     kd, vd = Hk * 128, Hv * Dv

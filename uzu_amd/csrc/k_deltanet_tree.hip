@@ -15,6 +15,7 @@
 // sequential delta-rule steps in reference order would be one thread per row (~100 us); the production form gives a row to a half-wave
 // (tolerance-class like the decode update), the reference-order form exists for uzu_hip_set_exact(1).
 #include "device_utils.h"
+#include "silu_near.h"
 #include "tree_pass.h"
 
 namespace uzu {
@@ -336,7 +337,7 @@ __global__ void __launch_bounds__(1024) dn_tree_step_kernel(const uint16_t* __re
             acc += sample * w[KS - 1 - h];
             if (files && h < history) suffix_state[((size_t)node * conv_dim + channel) * history + (history - 1 - h)] = sample;
         }
-        return f32_to_bf16(silu_f32_tab(acc, L.exp_tab));
+        return silu_bf16(acc, L.exp_tab);
     };
     if (wave < 4 * kGroups) {
         for (uint32_t node = wave / 4; node < n; node += kGroups) {

@@ -13,6 +13,7 @@
 //   * partial results lie as [column tile][share][element][32 columns], so that both launches move whole lines.
 // Layout of the operands as in k_attention_mfma.hip: scores transposed, so that a lane owns a column.
 #include "device_utils.h"
+#include "silu_near.h"
 #include "tree_pass.h"
 
 namespace uzu {
@@ -263,7 +264,7 @@ __global__ void __launch_bounds__(256) tree_attention_merge_kernel(const float* 
             }
         }
     uint16_t bits = f32_to_bf16(o / l_all);
-    if (gate) bits = f32_to_bf16(bf16_to_f32(bits) * (1.0f / (1.0f + expf_glibc_tab(-bf16_to_f32(g), s_exp_tab))));
+    if (gate) bits = scaled_sigmoid_bf16(bf16_to_f32(bits), bf16_to_f32(g), s_exp_tab);
     out[row * head_dim + element] = bits;
 }
 // kv heads x pairs of column tiles; the shares that put a workgroup on most of the 256 compute units
