@@ -813,6 +813,23 @@ def test_attention_prefill_matrix_core_path_full_chunks(hip_ctx, heads, kv_heads
     assert (want == got).mean() >= 0.97
 
 
+@pytest.mark.parametrize("heads,kv_heads,hd,seq,suffix", [(2, 1, 256, 900, 16), (2, 1, 64, 1600, 33), (8, 2, 256, 700, 700), (10, 2, 128, 1500, 700), (6, 2, 256, 1100, 257), (8, 2, 64, 1290, 1027)])
+def test_attention_prefill_with_uneven_key_shares(hip_ctx, heads, kv_heads, hd, seq, suffix):
+    """Groups of query rows with one to twelve shares of the keys, by what they see (KeyShares): a single group with more stretches than there can be shares, GQA factors whose groups
+    straddle tiles of queries, ragged last tiles; scores that grow by more than 8 along the keys, so that the running maximum is taken anew, and that don't.  The bar of the tests above."""
+    rng = np.random.default_rng(heads * hd + seq + suffix)
+    q, k, v, a = attention_case(rng, heads, kv_heads, hd, seq, suffix, seq + 8)
+    k = bf16(f32(k) * np.linspace(0.2, 6.0, len(k), dtype=np.float32)[:, None])
+    a.keys = k.ctypes.data
+    want = np.zeros((suffix, heads, hd), np.uint16)
+    O.lib().orc_attention_single_pass(C.byref(a), O.p(want))
+    kern = B.AttentionSinglePassKernel.new(hip_ctx, B.BF16, hd, 0, 0, 1, 0, 0)
+    bq, bk, bv, bo = hip_ctx.buffer_from(q), hip_ctx.buffer_from(k), hip_ctx.buffer_from(v), hip_ctx.create_buffer(want.nbytes)
+    run(hip_ctx, lambda cb: kern.encode(bq, bk, bv, bo, heads // kv_heads, seq, hd, kv_heads * hd, hd, kv_heads * hd, None, 1.0 / np.sqrt(hd), None, None, None, heads, suffix, cb))
+    got = bo.download(np.uint16, want.size).reshape(want.shape)
+    assert ((ulp_diff_bf16(want, got) <= 2.0) | (np.abs(f32(want) - f32(got)) <= 2e-3)).all()
+
+
 @pytest.mark.parametrize("heads,kv_heads,hd,seq,suffix", [(8, 2, 256, 2048, 1), (32, 8, 128, 1500, 1), (8, 2, 256, 1100, 3), (4, 2, 64, 40, 1)])
 def test_attention_two_pass(hip_ctx, heads, kv_heads, hd, seq, suffix):
     """Split-KV: pass 1 partials have the reference's meaning (block b = keys b, b+32, ...), pass 2 is bit-exact

@@ -14,6 +14,7 @@
 // the next input token and the sampled-token history live in device memory, so ONE captured hipGraph is
 // replayed for every decode step and steps are chained without a host round trip.
 #include "engine_types.h"
+#include "attention_prefill.h"
 #include "tree_pass.h"
 
 using namespace uzu;
@@ -401,7 +402,7 @@ void attention_core(Enc& e, DLayer& L, uint32_t batch, size_t row0, bool fuse_no
     }
     if (k::attention_prefill_mfma_supported(a)) { // prefill chunk: flash-attention tiles on the matrix cores, any context length
         uint32_t gate_done = 0; // SigmoidGate inside the key-split merge launch when the pass has one (bit-identical to the separate launch)
-        RUN("attention_prefill_mfma", kv_bytes, k::attention_prefill_mfma(e.s, a, attn_out, L.d.has_gate && attention_fusions_enabled() ? m->gate + row0 * nq * hd : nullptr, &gate_done));
+        RUN("attention_prefill_mfma", kv_bytes, k::attention_prefill_mfma_behind(e.s, a, W ? W : m->context_length, attn_out, L.d.has_gate && attention_fusions_enabled() ? m->gate + row0 * nq * hd : nullptr, &gate_done));
         gated = gate_done != 0;
     } else if (k::attention_tree_supported(a)) { // a speculated tree's rows, any context length (the gate with them)
         RUN("attention_tree", kv_bytes, k::attention_tree(e.s, a, m->d.max_context_length, m->partials, m->sums, m->maxs, attn_out, L.d.has_gate ? m->gate + row0 * nq * hd : nullptr));

@@ -22,9 +22,11 @@
 //     the summation order.
 #include <stdlib.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "device_utils.h"
+#include "attention_prefill.h"
 #include "kernels.h"
 #include "silu_near.h"
 
@@ -39,7 +41,23 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 namespace {
 constexpr int TK = 32; // keys per tile (one MFMA block)
 constexpr int TQ = 32; // queries per wave
-constexpr uint32_t kMaxKeySplits = 8;
+constexpr uint32_t kMaxKeySplits = 12;
+
+// How a launch's workgroups divide the keys.  A group of tasks (four consecutive ones) sees the keys in front of its last query, so equal numbers of shares would leave the last
+// group's the longest by far: group y has a share per `quantum` stretches of keys that it was thought to see, and works out its shares from the keys that it does see.
+struct KeyShares {
+    uint32_t quantum; // stretches a share; 0: no shares, every group to its end by itself
+    uint32_t prefix;  // cached keys, as far as the host knows
+};
+__host__ __device__ inline uint32_t key_stretches(const KeyShares& k, uint32_t y, uint32_t tpw, uint32_t gqa, uint32_t M, uint32_t stretch) {
+    const uint32_t n_tasks = gqa * ((M + TQ - 1) / TQ), task = y * tpw + tpw - 1, end = ((task < n_tasks ? task : n_tasks - 1) / gqa + 1) * TQ;
+    return (k.prefix + (end < M ? end : M) + stretch - 1) / stretch;
+}
+__host__ __device__ inline uint32_t key_shares(const KeyShares& k, uint32_t y, uint32_t tpw, uint32_t gqa, uint32_t M, uint32_t stretch) {
+    if (!k.quantum) return 1;
+    const uint32_t shares = (key_stretches(k, y, tpw, gqa, M, stretch) + k.quantum - 1) / k.quantum;
+    return shares < kMaxKeySplits ? shares : kMaxKeySplits;
+}
 
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
     const bf16x2_t v = {(__bf16)lo, (__bf16)hi};
@@ -52,8 +70,8 @@ __device__ __forceinline__ float other_half(float v) { return __shfl_xor(v, 32, 
 // grid: (kv heads, ceil(gqa * query tiles / tpw)); 256 KG threads.  Workgroups with the longest key ranges are numbered first.
 // tpw = wave tasks per workgroup (4, 2 or 1): models with few heads (Qwen3.5-0.8B: 8 q heads -> 256 tasks per 1024-token chunk)
 // would fill 64 CUs at four tasks per workgroup; with fewer tasks the idle waves still help staging the K / V tiles.
-// Key split (few-head models: Qwen3.5-0.8B has 2 kv heads -> 64 workgroups of four tasks per 1024-token chunk): gridDim.z workgroups share a
-// task group, each takes an equal share of the key tiles ITS queries can see and leaves the unnormalised O^T, the running maximum and the
+// Key split (few-head models: Qwen3.5-0.8B has 2 kv heads -> 64 workgroups of four tasks per 1024-token chunk): several workgroups share a
+// task group (KeyShares), each takes an equal share of the key tiles ITS queries can see and leaves the unnormalised O^T, the running maximum and the
 // sum as f32 partials ([split][query][head]); attention_prefill_merge_kernel folds them (the AttentionTwoPass2 step of the decode path).
 // GEN: the general mask of mask.rs:3-61 without the trie -- sliding window, ring KV prefix (AttentionStateType::Ring: the prefix rows are a
 // ring of `prefix` slots, key position = (prefix + i - ring_offset) mod prefix, live iff < ring_length) and attention sinks (the running
@@ -65,7 +83,7 @@ __device__ __forceinline__ float other_half(float v) { return __shfl_xor(v, 32, 
 // SEQS: several sequences, each with its own rows and cache, gridDim.x = kv heads x sequences and no key splits: the workgroups with the longest key ranges of all of them come first, and the
 // short ones fill what a sequence by itself leaves idle (four of 1021 rows, 32 heads of 128: 4 x 39 us -> 99).
 template <int HD, bool GEN, bool SEQS = false, int KG = HD <= 128 ? 2 : 1>
-__global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(AttentionParams a, uint16_t* out, uint32_t tpw, float* part_o, float* part_ml, std::conditional_t<SEQS, AttentionSeqs, uint32_t> seqs) {
+__global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(AttentionParams a, uint16_t* out, uint32_t tpw, float* part_o, float* part_ml, std::conditional_t<SEQS, AttentionSeqs, KeyShares> more) {
     constexpr int KP = HD * 2 + 16;  // K tile row pitch in bytes (conflict-free ds_read_b128)
     constexpr int VP = TK * 2 + 8;   // V^T tile row pitch in bytes: 32 keys + 8 bytes of pad (conflict-free ds_read_b64)
     constexpr int NS = HD / 16;      // k16 steps of the QK^T contraction
@@ -84,10 +102,16 @@ __global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(Attent
     if constexpr (SEQS) {
         const uint32_t kv_heads = a.num_heads / a.gqa_factor, seq = kv_head / kv_heads;
         kv_head -= seq * kv_heads;
-        a.queries = seqs.queries[seq], a.keys = seqs.keys[seq], a.values = seqs.values[seq], a.dyn = seqs.dyn[seq], out = (uint16_t*)seqs.out[seq];
+        a.queries = more.queries[seq], a.keys = more.keys[seq], a.values = more.values[seq], a.dyn = more.dyn[seq], out = (uint16_t*)more.out[seq];
     }
     const uint32_t n_tasks = a.gqa_factor * ((M + TQ - 1) / TQ);
-    const uint32_t task0 = (gridDim.y - 1 - blockIdx.y) * tpw; // heaviest (last query tiles) first
+    uint32_t y = gridDim.y - 1 - blockIdx.y, share = 0, shares = 1; // heaviest (last query tiles) first
+    if constexpr (!SEQS)
+        if (more.quantum) {
+            y = (n_tasks + tpw - 1) / tpw - 1, share = blockIdx.y;
+            while (share >= (shares = key_shares(more, y, tpw, a.gqa_factor, M, KEYS))) share -= shares, --y;
+        }
+    const uint32_t task0 = y * tpw;
     const uint32_t task = task0 + wave;
     const bool wave_live = (uint32_t)wave < tpw && task < n_tasks;
     const uint32_t task_c = wave_live ? task : n_tasks - 1;
@@ -121,8 +145,8 @@ __global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(Attent
     const uint32_t wg_last_q = (last_tile < M ? last_tile : M) - 1;
     const uint32_t key_end = prefix + wg_last_q + 1;
     const uint32_t n_tiles_all = (key_end + KEYS - 1) / KEYS; // (tiles of the workgroup: stretches of KEYS)
-    const uint32_t per_split = (n_tiles_all + gridDim.z - 1) / gridDim.z;
-    const uint32_t t_lo = min(blockIdx.z * per_split, n_tiles_all), n_tiles = min(t_lo + per_split, n_tiles_all); // this workgroup: tiles [t_lo, n_tiles)
+    const uint32_t per_share = (n_tiles_all + shares - 1) / shares;
+    const uint32_t t_lo = min(share * per_share, n_tiles_all), n_tiles = min(t_lo + per_share, n_tiles_all); // this workgroup: tiles [t_lo, n_tiles)
     auto load_tile = [&](uint32_t t) {
         const u32x4_v zero = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -166,15 +190,36 @@ __global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(Attent
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[b][r] = 0.f;
     float m_run = -INFINITY, l_run = 0.f; // l_run: this lane's half of the keys only (merged at the end)
+    // Exponents of 2: a weight is 2^(score c - m), c = scale log2 e in two floats and one rounding to f32 (the score scaled, the maximum taken off and the product with log2 e each rounded
+    // left weights 2^-22 off that the bf16 terms had right).  The smaller float has the larger one's sign, so that the infinity of a key that is not seen stays one.
+    constexpr float kLog2e = 0x1.715476p+0f;
+    float c_hi, c_lo;
+    {
+        const double c = (double)a.scale * 0x1.71547652b82fep+0;
+        c_hi = (float)c;
+        if (fabs((double)c_hi) >= fabs(c)) c_hi = bits_to_f32(f32_to_bits(c_hi) - 1);
+        c_lo = (float)(c - (double)c_hi);
+    }
+    const float unseen = a.scale < 0.f ? INFINITY : -INFINITY;
     const uint32_t my_last_key = prefix + qi; // causal: keys 0 .. prefix + qi
     if constexpr (GEN) {
-        if (a.sinks && blockIdx.z == 0 && kg == 0) { // the sink's unit of mass is counted once: by half 0 of the first group of the first key split
-            m_run = bf16_to_f32(((const uint16_t*)a.sinks)[head]);
-            l_run = half == 0 ? 1.0f : 0.0f;
+        if (a.sinks && share == 0 && kg == 0) { // the sink's unit of mass is counted once: by half 0 of the first group of the first key split
+            const float sink = bf16_to_f32(((const uint16_t*)a.sinks)[head]);
+            m_run = sink * kLog2e;
+            l_run = half == 0 ? (fabsf(m_run) < INFINITY ? __builtin_amdgcn_exp2f(fmaf(sink, kLog2e, -m_run)) : 1.0f) : 0.0f; // (one, but for what the maximum's rounding takes)
         }
     }
     const uint32_t query_position = suffix_position + qi;
+    // heads of 256: the results stay in the accumulation registers, beside the operands in the others, and leave them in a tile that rescales them alone (left to itself the compiler
+    // moves all of them every tile).  With the operands in front of the products, 2043 rows of 8 heads of 256: 77.5 -> 73.0 us; four times 1021 rows of 32 heads of 128: 99 -> 97
+    auto keep = [&]() {
+        if constexpr (HD > 128) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) asm volatile("" : "+a"(o[b]));
+        }
+    };
 
+    keep();
     if (t_lo < n_tiles) {
         load_tile(t_lo);
         store_tile(t_lo & 1);
@@ -183,6 +228,7 @@ __global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(Attent
     for (uint32_t t = t_lo; t < n_tiles; ++t) {
         const int buf = t & 1;
         load_tile(t + 1 < n_tiles ? t + 1 : t); // unconditional: the compiler can count the loads in flight
+        keep();
         // a wave whose queries all end before this tile has nothing to add (causal), but must keep the barriers
         const uint32_t wave_last_key = prefix + (q0 + TQ - 1 < M ? q0 + TQ - 1 : M - 1);
         const uint32_t kb = t * KEYS + kg * TK; // this group's first key
@@ -192,69 +238,98 @@ __global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(Attent
 #pragma unroll
             for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
             const uint8_t* kt = s_k(buf) + (kg * TK + l32) * KP + half * 16;
+            // (all of a product's operands are on their way before its first instruction: read two by two, each pair was waited for)
+            u32x4_t kf[NS];
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
                 const uint4 kv = *(const uint4*)(kt + s * 32);
-                const u32x4_t kfrag = {kv.x, kv.y, kv.z, kv.w};
-                sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kfrag), __builtin_bit_cast(bf16x8_t, qf[s]), sacc, 0, 0, 0);
+                kf[s] = u32x4_t{kv.x, kv.y, kv.z, kv.w};
             }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < NS; ++s) sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kf[s]), __builtin_bit_cast(bf16x8_t, qf[s]), sacc, 0, 0, 0);
+            // A = V^T: lane = (hd row b*32 + l32, half): keys 16 st + 4 half + {0..3} and 16 st + 8 + 4 half + {0..3}
+            u32x4_t vf[2][NB];
+            auto read_v = [&](int st) {
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const uint8_t* vr = s_vt(buf) + (kg * HD + b * 32 + l32) * VP + (16 * st + 4 * half) * 2;
+                    const uint2 v0 = *(const uint2*)vr, v1 = *(const uint2*)(vr + 16);
+                    vf[st][b] = u32x4_t{v0.x, v0.y, v1.x, v1.y};
+                }
+            };
+            read_v(0);
+            __builtin_amdgcn_sched_barrier(0);
             // ---- scale, causal mask, online softmax (lane = one query; its 16 keys: (r & 3) + 8 (r >> 2) + 4 half)
             float sc[16];
             float m_loc = -INFINITY;
+            if (!GEN && kb + TK <= prefix + q0 + 1) { // every query of the wave sees the whole tile (rows past the last are nobody's)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t key = kb + (r & 3) + 8 * (r >> 2) + 4 * half;
-                bool vis = q_live && key <= my_last_key;
-                if constexpr (GEN) { // mask.rs:31-60 on positions
-                    uint32_t key_position;
-                    if (key >= prefix) {
-                        key_position = suffix_position + (key - prefix);
-                    } else if (a.is_kv_cache_ring) {
-                        key_position = prefix + key - a.ring_offset;
-                        if (key_position >= prefix) key_position -= prefix;
-                        vis = vis && key_position < a.ring_length;
-                    } else {
-                        key_position = key;
+                for (int r = 0; r < 16; ++r) sc[r] = sacc[r];
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const uint32_t key = kb + (r & 3) + 8 * (r >> 2) + 4 * half;
+                    bool vis = q_live && key <= my_last_key;
+                    if constexpr (GEN) { // mask.rs:31-60 on positions
+                        uint32_t key_position;
+                        if (key >= prefix) {
+                            key_position = suffix_position + (key - prefix);
+                        } else if (a.is_kv_cache_ring) {
+                            key_position = prefix + key - a.ring_offset;
+                            if (key_position >= prefix) key_position -= prefix;
+                            vis = vis && key_position < a.ring_length;
+                        } else {
+                            key_position = key;
+                        }
+                        if (a.is_sliding_window) vis = vis && key_position <= query_position && query_position - key_position < a.sliding_window_size;
                     }
-                    if (a.is_sliding_window) vis = vis && key_position <= query_position && query_position - key_position < a.sliding_window_size;
+                    sc[r] = vis ? sacc[r] : unseen;
                 }
-                sc[r] = vis ? a.scale * sacc[r] : -INFINITY;
-                m_loc = fmaxf(m_loc, sc[r]);
             }
-            const float m_new = fmaxf(m_run, fmaxf(m_loc, other_half(m_loc)));
-            const float alpha = m_new == -INFINITY ? 1.0f : fast_exp(m_run - m_new); // m_run = -inf => exp(-inf) = 0
+#pragma unroll
+            for (int r = 0; r < 16; ++r) m_loc = fmaxf(m_loc, sc[r] * c_hi);
+            // (A tile that raises nobody's maximum leaves the results alone: 128 products of a head of 256, and as many moves out of the accumulators and back.  A maximum that is allowed to
+            // lag, so that hardly a tile rescales, was 8 us of 73 faster and is not taken: the largest weight is then no longer 1, which the two terms hold exactly, and 8 % more results
+            // miss the nearest bf16.)
+            m_loc = fmaxf(m_loc, other_half(m_loc));
+            keep();
+            if (__any(m_loc > m_run)) {
+                const float m_new = fmaxf(m_run, m_loc), alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new); // m_run = -inf => 2^-inf = 0
+                l_run *= alpha, m_run = m_new;
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o[b][r] *= alpha;
+                keep();
+            }
+            const float m_ref = m_run == -INFINITY ? 0.f : m_run; // (a query that has seen no key: every score is -inf)
             float psum = 0.f;
             uint32_t p_hi[8], p_lo[8];
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
-                const float p0 = m_new == -INFINITY ? 0.f : fast_exp(sc[r] - m_new), p1 = m_new == -INFINITY ? 0.f : fast_exp(sc[r + 1] - m_new);
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[r], c_hi, fmaf(sc[r], c_lo, -m_ref))), p1 = __builtin_amdgcn_exp2f(fmaf(sc[r + 1], c_hi, fmaf(sc[r + 1], c_lo, -m_ref)));
                 psum += p0 + p1;
                 const float h0 = round_bf16(p0), h1 = round_bf16(p1);
                 p_hi[r / 2] = pack2(h0, h1);
                 p_lo[r / 2] = pack2(p0 - h0, p1 - h1);
             }
-            l_run = l_run * alpha + psum;
-            m_run = m_new;
-#pragma unroll
-            for (int b = 0; b < NB; ++b)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[b][r] *= alpha;
+            l_run += psum;
             // ---- O^T += V^T P^T : two k16 steps (registers 0..7 and 8..15 of the score tile), P as hi + lo
 #pragma unroll
             for (int st = 0; st < 2; ++st) {
                 const u32x4_t ph = {p_hi[4 * st], p_hi[4 * st + 1], p_hi[4 * st + 2], p_hi[4 * st + 3]};
                 const u32x4_t pl = {p_lo[4 * st], p_lo[4 * st + 1], p_lo[4 * st + 2], p_lo[4 * st + 3]};
+                if (st == 0) read_v(1);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int b = 0; b < NB; ++b) {
-                    // A = V^T: lane = (hd row b*32 + l32, half): keys 16 st + 4 half + {0..3} and 16 st + 8 + 4 half + {0..3}
-                    const uint8_t* vr = s_vt(buf) + (kg * HD + b * 32 + l32) * VP + (16 * st + 4 * half) * 2;
-                    const uint2 v0 = *(const uint2*)vr, v1 = *(const uint2*)(vr + 16);
-                    const u32x4_t vfrag = {v0.x, v0.y, v1.x, v1.y};
-                    o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vfrag), __builtin_bit_cast(bf16x8_t, ph), o[b], 0, 0, 0);
-                    o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vfrag), __builtin_bit_cast(bf16x8_t, pl), o[b], 0, 0, 0);
-                }
+                for (int b = 0; b < NB; ++b) o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vf[st][b]), __builtin_bit_cast(bf16x8_t, ph), o[b], 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vf[st][b]), __builtin_bit_cast(bf16x8_t, pl), o[b], 0, 0, 0);
             }
+            keep();
         }
+        keep();
         if (t + 1 < n_tiles) store_tile(buf ^ 1);
         lds_barrier();
     }
@@ -274,7 +349,7 @@ __global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(Attent
         for (int other = 0; other < KG - 1; ++other) {
             const float* theirs = s_o + (other * 4 + wave) * PER + lane;
             const float m_o = theirs[16 * NB * 64], l_o = theirs[(16 * NB + 1) * 64], m_new = fmaxf(m_run, m_o);
-            const float x = m_run == -INFINITY ? 0.f : fast_exp(m_run - m_new), y = m_o == -INFINITY ? 0.f : fast_exp(m_o - m_new); // (a group that saw no key: m = -inf, l = 0)
+            const float x = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new), y = m_o == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_o - m_new); // (a group that saw no key: m = -inf, l = 0)
             l_run = l_run * x + l_o * y, m_run = m_new;
 #pragma unroll
             for (int b = 0; b < NB; ++b)
@@ -286,7 +361,7 @@ __global__ void __launch_bounds__(256 * KG) attention_prefill_mfma_kernel(Attent
     const float l_tot = l_run + other_half(l_run);
     if (part_o) { // key split: f32 partials, row = (split, query, head)
         if (q_live) {
-            const size_t row = ((size_t)blockIdx.z * M + qi) * a.num_heads + head;
+            const size_t row = ((size_t)share * M + qi) * a.num_heads + head;
             float* po = part_o + row * HD;
 #pragma unroll
             for (int b = 0; b < NB; ++b)
@@ -328,17 +403,20 @@ bool attention_prefill_mfma_supported(const AttentionParams& a) {
     if (a.suffix_length < min_m || !(a.head_dim == 64 || a.head_dim == 128 || a.head_dim == 256)) return false;
     if (a.gqa_factor == 0 || a.num_heads % a.gqa_factor) return false;
     if (a.k_head_stride % 8 || a.k_seq_stride % 8 || a.v_head_stride % 8 || a.v_seq_stride % 8) return false;
+    if (!(fabsf(a.scale) >= 1e-20f && fabsf(a.scale) <= 1e20f)) return false; // (two floats of it)
     return true;
 }
 
-// out[q][head][:] = sum_s w_s O_s / sum_s w_s l_s, w_s = exp(m_s - max m) (a split that saw no key has m = -inf, l = 0: weight 0).
+// out[q][head][:] = sum_s w_s O_s / sum_s w_s l_s, w_s = 2^(m_s - max m) (a split that saw no key has m = -inf, l = 0: weight 0).
 // grid = rows / 4, 256 threads: 64 threads per (query, head) row, HD / 64 elements each.
 template <int HD>
 // gate (optional): SigmoidGate (sigmoid_gate.rs:9-22) on the merged rows in the same launch -- out = bf16(bf16(o) * sigmoid(gate)), the separate kernel's two roundings
-__global__ void __launch_bounds__(256) attention_prefill_merge_kernel(const float* part_o, const float* part_ml, uint16_t* out, uint32_t rows, uint32_t splits, const uint16_t* gate) {
+__global__ void __launch_bounds__(256) attention_prefill_merge_kernel(const float* part_o, const float* part_ml, uint16_t* out, uint32_t rows, KeyShares shares, uint32_t tpw,
+                                                                      uint32_t gqa, uint32_t heads, const uint16_t* gate) {
     constexpr int EPT = HD / 64;
     const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6), e0 = (threadIdx.x & 63) * EPT;
     if (row >= rows) return;
+    const uint32_t query = row / heads, head = row - query * heads, splits = key_shares(shares, (query / TQ * gqa + head % gqa) / tpw, tpw, gqa, rows / heads, HD <= 128 ? 2 * TK : TK);
     // every share is requested before the first is used (one behind the other, a share was two trips to memory: 8 shares of 517 rows 11.2 us -> 9.3, 2 of 2043 15.4 -> 13.9)
     float ms[kMaxKeySplits], ls[kMaxKeySplits], po[kMaxKeySplits][EPT];
     uint16_t gs[EPT];
@@ -364,7 +442,7 @@ __global__ void __launch_bounds__(256) attention_prefill_merge_kernel(const floa
 #pragma unroll
     for (uint32_t sp = 0; sp < kMaxKeySplits; ++sp) {
         if (sp >= splits || ms[sp] == -INFINITY) continue;
-        const float w = fast_exp(ms[sp] - m);
+        const float w = __builtin_amdgcn_exp2f(ms[sp] - m);
         l = fmaf(ls[sp], w, l);
 #pragma unroll
         for (int e = 0; e < EPT; ++e) acc[e] = fmaf(po[sp][e], w, acc[e]);
@@ -390,6 +468,9 @@ __global__ void __launch_bounds__(256) attention_prefill_merge_kernel(const floa
 }
 
 uzu_status attention_prefill_mfma(hipStream_t s, const AttentionParams& a, void* out, const void* gate, uint32_t* gate_done) {
+    return attention_prefill_mfma_behind(s, a, a.sequence_length > a.suffix_length ? a.sequence_length - a.suffix_length : 0, out, gate, gate_done);
+}
+uzu_status attention_prefill_mfma_behind(hipStream_t s, const AttentionParams& a, uint32_t prefix, void* out, const void* gate, uint32_t* gate_done) {
     if (gate_done) *gate_done = 0;
     const uint32_t kv_heads = a.num_heads / a.gqa_factor;
     const uint32_t n_tasks = a.gqa_factor * ((a.suffix_length + TQ - 1) / TQ);
@@ -397,45 +478,55 @@ uzu_status attention_prefill_mfma(hipStream_t s, const AttentionParams& a, void*
         const char* e = lab_env("UZU_ATTN_TPW");
         return e ? (uint32_t)atoi(e) : 0u;
     }();
-    static const int force_split = [] { // UZU_ATTN_KSPLIT: 1 = never split the keys (A/B runs), n = that many splits
+    static const int force_split = [] { // UZU_ATTN_KSPLIT: 1 = never split the keys (A/B runs)
         const char* e = lab_env("UZU_ATTN_KSPLIT");
         return e ? atoi(e) : 0;
     }();
     // Few task groups (few kv heads x short chunks): keep four tasks per workgroup -- they share every staged K / V tile -- and split the KEYS
     // over workgroups until the chip is covered, instead of thinning the workgroups to one MFMA wave each (r2: 3.4 % MFMA busy at the 0.8B shape).
+    // The shortest shares that the CUs hold, a workgroup each, are the best: of 2043 rows of 8 heads of 256 two shares of every
+    // group took 98.7 us, the last group's being twice the average, one to three shares 77.5; of 517 rows eight shares 24.2, up to nine 18.5.
     uint32_t tpw = 4, splits = 1;
     float* part = nullptr;
-    const uint32_t groups4 = kv_heads * ((n_tasks + 3) / 4);
-    const uint32_t max_tiles = (a.sequence_length + TK - 1) / TK; // (host view: without the device-side dyn term -- only bounds the split count)
-    if (force_split != 1 && groups4 < 192) { // (a.dyn: the context length joins on the device -- the tile count here is a lower bound, a split may come up empty)
-        splits = (256 + groups4 - 1) / groups4;
-        if (force_split > 1) splits = (uint32_t)force_split;
-        if (splits > kMaxKeySplits) splits = kMaxKeySplits;
-        while (splits > 1 && max_tiles / splits < 2) --splits;
-        if (splits > 1) {
-            const size_t rows = (size_t)a.suffix_length * a.num_heads;
-            part = (float*)stream_workspace(s, (size_t)splits * rows * (a.head_dim + 2) * sizeof(float)); // null while a graph is being captured
-            if (!part) splits = 1;
+    KeyShares shares{0, prefix};
+    const uint32_t groups4 = kv_heads * ((n_tasks + 3) / 4), stretch = a.head_dim <= 128 ? 2 * TK : TK;
+    const size_t rows = (size_t)a.suffix_length * a.num_heads;
+    uint32_t units = 0;
+    if (force_split != 1 && groups4 < 192) {
+        const uint32_t n_groups = (n_tasks + 3) / 4;
+        uint64_t all = 0;
+        for (uint32_t y = 0; y < n_groups; ++y) all += key_stretches(shares, y, tpw, a.gqa_factor, a.suffix_length, stretch);
+        // 64 keys a share at least, and no more shares than there can be
+        shares.quantum = std::max({2 * TK / stretch, (uint32_t)(kv_heads * all / 256), key_stretches(shares, n_groups - 1, tpw, a.gqa_factor, a.suffix_length, stretch) / kMaxKeySplits});
+        for (;; ++shares.quantum) {
+            units = 0, splits = 1;
+            for (uint32_t y = 0; y < n_groups; ++y) {
+                const uint32_t n = key_shares(shares, y, tpw, a.gqa_factor, a.suffix_length, stretch);
+                units += n, splits = std::max(splits, n);
+            }
+            if (splits == 1 || kv_heads * units <= 256) break;
         }
+        if (splits > 1) part = (float*)stream_workspace(s, (size_t)splits * rows * (a.head_dim + 2) * sizeof(float)); // null while a graph is being captured
+        if (!part) splits = 1;
     }
     if (splits == 1) { // fewer tasks per workgroup until the grid covers most of the chip
+        shares.quantum = 0;
         while (tpw > 1 && kv_heads * ((n_tasks + tpw - 1) / tpw) < 192) tpw >>= 1;
+        if (force_tpw == 1 || force_tpw == 2 || force_tpw == 4) tpw = force_tpw;
     }
-    if (force_tpw == 1 || force_tpw == 2 || force_tpw == 4) tpw = force_tpw;
-    const dim3 grid(kv_heads, (n_tasks + tpw - 1) / tpw, splits);
-    const size_t rows = (size_t)a.suffix_length * a.num_heads;
+    const dim3 grid(kv_heads, splits > 1 ? units : (n_tasks + tpw - 1) / tpw);
     float* part_o = part;
     float* part_ml = part ? part + (size_t)splits * rows * a.head_dim : nullptr;
     const bool general = a.sinks || a.is_sliding_window || a.is_kv_cache_ring;
 #define UZU_LAUNCH(H)                                                                                                                                              \
     {                                                                                                                                                              \
         UZU_PROPAGATE(launch_check([&] {                                                                                                                           \
-            if (general) hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, true>), grid, dim3(H <= 128 ? 512 : 256), 0, s, a, (uint16_t*)out, tpw, part_o, part_ml, 0u);             \
-            else hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, false>), grid, dim3(H <= 128 ? 512 : 256), 0, s, a, (uint16_t*)out, tpw, part_o, part_ml, 0u);                    \
+            if (general) hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, true>), grid, dim3(H <= 128 ? 512 : 256), 0, s, a, (uint16_t*)out, tpw, part_o, part_ml, shares);         \
+            else hipLaunchKernelGGL((attention_prefill_mfma_kernel<H, false>), grid, dim3(H <= 128 ? 512 : 256), 0, s, a, (uint16_t*)out, tpw, part_o, part_ml, shares);                \
         }, "attention_prefill_mfma"));                                                                                                                             \
         if (!part) return UZU_OK;                                                                                                                                  \
         if (gate && gate_done) *gate_done = 1;                                                                                                                     \
-        return launch_check([&] { hipLaunchKernelGGL(attention_prefill_merge_kernel<H>, dim3((uint32_t)((rows + 3) / 4)), dim3(256), 0, s, part_o, part_ml, (uint16_t*)out, (uint32_t)rows, splits, gate_done ? (const uint16_t*)gate : nullptr); }, \
+        return launch_check([&] { hipLaunchKernelGGL(attention_prefill_merge_kernel<H>, dim3((uint32_t)((rows + 3) / 4)), dim3(256), 0, s, part_o, part_ml, (uint16_t*)out, (uint32_t)rows, shares, tpw, a.gqa_factor, a.num_heads, gate_done ? (const uint16_t*)gate : nullptr); }, \
                             "attention_prefill_merge");                                                                                                            \
     }
     switch (a.head_dim) {
