@@ -96,6 +96,25 @@ def test_attention_simple_form_true_f32(hip_ctx, H, G, dim, vd, window, cap, T, 
     assert np.abs(got - want).max() < 2e-5 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("H,G,dim,vd,window,cap,T,start", [(4, 2, 64, 64, 0, 0.0, 16, 0), (3, 1, 128, 64, 21, 4.0, 35, 2), (8, 2, 64, 128, 70, 0.0, 300, 3), (2, 2, 128, 128, 0, 0.0, 129, 97),
+                                                          (4, 1, 128, 128, 1, 0.0, 50, 17), (2, 1, 64, 64, 400, 30.0, 700, 260)])
+def test_attention_of_f32_rows_on_the_matrix_cores(hip_ctx, H, G, dim, vd, window, cap, T, start):
+    """Caches of f32 rows, sixteen rows and more (k_window_attention_f32.hip): tiles of rows that are full, ragged and a single row long, blocks of keys in front of a window, of one key,
+    fewer blocks than waves; the bound of the simple form, and the rows' independence of what else is in a pass: a pass that starts later gives its rows the same bits."""
+    rng = np.random.default_rng(H * 100 + T + dim)
+    q, K, V = qkv(rng, T, H, G, dim, vd)
+    mx = {"heads": H, "kv_heads": G, "scale": 1.7 / np.sqrt(dim), "mask": {"size": window}, "softcap": cap}
+    for sinks in ("unit", None):
+        got = attention(hip_ctx, q[start:], K, V, mx, start, sinks=sinks)
+        simple = attention(hip_ctx, q[start:], K, V, mx, start, sinks=sinks, form=1)
+        assert np.abs(got - simple).max() < 2e-5 * np.abs(simple).max()
+    want = O.attention_core(f32(q)[start:], f32(K), f32(V), mx, start)
+    got = attention(hip_ctx, q[start:], K, V, mx, start)
+    assert np.abs(got - want).max() < 2e-5 * np.abs(want).max()
+    if T - start > 24:
+        assert np.array_equal(attention(hip_ctx, q[start + 7:], K, V, mx, start + 7), got[7:])
+
+
 @pytest.mark.parametrize("H,G,dim,vd,window,cap,T,start", [c for c in CASES if c[2] % 8 == 0 and c[3] % 8 == 0] + MANY_TILES)
 def test_attention_matrix_core_form_equals_the_simple_form(hip_ctx, H, G, dim, vd, window, cap, T, start):
     rng = np.random.default_rng(H * 100 + T + 1)

@@ -297,6 +297,8 @@ uzu_status conv_rope_append(hipStream_t s, const RopeAppendParams& p, const Caus
 }
 
 uzu_status window_attention_mfma(hipStream_t s, const WindowAttentionParams& p); // k_window_attention_mfma.hip
+bool window_attention_f32_supported(const WindowAttentionParams& p);            // k_window_attention_f32.hip
+uzu_status window_attention_f32(hipStream_t s, const WindowAttentionParams& p);
 
 uzu_status window_attention(hipStream_t s, const WindowAttentionParams& params) {
     WindowAttentionParams p = params;
@@ -316,6 +318,7 @@ uzu_status window_attention(hipStream_t s, const WindowAttentionParams& params) 
         UZU_UNSUPPORTED(!window_attention_mfma_supported(p), "window_attention: the matrix-core form does not take this shape");
         return window_attention_mfma(s, p);
     }
+    if (p.form == 0 && window_attention_f32_supported(p)) return window_attention_f32(s, p); // (sixteen rows a sequence and more, as the bf16 caches' form)
     UZU_REQUIRE(p.heads <= 65535, "window_attention: too many heads for one launch");
     return launch_check([&] { hipLaunchKernelGGL(window_attention_simple_kernel, dim3(p.rows, p.heads), dim3(64), (size_t)(p.dim + 64) * 4, s, p); }, "window_attention");
 }
