@@ -62,23 +62,24 @@ __device__ __forceinline__ float quad_sum(float v) {
     v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, true)); // quad_perm [2, 3, 0, 1]
     return v;
 }
-// four neighbouring floats of a row, those from `left` on zero; aligned: one 16-byte load (the host has checked pitch, columns and widths)
-__device__ __forceinline__ f32x4_m load4(const float* at, uint32_t left, bool aligned) {
-    f32x4_m v{0.f, 0.f, 0.f, 0.f};
-    if (aligned) {
-        if (left) v = *(const f32x4_m*)at;
-    } else {
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u)
-            if (u < left) v[u] = at[u];
-    }
-    return v;
+// Loads of a chunk's rows and states: buffer loads, whose lanes past a bound read zero without a branch, and which want words aligned and no more: a body of branches for every load was half
+// of these kernels' code, and a launch of some twenty microseconds reads its code from memory as it goes.  With it and the products' operands in front of them, `out` of 5 chunks of 16 heads
+// of 128 x 64: 23 us -> 16, of 34 chunks of 32: 72 -> 59; a decay per channel, 128 x 128: 38 -> 32, 92 -> 79.  (The carried state a slab ahead: 70.)
+constexpr uint32_t kNowhere = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_from(const float* base) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, 0x7FFFFFFF, 0x00027000); }
+__device__ __forceinline__ float load1(__amdgpu_buffer_rsrc_t rows, uint32_t index, bool in) {
+    return __builtin_bit_cast(float, (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rows, in ? index * 4 : kNowhere, 0, 0));
+}
+// four neighbouring floats of a row, those from `left` on zero; FOURS: `left` is a multiple of four
+template <bool FOURS> __device__ __forceinline__ f32x4_m load4(__amdgpu_buffer_rsrc_t rows, uint32_t index, uint32_t left) {
+    if constexpr (FOURS) return __builtin_bit_cast(f32x4_m, __builtin_amdgcn_raw_buffer_load_b128(rows, left ? index * 4 : kNowhere, 0, 0));
+    else return f32x4_m{load1(rows, index, left > 0), load1(rows, index + 1, left > 1), load1(rows, index + 2, left > 2), load1(rows, index + 3, left > 3)};
 }
 
 // a workgroup per (chunk, head, tile of 64 key channels x 64 NQ value columns): v_mfma_f32_32x32x2_f32, lane l feeds A[l % 32][k = l / 32], B[k = l / 32][l % 32] and
 // holds rows 8 (r / 4) + 4 (l / 32) + r % 4 of column l % 32
-template <bool CHANNEL, int NQ>
-__global__ void __launch_bounds__(256) decayed_state_local_kernel(DecayedStateParams p, float* ws, uint32_t aligned) {
+template <bool CHANNEL, int NQ, bool FOURS>
+__global__ void __launch_bounds__(256) decayed_state_local_kernel(DecayedStateParams p, float* ws) {
     constexpr uint32_t KW = 64, VW = 64 * NQ;
     __shared__ __attribute__((aligned(16))) float s_k[kChunk][KW], s_v[kChunk][VW];
     __shared__ float s_tot[4][KW]; // a decay per channel: a block's whole decay
@@ -92,23 +93,24 @@ __global__ void __launch_bounds__(256) decayed_state_local_kernel(DecayedStatePa
     // thread = (channel i of the tile, block b of 16 rows): its keys (and decays) in registers, every load in front of the first use
     const uint32_t i = lane, b = wave;
     const bool in = i0 + i < p.dim;
-    const float* kcol = p.rows_in + (size_t)r0 * p.ld + p.k_col + (size_t)g * p.dim + i0 + i;
+    const auto k_rows = rows_from(p.rows_in + (size_t)r0 * p.ld + p.k_col + (size_t)g * p.dim + i0);
+    const auto e_rows = rows_from(CHANNEL ? p.decay + (size_t)r0 * p.lddecay + (size_t)a * p.dim + i0 : p.rows_in);
     float key[kBlock], dec[CHANNEL ? kBlock : 1];
 #pragma unroll
     for (uint32_t t = 0; t < kBlock; ++t) {
         const uint32_t row = b * kBlock + t;
-        key[t] = row < n && in ? kcol[(size_t)row * p.ld] : 0.0f;
-        if (CHANNEL) dec[CHANNEL ? t : 0] = row < n && in ? p.decay[(size_t)(r0 + row) * p.lddecay + (size_t)a * p.dim + i0 + i] : 0.0f;
+        key[t] = load1(k_rows, row * p.ld + i, row < n && in);
+        if (CHANNEL) dec[CHANNEL ? t : 0] = load1(e_rows, row * p.lddecay + i, row < n && in);
     }
     {   // values: thread = (rows tid / (16 NQ) + .., four columns)
         constexpr uint32_t TPR = 16 * NQ, RPP = 256 / TPR;
         const uint32_t col = (tid % TPR) * 4, left = j0 + col < p.vdim ? p.vdim - j0 - col : 0;
-        const float* vb = p.rows_in + (size_t)r0 * p.ld + p.v_col + (size_t)a * p.vdim + j0 + col;
+        const auto v_rows = rows_from(p.rows_in + (size_t)r0 * p.ld + p.v_col + (size_t)a * p.vdim + j0);
         f32x4_m v[kChunk / RPP];
 #pragma unroll
         for (uint32_t u = 0; u < kChunk / RPP; ++u) {
             const uint32_t t = tid / TPR + u * RPP;
-            v[u] = load4(vb + (size_t)t * p.ld, t < n ? left : 0, aligned);
+            v[u] = load4<FOURS>(v_rows, t * p.ld + col, t < n ? left : 0);
         }
 #pragma unroll
         for (uint32_t u = 0; u < kChunk / RPP; ++u) *(f32x4_m*)&s_v[tid / TPR + u * RPP][col] = v[u];
@@ -203,8 +205,8 @@ template <bool CHANNEL> __global__ void __launch_bounds__(256) decayed_state_sca
 // worked on, the carried state's rows go from memory straight into the products.  One decay per head: scores as two 32 x 32 tiles per wave row, times a table of decays.
 // A decay per channel: a wave owns the block of 16 x 16 scores on the diagonal that bears its number (running products, lane = (key row, quarter of the slab)) and up to
 // two of the six blocks below it (v_mfma_f32_16x16x4_f32).  Results: wave w has rows 32 (w / 2) .., column tiles NQ (w % 2) ..
-template <bool CHANNEL, int NQ>
-__global__ void __launch_bounds__(256, CHANNEL ? 2 : 3) decayed_state_out_kernel(DecayedStateParams p, const float* ws, uint32_t aligned) {
+template <bool CHANNEL, int NQ, bool FOURS>
+__global__ void __launch_bounds__(256, CHANNEL || NQ > 1 ? 2 : 3) decayed_state_out_kernel(DecayedStateParams p, const float* ws) {
     constexpr uint32_t SW = 32, PW = SW + 4, VW = 64 * NQ, ROWS = kChunk * PW; // a slab row's pitch: 16-byte aligned, rows on distinct banks
     constexpr uint32_t BUF = CHANNEL ? 5 * ROWS : 2 * ROWS;
     __shared__ __attribute__((aligned(16))) float s_buf[BUF > kChunk * VW ? BUF : kChunk * VW];
@@ -213,12 +215,12 @@ __global__ void __launch_bounds__(256, CHANNEL ? 2 : 3) decayed_state_out_kernel
     uint32_t z, c;
     SeqSpan sp;
     if (!find_chunk(p, blockIdx.x, z, c, sp)) return;
-    const uint32_t a = blockIdx.y, g = a / (p.heads / p.groups), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, half = lane >> 5, l16 = lane & 15, quarter = lane >> 4;
+    const uint32_t a = blockIdx.y, g = a / (p.heads / p.groups), tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(CHANNEL ? tid >> 6 : ((tid >> 6) + blockIdx.x) & 3), l32 = lane & 31, half = lane >> 5, l16 = lane & 15, quarter = lane >> 4;
     const uint32_t j0 = blockIdx.z * VW, dim = p.dim, vdim = p.vdim;
     const uint32_t r0 = sp.row0 + c * kChunk, n = sp.count - c * kChunk < kChunk ? sp.count - c * kChunk : kChunk;
     const float* base = p.rows_in + (size_t)r0 * p.ld;
-    const float *qb = base + p.q_col + (size_t)g * dim, *kb = base + p.k_col + (size_t)g * dim, *eb = p.decay + (size_t)r0 * p.lddecay + (size_t)a * dim;
-    const float* S = ws + ((size_t)blockIdx.x * p.heads + a) * dim * vdim + j0;
+    const auto q_rows = rows_from(base + p.q_col + (size_t)g * dim), k_rows = rows_from(base + p.k_col + (size_t)g * dim);
+    const auto e_rows = rows_from(CHANNEL ? p.decay + (size_t)r0 * p.lddecay + (size_t)a * dim : base), S = rows_from(ws + ((size_t)blockIdx.x * p.heads + a) * dim * vdim + j0);
     float *s_q = s_buf, *s_k = s_buf + ROWS;
     float *s_e = s_buf + 2 * ROWS, *s_qd = s_buf + 3 * ROWS, *s_kd = s_buf + 4 * ROWS; // a decay per channel: decays; queries decayed from their block's start; keys decayed to its end
     const uint32_t pi = wave >> 1, pj = wave & 1;
@@ -231,15 +233,14 @@ __global__ void __launch_bounds__(256, CHANNEL ? 2 : 3) decayed_state_out_kernel
 #pragma unroll
         for (uint32_t u = 0; u < 2; ++u) {
             const uint32_t r = lr + 32 * u, m = r < n ? left : 0;
-            fq[u] = load4(qb + (size_t)r * p.ld + d0 + lc, m, aligned);
-            fk[u] = load4(kb + (size_t)r * p.ld + d0 + lc, m, aligned);
-            if (CHANNEL) fe[CHANNEL ? u : 0] = load4(eb + (size_t)r * p.lddecay + d0 + lc, m, aligned);
+            fq[u] = load4<FOURS>(q_rows, r * p.ld + d0 + lc, m);
+            fk[u] = load4<FOURS>(k_rows, r * p.ld + d0 + lc, m);
+            if (CHANNEL) fe[CHANNEL ? u : 0] = load4<FOURS>(e_rows, r * p.lddecay + d0 + lc, m);
         }
     };
     fetch(0);
     if (!CHANNEL) {
-        for (uint32_t e = tid; e < kChunk * (kChunk + 1); e += 256) (&s_p[0][0])[e] = 0.0f;
-        if (wave == 0) {
+        if (tid < 64) {
             const float dt = lane < n ? head_step(p, r0 + lane, a) : 0.0f, e = -expf(p.a_log[a]) * dt;
             float upto = e, behind = __shfl_down(e, 1, 16); // inside the row's block of 16
             behind = l16 < 15 ? behind : 0.0f;
@@ -260,20 +261,19 @@ __global__ void __launch_bounds__(256, CHANNEL ? 2 : 3) decayed_state_out_kernel
         }
         __syncthreads();
         // thread = (key row j, block of 16 query rows): step_j e^(the log decays of rows j + 1 .. i)
-        const uint32_t j = lane, b = wave, jb = j / kBlock;
+        const uint32_t j = lane, b = tid >> 6, jb = j / kBlock; // zero above the diagonal and beyond the chunk's rows
         const float dt = s_h[1][j];
+        float sum = 0.0f;
         if (b > jb) {
-            float sum = s_h[4][j];
+            sum = s_h[4][j];
             for (uint32_t o = jb + 1; o < b; ++o) sum += s_h[5][o];
+        }
 #pragma unroll 4
-            for (uint32_t i = b * kBlock; i < b * kBlock + kBlock; ++i) s_p[i][j] = i < n ? expf(sum + s_h[3][i]) * dt : 0.0f;
-        } else if (b == jb) {
-            float sum = 0.0f;
-#pragma unroll 4
-            for (uint32_t i = b * kBlock; i < b * kBlock + kBlock; ++i) {
-                sum += i > j ? s_h[0][i] : 0.0f;
-                if (i >= j) s_p[i][j] = i < n ? expf(sum) * dt : 0.0f;
-            }
+        for (uint32_t i = b * kBlock; i < b * kBlock + kBlock; ++i) {
+            const float own = s_h[0][i], upto = s_h[3][i];
+            if (b == jb) sum += i > j ? own : 0.0f;
+            const float w = expf(b == jb ? sum : sum + upto) * dt;
+            s_p[i][j] = i >= j && i < n ? w : 0.0f;
         }
     } else {
         for (uint32_t e = tid; e < kChunk * (kChunk + 1); e += 256) (&s_p[0][0])[e] = 0.0f;
@@ -297,10 +297,10 @@ __global__ void __launch_bounds__(256, CHANNEL ? 2 : 3) decayed_state_out_kernel
         for (uint32_t d = 0; d < SW / 2; ++d)
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
-                const uint32_t dg = d0 + 2 * d + half, col = pj * 32 * NQ + 32 * q + l32;
-                sv[d][q] = carried && dg < dim && j0 + col < vdim ? S[(size_t)dg * vdim + col] : 0.0f;
+                const uint32_t dg = d0 + 16 * half + d, col = pj * 32 * NQ + 32 * q + l32;
+                sv[d][q] = load1(S, dg * vdim + col, carried && dg < dim && j0 + col < vdim);
             }
-        __syncthreads(); // the slab before has been read
+        lds_barrier(); // the slab before has been read
 #pragma unroll
         for (uint32_t u = 0; u < 2; ++u) {
             const uint32_t at = (lr + 32 * u) * PW + lc;
@@ -313,7 +313,7 @@ __global__ void __launch_bounds__(256, CHANNEL ? 2 : 3) decayed_state_out_kernel
                 *(f32x4_m*)(s_e + at) = e;
             }
         }
-        __syncthreads();
+        lds_barrier();
         if (d0 + SW < dim) fetch(d0 + SW);
         if (CHANNEL) { // thread = (channel, block, direction): running products onto the queries from the block's start, onto the keys from its end
             const uint32_t dd = tid & 31, first = ((tid >> 5) & 3) * kBlock;
@@ -370,7 +370,7 @@ __global__ void __launch_bounds__(256, CHANNEL ? 2 : 3) decayed_state_out_kernel
                 const uint32_t rb = row / kBlock;
 #pragma unroll
                 for (uint32_t d = 0; d < SW / 2; ++d) {
-                    const uint32_t dl = 2 * d + half;
+                    const uint32_t dl = 16 * half + d;
                     float qa = s_qd[row * PW + dl];
                     const float t0 = s_tot[0][dl], t1 = s_tot[1][dl], t2 = s_tot[2][dl];
                     qa *= rb > 0 ? t0 : 1.0f;
@@ -383,14 +383,20 @@ __global__ void __launch_bounds__(256, CHANNEL ? 2 : 3) decayed_state_out_kernel
             }
         } else {
             if (d0 == 0) from_start = s_h[2][row];
+            // (both operands out of LDS before the first product, and one condition around all of them)
+            f32x4_m qv[SW / 8], kv[SW / 8];
 #pragma unroll
-            for (uint32_t d = 0; d < SW / 2; ++d) {
-                const float qv = s_q[row * PW + 2 * d + half];
-                sc = __builtin_amdgcn_mfma_f32_32x32x2f32(qv, s_k[(pj * 32 + l32) * PW + 2 * d + half], sc, 0, 0, 0);
-                if (carried) {
+            for (uint32_t d = 0; d < SW / 8; ++d) qv[d] = *(const f32x4_m*)(s_q + row * PW + 16 * half + 4 * d), kv[d] = *(const f32x4_m*)(s_k + (pj * 32 + l32) * PW + 16 * half + 4 * d);
+            __builtin_amdgcn_sched_barrier(0);
+            if (pj <= pi) { // (the tile above the diagonal is nobody's)
 #pragma unroll
-                    for (int q = 0; q < NQ; ++q) o[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(qv * from_start, sv[d][q], o[q], 0, 0, 0);
-                }
+                for (uint32_t d = 0; d < SW / 2; ++d) sc = __builtin_amdgcn_mfma_f32_32x32x2f32(qv[d / 4][d % 4], kv[d / 4][d % 4], sc, 0, 0, 0);
+            }
+            if (carried) {
+#pragma unroll
+                for (uint32_t d = 0; d < SW / 2; ++d)
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) o[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(qv[d / 4][d % 4] * from_start, sv[d][q], o[q], 0, 0, 0);
             }
         }
     }
@@ -414,33 +420,42 @@ __global__ void __launch_bounds__(256, CHANNEL ? 2 : 3) decayed_state_out_kernel
     {
         constexpr uint32_t TPR = 16 * NQ, RPP = 256 / TPR;
         const uint32_t col = (tid % TPR) * 4, left = j0 + col < vdim ? vdim - j0 - col : 0;
-        const float* vb = base + p.v_col + (size_t)a * vdim + j0 + col;
+        const auto v_rows = rows_from(base + p.v_col + (size_t)a * vdim + j0);
+        f32x4_m v[kChunk / RPP];
 #pragma unroll
-        for (uint32_t u = 0; u < kChunk / RPP; ++u) {
-            const uint32_t t = tid / TPR + u * RPP;
-            *(f32x4_m*)(s_v + t * VW + col) = load4(vb + (size_t)t * p.ld, t < n ? left : 0, aligned);
-        }
+        for (uint32_t u = 0; u < kChunk / RPP; ++u) v[u] = load4<FOURS>(v_rows, (tid / TPR + u * RPP) * p.ld + col, tid / TPR + u * RPP < n ? left : 0);
+#pragma unroll
+        for (uint32_t u = 0; u < kChunk / RPP; ++u) *(f32x4_m*)(s_v + (tid / TPR + u * RPP) * VW + col) = v[u];
     }
     __syncthreads();
     if (!out_on) return;
     const uint32_t last = n < pi * 32 + 32 ? n : pi * 32 + 32; // keys up to this half's last row (beyond the chunk's rows: zero scores and values)
-    for (uint32_t t0 = 0; t0 < last; t0 += 8)
+    for (uint32_t t0 = 0; t0 < last; t0 += 16) {
+        float pa[8], va[8][NQ];
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
+        for (uint32_t u = 0; u < 8; ++u) {
             const uint32_t t = t0 + 2 * u + half;
-            const float pa = s_p[row][t];
+            pa[u] = s_p[row][t];
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) o[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(pa, s_v[t * VW + pj * 32 * NQ + 32 * q + l32], o[q], 0, 0, 0);
+            for (int q = 0; q < NQ; ++q) va[u][q] = s_v[t * VW + pj * 32 * NQ + 32 * q + l32];
         }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u)
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) o[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(pa[u], va[u][q], o[q], 0, 0, 0);
+    }
     const float skip = p.skip ? p.skip[a] : 0.0f;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         const uint32_t col = pj * 32 * NQ + 32 * q + l32;
         if (j0 + col >= vdim) continue;
+        float* out = p.out + ((size_t)r0 * p.heads + a) * vdim + j0 + col;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const uint32_t i = pi * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-            if (i < n) p.out[((size_t)(r0 + i) * p.heads + a) * vdim + j0 + col] = p.skip ? fmaf(skip, s_v[i * VW + col], o[q][r]) : o[q][r];
+            const float v = p.skip ? fmaf(skip, s_v[i * VW + col], o[q][r]) : o[q][r];
+            if (i < n) out[(size_t)i * p.heads * vdim] = v;
         }
     }
 }
@@ -460,23 +475,28 @@ uzu_status decayed_state(hipStream_t s, const DecayedStateParams& p) {
     if (p.form == 2 || (p.form == 0 && p.chunk_ws && p.rows > 16 * p.nseq)) { // prompt-sized: in chunks
         UZU_REQUIRE(p.chunk_ws && p.chunks && p.chunk_ws_bytes >= decayed_state_chunk_ws_bytes(p.chunks, p.heads, p.dim, p.vdim), "decayed_state: the chunked form needs its workspace");
         const uint32_t vw = p.vdim <= 64 ? 64 : 128, vt = (p.vdim + vw - 1) / vw, kt = (p.dim + 63) / 64;
-        const uint32_t aligned = p.ld % 4 == 0 && p.q_col % 4 == 0 && p.k_col % 4 == 0 && p.v_col % 4 == 0 && p.dim % 4 == 0 && p.vdim % 4 == 0 && (uintptr_t)p.rows_in % 16 == 0 &&
-                                 (p.per_head || (p.lddecay % 4 == 0 && (uintptr_t)p.decay % 16 == 0)) ? 1u : 0u;
+        const bool fours = p.dim % 4 == 0 && p.vdim % 4 == 0;
+        // (a chunk's rows and a head's state within the 2 GiB that a buffer's offsets span)
+        UZU_UNSUPPORTED((size_t)kChunk * p.ld >= 0x18000000u || (size_t)kChunk * p.lddecay >= 0x18000000u, "decayed_state: rows of pitch %u / %u", p.ld, p.lddecay);
         UZU_REQUIRE((size_t)vt * kt <= 65535 && ((size_t)p.dim * p.vdim + 255) / 256 <= 65535, "decayed_state: head widths %u x %u", p.dim, p.vdim);
         const dim3 lgrid(p.chunks, p.heads, vt * kt), sgrid(p.nseq, p.heads, (uint32_t)(((size_t)p.dim * p.vdim + 255) / 256)), ogrid(p.chunks, p.heads, vt);
         float* ws = p.chunk_ws;
-#define UZU_DC(CH, NQ)                                                                                                                                                             \
+#define UZU_DC(CH, NQ, FOURS)                                                                                                                                                      \
     do {                                                                                                                                                                           \
-        UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL((decayed_state_local_kernel<CH, NQ>), lgrid, dim3(256), 0, s, p, ws, aligned); }, "decayed_state_local"));             \
+        UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL((decayed_state_local_kernel<CH, NQ, FOURS>), lgrid, dim3(256), 0, s, p, ws); }, "decayed_state_local"));               \
         UZU_PROPAGATE(launch_check([&] { hipLaunchKernelGGL(decayed_state_scan_kernel<CH>, sgrid, dim3(256), 0, s, p, ws); }, "decayed_state_scan"));                              \
-        return launch_check([&] { hipLaunchKernelGGL((decayed_state_out_kernel<CH, NQ>), ogrid, dim3(256), 0, s, p, (const float*)ws, aligned); }, "decayed_state_out");           \
+        return launch_check([&] { hipLaunchKernelGGL((decayed_state_out_kernel<CH, NQ, FOURS>), ogrid, dim3(256), 0, s, p, (const float*)ws); }, "decayed_state_out");             \
     } while (0)
         if (p.per_head) {
-            if (vw == 64) UZU_DC(false, 1);
-            UZU_DC(false, 2);
+            if (vw == 64 && fours) UZU_DC(false, 1, true);
+            if (vw == 64) UZU_DC(false, 1, false);
+            if (fours) UZU_DC(false, 2, true);
+            UZU_DC(false, 2, false);
         }
-        if (vw == 64) UZU_DC(true, 1);
-        UZU_DC(true, 2);
+        if (vw == 64 && fours) UZU_DC(true, 1, true);
+        if (vw == 64) UZU_DC(true, 1, false);
+        if (fours) UZU_DC(true, 2, true);
+        UZU_DC(true, 2, false);
 #undef UZU_DC
     }
     const dim3 grid(p.nseq * p.heads, (p.vdim + 15) / 16);
