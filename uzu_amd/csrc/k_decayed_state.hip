@@ -62,9 +62,9 @@ __device__ __forceinline__ float quad_sum(float v) {
     v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, true)); // quad_perm [2, 3, 0, 1]
     return v;
 }
-// Loads of a chunk's rows and states: buffer loads, whose lanes past a bound read zero without a branch, and which want words aligned and no more: a body of branches for every load was half
-// of these kernels' code, and a launch of some twenty microseconds reads its code from memory as it goes.  With it and the products' operands in front of them, `out` of 5 chunks of 16 heads
-// of 128 x 64: 23 us -> 16, of 34 chunks of 32: 72 -> 59; a decay per channel, 128 x 128: 38 -> 32, 92 -> 79.  (The carried state a slab ahead: 70.)
+// Loads of a chunk's rows and states: buffer loads, whose lanes past a bound read zero without a branch, and which want words aligned and no more (one path where there were two).
+// With them and the products' operands read in front of the first product, under one condition for all of them, `out` of 5 chunks of 16 heads of 128 x 64: 23 us -> 16, of 34 chunks of 32:
+// 72 -> 59; a decay per channel, 128 x 128: 38 -> 32, 92 -> 79.  (The loads alone changed nothing; the carried state a slab ahead besides: 70.)
 constexpr uint32_t kNowhere = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_from(const float* base) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, 0x7FFFFFFF, 0x00027000); }
 __device__ __forceinline__ float load1(__amdgpu_buffer_rsrc_t rows, uint32_t index, bool in) {

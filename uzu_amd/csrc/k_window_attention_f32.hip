@@ -7,8 +7,8 @@
 //   results  O^T = V^T P^T: step s takes the keys 4 (lane / 16) + s, whose weights are the lane's own registers; the queries stay where they are
 // Keys and values go from memory into the operands' registers, a wave's next ones while it works.  A block's number counts from position 0, and a key that a row does not see has weight 0: a row's
 // sums do not depend on what else is in its tile or its pass.
-// 300 rows of 8 heads of 128: 44.7 us by the simple form, 15.3 here.  (Half of a first version's 29.5 were its code: a launch this short reads it from memory as it goes, so there is one body of
-// the loop, no second path for addresses of four bytes' alignment, which the loads take as they are, and the cap on the scores is an instance of its own.)
+// 300 rows of 8 heads of 128: 44.7 us by the simple form, 15.3 here.  (29.5 with a branch around every load for caches of four bytes' alignment, which the loads take as they are, and with the
+// values, too, a step ahead, which spilled.)
 #include "device_utils.h"
 #include "kernels_stream32.h"
 
@@ -19,7 +19,7 @@ namespace {
 constexpr uint32_t kRows = 16, kKeys = 16, kWaves = 8;
 
 // grid (row tiles at most, heads), 512 threads.  DG: key width / 16; VH: value width / 64
-// EXTRA: a cap on the scores or a bias by distance (their code, unrolled, is as long as everything else, and a launch of microseconds reads its code from memory)
+// EXTRA: a cap on the scores or a bias by distance (an instance of its own: the plain one has no branch between the products)
 template <int DG, int VH, bool EXTRA>
 __global__ void __launch_bounds__(64 * kWaves) window_attention_f32_kernel(WindowAttentionParams p) {
     constexpr int DIM = 16 * DG, VD = 64 * VH, OP = VD + 4;
