@@ -104,7 +104,7 @@ __global__ void __launch_bounds__(256, 2) gemm_rows_kernel(GemmRowsParams p) {
         gm_u32x4 codes[NB], xv[MT][4];
     };
     auto load_step = [&](uint32_t s, Step& st) {
-        const uint32_t c = min(s, G - 1); // (past the end: a reload that is never consumed)
+        const uint32_t c = min(s, G - 1); // (a wave without steps)
 #pragma unroll
         for (int b = 0; b < NB; ++b) st.codes[b] = *(const gm_u32x4*)(p.w + (size_t)wrow[b] * half_k + 16 * g + (size_t)c * 64);
 #pragma unroll
@@ -180,11 +180,13 @@ __global__ void __launch_bounds__(256, 2) gemm_rows_kernel(GemmRowsParams p) {
             of1[b] = offset_of(sc1[b], zp ? (float)((of2[b] >> 4) & 15u) : bits_to_f32(of2[b] & 0xFFFF0000u));
             sc0[b] *= 16.0f, sc1[b] *= 16.0f;
         }
-        load_scales(s + 2);
+        // (a wave of four has two steps of K = 1024: reloads past its end, though nobody waited for them, were a third of what it asked of the L2.  37 rows: 8224 x 1024 11.2 us -> 8.8, 7168 x 1024
+        // + GatedActMul 9.3 -> 8.4, 3072 x 1024 7.0 -> 5.6, 1024 x 2048 and x 3584 in four shares 5.6 -> 5.1)
+        if (s + 2 < s_hi) load_scales(s + 2);
         __builtin_amdgcn_sched_barrier(0); // (left alone, the scheduler sinks the loads to their uses and waits for each)
         compute(stA, sc0, of0);
         __builtin_amdgcn_sched_barrier(0);
-        load_step(s + 2, stA);
+        if (s + 2 < s_hi) load_step(s + 2, stA);
         __builtin_amdgcn_sched_barrier(0);
         compute(stB, sc1, of1);
         __builtin_amdgcn_sched_barrier(0);
