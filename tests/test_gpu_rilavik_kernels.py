@@ -180,3 +180,15 @@ def test_gated_norm_in_parts(hip_ctx, shape):
     _ffi.call("uzu_hip_s32_gated_norm", hip_ctx._h, ptr(y), ptr(g), ptr(w), ptr(out), f32c(1e-4), f32c(0.7), u32(rows), u32(width), u32(parts))
     want = 0.7 * O.rms_norm_in_parts(y.astype(np.float64) * O.silu(g.astype(np.float64)), w.astype(np.float64), parts, 1e-4)
     assert np.abs(out - want).max() < 3e-6 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("form", [0, 2])
+@pytest.mark.parametrize("pitch", [(1 << 29) // 64 * 3 // 4 - 1, (1 << 29) // 64 * 3 // 4])
+def test_decayed_state_of_far_apart_rows(hip_ctx, pitch, form):
+    """The last pitch whose rows of a chunk lie within a buffer's offsets, and the first beyond, which goes token by token."""
+    rng, T, H, dim, vd = np.random.default_rng(53), 17, 2, 24, 20
+    q, k, pre, v = rng.standard_normal((T, H, dim)), rng.standard_normal((T, H, dim)), rng.standard_normal((T, H, dim)), rng.standard_normal((T, H, vd))
+    q, k, pre, v, state = (f32(x).astype(np.float64) for x in (q, k, pre, v, rng.standard_normal((H, dim, vd))))
+    want, S = want_channel(q, k, v, pre, 16.0, state)
+    got, st = channel_state(hip_ctx, q, k, v, pre, 16.0, state, 5, form, pad=pitch - 2 * H * dim - H * vd)
+    assert close(got, want) and close(st, S)

@@ -472,12 +472,12 @@ uzu_status decayed_state(hipStream_t s, const DecayedStateParams& p) {
     UZU_REQUIRE(p.per_head ? (p.a_log && p.dt_bias) : p.inv_temperature > 0.0f, "decayed_state: the decays' constants");
     UZU_UNSUPPORTED(!decayed_state_supported(p.dim, p.vdim), "decayed_state: heads of %u x %u (keys up to 1024)", p.dim, p.vdim);
     UZU_REQUIRE((size_t)p.nseq * p.heads <= 0x7FFFFFFFu && p.heads <= 65535 && p.nseq <= 65535, "decayed_state: too many heads for one launch");
-    if (p.form == 2 || (p.form == 0 && p.chunk_ws && p.rows > 16 * p.nseq)) { // prompt-sized: in chunks
+    // in chunks: prompt-sized passes whose rows of a chunk lie within the 2 GiB that a buffer's offsets span (pitches from 6291456 floats on go token by token, whose addresses have 64 bits)
+    const bool spanned = (size_t)kChunk * p.ld < 0x18000000u && (size_t)kChunk * p.lddecay < 0x18000000u;
+    if (spanned && (p.form == 2 || (p.form == 0 && p.chunk_ws && p.rows > 16 * p.nseq))) {
         UZU_REQUIRE(p.chunk_ws && p.chunks && p.chunk_ws_bytes >= decayed_state_chunk_ws_bytes(p.chunks, p.heads, p.dim, p.vdim), "decayed_state: the chunked form needs its workspace");
         const uint32_t vw = p.vdim <= 64 ? 64 : 128, vt = (p.vdim + vw - 1) / vw, kt = (p.dim + 63) / 64;
         const bool fours = p.dim % 4 == 0 && p.vdim % 4 == 0;
-        // (a chunk's rows and a head's state within the 2 GiB that a buffer's offsets span)
-        UZU_UNSUPPORTED((size_t)kChunk * p.ld >= 0x18000000u || (size_t)kChunk * p.lddecay >= 0x18000000u, "decayed_state: rows of pitch %u / %u", p.ld, p.lddecay);
         UZU_REQUIRE((size_t)vt * kt <= 65535 && ((size_t)p.dim * p.vdim + 255) / 256 <= 65535, "decayed_state: head widths %u x %u", p.dim, p.vdim);
         const dim3 lgrid(p.chunks, p.heads, vt * kt), sgrid(p.nseq, p.heads, (uint32_t)(((size_t)p.dim * p.vdim + 255) / 256)), ogrid(p.chunks, p.heads, vt);
         float* ws = p.chunk_ws;
