@@ -115,6 +115,28 @@ def test_attention_of_f32_rows_on_the_matrix_cores(hip_ctx, H, G, dim, vd, windo
         assert np.array_equal(attention(hip_ctx, q[start + 7:], K, V, mx, start + 7), got[7:])
 
 
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("H,G,dim,vd,window,cap,T,start,at", [(2, 1, 64, 64, 0, 0.0, 40, 0, 21), (4, 2, 128, 128, 0, 0.0, 35, 2, 34), (2, 2, 64, 128, 21, 0.0, 70, 3, 30), (2, 1, 128, 64, 9, 4.0, 50, 17, 48),
+                                                             (1, 1, 64, 64, 1, 0.0, 33, 0, 15), (2, 1, 128, 128, 40, 0.0, 200, 20, 96)])
+def test_attention_of_f32_rows_keeps_what_a_row_does_not_see_out_of_it(hip_ctx, H, G, dim, vd, window, cap, T, start, at, bad):
+    """A key or a value that is not finite, among rows that do not see it yet, see it, and no longer see it (in one tile of 16 rows; at the end of a ragged one): every row is what the simple form
+    gives, which adds the visible keys alone, within the two forms' bound where it is finite."""
+    rng = np.random.default_rng(H * 100 + T + dim + at)
+    q, K, V = qkv(rng, T, H, G, dim, vd)
+    mx = {"heads": H, "kv_heads": G, "scale": 1.7 / np.sqrt(dim), "mask": {"size": window}, "softcap": cap}
+    rows = np.arange(start, T)
+    sees = (rows >= at) & ((rows < at + window) if window else True)
+    bad_v, bad_k = V.copy(), K.copy()
+    bad_v[at, :, ::3] = bad
+    bad_k[at, :, 5] = bad
+    for k, v in ((K, bad_v), (bad_k, V)):
+        got, simple = attention(hip_ctx, q[start:], k, v, mx, start), attention(hip_ctx, q[start:], k, v, mx, start, form=1)
+        finite = np.isfinite(simple)
+        assert finite[~sees].all() and (sees.any() and not finite[sees].all() or v is V) and np.array_equal(finite, np.isfinite(got))
+        assert np.array_equal(got[~finite], simple[~finite], equal_nan=True)
+        assert np.abs(got - simple)[finite].max() < 2e-5 * np.abs(simple[finite]).max()
+
+
 @pytest.mark.parametrize("H,G,dim,vd,window,cap,T,start", [c for c in CASES if c[2] % 8 == 0 and c[3] % 8 == 0] + MANY_TILES)
 def test_attention_matrix_core_form_equals_the_simple_form(hip_ctx, H, G, dim, vd, window, cap, T, start):
     rng = np.random.default_rng(H * 100 + T + 1)

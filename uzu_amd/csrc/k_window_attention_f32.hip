@@ -6,7 +6,7 @@
 //   scores   S^T = K Q^T: a lane holds four keys' scores of one query (key 4 (lane / 16) + r, query lane % 16), and its softmax statistics
 //   results  O^T = V^T P^T: step s takes the keys 4 (lane / 16) + s, whose weights are the lane's own registers; the queries stay where they are
 // Keys and values go from memory into the operands' registers, a wave's next ones while it works.  A block's number counts from position 0, and a key that a row does not see has weight 0: a row's
-// sums do not depend on what else is in its tile or its pass.
+// sums do not depend on what else is in its tile or its pass.  (Zero times a value that is not finite is no zero: where that shows, a row's sums are made again from its keys alone.)
 // 300 rows of 8 heads of 128: 44.7 us by the simple form, 15.3 here.  (29.5 with a branch around every load for caches of four bytes' alignment, which the loads take as they are, and with the
 // values, too, a step ahead, which spilled.)
 #include "device_utils.h"
@@ -17,6 +17,25 @@ namespace k {
 
 namespace {
 constexpr uint32_t kRows = 16, kKeys = 16, kWaves = 8;
+
+// Columns c .. c + 3 of a row's sums, those that are NaN, from the keys that the row (position t) sees, one after the other
+template <bool EXTRA>
+__device__ __forceinline__ void visible_sums(const WindowAttentionParams& p, size_t row, uint32_t t, uint32_t a, const float* K, const float* V, size_t kpitch, size_t vpitch, uint32_t dim, uint32_t c,
+                                          float top, f32x4_v& v) {
+    const float *q = p.q + row * p.ldq + (size_t)a * dim, hscale = p.head_scale ? p.scale * p.head_scale[a] : p.scale;
+    uint32_t j = p.window && t + 1 > p.window ? t + 1 - p.window : 0u;
+    f32x4_v sums = {0.f, 0.f, 0.f, 0.f};
+    for (j = p.chunk ? max(j, t / p.chunk * p.chunk) : j; j <= t; ++j) {
+        float s = 0.0f;
+        for (uint32_t i = 0; i < dim; ++i) s = fmaf(K[j * kpitch + i], q[i], s);
+        s *= hscale;
+        if (EXTRA && p.soft_cap != 0.0f) s = p.soft_cap * tanhf(s / p.soft_cap);
+        if (EXTRA && p.dist_bias) s += p.dist_bias[(size_t)min(t - j, p.dist_rows - 1) * p.heads + a];
+        const float w = expf(s - top);
+        for (uint32_t e = 0; e < 4; ++e) sums[e] = fmaf(w, V[j * vpitch + c + e], sums[e]);
+    }
+    for (uint32_t e = 0; e < 4; ++e) v[e] = v[e] != v[e] ? sums[e] : v[e];
+}
 
 // grid (row tiles at most, heads), 512 threads.  DG: key width / 16; VH: value width / 64
 // EXTRA: a cap on the scores or a bias by distance (an instance of its own: the plain one has no branch between the products)
@@ -133,6 +152,8 @@ __global__ void __launch_bounds__(64 * kWaves) window_attention_f32_kernel(Windo
     }
     if (p.sinks) sum += expf(p.sinks[a] - all);
     const size_t out_row = sp.row0 + row0 + row;
+    const f32x4_v lost = v - v; // (NaN or zero)
+    if (__builtin_expect(((lost[0] + lost[1]) + (lost[2] + lost[3])) != 0.0f && sum == sum, 0)) visible_sums<EXTRA>(p, out_row, sp.start + row0 + row, a, K, V, kpitch, vpitch, DIM, c, all, v);
     const float og = p.gate ? p.out_scale / (1.0f + expf(-p.gate[out_row * p.ldgate + a])) : p.out_scale;
     float* out = p.out + out_row * p.ldo + (size_t)a * VD + c;
 #pragma unroll
