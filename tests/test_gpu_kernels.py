@@ -1012,6 +1012,39 @@ def test_attention_of_a_tree_on_the_matrix_cores(hip_ctx, n, heads, kv_heads, hd
     assert np.isfinite(got).all() and (np.abs(got - want) <= bound).all(), np.max(np.abs(got - want) - bound)
 
 
+@pytest.mark.parametrize("bad", [0x7F80, 0xFF80, 0x7FC0])
+@pytest.mark.parametrize("n,heads,kv_heads,hd,prefix,at", [(3, 4, 2, 64, 5, 1), (13, 8, 2, 256, 1023, 4), (16, 4, 4, 128, 31, 9), (32, 8, 1, 64, 96, 20), (32, 6, 2, 256, 2090, 3), (4, 4, 2, 128, 61, 3)])
+def test_attention_of_a_tree_keeps_other_branches_values_out(hip_ctx, n, heads, kv_heads, hd, prefix, at, bad):
+    """Key or value rows of a node that are not finite: the nodes of other branches have what finite rows leave them (within a rounding to bf16, since an f32 sum may be made in another order),
+    its own subtree what float64 gives."""
+    parents = [-1] + [i - 1 if i % 3 else 0 for i in range(1, n)]  # chains of three that hang off the root
+    rng = np.random.default_rng(n * hd + prefix + at)
+    seq, trie = prefix + n, trie_from_parents(parents)
+    sees = np.array([trie[at][0] <= i <= trie[at][1] for i in range(n)])
+    assert sees.any() and not sees.all()
+    q, k, v, _ = attention_case(rng, heads, kv_heads, hd, seq, n, seq)
+    scale = 1.0 / np.sqrt(hd)
+    bad_v, bad_k = v.copy(), k.copy()
+    bad_v[prefix + at, ::3] = bad
+    bad_k[prefix + at, 1::hd] = bad
+    kern = B.AttentionSinglePassKernel.new(hip_ctx, B.BF16, hd, 0, 0, 1, 1, 0)
+    bq, bt, bo = hip_ctx.buffer_from(q), hip_ctx.buffer_from(trie), hip_ctx.create_buffer(n * heads * hd * 2)
+
+    def rows(k, v):
+        bk, bv = hip_ctx.buffer_from(k), hip_ctx.buffer_from(v)
+        run(hip_ctx, lambda cb: kern.encode(bq, bk, bv, bo, heads // kv_heads, seq, hd, kv_heads * hd, hd, kv_heads * hd, None, scale, bt, None, None, heads, n, cb))
+        return bo.download(np.uint16, n * heads * hd).reshape(n, heads, hd)
+    clean = rows(k, v)
+    bits = rows(bad_k, v)
+    assert ulp_diff_bf16(bits[~sees], clean[~sees]).max() <= 1.0 and (bad != 0x7FC0 or np.isnan(f32(bits[sees])).all())
+    bits = rows(k, bad_v)
+    assert ulp_diff_bf16(bits[~sees], clean[~sees]).max() <= 1.0
+    want, got = attention_float64(q, k, bad_v, heads, kv_heads, hd, seq, n, hd, kv_heads * hd, scale, 1, None, None, None, parents), f32(bits)
+    finite = np.isfinite(want)
+    assert np.array_equal(finite, np.isfinite(got)) and np.array_equal(got[~finite], want[~finite], equal_nan=True) and not finite[sees].all()
+    assert ulp_diff_bf16(bits[finite], clean[finite]).max() <= 1.0  # (a column of the values by itself)
+
+
 def test_trie_verify_then_compaction_equals_linear_decode(hip_ctx):
     """The speculative-decoding round trip at the kernel boundary (f4 starter): the K / V rows of a speculated tree sit behind the prefix in
     depth-first order; trie-masked attention gives every node the output a LINEAR sequence ending in its root path would give (same keys, same

@@ -10,6 +10,7 @@
 //   * waves = (column tile, half of the head's elements): both halves work the scores out for themselves, which is cheaper than handing them over;
 //   * the probabilities enter the second product as three bf16 terms, which hold all 24 bits of them, and the queries, keys and values are bf16: every product is exact
 //     and the sums are in f32, as they are in the vector form (k_attention.hip);
+//   * a key of another branch has weight zero, but zero times a value that is not finite is none: where that shows, the merge makes a share's sum again from the visible keys alone;
 //   * partial results lie as [column tile][share][element][32 columns], so that both launches move whole lines.
 // Layout of the operands as in k_attention_mfma.hip: scores transposed, so that a lane owns a column.
 #include "device_utils.h"
@@ -168,12 +169,12 @@ __global__ void __launch_bounds__(256) tree_attention_kernel(AttentionParams a, 
 #pragma unroll
             for (int r = 0; r < 16; ++r) m_mine = fmaxf(m_mine, score[r]);
             const float m_new = fmaxf(m_run, fmaxf(m_mine, __shfl_xor(m_mine, 32, 64)));
-            const float alpha = m_new == -INFINITY ? 1.0f : fast_exp(m_run - m_new);
+            const float alpha = m_new == -INFINITY ? 1.0f : fast_exp(m_run - m_new), m_ref = m_new == -INFINITY ? 0.f : m_new; // (-inf: no key seen, or NaNs)
             float sum = 0.f;
             u32x4_v p[3][2]; // the probabilities' three terms of two k16 steps
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
-                const float p0 = m_new == -INFINITY ? 0.f : fast_exp(score[r] - m_new), p1 = m_new == -INFINITY ? 0.f : fast_exp(score[r + 1] - m_new);
+                const float p0 = fast_exp(score[r] - m_ref), p1 = fast_exp(score[r + 1] - m_ref);
                 sum += p0 + p1;
                 const float h0 = round_bf16(p0), h1 = round_bf16(p1), r0 = p0 - h0, r1 = p1 - h1, i0 = round_bf16(r0), i1 = round_bf16(r1);
                 p[0][r / 8][r / 2 % 4] = pack2(h0, h1), p[1][r / 8][r / 2 % 4] = pack2(i0, i1), p[2][r / 8][r / 2 % 4] = pack2(r0 - i0, r1 - i1);
@@ -205,13 +206,32 @@ __global__ void __launch_bounds__(256) tree_attention_kernel(AttentionParams a, 
     if (part == 0 && half == 0) sums[at * kColumns + l32] = l, maxs[at * kColumns + l32] = m_run;
 }
 
+// A share's sum for one element of a column, from the keys that its node sees, one after the other
+template <int HD>
+__device__ __forceinline__ float visible_sum(const AttentionParams& a, uint32_t kv_head, uint32_t column, uint32_t node, uint32_t element, uint32_t share, uint32_t shares, float top) {
+    const uint32_t n = a.suffix_length, length = a.sequence_length + (a.dyn ? *a.dyn : 0u), prefix = length - n;
+    const uint16_t* q = (const uint16_t*)a.queries + ((size_t)kv_head * a.gqa_factor * n + column) * HD;
+    const uint16_t *keys = (const uint16_t*)a.keys + (size_t)kv_head * a.k_head_stride, *values = (const uint16_t*)a.values + (size_t)kv_head * a.v_head_stride + element;
+    float sum = 0.f;
+    for (uint32_t t = share; t * kKeys < length; t += shares)
+        for (uint32_t i = t * kKeys; i < min(t * kKeys + kKeys, length); ++i) {
+            if (i >= prefix && !(node >= a.trie[3 * (i - prefix)] && node <= a.trie[3 * (i - prefix) + 1])) continue;
+            float score = 0.f;
+            for (uint32_t d = 0; d < HD; ++d) score = fmaf(bf16_to_f32(q[d]), bf16_to_f32(keys[(size_t)i * a.k_seq_stride + d]), score);
+            sum = fmaf(fast_exp(a.scale * score - top), bf16_to_f32(values[(size_t)i * a.v_seq_stride]), sum);
+        }
+    return sum;
+}
+
 // The rows from their shares, and the gate: a workgroup has 8 elements of a column tile, a thread one of a column, everything requested before any of it is used.  6.7 us
 // behind 1500 keys (48 shares of 128 KB), where the two-pass form's second kernel and the gate's were 9.4.
 // grid (kv heads x column tiles, head_dim / 8), 256 threads
-__global__ void __launch_bounds__(256) tree_attention_merge_kernel(const float* __restrict__ partials, const float* __restrict__ sums, const float* __restrict__ maxs,
-                                                                   uint16_t* __restrict__ out, const uint16_t* __restrict__ gate, uint32_t n, uint32_t group_heads, uint32_t heads,
-                                                                   uint32_t head_dim, uint32_t tiles, uint32_t pairs, uint32_t shares, uint32_t sequence_length,
-                                                                   const uint32_t* __restrict__ dyn) {
+template <int HD>
+__global__ void __launch_bounds__(256) tree_attention_merge_kernel(AttentionParams a, const float* __restrict__ partials, const float* __restrict__ sums, const float* __restrict__ maxs,
+                                                                   uint16_t* __restrict__ out, const uint16_t* __restrict__ gate, uint32_t tiles, uint32_t pairs, uint32_t shares) {
+    constexpr uint32_t head_dim = HD;
+    const uint32_t n = a.suffix_length, group_heads = a.gqa_factor, heads = a.num_heads, sequence_length = a.sequence_length;
+    const uint32_t* const dyn = a.dyn;
     const uint32_t used = min(shares, (sequence_length + (dyn ? *dyn : 0u) + kKeys - 1) / kKeys); // shares with keys: nothing of the others but their maxima has been written
     constexpr uint32_t P = kTreeAttentionShares / 8;
     __shared__ float s_max[8][kColumns], s_sum[8][kColumns], s_w[kTreeAttentionShares][kColumns];
@@ -263,6 +283,16 @@ __global__ void __launch_bounds__(256) tree_attention_merge_kernel(const float* 
                 o += w == 0.f ? 0.f : v[b] * w; // (a share without keys has written no elements)
             }
         }
+    if (__builtin_expect(o != o && l_all == l_all, 0)) {
+        o = 0.f;
+        for (uint32_t b = 0; b < used; ++b) {
+            const float w = s_w[b][c];
+            if (w == 0.f) continue;
+            float part = partials[((at + b) * head_dim + element) * kColumns + c];
+            if (part != part) part = visible_sum<HD>(a, kv_head, column, node, element, b, shares, maxs[(at + b) * kColumns + c]);
+            o += part * w;
+        }
+    }
     uint16_t bits = f32_to_bf16(o / l_all);
     if (gate) bits = scaled_sigmoid_bf16(bf16_to_f32(bits), bf16_to_f32(g), s_exp_tab);
     out[row * head_dim + element] = bits;
@@ -300,8 +330,11 @@ uzu_status attention_tree(hipStream_t s, const AttentionParams& a, uint32_t key_
         else hipLaunchKernelGGL((tree_attention_kernel<256>), grid, dim3(256), 0, s, a, pairs, key_rows, partials, sums, maxs);
     }, "tree_attention"));
     return launch_check([&] {
-        hipLaunchKernelGGL(tree_attention_merge_kernel, dim3(kv_heads * tiles, a.head_dim / 8), dim3(256), 0, s, partials, sums, maxs, (uint16_t*)out, (const uint16_t*)gate, a.suffix_length,
-                           a.gqa_factor, a.num_heads, a.head_dim, tiles, pairs, shares, a.sequence_length, a.dyn);
+#define UZU_TM(HD) hipLaunchKernelGGL(tree_attention_merge_kernel<HD>, dim3(kv_heads * tiles, HD / 8), dim3(256), 0, s, a, partials, sums, maxs, (uint16_t*)out, (const uint16_t*)gate, tiles, pairs, shares)
+        if (a.head_dim == 64) UZU_TM(64);
+        else if (a.head_dim == 128) UZU_TM(128);
+        else UZU_TM(256);
+#undef UZU_TM
     }, "tree_attention_merge");
 }
 
