@@ -1045,6 +1045,26 @@ def test_attention_of_a_tree_keeps_other_branches_values_out(hip_ctx, n, heads, 
     assert ulp_diff_bf16(bits[finite], clean[finite]).max() <= 1.0  # (a column of the values by itself)
 
 
+def test_attention_of_a_tree_with_a_weight_of_zero(hip_ctx):
+    """Keys that every node sees, with weights below the smallest float, one of them with an infinite value: zero times infinity, as the vector form has it, also where a share has no other keys."""
+    n, heads, kv_heads, hd, prefix = 5, 4, 2, 64, 700
+    rng = np.random.default_rng(3)
+    seq, trie = prefix + n, trie_from_parents([-1, 0, 1, 0, 3])
+    q, k, v, a = attention_case(rng, heads, kv_heads, hd, seq, n, seq)
+    q[:, :, 0], k[:, ::hd] = bf16(np.float32(8.0)), bf16(np.float32(0.0))
+    bo = hip_ctx.create_buffer(n * heads * hd * 2)
+    kern = B.AttentionSinglePassKernel.new(hip_ctx, B.BF16, hd, 0, 0, 1, 1, 0)
+    for key in (0, 300, 650):
+        bad_k, bad_v = k.copy(), v.copy()
+        bad_k[key // 32 * 32:key // 32 * 32 + 32, ::hd], bad_v[key, 3] = bf16(np.float32(-400.0)), 0x7F80
+        bq, bk, bv, bt = hip_ctx.buffer_from(q), hip_ctx.buffer_from(bad_k), hip_ctx.buffer_from(bad_v), hip_ctx.buffer_from(trie)
+        run(hip_ctx, lambda cb: kern.encode(bq, bk, bv, bo, heads // kv_heads, seq, hd, kv_heads * hd, hd, kv_heads * hd, None, 1.0 / np.sqrt(hd), bt, None, None, heads, n, cb))
+        got = f32(bo.download(np.uint16, n * heads * hd)).reshape(n, heads, hd)
+        bad = np.zeros(got.shape, bool)
+        bad[:, :heads // kv_heads, 3] = True
+        assert np.isnan(got[bad]).all() and np.isfinite(got[~bad]).all(), key
+
+
 def test_trie_verify_then_compaction_equals_linear_decode(hip_ctx):
     """The speculative-decoding round trip at the kernel boundary (f4 starter): the K / V rows of a speculated tree sit behind the prefix in
     depth-first order; trie-masked attention gives every node the output a LINEAR sequence ending in its root path would give (same keys, same

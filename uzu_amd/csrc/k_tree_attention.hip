@@ -266,7 +266,7 @@ __global__ void __launch_bounds__(256) tree_attention_merge_kernel(AttentionPara
 #pragma unroll
     for (uint32_t i = 0; i < P; ++i) {
         const float w = expf_glibc_tab(m[i] - m_all, s_exp_tab);
-        s_w[e + 8 * i][c] = w, sum += l[i] * w;
+        s_w[e + 8 * i][c] = m[i] == -INFINITY ? -1.f : w, sum += l[i] * w; // (-1: no key seen, no elements written)
     }
     s_sum[e][c] = sum;
     __syncthreads();
@@ -280,14 +280,14 @@ __global__ void __launch_bounds__(256) tree_attention_merge_kernel(AttentionPara
 #pragma unroll
             for (uint32_t b = 8 * i; b < 8 * i + 8; ++b) {
                 const float w = s_w[b][c];
-                o += w == 0.f ? 0.f : v[b] * w; // (a share without keys has written no elements)
+                o += w < 0.f ? 0.f : v[b] * w;
             }
         }
     if (__builtin_expect(o != o && l_all == l_all, 0)) {
         o = 0.f;
         for (uint32_t b = 0; b < used; ++b) {
             const float w = s_w[b][c];
-            if (w == 0.f) continue;
+            if (w < 0.f) continue;
             float part = partials[((at + b) * head_dim + element) * kColumns + c];
             if (part != part) part = visible_sum<HD>(a, kv_head, column, node, element, b, shares, maxs[(at + b) * kColumns + c]);
             o += part * w;
