@@ -85,6 +85,29 @@ def test_rows_in_pair_order_are_refused_where_a_kernel_would_read_plain_ones(tmp
     assert out.returncode == 0 and out.stdout.endswith("\n0 bad\n"), out.stdout + out.stderr
 
 
+def _run_against_the_library(tmp_path, name, **env):
+    """tests/host/<name>.cpp, linked to the library and its C++ functions"""
+    import subprocess
+    from uzu_amd import _ffi
+    _ffi.lib()
+    exe, libdir = str(tmp_path / name), os.path.dirname(_ffi.LIB_PATH)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(ROOT, "tests", "host", name + ".cpp"),
+                    "-L", libdir, "-luzu_hip", "-L/opt/rocm/lib", "-lamdhip64", f"-Wl,-rpath,{libdir}", "-o", exe], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=100, env=dict(os.environ, **env))
+    assert out.returncode == 0 and out.stdout.endswith("0 bad\n"), out.stdout + out.stderr
+
+
+def test_calls_go_to_the_faster_kernel(tmp_path):
+    """tests/host/routes_check.cpp: the dispatch's rules at sizes on both sides of them, no device visible."""
+    _run_against_the_library(tmp_path, "routes_check", HIP_VISIBLE_DEVICES="")
+
+
+@pytest.mark.gpu
+def test_tree_attention_at_its_edges(tmp_path):
+    """tests/host/tree_attention_check.cpp: the tree form against the vector form, and with NaN rows behind the last key."""
+    _run_against_the_library(tmp_path, "tree_attention_check")
+
+
 @pytest.mark.gpu
 def test_gated_epilogue_has_the_exact_silu_for_every_gate(tmp_path):
     """tests/host/gated_silu_check.cpp: the quick quotient of csrc/gemm128_epilogue.h on the device, through the library's product, on each of its forms."""

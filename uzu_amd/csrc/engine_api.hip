@@ -399,19 +399,21 @@ uzu_status uzu_hip_model_verify_tree_seeded(uzu_hip_model* m, const uint32_t* to
     HIPCHK(hipMemcpyAsync(m->tree.d_parents, parents.data(), (size_t)tree_size * 4, hipMemcpyHostToDevice, s));
     m->tree.host_seeds = seeds != nullptr && m->sampling.on;
     if (m->tree.host_seeds) HIPCHK(hipMemcpyAsync(m->tree.d_seeds, seeds, (size_t)tree_size * 8, hipMemcpyHostToDevice, s));
+    const bool two_pass_regime = m->context_length + tree_size > 1024;
+    uint32_t tree_layers = 0;
     {
         // the largest of the layers' partial results, at any context: of the tree form (columns of all shares), or of the two-pass form behind 1024 keys (32 blocks a row)
         size_t rows = 0;
         uint32_t max_hd = 0;
         for (auto& L : m->layers)
             if (L.d.mixer_kind == UZU_MIXER_ATTENTION) {
+                tree_layers += L.d.num_groups && tree_attention_faster(m, L, tree_size, two_pass_regime) ? 1 : 0;
                 const size_t columns = L.d.num_groups ? k::attention_tree_columns(L.d.num_heads, L.d.num_heads / L.d.num_groups, tree_size) : 0;
                 rows = std::max({rows, (size_t)tree_size * L.d.num_heads, (columns + 31) / 32});
                 max_hd = max_hd > L.d.head_dim ? max_hd : L.d.head_dim;
             }
         if (rows) UZU_PROPAGATE(ensure_partials(m, (uint32_t)rows, max_hd));
     }
-    const bool two_pass_regime = m->context_length + tree_size > 1024;
     HIPCHK(hipEventRecord(m->ev0, s));
     if ((m->flags & UZU_MODEL_NO_GRAPH) || k::exact_mode()) {
         m->tree.active = true;
@@ -425,7 +427,7 @@ uzu_status uzu_hip_model_verify_tree_seeded(uzu_hip_model* m, const uint32_t* to
             m->tree.graph_epoch = m->sampling_epoch;
         }
         for (auto& g : m->tree.graphs)
-            if (g.state == m->bound && g.nodes == tree_size && g.two_pass == two_pass_regime && g.host_seeds == m->tree.host_seeds) exec = g.exec, m->launches = g.launches;
+            if (g.state == m->bound && g.nodes == tree_size && g.two_pass == two_pass_regime && g.tree_layers == tree_layers && g.host_seeds == m->tree.host_seeds) exec = g.exec, m->launches = g.launches;
         if (!exec) {
             HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
             m->regime_override = two_pass_regime ? 1 : 0;
@@ -442,7 +444,7 @@ uzu_status uzu_hip_model_verify_tree_seeded(uzu_hip_model* m, const uint32_t* to
             }
             HIPCHK(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0));
             HIPCHK(hipGraphDestroy(g));
-            m->tree.graphs.push_back({m->bound, tree_size, two_pass_regime, m->tree.host_seeds, exec, m->launches});
+            m->tree.graphs.push_back({m->bound, tree_size, two_pass_regime, tree_layers, m->tree.host_seeds, exec, m->launches});
         }
         HIPCHK(hipGraphLaunch(exec, s));
     }

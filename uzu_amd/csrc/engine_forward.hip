@@ -355,6 +355,10 @@ void attention_joined(Enc& e, DLayer& L, uint32_t batch, JoinedAttention& j) {
             RUN("sigmoid_gate", 0, k::sigmoid_gate(e.s, m->gate + j.row0[i] * nq * hd, m->attn_out + j.row0[i] * nq * hd, UZU_BF16, batch * nq * hd));
     j.seqs.n = 0;
 }
+// the form of a tree pass' attention, by the bound sequence's length: what a captured pass has chosen holds for others with as many of these layers and the same regime
+bool tree_attention_faster(const uzu_hip_model* m, const DLayer& L, uint32_t nodes, bool two_pass) {
+    return k::attention_tree_faster(L.d.num_heads, L.d.num_heads / L.d.num_groups, L.d.head_dim, nodes, m->context_length + nodes, two_pass, L.d.has_gate != 0);
+}
 // AttentionPrepare + attention of `batch` rows of the bound sequence, which start at row `row0` of qkv / queries / attn_out
 void attention_core(Enc& e, DLayer& L, uint32_t batch, size_t row0, bool fuse_norms, JoinedAttention* join) {
     uzu_hip_model* m = e.m;
@@ -404,7 +408,7 @@ void attention_core(Enc& e, DLayer& L, uint32_t batch, size_t row0, bool fuse_no
         uint32_t gate_done = 0; // SigmoidGate inside the key-split merge launch when the pass has one (bit-identical to the separate launch)
         RUN("attention_prefill_mfma", kv_bytes, k::attention_prefill_mfma_behind(e.s, a, W ? W : m->context_length, attn_out, L.d.has_gate && attention_fusions_enabled() ? m->gate + row0 * nq * hd : nullptr, &gate_done));
         gated = gate_done != 0;
-    } else if (k::attention_tree_supported(a)) { // a speculated tree's rows, any context length (the gate with them)
+    } else if (k::attention_tree_supported(a) && tree_attention_faster(m, L, batch, two_pass)) { // a speculated tree's rows (the gate with them)
         RUN("attention_tree", kv_bytes, k::attention_tree(e.s, a, m->d.max_context_length, m->partials, m->sums, m->maxs, attn_out, L.d.has_gate ? m->gate + row0 * nq * hd : nullptr));
         gated = L.d.has_gate != 0;
     } else if (two_pass) { // core/mod.rs:89-92

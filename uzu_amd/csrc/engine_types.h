@@ -285,12 +285,13 @@ struct uzu_hip_model {
         uzu_hip_state* state = nullptr; // the state it hangs off
         std::vector<int32_t> parents;
         std::vector<uint32_t> sampled;
-        // the tree pass of (sequence state, node count, attention regime) as a hipGraph: everything that changes from pass to pass --
+        // the tree pass of (sequence state, node count, attention regime and forms) as a hipGraph: everything that changes from pass to pass --
         // token ids, trie nodes, parents, context length -- sits in device buffers the kernels read, so the captured pass is replayable
         struct Graph {
             uzu_hip_state* state;
             uint32_t nodes;
             bool two_pass;
+            uint32_t tree_layers; // layers whose attention is of the tree form (the longer the context, the more of them)
             bool host_seeds; // the pass takes the caller's per-node seeds (no derive_tree_seeds launch in it)
             hipGraphExec_t exec;
             uint32_t launches;
@@ -401,6 +402,7 @@ k::NormParams norm_params(Enc& e, const DNorm& N, const uint16_t* input, uint16_
 void norm_issued(uzu_hip_model* m, const k::NormParams& p);
 void norm(Enc& e, const DNorm& N, const uint16_t* input, uint16_t* output, uint16_t* shortcut, int mode, uint32_t rows, uint32_t dim, const DLinear* consumer = nullptr);
 void attention_mixer(Enc& e, DLayer& L, const uint16_t* hidden, uint16_t* out, const Seqs& q, PostNorm* post = nullptr, bool first_done = false);
+bool tree_attention_faster(const uzu_hip_model* m, const DLayer& L, uint32_t nodes, bool two_pass);
 uzu_status ensure_tp_gather(uzu_hip_model* m, uint32_t rows);
 uzu_status ensure_partials(uzu_hip_model* m, uint32_t rows, uint32_t head_dim);
 uzu_status encode_forward(uzu_hip_model* m, hipStream_t s, uint32_t count, bool sample, uzu_hip_state** seqs = nullptr, uint32_t nseq = 0);

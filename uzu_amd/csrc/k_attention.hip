@@ -227,7 +227,8 @@ uzu_status attention_single_pass(hipStream_t s, const AttentionParams& a, void* 
     UZU_PROPAGATE(check_attention(a));
     if (exact_mode()) return attention_single_pass_exact(s, a, out);
     if (attention_prefill_mfma_supported(a)) return attention_prefill_mfma(s, a, out); // prefill-sized causal tiles
-    if (!a.dyn && a.sequence_length >= a.suffix_length && attention_tree_supported(a)) { // (at every length: k_tree_attention.hip; under capture there is no workspace, and the vector form runs)
+    if (!a.dyn && a.sequence_length >= a.suffix_length && attention_tree_supported(a) &&
+        attention_tree_faster(a.num_heads, a.gqa_factor, a.head_dim, a.suffix_length, a.sequence_length, false, false)) { // (under capture there is no workspace, and the vector form runs)
         const size_t columns = attention_tree_columns(a.num_heads, a.gqa_factor, a.suffix_length);
         if (float* ws = (float*)stream_workspace(s, columns * (a.head_dim + 2) * sizeof(float)))
             return attention_tree(s, a, a.sequence_length, ws, ws + columns * a.head_dim, ws + columns * (a.head_dim + 1), out, nullptr);

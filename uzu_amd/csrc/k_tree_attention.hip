@@ -315,6 +315,25 @@ bool attention_tree_supported(const AttentionParams& a) {
     return (((uintptr_t)a.queries | (uintptr_t)a.keys | (uintptr_t)a.values) & 15) == 0; // rows are read 16 bytes at a time
 }
 
+// The vector form (k_attention.hip) has a workgroup per node and group of `gs` heads, and shares of the keys in its two passes alone.  Single pass: 3.4 us for heads by themselves, 4.3 in pairs, 6 in
+// fours, and then 0.011 / 0.021 / 0.045 us a key of 64 / 128 / 256, half as much again in pairs; the tree form 7.8 / 8.4 / 9.5 us and next to nothing a key (heads by themselves, 13 nodes, us,
+// single pass and tree: 16 of 128 behind 80 keys 5.4 / 8.5, 250 9.1 / 9.1, 600 20.9 / 10.4; 8 of 64 behind 250 6.4 / 8.3, 450 8.6 / 8.3): where the two meet is below, and groups of eight are slower from
+// the first key on.  Two passes: what counts is how much work there is.  The tree form wants its columns filled, or the vector form's workgroups to be more than the chip holds.  Us, two passes
+// and tree, 1500 and 4000 keys: 16 heads of 128, 4 nodes 9.9 / 11.8 and 15.4 / 19.4, 8 nodes 14.6 / 11.8 and 24.1 / 19.2; 32 on 8 of 128, 1 node 9.4 / 11.5 and 12.3 / 14.1, 3 nodes 12.6 / 10.8 and
+// 18.4 / 13.4; 8 on 4 of 256, 6 nodes 11.5 / 12.4 and 19.0 / 16.0, 8 nodes 12.9 / 12.4 and 21.6 / 15.9; 8 on 2 of 256, 3 nodes 11.0 / 11.8 and 17.5 / 14.8, 4 nodes 11.1 / 11.8 and 17.6 / 14.7, with the gate
+// 3 .. 4 us less for the tree form.
+bool attention_tree_faster(uint32_t num_heads, uint32_t gqa_factor, uint32_t head_dim, uint32_t nodes, uint32_t keys, bool two_pass, bool gated) {
+    uint32_t gs = 0; // heads of a workgroup of the vector form: 1 << gs
+    while (gs < (head_dim >= 256 ? 2u : 3u) && gqa_factor % (2u << gs) == 0) ++gs;
+    if (gs == 3) return true;
+    if (!two_pass) {
+        static constexpr uint32_t meet[3][3] = {{430, 240, 90}, {240, 160, 75}, {135, 105, 60}}; // [heads of 64, 128, 256][gs]
+        return keys > meet[head_dim <= 64 ? 0 : head_dim <= 128 ? 1 : 2][gs];
+    }
+    const uint32_t rows = nodes * num_heads, columns = nodes * gqa_factor, half = gated ? 2 : 1;
+    return rows >= 128 / half || (columns >= (head_dim >= 256 ? 16 : 12) / half && rows * head_dim >= 6144 / half);
+}
+
 size_t attention_tree_columns(uint32_t num_heads, uint32_t gqa_factor, uint32_t nodes) {
     const uint32_t kv_heads = num_heads / gqa_factor, pairs = tree_pairs(gqa_factor, nodes);
     return (size_t)kv_heads * pairs * 2 * kColumns * tree_shares(kv_heads, pairs);

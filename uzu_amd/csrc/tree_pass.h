@@ -10,6 +10,9 @@ constexpr uint32_t kTreeAttentionShares = 64; // shares of the keys at most, eac
 
 // bf16 rows of at most 32 nodes under the trie mask alone (no window, ring or sinks), heads of 64, 128 or 256
 bool attention_tree_supported(const AttentionParams& a);
+// Whether that form is the faster one in front of `keys` keys, the nodes' own among them.  two_pass: the vector form's two passes are the other choice, at whatever length; else its single
+// pass.  gated: a gate follows, which the tree form applies itself.
+bool attention_tree_faster(uint32_t num_heads, uint32_t gqa_factor, uint32_t head_dim, uint32_t nodes, uint32_t keys, bool two_pass, bool gated);
 // columns of partial results over all shares: partials hold head_dim floats for each, sums and maxs one
 size_t attention_tree_columns(uint32_t num_heads, uint32_t gqa_factor, uint32_t nodes);
 // key_rows: rows that the caches hold memory for, at least sequence_length (with dyn).
