@@ -1,6 +1,7 @@
 // Which kernel a call goes to, where two are right and one is faster: the rules of the library's dispatch at the sizes that their comments quote measurements for.  Host arithmetic alone.
 #include <cstdio>
 
+#include "../../uzu_amd/csrc/attention_prefill.h"
 #include "../../uzu_amd/csrc/kernels.h"
 #include "../../uzu_amd/csrc/tree_pass.h"
 
@@ -25,6 +26,19 @@ int main() {
         char what[160];
         snprintf(what, sizeof what, "tree attention, %u heads on %u of %u, %u nodes behind %u keys", t.heads, t.kv_heads, t.head_dim, t.nodes, t.context);
         expect(attention_tree_faster(t.heads, t.heads / t.kv_heads, t.head_dim, t.nodes, t.context + t.nodes, t.two_pass, t.gated), t.want, what);
+    }
+    struct Prompt {
+        uint32_t heads, kv_heads, head_dim, rows, prefix;
+        bool gated;
+        uint32_t least, most; // shares of the keys
+    };
+    for (const Prompt& t : {Prompt{32, 8, 128, 100, 0, false, 1, 1}, {32, 8, 128, 257, 0, false, 1, 1}, {32, 8, 128, 517, 0, false, 1, 1}, {16, 4, 128, 257, 0, false, 1, 1}, {24, 8, 64, 517, 0, false, 1, 1},
+                            {40, 8, 128, 130, 0, false, 1, 1}, {8, 2, 256, 100, 0, false, 1, 1}, {32, 8, 128, 64, 1000, false, 4, 12}, {16, 4, 128, 517, 2000, false, 2, 12}, {4, 4, 64, 1024, 3000, false, 4, 12},
+                            {8, 2, 256, 517, 0, false, 4, 12}, {8, 2, 256, 517, 0, true, 4, 12}, {8, 2, 256, 2043, 0, true, 2, 4}, {8, 2, 256, 3000, 0, false, 2, 2}, {32, 8, 128, 1021, 0, false, 1, 1}}) {
+        AttentionParams a{};
+        a.dt = UZU_BF16, a.head_dim = t.head_dim, a.gqa_factor = t.heads / t.kv_heads, a.num_heads = t.heads, a.suffix_length = t.rows, a.sequence_length = t.rows + t.prefix, a.is_causal = 1;
+        const uint32_t shares = attention_prefill_mfma_shares(a, t.prefix, t.gated);
+        if (shares < t.least || shares > t.most) printf("prompt attention, %u heads on %u of %u, %u rows behind %u keys: %u shares\n", t.heads, t.kv_heads, t.head_dim, t.rows, t.prefix, shares), ++bad;
     }
     printf("%d bad\n", bad);
     return bad != 0;

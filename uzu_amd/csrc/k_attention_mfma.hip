@@ -409,7 +409,8 @@ bool attention_prefill_mfma_supported(const AttentionParams& a) {
 
 // out[q][head][:] = sum_s w_s O_s / sum_s w_s l_s, w_s = 2^(m_s - max m) (a split that saw no key has m = -inf, l = 0: weight 0).
 // grid = rows / 4, 256 threads: 64 threads per (query, head) row, HD / 64 elements each.
-template <int HD>
+// MOST: the shares that a row has at most (a body with twelve shares' loads and branches costs a launch of two shares 1.2 us of 3.4).
+template <int HD, uint32_t MOST>
 // gate (optional): SigmoidGate (sigmoid_gate.rs:9-22) on the merged rows in the same launch -- out = bf16(bf16(o) * sigmoid(gate)), the separate kernel's two roundings
 __global__ void __launch_bounds__(256) attention_prefill_merge_kernel(const float* part_o, const float* part_ml, uint16_t* out, uint32_t rows, KeyShares shares, uint32_t tpw,
                                                                       uint32_t gqa, uint32_t heads, const uint16_t* gate) {
@@ -418,10 +419,10 @@ __global__ void __launch_bounds__(256) attention_prefill_merge_kernel(const floa
     if (row >= rows) return;
     const uint32_t query = row / heads, head = row - query * heads, splits = key_shares(shares, (query / TQ * gqa + head % gqa) / tpw, tpw, gqa, rows / heads, HD <= 128 ? 2 * TK : TK);
     // every share is requested before the first is used (one behind the other, a share was two trips to memory: 8 shares of 517 rows 11.2 us -> 9.3, 2 of 2043 15.4 -> 13.9)
-    float ms[kMaxKeySplits], ls[kMaxKeySplits], po[kMaxKeySplits][EPT];
+    float ms[MOST], ls[MOST], po[MOST][EPT];
     uint16_t gs[EPT];
 #pragma unroll
-    for (uint32_t sp = 0; sp < kMaxKeySplits; ++sp) {
+    for (uint32_t sp = 0; sp < MOST; ++sp) {
         ms[sp] = -INFINITY;
         if (sp < splits) {
             const size_t r = (size_t)sp * rows + row;
@@ -435,12 +436,12 @@ __global__ void __launch_bounds__(256) attention_prefill_merge_kernel(const floa
     __builtin_amdgcn_sched_barrier(0);
     float m = -INFINITY;
 #pragma unroll
-    for (uint32_t sp = 0; sp < kMaxKeySplits; ++sp) m = fmaxf(m, ms[sp]);
+    for (uint32_t sp = 0; sp < MOST; ++sp) m = fmaxf(m, ms[sp]);
     float acc[EPT], l = 0.f;
 #pragma unroll
     for (int e = 0; e < EPT; ++e) acc[e] = 0.f;
 #pragma unroll
-    for (uint32_t sp = 0; sp < kMaxKeySplits; ++sp) {
+    for (uint32_t sp = 0; sp < MOST; ++sp) {
         if (sp >= splits || ms[sp] == -INFINITY) continue;
         const float w = __builtin_amdgcn_exp2f(ms[sp] - m);
         l = fmaf(ls[sp], w, l);
@@ -467,6 +468,58 @@ __global__ void __launch_bounds__(256) attention_prefill_merge_kernel(const floa
     }
 }
 
+// Few task groups (few kv heads x short chunks): four tasks a workgroup, which share every staged K / V tile, and the KEYS over workgroups until the chip is covered -- or the workgroups thinned to
+// one or two tasks, and no merge.  What a launch takes is estimated for both, and the less is taken: the longest share, `us` a stretch of keys; the whole work at 256 CUs' rate, when that is more; a
+// second round, when workgroups are more than CUs; the merge, and its 8 bytes an element and share.  Measured over 170 sizes (10 shapes of 64 .. 256, 33 .. 3000 rows, up to 3000 keys in front): the choice is
+// within 0.3 % of the better one on the average, 11 % at the worst.  Us, shares and none: 32 heads on 8 of 128, 100 rows 13.0 / 7.5, 257 17.7 / 11.7, 517 25.1 / 18.9; 8 on 2 of 256, 100 rows 16.6 / 12.8, 257
+// 20.0 / 23.3, 517 26.9 / 41.4.
+struct PrefillPlan {
+    uint32_t quantum = 0, units = 0, splits = 1; // units: workgroups a kv head
+};
+static uint32_t unsplit_tasks(uint32_t kv_heads, uint32_t n_tasks) { // fewer tasks per workgroup until the grid covers most of the chip
+    uint32_t tpw = 4;
+    while (tpw > 1 && kv_heads * ((n_tasks + tpw - 1) / tpw) < 192) tpw >>= 1;
+    return tpw;
+}
+static PrefillPlan prefill_plan(const AttentionParams& a, uint32_t prefix, bool gated) {
+    const uint32_t kv_heads = a.num_heads / a.gqa_factor, n_tasks = a.gqa_factor * ((a.suffix_length + TQ - 1) / TQ), n_groups = (n_tasks + 3) / 4, stretch = a.head_dim <= 128 ? 2 * TK : TK;
+    PrefillPlan best;
+    if (kv_heads * n_groups >= 192) return best;
+    KeyShares shares{0, prefix};
+    const float us = a.head_dim == 64 ? 0.95f : a.head_dim == 128 ? 1.55f : 2.1f;
+    auto work = [&](uint32_t tpw) {
+        uint64_t all = 0;
+        for (uint32_t y = 0; y < (n_tasks + tpw - 1) / tpw; ++y) all += key_stretches(shares, y, tpw, a.gqa_factor, a.suffix_length, stretch);
+        return all;
+    };
+    auto time = [&](uint32_t longest, uint64_t all, uint32_t units) {
+        const float l = (float)longest, w = 1.4f * (float)(kv_heads * all) / 256.0f, second = 0.57f * l * std::max(0.0f, (float)(kv_heads * units) / 256.0f - 1.0f);
+        return us * sqrtf(sqrtf(l * l * l * l + w * w * w * w + second * second * second * second));
+    };
+    const uint32_t top = key_stretches(shares, n_groups - 1, 4, a.gqa_factor, a.suffix_length, stretch);
+    float least = time(top, work(unsplit_tasks(kv_heads, n_tasks)), 0) + (gated ? 3.5f : 0.0f); // (the gate's own launch)
+    const uint64_t all = work(4);
+    auto consider = [&](uint32_t quantum, uint32_t most_units) { // whether the workgroups are few enough
+        shares.quantum = quantum;
+        PrefillPlan p{quantum, 0, 1};
+        uint32_t longest = 0;
+        for (uint32_t y = 0; y < n_groups; ++y) {
+            const uint32_t n = key_shares(shares, y, 4, a.gqa_factor, a.suffix_length, stretch);
+            p.units += n, p.splits = std::max(p.splits, n), longest = std::max(longest, (key_stretches(shares, y, 4, a.gqa_factor, a.suffix_length, stretch) + n - 1) / n);
+        }
+        if (p.splits > 1 && kv_heads * p.units > most_units) return false;
+        const float t = time(longest, all, p.units) + (a.head_dim <= 128 ? 4.0f : 8.0f) + 0.44e-6f * 8.0f * (float)kv_heads * (float)p.units * 128.0f * (float)a.head_dim;
+        if (p.splits > 1 && t < least) least = t, best = p;
+        return true;
+    };
+    // the shortest shares that the CUs hold, a workgroup each: 64 keys a share at least, and no more shares than there can be
+    uint32_t quantum = std::max({2 * TK / stretch, (uint32_t)(kv_heads * all / 256), top / kMaxKeySplits});
+    while (!consider(quantum, 256)) ++quantum;
+    if (a.head_dim > 128) consider((top + 1) / 2, 512); // (two shares of every other group: 3000 rows of 8 heads on 2 of 256 138 us, with a workgroup a CU at most 167)
+    return best;
+}
+uint32_t attention_prefill_mfma_shares(const AttentionParams& a, uint32_t prefix, bool gated) { return prefill_plan(a, prefix, gated).splits; }
+
 uzu_status attention_prefill_mfma(hipStream_t s, const AttentionParams& a, void* out, const void* gate, uint32_t* gate_done) {
     return attention_prefill_mfma_behind(s, a, a.sequence_length > a.suffix_length ? a.sequence_length - a.suffix_length : 0, out, gate, gate_done);
 }
@@ -482,36 +535,16 @@ uzu_status attention_prefill_mfma_behind(hipStream_t s, const AttentionParams& a
         const char* e = lab_env("UZU_ATTN_KSPLIT");
         return e ? atoi(e) : 0;
     }();
-    // Few task groups (few kv heads x short chunks): keep four tasks per workgroup -- they share every staged K / V tile -- and split the KEYS
-    // over workgroups until the chip is covered, instead of thinning the workgroups to one MFMA wave each (r2: 3.4 % MFMA busy at the 0.8B shape).
-    // The shortest shares that the CUs hold, a workgroup each, are the best: of 2043 rows of 8 heads of 256 two shares of every
-    // group took 98.7 us, the last group's being twice the average, one to three shares 77.5; of 517 rows eight shares 24.2, up to nine 18.5.
-    uint32_t tpw = 4, splits = 1;
-    float* part = nullptr;
-    KeyShares shares{0, prefix};
-    const uint32_t groups4 = kv_heads * ((n_tasks + 3) / 4), stretch = a.head_dim <= 128 ? 2 * TK : TK;
     const size_t rows = (size_t)a.suffix_length * a.num_heads;
-    uint32_t units = 0;
-    if (force_split != 1 && groups4 < 192) {
-        const uint32_t n_groups = (n_tasks + 3) / 4;
-        uint64_t all = 0;
-        for (uint32_t y = 0; y < n_groups; ++y) all += key_stretches(shares, y, tpw, a.gqa_factor, a.suffix_length, stretch);
-        // 64 keys a share at least, and no more shares than there can be
-        shares.quantum = std::max({2 * TK / stretch, (uint32_t)(kv_heads * all / 256), key_stretches(shares, n_groups - 1, tpw, a.gqa_factor, a.suffix_length, stretch) / kMaxKeySplits});
-        for (;; ++shares.quantum) {
-            units = 0, splits = 1;
-            for (uint32_t y = 0; y < n_groups; ++y) {
-                const uint32_t n = key_shares(shares, y, tpw, a.gqa_factor, a.suffix_length, stretch);
-                units += n, splits = std::max(splits, n);
-            }
-            if (splits == 1 || kv_heads * units <= 256) break;
-        }
-        if (splits > 1) part = (float*)stream_workspace(s, (size_t)splits * rows * (a.head_dim + 2) * sizeof(float)); // null while a graph is being captured
-        if (!part) splits = 1;
-    }
-    if (splits == 1) { // fewer tasks per workgroup until the grid covers most of the chip
-        shares.quantum = 0;
-        while (tpw > 1 && kv_heads * ((n_tasks + tpw - 1) / tpw) < 192) tpw >>= 1;
+    PrefillPlan plan = force_split == 1 ? PrefillPlan{} : prefill_plan(a, prefix, gate != nullptr);
+    float* part = nullptr;
+    if (plan.splits > 1) part = (float*)stream_workspace(s, (size_t)plan.splits * rows * (a.head_dim + 2) * sizeof(float)); // null while a graph is being captured
+    if (!part) plan = PrefillPlan{};
+    const uint32_t splits = plan.splits, units = plan.units;
+    const KeyShares shares{plan.quantum, prefix};
+    uint32_t tpw = 4;
+    if (splits == 1) {
+        tpw = unsplit_tasks(kv_heads, n_tasks);
         if (force_tpw == 1 || force_tpw == 2 || force_tpw == 4) tpw = force_tpw;
     }
     const dim3 grid(kv_heads, splits > 1 ? units : (n_tasks + tpw - 1) / tpw);
@@ -526,7 +559,8 @@ uzu_status attention_prefill_mfma_behind(hipStream_t s, const AttentionParams& a
         }, "attention_prefill_mfma"));                                                                                                                             \
         if (!part) return UZU_OK;                                                                                                                                  \
         if (gate && gate_done) *gate_done = 1;                                                                                                                     \
-        return launch_check([&] { hipLaunchKernelGGL(attention_prefill_merge_kernel<H>, dim3((uint32_t)((rows + 3) / 4)), dim3(256), 0, s, part_o, part_ml, (uint16_t*)out, (uint32_t)rows, shares, tpw, a.gqa_factor, a.num_heads, gate_done ? (const uint16_t*)gate : nullptr); }, \
+        const auto merge = splits <= 2 ? attention_prefill_merge_kernel<H, 2> : splits <= 4 ? attention_prefill_merge_kernel<H, 4> : splits <= 8 ? attention_prefill_merge_kernel<H, 8> : attention_prefill_merge_kernel<H, kMaxKeySplits>; \
+        return launch_check([&] { hipLaunchKernelGGL(merge, dim3((uint32_t)((rows + 3) / 4)), dim3(256), 0, s, part_o, part_ml, (uint16_t*)out, (uint32_t)rows, shares, tpw, a.gqa_factor, a.num_heads, gate_done ? (const uint16_t*)gate : nullptr); }, \
                             "attention_prefill_merge");                                                                                                            \
     }
     switch (a.head_dim) {
