@@ -1,11 +1,15 @@
 // Which kernel a call goes to, where two are right and one is faster: the rules of the library's dispatch at the sizes that their comments quote measurements for.  Host arithmetic alone.
 #include <cstdio>
+#include <vector>
 
 #include "../../uzu_amd/csrc/attention_prefill.h"
 #include "../../uzu_amd/csrc/kernels.h"
+#include "../../uzu_amd/csrc/kernels_stream32.h"
 #include "../../uzu_amd/csrc/tree_pass.h"
 
 using namespace uzu::k;
+
+namespace uzu { namespace k { bool window_attention_f32_supported(const WindowAttentionParams& p); } } // (between k_window_attention.hip and k_window_attention_f32.hip)
 
 static int bad = 0;
 static void expect(bool got, bool want, const char* what) {
@@ -40,6 +44,29 @@ int main() {
         const uint32_t shares = attention_prefill_mfma_shares(a, t.prefix, t.gated);
         if (shares < t.least || shares > t.most) printf("prompt attention, %u heads on %u of %u, %u rows behind %u keys: %u shares\n", t.heads, t.kv_heads, t.head_dim, t.rows, t.prefix, shares), ++bad;
     }
+    struct Window {
+        uint32_t rows, heads, kv_heads, dim, window;
+        bool want;
+    };
+    for (const bool step : {true, false})
+        for (const Window& t : step ? std::vector<Window>{{8, 16, 4, 128, 1024, true}, {48, 32, 8, 128, 0, true}, {2, 64, 8, 64, 1024, true}, {8, 64, 8, 64, 1024, false}, {48, 64, 8, 64, 256, true}, {48, 64, 8, 64, 1024, true},
+                                                          {12, 64, 8, 64, 0, true}, {12, 40, 8, 128, 1024, true}, {4, 24, 2, 128, 1024, true}, {12, 24, 2, 128, 1024, false}, {12, 24, 2, 128, 0, false}, {24, 24, 2, 128, 512, false}}
+                                    : std::vector<Window>{{300, 8, 2, 128, 0, true}, {16, 8, 2, 128, 0, true}, {16, 8, 2, 128, 64, false}, {64, 16, 4, 128, 64, false}, {200, 8, 2, 128, 64, true}, {32, 8, 2, 128, 128, false},
+                                                          {16, 8, 2, 128, 192, true}, {300, 8, 2, 128, 1024, true}}) {
+            WindowAttentionParams p{};
+            p.rows = t.rows, p.nseq = step ? t.rows : 1, p.heads = t.heads, p.kv_heads = t.kv_heads, p.dim = p.vdim = t.dim, p.ldq = t.heads * t.dim, p.window = t.window, p.splits = 1, p.one_row = step, p.cache_bf16 = step;
+            char what[160];
+            snprintf(what, sizeof what, "%s attention, %u rows of %u heads on %u of %u, window %u", step ? "step" : "f32 prompt", t.rows, t.heads, t.kv_heads, t.dim, t.window);
+            expect(step ? window_attention_step_supported(p) : window_attention_f32_supported(p), t.want, what);
+        }
+    for (const uint32_t outputs : {8u, 32u, 64u})
+        for (const uint32_t d : {256u, 1024u, 2048u}) {
+            RouteGroupsParams p{};
+            p.outputs = outputs, p.d = d, p.rows = 8, p.top = 2;
+            char what[100];
+            snprintf(what, sizeof what, "norm and routing of %u outputs, rows of %u", outputs, d);
+            expect(norm_route_faster(p), outputs <= 32 || d == 2048, what);
+        }
     printf("%d bad\n", bad);
     return bad != 0;
 }

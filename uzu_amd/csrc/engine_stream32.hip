@@ -418,7 +418,9 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
                 join_add.y = S.tmp, join_add.residual = cur, join_add.out = slot, join_add.scales = L.post_mixer.scales, join_add.layer_scale = X.ls1, join_add.offset = L.post_mixer.offset;
                 join_add.eps = L.post_mixer.eps, join_add.next = S.normed, join_add.next_scales = next->scales, join_add.next_offset = next->offset, join_add.next_eps = next->eps;
                 join_add.rows = rows, join_add.d = d;
-                join_waits = k::norm_route_supported(join_add, route_params(S.normed));
+                const k::RouteGroupsParams route = route_params(S.normed);
+                join_waits = k::norm_route_supported(join_add, route) &&
+                             (k::norm_route_faster(route) || k::norm_route_gate_up_supported(join_add, route, L.moe.w13, h.moe.expert_hidden_dim, expert_act(h.moe)));
             }
             if (!join_waits) add_normed(S.tmp, cur, slot, L.post_mixer, X.ls1, next);
             normed_ready = h.no_mlp && !h.has_ple && next_pre;

@@ -317,9 +317,16 @@ uzu_status norm_linear(hipStream_t s, const NormAddParams& n, const LinearF32Par
         if (part_value) hipLaunchKernelGGL((norm_linear_kernel<J, true>), grid, dim3(kStepThreads), (size_t)n.d * 4, s, n, p, part_value, part_index);                           \
         else hipLaunchKernelGGL((norm_linear_kernel<J, false>), grid, dim3(kStepThreads), (size_t)n.d * 4, s, n, p, part_value, part_index);                                     \
     }, "norm_linear")
-    if (n.d <= 1024) UZU_NL(2);
-    if (n.d <= 2048) UZU_NL(4);
-    UZU_NL(8);
+    switch ((n.d + 511) / 512) { // (a piece that lies past the row's end is loaded for nothing: 2560 with eight, 4096 columns 14.5 us; with five XX)
+    case 1: UZU_NL(1);
+    case 2: UZU_NL(2);
+    case 3: UZU_NL(3);
+    case 4: UZU_NL(4);
+    case 5: UZU_NL(5);
+    case 6: UZU_NL(6);
+    case 7: UZU_NL(7);
+    default: UZU_NL(8);
+    }
 #undef UZU_NL
 }
 bool step_turn_supported(const StepTurnParams& p) {
@@ -338,6 +345,11 @@ bool norm_route_supported(const NormAddParams& n, const RouteGroupsParams& p) {
     return norm_add_step_supported(n) && p.d == n.d && n.rows == p.rows && p.keep == p.groups && p.outputs >= 1 && p.outputs <= kStepMaxOutputs && p.top >= 1 && p.top <= std::min(p.outputs, kStepMaxTop) &&
            p.router && p.ids && p.weights && ((uintptr_t)p.router & 15) == 0;
 }
+// Eight waves have a workgroup's outputs here, sixteen in moe_route_groups: of many outputs of short rows, whose row is no work, the second is as much faster as a launch costs.  Us, apart and joined (with the
+// experts behind): 64 outputs, 8 rows of 256 15.3 / 16.2, 1024 22.0 / 22.1, 2048 43.3 / 41.1, 64 rows of 512 31.0 / 31.9; 32 outputs, 8 rows of 1024 25.5 / 23.5.  With the first products in the same launch it
+// is the faster one at every size that it takes, though every workgroup works the choice out for itself: one row, 2 winners of 1024, 64 outputs of 256 11.6 / 10.9 (512 hidden units), of 1024 18.2 / 13.5, of 2048
+// 21.9 / 14.8, of 4096 54.3 / 24.0; 8 winners of 64, 4096 83.1 / 41.5.
+bool norm_route_faster(const RouteGroupsParams& p) { return p.outputs <= 32 || p.d >= 1536; }
 uzu_status norm_route_rows(hipStream_t s, const NormAddParams& n, const RouteGroupsParams& p) {
     if (!p.rows) return UZU_OK;
     UZU_REQUIRE(norm_route_supported(n, p), "norm_route: rows of %u, %u of %u outputs", n.d, p.top, p.outputs);

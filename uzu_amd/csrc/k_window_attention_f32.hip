@@ -161,7 +161,10 @@ __global__ void __launch_bounds__(64 * kWaves) window_attention_f32_kernel(Windo
 }
 } // namespace
 
+// Short windows and few rows are left to the simple form: a wave has few keys there, and a tile of sixteen rows has the windows of all of them.  Us, simple and here: 8 heads of 128, window 64, 16 / 64 /
+// 100 rows 6.8 / 9.7, 7.6 / 9.7, 9.4 / 9.9; window 128, 48 rows 11.3 / 11.7; 16 heads, window 64, 64 / 100 rows 9.5 / 9.9, 12.6 / 10.0; 32 heads of 64, window 64, 32 rows 6.8 / 6.7; window 192 is here always.
 bool window_attention_f32_supported(const WindowAttentionParams& p) {
+    if (p.window && p.window <= 128 && (uint64_t)p.rows * p.heads * p.window <= 65536) return false;
     return !p.cache_bf16 && (p.dim == 64 || p.dim == 128) && (p.vdim == 64 || p.vdim == 128) && p.nseq && p.rows >= kRows * p.nseq && p.ldq % 4 == 0 && ((uintptr_t)p.q & 15) == 0 && p.heads <= 65535;
 }
 

@@ -190,6 +190,7 @@ struct NormAddParams {
 bool norm_add_step_supported(const NormAddParams& n); // rows of up to 4096, a multiple of 8
 // ... and moe_route_groups of next (one group of outputs, up to 64 of them, up to 8 winners) in one launch; p.x is not read
 bool norm_route_supported(const NormAddParams& n, const RouteGroupsParams& p);
+bool norm_route_faster(const RouteGroupsParams& p); // than the two launches, without the experts' first products
 uzu_status norm_route_rows(hipStream_t s, const NormAddParams& n, const RouteGroupsParams& p);
 // ... and, one row, moe_experts_gate_up of the winners as well (weight_on_input: the winners' weights multiply their products).  n.out apart from n.residual and n.y.
 bool norm_route_gate_up_supported(const NormAddParams& n, const RouteGroupsParams& p, const uint16_t* w13, uint32_t ff, const ExpertAct& act);
