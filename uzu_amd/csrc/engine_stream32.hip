@@ -283,9 +283,10 @@ k::StepTurnParams s32_turn_params(const uzu_hip_model* m, const uzu_hip_state* s
 // The launches of one pass (tables uploaded before): rows = sum of the sequences' counts (<= max_rows), token ids on the device, row-major in sequence order;
 // n_out rows (S.d_out_rows) get logits in S.logits [n_out][vocab] f32.  Nothing here depends on the sequences' positions -- the kernels read them from the
 // device-side spans -- so a one-token step can be captured once and replayed.  Does not move the sequences' context lengths.
+// longest: the keys of the longest sequence, this pass's among them (0: a captured pass, which holds for every length).
 // in_order: row i of the wanted logits is row i of the pass, all of them.  turn (decode steps that chain, s32_turn_params): the rows' embedding and the first norm are there already, and the
 // read-out leaves its parts' largest logits in S.turn_value / turn_index, *turn of them.
-uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, const uint32_t* d_tokens, uint32_t n_out, bool in_order = false, uint32_t* turn = nullptr) {
+uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, const uint32_t* d_tokens, uint32_t n_out, bool in_order = false, uint32_t* turn = nullptr, uint32_t longest = 0) {
     Stream32& S = *m->s32;
     hipStream_t s = m->ctx->stream; // (the stream the next launch goes to: a pair's first mixer switches it to S.side and back)
     const hipStream_t main_stream = s;
@@ -554,6 +555,7 @@ uzu_status s32_encode(uzu_hip_model* m, const std::vector<uint32_t>& counts, con
             // decode-sized passes: spread a tile's key blocks over workgroups (a constant of the layer, so that a captured step stays valid as the context grows)
             uint32_t keys = h.sliding_window_size ? h.sliding_window_size : m->d.max_context_length;
             if (h.attention_chunk_size) keys = std::min(keys, h.attention_chunk_size);
+            ap.keys = longest;
             ap.one_row = max_count == 1;
             if (rows <= 4 * S.max_seqs && rows * H <= 4096) ap.split_ws = S.att_ws, ap.split_ws_bytes = S.att_ws_bytes, k::window_attention_split_keys(ap, keys, m->ctx->num_cus);
             state_beside = joint && k::window_attention_step_supported(ap) && k::window_attention_step_beside(state_params());
@@ -841,7 +843,9 @@ uzu_status s32_pass(uzu_hip_model* m, const std::vector<PassSeq>& seqs, const ui
     for (const PassSeq& q : seqs) counts.push_back(q.count);
     bool in_order = true;
     for (size_t i = 0; i < out_rows.size(); ++i) in_order &= out_rows[i] == i;
-    return s32_encode(m, counts, d_tokens, (uint32_t)out_rows.size(), in_order);
+    uint32_t longest = 0;
+    for (const PassSeq& q : seqs) longest = std::max(longest, q.start + q.count);
+    return s32_encode(m, counts, d_tokens, (uint32_t)out_rows.size(), in_order, nullptr, longest);
 }
 
 uzu_status ensure_logits(uzu_hip_model* m, size_t rows) {

@@ -32,7 +32,7 @@ __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hi, uint3
 // itself at every exponential and every staged block (the next block's loads are in flight meanwhile; values are transposed two keys at a time).  2048 rows of 16 heads on 4,
 // width 128, window 1024: 147 us with four waves and no look-ahead, 61 so.  SPLIT (few items, many keys: passes of a few rows a sequence, which k_window_attention_step.hip does not take): grid.z
 // workgroups share an item tile's stretches (stretch i goes to workgroup i mod grid.z) and leave unnormalised sums with their running maximum / denominator in p.split_ws;
-// window_attention_merge (k_window_attention_step.hip) combines them.  Two forms (window_attention_split_keys): IW 4, KG 1, stretches of 32 keys, and IW 1, KG 4, stretches of 128 (with IW 4 three waves
+// window_attention_mfma_merge_kernel combines them.  Two forms (window_attention_split_keys): IW 4, KG 1, stretches of 32 keys, and IW 1, KG 4, stretches of 128 (with IW 4 three waves
 // of four have no items, but they help staging).  The sink belongs to group 0 of split 0.
 // AHEAD: the next stretch's loads are in flight while one is computed.
 template <int NB, int IW, int KG, bool SPLIT, bool AHEAD> // dim and vdim padded to RP = 32 NB
@@ -261,6 +261,32 @@ __global__ void __launch_bounds__(64 * IW * KG) window_attention_mfma_kernel(Win
         }
 }
 
+// a workgroup per item: out = sum_s e^(m_s - M) O_s / sum_s e^(m_s - M) l_s over the splits, in split order (a split that saw no key has l = 0 and m = -1e30).  (The step form's merge, for up to 32
+// shares and with a norm beside it, is slower behind this form: 64 heads on 8 of 64, 4 rows, window 1024 11.7 us in all for 10.7.)
+// (gate: the item's result times sigmoid(gate[row, head]), item = row * heads + head)
+__global__ void __launch_bounds__(128) window_attention_mfma_merge_kernel(const float* ws, float* out, uint32_t splits, uint32_t vdim, uint32_t rp, const float* gate, uint32_t ldgate,
+                                                                     uint32_t heads, uint32_t ldo, float out_scale) {
+    const uint32_t item = blockIdx.x, tid = threadIdx.x;
+    const float* base = ws + (size_t)item * splits * (rp + 4);
+    // the splits' weights once, a lane per split (at most 64 splits); the sums over the splits run in split order
+    __shared__ float s_w[64], s_l[64];
+    if (tid < 64) {
+        const float m = tid < splits ? base[(size_t)tid * (rp + 4) + rp] : -1.0e30f;
+        s_l[tid] = tid < splits ? base[(size_t)tid * (rp + 4) + rp + 1] : 0.0f;
+        s_w[tid] = fast_exp(m - wave_max(m));
+    }
+    __syncthreads();
+    float den = 0.0f;
+    for (uint32_t s = 0; s < splits; ++s) den = fmaf(s_w[s], s_l[s], den);
+    if (gate) den *= 1.0f + expf(-gate[(size_t)(item / heads) * ldgate + item % heads]);
+    for (uint32_t c = tid; c < vdim; c += 128) {
+        float acc = 0.0f;
+#pragma unroll 8
+        for (uint32_t s = 0; s < splits; ++s) acc = fmaf(s_w[s], base[(size_t)s * (rp + 4) + c], acc);
+        out[(size_t)(item / heads) * ldo + (size_t)(item % heads) * vdim + c] = acc / den * out_scale;
+    }
+}
+
 uint32_t blocks_of(const WindowAttentionParams& p) {
     const uint32_t w = p.dim > p.vdim ? p.dim : p.vdim;
     return w <= 32 ? 1 : w <= 64 ? 2 : w <= 128 ? 4 : 0;
@@ -275,7 +301,7 @@ size_t window_attention_split_ws_bytes(uint32_t rows, uint32_t heads, uint32_t s
 // of 128: one sequence, window 40 9.8 / 14.0, 128 10.5 / 14.4, 512 (16 splits) 10.1 / 15.4 (4), 1024 (16) 12.6 / 14.6 (8); 8 sequences, window 256 (8) 10.5 / 14.8 (2),
 // 512 (8) 13.0 / 15.1 (4), 1024 (8) 18.3 / 14.1 (8); 32 sequences, window 128 (2) 13.3 / 14.5 (2), 256 (2) 18.5 / 14.6 (2).  Up to 32 keys the simple form is as fast.
 void window_attention_split_keys(WindowAttentionParams& p, uint32_t keys, uint32_t num_cus) {
-    p.splits = 1; // (the step form with one share: whether it takes the shape at all)
+    p.keys = p.keys ? std::min(p.keys, keys) : keys, p.splits = 1; // (the step form with one share: whether it takes the shape at all)
     if (window_attention_step_supported(p)) {
         p.splits = window_attention_step_splits(p, keys, num_cus);
         if (p.split_ws) p.splits = std::max<uint32_t>(1, std::min<size_t>(p.splits, p.split_ws_bytes / window_attention_split_ws_bytes(p.rows, p.heads, 1)));
@@ -312,7 +338,8 @@ uzu_status window_attention_mfma(hipStream_t s, const WindowAttentionParams& p) 
     if (use_split(p)) {
         if (p.split_items == 128) UZU_PROPAGATE(nb == 1 ? (launch<1, 4, 1, true>(s, p)) : nb == 2 ? (launch<2, 4, 1, true>(s, p)) : (launch<4, 4, 1, true>(s, p)));
         else UZU_PROPAGATE(nb == 1 ? (launch<1, 1, 4, true>(s, p)) : nb == 2 ? (launch<2, 1, 4, true>(s, p)) : (launch<4, 1, 4, true>(s, p)));
-        return window_attention_merge(s, p, nullptr);
+        return launch_check([&] { hipLaunchKernelGGL(window_attention_mfma_merge_kernel, dim3(p.rows * p.heads), dim3(128), 0, s, (const float*)p.split_ws, p.out, p.splits, p.vdim, 32 * nb, p.gate, p.ldgate, p.heads, p.ldo, p.out_scale); },
+                            "window_attention_merge");
     }
     // Prompts with more tiles than CUs: a second tile on the CU covers a wave's waits as the second key group does, and the groups have to meet.  Us, one group and two: heads of 64, 2048
     // rows of 32 heads on 8 (512 tiles), window 64 / 256 / 512 / none 16.3 / 30.8 / 50.0 / 158 and 21.5 / 35.3 / 53.3 / 157; 1500 rows of 64 on 8 (752), 64 / 512 / none 21.8 / 61.1 / 124 and

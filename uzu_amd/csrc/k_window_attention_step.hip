@@ -216,14 +216,14 @@ uint32_t heads_a_block(const WindowAttentionParams& p) { return p.heads / p.kv_h
 
 } // namespace
 
-// A key / value head with more than four query heads has its keys read once per four of them here, and once by the matrix-core form, whose tiles they fill better: with many rows over long windows that form
-// is the faster one (us, matrix cores and here, window 1024: 64 heads on 8 of 64, 2 / 8 / 48 rows 11.4 / 9.4, 11.9 / 15.4, 50 / 37; 24 on 2 of 128, 4 / 8 / 48 rows 13.5 / 11.6, 13.9 / 15.6, 38 / 55; window 512
-// 11.1 / 9.0, 11.5 / 11.8, 25 / 31; 40 on 8 of 128 is here always).  Without a window the rows see what there is: groups of more than eight count as of 1024 keys.
+// A key / value head with more than four query heads has its keys read once per four of them here, and once by the matrix-core form, whose tiles they fill better: with many rows over long stretches of
+// keys that form is the faster one.  Us, matrix cores and here, 1024 keys: 64 heads on 8 of 64, 2 / 8 / 48 rows 11.4 / 9.4, 11.9 / 15.4, 50 / 37; 24 on 2 of 128, 4 / 8 / 48 rows 13.5 / 11.6, 13.9 / 15.6,
+// 38 / 55; 512 keys 11.1 / 9.0, 11.5 / 11.8, 25 / 31; 40 on 8 of 128, 12 rows, 300 / 1500 / 4000 keys 46 / 16, 61 / 46, 90 / 107.
 static bool step_faster(const WindowAttentionParams& p) {
-    const uint32_t blocks = (p.heads / p.kv_heads + 3) / 4, units = p.rows * p.kv_heads * blocks;
-    if (blocks == 1 || (p.window && p.window <= 256)) return true;
-    if (blocks > 2) return units * (uint64_t)(p.window ? std::min(p.window, 1024u) : 1024u) <= 32 * 1024;
-    return width_blocks(p) > 2 || p.window < 1024 || units < 48 || units >= 512;
+    const uint32_t blocks = (p.heads / p.kv_heads + 3) / 4, units = p.rows * p.kv_heads * blocks, keys = p.keys ? p.keys : p.window ? p.window : 1024u;
+    if (blocks == 1 || keys <= 128 || (!p.window && keys < 1000)) return true; // (without a window the matrix-core form's shares are cut for as many keys as there can be)
+    if (blocks > 2) return (uint64_t)units * std::min(keys, 2048u) <= 40 * 1024;
+    return width_blocks(p) > 2 ? keys < 3000 || units < 32 || units >= 512 : keys < 1024 || units < 48 || units >= 512;
 }
 bool window_attention_step_supported(const WindowAttentionParams& p) {
     return p.one_row && p.rows == p.nseq && p.cache_bf16 && width_blocks(p) && p.dim % 8 == 0 && p.vdim % 8 == 0 && p.ldq % 4 == 0 && p.kv_heads && p.heads % p.kv_heads == 0 && step_faster(p) &&

@@ -391,6 +391,7 @@ struct WindowAttentionParams {
     uint32_t splits, split_items; // split_items: items a workgroup takes, 128 (stretches of 32 keys) or 32 (of 128; also 0)
     float* split_ws;
     size_t split_ws_bytes;
+    uint32_t keys;    // that a row of this pass sees at the most, as far as the caller knows (the form rests on it); 0: not known (window_attention_split_keys sets its own)
     uint32_t one_row; // every sequence of the pass brings exactly one row (row r is sequence r's): the step form, with `splits` >= 1 shares of a row's keys
 };
 // `splits` and `split_items` of a decode-sized pass whose rows see `keys` keys at the most, from `rows`, `tiles` and `kv_heads`: at most 16 splits, of the step form at most 32
