@@ -109,6 +109,12 @@ def test_tree_attention_at_its_edges(tmp_path):
 
 
 @pytest.mark.gpu
+def test_norm_and_projection_in_one_launch(tmp_path):
+    """tests/host/step_linear_check.cpp: widths with and without a ragged end, the largest result, an infinite weight."""
+    _run_against_the_library(tmp_path, "step_linear_check")
+
+
+@pytest.mark.gpu
 def test_gated_epilogue_has_the_exact_silu_for_every_gate(tmp_path):
     """tests/host/gated_silu_check.cpp: the quick quotient of csrc/gemm128_epilogue.h on the device, through the library's product, on each of its forms."""
     import subprocess

@@ -209,9 +209,10 @@ __global__ void __launch_bounds__(kStepThreads) norm_linear_kernel(NormAddParams
     auto load = [&](uint32_t col, u32x4_v (&to)[J]) {
         const uint16_t* row = p.w + (size_t)min(col, p.n - 1) * k;
 #pragma unroll
-        for (int j = 0; j < J; ++j) to[j] = *(const u32x4_v*)(row + min(j * 512 + lane * 8, k - 8)); // (pieces past the row's end meet zeros)
+        for (int j = 0; j < J; ++j) to[j] = *(const u32x4_v*)(row + min(j * 512 + lane * 8, k - 8)); // (the last piece may pass the row's end: `in_last`)
     };
     uint32_t col = blockIdx.x * kStepWaves + wave;
+    const bool in_last = (J - 1) * 512 + lane * 8 < k;
     load(col, w);
     step_norm_add(n, 0, s_x, s_red, p.bf16_products, blockIdx.x == 0);
     __syncthreads();
@@ -224,6 +225,8 @@ __global__ void __launch_bounds__(kStepThreads) norm_linear_kernel(NormAddParams
     uint32_t bi = 0xFFFFFFFFu;
     for (; col < p.n; col += waves) {
         load(col + waves, next);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[J - 1][i] = in_last ? w[J - 1][i] : 0u; // (a zero coordinate does not stand against a weight that is not finite)
         float acc = 0.0f;
 #pragma unroll
         for (int j = 0; j < J; ++j)
