@@ -69,6 +69,12 @@ int main() {
             snprintf(what, sizeof what, "norm and routing of %u outputs, rows of %u", outputs, d);
             expect(norm_route_faster(p), outputs <= 32 || d == 2048, what);
         }
+    for (const uint32_t heads : {4u, 32u, 48u, 64u, 72u})
+        for (const uint32_t nodes : {1u, 10u, 13u, 16u, 17u, 28u, 32u}) {
+            char what[100];
+            snprintf(what, sizeof what, "a tree's DeltaNet layer in one launch, %u heads, %u nodes", heads, nodes);
+            expect(delta_net_tree_step_faster(nodes, heads), heads <= 32 || (heads == 72 ? nodes >= 13 : nodes == 17 || nodes == 28), what);
+        }
     printf("%d bad\n", bad);
     return bad != 0;
 }

@@ -432,7 +432,7 @@ void delta_net_tree_core(Enc& e, DLayer& L, uint32_t layer, uint32_t n) {
     const uint32_t key_dim = Hk * Dk, value_dim = Hv * Dv, conv_dim = 2 * key_dim + value_dim;
     const uint32_t total_proj_dim = conv_dim + value_dim + 2 * Hv, ks = L.d.dn_kernel_size;
     uzu_hip_model::TreeLayer& T = m->tree.layers[layer];
-    if (k::delta_net_tree_step_supported(m->in_proj, L.ssm_state, n, ks, Hk, Hv, Dk, Dv)) {
+    if (k::delta_net_tree_step_supported(m->in_proj, L.ssm_state, n, ks, Hk, Hv, Dk, Dv) && k::delta_net_tree_step_faster(n, Hv)) {
         RUN("dn_tree_step", (size_t)Hv * Dv * Dk * 4, k::delta_net_tree_step(e.s, m->in_proj, L.conv_w, L.conv_b, L.conv_state, m->tree.d_parents, m->tree.d_trie, L.a_log, L.dt_bias, L.ssm_state,
                                                                            T.conv_states, T.k, T.v, T.beta, T.log_decay, m->delta_out, n, ks, Hk, Hv));
     } else {

@@ -606,6 +606,10 @@ bool delta_net_tree_step_supported(const uint16_t* in_proj, const float* h0, uin
     return n && n <= kDnTreeMaxNodes && kernel_size >= 2 && kernel_size <= kTreeStepMaxKernel && Dk == 128 && Dv == 128 && Hk && Hv && Hv % Hk == 0 && Hv % 4 == 0 /* rows of 16 bytes' multiples */ &&
            (((uintptr_t)in_proj | (uintptr_t)h0) & 15) == 0;
 }
+// A workgroup has a CU to itself (82 KB of LDS), so from 33 heads on they come in rounds of 32 heads, and it depends on the nodes what a round more costs.  Us, the two launches and this one:
+// 32 heads, 2 / 13 / 32 nodes 12.2 / 7.9, 18.0 / 10.4, 31.4 / 18.9; 48 heads, 2 / 8 / 16 / 17 / 28 / 32 nodes 12.8 / 14.4, 14.8 / 16.3, 20.7 / 20.8, 25.9 / 22.8, 32.4 / 31.7, 33.2 / 34.9, of 64 heads
+// within 0.4 of these; 72 heads, 2 / 10 / 13 / 32 nodes 18.5 / 20.8, 25.3 / 25.5, 29.6 / 27.7, 57.3 / 51.3.
+bool delta_net_tree_step_faster(uint32_t n, uint32_t Hv) { return Hv <= 32 || (Hv <= 64 ? n > 16 && n <= 28 : n > 10); }
 uzu_status delta_net_tree_step(hipStream_t s, const uint16_t* in_proj, const float* conv_w, const float* conv_b, const float* base_state, const int32_t* parents, const uint32_t* trie,
                                const float* a_log, const float* dt_bias, const float* h0, float* suffix_state, uint16_t* k_out, uint16_t* v_out, float* beta_out, float* log_decay_out,
                                uint16_t* out, uint32_t n, uint32_t kernel_size, uint32_t Hk, uint32_t Hv) {

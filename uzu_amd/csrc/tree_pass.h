@@ -22,6 +22,7 @@ uzu_status attention_tree(hipStream_t s, const AttentionParams& a, uint32_t key_
 // ConvTreeScan, the tree's preparation and the tree-verify composite in one launch, bit-identical to delta_net_tree_prep + delta_net_tree_verify (k_deltanet_tree.hip).  Nodes in
 // depth-first order (an ancestor in front of its descendants).
 bool delta_net_tree_step_supported(const uint16_t* in_proj, const float* h0, uint32_t n, uint32_t kernel_size, uint32_t Hk, uint32_t Hv, uint32_t Dk, uint32_t Dv);
+bool delta_net_tree_step_faster(uint32_t n, uint32_t Hv); // than the two
 uzu_status delta_net_tree_step(hipStream_t s, const uint16_t* in_proj, const float* conv_w, const float* conv_b, const float* base_state, const int32_t* parents, const uint32_t* trie,
                                const float* a_log, const float* dt_bias, const float* h0, float* suffix_state, uint16_t* k_out, uint16_t* v_out, float* beta_out, float* log_decay_out,
                                uint16_t* out, uint32_t n, uint32_t kernel_size, uint32_t Hk, uint32_t Hv);
