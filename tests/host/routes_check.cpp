@@ -4,6 +4,7 @@
 
 #include "../../uzu_amd/csrc/attention_prefill.h"
 #include "../../uzu_amd/csrc/kernels.h"
+#include "../../uzu_amd/csrc/kernels_decode.h"
 #include "../../uzu_amd/csrc/kernels_stream32.h"
 #include "../../uzu_amd/csrc/tree_pass.h"
 
@@ -75,6 +76,18 @@ int main() {
             snprintf(what, sizeof what, "a tree's DeltaNet layer in one launch, %u heads, %u nodes", heads, nodes);
             expect(delta_net_tree_step_faster(nodes, heads), heads <= 32 || (heads == 72 ? nodes >= 13 : nodes == 17 || nodes == 28), what);
         }
+    struct Large {
+        uint32_t n, k, act_mul;
+        bool want;
+    };
+    for (const Large& t : {Large{2048, 4096, 0, true}, {2046, 4096, 0, false}, {2048, 4096, 1, false}, {2144, 4096, 1, true}, {2048, 8192, 1, false}, {2560, 8192, 1, true}, {6144, 2048, 1, false}, {6400, 2048, 1, true},
+                           {4096, 2048, 0, true}, {28672, 4096, 1, true}, {28672, 4064, 0, false}}) {
+        DecGemvParams p{};
+        p.n[0] = t.n, p.k = t.k, p.bits = 8, p.b_kind = UZU_MATMUL_B_SCALE_BIAS, p.group_size = 32, p.act_mul = t.act_mul;
+        char what[100];
+        snprintf(what, sizeof what, "the stream of an int8 matrix of %u rows of %u%s", t.n, t.k, t.act_mul ? ", gated" : "");
+        expect(gemv_large_wanted(p, 256), t.want, what);
+    }
     printf("%d bad\n", bad);
     return bad != 0;
 }

@@ -1156,7 +1156,7 @@ uzu_status gemv_dec(hipStream_t s, const DecGemvParams& p_in, int num_cus, uint3
         const uzu_status st = gemv_stream(s, p_in, num_cus, grid_out);
         if (st != UZU_ERR_UNSUPPORTED) return st;
     }
-    if (gemv_large_wanted(p)) return gemv_large(s, p, num_cus, grid_out); // (k_decode_large.hip)
+    if (gemv_large_wanted(p, num_cus)) return gemv_large(s, p, num_cus, grid_out); // (k_decode_large.hip)
     int lpr_log2, R;
     bool wide = false;
     const uint32_t want = gemv_dec_plan(p, num_cus, &lpr_log2, &R, &wide);

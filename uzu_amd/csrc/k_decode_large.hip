@@ -277,10 +277,13 @@ template <int D, bool ACT> uzu_status launch_large_p(hipStream_t s, const DecGem
 
 // int8 with bf16 scales and offsets, whole steps of a wave, from 8 MB on (below, a CU's share is over before the row is staged).  int4 is not better off: its conversion wants the sixteen
 // waves of gemv_dec (Llama-3-8B's up, down and read-out 16.3 / 9.0 / 50.9 us there, 17.3 / 9.5 / 68.5 as a stream).
-bool gemv_large_wanted(const DecGemvParams& p) {
+// Gated rows: gemv_dec holds four pairs a CU at once, of K = 2048 twelve, and is the faster one up to there (up / gate, us, gemv_dec and here: 2048 x 4096 6.7 / 8.3, 2144 x 4096 9.0 / 8.4, 2048 x 8192
+// 12.7 / 13.0, 2560 x 8192 17.4 / 13.4, 6144 x 2048 7.7 / 8.0, 6400 x 2048 9.3 / 8.1).
+bool gemv_large_wanted(const DecGemvParams& p, int num_cus) {
     const bool normed = p.norm_scales || p.norm_plain;
     if (p.bits != 8 || p.b_kind != UZU_MATMUL_B_SCALE_BIAS || p.k % 2048 || p.k > 32768 || p.group_size < 32 || (p.group_size & (p.group_size - 1)) || p.k % p.group_size || (normed && p.k > 8192)) return false;
     if (p.conv_w || p.dg_o || p.x_rht_bits || p.in_rht_bits || p.ep_out_bits || (p.act_mul && (p.n[1] || p.part_val || p.out_f32))) return false;
+    if (p.act_mul && p.n[0] / 2 <= (p.k == 2048 ? 12u : 4u) * (uint32_t)num_cus) return false;
     return (uint64_t)std::max(p.n[0], p.n[1]) * p.k < 0xFFFFF000ull && ((uint64_t)p.n[0] + p.n[1]) * p.k >= (8ull << 20);
 }
 uzu_status gemv_large(hipStream_t s, const DecGemvParams& p, int num_cus, uint32_t* grid_out) {

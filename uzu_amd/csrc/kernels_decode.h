@@ -116,7 +116,7 @@ struct DecGemvParams {
 bool gemv_dec_stripe_supported(const DecGemvParams& p, int num_cus);
 uint32_t gemv_dec_grid(const DecGemvParams& p, int num_cus, int* lpr_log2, int* R);
 uzu_status gemv_dec(hipStream_t s, const DecGemvParams& p, int num_cus, uint32_t* grid_out);
-bool gemv_large_wanted(const DecGemvParams& p); // k_decode_large.hip: matrices of the bandwidth regime
+bool gemv_large_wanted(const DecGemvParams& p, int num_cus); // k_decode_large.hip: matrices of the bandwidth regime
 uzu_status gemv_large(hipStream_t s, const DecGemvParams& p, int num_cus, uint32_t* grid_out);
 bool gemv_dec_plain_in_rht_supported(uint32_t k, uint32_t bits); // in_rht_bits on a plain (not normalised, not norm-gated) input row
 // The weight-streaming engine (k_stream.hip): LDS-DMA loader wave + consumer waves per CU; same arithmetic as gemv_dec.  gemv_dec
