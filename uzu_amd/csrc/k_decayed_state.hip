@@ -206,7 +206,7 @@ template <bool CHANNEL> __global__ void __launch_bounds__(256) decayed_state_sca
 // A decay per channel: a wave owns the block of 16 x 16 scores on the diagonal that bears its number (running products, lane = (key row, quarter of the slab)) and up to
 // two of the six blocks below it (v_mfma_f32_16x16x4_f32).  Results: wave w has rows 32 (w / 2) .., column tiles NQ (w % 2) ..
 template <bool CHANNEL, int NQ, bool FOURS>
-__global__ void __launch_bounds__(256, CHANNEL || NQ > 1 ? 2 : 3) decayed_state_out_kernel(DecayedStateParams p, const float* ws) {
+__global__ void __launch_bounds__(256, CHANNEL || NQ > 1 ? 2 : FOURS ? 4 : 3) decayed_state_out_kernel(DecayedStateParams p, const float* ws) {
     constexpr uint32_t SW = 32, PW = SW + 4, VW = 64 * NQ, ROWS = kChunk * PW; // a slab row's pitch: 16-byte aligned, rows on distinct banks
     constexpr uint32_t BUF = CHANNEL ? 5 * ROWS : 2 * ROWS;
     __shared__ __attribute__((aligned(16))) float s_buf[BUF > kChunk * VW ? BUF : kChunk * VW];
@@ -290,7 +290,6 @@ __global__ void __launch_bounds__(256, CHANNEL || NQ > 1 ? 2 : 3) decayed_state_
     auto below_j = [&](uint32_t pair) { const uint32_t i = below_i(pair); return pair - i * (i - 1) / 2; };
     f32x4_m lower[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     const uint32_t row = pi * 32 + l32; // this lane's row of the query operand
-    float from_start = 1.0f;
     for (uint32_t d0 = 0; d0 < dim; d0 += SW) {
         float sv[SW / 2][NQ]; // the carried state's rows of the slab
 #pragma unroll
@@ -382,7 +381,6 @@ __global__ void __launch_bounds__(256, CHANNEL || NQ > 1 ? 2 : 3) decayed_state_
                 }
             }
         } else {
-            if (d0 == 0) from_start = s_h[2][row];
             // (both operands out of LDS before the first product, and one condition around all of them)
             f32x4_m qv[SW / 8], kv[SW / 8];
 #pragma unroll
@@ -393,6 +391,7 @@ __global__ void __launch_bounds__(256, CHANNEL || NQ > 1 ? 2 : 3) decayed_state_
                 for (uint32_t d = 0; d < SW / 2; ++d) sc = __builtin_amdgcn_mfma_f32_32x32x2f32(qv[d / 4][d % 4], kv[d / 4][d % 4], sc, 0, 0, 0);
             }
             if (carried) {
+                const float from_start = s_h[2][row]; // (read here: a register held across the slabs was the 129th of 128)
 #pragma unroll
                 for (uint32_t d = 0; d < SW / 2; ++d)
 #pragma unroll
