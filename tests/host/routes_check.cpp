@@ -88,6 +88,23 @@ int main() {
         snprintf(what, sizeof what, "the stream of an int8 matrix of %u rows of %u%s", t.n, t.k, t.act_mul ? ", gated" : "");
         expect(gemv_large_wanted(p, 256), t.want, what);
     }
+    { // a decode step's joined launches: refused where a workgroup would write what another may still read
+        const auto at = [](size_t floats) { return (float*)(0x10000000 + 4 * floats); }; // (never read)
+        const uint32_t d = 1024;
+        for (const size_t written : {0u, 1020u, 1024u, 2044u, 2048u, 4096u}) // the sublayer's result lies at 0, the stream's row at 1024
+            for (const int which : {0, 1, 2}) {
+                NormAddParams n{};
+                n.y = at(0), n.residual = at(d), n.out = at(which == 0 ? written : 8192), n.next = at(which == 1 ? written : 16384), n.scales = n.next_scales = at(32768), n.rows = 1, n.d = d;
+                LinearF32Params p{};
+                p.w = (const uint16_t*)at(65536), p.y = at(which == 2 ? written : 131072), p.rows = p.batch = 1, p.n = 4112, p.k = d;
+                RouteGroupsParams r{};
+                r.router = (const uint16_t*)at(65536), r.ids = (int32_t*)at(262144), r.weights = at(262208), r.rows = 1, r.d = d, r.outputs = 8, r.top = 2, r.groups = r.keep = 1;
+                char what[100];
+                snprintf(what, sizeof what, "a step's launch whose %s lies %zu floats behind the sublayer's result", which == 0 ? "new row" : which == 1 ? "norm" : "product", written);
+                expect(norm_linear_supported(n, p), written >= 2048, what);
+                if (which < 2) expect(norm_route_gate_up_supported(n, r, (const uint16_t*)at(524288), 1024, ExpertAct()), written >= 2048, what);
+            }
+    }
     printf("%d bad\n", bad);
     return bad != 0;
 }

@@ -307,8 +307,13 @@ uint32_t norm_linear_blocks(uint32_t n) {
 
 } // namespace
 
+// One workgroup writes the row's new stream and norm, and all of them their results, while others may still read the old stream and the sublayer's result
+static bool apart_from_row(const NormAddParams& n, const float* written, size_t count) {
+    const auto apart = [&](const float* read) { return (uintptr_t)(written + count) <= (uintptr_t)read || (uintptr_t)(read + n.d) <= (uintptr_t)written; };
+    return apart(n.y) && apart(n.residual);
+}
 bool norm_linear_supported(const NormAddParams& n, const LinearF32Params& p) {
-    return n.rows == 1 && p.rows == 1 && p.batch == 1 && norm_add_step_supported(n) && n.out != n.residual && n.out != n.y && p.k == n.d && p.n && p.y && p.w && ((uintptr_t)p.w & 15) == 0 && !p.residual &&
+    return n.rows == 1 && p.rows == 1 && p.batch == 1 && norm_add_step_supported(n) && apart_from_row(n, n.out, n.d) && apart_from_row(n, n.next, n.d) && apart_from_row(n, p.y, p.n) && p.k == n.d && p.n && p.y && p.w && ((uintptr_t)p.w & 15) == 0 && !p.residual &&
            !p.gate && !p.mul_table && !p.row_offsets && !p.row_map;
 }
 uzu_status norm_linear(hipStream_t s, const NormAddParams& n, const LinearF32Params& p, float* part_value, uint32_t* part_index, uint32_t* parts) {
@@ -320,7 +325,7 @@ uzu_status norm_linear(hipStream_t s, const NormAddParams& n, const LinearF32Par
         if (part_value) hipLaunchKernelGGL((norm_linear_kernel<J, true>), grid, dim3(kStepThreads), (size_t)n.d * 4, s, n, p, part_value, part_index);                           \
         else hipLaunchKernelGGL((norm_linear_kernel<J, false>), grid, dim3(kStepThreads), (size_t)n.d * 4, s, n, p, part_value, part_index);                                     \
     }, "norm_linear")
-    switch ((n.d + 511) / 512) { // (a piece that lies past the row's end is loaded for nothing: 2560 with eight, 4096 columns 14.5 us; with five XX)
+    switch ((n.d + 511) / 512) { // (a piece that lies past the row's end is loaded for nothing: 2560 with eight, 4096 columns 14.4 us; with five 11.7)
     case 1: UZU_NL(1);
     case 2: UZU_NL(2);
     case 3: UZU_NL(3);
@@ -359,11 +364,11 @@ uzu_status norm_route_rows(hipStream_t s, const NormAddParams& n, const RouteGro
     return launch_check([&] { hipLaunchKernelGGL(norm_route_rows_kernel, dim3(p.rows), dim3(kStepThreads), (size_t)p.d * 4, s, n, p); }, "norm_route_rows");
 }
 bool norm_route_gate_up_supported(const NormAddParams& n, const RouteGroupsParams& p, const uint16_t* w13, uint32_t ff, const ExpertAct& act) {
-    // (the first workgroup replaces the stream's row while others may still read the old one)
-    return p.rows == 1 && norm_route_supported(n, p) && n.out != n.residual && n.out != n.y && !act.plain && ff >= 1 && ((uintptr_t)w13 & 15) == 0;
+    return p.rows == 1 && norm_route_supported(n, p) && apart_from_row(n, n.out, n.d) && apart_from_row(n, n.next, n.d) && !act.plain && ff >= 1 && ((uintptr_t)w13 & 15) == 0;
 }
 uzu_status norm_route_gate_up(hipStream_t s, const NormAddParams& n, const RouteGroupsParams& p, const uint16_t* w13, float* hidden, uint32_t ff, const ExpertAct& act, uint32_t weight_on_input) {
-    UZU_REQUIRE(w13 && hidden && norm_route_gate_up_supported(n, p, w13, ff, act), "norm_route_gate_up: one row, gated experts, the stream's new row apart from the old one");
+    UZU_REQUIRE(w13 && hidden && norm_route_gate_up_supported(n, p, w13, ff, act) && apart_from_row(n, hidden, (size_t)p.top * ff),
+                "norm_route_gate_up: one row, gated experts, what is written apart from the old row and what joins it");
     const uint32_t blocks = std::min((p.top * ff + kStepWaves - 1) / kStepWaves, 512u);
     return launch_check([&] { hipLaunchKernelGGL(norm_route_gate_up_kernel, dim3(blocks), dim3(kStepThreads), (size_t)p.d * 4, s, n, p, w13, hidden, ff, act, weight_on_input); }, "norm_route_gate_up");
 }

@@ -192,11 +192,11 @@ bool norm_add_step_supported(const NormAddParams& n); // rows of up to 4096, a m
 bool norm_route_supported(const NormAddParams& n, const RouteGroupsParams& p);
 bool norm_route_faster(const RouteGroupsParams& p); // than the two launches, without the experts' first products
 uzu_status norm_route_rows(hipStream_t s, const NormAddParams& n, const RouteGroupsParams& p);
-// ... and, one row, moe_experts_gate_up of the winners as well (weight_on_input: the winners' weights multiply their products).  n.out apart from n.residual and n.y.
+// ... and, one row, moe_experts_gate_up of the winners as well (weight_on_input: the winners' weights multiply their products).  n.out, n.next and hidden apart from n.residual and n.y.
 bool norm_route_gate_up_supported(const NormAddParams& n, const RouteGroupsParams& p, const uint16_t* w13, uint32_t ff, const ExpertAct& act);
 uzu_status norm_route_gate_up(hipStream_t s, const NormAddParams& n, const RouteGroupsParams& p, const uint16_t* w13, float* hidden, uint32_t ff, const ExpertAct& act, uint32_t weight_on_input);
 // ... and, one row, a linear of next (p.x is not read; no residual, gate or table); with part_value / part_index the largest result of each of up to kNormLinearParts workgroups and its
-// column, *parts of them.  n.out apart from n.residual and n.y.
+// column, *parts of them.  n.out, n.next and p.y apart from n.residual and n.y.
 constexpr uint32_t kNormLinearParts = 512;
 bool norm_linear_supported(const NormAddParams& n, const LinearF32Params& p);
 uzu_status norm_linear(hipStream_t s, const NormAddParams& n, const LinearF32Params& p, float* part_value = nullptr, uint32_t* part_index = nullptr, uint32_t* parts = nullptr);
