@@ -115,6 +115,12 @@ def test_norm_and_projection_in_one_launch(tmp_path):
 
 
 @pytest.mark.gpu
+def test_large_int8_matrices_have_the_decode_products_bits(tmp_path):
+    """tests/host/int8_stream_check.cpp: the weight stream of a decode step against the general decode GEMV on parts of the same matrices."""
+    _run_against_the_library(tmp_path, "int8_stream_check")
+
+
+@pytest.mark.gpu
 def test_gated_epilogue_has_the_exact_silu_for_every_gate(tmp_path):
     """tests/host/gated_silu_check.cpp: the quick quotient of csrc/gemm128_epilogue.h on the device, through the library's product, on each of its forms."""
     import subprocess

@@ -97,12 +97,25 @@ def test_gemv_int4_scale_bias_qwen_shapes(hip_ctx, n, k):
                                              (5001, 17408, 4, 1)])
 def test_gemv_bandwidth_regime(hip_ctx, n, k, bits, method):
     """M = 1 over >= 16 MB of weights: the persistent-grid plan of the decode GEMV -- K > 8192 on the LDS-resident activation row with
-    16-wave workgroups and batches drawn from an LDS counter (int4), the register-resident paths for K <= 8192, int8 on 4-wave
-    workgroups -- and an 8 MB matrix just below it; 5001 x 17408 is the Qwen3-14B-class down-projection (20 rows per 16-wave workgroup:
+    16-wave workgroups and batches drawn from an LDS counter (int4), the register-resident paths for K <= 8192, int8 through the
+    weight stream (csrc/k_decode_large.hip) -- and an 8 MB matrix just below it; 5001 x 17408 is the Qwen3-14B-class down-projection (20 rows per 16-wave workgroup:
     the plan takes two rows per lane group).  Which wave computes a row does not change the row: <= 1 bf16 ulp, >= 99 % bit-identical
     to the CPU restatement, ragged row counts included."""
     rng = np.random.default_rng(n + k + bits)
     q = quant_matrix(rng, n, k, bits, 128, method)
+    a = activations(rng, 1, k)
+    want, got = oracle_matmul(a, q, 1), hip_matmul(hip_ctx, a, q, 1)
+    ulps = ulp_diff_bf16(want, got)
+    assert ulps.max() <= 1.0, f"max {ulps.max()} bf16 ulps"
+    assert (want == got).mean() >= 0.99
+
+
+@pytest.mark.parametrize("n,k,group_size", [(4099, 2048, 128), (263, 32768, 32), (835, 10240, 64), (16401, 8192, 128)])
+def test_int8_weight_stream(hip_ctx, n, k, group_size):
+    """One row by int8 matrices from 8 MB on (csrc/k_decode_large.hip): the shortest and the longest row, row counts that the 2048 waves do not divide, and 128 MB, where a wave has three items on
+    their way.  <= 1 bf16 ulp against the CPU kernel, >= 99 % bit-identical, as the decode GEMV above."""
+    rng = np.random.default_rng(n + k)
+    q = quant_matrix(rng, n, k, 8, group_size, 0)
     a = activations(rng, 1, k)
     want, got = oracle_matmul(a, q, 1), hip_matmul(hip_ctx, a, q, 1)
     ulps = ulp_diff_bf16(want, got)

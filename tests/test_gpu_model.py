@@ -318,7 +318,8 @@ def test_fused_decode_matches_unfused(hip_ctx):
 @pytest.mark.parametrize("hidden,vocab,attention", [(4096, 4099, False), (6144, 4099, True), (4096, 65601, False)])
 def test_large_int8_matrices_of_a_decode_step_match_unfused(hip_ctx, hidden, vocab, attention):
     """Matrices from 8 MB on go through the weight stream (k_decode_large.hip): gated rows behind the Normalization, plain rows of two and three steps, a read-out with its arg-max whose rows do not
-    divide by the waves (and one long enough for three items a wave), qkv beside a gate.  Its arithmetic is the one-kernel-per-reference-kernel path's: bit-identical logits without attention."""
+    divide by the waves (and one long enough for three items a wave), qkv beside a gate.  The unfused path's one-row products go through the same stream, so what is compared here is what the fused
+    launches add to it (the Normalization, the activation, the arg-max): bit-identical logits without attention.  The stream against other kernels: test_int8_weight_stream, int8_stream_check.cpp."""
     kinds = [D.MIXER_DELTA_NET, D.MIXER_ATTENTION] if attention else [D.MIXER_DELTA_NET]
     extra = dict(num_heads=16, num_groups=4, head_dim=128) if attention else {}
     bundle = S.build_model(S.tiny_qwen(model_dim=2048, hidden_dim=hidden, vocab_size=vocab, bits=8, layer_kinds=kinds, group_size=128, **extra))
