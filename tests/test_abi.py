@@ -92,7 +92,7 @@ def _run_against_the_library(tmp_path, name, **env):
     _ffi.lib()
     exe, libdir = str(tmp_path / name), os.path.dirname(_ffi.LIB_PATH)
     subprocess.run(["g++", "-std=c++17", "-O1", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(ROOT, "tests", "host", name + ".cpp"),
-                    "-L", libdir, "-luzu_hip", "-L/opt/rocm/lib", "-lamdhip64", f"-Wl,-rpath,{libdir}", "-o", exe], check=True)
+                    "-L", libdir, "-luzu_hip", "-L/opt/rocm/lib", "-lamdhip64", "-lpthread", f"-Wl,-rpath,{libdir}", "-o", exe], check=True)
     out = subprocess.run([exe], capture_output=True, text=True, timeout=100, env=dict(os.environ, **env))
     assert out.returncode == 0 and out.stdout.endswith("0 bad\n"), out.stdout + out.stderr
 
@@ -118,6 +118,12 @@ def test_norm_and_projection_in_one_launch(tmp_path):
 def test_large_int8_matrices_have_the_decode_products_bits(tmp_path):
     """tests/host/int8_stream_check.cpp: the weight stream of a decode step against the general decode GEMV on parts of the same matrices."""
     _run_against_the_library(tmp_path, "int8_stream_check")
+
+
+@pytest.mark.gpu
+def test_convolution_has_the_exact_silu(tmp_path):
+    """tests/host/silu_conv_check.cpp: the quick quotient of csrc/silu_near.h on the device, for every f32 sum from 2^-8 to 128 in size and one in 61 of the others."""
+    _run_against_the_library(tmp_path, "silu_conv_check")
 
 
 @pytest.mark.gpu
