@@ -39,7 +39,8 @@ int main() {
     };
     for (const Prompt& t : {Prompt{32, 8, 128, 100, 0, false, 1, 1}, {32, 8, 128, 257, 0, false, 1, 1}, {32, 8, 128, 517, 0, false, 1, 1}, {16, 4, 128, 257, 0, false, 1, 1}, {24, 8, 64, 517, 0, false, 1, 1},
                             {40, 8, 128, 130, 0, false, 1, 1}, {8, 2, 256, 100, 0, false, 1, 1}, {32, 8, 128, 64, 1000, false, 4, 12}, {16, 4, 128, 517, 2000, false, 2, 12}, {4, 4, 64, 1024, 3000, false, 4, 12},
-                            {8, 2, 256, 517, 0, false, 4, 12}, {8, 2, 256, 517, 0, true, 4, 12}, {8, 2, 256, 2043, 0, true, 2, 4}, {8, 2, 256, 3000, 0, false, 2, 2}, {32, 8, 128, 1021, 0, false, 1, 1}}) {
+                            {8, 2, 256, 517, 0, false, 4, 12}, {8, 2, 256, 517, 0, true, 4, 12}, {8, 2, 256, 2043, 0, true, 2, 4}, {8, 2, 256, 3000, 0, false, 2, 5}, {32, 8, 128, 1021, 0, false, 1, 1}, {8, 2, 256, 831, 0, false, 6, 12},
+                            {8, 2, 256, 347, 600, false, 6, 12}, {8, 2, 256, 654, 0, true, 4, 12}, {24, 4, 256, 90, 600, true, 6, 12}, {16, 4, 128, 1025, 4500, false, 3, 5}, {32, 8, 128, 90, 600, false, 1, 6}}) {
         AttentionParams a{};
         a.dt = UZU_BF16, a.head_dim = t.head_dim, a.gqa_factor = t.heads / t.kv_heads, a.num_heads = t.heads, a.suffix_length = t.rows, a.sequence_length = t.rows + t.prefix, a.is_causal = 1;
         const uint32_t shares = attention_prefill_mfma_shares(a, t.prefix, t.gated);

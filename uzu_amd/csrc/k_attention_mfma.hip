@@ -468,11 +468,13 @@ __global__ void __launch_bounds__(256) attention_prefill_merge_kernel(const floa
     }
 }
 
-// Few task groups (few kv heads x short chunks): four tasks a workgroup, which share every staged K / V tile, and the KEYS over workgroups until the chip is covered -- or the workgroups thinned to
-// one or two tasks, and no merge.  What a launch takes is estimated for both, and the less is taken: the longest share, `us` a stretch of keys; the whole work at 256 CUs' rate, when that is more; a
-// second round, when workgroups are more than CUs; the merge, and its 8 bytes an element and share.  Measured over 170 sizes (10 shapes of 64 .. 256, 33 .. 3000 rows, up to 3000 keys in front): the choice is
-// within 0.3 % of the better one on the average, 11 % at the worst.  Us, shares and none: 32 heads on 8 of 128, 100 rows 13.0 / 7.5, 257 17.7 / 11.7, 517 25.1 / 18.9; 8 on 2 of 256, 100 rows 16.6 / 12.8, 257
-// 20.0 / 23.3, 517 26.9 / 41.4.
+// Few task groups (few kv heads x short chunks): four tasks a workgroup, which share every staged K / V tile, and the KEYS over workgroups until the chip is covered, once or twice -- or the workgroups
+// thinned to one or two tasks, and no merge.  What a launch takes is estimated for each, and the least is taken.  Shares: their launch and the merge's; `stretch` us a stretch of the longest share of every
+// 256 workgroups, which start the longest first; `workgroups` us per 256 of them for what they leave to the merge, and `rows` us per 10000 rows of a head that it writes.  None: the longest task, or
+// the whole work at the chip's rate or the rounds' longest where those are more.  Fitted to 7600 launches, every quantum at 684 sizes (12 shapes of 64 .. 256, 40 .. 3000 rows, up to 4500 keys in front); what
+// it picks is within 0.6 % of the fastest of them on the average, 4 of 684 are off by more than 10 % (20 % at the worst, 844 rows of 14 heads on 2 of 64).  Us, equal numbers of shares, one round of the
+// shortest shares, and this: 32 heads on 8 of 128, 98 rows 11.9 / 12.8 / 7.3, 261 18.7 / 18.2 / 12.3, 532 24.4 / 25.9 / 20.5; 8 on 2 of 256, 831 rows 35.3 / 30.5 / 30.5, 2298 behind 2000 keys 224 / 212 /
+// 195; 16 on 2 of 256, 154 behind 600 34.1 / 29.9 / 29.6.  528 sizes of eight shapes: 1.20x and 1.09x on the average.
 struct PrefillPlan {
     uint32_t quantum = 0, units = 0, splits = 1; // units: workgroups a kv head
 };
@@ -485,37 +487,56 @@ static PrefillPlan prefill_plan(const AttentionParams& a, uint32_t prefix, bool 
     const uint32_t kv_heads = a.num_heads / a.gqa_factor, n_tasks = a.gqa_factor * ((a.suffix_length + TQ - 1) / TQ), n_groups = (n_tasks + 3) / 4, stretch = a.head_dim <= 128 ? 2 * TK : TK;
     PrefillPlan best;
     if (kv_heads * n_groups >= 192) return best;
-    KeyShares shares{0, prefix};
-    const float us = a.head_dim == 64 ? 0.95f : a.head_dim == 128 ? 1.55f : 2.1f;
-    auto work = [&](uint32_t tpw) {
-        uint64_t all = 0;
-        for (uint32_t y = 0; y < (n_tasks + tpw - 1) / tpw; ++y) all += key_stretches(shares, y, tpw, a.gqa_factor, a.suffix_length, stretch);
-        return all;
+    struct Cost {
+        float none, none_stretch, shares, stretch, workgroups, rows;
     };
-    auto time = [&](uint32_t longest, uint64_t all, uint32_t units) {
-        const float l = (float)longest, w = 1.4f * (float)(kv_heads * all) / 256.0f, second = 0.57f * l * std::max(0.0f, (float)(kv_heads * units) / 256.0f - 1.0f);
-        return us * sqrtf(sqrtf(l * l * l * l + w * w * w * w + second * second * second * second));
+    const Cost us = a.head_dim == 64 ? Cost{4.0f, 1.09f, 7.6f, 1.08f, 7.8f, 2.1f} : a.head_dim == 128 ? Cost{4.6f, 1.47f, 10.6f, 1.60f, 9.9f, 1.0f} : Cost{5.3f, 2.12f, 12.3f, 2.28f, 12.6f, 3.3f};
+    constexpr uint32_t kRound = 256; // workgroups that the chip has at once
+    const uint32_t round = std::max(1u, kRound / kv_heads);
+    KeyShares shares{0, prefix};
+    auto longest_of_rounds = [&](uint32_t tpw, uint64_t* all) { // the longest share of every round, added up
+        uint32_t longest = 0, total = 0, in_round = 0;
+        for (uint32_t y = (n_tasks + tpw - 1) / tpw; y-- > 0;) { // (as they start)
+            const uint32_t length = key_stretches(shares, y, tpw, a.gqa_factor, a.suffix_length, stretch), n = key_shares(shares, y, tpw, a.gqa_factor, a.suffix_length, stretch);
+            if (all) *all += length;
+            for (uint32_t left = n; left;) {
+                const uint32_t now = std::min(left, round - in_round);
+                longest = std::max(longest, (length + n - 1) / n), left -= now, in_round += now;
+                if (in_round == round) total += longest, longest = in_round = 0;
+            }
+        }
+        return total + longest;
     };
     const uint32_t top = key_stretches(shares, n_groups - 1, 4, a.gqa_factor, a.suffix_length, stretch);
-    float least = time(top, work(unsplit_tasks(kv_heads, n_tasks)), 0) + (gated ? 3.5f : 0.0f); // (the gate's own launch)
-    const uint64_t all = work(4);
-    auto consider = [&](uint32_t quantum, uint32_t most_units) { // whether the workgroups are few enough
+    uint64_t all = 0;
+    const float rounds_none = (float)longest_of_rounds(unsplit_tasks(kv_heads, n_tasks), &all), l = (float)top, w = 1.31f * (float)(kv_heads * all) / (float)kRound;
+    float least = us.none + us.none_stretch * std::max(rounds_none, sqrtf(sqrtf(l * l * l * l + w * w * w * w)));
+    if (gated) least += 2.1f + 2.3e-6f * (float)a.suffix_length * (float)(a.num_heads * a.head_dim); // (the gate's own launch)
+    auto plan_of = [&](uint32_t quantum) {
         shares.quantum = quantum;
         PrefillPlan p{quantum, 0, 1};
-        uint32_t longest = 0;
         for (uint32_t y = 0; y < n_groups; ++y) {
             const uint32_t n = key_shares(shares, y, 4, a.gqa_factor, a.suffix_length, stretch);
-            p.units += n, p.splits = std::max(p.splits, n), longest = std::max(longest, (key_stretches(shares, y, 4, a.gqa_factor, a.suffix_length, stretch) + n - 1) / n);
+            p.units += n, p.splits = std::max(p.splits, n);
         }
-        if (p.splits > 1 && kv_heads * p.units > most_units) return false;
-        const float t = time(longest, all, p.units) + (a.head_dim <= 128 ? 4.0f : 8.0f) + 0.44e-6f * 8.0f * (float)kv_heads * (float)p.units * 128.0f * (float)a.head_dim;
-        if (p.splits > 1 && t < least) least = t, best = p;
-        return true;
+        return p;
     };
-    // the shortest shares that the CUs hold, a workgroup each: 64 keys a share at least, and no more shares than there can be
-    uint32_t quantum = std::max({2 * TK / stretch, (uint32_t)(kv_heads * all / 256), top / kMaxKeySplits});
-    while (!consider(quantum, 256)) ++quantum;
-    if (a.head_dim > 128) consider((top + 1) / 2, 512); // (two shares of every other group: 3000 rows of 8 heads on 2 of 256 138 us, with a workgroup a CU at most 167)
+    auto consider = [&](uint32_t quantum) {
+        const PrefillPlan p = plan_of(quantum);
+        if (p.splits == 1) return;
+        const float t = us.shares + us.stretch * (float)longest_of_rounds(4, nullptr) + us.workgroups * (float)(kv_heads * p.units) / (float)kRound + us.rows * 1e-4f * (float)a.suffix_length * (float)a.num_heads;
+        if (t < least) least = t, best = p;
+    };
+    for (uint32_t rounds = 1; rounds <= 2; ++rounds) { // the shortest shares that so many rounds hold (the longer the shares, the fewer workgroups)
+        uint32_t low = 1, high = top;
+        while (low < high) {
+            const uint32_t mid = (low + high) / 2;
+            if (kv_heads * plan_of(mid).units <= rounds * kRound) high = mid;
+            else low = mid + 1;
+        }
+        consider(low);
+        if (rounds == 1) consider((3 * low + 1) / 2); // (fewer, and less to merge)
+    }
     return best;
 }
 uint32_t attention_prefill_mfma_shares(const AttentionParams& a, uint32_t prefix, bool gated) { return prefill_plan(a, prefix, gated).splits; }
