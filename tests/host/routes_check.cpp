@@ -51,17 +51,18 @@ int main() {
         bool want;
     };
     for (const bool step : {true, false})
-        for (const Window& t : step ? std::vector<Window>{{8, 16, 4, 128, 1024, 0, true}, {48, 32, 8, 128, 0, 4000, true}, {2, 64, 8, 64, 1024, 0, true}, {8, 64, 8, 64, 1024, 0, false}, {48, 64, 8, 64, 256, 0, true},
-                                                          {24, 64, 8, 64, 1024, 0, false}, {64, 64, 8, 64, 1024, 0, true}, {12, 64, 8, 64, 0, 300, true}, {12, 64, 8, 64, 0, 4000, false}, {12, 40, 8, 128, 1024, 0, true},
-                                                          {12, 40, 8, 128, 0, 4000, false}, {4, 24, 2, 128, 1024, 0, true}, {12, 24, 2, 128, 1024, 0, false}, {12, 24, 2, 128, 0, 300, true},
-                                                          {12, 24, 2, 128, 0, 1500, false}, {24, 24, 2, 128, 512, 0, false}}
+        for (const Window& t : step ? std::vector<Window>{{8, 16, 4, 128, 1024, 0, true}, {48, 32, 8, 128, 0, 4000, true}, {2, 64, 8, 64, 1024, 1300, true}, {8, 64, 8, 64, 1024, 1300, false}, {12, 64, 8, 64, 0, 300, true},
+                                                          {12, 64, 8, 64, 0, 3900, false}, {6, 64, 8, 64, 1024, 1300, false}, {24, 64, 8, 64, 3000, 150, true}, {4, 40, 8, 128, 512, 450, true}, {12, 40, 8, 128, 1024, 1300, true},
+                                                          {4, 24, 2, 128, 1024, 1300, true}, {32, 24, 2, 128, 512, 450, false}, {12, 24, 2, 128, 0, 300, true}, {48, 24, 2, 128, 3000, 150, true},
+                                                          {48, 24, 2, 128, 0, 3900, false}, {32, 48, 3, 64, 3000, 150, true}, {32, 48, 3, 64, 3000, 1999, false}, {1, 16, 1, 128, 0, 0, true}}
                                     : std::vector<Window>{{300, 8, 2, 128, 0, 0, true}, {16, 8, 2, 128, 0, 0, true}, {16, 8, 2, 128, 64, 0, false}, {64, 16, 4, 128, 64, 0, false}, {200, 8, 2, 128, 64, 0, true},
                                                           {32, 8, 2, 128, 128, 0, false}, {16, 8, 2, 128, 192, 0, true}, {300, 8, 2, 128, 1024, 0, true}}) {
             WindowAttentionParams p{};
-            p.rows = t.rows, p.nseq = step ? t.rows : 1, p.heads = t.heads, p.kv_heads = t.kv_heads, p.dim = p.vdim = t.dim, p.ldq = t.heads * t.dim, p.window = t.window, p.keys = t.keys, p.splits = 1, p.one_row = step, p.cache_bf16 = step;
+            p.rows = t.rows, p.nseq = step ? t.rows : 1, p.heads = t.heads, p.kv_heads = t.kv_heads, p.dim = p.vdim = t.dim, p.ldq = t.heads * t.dim, p.window = t.window, p.keys = t.keys, p.one_row = step, p.cache_bf16 = step;
+            if (step) p.tiles = p.tiles32 = t.rows, window_attention_split_keys(p, t.window ? t.window : 4096, 256);
             char what[160];
-            snprintf(what, sizeof what, "%s attention, %u rows of %u heads on %u of %u, window %u", step ? "step" : "f32 prompt", t.rows, t.heads, t.kv_heads, t.dim, t.window);
-            expect(step ? window_attention_step_supported(p) : window_attention_f32_supported(p), t.want, what);
+            snprintf(what, sizeof what, "%s attention, %u rows of %u heads on %u of %u, window %u, %u keys", step ? "step" : "f32 prompt", t.rows, t.heads, t.kv_heads, t.dim, t.window, t.keys);
+            expect(step ? p.split_items == 0 : window_attention_f32_supported(p), t.want, what);
         }
     for (const uint32_t outputs : {8u, 32u, 64u})
         for (const uint32_t d : {256u, 1024u, 2048u}) {

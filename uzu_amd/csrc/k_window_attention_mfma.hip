@@ -300,16 +300,32 @@ size_t window_attention_split_ws_bytes(uint32_t rows, uint32_t heads, uint32_t s
 // waves are the faster walkers.  How few it can have is how many workgroups run at once: one a CU.  Heads of 128, 4 key / value heads, us a launch with its merge, stretches of 32 /
 // of 128: one sequence, window 40 9.8 / 14.0, 128 10.5 / 14.4, 512 (16 splits) 10.1 / 15.4 (4), 1024 (16) 12.6 / 14.6 (8); 8 sequences, window 256 (8) 10.5 / 14.8 (2),
 // 512 (8) 13.0 / 15.1 (4), 1024 (8) 18.3 / 14.1 (8); 32 sequences, window 128 (2) 13.3 / 14.5 (2), 256 (2) 18.5 / 14.6 (2).  Up to 32 keys the simple form is as fast.
+static float split_us(const WindowAttentionParams& p, uint32_t seen) { // with the merge: a workgroup's stretches, the work over the chip's units of 256, the workgroups, and what the merge adds
+    struct Cost {
+        float launch, stretch, work, workgroups, shares;
+    };
+    const bool wide = blocks_of(p) > 2, short_stretches = p.split_items == 128;
+    const Cost us = short_stretches ? (wide ? Cost{7.25f, 2.69f, -1.64f, 4.34f, 0.026f} : Cost{7.2f, 1.85f, -0.37f, 1.08f, 0.146f}) : (wide ? Cost{9.0f, 2.1f, 4.17f, 4.34f, 0.026f} : Cost{8.0f, 1.43f, 1.52f, 1.08f, 0.146f});
+    const uint32_t stretches = short_stretches ? (seen + 31) / 32 : (seen + 127) / 128;
+    const float units = (float)(p.rows * p.kv_heads) / 256.0f;
+    return us.launch + us.stretch * (float)((stretches + p.splits - 1) / p.splits) + units * (us.work * (float)stretches + us.workgroups * (float)p.splits) + us.shares * 1e-3f * (float)p.rows * (float)(p.heads * p.splits);
+}
+// One row a sequence: the step form (k_window_attention_step.hip) or this one.  The step form reads a key once per four query heads of its key / value head, this one once, and its tiles are filled the better the
+// more of those there are; its shares are cut for `keys`, however few a pass has.  Up to four of them, or over up to 224 keys, the step form is the faster one.  Else what either takes is estimated, from the
+// keys that the pass' rows do see where it knows them (a captured one does not: up to 1000).  Us, this form and the step form: 24 heads on 2 of 128, 48 rows behind 150 / 700 / 2000 keys, no window 46 / 12,
+// 52 / 40, 66 / 102; 64 on 8 of 64, window 1024, 6 rows 11.5 / 14.1, 32 rows 35.6 / 31.4.  8580 passes of five query heads and more: within 0.5 % of the faster form on the average, 141 off by more than
+// 10 %, by at most 24 %.
 void window_attention_split_keys(WindowAttentionParams& p, uint32_t keys, uint32_t num_cus) {
-    p.keys = p.keys ? std::min(p.keys, keys) : keys, p.splits = 1; // (the step form with one share: whether it takes the shape at all)
-    if (window_attention_step_supported(p)) {
-        p.splits = window_attention_step_splits(p, keys, num_cus);
-        if (p.split_ws) p.splits = std::max<uint32_t>(1, std::min<size_t>(p.splits, p.split_ws_bytes / window_attention_split_ws_bytes(p.rows, p.heads, 1)));
-        return;
-    }
+    WindowAttentionParams step = p;
+    step.split_items = 0, step.splits = 1; // (one share: whether it takes the shape at all)
     const uint32_t blocks = (keys + 31) / 32, at_once = num_cus / std::max(1u, p.tiles * p.kv_heads), splits = std::min(blocks, std::max(2u, std::min(16u, at_once)));
     if (blocks <= 2 * splits) p.split_items = 128, p.splits = splits;
     else p.split_items = 32, p.splits = std::min(16u, std::max(2u, (keys + 127) / 128));
+    if (!window_attention_step_supported(step)) return;
+    step.splits = window_attention_step_splits(p, keys, num_cus);
+    if (p.split_ws) step.splits = std::max<uint32_t>(1, std::min<size_t>(step.splits, p.split_ws_bytes / window_attention_split_ws_bytes(p.rows, p.heads, 1)));
+    const uint32_t seen = std::min(keys, p.keys ? p.keys : 1000u);
+    if (p.heads / p.kv_heads <= 4 || keys <= 224 || (p.split_ws && !window_attention_mfma_supported(p)) || window_attention_step_us(step, seen) <= split_us(p, seen)) p = step;
 }
 
 // bf16 caches, head widths that are multiples of 8 up to 128 (16-byte rows); prompt-sized passes, or a decode-sized pass with a workspace to split its keys

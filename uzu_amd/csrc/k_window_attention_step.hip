@@ -216,17 +216,8 @@ uint32_t heads_a_block(const WindowAttentionParams& p) { return p.heads / p.kv_h
 
 } // namespace
 
-// A key / value head with more than four query heads has its keys read once per four of them here, and once by the matrix-core form, whose tiles they fill better: with many rows over long stretches of
-// keys that form is the faster one.  Us, matrix cores and here, 1024 keys: 64 heads on 8 of 64, 2 / 8 / 48 rows 11.4 / 9.4, 11.9 / 15.4, 50 / 37; 24 on 2 of 128, 4 / 8 / 48 rows 13.5 / 11.6, 13.9 / 15.6,
-// 38 / 55; 512 keys 11.1 / 9.0, 11.5 / 11.8, 25 / 31; 40 on 8 of 128, 12 rows, 300 / 1500 / 4000 keys 46 / 16, 61 / 46, 90 / 107.
-static bool step_faster(const WindowAttentionParams& p) {
-    const uint32_t blocks = (p.heads / p.kv_heads + 3) / 4, units = p.rows * p.kv_heads * blocks, keys = p.keys ? p.keys : p.window ? p.window : 1024u;
-    if (blocks == 1 || keys <= 128 || (!p.window && keys < 1000)) return true; // (without a window the matrix-core form's shares are cut for as many keys as there can be)
-    if (blocks > 2) return (uint64_t)units * std::min(keys, 2048u) <= 40 * 1024;
-    return width_blocks(p) > 2 ? keys < 3000 || units < 32 || units >= 512 : keys < 1024 || units < 48 || units >= 512;
-}
 bool window_attention_step_supported(const WindowAttentionParams& p) {
-    return p.one_row && p.rows == p.nseq && p.cache_bf16 && width_blocks(p) && p.dim % 8 == 0 && p.vdim % 8 == 0 && p.ldq % 4 == 0 && p.kv_heads && p.heads % p.kv_heads == 0 && step_faster(p) &&
+    return p.one_row && p.rows == p.nseq && p.cache_bf16 && width_blocks(p) && p.dim % 8 == 0 && p.vdim % 8 == 0 && p.ldq % 4 == 0 && p.kv_heads && p.heads % p.kv_heads == 0 && !p.split_items &&
            ((uintptr_t)p.q & 15) == 0 && (uint64_t)p.kv_heads * 128 * 2 < (1ull << 32) && (p.splits == 1 || (p.splits > 1 && p.splits <= 64 && p.split_ws && p.split_ws_bytes >= window_attention_split_ws_bytes(p.rows, p.heads, p.splits)));
 }
 // Shares: a turn of keys each, at most 32, and two workgroups a CU in all (8 sequences of 4 key / value heads: 8 / 16 / 32 shares 14.5 / 12.1 .. 13.4 / 14.6 us); up to two turns one
@@ -235,6 +226,14 @@ uint32_t window_attention_step_splits(const WindowAttentionParams& p, uint32_t k
     const uint32_t turn = 128 / width_blocks(p), blocks = (keys + turn - 1) / turn, hg = p.heads / p.kv_heads, hq = heads_a_block(p), each = p.rows * p.kv_heads * ((hg + hq - 1) / hq);
     if (blocks <= 2) return 1;
     return std::min(blocks, std::max(1u, std::min(32u, 2 * num_cus / std::max(1u, each))));
+}
+
+// Us, with the merge: every share is a workgroup's turns, one behind the other.  (8580 passes of key / value heads with five query heads and more: within 5 % on the average)
+float window_attention_step_us(const WindowAttentionParams& p, uint32_t seen) {
+    const bool wide = width_blocks(p) > 2;
+    const uint32_t turn = 128 / width_blocks(p), hg = p.heads / p.kv_heads, hq = heads_a_block(p), share = turn * p.splits;
+    return (wide ? 4.0f : 4.35f) + (wide ? 0.033f : 0.020f) * 1e-3f * (float)seen * (float)(p.rows * p.kv_heads * ((hg + hq - 1) / hq)) + (wide ? 1.21f : 1.06f) * (float)((seen + share - 1) / share) +
+           (p.splits > 1 ? 3.7f : 0.0f) + (wide ? 0.43e-3f : 0.27e-3f) * (float)p.rows * (float)(p.heads * p.splits);
 }
 
 uzu_status window_attention_step(hipStream_t s, const WindowAttentionParams& p, const DecayedStateParams* beside) {

@@ -388,10 +388,10 @@ struct WindowAttentionParams {
     uint32_t tiles32; // ... of ceil(count * (heads / kv_heads) / 32): its key-split form's with split_items = 32
     // matrix-core form, few rows over many keys (decode): `splits` > 1 workgroups share the key blocks of an item tile, partial sums go through split_ws
     // (window_attention_split_ws_bytes(rows, heads, splits) bytes) and a merge launch.  0 / null: one workgroup walks all keys of its tile.
-    uint32_t splits, split_items; // split_items: items a workgroup takes, 128 (stretches of 32 keys) or 32 (of 128; also 0)
+    uint32_t splits, split_items; // split_items: items a workgroup takes, 128 (stretches of 32 keys) or 32 (of 128; also 0); set, the pass is not the step form's
     float* split_ws;
     size_t split_ws_bytes;
-    uint32_t keys;    // that a row of this pass sees at the most, as far as the caller knows (the form rests on it); 0: not known (window_attention_split_keys sets its own)
+    uint32_t keys;    // that a row of this pass sees at the most, as far as the caller knows (which form is the faster rests on it); 0: not known
     uint32_t one_row; // every sequence of the pass brings exactly one row (row r is sequence r's): the step form, with `splits` >= 1 shares of a row's keys
 };
 // `splits` and `split_items` of a decode-sized pass whose rows see `keys` keys at the most, from `rows`, `tiles` and `kv_heads`: at most 16 splits, of the step form at most 32
@@ -406,6 +406,7 @@ struct GatedNormParams;
 bool window_attention_step_supported(const WindowAttentionParams& p);
 bool window_attention_step_beside(const DecayedStateParams& d);
 uint32_t window_attention_step_splits(const WindowAttentionParams& p, uint32_t keys, uint32_t num_cus);
+float window_attention_step_us(const WindowAttentionParams& p, uint32_t seen);
 uzu_status window_attention_step(hipStream_t s, const WindowAttentionParams& p, const DecayedStateParams* beside);
 uzu_status window_attention_merge(hipStream_t s, const WindowAttentionParams& p, const GatedNormParams* beside);
 
