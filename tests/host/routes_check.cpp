@@ -24,7 +24,7 @@ int main() {
     };
     for (const Tree& t : {Tree{16, 16, 128, 13, 80, false, false, false}, {16, 16, 128, 13, 600, false, false, true}, {8, 8, 64, 13, 250, false, false, false}, {8, 8, 64, 13, 600, false, false, true},
                           {8, 8, 256, 2, 80, false, false, false}, {8, 8, 256, 2, 250, false, false, true}, {32, 8, 128, 1, 30, false, false, false}, {32, 8, 128, 1, 250, false, false, true},
-                          {24, 8, 64, 4, 180, false, false, false}, {40, 8, 128, 16, 120, false, false, false}, {16, 2, 128, 1, 10, false, false, true}, {8, 2, 256, 13, 300, false, true, true},
+                          {24, 8, 64, 4, 180, false, false, false}, {32, 8, 128, 20, 70, false, false, false}, {32, 8, 128, 13, 110, false, false, true}, {12, 4, 128, 4, 1700, true, false, false}, {40, 8, 128, 16, 120, false, false, false}, {16, 2, 128, 1, 10, false, false, true}, {8, 2, 256, 13, 300, false, true, true},
                           {16, 16, 128, 4, 1500, true, false, false}, {16, 16, 128, 8, 1500, true, false, true}, {32, 8, 128, 1, 4000, true, false, false}, {32, 8, 128, 3, 1500, true, false, true},
                           {8, 4, 256, 6, 1500, true, false, false}, {8, 4, 256, 8, 4000, true, false, true}, {8, 2, 256, 2, 1500, true, true, true}, {8, 2, 256, 13, 1500, true, true, true},
                           {2, 2, 128, 16, 8000, true, false, false}, {32, 32, 128, 2, 8000, true, false, false}, {32, 32, 128, 6, 8000, true, false, true}, {64, 8, 64, 1, 1100, true, false, true}}) {

@@ -327,11 +327,11 @@ bool attention_tree_faster(uint32_t num_heads, uint32_t gqa_factor, uint32_t hea
     while (gs < (head_dim >= 256 ? 2u : 3u) && gqa_factor % (2u << gs) == 0) ++gs;
     if (gs == 3) return true;
     if (!two_pass) {
-        static constexpr uint32_t meet[3][3] = {{430, 240, 90}, {240, 160, 75}, {135, 105, 60}}; // [heads of 64, 128, 256][gs]
+        static constexpr uint32_t meet[3][3] = {{440, 240, 90}, {260, 160, 110}, {135, 90, 70}}; // [heads of 64, 128, 256][gs]
         return keys > meet[head_dim <= 64 ? 0 : head_dim <= 128 ? 1 : 2][gs];
     }
     const uint32_t rows = nodes * num_heads, columns = nodes * gqa_factor, half = gated ? 2 : 1;
-    return rows >= 128 / half || (columns >= (head_dim >= 256 ? 16 : 12) / half && rows * head_dim >= 6144 / half);
+    return rows >= 128 / half || (columns >= (head_dim >= 256 ? 16 : 12) / half && rows * head_dim > 6144 / half);
 }
 
 size_t attention_tree_columns(uint32_t num_heads, uint32_t gqa_factor, uint32_t nodes) {
