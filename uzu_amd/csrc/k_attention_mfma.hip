@@ -418,7 +418,8 @@ __global__ void __launch_bounds__(256) attention_prefill_merge_kernel(const floa
     const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6), e0 = (threadIdx.x & 63) * EPT;
     if (row >= rows) return;
     const uint32_t query = row / heads, head = row - query * heads, splits = key_shares(shares, (query / TQ * gqa + head % gqa) / tpw, tpw, gqa, rows / heads, HD <= 128 ? 2 * TK : TK);
-    // every share is requested before the first is used (one behind the other, a share was two trips to memory: 8 shares of 517 rows 11.2 us -> 9.3, 2 of 2043 15.4 -> 13.9)
+    // every share is requested before the first is used (one behind the other, a share was two trips to memory: eight shares of 517 rows 11.2 us, 9.3 so; 6.9 in a body for eight, and 14.3 for 2043 rows
+    // of up to three)
     float ms[MOST], ls[MOST], po[MOST][EPT];
     uint16_t gs[EPT];
 #pragma unroll
@@ -491,7 +492,7 @@ static PrefillPlan prefill_plan(const AttentionParams& a, uint32_t prefix, bool 
         float none, none_stretch, shares, stretch, workgroups, rows;
     };
     const Cost us = a.head_dim == 64 ? Cost{4.0f, 1.09f, 7.6f, 1.08f, 7.8f, 2.1f} : a.head_dim == 128 ? Cost{4.6f, 1.47f, 10.6f, 1.60f, 9.9f, 1.0f} : Cost{5.3f, 2.12f, 12.3f, 2.28f, 12.6f, 3.3f};
-    constexpr uint32_t kRound = 256; // workgroups that the chip has at once
+    constexpr uint32_t kRound = kChipCus; // workgroups that the chip has at once
     const uint32_t round = std::max(1u, kRound / kv_heads);
     KeyShares shares{0, prefix};
     auto longest_of_rounds = [&](uint32_t tpw, uint64_t* all) { // the longest share of every round, added up

@@ -737,7 +737,7 @@ __global__ void __launch_bounds__(256) delta_net_norm_gate_kernel(uint16_t* in_o
     }
 }
 // The same for heads of 128: sixteen lanes a (token, head), eight elements a lane, every load 16 bytes and in front of the sum (a wave a head with two-byte loads, z's behind the
-// sum: 4.5 -> 3.3 us for 13 rows of 16 heads, 6.8 -> 5.1 for 517, 17.1 -> 8.7 for 2043)
+// sum: 16 heads, 517 rows 6.8 -> 4.9 us, 2043 17.1 -> 8.7; up to 100 rows either is a launch and a trip to memory, 4.7 and 4.6 of 13 rows in a verify pass)
 __global__ void __launch_bounds__(256) delta_net_norm_gate128_kernel(uint16_t* in_out, const uint16_t* in_proj, const float* norm_weight, uint32_t num_v_heads, uint32_t conv_dim,
                                                                      uint32_t total_proj_dim, float norm_epsilon, uint32_t suffix_len, float* rowsum_out, uint32_t rowsum_stride,
                                                                      uint32_t rowsum_row0, uint32_t rowsum_pad_to) {

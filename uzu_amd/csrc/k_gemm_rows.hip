@@ -181,7 +181,8 @@ __global__ void __launch_bounds__(256, 2) gemm_rows_kernel(GemmRowsParams p) {
             sc0[b] *= 16.0f, sc1[b] *= 16.0f;
         }
         // (a wave of four has two steps of K = 1024: reloads past its end, though nobody waited for them, were a third of what it asked of the L2.  37 rows: 8224 x 1024 11.2 us -> 8.8, 7168 x 1024
-        // + GatedActMul 9.3 -> 8.4, 3072 x 1024 7.0 -> 5.6, 1024 x 2048 and x 3584 in four shares 5.6 -> 5.1)
+        // + GatedActMul 9.3 -> 8.4, 3072 x 1024 7.0 -> 5.6, 1024 x 2048 and x 3584 in four shares 5.6 -> 5.1; 1600 products of 17 .. 128 rows 1.06x on the average.  17 rows of K = 2560 and 3584 lose
+        // 1 %, 6144 x 3584 9.2 -> 9.9; a last pair of steps without loads behind a loop with them gives that back, and takes 8 % of every product of K = 512: more code to fetch)
         if (s + 2 < s_hi) load_scales(s + 2);
         __builtin_amdgcn_sched_barrier(0); // (left alone, the scheduler sinks the loads to their uses and waits for each)
         compute(stA, sc0, of0);

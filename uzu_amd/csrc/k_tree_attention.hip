@@ -297,11 +297,11 @@ __global__ void __launch_bounds__(256) tree_attention_merge_kernel(AttentionPara
     if (gate) bits = scaled_sigmoid_bf16(bf16_to_f32(bits), bf16_to_f32(g), s_exp_tab);
     out[row * head_dim + element] = bits;
 }
-// kv heads x pairs of column tiles; the shares that put a workgroup on most of the 256 compute units
+// kv heads x pairs of column tiles; the shares that put a workgroup on most of the compute units
 uint32_t tree_pairs(uint32_t group_heads, uint32_t nodes) { return (group_heads * nodes + 2 * kColumns - 1) / (2 * kColumns); }
 uint32_t tree_shares(uint32_t kv_heads, uint32_t pairs) {
     uint32_t shares = kTreeAttentionShares;
-    while (shares > 8 && kv_heads * pairs * shares > 256) shares >>= 1;
+    while (shares > 8 && kv_heads * pairs * shares > kChipCus) shares >>= 1;
     return shares;
 }
 } // namespace

@@ -17,6 +17,8 @@ namespace k {
 
 enum DT : uint32_t { BF16 = UZU_BF16, F32 = UZU_F32 };
 
+constexpr uint32_t kChipCus = 256; // compute units of an MI355X: for plans of kernels that are called without a device to ask
+
 struct NormParams;
 // ---------------------------------------------------------------- matmul (quantised / full-precision B)
 struct MatmulParams {
