@@ -1000,8 +1000,9 @@ def test_attention_trie_mask(hip_ctx, tree, window, heads, kv_heads, hd, prefix)
 
 @pytest.mark.parametrize("n,heads,kv_heads,hd,prefix", [(1, 4, 4, 64, 0), (2, 8, 2, 128, 1), (13, 8, 2, 256, 1023), (16, 16, 4, 64, 31), (17, 14, 2, 64, 96), (31, 6, 3, 256, 32), (32, 8, 1, 128, 2100)])
 def test_attention_of_a_tree_on_the_matrix_cores(hip_ctx, n, heads, kv_heads, hd, prefix):
-    """The tree form (k_tree_attention.hip) at its edges against float64: a column tile that is full, one over and nearly empty, groups of columns (heads a kv head x nodes
-    past 64), a first tile of keys that is the tree's own, shares with none, one and several tiles, rows behind the last key that hold NaN.
+    """Attention of a tree through its entry, by the tree form (k_tree_attention.hip) or the vector form, whichever is the faster one there, against float64: the sizes of the tree form's edges (which
+    tree_attention_check.cpp calls by itself, also with rows behind the last key that it loads): a column tile that is full, one over and nearly empty, groups of columns (heads a kv head x nodes past
+    64), a first tile of keys that is the tree's own, shares with none, one and several tiles.
     The bound: the bf16 rounding of the result, and the f32 sums of the scores (hd terms) and of the rows (a key a term), carried to the result by at most max |v|."""
     rng = np.random.default_rng(n * hd + prefix)
     parents, path = [-1], [0]
@@ -1026,7 +1027,7 @@ def test_attention_of_a_tree_on_the_matrix_cores(hip_ctx, n, heads, kv_heads, hd
 
 
 @pytest.mark.parametrize("bad", [0x7F80, 0xFF80, 0x7FC0])
-@pytest.mark.parametrize("n,heads,kv_heads,hd,prefix,at", [(3, 4, 2, 64, 5, 1), (13, 8, 2, 256, 1023, 4), (16, 4, 4, 128, 31, 9), (32, 8, 1, 64, 96, 20), (32, 6, 2, 256, 2090, 3), (4, 4, 2, 128, 61, 3)])
+@pytest.mark.parametrize("n,heads,kv_heads,hd,prefix,at", [(3, 4, 2, 64, 5, 1), (13, 8, 2, 256, 1023, 4), (16, 4, 4, 128, 31, 9), (32, 8, 1, 64, 96, 20), (32, 6, 2, 256, 2090, 3), (4, 4, 2, 128, 61, 3), (16, 8, 2, 128, 300, 9)])
 def test_attention_of_a_tree_keeps_other_branches_values_out(hip_ctx, n, heads, kv_heads, hd, prefix, at, bad):
     """Key or value rows of a node that are not finite: the nodes of other branches have what finite rows leave them (within a rounding to bf16, since an f32 sum may be made in another order),
     its own subtree what float64 gives."""
