@@ -64,7 +64,7 @@ __device__ __forceinline__ float quad_sum(float v) {
 }
 // Loads of a chunk's rows and states: buffer loads, whose lanes past a bound read zero without a branch, and which want words aligned and no more (one path where there were two).
 // With them and the products' operands read in front of the first product, under one condition for all of them, `out` of 5 chunks of 16 heads of 128 x 64: 23 us -> 16, of 34 chunks of 32:
-// 72 -> 59; a decay per channel, 128 x 128: 38 -> 32, 92 -> 79.  (The loads alone changed nothing; the carried state a slab ahead besides: 70.)
+// 72 -> 62; a decay per channel, 128 x 128: 38 -> 32, 92 -> 79.  (The loads alone changed nothing; the carried state a slab ahead besides: 70.)
 constexpr uint32_t kNowhere = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_from(const float* base) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, 0x7FFFFFFF, 0x00027000); }
 __device__ __forceinline__ float load1(__amdgpu_buffer_rsrc_t rows, uint32_t index, bool in) {
@@ -205,6 +205,7 @@ template <bool CHANNEL> __global__ void __launch_bounds__(256) decayed_state_sca
 // worked on, the carried state's rows go from memory straight into the products.  One decay per head: scores as two 32 x 32 tiles per wave row, times a table of decays.
 // A decay per channel: a wave owns the block of 16 x 16 scores on the diagonal that bears its number (running products, lane = (key row, quarter of the slab)) and up to
 // two of the six blocks below it (v_mfma_f32_16x16x4_f32).  Results: wave w has rows 32 (w / 2) .., column tiles NQ (w % 2) ..
+// One decay per head, values of up to 64: four workgroups a CU, in 128 registers (three with one more: 830 .. 1080 workgroups 5 to 11 % slower, more of them 2 to 6 %, 1090 .. 1215 1 to 2 % faster)
 template <bool CHANNEL, int NQ, bool FOURS>
 __global__ void __launch_bounds__(256, CHANNEL || NQ > 1 ? 2 : FOURS ? 4 : 3) decayed_state_out_kernel(DecayedStateParams p, const float* ws) {
     constexpr uint32_t SW = 32, PW = SW + 4, VW = 64 * NQ, ROWS = kChunk * PW; // a slab row's pitch: 16-byte aligned, rows on distinct banks
