@@ -97,6 +97,20 @@ def _run_against_the_library(tmp_path, name, **env):
     assert out.returncode == 0 and out.stdout.endswith("0 bad\n"), out.stdout + out.stderr
 
 
+def test_kernel_parameters_declared_without_braces_are_defined(tmp_path):
+    """tests/host/params_check.cpp over every *Params struct of the kernels' headers: a member that is not set is null or zero, never what the stack held (a kernel reads optional pointers when
+    they are not null)."""
+    import subprocess
+    csrc = os.path.join(ROOT, "uzu_amd", "csrc")
+    names = [n for h in ("kernels.h", "kernels_decode.h", "kernels_stream32.h") for n in re.findall(r"^struct (\w+Params) \{", open(os.path.join(csrc, h)).read(), re.M)]
+    assert len(names) >= 27
+    exe = str(tmp_path / "params_check")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fno-lifetime-dse", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-DALL_PARAMS=" + " ".join(f"CHECK({n})" for n in names),
+                    os.path.join(ROOT, "tests", "host", "params_check.cpp"), "-o", exe], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0 and out.stdout.endswith(f"{len(names)} structs\n0 bad\n"), out.stdout + out.stderr
+
+
 def test_calls_go_to_the_faster_kernel(tmp_path):
     """tests/host/routes_check.cpp: the dispatch's rules at sizes on both sides of them, no device visible."""
     _run_against_the_library(tmp_path, "routes_check", HIP_VISIBLE_DEVICES="")

@@ -36,15 +36,15 @@ typedef __attribute__((ext_vector_type(4))) float gm_f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t gm_u32x4;
 
 struct GemmRowsParams {
-    const uint16_t* a; // [m, k] bf16
-    const uint8_t* w;  // [n, k / 2]
-    const uint16_t* scales;
-    const uint16_t* biases;
-    const uint8_t* zp;
-    const uint16_t* out_bias; // [n] or null
-    void* d;                  // [m, n] (ACT: [m, n / 2]) bf16 or f32
-    float* partials;          // [splits][m, n] f32, or null: the whole sum is here
-    uint32_t m, n, k, d_f32, act_type, splits;
+    const uint16_t* a = nullptr; // [m, k] bf16
+    const uint8_t* w = nullptr;  // [n, k / 2]
+    const uint16_t* scales = nullptr;
+    const uint16_t* biases = nullptr;
+    const uint8_t* zp = nullptr;
+    const uint16_t* out_bias = nullptr; // [n] or null
+    void* d = nullptr;                  // [m, n] (ACT: [m, n / 2]) bf16 or f32
+    float* partials = nullptr;          // [splits][m, n] f32, or null: the whole sum is here
+    uint32_t m = 0, n = 0, k = 0, d_f32 = 0, act_type = 0, splits = 0;
 };
 
 // (lane group g, word j) -> (lane group j, word g): register i of lane group g afterwards holds what word g of lane group i was

@@ -40,17 +40,17 @@ template <int SRC> __device__ __forceinline__ float row_share(float v) {
 }
 
 struct RowsParams {
-    const uint16_t* a; // [m, k] bf16
-    const uint8_t* w;  // [n, k / 2]
-    const uint16_t* scales;
-    const uint16_t* biases;
-    const uint8_t* zp;
-    const uint16_t* out_bias; // [n] or null
-    void* d;                  // [m, n] bf16 or f32
-    uint32_t m, n, k, group_size, kind, d_f32;
-    uint32_t act_type; // ACT instances: n = 2 h weight rows [up | gate]; d = [m, h] = up * act(gate) (GatedActMul, gated_act_mul.rs:36-70)
-    float* partials;   // [gridDim.y][m, n] f32, or null: the whole sum is here
-    RowsNorm norm;     // NORM instances: `a` holds the raw rows
+    const uint16_t* a = nullptr; // [m, k] bf16
+    const uint8_t* w = nullptr;  // [n, k / 2]
+    const uint16_t* scales = nullptr;
+    const uint16_t* biases = nullptr;
+    const uint8_t* zp = nullptr;
+    const uint16_t* out_bias = nullptr; // [n] or null
+    void* d = nullptr;                  // [m, n] bf16 or f32
+    uint32_t m = 0, n = 0, k = 0, group_size = 0, kind = 0, d_f32 = 0;
+    uint32_t act_type = 0;     // ACT instances: n = 2 h weight rows [up | gate]; d = [m, h] = up * act(gate) (GatedActMul, gated_act_mul.rs:36-70)
+    float* partials = nullptr; // [gridDim.y][m, n] f32, or null: the whole sum is here
+    RowsNorm norm;             // NORM instances: `a` holds the raw rows
 };
 
 // ACT: the workgroup owns the 16 up rows row0 .. and the 16 gate rows h + row0 .. (two accumulators, one activation stream), and its epilogue is

@@ -22,49 +22,49 @@ constexpr uint32_t kChipCus = 256; // compute units of an MI355X: for plans of k
 struct NormParams;
 // ---------------------------------------------------------------- matmul (quantised / full-precision B)
 struct MatmulParams {
-    const void* a;      // [m,k] input dtype
-    const void* b;      // codes [n, k*bits/8] or full precision [n,k]
-    const void* scales; // weights dtype [n, groups]
-    const void* biases; // weights dtype [n, groups] (ScaleBias)
-    const uint8_t* zero_points;
-    void* d;            // [m,n] output dtype
-    const void* bias;   // weights dtype [n]
-    const uint32_t* gather; // [m,n] or null
-    uint32_t w_dt, a_dt, d_dt;
-    uint32_t b_kind;    // uzu_matmul_b_kind
-    uint32_t bits;      // 4 / 8 (quantised)
-    uint32_t group_size;
-    uint32_t signed_codes;
-    float ab_scale;
-    uint32_t accumulate;
-    uint32_t has_soft_cap;
-    float soft_cap;
-    uint32_t m, n, k;
+    const void* a = nullptr;      // [m,k] input dtype
+    const void* b = nullptr;      // codes [n, k*bits/8] or full precision [n,k]
+    const void* scales = nullptr; // weights dtype [n, groups]
+    const void* biases = nullptr; // weights dtype [n, groups] (ScaleBias)
+    const uint8_t* zero_points = nullptr;
+    void* d = nullptr;          // [m,n] output dtype
+    const void* bias = nullptr; // weights dtype [n]
+    const uint32_t* gather = nullptr; // [m,n] or null
+    uint32_t w_dt = 0, a_dt = 0, d_dt = 0;
+    uint32_t b_kind = 0; // uzu_matmul_b_kind
+    uint32_t bits = 0;   // 4 / 8 (quantised)
+    uint32_t group_size = 0;
+    uint32_t signed_codes = 0;
+    float ab_scale = 0.0f;
+    uint32_t accumulate = 0;
+    uint32_t has_soft_cap = 0;
+    float soft_cap = 0.0f;
+    uint32_t m = 0, n = 0, k = 0;
     // ---- fused prologue / epilogue options used by the engine (all 0 through the C ABI) ----
-    uint32_t act_mul;   // epilogue: rows [0,n/2) = up, [n/2,n) = gate; writes d[m, n/2] = up * act(gate)
-    uint32_t act_type;
+    uint32_t act_mul = 0; // epilogue: rows [0,n/2) = up, [n/2,n) = gate; writes d[m, n/2] = up * act(gate)
+    uint32_t act_type = 0;
     // Offset-term tables of the large-tile prefill GEMM (k_gemm128.hip) supplied by the caller instead of its pre-pass launch:
     // pre_coef [groups][n] f32 depends on the weights only (gemm_coef_table, once at load); pre_rowsum [groups][Mp] f32, Mp = m rounded up
     // to 4, pad rows zero = the group row sums of A, written by the kernel that produced A (NormParams::rowsum_out).  Both given: no pre-pass.
-    const float* pre_rowsum;
-    const float* pre_coef;
+    const float* pre_rowsum = nullptr;
+    const float* pre_coef = nullptr;
     // pre_rowsum may hold 2^x partial sums per quant group, [groups << x][Mp] (a producer whose workgroups own less than a group of a row: the gated
     // epilogue's 64 columns, a DeltaNet head narrower than the group): the offset term then walks the parts against the group's coefficient row
-    uint32_t rowsum_parts_log2;
+    uint32_t rowsum_parts_log2 = 0;
     // act_mul: the epilogue also files the f32 sums of the 64 gated columns it writes per row, [n / 2 / 64][Mp] (Mp = m rounded up to 4, pad rows zero) --
     // pre_rowsum (parts of 64 columns) of the GEMM that reads D next, which then needs no pre-pass launch.  The large-tile kernel only; null = not filed.
-    float* gated_rowsum_out;
+    float* gated_rowsum_out = nullptr;
     // The int4 DMA form (k_gemm_dma.hip) multiplies rows in pair order: every eight consecutive k as 0 4 1 5 2 6 3 7 (gemm_convert.h).  a_pairs: A's rows in that order, where their
     // producer wrote them so; null: the product's pre-pass makes the copy.  a null beside it: no other form of the rows exists (only where gemm_pairs_wanted said so, and
     // with pre_rowsum).
-    const uint16_t* a_pairs;
-    uint32_t d_pairs; // act_mul on the large tile: D leaves in pair order
+    const uint16_t* a_pairs = nullptr;
+    uint32_t d_pairs = 0; // act_mul on the large tile: D leaves in pair order
     // The Normalization that reads D next (engine prefill: out-projection -> pre-MLP norm, down-projection -> the next layer's pre-mixer norm; its
     // `input` is D).  A split-K GEMM then finishes with ONE launch that adds the partial tiles, applies the epilogue, stores D and normalises the rows
     // (normalization_from_partials) and sets *post_norm_done; every other kernel choice ignores it and the caller runs the normalisation itself.
-    const NormParams* post_norm;
-    uint32_t* post_norm_done;
-    float* few_partials; // optional: kFewPartials floats for the few-rows kernel's shares of K (k_gemv_rows.hip), also while the stream is captured
+    const NormParams* post_norm = nullptr;
+    uint32_t* post_norm_done = nullptr;
+    float* few_partials = nullptr; // optional: kFewPartials floats for the few-rows kernel's shares of K (k_gemv_rows.hip), also while the stream is captured
 };
 bool gemm_coef_table_supported(const MatmulParams& p);                          // the large-tile kernel's quantisation family
 uzu_status gemm_coef_table(hipStream_t s, const MatmulParams& p, float* coef); // coef[g][n]; p needs b / scales / biases / zero_points, n, k, bits, group_size, b_kind
@@ -91,12 +91,12 @@ constexpr size_t kFewPartials = 16 * 4096; // 16 rows x (splits x n), which is 1
 // (speculative verify passes, prefill tails: round 5): every workgroup normalises the rows while it stages them, with the element mapping and
 // reduction order of normalization_kernel (bit-identical rows); workgroup 0 also writes the residual rows and, if asked, the normalised rows.
 struct RowsNorm {
-    const float* scales;         // f32 [k] or null (plain RMS norm)
-    float eps, offset;
-    uint32_t full_layer, residual_add;
-    const uint16_t* shortcut_in; // residual_add: bf16 [m, k], added to the rows first
-    uint16_t* shortcut_out;      // bf16 [m, k] or null: the (summed) rows, i.e. the new residual -- must not alias shortcut_in (other workgroups still read it)
-    uint16_t* normed_out;        // bf16 [m, k] or null: the normalised rows (for a second linear that reads the same rows)
+    const float* scales = nullptr; // f32 [k] or null (plain RMS norm)
+    float eps = 0.0f, offset = 0.0f;
+    uint32_t full_layer = 0, residual_add = 0;
+    const uint16_t* shortcut_in = nullptr; // residual_add: bf16 [m, k], added to the rows first
+    uint16_t* shortcut_out = nullptr;      // bf16 [m, k] or null: the (summed) rows, i.e. the new residual -- must not alias shortcut_in (other workgroups still read it)
+    uint16_t* normed_out = nullptr;        // bf16 [m, k] or null: the normalised rows (for a second linear that reads the same rows)
 };
 bool gemv_rows_norm_supported(const MatmulParams& p);
 uzu_status gemv_rows_mfma(hipStream_t s, const MatmulParams& p, int num_cus, const RowsNorm* norm = nullptr);
@@ -115,31 +115,31 @@ size_t matmul_algorithmic_bytes(const MatmulParams& p); // codes + scales + corr
 
 // ---------------------------------------------------------------- normalization
 struct NormParams {
-    const void* input; // null => in place
-    const void* scales;
-    const void* biases;
-    void* output;
-    void* shortcut;
-    uint32_t io_dt, affine_dt;
-    uint32_t batch_size, element_count;
-    float epsilon, scale_offset, post_layer_scalar;
-    uint32_t subtract_mean, full_layer, copy_to_shortcut, residual_add, scale_residual_sum, scale_output;
+    const void* input = nullptr; // null => in place
+    const void* scales = nullptr;
+    const void* biases = nullptr;
+    void* output = nullptr;
+    void* shortcut = nullptr;
+    uint32_t io_dt = 0, affine_dt = 0;
+    uint32_t batch_size = 0, element_count = 0;
+    float epsilon = 0.0f, scale_offset = 0.0f, post_layer_scalar = 0.0f;
+    uint32_t subtract_mean = 0, full_layer = 0, copy_to_shortcut = 0, residual_add = 0, scale_residual_sum = 0, scale_output = 0;
     // optional: the sums of the OUTPUT row over groups of `rowsum_group` elements, f32 [element_count / rowsum_group][Mp], Mp = batch_size
     // rounded up to 4 (pad rows zeroed) -- MatmulParams::pre_rowsum of the GEMM that consumes the rows (see normalization_rowsum_supported)
-    float* rowsum_out;
-    uint32_t rowsum_group;
-    uint16_t* pairs_out; // optional: the output rows once more, in pair order (MatmulParams::a_pairs); normalization_pairs_supported
+    float* rowsum_out = nullptr;
+    uint32_t rowsum_group = 0;
+    uint16_t* pairs_out = nullptr; // optional: the output rows once more, in pair order (MatmulParams::a_pairs); normalization_pairs_supported
 };
 bool normalization_pairs_supported(uint32_t element_count);
 uzu_status normalization(hipStream_t s, const NormParams& p);
 bool normalization_rowsum_supported(uint32_t element_count, uint32_t group);
 // rows that are still split-K partial tiles [splits][total] f32 of the GEMM producing them (`d` = that GEMM's bf16 output, `bias` its bf16 epilogue bias or null)
 struct NormPartials {
-    const float* partials;
-    uint32_t splits;
-    size_t total;
-    const uint16_t* bias;
-    uint16_t* d;
+    const float* partials = nullptr;
+    uint32_t splits = 0;
+    size_t total = 0;
+    const uint16_t* bias = nullptr;
+    uint16_t* d = nullptr;
 };
 bool normalization_from_partials_supported(const NormParams& p, const NormPartials& sp);
 uzu_status normalization_from_partials(hipStream_t s, const NormParams& p, const NormPartials& sp);
@@ -157,9 +157,9 @@ uzu_status attention_prepare(hipStream_t s, const uint16_t* qkv, uint16_t* queri
                              uint32_t has_kv, const uint32_t* dyn, uint32_t kv_rows_fixed = 0, const uint32_t* trie = nullptr);
 // QKVNorm of the query / key / value heads + AttentionPrepare in one launch (k_elementwise.hip::attention_prepare_normed_kernel; bit-identical to the separate launches)
 struct PrepNorm {
-    const float* scales;
-    float epsilon, scale_offset;
-    uint32_t full_layer, present;
+    const float* scales = nullptr;
+    float epsilon = 0.0f, scale_offset = 0.0f;
+    uint32_t full_layer = 0, present = 0;
 };
 bool attention_prepare_normed_supported(uint32_t head_dim);
 uzu_status attention_prepare_normed(hipStream_t s, const uint16_t* qkv, uint16_t* queries, uint16_t* keys, uint16_t* values, const float* cosines, const float* sines,
@@ -174,26 +174,26 @@ uzu_status kv_ring_insert(hipStream_t s, void* keys, void* values, uint32_t dt, 
                           uint32_t element_dim);
 
 struct AttentionParams {
-    const void* queries;
-    const void* keys;
-    const void* values;
-    uint32_t dt;
-    uint32_t head_dim, gqa_factor, sequence_length; // dyn: sequence_length += *dyn
-    uint32_t k_head_stride, k_seq_stride, v_head_stride, v_seq_stride;
-    uint32_t is_kv_cache_ring, ring_offset, ring_length;
-    float scale;
-    uint32_t is_sliding_window, sliding_window_size;
-    const void* sinks;
-    uint32_t num_heads, suffix_length, is_causal;
-    const uint32_t* dyn;
+    const void* queries = nullptr;
+    const void* keys = nullptr;
+    const void* values = nullptr;
+    uint32_t dt = 0;
+    uint32_t head_dim = 0, gqa_factor = 0, sequence_length = 0; // dyn: sequence_length += *dyn
+    uint32_t k_head_stride = 0, k_seq_stride = 0, v_head_stride = 0, v_seq_stride = 0;
+    uint32_t is_kv_cache_ring = 0, ring_offset = 0, ring_length = 0;
+    float scale = 0.0f;
+    uint32_t is_sliding_window = 0, sliding_window_size = 0;
+    const void* sinks = nullptr;
+    uint32_t num_heads = 0, suffix_length = 0, is_causal = 0;
+    const uint32_t* dyn = nullptr;
     // Ring KV state driven from the device-resident context length (engine; AttentionStateType::Ring, state.rs:16-55): when non-zero (with
     // `dyn`), the prefix is a ring of `ring_window` rows and n = *dyn tokens have been accepted so far, so sequence_length = ring_window +
     // suffix_length, ring_length = min(n, W), ring_offset = n > W ? (n - W) % W : 0 (what encode_accept's offset / length bookkeeping
     // amounts to, state.rs:200-219) -- a replayed graph cannot carry host-side ring parameters.
-    uint32_t ring_window;
+    uint32_t ring_window = 0;
     // Speculative tree (is_trie): one {trie_start, trie_end, height} node per suffix token (gpu_types/trie.rs); a suffix key sits at position
     // suffix_position + height and is visible to the queries trie_start .. trie_end (mask.rs:21-29); null = linear suffix
-    const uint32_t* trie;
+    const uint32_t* trie = nullptr;
 };
 // the (sequence_length, ring_offset, ring_length) a kernel works with: `dyn` applied (host code only reads the fields)
 __host__ __device__ inline void attention_resolve_dyn(AttentionParams& a) {
@@ -218,12 +218,12 @@ bool attention_prefill_mfma_supported(const AttentionParams& p); // k_attention_
 // the same attention of several sequences in one launch (equal suffix lengths; `p` is any one of them): kMost at a time
 struct AttentionSeqs {
     static constexpr uint32_t kMost = 8;
-    const void* queries[kMost];
-    const void* keys[kMost];
-    const void* values[kMost];
-    const uint32_t* dyn[kMost];
-    void* out[kMost];
-    uint32_t n;
+    const void* queries[kMost] = {};
+    const void* keys[kMost] = {};
+    const void* values[kMost] = {};
+    const uint32_t* dyn[kMost] = {};
+    void* out[kMost] = {};
+    uint32_t n = 0;
 };
 bool attention_prefill_mfma_joins(const AttentionParams& p, uint32_t sequences); // whether a sequence goes into an AttentionSeqs launch, of which a full one has that many
 uzu_status attention_prefill_mfma_seqs(hipStream_t s, const AttentionParams& p, const AttentionSeqs& q);
@@ -274,16 +274,16 @@ uzu_status matmul_a8(hipStream_t s, const MatmulParams& p, const int8_t* a_q, co
 // UnifiedSampling with any of: grammar bitmask, temperature, top-k / top-p / min-p, Gumbel-max noise (k_sampling.hip).
 // `scratch` (unified_sampling_scratch_bytes) is only used when no filter is set (two-level arg-max over 256 workgroups).
 struct UnifiedSamplingParams {
-    const void* logits;      // [batch, vocab] of dt
-    uint32_t dt;
-    uint32_t* output;        // [batch]
-    const uint64_t* seeds;   // [batch] or null (greedy)
-    const uint32_t* bitmask; // [batch, ceil(vocab / 32)] or null
-    uint32_t has_temperature, has_top_k, has_top_p, has_min_p;
-    float temperature;
-    uint32_t top_k;
-    float top_p, min_p;
-    uint32_t vocab_size, batch_size;
+    const void* logits = nullptr; // [batch, vocab] of dt
+    uint32_t dt = 0;
+    uint32_t* output = nullptr;        // [batch]
+    const uint64_t* seeds = nullptr;   // [batch] or null (greedy)
+    const uint32_t* bitmask = nullptr; // [batch, ceil(vocab / 32)] or null
+    uint32_t has_temperature = 0, has_top_k = 0, has_top_p = 0, has_min_p = 0;
+    float temperature = 0.0f;
+    uint32_t top_k = 0;
+    float top_p = 0.0f, min_p = 0.0f;
+    uint32_t vocab_size = 0, batch_size = 0;
 };
 uzu_status unified_sampling(hipStream_t s, const UnifiedSamplingParams& p, void* scratch);
 // PRng::derive (sampling/prng.rs): *out = finaliser(base + *position + offset)
@@ -405,8 +405,8 @@ uzu_status fill_u32(hipStream_t s, uint32_t* dst, uint32_t value, uint32_t count
 
 // ---- Mixture of experts (k_moe.hip; MoeBlock::encode, encodable_block/mlp/moe/mod.rs:204-350); bf16 tensors
 struct MoeExpertParams {
-    uint32_t d_model, d_ff, gating_sel; // 0 GELU(up), 1 SiLU(up), 2 SwiGLU, 3 GEGLU
-    float gate_clip_min, gate_clip_max, up_clip_min, up_clip_max, silu_alpha;
+    uint32_t d_model = 0, d_ff = 0, gating_sel = 0; // 0 GELU(up), 1 SiLU(up), 2 SwiGLU, 3 GEGLU
+    float gate_clip_min = 0.0f, gate_clip_max = 0.0f, up_clip_min = 0.0f, up_clip_max = 0.0f, silu_alpha = 0.0f;
 };
 uzu_status moe_router_topk(hipStream_t s, const uint16_t* input, const uint16_t* weight, const uint16_t* bias, int32_t* topk_ids, uint16_t* topk_probs, uint32_t t, uint32_t d_model, uint32_t e,
                            uint32_t k, uint32_t renorm);

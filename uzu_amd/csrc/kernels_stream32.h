@@ -42,16 +42,16 @@ uzu_status rms_norm_rows(hipStream_t s, const float* x, float* out, const float*
 //   the sequence's state *prev[z]; a sequence's position 0 reads row `buckets` (pair_table bf16 [buckets + 1, d]).  A second launch leaves every sequence's
 //   last token of the pass in *prev[z].
 struct EmbedPairParams {
-    const uint32_t* tokens;
-    const uint16_t *table, *pair_table;
-    float* out;
-    uint32_t rows, vocab, d;
-    float scale;
-    uint32_t buckets, mul_prev, mul_cur;
-    const SeqSpan* spans;
-    const uint32_t* row_seq;
-    uint32_t* const* prev; // device array [nseq] of device pointers
-    uint32_t nseq, max_count; // max_count (the longest share of the pass, 0 = unknown) == 1: no second launch, the row's own workgroup stores the token
+    const uint32_t* tokens = nullptr;
+    const uint16_t *table = nullptr, *pair_table = nullptr;
+    float* out = nullptr;
+    uint32_t rows = 0, vocab = 0, d = 0;
+    float scale = 0.0f;
+    uint32_t buckets = 0, mul_prev = 0, mul_cur = 0;
+    const SeqSpan* spans = nullptr;
+    const uint32_t* row_seq = nullptr;
+    uint32_t* const* prev = nullptr; // device array [nseq] of device pointers
+    uint32_t nseq = 0, max_count = 0; // max_count (the longest share of the pass, 0 = unknown) == 1: no second launch, the row's own workgroup stores the token
 };
 uzu_status embed_pair_rows_f32(hipStream_t s, const EmbedPairParams& p);
 
@@ -68,17 +68,17 @@ uzu_status rms_norm_add_rows(hipStream_t s, const float* y, const float* residua
 // The predecessor of a sequence's first row of the pass is prev[seq] (f32 [d], the state; zeros are used instead at position 0); the launch leaves the
 // sequence's last h there.  shift == nullptr: spans / row_seq / prev are unused.
 struct DynTanhParams {
-    const float* x;
-    float* out;
-    const float* scales;
-    const float* biases;
-    float alpha;
-    const float* shift;
-    const uint32_t* row_index;
-    const SeqSpan* spans;
-    const uint32_t* row_seq;
-    float* const* prev; // device array [nseq] of device pointers
-    uint32_t rows, d;
+    const float* x = nullptr;
+    float* out = nullptr;
+    const float* scales = nullptr;
+    const float* biases = nullptr;
+    float alpha = 0.0f;
+    const float* shift = nullptr;
+    const uint32_t* row_index = nullptr;
+    const SeqSpan* spans = nullptr;
+    const uint32_t* row_seq = nullptr;
+    float* const* prev = nullptr; // device array [nseq] of device pointers
+    uint32_t rows = 0, d = 0;
 };
 uzu_status dyn_tanh_norm(hipStream_t s, const DynTanhParams& p);
 
@@ -89,34 +89,34 @@ uzu_status depth_mix(hipStream_t s, const float* slots, size_t slot_stride, cons
 //   X[z] = x + z * x_batch (row pitch ldx), W[z] = w + z * w_batch ([n, k] bf16), Y[z] = y + z * y_batch (row pitch ldy)
 //   act: 0 none, 1 max(.,0)^2, 2 gelu (tanh form), 3 xIELU (v > 0: act_a v^2 + v / 2, else act_b (e^v - 1 - v) + v / 2).  residual (pitch ldr, only with batch == 1) may alias y.
 struct LinearF32Params {
-    const float* x;
-    const uint16_t* w;
-    const uint16_t* bias; // bf16 [n] or null
-    const float* residual;
-    float* y;
-    uint32_t rows, n, k;
-    uint32_t ldx, ldy, ldr;
-    uint32_t batch;
-    size_t x_batch, w_batch, y_batch; // element strides
-    uint32_t act;
-    uint32_t bf16_products;
-    float y_scale;     // != 0: the product (behind bias and act, before the residual) is multiplied by it
-    float soft_cap;    // != 0: ... and then capped, cap * tanh(v / cap) (the read-out's logit cap)
-    float act_a, act_b; // act 3
+    const float* x = nullptr;
+    const uint16_t* w = nullptr;
+    const uint16_t* bias = nullptr; // bf16 [n] or null
+    const float* residual = nullptr;
+    float* y = nullptr;
+    uint32_t rows = 0, n = 0, k = 0;
+    uint32_t ldx = 0, ldy = 0, ldr = 0;
+    uint32_t batch = 0;
+    size_t x_batch = 0, w_batch = 0, y_batch = 0; // element strides
+    uint32_t act = 0;
+    uint32_t bf16_products = 0;
+    float y_scale = 0.0f;  // != 0: the product (behind bias and act, before the residual) is multiplied by it
+    float soft_cap = 0.0f; // != 0: ... and then capped, cap * tanh(v / cap) (the read-out's logit cap)
+    float act_a = 0.0f, act_b = 0.0f; // act 3
     // batched products: product z of row r is multiplied by sigmoid(gate[r * ldgate + z]) (a scalar gate per head) or, with gate_batch != 0, element by element by
     // sigmoid(gate[r * ldgate + z * gate_batch + n]); null = none
-    const float* gate;
-    uint32_t ldgate, gate_batch;
+    const float* gate = nullptr;
+    uint32_t ldgate = 0, gate_batch = 0;
     // a multiplier per (row's token, column) behind all of that: y[r, n] *= f32(mul_table[token[r] * mul_ld + mul_col0 + n])  (bf16 table, an id >= mul_vocab reads
     // row 0; one product per launch; null = none) -- the gate of a per-layer token input
-    const uint16_t* mul_table;
-    const uint32_t* mul_tokens;
-    uint32_t mul_ld, mul_col0, mul_vocab;
+    const uint16_t* mul_table = nullptr;
+    const uint32_t* mul_tokens = nullptr;
+    uint32_t mul_ld = 0, mul_col0 = 0, mul_vocab = 0;
     // Grouped form (matrix-core kernel only; the experts of a mixture, each with its own bucket of rows): product z covers rows row_offsets[z] ..
     // row_offsets[z + 1] - 1 of X and Y (device array [batch + 1]; x_batch / y_batch unused, `rows` = an upper bound of the total for the grid).
-    const uint32_t* row_offsets;
+    const uint32_t* row_offsets = nullptr;
     // row r of X is x[row_map[r]] (device array, or null): a gather folded into the operand load
-    const uint32_t* row_map;
+    const uint32_t* row_map = nullptr;
 };
 uzu_status linear_f32(hipStream_t s, const LinearF32Params& p, const char** variant = nullptr);
 // ... without the matrix cores, in f32 arithmetic throughout: a wave per output column up to 16 rows, 64 x 64 tiles that add in the order of k above
@@ -150,13 +150,13 @@ uzu_status moe_route_topk(hipStream_t s, const float* x, const uint16_t* router,
 // `groups` equal groups of neighbours; a group's strength is the sum of its two largest c (of its one, if it has one); only outputs of the `keep` strongest groups
 // can be chosen (ties: the lower group).  The `top` largest c among them win (ties: the lower index); weights = s / (sum of the winners' s + 1e-20) * scale, or (raw) s * scale.
 struct RouteGroupsParams {
-    const float* x;
-    const uint16_t* router;
-    const float* selection_bias;
-    int32_t* ids;
-    float* weights;
-    uint32_t rows, d, outputs, top, groups, keep, bf16_products, raw;
-    float scale;
+    const float* x = nullptr;
+    const uint16_t* router = nullptr;
+    const float* selection_bias = nullptr;
+    int32_t* ids = nullptr;
+    float* weights = nullptr;
+    uint32_t rows = 0, d = 0, outputs = 0, top = 0, groups = 0, keep = 0, bf16_products = 0, raw = 0;
+    float scale = 0.0f;
 };
 uzu_status moe_route_groups(hipStream_t s, const RouteGroupsParams& p);
 // The gated product of an expert's hidden unit: g = clamp(gate, gate_min, gate_max), u = clamp(up, up_min, up_max), g * sigmoid(alpha * g) * (u + up_offset).
@@ -178,14 +178,14 @@ uzu_status gated_act_rows(hipStream_t s, const float* y1, float* hidden, uint32_
 
 // rms_norm_add_rows with its `next`, as a part of other launches: out[r] = residual[r] + rms(y[r]) * (scales + offset) * layer_scale, next[r] = rms(out[r]) * (next_scales + next_offset)
 struct NormAddParams {
-    const float *y, *residual;
-    float* out;
-    const float *scales, *layer_scale; // layer_scale: f32 [d] or null
-    float offset, eps;
-    float* next;
-    const float* next_scales;
-    float next_offset, next_eps;
-    uint32_t rows, d;
+    const float *y = nullptr, *residual = nullptr;
+    float* out = nullptr;
+    const float *scales = nullptr, *layer_scale = nullptr; // layer_scale: f32 [d] or null
+    float offset = 0.0f, eps = 0.0f;
+    float* next = nullptr;
+    const float* next_scales = nullptr;
+    float next_offset = 0.0f, next_eps = 0.0f;
+    uint32_t rows = 0, d = 0;
 };
 bool norm_add_step_supported(const NormAddParams& n); // rows of up to 4096, a multiple of 8
 // ... and moe_route_groups of next (one group of outputs, up to 64 of them, up to 8 winners) in one launch; p.x is not read
@@ -203,18 +203,18 @@ uzu_status norm_linear(hipStream_t s, const NormAddParams& n, const LinearF32Par
 // Between two decode steps of one sequence: the greedy choice among such parts (of equal values the lowest index), *out_token, sampled[*ctx_len], tokens[0], *ctx_len + 1 and the span behind it;
 // then out = scale * the token's embedding row and, with `normed`, its RMS norm * (scales + offset).  parts 0: only the latter two, for tokens[0].
 struct StepTurnParams {
-    const float* part_value;
-    const uint32_t* part_index;
-    uint32_t parts;
-    uint32_t *ctx_len, *tokens, *out_token, *sampled;
-    SeqSpan* span;
-    const uint16_t* table;
-    uint32_t vocab, d;
-    float scale;
-    float* out;
-    float* normed;
-    const float* scales;
-    float offset, eps;
+    const float* part_value = nullptr;
+    const uint32_t* part_index = nullptr;
+    uint32_t parts = 0;
+    uint32_t *ctx_len = nullptr, *tokens = nullptr, *out_token = nullptr, *sampled = nullptr;
+    SeqSpan* span = nullptr;
+    const uint16_t* table = nullptr;
+    uint32_t vocab = 0, d = 0;
+    float scale = 0.0f;
+    float* out = nullptr;
+    float* normed = nullptr;
+    const float* scales = nullptr;
+    float offset = 0.0f, eps = 0.0f;
 };
 bool step_turn_supported(const StepTurnParams& p);
 uzu_status step_turn(hipStream_t s, const StepTurnParams& p);
@@ -241,15 +241,15 @@ uzu_status experts_few_down(hipStream_t s, const float* hidden, const float* x, 
 // [rows * top][2 ff], hidden [rows * top][ff], y2 [rows * top][d] f32; perm / slot_pos [rows * top], offsets [routed + 1], cursor [routed] u32.
 // pos_weight (f32 [rows * top] or null): the winners' weights multiply the experts' inputs instead of their results (not with plain experts).
 struct MoeGroupedParams {
-    const float* x;
-    const int32_t* ids;
-    const float* weights;
-    const uint16_t *w13, *w2;
-    const float* residual;
-    float* y;
-    float *y1, *hidden, *y2, *pos_weight;
-    uint32_t *perm, *slot_pos, *offsets, *cursor;
-    uint32_t rows, d, ff, routed, top;
+    const float* x = nullptr;
+    const int32_t* ids = nullptr;
+    const float* weights = nullptr;
+    const uint16_t *w13 = nullptr, *w2 = nullptr;
+    const float* residual = nullptr;
+    float* y = nullptr;
+    float *y1 = nullptr, *hidden = nullptr, *y2 = nullptr, *pos_weight = nullptr;
+    uint32_t *perm = nullptr, *slot_pos = nullptr, *offsets = nullptr, *cursor = nullptr;
+    uint32_t rows = 0, d = 0, ff = 0, routed = 0, top = 0;
     ExpertAct act;
     uint32_t f32_products = 0; // true f32 products (y1 unused)
 };
@@ -266,31 +266,31 @@ uzu_status latent_norm_append(hipStream_t s, const float* x, const float* scales
 //   s_j = scale * <qlat[r, h, :], c_j>,  weights = exp(s_j - m) / (sum_j exp(s_j - m) + exp(sink_h - m)),  out[r, h, :] = sum_j weights_j c_j
 // qlat / out f32 [rows, heads * rank]; c_j = caches[q][j * rank ...] (bf16 or f32); sinks f32 [heads] or null (no sink term).
 struct LatentAttentionParams {
-    const float* qlat;
-    float* out;
-    void* const* caches;
-    uint32_t cache_bf16;
-    const float* sinks;
-    const SeqSpan* spans;
-    const uint32_t* row_seq;
-    uint32_t rows, heads, rank, window;
-    float scale;
-    uint32_t form; // 0: chosen by shape; 1: the simple form (a wave per row and head, keys one after the other); 2: the tiled form
+    const float* qlat = nullptr;
+    float* out = nullptr;
+    void* const* caches = nullptr;
+    uint32_t cache_bf16 = 0;
+    const float* sinks = nullptr;
+    const SeqSpan* spans = nullptr;
+    const uint32_t* row_seq = nullptr;
+    uint32_t rows = 0, heads = 0, rank = 0, window = 0;
+    float scale = 0.0f;
+    uint32_t form = 0; // 0: chosen by shape; 1: the simple form (a wave per row and head, keys one after the other); 2: the tiled form
     // != 0: only the first value_rank columns of a cache row are values -- the rest (a rotated key part) takes part in the scores alone, and the matching columns of
     // `out` are left unwritten by the tiled form (a multiple of 4, at most rank); 0: the whole row
-    uint32_t nseq;  // entries of `spans`
-    uint32_t tiles; // sum over the sequences of ceil(count * heads / 128): the tiled form's workgroups (the caller knows the counts)
-    uint32_t value_rank;
+    uint32_t nseq = 0;  // entries of `spans`
+    uint32_t tiles = 0; // sum over the sequences of ceil(count * heads / 128): the tiled form's workgroups (the caller knows the counts)
+    uint32_t value_rank = 0;
     // rope_dim != 0: the last rope_dim columns of a query are not in qlat but turned as they are loaded: the last rope_dim coordinates of head a of `queries`
     // (f32 rows of pitch ldqueries, a head q_width wide), by the row's position (tables and pairs as latent_rope_append reads them)
-    const float* queries;
-    uint32_t ldqueries, q_width, rope_dim, interleaved;
-    const float *cosines, *sines;
+    const float* queries = nullptr;
+    uint32_t ldqueries = 0, q_width = 0, rope_dim = 0, interleaved = 0;
+    const float *cosines = nullptr, *sines = nullptr;
     // tiled form, few rows over many keys (decode): `splits` > 1 workgroups share the key blocks of an item tile, partial sums go through split_ws
     // (latent_attention_split_ws_bytes(rows, heads, rank, splits) bytes) and a merge launch.  0 / null: one workgroup walks all keys of its tile.
-    uint32_t splits;
-    float* split_ws;
-    size_t split_ws_bytes;
+    uint32_t splits = 0;
+    float* split_ws = nullptr;
+    size_t split_ws_bytes = 0;
 };
 size_t latent_attention_split_ws_bytes(uint32_t rows, uint32_t heads, uint32_t rank, uint32_t splits);
 bool latent_attention_tiled_supported(const LatentAttentionParams& p);
@@ -307,22 +307,22 @@ constexpr uint32_t kLatentMaxRank = 2048;
 // q_rank != 0: the row's first q_rank numbers (column 0) are a query latent, not queries: its RMS norm (q_scales, eps) goes to q_latent[r, :] (f32 [rows][q_rank]) and
 // qlat must be null -- the queries are turned by a second launch over their own rows (caches null).
 struct LatentRopeAppendParams {
-    uint32_t q_rank;
-    const float* q_scales;
-    float* q_latent;
-    const float* x;
-    uint32_t ldx, c_col, rank, rope_dim;
-    const float* scales;
-    float eps;
-    void* const* caches;
-    uint32_t cache_bf16;
-    uint32_t heads, q_width;
-    float* qlat;
-    const float *cosines, *sines;
-    uint32_t interleaved;
-    const SeqSpan* spans;
-    const uint32_t* row_seq;
-    uint32_t rows;
+    uint32_t q_rank = 0;
+    const float* q_scales = nullptr;
+    float* q_latent = nullptr;
+    const float* x = nullptr;
+    uint32_t ldx = 0, c_col = 0, rank = 0, rope_dim = 0;
+    const float* scales = nullptr;
+    float eps = 0.0f;
+    void* const* caches = nullptr;
+    uint32_t cache_bf16 = 0;
+    uint32_t heads = 0, q_width = 0;
+    float* qlat = nullptr;
+    const float *cosines = nullptr, *sines = nullptr;
+    uint32_t interleaved = 0;
+    const SeqSpan* spans = nullptr;
+    const uint32_t* row_seq = nullptr;
+    uint32_t rows = 0;
 };
 uzu_status latent_rope_append(hipStream_t s, const LatentRopeAppendParams& p);
 
@@ -336,21 +336,21 @@ uzu_status latent_rope_append(hipStream_t s, const LatentRopeAppendParams& p);
 // q_norm / k_norm (f32 [dim], optional): every query / key head is RMS-normed over its dim coordinates (norm_eps, plain weights) in front of the rotation.
 // Values go to the cache first, as the projection left them: v_col == k_col (vdim == dim) makes the values the keys in front of their norm and rotation.
 struct RopeAppendParams {
-    float* qkv;
-    uint32_t ld, k_col, v_col;
-    uint32_t heads, kv_heads, dim, vdim, rope_dim;
-    const float *cosines, *sines;
-    float key_scale;
-    const float *q_norm, *k_norm;
-    float norm_eps;
-    uint32_t norm_whole;  // q_norm / k_norm are f32 [heads * dim] / [kv_heads * dim]: ONE RMS norm over all of a row's query (key) coordinates instead of one per head
-    uint32_t interleaved; // the rotation pairs coordinates (2i, 2i + 1) instead of (i, i + rope_dim / 2)
-    void* const* key_caches;
-    void* const* value_caches;
-    uint32_t cache_bf16;
-    const SeqSpan* spans;
-    const uint32_t* row_seq;
-    uint32_t rows;
+    float* qkv = nullptr;
+    uint32_t ld = 0, k_col = 0, v_col = 0;
+    uint32_t heads = 0, kv_heads = 0, dim = 0, vdim = 0, rope_dim = 0;
+    const float *cosines = nullptr, *sines = nullptr;
+    float key_scale = 0.0f;
+    const float *q_norm = nullptr, *k_norm = nullptr;
+    float norm_eps = 0.0f;
+    uint32_t norm_whole = 0;  // q_norm / k_norm are f32 [heads * dim] / [kv_heads * dim]: ONE RMS norm over all of a row's query (key) coordinates instead of one per head
+    uint32_t interleaved = 0; // the rotation pairs coordinates (2i, 2i + 1) instead of (i, i + rope_dim / 2)
+    void* const* key_caches = nullptr;
+    void* const* value_caches = nullptr;
+    uint32_t cache_bf16 = 0;
+    const SeqSpan* spans = nullptr;
+    const uint32_t* row_seq = nullptr;
+    uint32_t rows = 0;
 };
 uzu_status rope_append(hipStream_t s, const RopeAppendParams& p);
 
@@ -359,40 +359,40 @@ uzu_status rope_append(hipStream_t s, const RopeAppendParams& p);
 //   p_j = exp(s_j - m) / (sum_j exp(s_j - m) + exp(sink_a - m))   (sinks f32 [heads] or null: no sink term),   out[r, a, :] = sum_j p_j V_z[j, g, :]
 // q f32 rows of pitch ldq (head a at column a * dim), out f32 [rows][heads * vdim]; caches as rope_append writes them.
 struct WindowAttentionParams {
-    const float* q;
-    uint32_t ldq;
-    float* out;
-    void* const* key_caches;
-    void* const* value_caches;
-    uint32_t cache_bf16;
-    const float* sinks;
-    const SeqSpan* spans;
-    const uint32_t* row_seq;
-    uint32_t rows, heads, kv_heads, dim, vdim, window;
-    float scale, soft_cap;
+    const float* q = nullptr;
+    uint32_t ldq = 0;
+    float* out = nullptr;
+    void* const* key_caches = nullptr;
+    void* const* value_caches = nullptr;
+    uint32_t cache_bf16 = 0;
+    const float* sinks = nullptr;
+    const SeqSpan* spans = nullptr;
+    const uint32_t* row_seq = nullptr;
+    uint32_t rows = 0, heads = 0, kv_heads = 0, dim = 0, vdim = 0, window = 0;
+    float scale = 0.0f, soft_cap = 0.0f;
     // chunk != 0: the row at position t sees keys j <= t of its own chunk only, j >= floor(t / chunk) * chunk (chunks counted from position 0 of the sequence).
     // head_scale (f32 [heads] or null): the scaled score of head a is multiplied by head_scale[a].  dist_bias (f32 [dist_rows][heads] or null): dist_bias[min(t - j,
     // dist_rows - 1), a] is added behind scale, head_scale and cap.  gate (f32 rows of pitch ldgate or null): out[r, a, :] is multiplied by sigmoid(gate[r, a]).
-    uint32_t chunk;
-    const float* head_scale;
-    const float* dist_bias;
-    uint32_t dist_rows;
-    const float* gate;
-    uint32_t ldgate;
+    uint32_t chunk = 0;
+    const float* head_scale = nullptr;
+    const float* dist_bias = nullptr;
+    uint32_t dist_rows = 0;
+    const float* gate = nullptr;
+    uint32_t ldgate = 0;
     // ldo: row pitch of `out` (0 = heads * vdim); out_scale: everything above times it (0 = 1)
-    uint32_t ldo;
-    float out_scale;
-    uint32_t form;  // 0: chosen by shape; 1: the simple form (a wave per row and head); 2: the matrix-core form
-    uint32_t nseq;  // entries of `spans`
-    uint32_t tiles; // sum over the sequences of ceil(count * (heads / kv_heads) / 128): the matrix-core form's item tiles (the caller knows the counts)
-    uint32_t tiles32; // ... of ceil(count * (heads / kv_heads) / 32): its key-split form's with split_items = 32
+    uint32_t ldo = 0;
+    float out_scale = 0.0f;
+    uint32_t form = 0;  // 0: chosen by shape; 1: the simple form (a wave per row and head); 2: the matrix-core form
+    uint32_t nseq = 0;  // entries of `spans`
+    uint32_t tiles = 0; // sum over the sequences of ceil(count * (heads / kv_heads) / 128): the matrix-core form's item tiles (the caller knows the counts)
+    uint32_t tiles32 = 0; // ... of ceil(count * (heads / kv_heads) / 32): its key-split form's with split_items = 32
     // matrix-core form, few rows over many keys (decode): `splits` > 1 workgroups share the key blocks of an item tile, partial sums go through split_ws
     // (window_attention_split_ws_bytes(rows, heads, splits) bytes) and a merge launch.  0 / null: one workgroup walks all keys of its tile.
-    uint32_t splits, split_items; // split_items: items a workgroup takes, 128 (stretches of 32 keys) or 32 (of 128; also 0); set, the pass is not the step form's
-    float* split_ws;
-    size_t split_ws_bytes;
-    uint32_t keys;    // that a row of this pass sees at the most, as far as the caller knows (which form is the faster rests on it); 0: not known
-    uint32_t one_row; // every sequence of the pass brings exactly one row (row r is sequence r's): the step form, with `splits` >= 1 shares of a row's keys
+    uint32_t splits = 0, split_items = 0; // split_items: items a workgroup takes, 128 (stretches of 32 keys) or 32 (of 128; also 0); set, the pass is not the step form's
+    float* split_ws = nullptr;
+    size_t split_ws_bytes = 0;
+    uint32_t keys = 0;    // that a row of this pass sees at the most, as far as the caller knows (which form is the faster rests on it); 0: not known
+    uint32_t one_row = 0; // every sequence of the pass brings exactly one row (row r is sequence r's): the step form, with `splits` >= 1 shares of a row's keys
 };
 // `splits` and `split_items` of a decode-sized pass whose rows see `keys` keys at the most, from `rows`, `tiles` and `kv_heads`: at most 16 splits, of the step form at most 32
 void window_attention_split_keys(WindowAttentionParams& p, uint32_t keys, uint32_t num_cus);
@@ -419,25 +419,25 @@ uzu_status window_attention_merge(hipStream_t s, const WindowAttentionParams& p,
 // join = f32 [s | s | s s]: in | out | mix[from, to] of the sublayer that yielded y; read = in of the sublayer that follows.  src_stride 0: all copies equal the one
 // row (the embedding rows).  row_index: row r of `h` is row row_index[r] of the stream.
 struct HyperStepParams {
-    const float* src;
-    float* dst;
-    size_t src_stride, dst_stride;
-    const float* y;
-    const float* join;
-    float mult;
-    float* sum_out;
-    const float* read;
-    float* h;
-    const float* scales;
-    float offset, eps;
-    const uint32_t* row_index;
-    uint32_t rows, d, streams;
-    const float* conv_w;
-    uint32_t taps;
-    float* const* states;
-    size_t state_offset;
-    const SeqSpan* spans;
-    const uint32_t* row_seq;
+    const float* src = nullptr;
+    float* dst = nullptr;
+    size_t src_stride = 0, dst_stride = 0;
+    const float* y = nullptr;
+    const float* join = nullptr;
+    float mult = 0.0f;
+    float* sum_out = nullptr;
+    const float* read = nullptr;
+    float* h = nullptr;
+    const float* scales = nullptr;
+    float offset = 0.0f, eps = 0.0f;
+    const uint32_t* row_index = nullptr;
+    uint32_t rows = 0, d = 0, streams = 0;
+    const float* conv_w = nullptr;
+    uint32_t taps = 0;
+    float* const* states = nullptr;
+    size_t state_offset = 0;
+    const SeqSpan* spans = nullptr;
+    const uint32_t* row_seq = nullptr;
 };
 constexpr uint32_t kHyperMaxStreams = 16, kHyperMaxWidth = 32768;
 uzu_status hyper_step(hipStream_t s, const HyperStepParams& p);
@@ -449,19 +449,19 @@ uzu_status hyper_step(hipStream_t s, const HyperStepParams& p);
 // by token; 2: in chunks of 64 rows (scores of the chunk's own rows + the carried state, a decayed state update per chunk; head widths up to 128 on the matrix
 // cores with f32 operands); 3: the chunks without the matrix cores.
 struct RetentionParams {
-    const float* qkv;
-    uint32_t ld, q_col, k_col, v_col;
-    float* out; // [rows][heads * vdim]
-    float* const* states;
-    const float* decay; // f32 [heads]
-    const SeqSpan* spans;
-    uint32_t nseq, rows, heads, dim, vdim;
-    uint32_t form;
+    const float* qkv = nullptr;
+    uint32_t ld = 0, q_col = 0, k_col = 0, v_col = 0;
+    float* out = nullptr; // [rows][heads * vdim]
+    float* const* states = nullptr;
+    const float* decay = nullptr; // f32 [heads]
+    const SeqSpan* spans = nullptr;
+    uint32_t nseq = 0, rows = 0, heads = 0, dim = 0, vdim = 0;
+    uint32_t form = 0;
     // the chunked form: chunks = sum over the sequences of ceil(count / 64) (the caller knows the counts) and a workspace of
     // retention_chunk_ws_bytes(chunks, heads, dim, vdim) bytes; without one, form 0 goes token by token
-    uint32_t chunks;
-    float* chunk_ws;
-    size_t chunk_ws_bytes;
+    uint32_t chunks = 0;
+    float* chunk_ws = nullptr;
+    size_t chunk_ws_bytes = 0;
 };
 size_t retention_chunk_ws_bytes(uint32_t chunks, uint32_t heads, uint32_t dim, uint32_t vdim);
 bool retention_supported(uint32_t dim, uint32_t vdim);
@@ -482,23 +482,23 @@ uzu_status head_rms_gate(hipStream_t s, float* x, const float* gate, uint32_t ld
 //              the pieces' carries joined in order (differs from form 1 by f32 rounding only); needs `pieces` = sum over the sequences of ceil(count / 32) and a
 //              workspace of lru_piece_ws_bytes(pieces, width) bytes, without which form 0 goes position by position.
 struct GatedLruParams {
-    const float* branches;
-    uint32_t ld, x_col;
-    float* u;            // [rows][width]
-    const float* gates;  // [rows][2 width]
-    float* out;          // [rows][width]
-    const float *conv_w, *conv_b, *gate_b, *lambda;
-    float rate;
-    float* const* states;      // device array [nseq]: f32 [width]
-    float* const* conv_states; // device array [nseq]: f32 [taps - 1][width]
-    const SeqSpan* spans;
-    const uint32_t* row_seq;
-    uint32_t nseq, rows, width, blocks, taps;
-    uint32_t form;
-    uint32_t max_count; // the longest sequence share of the pass (the caller knows the counts)
-    uint32_t pieces;
-    float* piece_ws;
-    size_t piece_ws_bytes;
+    const float* branches = nullptr;
+    uint32_t ld = 0, x_col = 0;
+    float* u = nullptr;           // [rows][width]
+    const float* gates = nullptr; // [rows][2 width]
+    float* out = nullptr;         // [rows][width]
+    const float *conv_w = nullptr, *conv_b = nullptr, *gate_b = nullptr, *lambda = nullptr;
+    float rate = 0.0f;
+    float* const* states = nullptr;      // device array [nseq]: f32 [width]
+    float* const* conv_states = nullptr; // device array [nseq]: f32 [taps - 1][width]
+    const SeqSpan* spans = nullptr;
+    const uint32_t* row_seq = nullptr;
+    uint32_t nseq = 0, rows = 0, width = 0, blocks = 0, taps = 0;
+    uint32_t form = 0;
+    uint32_t max_count = 0; // the longest sequence share of the pass (the caller knows the counts)
+    uint32_t pieces = 0;
+    float* piece_ws = nullptr;
+    size_t piece_ws_bytes = 0;
 };
 size_t lru_piece_ws_bytes(uint32_t pieces, uint32_t width);
 uzu_status lru_conv(hipStream_t s, const GatedLruParams& p);
@@ -512,17 +512,17 @@ uzu_status lru_scan(hipStream_t s, const GatedLruParams& p);
 // same `x`, which must still hold the pass's inputs.  A sequence that brings one row has its window replaced by causal_conv_rows itself; max_count (the longest
 // share of the pass, 0 = unknown) == 1 makes causal_conv_commit a no-op.
 struct CausalConvParams {
-    const float* x;
-    uint32_t ldx, x_col;
-    float* out;
-    uint32_t ldo, o_col;
-    const float *w, *bias;
-    uint32_t channels, taps, add_input, act, act_from;
-    float* const* states; // device array [nseq]
-    size_t state_offset;  // floats
-    const SeqSpan* spans;
-    const uint32_t* row_seq;
-    uint32_t nseq, rows, max_count;
+    const float* x = nullptr;
+    uint32_t ldx = 0, x_col = 0;
+    float* out = nullptr;
+    uint32_t ldo = 0, o_col = 0;
+    const float *w = nullptr, *bias = nullptr;
+    uint32_t channels = 0, taps = 0, add_input = 0, act = 0, act_from = 0;
+    float* const* states = nullptr; // device array [nseq]
+    size_t state_offset = 0;        // floats
+    const SeqSpan* spans = nullptr;
+    const uint32_t* row_seq = nullptr;
+    uint32_t nseq = 0, rows = 0, max_count = 0;
 };
 uzu_status causal_conv_rows(hipStream_t s, const CausalConvParams& p);
 uzu_status causal_conv_commit(hipStream_t s, const CausalConvParams& p);
@@ -535,26 +535,26 @@ uzu_status conv_rope_append(hipStream_t s, const RopeAppendParams& p, const Caus
 // Per head, in place: x[r, a, :] <- x[r, a, :] / sqrt(mean(x[r, a, :]^2) + eps) * weight[:] * gate(g[r, a, :])    (x f32 rows of pitch ldx, heads * width used;
 // weight f32 [width] or null; g f32 rows of pitch ldgate or null; gate = sigmoid (gate_sigmoid) or silu)
 struct HeadNormGateParams {
-    float* x;
-    uint32_t ldx;
-    const float* weight;
-    const float* gate;
-    uint32_t ldgate, gate_sigmoid;
-    float eps;
-    uint32_t rows, heads, width;
+    float* x = nullptr;
+    uint32_t ldx = 0;
+    const float* weight = nullptr;
+    const float* gate = nullptr;
+    uint32_t ldgate = 0, gate_sigmoid = 0;
+    float eps = 0.0f;
+    uint32_t rows = 0, heads = 0, width = 0;
 };
 uzu_status head_norm_gate_rows(hipStream_t s, const HeadNormGateParams& p);
 
 // The gate in front of the norm, the norm in `parts` equal consecutive parts of the row:  u = y * silu(gate),  out[r, i] = u[i] / sqrt(mean over i's part of u^2 + eps) *
 // weight[i] * out_scale   (y / gate / out: f32 rows of pitch ldy / ldgate / ldo, `width` used; weight f32 [width]; out may be y)
 struct GatedNormParams {
-    const float* y;
-    const float* gate;
-    const float* weight;
-    float* out;
-    uint32_t ldy, ldgate, ldo;
-    float eps, out_scale;
-    uint32_t rows, width, parts;
+    const float* y = nullptr;
+    const float* gate = nullptr;
+    const float* weight = nullptr;
+    float* out = nullptr;
+    uint32_t ldy = 0, ldgate = 0, ldo = 0;
+    float eps = 0.0f, out_scale = 0.0f;
+    uint32_t rows = 0, width = 0, parts = 0;
 };
 uzu_status gated_norm_rows(hipStream_t s, const GatedNormParams& p);
 
@@ -567,17 +567,17 @@ uzu_status gated_norm_rows(hipStream_t s, const GatedNormParams& p);
 // behind its last.  decay f32 [rows][heads * dim], beta f32 rows of pitch ldbeta, out f32 [rows][heads * vdim].  All f32; every sum runs in the same order
 // whatever else the pass carries and however the rows were cut into passes.
 struct ChannelDeltaParams {
-    float* qkv;
-    uint32_t ld, q_col, k_col, v_col;
-    float* decay;
-    float* beta;
-    uint32_t ldbeta;
-    const float *a_log, *dt_bias;
-    float unit_eps;
-    float* out;
-    float* const* states;
-    const SeqSpan* spans;
-    uint32_t nseq, rows, heads, groups, dim, vdim;
+    float* qkv = nullptr;
+    uint32_t ld = 0, q_col = 0, k_col = 0, v_col = 0;
+    float* decay = nullptr;
+    float* beta = nullptr;
+    uint32_t ldbeta = 0;
+    const float *a_log = nullptr, *dt_bias = nullptr;
+    float unit_eps = 0.0f;
+    float* out = nullptr;
+    float* const* states = nullptr;
+    const SeqSpan* spans = nullptr;
+    uint32_t nseq = 0, rows = 0, heads = 0, groups = 0, dim = 0, vdim = 0;
 };
 bool channel_delta_supported(uint32_t dim, uint32_t vdim);
 uzu_status channel_delta_prep(hipStream_t s, const ChannelDeltaParams& p);
@@ -593,20 +593,20 @@ uzu_status channel_delta(hipStream_t s, const ChannelDeltaParams& p);
 // chunks = sum over the sequences of ceil(count / 64) and a workspace of decayed_state_chunk_ws_bytes(chunks, heads, dim, vdim) bytes, without which form 0 goes
 // token by token).
 struct DecayedStateParams {
-    const float* rows_in;
-    uint32_t ld, q_col, k_col, v_col;
-    const float* decay;
-    uint32_t lddecay, per_head;
-    float inv_temperature;
-    const float *a_log, *dt_bias, *skip;
-    float q_scale;
-    float* out; // [rows][heads * vdim]
-    float* const* states;
-    const SeqSpan* spans;
-    uint32_t nseq, rows, heads, groups, dim, vdim;
-    uint32_t form, chunks;
-    float* chunk_ws;
-    size_t chunk_ws_bytes;
+    const float* rows_in = nullptr;
+    uint32_t ld = 0, q_col = 0, k_col = 0, v_col = 0;
+    const float* decay = nullptr;
+    uint32_t lddecay = 0, per_head = 0;
+    float inv_temperature = 0.0f;
+    const float *a_log = nullptr, *dt_bias = nullptr, *skip = nullptr;
+    float q_scale = 0.0f;
+    float* out = nullptr; // [rows][heads * vdim]
+    float* const* states = nullptr;
+    const SeqSpan* spans = nullptr;
+    uint32_t nseq = 0, rows = 0, heads = 0, groups = 0, dim = 0, vdim = 0;
+    uint32_t form = 0, chunks = 0;
+    float* chunk_ws = nullptr;
+    size_t chunk_ws_bytes = 0;
 };
 size_t decayed_state_chunk_ws_bytes(uint32_t chunks, uint32_t heads, uint32_t dim, uint32_t vdim);
 bool decayed_state_supported(uint32_t dim, uint32_t vdim);
