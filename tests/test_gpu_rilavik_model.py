@@ -775,7 +775,7 @@ def test_refusals_of_the_engine(hip_ctx, tmp_path):
                         (changed(1, kv_source_layer_index=0), "convolved queries on another layer's cache"), (changed(0, decay_temperature=0.0), "temperature"),
                         (changed(0, sliding_window_size=4), "attention options on gated linear attention"), (changed(0, qkv_conv=p.qkv_conv), "options of attention"),
                         (changed(0, moe=dataclasses.replace(g.moe, plain_experts=True)), "weights on the inputs"),
-                        (changed(0, moe=dataclasses.replace(g.moe, routing=D.MOE_ROUTE_TOPK_LOGITS)), "raw scores"), (dataclasses.replace(bundle, f32_stream=False), "")):
+                        (changed(0, moe=dataclasses.replace(g.moe, routing=D.MOE_ROUTE_TOPK_LOGITS)), "raw scores"), (dataclasses.replace(bundle, f32_stream=False), "layer 0 uses a mechanism of the f32-stream designs")):
         with pytest.raises(_ffi.UzuHipError, match=why):
             HipModel(hip_ctx, broken, MODEL_FULL_F32 if broken.f32_stream else 0)
 
